@@ -666,7 +666,7 @@ inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 void op_softmax(Handle& h, const void* beta, const Layout& lb, void* alpha, const Layout& la,
                 void* mask, const Layout& lm, void* drop, const Layout& ld, float scale, float p,
                 uint32_t site, const void* amask = nullptr, const Layout* lam = nullptr,
-                float mscale = 1.f) {
+                float mscale = 1.f, const AttnArgs* stats = nullptr) {
     Space sp = make_space(h.sz, {dH, dB, dJ}, dK);
     View vb = make_view(beta, lb, sp), va = make_view(alpha, la, sp), vm = make_view(mask, lm, sp),
          vd = make_view(drop, ld, sp);
@@ -679,7 +679,8 @@ void op_softmax(Handle& h, const void* beta, const Layout& lb, void* alpha, cons
     } else {
         flatten(sp.rs, {&vb, &va, &vm, &vd});
     }
-    launch_softmax(sp.rs, vb, va, vm, vd, vam, scale, mscale, make_key(h, site, p), h.stream);
+    launch_softmax(sp.rs, vb, va, vm, vd, vam, scale, mscale, make_key(h, site, p), h.stream, stats ? stats->lse : nullptr,
+                   stats ? stats->keep : nullptr, mha_keep_pitch((unsigned)h.sz.n[dK]));
 }
 
 void op_bs(Handle& h, const void* alpha, const Layout& la, const void* mask, const Layout& lm,
@@ -852,7 +853,17 @@ bool attention_planned(const Handle& h) {
            attn_side(nullptr, h.lf[GAMMA], dJ, t) && attn_side(nullptr, h.lb[DGAMMA], dJ, t) &&
            attn_side(nullptr, h.lDQQ, dJ, t) && attn_side(nullptr, h.lDKK, dK, t) &&
            mha_stat_bytes(z.n[dH], z.n[dB], z.n[dJ]) <=
+               (size_t)(z.n[dH] * z.n[dB] * z.n[dJ] * z.n[dK]) * sizeof(half_t) &&
+           mha_keep_bytes(z.n[dH], z.n[dB], z.n[dJ], z.n[dK]) <=
                (size_t)(z.n[dH] * z.n[dB] * z.n[dJ] * z.n[dK]) * sizeof(half_t);
+}
+
+// The forward pass of a ReLU layer whose sequence length is not a multiple of 128 keeps the operators (scores and dropped
+// probabilities rounded to fp16 in memory) although the backward pass runs in registers: there the kernels that keep the
+// scores in registers round differently, and a pre-activation that rounds to the other side of zero moves whole elements
+// of the weight gradients.  The softmax operator then leaves what the backward kernels read.
+bool forward_in_operators(const Handle& h) {
+    return h.act == ACT_RELU && (h.sz.n[dJ] % 128 != 0 || h.sz.n[dK] % 128 != 0);
 }
 
 // Decided from what the forward pass sees, so that both passes take the same path.
@@ -876,7 +887,7 @@ bool attention_fused(const Handle& h, void* const* F, AttnArgs& a) {
         }
         ok = mha_forward_ok(a, (int)z.n[dP]);
     }
-    if (!ok && h.fuse_attention == SUB_FUSE_REQUIRED)
+    if ((!ok || forward_in_operators(h)) && h.fuse_attention == SUB_FUSE_REQUIRED)
         fail("attention with the scores in registers was required (SUB_OPT_FUSE_ATTENTION = 2) but the sizes, "
              "layouts or tensor alignment rule it out");
     return ok;
@@ -1064,12 +1075,14 @@ void forward(Handle& h, const FwdPtrs& t0) {
     }
     void* const* W = t.W; void* const* F = t.F;
     AttnArgs at;
-    const bool fused_attention = attention_fused(h, F, at);
+    // (registers: the backward pass runs its attention in registers and reads what this pass leaves for it)
+    const bool registers = attention_fused(h, F, at);
+    const bool fused_attention = registers && !forward_in_operators(h);
     if (h.fuse_epilogues && h.gemm[G_QKV_BIAS].ok && aligned16(W[BKQV]) && aligned16(F[KKQQVV])) {
         // projection + bias in one pass; WKKWQQWVV (the pre-bias copy) is not written.  The CUs its tiles
         // leave idle draw part of the attention's dropout bits, which depend on nothing but the seed.
         GemmSideJob side;
-        if (fused_attention && (h.side_jobs & 1)) {
+        if (fused_attention && (h.side_jobs & 1) && at.K % 128 == 0) {
             side.key = make_key(h, SUB_SITE_SOFTMAX, h.p_softmax);
             side.keep = at.keep; side.rows = (uint32_t)((long)at.H * at.B * at.J); side.nk = (uint32_t)at.K;
         }
@@ -1087,7 +1100,7 @@ void forward(Handle& h, const FwdPtrs& t0) {
         launch_mha_forward(at, (int)h.sz.n[dP], make_key(h, SUB_SITE_SOFTMAX, h.p_softmax), h.stream);
     }
     bool fused_scores = fused_attention;
-    if (!fused_attention && h.fuse_scores) {
+    if (!registers && h.fuse_scores) {
         ProfScope ps(h, "QKT+softmax");
         fused_scores = op_scores_softmax(h, QQ, KK, F[ALPHA], h.lf[ALPHA], F[ATTN_DROP_MASK],
                                          h.lf[ATTN_DROP_MASK], F[ATTN_DROP], h.lf[ATTN_DROP]);
@@ -1098,7 +1111,8 @@ void forward(Handle& h, const FwdPtrs& t0) {
         ProfScope ps(h, "softmax");
         op_softmax(h, F[BETA], h.lf[BETA], F[ALPHA], h.lf[ALPHA], F[ATTN_DROP_MASK], h.lf[ATTN_DROP_MASK],
                    F[ATTN_DROP], h.lf[ATTN_DROP], 1.0f, h.p_softmax, SUB_SITE_SOFTMAX, h.attn_mask,
-                   &h.l_attn_mask, h.gemm[G_QKT].alpha);
+                   &h.l_attn_mask, h.gemm[G_QKT].alpha, registers ? &at : nullptr);
+        h.mask_plan_built = false;          // the backward pass makes its plan from the mask as it is now
     }
     if (!fused_attention) run_gemm(h, G_GAMMA, VV, F[ATTN_DROP], F[GAMMA], "gamma");
     run_gemm(h, G_OUT, W[WO], F[GAMMA], F[ATT], "out");
@@ -1344,7 +1358,7 @@ void backward(Handle& h, const BwdPtrs& t0) {
         const Layout& lbias = h.lp[BKQV];
         attn_bias = lbias.has[dQ] && lbias.has[dH] && lbias.has[dP];
         const int P = (int)h.sz.n[dP], H = (int)h.sz.n[dH];
-        const int ntq = at.B * (at.J / 128), ntk = at.B * (at.K / 128);
+        const int ntq = at.B * ((at.J + 127) / 128), ntk = at.B * ((at.K + 127) / 128);
         half_t* dbias = (half_t*)DW[BKQV];
         auto finish = [&](float* ws, int ns, int ntc, half_t* o0, half_t* o1) {
             FinishJob job{ws, FinishArgs{{o0, o1, nullptr, nullptr}, 0, lbias.stride[dH], lbias.stride[dP], H}, ns, H,
@@ -1635,7 +1649,7 @@ int sub_attention_in_registers(void* handle, int* planned) {
         Handle& h = as_handle(handle);
         need_cfg(h);
         if (!planned) fail("sub_attention_in_registers: null result pointer");
-        *planned = attention_planned(h) ? 1 : 0;
+        *planned = attention_planned(h) && !forward_in_operators(h) ? 1 : 0;
     });
 }
 
@@ -1737,6 +1751,8 @@ void op_attention_args(Handle& h, int n_queries, int n_keys, const void* q, cons
                        const void* v, const char* l_kv, const void* out, const char* l_out, void* stats,
                        void* keep, const void* attn_mask, const char* l_attn_mask, float scale, AttnArgs& a) {
     if (n_queries <= 0 || n_keys <= 0) fail("attention: numbers of query and key positions must be positive");
+    // (the size of `keep` that these entry points promise is that of whole blocks)
+    if (n_queries % 128 || n_keys % 128) fail("attention: numbers of query and key positions must be multiples of 128");
     Sizes z = h.sz;
     z.n[dJ] = n_queries; z.n[dK] = n_keys;
     const Layout lq = make_layout(l_q, z), lkv = make_layout(l_kv, z), lo = make_layout(l_out, z);
@@ -1823,7 +1839,7 @@ int sub_set_attention_mask(void* handle, const void* attn_mask, const char* layo
         if (l.rank != 2 || !l.has[dJ] || !l.has[dK]) fail("sub_set_attention_mask: layout must be JK or KJ");
         h.attn_mask = attn_mask; h.l_attn_mask = l;
         const Sizes& z = h.sz;
-        if (z.n[dJ] % 128 == 0 && z.n[dK] % 128 == 0 && !h.mask_plan) {
+        if (mha_shape_ok(z.n[dH], z.n[dB], z.n[dJ], z.n[dK], z.n[dP]) && !h.mask_plan) {
             hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
             if (hipStreamIsCapturing(h.stream, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone)
                 fail("sub_set_attention_mask: allocates a small table, call it outside the graph capture");

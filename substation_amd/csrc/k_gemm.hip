@@ -81,28 +81,79 @@ __device__ __forceinline__ void side_block(const GemmArgs& g, unsigned sb, unsig
 }
 
 // ---------------------------------------------------------------------------
-// Scalar fallback: any strides, any sizes.  One thread per output element.
+// Any strides, any sizes: what the matrix-core kernels do not take (mostly rows that are not whole 16-byte words: the
+// score-sized products of sequence lengths that are not multiples of 8).  64 x 64 outputs per workgroup, 4 x 4 per
+// thread, operands converted into LDS 32 k at a time; every output is one fp32 chain of fused multiply-adds in the
+// order of k.  (One thread per output, straight from memory, before: 750 us for the scores of B=8 L=197 H=12, 0.5 GFLOP,
+// bound by the latency of that chain's single-element loads.)
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_gemm_scalar(GemmArgs g, long total) {
-    long idx = (long)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= total) return;
-    int n = (int)(idx % g.N); long r = idx / g.N;
-    int m = (int)(r % g.M); long b = r / g.M;
-    long b2 = b % g.nb2; long t = b / g.nb2;
-    long b1 = t % g.nb1; long b0 = t / g.nb1;
-    const half_t* a = g.A + b0 * g.sAb[0] + b1 * g.sAb[1] + b2 * g.sAb[2] + (long)m * g.sAM;
-    const half_t* bp = g.B + b0 * g.sBb[0] + b1 * g.sBb[1] + b2 * g.sBb[2] + (long)n * g.sBN;
-    float acc = 0.f;
-    for (int k0 = 0; k0 < g.K0; ++k0) {
-        const half_t* a0 = a + (long)k0 * g.sAK0;
-        const half_t* b0p = bp + (long)k0 * g.sBK0;
-        for (int k = 0; k < g.K1; ++k) acc += (float)a0[(long)k * g.sAK1] * (float)b0p[(long)k * g.sBK1];
+constexpr int FB = 64, FK = 32, FPITCH = FB + 4;
+
+// One operand's 64 x 32 elements into LDS as [k][row].  vec: whole 16-byte words along k.
+__device__ __forceinline__ void fma_tile(float (*dst)[FPITCH], const half_t* p, long s_row, long s_k, int rows, int ks, bool vec,
+                                         int tid) {
+    if (vec) {
+        const int row = tid >> 2, k = (tid & 3) * 8;
+        h8 v = (h8)(half_t)0.0f;
+        if (row < rows && k < ks) v = *reinterpret_cast<const h8*>(p + (long)row * s_row + k);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) dst[k + i][row] = (float)v[i];
+        return;
     }
-    half_t out = (half_t)(acc * g.alpha);
-    if (g.bias)     // same two roundings as the product followed by a separate add
-        out = (half_t)((float)out + (float)g.bias[b0 * g.sbb[0] + b1 * g.sbb[1] + b2 * g.sbb[2] +
-                                                  (long)m * g.sbM + (long)n * g.sbN]);
-    g.C[b0 * g.sCb[0] + b1 * g.sCb[1] + b2 * g.sCb[2] + (long)m * g.sCM + (long)n * g.sCN] = out;
+    half_t v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int e = tid + i * 256, row = s_k == 1 ? e / FK : e % FB, k = s_k == 1 ? e % FK : e / FB;
+        v[i] = row < rows && k < ks ? p[(long)row * s_row + (long)k * s_k] : (half_t)0.0f;
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int e = tid + i * 256, row = s_k == 1 ? e / FK : e % FB, k = s_k == 1 ? e % FK : e / FB;
+        dst[k][row] = (float)v[i];
+    }
+}
+
+__global__ __launch_bounds__(256) void k_gemm_fma(GemmArgs g, bool vec_a, bool vec_b) {
+    __shared__ __attribute__((aligned(16))) float ta[FK][FPITCH], tb[FK][FPITCH];
+    const int tid = threadIdx.x, tm = (tid >> 4) * 4, tn = (tid & 15) * 4;
+    const unsigned tiles_m = (g.M + FB - 1) / FB, tiles_n = (g.N + FB - 1) / FB;
+    unsigned id = blockIdx.x;
+    const unsigned n0 = id % tiles_n * FB; id /= tiles_n;
+    const unsigned m0 = id % tiles_m * FB; id /= tiles_m;
+    const long b2 = id % g.nb2; id /= g.nb2;
+    const long b1 = id % g.nb1, b0 = id / g.nb1;
+    const half_t* a = g.A + b0 * g.sAb[0] + b1 * g.sAb[1] + b2 * g.sAb[2] + (long)m0 * g.sAM;
+    const half_t* b = g.B + b0 * g.sBb[0] + b1 * g.sBb[1] + b2 * g.sBb[2] + (long)n0 * g.sBN;
+    float acc[4][4] = {};
+    for (int k0 = 0; k0 < g.K0; ++k0)
+        for (int k = 0; k < g.K1; k += FK) {
+            const int ks = min(FK, g.K1 - k);
+            __syncthreads();
+            fma_tile(ta, a + (long)k0 * g.sAK0 + (long)k * g.sAK1, g.sAM, g.sAK1, g.M - (int)m0, ks, vec_a, tid);
+            fma_tile(tb, b + (long)k0 * g.sBK0 + (long)k * g.sBK1, g.sBN, g.sBK1, g.N - (int)n0, ks, vec_b, tid);
+            __syncthreads();
+#pragma unroll 8
+            for (int i = 0; i < ks; ++i) {
+                const float4 x = *reinterpret_cast<const float4*>(&ta[i][tm]), y = *reinterpret_cast<const float4*>(&tb[i][tn]);
+                const float xv[4] = {x.x, x.y, x.z, x.w}, yv[4] = {y.x, y.y, y.z, y.w};
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) acc[r][c] = __builtin_fmaf(xv[r], yv[c], acc[r][c]);
+            }
+        }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const int m = (int)m0 + tm + r, n = (int)n0 + tn + c;
+            if (m >= g.M || n >= g.N) continue;
+            half_t out = (half_t)(acc[r][c] * g.alpha);
+            if (g.bias)     // same two roundings as the product followed by a separate add
+                out = (half_t)((float)out + (float)g.bias[b0 * g.sbb[0] + b1 * g.sbb[1] + b2 * g.sbb[2] +
+                                                          (long)m * g.sbM + (long)n * g.sbN]);
+            g.C[b0 * g.sCb[0] + b1 * g.sCb[1] + b2 * g.sCb[2] + (long)m * g.sCM + (long)n * g.sCN] = out;
+        }
 }
 
 // ---------------------------------------------------------------------------
@@ -1483,10 +1534,13 @@ void launch_gemm(const GemmShape& s, const half_t* A, const half_t* B, half_t* C
         else launch_mfma<2, 2, true>(c.a, akc, bkc, batch, dma, st);
     } else {
         if (ep.relu_dropout || ep.gate) fail("gemm: the ReLU-dropout epilogue needs the MFMA kernel");
-        long total = batch * (long)c.a.M * c.a.N;
-        long blocks = (total + 255) / 256;
+        const long blocks = batch * ((c.a.M + FB - 1) / FB) * ((c.a.N + FB - 1) / FB);
         if (blocks > 0x7fffffffL) fail("gemm: problem too large for the scalar kernel");
-        hipLaunchKernelGGL(k_gemm_scalar, dim3((unsigned)blocks), dim3(256), 0, st, c.a, total);
+        auto words = [&](const half_t* p, long s_row, long s_k, long s_k0, const long (&sb)[3]) {
+            return s_k == 1 && al16(p) && mult8(s_row) && mult8(c.a.K1) && mult8(s_k0) && mult8(sb[0]) && mult8(sb[1]) && mult8(sb[2]);
+        };
+        hipLaunchKernelGGL(k_gemm_fma, dim3((unsigned)blocks), dim3(256), 0, st, c.a,
+                           words(c.a.A, c.a.sAM, c.a.sAK1, c.a.sAK0, c.a.sAb), words(c.a.B, c.a.sBN, c.a.sBK1, c.a.sBK0, c.a.sBb));
     }
     check_launch("gemm");
 }

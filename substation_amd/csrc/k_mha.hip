@@ -22,6 +22,8 @@
 //   element i of step s  <->  index (2s + i/4)*8 + 4*(lane/32) + i%4 ;
 // the A operand is gathered in the same order from an LDS tile with the
 // transposing read, so no score ever moves between lanes.
+#include <type_traits>
+
 #include "sub_ops.hpp"
 
 namespace sub {
@@ -72,15 +74,16 @@ __device__ __forceinline__ void row_frags_lds(const half_t* tile, int l32, int h
         f[ks] = *reinterpret_cast<const h8*>(tile + Geo<P>::at(l32, 2 * ks + hi));
 }
 
-// A tile of 32 positions x P features: global -> registers -> LDS, all threads.
-template <int P>
-__device__ __forceinline__ void tile_fetch(const AttnSide& t, unsigned h, unsigned b, unsigned pos0, int tid,
+// A tile of 32 positions x P features: global -> registers -> LDS, all threads.  RAGGED: positions from `limit` on
+// read the last one that there is (their scores are taken out where they would count).
+template <int P, bool RAGGED>
+__device__ __forceinline__ void tile_fetch(const AttnSide& t, unsigned h, unsigned b, unsigned pos0, unsigned limit, int tid,
                                            h8 (&r)[Geo<P>::VL]) {
 #pragma unroll
     for (int i = 0; i < Geo<P>::VL; ++i) {
         const int id = tid + i * 256, row = id / (P / 8), c = id % (P / 8);
-        r[i] = *reinterpret_cast<const h8*>(t.p + (long)h * t.sh + (long)b * t.sb + (long)(pos0 + row) * t.sr +
-                                            c * 8);
+        const unsigned pos = RAGGED ? min(pos0 + row, limit - 1) : pos0 + row;
+        r[i] = *reinterpret_cast<const h8*>(t.p + (long)h * t.sh + (long)b * t.sb + (long)pos * t.sr + c * 8);
     }
 }
 template <int P>
@@ -140,6 +143,16 @@ __device__ __forceinline__ float keep_if(float x, uint32_t bits, int pos) {
     return __int_as_float(__float_as_int(x) & __builtin_amdgcn_sbfe((int)bits, pos, 1));
 }
 
+// Scores of positions from `limit` on (the tile starts at tile0, register v of a lane holds position reg_pos(v, hi) of
+// it) vanish from everything that is formed from them.
+__device__ __forceinline__ void drop_past_end(f16v& s, unsigned tile0, unsigned limit, int hi) {
+#pragma unroll
+    for (int v = 0; v < 16; ++v) s[v] = tile0 + reg_pos(v, hi) < limit ? s[v] : -INFINITY;
+}
+
+// Words of keep bits per score row: one per 32 keys, in whole groups of four (mha_keep_pitch).
+__device__ __forceinline__ unsigned keep_pitch(unsigned K) { return (K + QB - 1) / QB * 4; }
+
 // Sums over the 128 positions of a workgroup of the rows store_rows() writes
 // (same rounding), one value per feature: 32 lanes hold the positions of a
 // wave, the four waves meet in LDS (`red`: 4 * P floats, free to use).
@@ -184,11 +197,16 @@ __device__ __forceinline__ void column_sums(const f16v (&acc)[P / 32], float sca
 // also wait for them.
 struct MaskRegs { h4 q[4]; };
 
-template <bool QUERY_LANES>
+template <bool QUERY_LANES, bool RAGGED>
 __device__ __forceinline__ void load_mask(const AttnArgs& a, unsigned lane_pos, unsigned tile0, int hi, MaskRegs& mk) {
     const long lane_stride = QUERY_LANES ? a.am_sj : a.am_sk, reg_stride = QUERY_LANES ? a.am_sk : a.am_sj;
     const half_t* m = a.amask + (long)lane_pos * lane_stride + (long)tile0 * reg_stride;
-    if (reg_stride == 1) {
+    const unsigned limit = QUERY_LANES ? a.K : a.J;
+    if (RAGGED && (reg_stride != 1 || (lane_stride & 3) != 0 || tile0 + 32 > limit)) {
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+            mk.q[v >> 2][v & 3] = m[(long)(min(tile0 + reg_pos(v, hi), limit - 1) - tile0) * reg_stride];
+    } else if (reg_stride == 1) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) mk.q[q] = *reinterpret_cast<const h4*>(m + q * 8 + hi * 4);
     } else {
@@ -219,13 +237,14 @@ constexpr uint32_t kAllDead = BLOCK_DEAD * 0x55u << 16;
 constexpr int kListPad = 4;       // the count and three entries of padding
 
 // One wave per 32x32 block of the mask.
-__global__ __launch_bounds__(64) void k_mha_mask_classes(const half_t* mask, long sj, long sk, int K, uint8_t* cls) {
-    const int lane = threadIdx.x, nkb = K / 32;
+__global__ __launch_bounds__(64) void k_mha_mask_classes(const half_t* mask, long sj, long sk, int J, int K, uint8_t* cls) {
+    const int lane = threadIdx.x, nkb = (K + 31) / 32;
     const int qb = blockIdx.x / nkb, kb = blockIdx.x % nkb;
-    const half_t* p = mask + (long)(qb * 32 + (lane & 31)) * sj + (long)(kb * 32 + (lane >> 5) * 16) * sk;
+    // positions past the end stand for the last one that there is: they change nobody's class
+    const half_t* p = mask + (long)min(qb * 32 + (lane & 31), J - 1) * sj;
     bool dead = true, clear = true;
     for (int i = 0; i < 16; ++i) {
-        const float x = (float)p[(long)i * sk];
+        const float x = (float)p[(long)min(kb * 32 + (lane >> 5) * 16 + i, K - 1) * sk];
         dead = dead && (x == -INFINITY);
         clear = clear && (x == 0.f);
     }
@@ -234,12 +253,12 @@ __global__ __launch_bounds__(64) void k_mha_mask_classes(const half_t* mask, lon
     if (lane == 0) cls[blockIdx.x] = all_dead ? BLOCK_DEAD : all_clear ? BLOCK_CLEAR : BLOCK_MIXED;
 }
 
-// One wave per list row: blocks 0 .. J/128-1 build the key-tile lists of the query
+// One wave per list row: the first ceil(J/128) blocks build the key-tile lists of the query
 // blocks, the others the query-tile lists of the key blocks.
 __global__ __launch_bounds__(64) void k_mha_mask_lists(const uint8_t* cls, int J, int K, uint32_t* qlist, uint32_t* klist) {
-    const int lane = threadIdx.x, nqb = J / 32, nkb = K / 32;
-    const bool by_query = (int)blockIdx.x < J / QB;
-    const int blk = by_query ? blockIdx.x : blockIdx.x - J / QB;
+    const int lane = threadIdx.x, nqb = (J + 31) / 32, nkb = (K + 31) / 32, nblk = (J + QB - 1) / QB;
+    const bool by_query = (int)blockIdx.x < nblk;
+    const int blk = by_query ? blockIdx.x : blockIdx.x - nblk;
     const int ntiles = by_query ? nkb : nqb;
     uint32_t* row = (by_query ? qlist : klist) + (size_t)blk * (ntiles + kListPad);
     unsigned count = 0;
@@ -249,7 +268,10 @@ __global__ __launch_bounds__(64) void k_mha_mask_lists(const uint8_t* cls, int J
         if (t < ntiles) {
             e = (uint32_t)t;
             for (int w = 0; w < 4; ++w) {
-                const uint32_t c = by_query ? cls[(size_t)(blk * 4 + w) * nkb + t] : cls[(size_t)t * nkb + blk * 4 + w];
+                // (a wave whose 32 positions all lie past the end has nothing to do)
+                uint32_t c = BLOCK_DEAD;
+                if (blk * 4 + w < (by_query ? nqb : nkb))
+                    c = by_query ? cls[(size_t)(blk * 4 + w) * nkb + t] : cls[(size_t)t * nkb + blk * 4 + w];
                 e |= c << (16 + 2 * w);
             }
         }
@@ -309,22 +331,31 @@ constexpr int RING = 3;
 __device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }   // vmcnt(0)
 
 // ---------------------------------------------------------------------------
-// forward.  grid = H * B * (J / 128); wave = 32 queries.
+// forward.  grid = H * B * ceil(J / 128); wave = 32 queries.
+//
+// RAGGED: J or K is not a multiple of 128.  Loads of positions past the end are clamped, the scores of the last key
+// tile's missing keys are set to -inf, and rows past the end are not written.  Without it such lengths took the operators
+// one by one, with the score-sized tensors in memory and, for lengths that are not multiples of 8, products
+// through the scalar kernel: the layer's forward and backward at B=13 L=201 E=768 took 3990 us.
 // ---------------------------------------------------------------------------
-template <int P, bool MASKED>
+template <int P, bool MASKED, bool RAGGED>
 __global__ __launch_bounds__(256) void k_mha_fwd(AttnArgs a, PhiloxKey key_) {
     using G = Geo<P>;
     __shared__ __attribute__((aligned(16))) half_t kt[RING][G::TILE];
     __shared__ __attribute__((aligned(16))) half_t vt[RING][G::TILE];
     const PhiloxKey key = resolved(key_);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, hi = lane >> 5;
-    const unsigned qblocks = a.J / QB;
+    const unsigned qblocks = RAGGED ? (a.J + QB - 1) / QB : a.J / QB;
     const unsigned lb = logical_block();
-    const unsigned nt = a.K / 32;
+    const unsigned nt = RAGGED ? (a.K + 31) / 32 : a.K / 32, pitch = RAGGED ? keep_pitch(a.K) : nt;
     unsigned qb = lb % qblocks, hb = lb / qblocks;
     if (MASKED) masked_order(a.qlist, qblocks, nt, a.H * a.B, lb, qb, hb);
     const unsigned b = hb % a.B, h = hb / a.B;
-    const unsigned j = qb * QB + wave * 32 + l32;                    // this lane's query
+    const unsigned j_ = qb * QB + wave * 32 + l32;                   // this lane's query
+    const bool mine_ = !RAGGED || j_ < (unsigned)a.J;                // (RAGGED: lanes past the end follow the last query)
+    const unsigned j = RAGGED ? min(j_, (unsigned)a.J - 1) : j_;
+    // waves whose queries all lie past the end only help with the tiles
+    const bool working = !RAGGED || __builtin_amdgcn_readfirstlane((int)(qb * QB + wave * 32)) < a.J;
     const unsigned row = (h * a.B + b) * a.J + j;                    // its score row
     const float c = a.alpha * LOG2E;
     // the key tiles to walk: all of them, or those a mask leaves for these 128 queries
@@ -335,10 +366,10 @@ __global__ __launch_bounds__(256) void k_mha_fwd(AttnArgs a, PhiloxKey key_) {
     h8 fq[G::NKS], fk[G::NKS], kr[G::VL], vr[G::VL];
     {   // the first two tiles and the query rows: all loads in flight together
         h8 kr1[G::VL], vr1[G::VL];
-        tile_fetch<P>(a.k, h, b, entry_tile(e0) * 32, tid, kr);
-        tile_fetch<P>(a.v, h, b, entry_tile(e0) * 32, tid, vr);
-        tile_fetch<P>(a.k, h, b, entry_tile(e1) * 32, tid, kr1);
-        tile_fetch<P>(a.v, h, b, entry_tile(e1) * 32, tid, vr1);
+        tile_fetch<P, RAGGED>(a.k, h, b, entry_tile(e0) * 32, a.K, tid, kr);
+        tile_fetch<P, RAGGED>(a.v, h, b, entry_tile(e0) * 32, a.K, tid, vr);
+        tile_fetch<P, RAGGED>(a.k, h, b, entry_tile(e1) * 32, a.K, tid, kr1);
+        tile_fetch<P, RAGGED>(a.v, h, b, entry_tile(e1) * 32, a.K, tid, vr1);
         row_frags<P>(a.q, h, b, j, hi, fq);
         tile_put<P>(kt[0], tid, kr);
         tile_put<P>(vt[0], tid, vr);
@@ -357,11 +388,16 @@ __global__ __launch_bounds__(256) void k_mha_fwd(AttnArgs a, PhiloxKey key_) {
     const float slack = RESCALE_SLACK / c;
     int cur = 0, nxt = 1, nn = 2;
     MaskRegs mk = {};
-    if (MASKED && n > 0 && entry_class(e0, wave) != BLOCK_CLEAR) load_mask<true>(a, j, entry_tile(e0) * 32, hi, mk);
+    if (MASKED && n > 0 && entry_class(e0, wave) != BLOCK_CLEAR) load_mask<true, RAGGED>(a, j, entry_tile(e0) * 32, hi, mk);
     // keep words drawn ahead of this launch are fetched a tile early: at the place of their
     // use the load would stand between the scores and their exponentials
     uint32_t word_ahead = 0;
-    if (key.thr && n > 0 && entry_tile(e0) < a.keep_tiles_ready) word_ahead = a.keep[(size_t)row * nt + entry_tile(e0)];
+    if (key.thr && n > 0 && entry_tile(e0) < a.keep_tiles_ready) word_ahead = a.keep[(size_t)row * pitch + entry_tile(e0)];
+    // RAGGED: a score row starts anywhere in a Philox group of 8 when K is not a multiple of 8.  The bits of a tile are
+    // then cut out of five groups, the first of which the tile before has drawn as its last (`carry`).
+    const uint64_t e_row = (uint64_t)row * (unsigned)a.K;
+    const uint32_t shift = (uint32_t)e_row & 7u;
+    uint32_t carry = 0, carry_tile = ~0u;
     wait_loads();
 
     for (unsigned i = 0; i < n; ++i) {
@@ -371,16 +407,17 @@ __global__ __launch_bounds__(256) void k_mha_fwd(AttnArgs a, PhiloxKey key_) {
         const bool fetch = i + 2 < n;
         const uint32_t word_ready = word_ahead;
         if (key.thr && i + 1 < n && entry_tile(e1) < a.keep_tiles_ready)
-            word_ahead = a.keep[(size_t)row * nt + entry_tile(e1)];
+            word_ahead = a.keep[(size_t)row * pitch + entry_tile(e1)];
         if (fetch) {
-            tile_fetch<P>(a.k, h, b, entry_tile(e2) * 32, tid, kr);
-            tile_fetch<P>(a.v, h, b, entry_tile(e2) * 32, tid, vr);
+            tile_fetch<P, RAGGED>(a.k, h, b, entry_tile(e2) * 32, a.K, tid, kr);
+            tile_fetch<P, RAGGED>(a.v, h, b, entry_tile(e2) * 32, a.K, tid, vr);
         }
+        if (working) {
         f16v s;
 #pragma unroll
         for (int v = 0; v < 16; ++v) s[v] = 0.f;
         if (from_mask) start_from_mask(mk, s);
-        if (MASKED && i + 1 < n && entry_class(e1, wave) != BLOCK_CLEAR) load_mask<true>(a, j, entry_tile(e1) * 32, hi, mk);
+        if (MASKED && i + 1 < n && entry_class(e1, wave) != BLOCK_CLEAR) load_mask<true, RAGGED>(a, j, entry_tile(e1) * 32, hi, mk);
 #pragma unroll
         for (int ks = 0; ks < G::NKS; ++ks) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(fk[ks], fq[ks], s, 0, 0, 0);
         // fragments for the second product of this tile and the first of the next
@@ -390,12 +427,21 @@ __global__ __launch_bounds__(256) void k_mha_fwd(AttnArgs a, PhiloxKey key_) {
 #pragma unroll
             for (int pt = 0; pt < G::NPT; ++pt) va[st][pt] = tr_frag<P>(vt[cur], pt * 32, st, lane);
         row_frags_lds<P>(kt[nxt], l32, hi, fk);
+        if (RAGGED && t * 32 + 32 > (unsigned)a.K) drop_past_end(s, t * 32, a.K, hi);
 
         // keep bits of the 32 scores (this query, keys of tile t): each half of the
         // wave draws two of the four groups of 8 and the halves trade them
         uint32_t word = 0xffffffffu;
         if (key.thr && t < a.keep_tiles_ready) {
             word = word_ready;                                       // drawn ahead of this launch
+        } else if (RAGGED && key.thr) {
+            const uint64_t g0 = (e_row >> 3) + 4 * t;
+            if (carry_tile != t) carry = keep8(philox_group_dev(key, g0), key.thr);
+            const uint32_t mine = keep8(philox_group_dev(key, g0 + 1 + 2 * hi), key.thr) |
+                                  (keep8(philox_group_dev(key, g0 + 2 + 2 * hi), key.thr) << 8);
+            const auto both = __builtin_amdgcn_permlane32_swap(mine, mine, false, false);
+            word = __builtin_amdgcn_alignbit(both[1] >> 8, carry | (both[0] << 8) | (both[1] << 24), shift);
+            carry = both[1] >> 8; carry_tile = t + 1;
         } else if (key.thr) {
             const uint64_t g0 = (uint64_t)row * (a.K / 8) + 4 * t + 2 * hi;
             const uint32_t mine = keep8(philox_group_dev(key, g0), key.thr) |
@@ -405,7 +451,7 @@ __global__ __launch_bounds__(256) void k_mha_fwd(AttnArgs a, PhiloxKey key_) {
             const auto both = __builtin_amdgcn_permlane32_swap(mine, mine, false, false);
             word = both[0] | (both[1] << 16);
         }
-        if (hi == 0 && t >= a.keep_tiles_ready) a.keep[(size_t)row * nt + t] = word;
+        if (hi == 0 && mine_ && t >= a.keep_tiles_ready) a.keep[(size_t)row * pitch + t] = word;
         const uint32_t nib = word >> (hi * 4);                       // bit reg_pos(v, 0) of nib = keep of register v
 
         // Running softmax with a reference value per query that trails the running
@@ -463,6 +509,7 @@ __global__ __launch_bounds__(256) void k_mha_fwd(AttnArgs a, PhiloxKey key_) {
 #pragma unroll
             for (int pt = 0; pt < G::NPT; ++pt)
                 o[pt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[st][pt], pb[st], o[pt], 0, 0, 0);
+        }
         if (fetch) {
             tile_put<P>(kt[nn], tid, kr);
             tile_put<P>(vt[nn], tid, vr);
@@ -472,14 +519,15 @@ __global__ __launch_bounds__(256) void k_mha_fwd(AttnArgs a, PhiloxKey key_) {
         e0 = e1; e1 = e2; e2 = e3;
     }
     const float l_tot = l_run + __shfl_xor(l_run, 32);
+    if (!mine_) return;
     store_rows<P>(a.o, h, b, j, hi, o, 1.0f / l_tot);
     if (hi == 0) a.lse[row] = m_ref * c + __builtin_amdgcn_logf(l_tot);
 }
 
 // ---------------------------------------------------------------------------
-// backward, dQ.  grid = H * B * (J / 128); wave = 32 queries.
+// backward, dQ.  grid = H * B * ceil(J / 128); wave = 32 queries.
 // ---------------------------------------------------------------------------
-template <int P, bool MASKED>
+template <int P, bool MASKED, bool RAGGED>
 __global__ __launch_bounds__(256, !MASKED ? (P == 128 ? 2 : 3) : 1) void k_mha_bwd_dq(AttnArgs a) {
     using G = Geo<P>;
     // Head size 128: with the key and value fragments of a whole tile in registers a tile ahead the kernel
@@ -489,13 +537,16 @@ __global__ __launch_bounds__(256, !MASKED ? (P == 128 ? 2 : 3) : 1) void k_mha_b
     __shared__ __attribute__((aligned(16))) half_t kt[RING][G::TILE];
     __shared__ __attribute__((aligned(16))) half_t vt[RING][G::TILE];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, hi = lane >> 5;
-    const unsigned qblocks = a.J / QB;
+    const unsigned qblocks = RAGGED ? (a.J + QB - 1) / QB : a.J / QB;
     const unsigned lb = logical_block();
-    const unsigned nt = a.K / 32;
+    const unsigned nt = RAGGED ? (a.K + 31) / 32 : a.K / 32, pitch = RAGGED ? keep_pitch(a.K) : nt;
     unsigned qb = lb % qblocks, hb = lb / qblocks;
     if (MASKED) masked_order(a.qlist, qblocks, nt, a.H * a.B, lb, qb, hb);
     const unsigned b = hb % a.B, h = hb / a.B;
-    const unsigned j = qb * QB + wave * 32 + l32;
+    const unsigned j_ = qb * QB + wave * 32 + l32;
+    const bool mine_ = !RAGGED || j_ < (unsigned)a.J;
+    const unsigned j = RAGGED ? min(j_, (unsigned)a.J - 1) : j_;
+    const bool working = !RAGGED || __builtin_amdgcn_readfirstlane((int)(qb * QB + wave * 32)) < a.J;
     const unsigned row = (h * a.B + b) * a.J + j;
     const float c = a.alpha * LOG2E;
     const uint32_t* live = (MASKED && a.qlist) ? a.qlist + (size_t)qb * (nt + kListPad) : nullptr;
@@ -508,15 +559,15 @@ __global__ __launch_bounds__(256, !MASKED ? (P == 128 ? 2 : 3) : 1) void k_mha_b
     {   // the first two tiles, the rows of this lane's query and its statistics: all
         // loads in flight together
         h8 kr1[G::VL], vr1[G::VL], fo[G::NKS];
-        tile_fetch<P>(a.k, h, b, entry_tile(e0) * 32, tid, kr);
-        tile_fetch<P>(a.v, h, b, entry_tile(e0) * 32, tid, vr);
-        tile_fetch<P>(a.k, h, b, entry_tile(e1) * 32, tid, kr1);
-        tile_fetch<P>(a.v, h, b, entry_tile(e1) * 32, tid, vr1);
+        tile_fetch<P, RAGGED>(a.k, h, b, entry_tile(e0) * 32, a.K, tid, kr);
+        tile_fetch<P, RAGGED>(a.v, h, b, entry_tile(e0) * 32, a.K, tid, vr);
+        tile_fetch<P, RAGGED>(a.k, h, b, entry_tile(e1) * 32, a.K, tid, kr1);
+        tile_fetch<P, RAGGED>(a.v, h, b, entry_tile(e1) * 32, a.K, tid, vr1);
         row_frags<P>(a.q, h, b, j, hi, fq);
         row_frags<P>(a.d_o, h, b, j, hi, fdo);
         row_frags<P>(a.o, h, b, j, hi, fo);
         lse = a.lse[row];
-        word = a.keep[(size_t)row * nt + entry_tile(e0)];
+        word = a.keep[(size_t)row * pitch + entry_tile(e0)];
         tile_put<P>(kt[0], tid, kr);
         tile_put<P>(vt[0], tid, vr);
         tile_put<P>(kt[1], tid, kr1);
@@ -527,7 +578,7 @@ __global__ __launch_bounds__(256, !MASKED ? (P == 128 ? 2 : 3) : 1) void k_mha_b
 #pragma unroll
             for (int i = 0; i < 8; ++i) part += (float)fdo[ks][i] * (float)fo[ks][i];
         dsum = part + __shfl_xor(part, 32);
-        if (hi == 0) a.dsum[row] = dsum;
+        if (hi == 0 && mine_) a.dsum[row] = dsum;
     }
     __syncthreads();
     if constexpr (!JIT) {
@@ -542,7 +593,7 @@ __global__ __launch_bounds__(256, !MASKED ? (P == 128 ? 2 : 3) : 1) void k_mha_b
         for (int v = 0; v < 16; ++v) dq[pt][v] = 0.f;
     int cur = 0, nxt = 1, nn = 2;
     MaskRegs mk = {};
-    if (MASKED && n > 0 && entry_class(e0, wave) != BLOCK_CLEAR) load_mask<true>(a, j, entry_tile(e0) * 32, hi, mk);
+    if (MASKED && n > 0 && entry_class(e0, wave) != BLOCK_CLEAR) load_mask<true, RAGGED>(a, j, entry_tile(e0) * 32, hi, mk);
     wait_loads();
 
     for (unsigned i = 0; i < n; ++i) {
@@ -550,15 +601,16 @@ __global__ __launch_bounds__(256, !MASKED ? (P == 128 ? 2 : 3) : 1) void k_mha_b
         const bool from_mask = MASKED && entry_class(e0, wave) != BLOCK_CLEAR;
         const bool fetch = i + 2 < n;
         if (fetch) {
-            tile_fetch<P>(a.k, h, b, entry_tile(e2) * 32, tid, kr);
-            tile_fetch<P>(a.v, h, b, entry_tile(e2) * 32, tid, vr);
+            tile_fetch<P, RAGGED>(a.k, h, b, entry_tile(e2) * 32, a.K, tid, kr);
+            tile_fetch<P, RAGGED>(a.v, h, b, entry_tile(e2) * 32, a.K, tid, vr);
         }
-        const uint32_t wordn = i + 1 < n ? a.keep[(size_t)row * nt + entry_tile(e1)] : 0u;
+        const uint32_t wordn = i + 1 < n ? a.keep[(size_t)row * pitch + entry_tile(e1)] : 0u;
+        if (working) {
         f16v s, dp;
 #pragma unroll
         for (int v = 0; v < 16; ++v) { s[v] = 0.f; dp[v] = 0.f; }
         if (from_mask) start_from_mask(mk, s);
-        if (MASKED && i + 1 < n && entry_class(e1, wave) != BLOCK_CLEAR) load_mask<true>(a, j, entry_tile(e1) * 32, hi, mk);
+        if (MASKED && i + 1 < n && entry_class(e1, wave) != BLOCK_CLEAR) load_mask<true, RAGGED>(a, j, entry_tile(e1) * 32, hi, mk);
         if constexpr (JIT) {
             h8 ck[2], cv[2];
             ck[0] = *reinterpret_cast<const h8*>(kt[cur] + G::at(l32, hi));
@@ -587,6 +639,7 @@ __global__ __launch_bounds__(256, !MASKED ? (P == 128 ? 2 : 3) : 1) void k_mha_b
             row_frags_lds<P>(kt[nxt], l32, hi, fk);
             row_frags_lds<P>(vt[nxt], l32, hi, fv);
         }
+        if (RAGGED && entry_tile(e0) * 32 + 32 > (unsigned)a.K) drop_past_end(s, entry_tile(e0) * 32, a.K, hi);
         const uint32_t nib = word >> (hi * 4);
         // stage by stage over the 16 scores of the lane, so that consecutive
         // instructions do not depend on one another
@@ -608,6 +661,7 @@ __global__ __launch_bounds__(256, !MASKED ? (P == 128 ? 2 : 3) : 1) void k_mha_b
 #pragma unroll
             for (int pt = 0; pt < G::NPT; ++pt)
                 dq[pt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka[st][pt], ds[st], dq[pt], 0, 0, 0);
+        }
         if (fetch) {
             tile_put<P>(kt[nn], tid, kr);
             tile_put<P>(vt[nn], tid, vr);
@@ -617,14 +671,20 @@ __global__ __launch_bounds__(256, !MASKED ? (P == 128 ? 2 : 3) : 1) void k_mha_b
         const int x = cur; cur = nxt; nxt = nn; nn = x;
         e0 = e1; e1 = e2; e2 = e3;
     }
-    store_rows<P>(a.dq, h, b, j, hi, dq, a.alpha);
+    if (mine_) store_rows<P>(a.dq, h, b, j, hi, dq, a.alpha);
+    if (RAGGED && !mine_) {       // nothing to the column sums
+#pragma unroll
+        for (int pt = 0; pt < G::NPT; ++pt)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) dq[pt][v] = 0.f;
+    }
     if (a.bias_q)
         column_sums<P>(dq, a.alpha, reinterpret_cast<float*>(&kt[0][0]),
                        a.bias_q + ((size_t)h * (a.B * qblocks) + b * qblocks + qb) * P, tid);
 }
 
 // ---------------------------------------------------------------------------
-// backward, dK and dV.  grid = H * B * (K / 128); wave = 32 keys.
+// backward, dK and dV.  grid = H * B * ceil(K / 128); wave = 32 keys.
 // Per tile of 32 queries the workgroup stages Q, dO, the two row statistics and
 // the keep words of its four key tiles in LDS.
 // ---------------------------------------------------------------------------
@@ -637,18 +697,21 @@ struct KvStage {
     uint32_t keep[4][32];         // [wave's key tile][query]
 };
 
-template <int P, bool MASKED>
+template <int P, bool MASKED, bool RAGGED>
 __global__ __launch_bounds__(256, (P == 64 && MASKED) ? 2 : 1) void k_mha_bwd_dkv(AttnArgs a) {
     using G = Geo<P>;
     __shared__ __attribute__((aligned(16))) KvStage<P> stage[RING];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, hi = lane >> 5;
-    const unsigned kblocks = a.K / QB;
+    const unsigned kblocks = RAGGED ? (a.K + QB - 1) / QB : a.K / QB;
     const unsigned lb = logical_block();
-    const unsigned nq = a.J / 32, nkt = a.K / 32;
+    const unsigned nq = RAGGED ? (a.J + 31) / 32 : a.J / 32, nkt = RAGGED ? keep_pitch(a.K) : a.K / 32;
     unsigned kb = lb % kblocks, hb = lb / kblocks;
     if (MASKED) masked_order(a.klist, kblocks, nq, a.H * a.B, lb, kb, hb);
     const unsigned b = hb % a.B, h = hb / a.B;
-    const unsigned kpos = kb * QB + wave * 32 + l32;                 // this lane's key
+    const unsigned kpos_ = kb * QB + wave * 32 + l32;                // this lane's key
+    const bool mine_ = !RAGGED || kpos_ < (unsigned)a.K;
+    const unsigned kpos = RAGGED ? min(kpos_, (unsigned)a.K - 1) : kpos_;
+    const bool working = !RAGGED || __builtin_amdgcn_readfirstlane((int)(kb * QB + wave * 32)) < a.K;
     const unsigned row0 = (h * a.B + b) * a.J;                       // score row of query 0
     const float c = a.alpha * LOG2E;
     // the query tiles to walk: all of them, or those a mask leaves for these 128 keys
@@ -663,10 +726,12 @@ __global__ __launch_bounds__(256, (P == 64 && MASKED) ? 2 : 1) void k_mha_bwd_dk
         uint4 kw;
     };
     auto fetch = [&](unsigned qt, InFlight& f) {
-        tile_fetch<P>(a.q, h, b, qt * 32, tid, f.q);
-        tile_fetch<P>(a.d_o, h, b, qt * 32, tid, f.d_o);
-        const unsigned r = row0 + qt * 32 + (tid & 31);
-        if (tid < 32) f.stat = a.lse[r];
+        tile_fetch<P, RAGGED>(a.q, h, b, qt * 32, a.J, tid, f.q);
+        tile_fetch<P, RAGGED>(a.d_o, h, b, qt * 32, a.J, tid, f.d_o);
+        const unsigned q = qt * 32 + (tid & 31);
+        const unsigned r = row0 + (RAGGED ? min(q, (unsigned)a.J - 1) : q);
+        // (a log-sum-exp of +inf: the probabilities of a query past the end are zero)
+        if (tid < 32) f.stat = !RAGGED || q < (unsigned)a.J ? a.lse[r] : INFINITY;
         else if (tid < 64) f.stat = a.dsum[r];
         else if (tid < 96) f.kw = *reinterpret_cast<const uint4*>(a.keep + (size_t)r * nkt + kb * 4);
     };
@@ -703,7 +768,7 @@ __global__ __launch_bounds__(256, (P == 64 && MASKED) ? 2 : 1) void k_mha_bwd_dk
         for (int v = 0; v < 16; ++v) { dk[pt][v] = 0.f; dv[pt][v] = 0.f; }
     int cur = 0, nxt = 1, nn = 2;
     MaskRegs mk = {};
-    if (MASKED && n > 0 && entry_class(e0, wave) != BLOCK_CLEAR) load_mask<false>(a, kpos, entry_tile(e0) * 32, hi, mk);
+    if (MASKED && n > 0 && entry_class(e0, wave) != BLOCK_CLEAR) load_mask<false, RAGGED>(a, kpos, entry_tile(e0) * 32, hi, mk);
     wait_loads();
 
     for (unsigned i = 0; i < n; ++i) {
@@ -712,11 +777,12 @@ __global__ __launch_bounds__(256, (P == 64 && MASKED) ? 2 : 1) void k_mha_bwd_dk
         const bool more = i + 2 < n;
         if (more) fetch(entry_tile(e2), fl);
         const KvStage<P>& sg = stage[cur];
+        if (working) {
         f16v s, dp;
 #pragma unroll
         for (int v = 0; v < 16; ++v) { s[v] = 0.f; dp[v] = 0.f; }
         if (from_mask) start_from_mask(mk, s);
-        if (MASKED && i + 1 < n && entry_class(e1, wave) != BLOCK_CLEAR) load_mask<false>(a, kpos, entry_tile(e1) * 32, hi, mk);
+        if (MASKED && i + 1 < n && entry_class(e1, wave) != BLOCK_CLEAR) load_mask<false, RAGGED>(a, kpos, entry_tile(e1) * 32, hi, mk);
 #pragma unroll
         for (int ks = 0; ks < G::NKS; ++ks) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(fq[ks], fk[ks], s, 0, 0, 0);
 #pragma unroll
@@ -756,13 +822,21 @@ __global__ __launch_bounds__(256, (P == 64 && MASKED) ? 2 : 1) void k_mha_bwd_dk
                 dv[pt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(da[st][pt], pd[st], dv[pt], 0, 0, 0);
                 dk[pt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(qa[st][pt], ds[st], dk[pt], 0, 0, 0);
             }
+        }
         if (more) put(stage[nn], fl);
         __syncthreads();
         const int x = cur; cur = nxt; nxt = nn; nn = x;
         e0 = e1; e1 = e2; e2 = e3;
     }
-    store_rows<P>(a.dk, h, b, kpos, hi, dk, a.alpha);
-    store_rows<P>(a.dv, h, b, kpos, hi, dv, 1.0f);
+    if (mine_) {
+        store_rows<P>(a.dk, h, b, kpos, hi, dk, a.alpha);
+        store_rows<P>(a.dv, h, b, kpos, hi, dv, 1.0f);
+    } else if (RAGGED) {          // nothing to the column sums
+#pragma unroll
+        for (int pt = 0; pt < G::NPT; ++pt)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) { dk[pt][v] = 0.f; dv[pt][v] = 0.f; }
+    }
     if (a.bias_kv) {
         const size_t ntc = (size_t)a.B * kblocks, part = (size_t)h * ntc + b * kblocks + kb;
         float* red = reinterpret_cast<float*>(&stage[0]);
@@ -771,9 +845,13 @@ __global__ __launch_bounds__(256, (P == 64 && MASKED) ? 2 : 1) void k_mha_bwd_dk
     }
 }
 
-// 8-byte loads of four mask values along whichever dim is contiguous
+// Whether the kernels have to watch the ends of the sequences.
+bool ragged(const AttnArgs& a) { return a.J % QB != 0 || a.K % QB != 0; }
+
+// 8-byte loads of four mask values along whichever dim is contiguous; the ragged kernels look at the strides themselves
 bool mask_ok(const AttnArgs& a) {
     if (!a.amask) return true;
+    if (ragged(a)) return (reinterpret_cast<uintptr_t>(a.amask) & (a.am_sk % 4 == 0 || a.am_sj % 4 == 0 ? 7 : 1)) == 0;
     if ((reinterpret_cast<uintptr_t>(a.amask) & 7) != 0) return false;
     if (a.am_sk == 1) return a.am_sj % 4 == 0;
     if (a.am_sj == 1) return a.am_sk % 4 == 0;
@@ -788,13 +866,11 @@ bool side_ok(const AttnSide& s) {
 
 bool mha_shape_ok(long H, long B, long J, long K, long P) {
     if (P != 64 && P != 128) return false;
-    if (J <= 0 || K <= 0 || J % QB != 0 || K % QB != 0) return false;
-    if (H * B * J > 0x7fffffffL || H * B * (J / QB) > 0x7fffffffL || H * B * (K / QB) > 0x7fffffffL) return false;
-    return true;
+    return J > 0 && K > 0 && J < (1L << 21) && K < (1L << 21) && H * B * J <= 0x7fffffffL && H * B * K <= 0x7fffffffL;
 }
 
 size_t mha_stat_bytes(long H, long B, long J) { return (size_t)(H * B * J) * 2 * sizeof(float); }
-size_t mha_keep_bytes(long H, long B, long J, long K) { return (size_t)(H * B * J) * (size_t)(K / 32) * 4; }
+size_t mha_keep_bytes(long H, long B, long J, long K) { return (size_t)(H * B * J) * mha_keep_pitch((unsigned)K) * 4; }
 
 bool mha_forward_ok(const AttnArgs& a, int P) {
     return mha_shape_ok(a.H, a.B, a.J, a.K, P) && a.alpha > 0.f && side_ok(a.q) && side_ok(a.k) && side_ok(a.v) && side_ok(a.o) &&
@@ -804,12 +880,14 @@ bool mha_forward_ok(const AttnArgs& a, int P) {
 
 namespace {
 size_t up16(size_t x) { return (x + 15) & ~(size_t)15; }
-size_t qlist_bytes(long J, long K) { return up16((size_t)(J / QB) * (size_t)(K / 32 + kListPad) * 4); }
-size_t klist_bytes(long J, long K) { return up16((size_t)(K / QB) * (size_t)(J / 32 + kListPad) * 4); }
+long tiles(long n) { return (n + 31) / 32; }
+long blocks(long n) { return (n + QB - 1) / QB; }
+size_t qlist_bytes(long J, long K) { return up16((size_t)blocks(J) * (size_t)(tiles(K) + kListPad) * 4); }
+size_t klist_bytes(long J, long K) { return up16((size_t)blocks(K) * (size_t)(tiles(J) + kListPad) * 4); }
 }  // namespace
 
 size_t mha_mask_plan_bytes(long J, long K) {
-    return qlist_bytes(J, K) + klist_bytes(J, K) + up16((size_t)(J / 32) * (size_t)(K / 32));
+    return qlist_bytes(J, K) + klist_bytes(J, K) + up16((size_t)tiles(J) * (size_t)tiles(K));
 }
 
 void launch_mha_mask_plan(AttnArgs& a, void* plan, bool rebuild, hipStream_t st) {
@@ -817,24 +895,37 @@ void launch_mha_mask_plan(AttnArgs& a, void* plan, bool rebuild, hipStream_t st)
     uint32_t* klist = (uint32_t*)((char*)plan + qlist_bytes(a.J, a.K));
     uint8_t* cls = (uint8_t*)plan + qlist_bytes(a.J, a.K) + klist_bytes(a.J, a.K);
     if (rebuild) {
-        hipLaunchKernelGGL(k_mha_mask_classes, dim3((unsigned)((a.J / 32) * (a.K / 32))), dim3(64), 0, st, a.amask,
-                           a.am_sj, a.am_sk, a.K, cls);
-        hipLaunchKernelGGL(k_mha_mask_lists, dim3((unsigned)(a.J / QB + a.K / QB)), dim3(64), 0, st, cls, a.J, a.K, qlist,
+        hipLaunchKernelGGL(k_mha_mask_classes, dim3((unsigned)(tiles(a.J) * tiles(a.K))), dim3(64), 0, st, a.amask,
+                           a.am_sj, a.am_sk, a.J, a.K, cls);
+        hipLaunchKernelGGL(k_mha_mask_lists, dim3((unsigned)(blocks(a.J) + blocks(a.K))), dim3(64), 0, st, cls, a.J, a.K, qlist,
                            klist);
     }
     a.qlist = qlist; a.klist = klist;
 }
 
+namespace {
+// Calls fn with (head size, has a mask, ragged) as compile-time constants.
+template <class Fn>
+void for_variant(int P, const AttnArgs& a, Fn&& fn) {
+    auto rag = [&](auto p, auto masked) {
+        if (ragged(a)) fn(p, masked, std::true_type{});
+        else fn(p, masked, std::false_type{});
+    };
+    auto msk = [&](auto p) {
+        if (a.amask) rag(p, std::true_type{});
+        else rag(p, std::false_type{});
+    };
+    if (P == 64) msk(std::integral_constant<int, 64>{});
+    else msk(std::integral_constant<int, 128>{});
+}
+}  // namespace
+
 void launch_mha_forward(const AttnArgs& a, int P, PhiloxKey key, hipStream_t st) {
     if (!mha_forward_ok(a, P)) fail("attention forward: shape, strides or alignment not supported");
-    dim3 grid((unsigned)(a.H * a.B * (a.J / QB)));
-    if (a.amask) {
-        if (P == 64) hipLaunchKernelGGL((k_mha_fwd<64, true>), grid, dim3(256), 0, st, a, key);
-        else hipLaunchKernelGGL((k_mha_fwd<128, true>), grid, dim3(256), 0, st, a, key);
-    } else {
-        if (P == 64) hipLaunchKernelGGL((k_mha_fwd<64, false>), grid, dim3(256), 0, st, a, key);
-        else hipLaunchKernelGGL((k_mha_fwd<128, false>), grid, dim3(256), 0, st, a, key);
-    }
+    dim3 grid((unsigned)(a.H * a.B * blocks(a.J)));
+    for_variant(P, a, [&](auto p, auto masked, auto rag) {
+        hipLaunchKernelGGL((k_mha_fwd<p(), masked(), rag()>), grid, dim3(256), 0, st, a, key);
+    });
     check_launch("attention forward");
 }
 
@@ -844,27 +935,19 @@ bool mha_backward_ok(const AttnArgs& a, int P) {
 
 void launch_mha_backward_dq(const AttnArgs& a, int P, hipStream_t st) {
     if (!mha_backward_ok(a, P)) fail("attention backward: shape, strides or alignment not supported");
-    dim3 grid((unsigned)(a.H * a.B * (a.J / QB)));
-    if (a.amask) {
-        if (P == 64) hipLaunchKernelGGL((k_mha_bwd_dq<64, true>), grid, dim3(256), 0, st, a);
-        else hipLaunchKernelGGL((k_mha_bwd_dq<128, true>), grid, dim3(256), 0, st, a);
-    } else {
-        if (P == 64) hipLaunchKernelGGL((k_mha_bwd_dq<64, false>), grid, dim3(256), 0, st, a);
-        else hipLaunchKernelGGL((k_mha_bwd_dq<128, false>), grid, dim3(256), 0, st, a);
-    }
+    dim3 grid((unsigned)(a.H * a.B * blocks(a.J)));
+    for_variant(P, a, [&](auto p, auto masked, auto rag) {
+        hipLaunchKernelGGL((k_mha_bwd_dq<p(), masked(), rag()>), grid, dim3(256), 0, st, a);
+    });
     check_launch("attention backward (dQ)");
 }
 
 void launch_mha_backward_dkv(const AttnArgs& a, int P, hipStream_t st) {
     if (!mha_backward_ok(a, P)) fail("attention backward: shape, strides or alignment not supported");
-    dim3 grid((unsigned)(a.H * a.B * (a.K / QB)));
-    if (a.amask) {
-        if (P == 64) hipLaunchKernelGGL((k_mha_bwd_dkv<64, true>), grid, dim3(256), 0, st, a);
-        else hipLaunchKernelGGL((k_mha_bwd_dkv<128, true>), grid, dim3(256), 0, st, a);
-    } else {
-        if (P == 64) hipLaunchKernelGGL((k_mha_bwd_dkv<64, false>), grid, dim3(256), 0, st, a);
-        else hipLaunchKernelGGL((k_mha_bwd_dkv<128, false>), grid, dim3(256), 0, st, a);
-    }
+    dim3 grid((unsigned)(a.H * a.B * blocks(a.K)));
+    for_variant(P, a, [&](auto p, auto masked, auto rag) {
+        hipLaunchKernelGGL((k_mha_bwd_dkv<p(), masked(), rag()>), grid, dim3(256), 0, st, a);
+    });
     check_launch("attention backward (dK, dV)");
 }
 

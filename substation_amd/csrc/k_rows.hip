@@ -5,6 +5,8 @@
 // processed several per wave at once so that enough loads are in flight.
 // Counterparts: pytorch_module/block_softmax.cuh:12-188, block_bs.cuh:13-156,
 // block_bdrln.cuh:17-352, block_blnrd.cuh:14-259.
+#include <initializer_list>
+
 #include "sub_ops.hpp"
 
 namespace sub {
@@ -20,17 +22,39 @@ __device__ __forceinline__ int nvalid_at(int R, int e0) {
     return n < 0 ? 0 : (n > 8 ? 8 : n);
 }
 
+// What k_softmax writes for the attention kernels' backward pass instead of the probabilities and the mask: per row
+// the log2-domain log-sum-exp, and the keep bits (bit k % 32 of word k / 32, `pitch` words per row).
+struct SoftmaxStats {
+    float* lse = nullptr;
+    uint8_t* keep = nullptr;
+    unsigned pitch = 0;
+};
+
+template <int MODE, bool NT>
+__device__ __forceinline__ F8 row_load(const View& t, long base, int e0, int nv, int R, float fill = 0.f) {
+    if constexpr (MODE == ROW_PACKED) return ld8_packed<NT>(t, base, e0, nv, R, fill);
+    else return ld8<MODE == ROW_FAST, NT>(t, base, e0, nv, fill);
+}
+template <int MODE, bool NT>
+__device__ __forceinline__ void row_store(const View& t, long base, int e0, int nv, h8 v) {
+    if constexpr (MODE == ROW_PACKED) st8_packed<NT>(t, base, e0, nv, v);
+    else st8h<MODE == ROW_FAST, NT>(t, base, e0, nv, v);
+}
+
 // VPL: 8-packs per lane (row length <= 8*GRP*VPL).  RPW: rows per lane group per
-// step.  FAST: all views vectorisable (see ld8).  GRP: lanes per row; rows of up
+// step.  MODE: how the views are accessed (RowMode).  GRP: lanes per row; rows of up
 // to 256 (128) elements take half (a quarter) of a wave, so that two (four) of
 // them are processed side by side and no lane idles.
+// ROW_PACKED bounds: as the other modes memory, and one more instruction or two per element; through single-element
+// accesses, two Philox calls per pack and one row per wave, softmax took 34 us at [12,8,197,197] (softmax + backward
+// at L=201: see launch_softmax).
 // amask (optional, p == nullptr when absent): additive attention mask indexed by
 // (query position, key position) only, x = beta * scale + amask * mscale
 // (substation/attention.py:65-68 adds it before the scaling, hence mscale).
-template <int VPL, int RPW, bool FAST, bool FLAT = false, int GRP = WAVE, bool MASKED = false>
+template <int VPL, int RPW, int MODE, bool FLAT = false, int GRP = WAVE, bool MASKED = false, bool STATS = false>
 __global__ __launch_bounds__(BLOCK) void k_softmax(RowSpace rs, View beta, View alpha, View mask,
                                                    View drop, View amask, float scale, float mscale,
-                                                   PhiloxKey key_, unsigned nrows) {
+                                                   PhiloxKey key_, unsigned nrows, SoftmaxStats stats) {
     const PhiloxKey key = resolved(key_);
     constexpr int SPW = WAVE / GRP;                    // rows side by side in a wave
     const int lane = threadIdx.x & 63, gl = lane % GRP, sub = lane / GRP;
@@ -51,7 +75,7 @@ __global__ __launch_bounds__(BLOCK) void k_softmax(RowSpace rs, View beta, View 
             for (int c = 0; c < VPL; ++c) {
                 int e0 = (c * GRP + gl) * 8;
                 int nv = live ? nvalid_at(rs.R, e0) : 0;
-                F8 f = ld8<FAST, true>(beta, ob, e0, nv, -INFINITY);
+                F8 f = row_load<MODE, true>(beta, ob, e0, nv, rs.R, -INFINITY);
                 if (MASKED) {
                     // every (head, sample) re-reads the mask: plain loads, it stays in cache
                     F8 am = load8(amask, oam, e0, nv, 0.f);
@@ -86,31 +110,40 @@ __global__ __launch_bounds__(BLOCK) void k_softmax(RowSpace rs, View beta, View 
 #pragma unroll
         for (int r = 0; r < RPW; ++r) {
             const unsigned row = row0 + r * SPW + sub;
+            uint32_t packed[VPL];
+            if constexpr (MODE == ROW_PACKED) keep_packs<VPL, GRP>(key, (uint64_t)row * (uint64_t)rs.R, rs.R, gl, packed);
             if (row >= nrows) continue;
             const float inv = 1.0f / s[r];
             const long oa = view_offset_of<FLAT>(alpha, ix[r]), om = view_offset_of<FLAT>(mask, ix[r]), od = view_offset_of<FLAT>(drop, ix[r]);
+            if (STATS && gl == 0) stats.lse[row] = m[r] * LOG2E + __builtin_amdgcn_logf(s[r]);
 #pragma unroll
             for (int c = 0; c < VPL; ++c) {
                 int e0 = (c * GRP + gl) * 8;
                 int nv = nvalid_at(rs.R, e0);
                 if (nv > 0) {
                     h8 a, d;
-                    uint32_t bits = keep_pack<FAST>(key, (uint64_t)row * (uint64_t)rs.R + (uint64_t)e0);
+                    uint32_t bits;
+                    if constexpr (MODE == ROW_PACKED) bits = packed[c];
+                    else bits = keep_pack<MODE == ROW_FAST>(key, (uint64_t)row * (uint64_t)rs.R + (uint64_t)e0);
 #pragma unroll
                     for (int i = 0; i < 8; ++i) a[i] = (half_t)(x[r][c][i] * inv);
                     a = pin(a);
 #pragma unroll
                     for (int i = 0; i < 8; ++i) d[i] = ((bits >> i) & 1u) ? a[i] : (half_t)0.0f;
-                    st8h<FAST, true>(alpha, oa, e0, nv, a);
-                    st8h<FAST, true>(mask, om, e0, nv, mask_h8(bits));
-                    st8h<FAST>(drop, od, e0, nv, d);
+                    if (STATS) {
+                        stats.keep[(size_t)row * (stats.pitch * 4) + (e0 >> 3)] = (uint8_t)bits;
+                    } else {
+                        row_store<MODE, true>(alpha, oa, e0, nv, a);
+                        row_store<MODE, true>(mask, om, e0, nv, mask_h8(bits));
+                    }
+                    row_store<MODE, false>(drop, od, e0, nv, d);
                 }
             }
         }
     }
 }
 
-template <int VPL, int RPW, bool FAST, bool FLAT = false, int GRP = WAVE>
+template <int VPL, int RPW, int MODE, bool FLAT = false, int GRP = WAVE>
 __global__ __launch_bounds__(BLOCK) void k_bs(RowSpace rs, View alpha, View mask, View ddrop,
                                               View dbeta, float scale, unsigned nrows) {
     constexpr int SPW = WAVE / GRP;
@@ -131,7 +164,8 @@ __global__ __launch_bounds__(BLOCK) void k_bs(RowSpace rs, View alpha, View mask
             for (int c = 0; c < VPL; ++c) {
                 int e0 = (c * GRP + gl) * 8;
                 int nv = live ? nvalid_at(rs.R, e0) : 0;
-                F8 fa = ld8<FAST, true>(alpha, oa, e0, nv), fm = ld8<FAST, true>(mask, om, e0, nv), fd = ld8<FAST, true>(ddrop, od, e0, nv);
+                F8 fa = row_load<MODE, true>(alpha, oa, e0, nv, rs.R), fm = row_load<MODE, true>(mask, om, e0, nv, rs.R),
+                   fd = row_load<MODE, true>(ddrop, od, e0, nv, rs.R);
 #pragma unroll
                 for (int i = 0; i < 8; ++i) {
                     a[r][c][i] = fa.v[i];
@@ -154,7 +188,7 @@ __global__ __launch_bounds__(BLOCK) void k_bs(RowSpace rs, View alpha, View mask
                     h8 o;
 #pragma unroll
                     for (int i = 0; i < 8; ++i) o[i] = (half_t)(scale * a[r][c][i] * (g[r][c][i] - s[r]));
-                    st8h<FAST>(dbeta, oo, e0, nv, o);
+                    row_store<MODE, false>(dbeta, oo, e0, nv, o);
                 }
             }
         }
@@ -562,64 +596,122 @@ inline unsigned check_rows(const RowSpace& rs, const char* what) {
         }                                                                          \
     } while (0)
 
+// How softmax and its backward access their rows.  ROW_PACKED where the row dim is contiguous everywhere and the row
+// long enough to be read from its end; what is left (a strided row dim) goes element by element.
+namespace {
+int row_mode(const RowSpace& rs, std::initializer_list<View> views) {
+    bool vec = true, packed = rs.R >= 8;
+    for (const View& v : views) { vec = vec && v.vec; packed = packed && v.sr == 1; }
+    return vec ? ROW_FAST : packed ? ROW_PACKED : ROW_STRIDED;
+}
+// Short rows sit two or four side by side in a wave, and several waves' worth of rows are in flight per wave, once there
+// are enough of them to leave 16 waves per CU.
+bool many_rows(unsigned nrows) { return nrows >= 256u * 16u * 4u; }
+}  // namespace
+
 void launch_softmax(const RowSpace& rs, View beta, View alpha, View mask, View drop, View amask,
-                    float scale, float mscale, PhiloxKey key, hipStream_t st) {
-    const unsigned extra_blocks = 0;
+                    float scale, float mscale, PhiloxKey key, hipStream_t st, float* lse, uint32_t* keep, unsigned keep_pitch) {
     unsigned nrows = check_rows(rs, "softmax");
     if (nrows == 0) return;
-    int vpl = pick_vpl(rs.R, "softmax");
-    bool fast = beta.vec && alpha.vec && mask.vec && drop.vec;
-    const bool masked = amask.p != nullptr;
-    if (fast && rs.R <= 256 && nrows >= 256u * 16u * 4u) {
-        // short rows: two or four side by side in every wave
-#define SUB_SM_SHORT(G, RPS, M)                                                                        \
-        hipLaunchKernelGGL((k_softmax<1, 4, true, false, G, M>), dim3(row_grid(nrows, RPS)), dim3(BLOCK), 0, st, rs, \
-                           beta, alpha, mask, drop, amask, scale, mscale, key, nrows)
-        if (rs.R <= 128) { if (masked) SUB_SM_SHORT(16, 16, true); else SUB_SM_SHORT(16, 16, false); }
-        else { if (masked) SUB_SM_SHORT(32, 8, true); else SUB_SM_SHORT(32, 8, false); }
-#undef SUB_SM_SHORT
+    const int vpl = pick_vpl(rs.R, "softmax");
+    const bool masked = amask.p != nullptr, many = many_rows(nrows);
+    const SoftmaxStats stats{lse, (uint8_t*)keep, keep_pitch};
+#define SUB_SM(V, RPW, MODE, FLAT, G, M, ST)                                                                                \
+    hipLaunchKernelGGL((k_softmax<V, RPW, MODE, FLAT, G, M, ST>), dim3(row_grid(nrows, (RPW) * (WAVE / (G)))), dim3(BLOCK), 0, \
+                       st, rs, beta, alpha, mask, drop, amask, scale, mscale, key, nrows, stats)
+#define SUB_SM_VPL(RPW1, RPW2, MODE, FLAT, M, ST)                                                                           \
+    switch (vpl) {                                                                                                          \
+        case 1: SUB_SM(1, RPW1, MODE, FLAT, WAVE, M, ST); break;                                                            \
+        case 2: SUB_SM(2, RPW2, MODE, FLAT, WAVE, M, ST); break;                                                            \
+        case 4: SUB_SM(4, 1, MODE, FLAT, WAVE, M, ST); break;                                                               \
+        default: SUB_SM(8, 1, MODE, FLAT, WAVE, M, ST); break;                                                              \
+    }
+    if (lse) {
+        // what the attention kernels' backward pass reads takes the place of the probabilities and the mask
+        const int mode = row_mode(rs, {beta, drop});
+        if (mode == ROW_FAST) {
+            if (masked) { SUB_SM_VPL(1, 1, ROW_FAST, false, true, true) } else { SUB_SM_VPL(1, 1, ROW_FAST, false, false, true) }
+        } else if (mode == ROW_PACKED) {
+            if (masked) { SUB_SM_VPL(1, 1, ROW_PACKED, false, true, true) } else { SUB_SM_VPL(1, 1, ROW_PACKED, false, false, true) }
+        } else {
+            if (masked) { SUB_SM_VPL(1, 1, ROW_STRIDED, false, true, true) } else { SUB_SM_VPL(1, 1, ROW_STRIDED, false, false, true) }
+        }
         check_launch("softmax");
         return;
+    }
+    const int mode = row_mode(rs, {beta, alpha, mask, drop});
+    if (mode != ROW_STRIDED && rs.R <= 256 && many) {
+        // short rows: two or four side by side in every wave
+        if (mode == ROW_FAST) {
+            if (rs.R <= 128) { if (masked) SUB_SM(1, 4, ROW_FAST, false, 16, true, false); else SUB_SM(1, 4, ROW_FAST, false, 16, false, false); }
+            else { if (masked) SUB_SM(1, 4, ROW_FAST, false, 32, true, false); else SUB_SM(1, 4, ROW_FAST, false, 32, false, false); }
+            check_launch("softmax");
+            return;
+        }
+        if (!masked && rs.flat) {
+            if (rs.R <= 128) SUB_SM(1, 2, ROW_PACKED, true, 16, false, false);
+            else SUB_SM(1, 2, ROW_PACKED, true, 32, false, false);
+            check_launch("softmax");
+            return;
+        }
     }
     if (masked) {
         // one row per wave; the mask rows are re-read by every head and sample from cache
-#define SUB_SM_MASKED(V, F)                                                                            \
-        hipLaunchKernelGGL((k_softmax<V, 1, F, false, WAVE, true>), dim3(row_grid(nrows, 1)), dim3(BLOCK), 0, st, rs, \
-                           beta, alpha, mask, drop, amask, scale, mscale, key, nrows)
-        switch (vpl) {
-            case 1: if (fast) SUB_SM_MASKED(1, true); else SUB_SM_MASKED(1, false); break;
-            case 2: if (fast) SUB_SM_MASKED(2, true); else SUB_SM_MASKED(2, false); break;
-            case 4: if (fast) SUB_SM_MASKED(4, true); else SUB_SM_MASKED(4, false); break;
-            default: if (fast) SUB_SM_MASKED(8, true); else SUB_SM_MASKED(8, false); break;
-        }
-#undef SUB_SM_MASKED
-        check_launch("softmax");
-        return;
+        if (mode == ROW_FAST) { SUB_SM_VPL(1, 1, ROW_FAST, false, true, false) }
+        else if (mode == ROW_PACKED) { SUB_SM_VPL(1, 1, ROW_PACKED, false, true, false) }
+        else { SUB_SM_VPL(1, 1, ROW_STRIDED, false, true, false) }
+    } else if (mode == ROW_FAST && rs.flat) {
+        if (many) { SUB_SM_VPL(4, 2, ROW_FAST, true, false, false) } else { SUB_SM_VPL(1, 1, ROW_FAST, true, false, false) }
+    } else if (mode == ROW_FAST) {
+        if (many) { SUB_SM_VPL(4, 2, ROW_FAST, false, false, false) } else { SUB_SM_VPL(1, 1, ROW_FAST, false, false, false) }
+    } else if (mode == ROW_PACKED && rs.flat) {
+        if (many) { SUB_SM_VPL(2, 1, ROW_PACKED, true, false, false) } else { SUB_SM_VPL(1, 1, ROW_PACKED, true, false, false) }
+    } else if (mode == ROW_PACKED) {
+        SUB_SM_VPL(1, 1, ROW_PACKED, false, false, false)
+    } else {
+        SUB_SM_VPL(1, 1, ROW_STRIDED, false, false, false)
     }
-    if (fast && rs.flat) SUB_ROW_DISPATCH_FLAT(k_softmax, vpl, rs, beta, alpha, mask, drop, amask, scale, mscale, key, nrows);
-    else SUB_ROW_DISPATCH(k_softmax, vpl, fast, rs, beta, alpha, mask, drop, amask, scale, mscale, key, nrows);
+#undef SUB_SM_VPL
+#undef SUB_SM
     check_launch("softmax");
 }
 
 void launch_bs(const RowSpace& rs, View alpha, View mask, View ddrop, View dbeta, float scale,
                hipStream_t st) {
-    const unsigned extra_blocks = 0;
     unsigned nrows = check_rows(rs, "softmax backward");
     if (nrows == 0) return;
-    int vpl = pick_vpl(rs.R, "softmax backward");
-    bool fast = alpha.vec && mask.vec && ddrop.vec && dbeta.vec;
-    if (fast && rs.R <= 256 && nrows >= 256u * 16u * 4u) {
-        if (rs.R <= 128)
-            hipLaunchKernelGGL((k_bs<1, 4, true, false, 16>), dim3(row_grid(nrows, 16)), dim3(BLOCK), 0, st, rs, alpha,
-                               mask, ddrop, dbeta, scale, nrows);
-        else
-            hipLaunchKernelGGL((k_bs<1, 4, true, false, 32>), dim3(row_grid(nrows, 8)), dim3(BLOCK), 0, st, rs, alpha,
-                               mask, ddrop, dbeta, scale, nrows);
-        check_launch("softmax backward");
-        return;
+    const int vpl = pick_vpl(rs.R, "softmax backward");
+    const int mode = row_mode(rs, {alpha, mask, ddrop, dbeta});
+    const bool many = many_rows(nrows);
+#define SUB_BS(V, RPW, MODE, FLAT, G)                                                                                       \
+    hipLaunchKernelGGL((k_bs<V, RPW, MODE, FLAT, G>), dim3(row_grid(nrows, (RPW) * (WAVE / (G)))), dim3(BLOCK), 0, st, rs,      \
+                       alpha, mask, ddrop, dbeta, scale, nrows)
+#define SUB_BS_VPL(RPW1, RPW2, MODE, FLAT)                                                                                  \
+    switch (vpl) {                                                                                                          \
+        case 1: SUB_BS(1, RPW1, MODE, FLAT, WAVE); break;                                                                   \
+        case 2: SUB_BS(2, RPW2, MODE, FLAT, WAVE); break;                                                                   \
+        case 4: SUB_BS(4, 1, MODE, FLAT, WAVE); break;                                                                      \
+        default: SUB_BS(8, 1, MODE, FLAT, WAVE); break;                                                                     \
     }
-    if (fast && rs.flat) SUB_ROW_DISPATCH_FLAT(k_bs, vpl, rs, alpha, mask, ddrop, dbeta, scale, nrows);
-    else SUB_ROW_DISPATCH(k_bs, vpl, fast, rs, alpha, mask, ddrop, dbeta, scale, nrows);
+    if (mode == ROW_FAST && rs.R <= 256 && many) {
+        if (rs.R <= 128) SUB_BS(1, 4, ROW_FAST, false, 16);
+        else SUB_BS(1, 4, ROW_FAST, false, 32);
+    } else if (mode == ROW_PACKED && rs.flat && rs.R <= 256 && many) {
+        if (rs.R <= 128) SUB_BS(1, 2, ROW_PACKED, true, 16);
+        else SUB_BS(1, 2, ROW_PACKED, true, 32);
+    } else if (mode == ROW_FAST && rs.flat) {
+        if (many) { SUB_BS_VPL(4, 2, ROW_FAST, true) } else { SUB_BS_VPL(1, 1, ROW_FAST, true) }
+    } else if (mode == ROW_FAST) {
+        if (many) { SUB_BS_VPL(4, 2, ROW_FAST, false) } else { SUB_BS_VPL(1, 1, ROW_FAST, false) }
+    } else if (mode == ROW_PACKED && rs.flat) {
+        if (many) { SUB_BS_VPL(2, 1, ROW_PACKED, true) } else { SUB_BS_VPL(1, 1, ROW_PACKED, true) }
+    } else if (mode == ROW_PACKED) {
+        SUB_BS_VPL(1, 1, ROW_PACKED, false)
+    } else {
+        SUB_BS_VPL(1, 1, ROW_STRIDED, false)
+    }
+#undef SUB_BS_VPL
+#undef SUB_BS
     check_launch("softmax backward");
 }
 

@@ -133,6 +133,50 @@ __device__ __forceinline__ void stg8(half_t* p, h8 v) {
     else *reinterpret_cast<h8*>(p) = v;
 }
 
+// Access modes of the row kernels.  ROW_FAST as above.  ROW_PACKED: the row dim is contiguous in every view and rows
+// are at least 8 elements long, but start and end anywhere (lengths that are not multiples of 8): packs are still 16
+// bytes, at 2-byte alignment, and the pack that the end of the row cuts through is read as the row's last 8 elements,
+// shifted down.
+enum RowMode : int { ROW_STRIDED = 0, ROW_FAST = 1, ROW_PACKED = 2 };
+typedef _Float16 h8u __attribute__((ext_vector_type(8), aligned(2)));
+
+// v[i] = v[i + s], zeros from above (0 <= s < 8)
+__device__ __forceinline__ h8 shift_down(h8 v, int s) {
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    u4 w = __builtin_bit_cast(u4, v);
+    if (s & 4) { w[0] = w[2]; w[1] = w[3]; w[2] = 0u; w[3] = 0u; }
+    if (s & 2) { w[0] = w[1]; w[1] = w[2]; w[2] = w[3]; w[3] = 0u; }
+    if (s & 1) {
+        w[0] = __builtin_amdgcn_alignbit(w[1], w[0], 16); w[1] = __builtin_amdgcn_alignbit(w[2], w[1], 16);
+        w[2] = __builtin_amdgcn_alignbit(w[3], w[2], 16); w[3] >>= 16;
+    }
+    return __builtin_bit_cast(h8, w);
+}
+
+// ROW_PACKED: elements e0 .. e0 + nvalid - 1 of the row of R elements at `base`, no branch around the load (see ld8).
+template <bool NT>
+__device__ __forceinline__ F8 ld8_packed(const View& t, long base, int e0, int nvalid, int R, float fill = 0.f) {
+    const int at = nvalid == 8 ? e0 : nvalid ? R - 8 : 0;
+    const h8u* p = reinterpret_cast<const h8u*>(t.p + base + at);
+    const h8 v = shift_down(NT ? (h8)__builtin_nontemporal_load(p) : (h8)*p, nvalid ? 8 - nvalid : 0);
+    F8 r;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) r.v[i] = i < nvalid ? (float)v[i] : fill;
+    return r;
+}
+template <bool NT>
+__device__ __forceinline__ void st8_packed(const View& t, long base, int e0, int nvalid, h8 v) {
+    half_t* p = t.p + base + e0;
+    if (nvalid == 8) {
+        if (NT) __builtin_nontemporal_store((h8u)v, reinterpret_cast<h8u*>(p));
+        else *reinterpret_cast<h8u*>(p) = v;
+    } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (i < nvalid) p[i] = v[i];
+    }
+}
+
 template <bool FAST, bool NT = false>
 __device__ __forceinline__ F8 ld8(const View& t, long base, int e0, int nvalid, float fill = 0.f) {
     if (FAST) {
@@ -213,6 +257,27 @@ __device__ __forceinline__ U4 philox_group_dev(const PhiloxKey& k, uint64_t g) {
 template <bool FAST>
 __device__ __forceinline__ uint32_t keep_pack(const PhiloxKey& key, uint64_t e) {
     return FAST ? keep8(philox_group_dev(key, e >> 3), key.thr) : keep_bits8(key, e);
+}
+
+// Keep bits of the packs of a row that starts anywhere in a Philox group (ROW_PACKED): pack c of lane `gl` of a group
+// of GRP lanes starts at canonical element row0 + (c * GRP + gl) * 8 and needs two groups, the second of which the
+// lane above draws as its first.  All lanes take part; R = elements of the row.
+template <int VPL, int GRP>
+__device__ __forceinline__ void keep_packs(const PhiloxKey& key, uint64_t row0, int R, int gl, uint32_t (&bits)[VPL]) {
+    const int off = (int)(row0 & 7);
+    uint32_t own[VPL];
+#pragma unroll
+    for (int c = 0; c < VPL; ++c) own[c] = keep8(philox_group_dev(key, (row0 >> 3) + (uint64_t)(c * GRP + gl)), key.thr);
+    // the group behind the last lane's last pack, which only a row that reaches that far needs
+    uint32_t behind = 0;
+    if (R > VPL * GRP * 8 - 8) behind = keep8(philox_group_dev(key, (row0 >> 3) + (uint64_t)(VPL * GRP)), key.thr);
+#pragma unroll
+    for (int c = 0; c < VPL; ++c) {
+        const uint32_t up = (uint32_t)__shfl_down((int)own[c], 1, GRP);
+        const uint32_t wrap = c + 1 < VPL ? (uint32_t)__shfl((int)own[c + 1 < VPL ? c + 1 : c], 0, GRP) : behind;
+        const uint32_t next = gl == GRP - 1 ? wrap : up;
+        bits[c] = ((own[c] | (next << 8)) >> off) & 0xffu;
+    }
 }
 
 // The 32 keep bits of key tile t of score row `row` in the attention kernels' format (bit k =

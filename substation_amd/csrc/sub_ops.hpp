@@ -17,8 +17,11 @@ inline void check_launch(const char* what) {
 
 // --- row operators (one wave per row, row held in registers) -----------------
 // amask: optional additive attention mask over (query, key) positions (p == nullptr: none)
+// lse, keep (optional, both or neither; rs over H, B, J in this order): per row the log2-domain log-sum-exp and the keep
+// bits in the attention kernels' format (keep_pitch words per row) instead of alpha and mask, which are not written
 void launch_softmax(const RowSpace& rs, View beta, View alpha, View mask, View drop, View amask,
-                    float scale, float mscale, PhiloxKey key, hipStream_t st);
+                    float scale, float mscale, PhiloxKey key, hipStream_t st, float* lse = nullptr, uint32_t* keep = nullptr,
+                    unsigned keep_pitch = 0);
 void launch_bs(const RowSpace& rs, View alpha, View mask, View ddrop, View dbeta, float scale,
                hipStream_t st);
 // Side job of launch_bdrln (a launch that waits for memory with its vector units idle): `blocks`
@@ -160,15 +163,15 @@ struct AttnArgs {
     AttnSide dq, dk, dv;       // backward: gradients of the projections (written)
     float* lse = nullptr;      // [H*B*J]  log2-domain log-sum-exp of each score row
     float* dsum = nullptr;     // [H*B*J]  row sums of dO o O (written by the dQ launch, read by the dK/dV one)
-    uint32_t* keep = nullptr;  // [H*B*J][K/32]  keep bits of the softmax dropout, bit k%32 of word k/32
+    uint32_t* keep = nullptr;  // [H*B*J][mha_keep_pitch(K)]  keep bits of the softmax dropout, bit k%32 of word k/32
     // forward: the words of key tiles 0 .. keep_tiles_ready-1 of every row are in `keep` already
     // (GemmSideJob); the kernel draws and stores the others
     uint32_t keep_tiles_ready = 0;
     int H = 0, B = 0, J = 0, K = 0;
     float alpha = 1.f;         // score scale
     // optional (backward): per-workgroup sums over positions of the rounded dq resp.
-    // dk, dv rows, for the gradient of the projection biases.  bias_q: [H][B*J/128][P]
-    // floats, bias_kv: [2][H][B*K/128][P] (dk, then dv).
+    // dk, dv rows, for the gradient of the projection biases.  bias_q: [H][B*ceil(J/128)][P]
+    // floats, bias_kv: [2][H][B*ceil(K/128)][P] (dk, then dv).
     float* bias_q = nullptr;
     float* bias_kv = nullptr;
     const half_t* amask = nullptr;   // optional additive mask over (query, key), added before the scaling
@@ -180,8 +183,10 @@ struct AttnArgs {
     const uint32_t* qlist = nullptr;
     const uint32_t* klist = nullptr;
 };
-// head_size 64 or 128, J and K multiples of 128
+// head_size 64 or 128
 bool mha_shape_ok(long H, long B, long J, long K, long head_size);
+// Words of keep bits per score row.
+inline unsigned mha_keep_pitch(unsigned K) { return (K + 127) / 128 * 4; }
 size_t mha_stat_bytes(long H, long B, long J);          // lse followed by dsum
 size_t mha_keep_bytes(long H, long B, long J, long K);
 bool mha_forward_ok(const AttnArgs& a, int head_size);
@@ -189,7 +194,7 @@ bool mha_backward_ok(const AttnArgs& a, int head_size);
 void launch_mha_forward(const AttnArgs& a, int head_size, PhiloxKey key, hipStream_t st);
 // skip[J/32][K/32] = 1 where mask[j][k] is -inf for every (j, k) of the block
 // Device bytes of the plan of a [J, K] mask, and the launches that fill it (rebuild)
-// and point the arguments at it.  J and K multiples of 128.
+// and point the arguments at it.
 size_t mha_mask_plan_bytes(long J, long K);
 void launch_mha_mask_plan(AttnArgs& a, void* plan, bool rebuild, hipStream_t st);
 void launch_mha_backward_dq(const AttnArgs& a, int head_size, hipStream_t st);

@@ -104,11 +104,7 @@ SUB_HD uint32_t keep_bits8(const PhiloxKey& k, uint64_t e0) {
         bits = keep8(r0, k.thr);
     } else {
         U4 r1 = philox_group(k, g + 1);
-        for (int i = 0; i < 8; ++i) {
-            int f = off + i;
-            uint32_t v = f < 8 ? field16(r0, f) : field16(r1, f - 8);
-            bits |= (v >= k.thr ? 1u : 0u) << i;
-        }
+        bits = ((keep8(r0, k.thr) | (keep8(r1, k.thr) << 8)) >> off) & 0xffu;
     }
     return bits;
 }

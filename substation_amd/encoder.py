@@ -102,7 +102,7 @@ class Encoder(torch.nn.Module):
             self._handle.set_option(_lib.OPT_PRIVATE_LAYOUTS, 0)
         # compact_attention: when self-attention runs with the scores in registers,
         # four of the six score-sized tensors ([H,B,J,K]) are never touched and the
-        # other two only hold 8 resp. K/8 bytes per score row; allocate just that
+        # other two only hold 8 resp. K/8 (K rounded up to 128) bytes per score row; allocate just that
         # (at B=8 L=512 H=16: 5 MiB instead of 384 MiB per layer call).  The path is
         # then required: a later change that rules it out (option 4 = 0, a misaligned
         # tensor) makes forward() raise instead of writing through the small buffers.
@@ -114,7 +114,7 @@ class Encoder(torch.nn.Module):
         compact = {}
         if self.compact_attention:
             compact = {'BETA': 8, 'ATTN_DROP': 8, 'DATTN_DROP': 8, 'DBETA': 8,
-                       'ALPHA': rows * 4, 'ATTN_DROP_MASK': rows * max(max_seq_len // 16, 1)}
+                       'ALPHA': rows * 4, 'ATTN_DROP_MASK': rows * 8 * -(-max_seq_len // 128)}
         # compact_activation: as above for the two feed-forward tensors that the ReLU
         # path leaves untouched while option 6 is on; forward() and backward() check it.
         self.compact_activation = bool(compact_activation and not enable_debug and activation == 'relu'

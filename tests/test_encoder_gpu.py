@@ -214,6 +214,34 @@ def test_default_path_matches_the_oracle(dims, p, masked, compact):
     _compare(want, got, names=OUTPUTS)
 
 
+# one key tile and less, one position past a tile and past a block, rows that start anywhere in a group of keep bits
+@pytest.mark.parametrize('dims,masked,compact', [
+    ((3, 8, 2, 128), False, False), ((2, 33, 2, 128), True, False), ((5, 77, 3, 192), False, True),
+    ((2, 127, 1, 128), False, False), ((3, 129, 2, 128), True, True), ((2, 201, 2, 256), False, True),
+    ((1, 200, 2, 256), True, False), ((1, 285, 3, 192), True, True)])
+def test_attention_in_registers_at_any_sequence_length(dims, masked, compact):
+    """Sequence lengths that are not multiples of 128, head sizes 64 and 128: the layer as shipped against the oracle."""
+    L, launches = dims[1], []
+    am = np.triu(np.full((L, L), -np.inf), 1) if masked else None
+    if masked and L > 128:
+        am[L - 1, :40] = -np.inf                  # a mixed block in the last row of blocks
+    want, got = run_layer_default(*dims, 0.1, seed_data=L, attn_mask=am, compact=compact, launches=launches)
+    assert 'attention' in launches and 'attention-bwd-dKdV' in launches, launches
+    _compare(want, got, names=OUTPUTS)
+
+
+@pytest.mark.parametrize('dims,masked', [((3, 8, 2, 128), False), ((2, 77, 2, 128), False), ((2, 72, 2, 256), True),
+                                         ((1, 519, 2, 128), True), ((1, 1030, 1, 64), False)])
+def test_relu_forward_in_operators_backward_in_registers(dims, masked):
+    """ReLU layers at sequence lengths that are not multiples of 128: the softmax operator leaves the statistics and keep
+    bits that the attention kernels' backward pass reads; rows that start anywhere in a group of keep bits."""
+    L, launches = dims[1], []
+    am = np.triu(np.full((L, L), -np.inf), 1) if masked else None
+    want, got = run_layer_default(*dims, 0.1, seed_data=L, attn_mask=am, act='relu', launches=launches)
+    assert 'softmax' in launches and 'attention-bwd-dKdV' in launches, launches
+    _compare(want, got, names=OUTPUTS)
+
+
 @pytest.mark.parametrize('dims,which', [((8, 512, 16, 1024), 'mi355x:bert-b8-l512-h16-e1024'),
                                         ((96, 128, 16, 1024), 'mi355x:bert-b96-l128-h16-e1024'),
                                         # 96 + 96 and 96 + 96 + 32 tiles of 256 x 128 in the paired launches

@@ -42,6 +42,12 @@ def test_all_contractions(B, L, H, E):
         assert 1 in kinds, 'the MFMA kernel was never selected'
 
 
+@pytest.mark.parametrize('B,L,H,E', [(2, 67, 2, 128), (1, 129, 1, 40), (3, 5, 2, 6)])
+def test_contractions_of_odd_sizes(B, L, H, E):
+    """Rows that are not whole 16-byte words: the kernel for any strides and sizes, tiles with remainders on every side."""
+    test_all_contractions(B, L, H, E)
+
+
 def test_k_remainder_and_tile_edges():
     """K not a multiple of the 64-wide LDS tile, M/N not multiples of 128."""
     from substation_amd.ops import Ops

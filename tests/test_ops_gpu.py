@@ -73,6 +73,14 @@ def test_softmax_and_backward(B, L, H, E, p):
                      name='DBETA ' + lin)
 
 
+# rows that are contiguous but end and start anywhere: the shortest, one short of a lane's last pack, several side by side
+# in a wave (>= 16384 rows), two and four packs per lane, the last lane's last pack cut
+@pytest.mark.parametrize('B,L,H,E', [(2, 9, 2, 16), (1, 65, 3, 48), (14, 77, 16, 32), (6, 201, 16, 32), (2, 511, 1, 16),
+                                     (1, 523, 2, 16), (17, 517, 2, 16), (1, 2047, 1, 16)])
+def test_softmax_and_backward_on_rows_of_any_length(B, L, H, E):
+    test_softmax_and_backward(B, L, H, E, 0.3)
+
+
 def test_softmax_baseline_config_full_size():
     """scores [H=16,B=8,J=512,K=512] ~ N(0,1), scale 1/sqrt(64),
     p=0.1 seeded, forward plus softmax backward with dY ~ N(0,1), at full size."""
