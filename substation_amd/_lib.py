@@ -46,6 +46,7 @@ class SubConfig(ctypes.Structure):
 
 
 _lib = None
+_host = None
 
 _VP, _CP, _F, _U32, _U64, _I = (ctypes.c_void_p, ctypes.c_char_p, ctypes.c_float, ctypes.c_uint32,
                                 ctypes.c_uint64, ctypes.c_int)
@@ -135,6 +136,25 @@ def load():
 
 class SubstationError(RuntimeError):
     pass
+
+
+def host():
+    """The extension module that carries a layer call from torch to the library (csrc/host.cpp)."""
+    global _host
+    if _host is None:
+        import importlib.machinery
+        import importlib.util
+        path = os.path.join(HERE, 'lib', '_host.so')
+        if not os.path.exists(path):
+            raise RuntimeError(f'{path} is missing: build it with `python -m substation_amd.build` '
+                               '(there is no fallback implementation)')
+        loader = importlib.machinery.ExtensionFileLoader('_host', path)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader('_host', loader))
+        loader.exec_module(module)
+        load()
+        module.load(LIB_PATH, SubstationError)
+        _host = module
+    return _host
 
 
 def check(rc, what=''):

@@ -16,6 +16,7 @@ CSRC = os.path.join(HERE, 'csrc')
 OBJ = os.path.join(CSRC, 'build')
 LIB_DIR = os.path.join(HERE, 'lib')
 LIB = os.path.join(LIB_DIR, 'libsubstation_amd.so')
+HOST_LIB = os.path.join(LIB_DIR, '_host.so')       # the host side of a layer call (torch extension module)
 SOURCES = ['encoder.hip', 'k_rows.hip', 'k_elem.hip', 'k_cols.hip', 'k_lnbwd.hip', 'k_attn.hip', 'k_mha.hip', 'k_relayout.hip', 'k_probe.hip', 'k_gemm.hip']
 FLAGS = ['--offload-arch=gfx950', '-O3', '-std=c++17', '-fPIC', '-Wall', '-Wno-unused-function',
          # packed-fp32 VALU forms are switched off for every kernel of this library
@@ -42,6 +43,19 @@ def _run(cmd):
     return out
 
 
+def _build_host():
+    """The extension module takes its headers and libraries from the torch that is installed; no device code."""
+    import sysconfig
+    import torch
+    root = os.path.dirname(torch.__file__)
+    inc = [os.path.join(root, 'include'), os.path.join(root, 'include', 'torch', 'csrc', 'api', 'include'),
+           '/opt/rocm/include', sysconfig.get_paths()['include']]
+    return _run(['g++', '-O2', '-std=c++17', '-fPIC', '-shared', '-Wall', '-D__HIP_PLATFORM_AMD__=1', '-DUSE_ROCM=1',
+                 '-DTORCH_EXTENSION_NAME=_host', '-DTORCH_API_INCLUDE_EXTENSION_H', *['-I' + d for d in inc],
+                 os.path.join(CSRC, 'host.cpp'), '-o', HOST_LIB, '-L' + os.path.join(root, 'lib'), '-lc10', '-lc10_hip',
+                 '-ltorch_cpu', '-ltorch', '-ltorch_python', '-Wl,-rpath,' + os.path.join(root, 'lib')])
+
+
 def build(verbose=False, jobs=8):
     os.makedirs(OBJ, exist_ok=True)
     os.makedirs(LIB_DIR, exist_ok=True)
@@ -55,7 +69,9 @@ def build(verbose=False, jobs=8):
         return obj
 
     with ThreadPoolExecutor(max_workers=jobs) as ex:
+        host = ex.submit(_build_host)
         objs = list(ex.map(compile_one, SOURCES))
+        host.result()
     _run([hipcc, '--offload-arch=gfx950', '-shared', '-fPIC', *objs, '-o', LIB])
     return LIB
 

@@ -1,0 +1,253 @@
+// The host side of a layer call: tensors in, autograd node out, one call into the kernel library per pass.
+//
+// A training step of a small layer is as long as the host takes to issue it.  Written in Python (a torch.autograd.Function
+// with 37 torch.empty, 130 data_ptr and two ctypes calls per step) that was 240 to 480 us at B=2 L=128 E=768, of which
+// the library's own launches were 75; here a pass is one allocation for its intermediates, the launches, and a node that
+// the engine runs without taking the interpreter's lock.
+#include <dlfcn.h>
+
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/saved_variable.h>
+#include <torch/extension.h>
+
+#include "../../include/substation_amd.h"
+
+namespace py = pybind11;
+using torch::autograd::Node;
+using torch::autograd::SavedVariable;
+using torch::autograd::variable_list;
+
+namespace {
+
+// The kernel library, at the path the Python package has loaded it from.
+struct Lib {
+    decltype(&sub_last_error) last_error = nullptr;
+    decltype(&sub_set_stream) set_stream = nullptr;
+    decltype(&sub_get_option) get_option = nullptr;
+    decltype(&sub_attention_in_registers) attention_in_registers = nullptr;
+    decltype(&sub_encoder_forward) encoder_forward = nullptr;
+    decltype(&sub_encoder_backward) encoder_backward = nullptr;
+} lib;
+PyObject* g_error = nullptr;          // substation_amd._lib.SubstationError
+
+void load(const std::string& path, py::object error) {
+    void* so = dlopen(path.c_str(), RTLD_NOW | RTLD_LOCAL);
+    if (!so) throw std::runtime_error(std::string("substation_amd host: ") + dlerror());
+    auto get = [&](auto& fn, const char* name) {
+        fn = reinterpret_cast<std::decay_t<decltype(fn)>>(dlsym(so, name));
+        if (!fn) throw std::runtime_error(std::string("substation_amd host: the library has no ") + name);
+    };
+    get(lib.last_error, "sub_last_error");
+    get(lib.set_stream, "sub_set_stream");
+    get(lib.get_option, "sub_get_option");
+    get(lib.attention_in_registers, "sub_attention_in_registers");
+    get(lib.encoder_forward, "sub_encoder_forward");
+    get(lib.encoder_backward, "sub_encoder_backward");
+    g_error = error.release().ptr();
+}
+
+// An error of the library as the exception the Python binding raises for it; from any thread.
+[[noreturn]] void raise(const std::string& what, PyObject* type = nullptr) {
+    py::gil_scoped_acquire gil;
+    PyErr_SetString(type ? type : g_error, what.c_str());
+    python_error e;
+    e.persist();
+    throw e;
+}
+void check(int rc, const char* what) {
+    if (rc < 0) raise(std::string(what) + ": " + lib.last_error());
+}
+
+void use_current_stream(void* handle, c10::DeviceIndex device) {
+    check(lib.set_stream(handle, c10::hip::getCurrentHIPStream(device).stream()), "sub_set_stream");
+}
+
+// Sizes of a list of buffers that live side by side in one allocation, each from a multiple of 256 bytes on.
+struct Buffers {
+    std::vector<int64_t> offset;      // in halves
+    int64_t total = 0;
+    explicit Buffers(const std::vector<int64_t>& numels) {
+        for (int64_t n : numels) {
+            offset.push_back(total);
+            total += (n + 127) / 128 * 128;
+        }
+    }
+    void pointers(const at::Tensor& flat, std::vector<void*>& out) const {
+        auto* base = static_cast<char*>(flat.data_ptr());
+        for (int64_t o : offset) out.push_back(base + 2 * o);
+    }
+};
+
+struct EncoderLayer : std::enable_shared_from_this<EncoderLayer> {
+    void* handle;
+    py::object keep_alive;            // the Python object that owns `handle`
+    std::vector<int64_t> in_shape, out_shape;
+    std::vector<std::vector<int64_t>> param_shapes;
+    Buffers fwd, bwd;
+    bool persistent, need_registers, need_relu_gate;
+    // persistent: allocates (or finds) the two lists of tensors, given (which, tensor of the device)
+    py::object workspace;
+    std::vector<at::Tensor> kept_fwd, kept_bwd;
+    uint64_t generation = 0;
+
+    EncoderLayer(uintptr_t handle_, py::object owner, std::vector<int64_t> in, std::vector<int64_t> out,
+                 std::vector<std::vector<int64_t>> params, const std::vector<int64_t>& fwd_numels,
+                 const std::vector<int64_t>& bwd_numels, bool persistent_, bool need_registers_, bool need_relu_gate_,
+                 py::object workspace_)
+        : handle(reinterpret_cast<void*>(handle_)), keep_alive(std::move(owner)), in_shape(std::move(in)),
+          out_shape(std::move(out)), param_shapes(std::move(params)), fwd(fwd_numels), bwd(bwd_numels),
+          persistent(persistent_), need_registers(need_registers_), need_relu_gate(need_relu_gate_),
+          workspace(std::move(workspace_)) {}
+    ~EncoderLayer() {
+        if (!Py_IsInitialized()) { keep_alive.release(); workspace.release(); return; }
+        py::gil_scoped_acquire gil;
+        keep_alive = py::object();
+        workspace = py::object();
+    }
+
+    // A layer built with token buffers for what its path leaves alone must be on that path.
+    void check_compact() const {
+        int v = 0;
+        if (need_registers) {
+            check(lib.attention_in_registers(handle, &v), "sub_attention_in_registers");
+            if (!v)
+                raise("this Encoder was built with compact_attention=True but the attention kernels that keep the scores "
+                      "in registers are switched off", PyExc_RuntimeError);
+        }
+        check_relu_gate();
+    }
+    void check_relu_gate() const {
+        int v = 0;
+        if (!need_relu_gate) return;
+        check(lib.get_option(handle, SUB_OPT_RELU_FROM_OUTPUT, &v), "sub_get_option");
+        if (!v)
+            raise("this Encoder was built with compact_activation=True but the ReLU gate from the dropout output (option 6) "
+                  "is switched off: LIN1 and DROP2MASK would be written through 8-element buffers", PyExc_RuntimeError);
+    }
+    void keep(std::vector<at::Tensor>& list, const char* which, const at::Tensor& X) {
+        if (list.empty() || list[0].device() != X.device()) list = workspace(which, X).cast<std::vector<at::Tensor>>();
+    }
+
+    at::Tensor forward(const at::Tensor& X, const std::vector<at::Tensor>& params);
+};
+
+struct EncoderBackward : Node {
+    std::shared_ptr<EncoderLayer> layer;
+    std::vector<SavedVariable> saved;         // the parameters as the forward pass read them, then X
+    at::Tensor flat;                          // the forward intermediates (unless the layer keeps its own)
+    uint64_t generation = 0;
+
+    std::string name() const override { return "EncoderFunctionBackward"; }
+    void release_variables() override {
+        for (auto& s : saved) s.reset_data();
+        flat.reset();
+    }
+
+    variable_list apply(variable_list&& grads) override {
+        EncoderLayer& l = *layer;
+        if (l.persistent && generation != l.generation)
+            raise("persistent_workspace: forward() ran again before this backward pass; what it had saved has been "
+                  "overwritten", PyExc_RuntimeError);
+        l.check_relu_gate();
+        variable_list in;
+        in.reserve(saved.size());
+        for (auto& s : saved) in.push_back(s.unpack());
+        const at::Tensor& X = in.back();
+        const c10::DeviceGuard guard(X.device());
+        at::Tensor DY = grads[0].defined() ? grads[0].contiguous() : at::zeros(l.out_shape, X.options());
+        variable_list out;
+        out.reserve(1 + l.param_shapes.size());
+        const auto opt = X.options();
+        out.push_back(at::empty(l.in_shape, DY.options()));
+        for (const auto& s : l.param_shapes) out.push_back(at::empty(s, opt));
+        at::Tensor scratch;
+        std::vector<void*> p;
+        p.reserve(96);
+        p.push_back(DY.data_ptr());
+        for (size_t i = 1; i < out.size(); ++i) p.push_back(out[i].data_ptr());
+        if (l.persistent) {
+            for (const auto& t : l.kept_bwd) p.push_back(t.data_ptr());
+        } else {
+            scratch = at::empty({l.bwd.total}, opt);
+            l.bwd.pointers(scratch, p);
+        }
+        for (size_t i = 0; i + 1 < in.size(); ++i) p.push_back(in[i].data_ptr());
+        if (l.persistent) for (const auto& t : l.kept_fwd) p.push_back(t.data_ptr());
+        else l.fwd.pointers(flat, p);
+        p.push_back(X.data_ptr());
+        p.push_back(out[0].data_ptr());
+        use_current_stream(l.handle, X.device().index());
+        check(lib.encoder_backward(l.handle, p.data(), (int)p.size()), "encoder_backward");
+        return out;
+    }
+};
+
+at::Tensor EncoderLayer::forward(const at::Tensor& X_, const std::vector<at::Tensor>& params) {
+    if (!X_.is_cuda()) raise("Encoder.forward needs a tensor on the GPU", PyExc_RuntimeError);
+    if (X_.sizes() != at::IntArrayRef(in_shape)) {
+        std::ostringstream m;
+        m << "X has shape " << X_.sizes() << ", the configured input layout needs " << at::IntArrayRef(in_shape);
+        raise(m.str(), PyExc_ValueError);
+    }
+    check_compact();
+    const c10::DeviceGuard guard(X_.device());
+    bool grad = false;
+    if (at::GradMode::is_enabled()) {
+        grad = X_.requires_grad();
+        for (size_t i = 0; !grad && i < params.size(); ++i) grad = params[i].requires_grad();
+    }
+    at::Tensor X, Y, flat;
+    std::vector<at::Tensor> w;
+    std::vector<void*> p;
+    p.reserve(48);
+    {
+        at::NoGradGuard no_grad;
+        X = X_.contiguous();
+        w.reserve(params.size());
+        for (const auto& t : params) w.push_back(t.contiguous());
+        // same element count as X, shaped in the output's own dimension order
+        Y = at::empty(out_shape, X.options().requires_grad(false));
+        p.push_back(X.data_ptr());
+        for (const auto& t : w) p.push_back(t.data_ptr());
+        if (persistent) {
+            keep(kept_fwd, "forward_interm", X);
+            if (grad) keep(kept_bwd, "backward_interm", X);
+            for (const auto& t : kept_fwd) p.push_back(t.data_ptr());
+        } else {
+            flat = at::empty({fwd.total}, Y.options());
+            fwd.pointers(flat, p);
+        }
+        p.push_back(Y.data_ptr());
+    }
+    ++generation;
+    {
+        py::gil_scoped_release nogil;
+        use_current_stream(handle, X.device().index());
+        check(lib.encoder_forward(handle, p.data(), (int)p.size()), "encoder_forward");
+    }
+    if (grad) {
+        std::shared_ptr<EncoderBackward> node(new EncoderBackward(), torch::autograd::deleteNode);
+        node->set_next_edges(torch::autograd::collect_next_edges(X_, params));
+        node->layer = shared_from_this();
+        node->saved.reserve(w.size() + 1);
+        for (const auto& t : w) node->saved.emplace_back(t, false);
+        node->saved.emplace_back(X, false);
+        node->flat = flat;
+        node->generation = generation;
+        torch::autograd::set_history(Y, node);
+    }
+    return Y;
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_host, m) {
+    m.def("load", &load);
+    py::class_<EncoderLayer, std::shared_ptr<EncoderLayer>>(m, "EncoderLayer")
+        .def(py::init<uintptr_t, py::object, std::vector<int64_t>, std::vector<int64_t>, std::vector<std::vector<int64_t>>,
+                      const std::vector<int64_t>&, const std::vector<int64_t>&, bool, bool, bool, py::object>())
+        .def("forward", &EncoderLayer::forward);
+}

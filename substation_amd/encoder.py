@@ -13,6 +13,8 @@ the caller's current stream, and keyword-only extras exist: ``activation``
 """
 import ctypes
 import math
+import types
+import weakref
 
 import torch
 
@@ -25,6 +27,62 @@ _SUPPORTED_DTYPES = (torch.float16,)
 def causal_mask(seq_len, device='cuda', dtype=torch.float16):
     """-inf above the diagonal, 0 elsewhere (gen_attn_mask, substation/transformer.py:151-157)."""
     return torch.triu(torch.full((seq_len, seq_len), float('-inf'), dtype=dtype, device=device), diagonal=1)
+
+
+def _debug_function(module, in_shape, out_shape, workspace):
+    """The layer call of ``enable_debug=True``: every named tensor in a buffer of its own, captured after each pass."""
+    handle, lib, layouts = module._handle, module._handle.lib, module.layouts
+    n_params = len(layouts['params'])
+
+    def tensors(key, like):
+        if module.persistent_workspace:
+            return workspace(key, like)
+        return [torch.empty(tuple(module.sizes[s] for s in layout), device=like.device, dtype=module.torch_dtype)
+                for _, layout in layouts[key]]
+
+    def call(fn, device, args, what):
+        handle.set_stream(torch.cuda.current_stream(device).cuda_stream)
+        ptrs = (ctypes.c_void_p * len(args))(*(t.data_ptr() for t in args))
+        _lib.check(fn(handle.ptr, ptrs, len(args)), what)
+        torch.cuda.synchronize()
+
+    class EncoderFunction(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, X, *weights):
+            if not X.is_cuda:
+                raise RuntimeError('Encoder.forward needs a tensor on the GPU')
+            if tuple(X.shape) != in_shape:
+                raise ValueError(f"X has shape {tuple(X.shape)}, the configured input layout "
+                                 f"{layouts['input'][1]} needs {in_shape}")
+            X = X.contiguous()
+            Y = torch.empty(out_shape, device=X.device, dtype=X.dtype)
+            interm = tensors('forward_interm', X)
+            module._generation += 1
+            ctx.generation = module._generation
+            weights = [t.contiguous() for t in weights]
+            call(lib.sub_encoder_forward, X.device, [X, *weights, *interm, Y], 'encoder_forward')
+            ctx.save_for_backward(*weights, *interm, X)
+            for (name, _), t in zip(list(layouts['forward_interm']) + list(layouts['params']), interm + weights):
+                module.debug[name] = t.detach().cpu().numpy()
+            return Y
+
+        @staticmethod
+        def backward(ctx, DY):
+            if module.persistent_workspace and ctx.generation != module._generation:
+                raise RuntimeError('persistent_workspace: forward() ran again before this backward pass; '
+                                   'what it had saved has been overwritten')
+            DY = DY.contiguous()
+            DX = torch.empty(in_shape, device=DY.device, dtype=DY.dtype)
+            interm = tensors('backward_interm', DY)
+            grads = [torch.empty_like(t) for t in ctx.saved_tensors[:n_params]]
+            call(lib.sub_encoder_backward, DY.device, [DY, *grads, *interm, *ctx.saved_tensors, DX], 'encoder_backward')
+            for (name, _), t in zip(layouts['backward_interm'], interm):
+                module.debug[name] = t.detach().cpu().numpy()
+            for (name, _), t in zip(layouts['params'], grads):
+                module.debug['D' + name] = t.detach().cpu().numpy()
+            return (DX, *grads)
+
+    return EncoderFunction
 
 
 class Encoder(torch.nn.Module):
@@ -123,103 +181,38 @@ class Encoder(torch.nn.Module):
             compact.update({'LIN1': 8, 'DROP2MASK': 8})
         self.persistent_workspace = bool(persistent_workspace)
         self.canonical_state_dict = bool(canonical_state_dict)
+        self._generation = 0
         self._workspace = {}           # 'forward_interm' / 'backward_interm' -> tensors, when persistent
         self._shared_backward = None   # set by EncoderStack: one backward workspace for all layers
-        self._generation = 0
         handle = self._handle
-        lib = handle.lib
-        module = self
-        n_fwd = 1 + len(layouts['params']) + len(layouts['forward_interm']) + 1
-        n_bwd = 1 + len(layouts['params']) + len(layouts['backward_interm']) + (
-            len(layouts['params']) + len(layouts['forward_interm']) + 1) + 1
-        fwd_array = ctypes.c_void_p * n_fwd
-        bwd_array = ctypes.c_void_p * n_bwd
-
         in_shape = tuple(sizes[s] for s in layouts['input'][1])
         out_shape = tuple(sizes[s] for s in layouts['output'][1])
 
-        def _alloc(key, device):
-            return [torch.empty(*((compact[name],) if name in compact else tuple(sizes[s] for s in layout)),
-                                device=device, dtype=module.torch_dtype, requires_grad=False)
+        def _shapes(key):
+            return [(compact[name],) if name in compact else tuple(sizes[s] for s in layout)
                     for name, layout in layouts[key]]
 
-        def _workspace(key, device):
-            if not module.persistent_workspace:
-                return _alloc(key, device)
+        weak = weakref.ref(self)       # (the layer object below outlives no module: no cycle through native code)
+
+        def _workspace(key, like):
+            module = weak()
+            store = module._workspace
             if key == 'backward_interm' and module._shared_backward is not None:
                 store = module._shared_backward
-            else:
-                store = module._workspace
-            if key not in store or store[key][0].device != device:
-                store[key] = _alloc(key, device)
+            if key not in store or store[key][0].device != like.device:
+                store[key] = [torch.empty(shape, device=like.device, dtype=torch_dtype) for shape in _shapes(key)]
             return store[key]
 
-        class EncoderFunction(torch.autograd.Function):
-            @staticmethod
-            def forward(ctx, X, *weights):
-                if not X.is_cuda:
-                    raise RuntimeError('Encoder.forward needs a tensor on the GPU')
-                if tuple(X.shape) != in_shape:
-                    raise ValueError(f"X has shape {tuple(X.shape)}, the configured input layout "
-                                     f"{layouts['input'][1]} needs {in_shape}")
-                if module.compact_attention and not handle.attention_in_registers():
-                    raise RuntimeError('this Encoder was built with compact_attention=True but the attention '
-                                       'kernels that keep the scores in registers are switched off')
-                module._check_compact_activation()
-                dev = X.device
-                X = X.contiguous()
-                # same element count as X, shaped in the output's own dimension order
-                Y = torch.empty(out_shape, device=dev, dtype=X.dtype)
-                forward_intermediate = _workspace('forward_interm', dev)
-                module._generation += 1
-                ctx.generation = module._generation
-                weights_c = [t.contiguous() for t in weights]
-                handle.set_stream(torch.cuda.current_stream(dev).cuda_stream)
-                ptrs = fwd_array(X.data_ptr(), *(t.data_ptr() for t in weights_c),
-                                 *(t.data_ptr() for t in forward_intermediate), Y.data_ptr())
-                _lib.check(lib.sub_encoder_forward(handle.ptr, ptrs, n_fwd), 'encoder_forward')
-                ctx.save_for_backward(*weights_c, *forward_intermediate, X)
-
-                if module.enable_debug:
-                    torch.cuda.synchronize()
-                    for idx, (name, _) in enumerate(layouts['forward_interm']):
-                        module.debug[name] = forward_intermediate[idx].detach().cpu().numpy()
-                    for idx, (name, _) in enumerate(layouts['params']):
-                        module.debug[name] = weights[idx].detach().cpu().numpy()
-                return Y
-
-            @staticmethod
-            def backward(ctx, DY):
-                if module.persistent_workspace and ctx.generation != module._generation:
-                    raise RuntimeError('persistent_workspace: forward() ran again before this backward pass; '
-                                       'what it had saved has been overwritten')
-                module._check_compact_activation()
-                dev = DY.device
-                DY = DY.contiguous()
-                DX = torch.empty(in_shape, device=dev, dtype=DY.dtype)
-                backward_intermediate = _workspace('backward_interm', dev)
-                param_gradients = _alloc('params', dev)
-                handle.set_stream(torch.cuda.current_stream(dev).cuda_stream)
-                ptrs = bwd_array(DY.data_ptr(), *(t.data_ptr() for t in param_gradients),
-                                 *(t.data_ptr() for t in backward_intermediate),
-                                 *(t.data_ptr() for t in ctx.saved_tensors), DX.data_ptr())
-                _lib.check(lib.sub_encoder_backward(handle.ptr, ptrs, n_bwd), 'encoder_backward')
-
-                if module.enable_debug:
-                    torch.cuda.synchronize()
-                    for idx, (name, _) in enumerate(layouts['backward_interm']):
-                        module.debug[name] = backward_intermediate[idx].detach().cpu().numpy()
-                    for idx, (name, _) in enumerate(layouts['params']):
-                        module.debug['D' + name] = param_gradients[idx].detach().cpu().numpy()
-                return (DX, *param_gradients)
-
-        self.encoder_func = EncoderFunction
-
-    def _check_compact_activation(self):
-        if self.compact_activation and not self._handle.get_option(_lib.OPT_RELU_FROM_OUTPUT):
-            raise RuntimeError('this Encoder was built with compact_activation=True but the ReLU gate from '
-                               'the dropout output (option 6) is switched off: LIN1 and DROP2MASK would be '
-                               'written through 8-element buffers')
+        if enable_debug:
+            self._layer = None
+            self.encoder_func = _debug_function(self, in_shape, out_shape, _workspace)
+        else:
+            self._layer = _lib.host().EncoderLayer(
+                handle.ptr, handle, in_shape, out_shape, _shapes('params'),
+                [math.prod(s) for s in _shapes('forward_interm')], [math.prod(s) for s in _shapes('backward_interm')],
+                self.persistent_workspace, self.compact_attention, self.compact_activation, _workspace)
+            layer = self._layer
+            self.encoder_func = types.SimpleNamespace(apply=lambda X, *weights: layer.forward(X, weights))
 
     def _canonical_perm(self, name, layout):
         canon = _lay.CANONICAL[name]
@@ -305,6 +298,8 @@ class Encoder(torch.nn.Module):
     def forward(self, X):
         """Run the encoder.  X is in ``layouts['input'][1]`` order; the result is
         in ``layouts['output'][1]`` order."""
+        if self._layer is not None:
+            return self._layer.forward(X, self.params)
         return self.encoder_func.apply(X, *self.params)
 
 
