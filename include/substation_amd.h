@@ -181,9 +181,9 @@ int sub_set_attention_mask(void* handle, const void* attn_mask, const char* layo
 /* SUB_OPT_PAIR_PRODUCTS (default 1): in encoder_backward a data-gradient product
  * and the weight-gradient product next to it (encoder.cu:205-216 DLIN1_LINW1 and
  * DLINW1; :262-276 DXATT and DWKQV), which do not depend on one another, run as
- * one launch with their workgroups interleaved when both have about one 128x128
- * tile per CU: every CU then holds one workgroup of each and one runs while the
- * other waits.  Results are unchanged.  Profiling names: `dXlin1+dWlin1`,
+ * one launch, their tiles in one list, where that is expected to be faster than a
+ * launch each; a third product joins them on the same terms.  Results are unchanged
+ * to rounding.  Profiling names: `dXlin1+dWlin1`, `dXlin1+dWlin1+dWlin2`,
  * `dXQKV-fused+dWQKV-fused`. */
 #define SUB_OPT_PAIR_PRODUCTS 5
 /* SUB_OPT_RELU_FROM_OUTPUT (default 1).  ReLU layers: the backward pass reads

@@ -600,6 +600,7 @@ void run_gemm(Handle& h, int id, const void* A, const void* B, void* C, const ch
     ProfScope ps(h, name);
     const GemmPlan& p = h.gemm[id];
     GemmEpilogue ep;
+    ep.any_split = id >= G_DXLIN2 || id == G_DXQKV_RESID;      // the backward pass
     if (addend) {
         ep.bias = (const half_t*)addend; ep.sbM = p.sM; ep.sbN = p.sN;
         for (int i = 0; i < 3; ++i) ep.sbb[i] = p.sb[i];
@@ -648,17 +649,6 @@ bool pair_takes_third(Handle& h, int id1, const void* A1, const void* B1, void* 
     return gemm_pair_takes_third(p1.shape, (const half_t*)A1, (const half_t*)B1, (half_t*)C1,
                                  addend_epilogue(p1, addend1), p2.shape, (const half_t*)A2, (const half_t*)B2,
                                  (half_t*)C2, GemmEpilogue{}, h.gws, h.gws_floats, third);
-}
-
-// Would run_gemm_pair run these two products as one launch?
-bool pair_ok(Handle& h, int id1, const void* A1, const void* B1, void* C1, const void* addend1, int id2,
-             const void* A2, const void* B2, void* C2) {
-    if (!h.pair_products) return false;
-    const GemmPlan& p1 = h.gemm[id1];
-    const GemmPlan& p2 = h.gemm[id2];
-    ensure_gws(h, h.gws_need);
-    return gemm_pair_ok(p1.shape, (const half_t*)A1, (const half_t*)B1, (half_t*)C1, addend_epilogue(p1, addend1),
-                        p2.shape, (const half_t*)A2, (const half_t*)B2, (half_t*)C2, GemmEpilogue{}, h.gws, h.gws_floats);
 }
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -1276,14 +1266,17 @@ void backward(Handle& h, const BwdPtrs& t0) {
     } else {
         run_gemm(h, G_DXLIN2, D[DLIN2], W[LINW2], D[DDROP2], "dXlin2");
     }
-    // With many tokens the data gradient of linear1 has too many tiles to share a launch with the weight
-    // gradient next to it; the two weight gradients of the feed-forward block -- one tile per CU each, their
-    // contraction as long as the token count -- then run as a pair of their own on 256 x 128 tiles (a quarter
-    // less operand traffic from L2 than alone on 128 x 128 tiles), dWlin2 waiting for dWlin1's operands.
-    const bool pair_weights = !pair_ok(h, G_DXLIN1, D[DLIN1], W[LINW1], D[DLIN1_LINW1], nullptr, G_DWLIN1, D[DLIN1], F[SB1],
-                                       DW[LINW1]) &&
-                              pair_ok(h, G_DWLIN1, D[DLIN1], F[SB1], DW[LINW1], nullptr, G_DWLIN2, D[DLIN2], F[DROP2], DW[LINW2]);
-    if (!pair_weights) run_gemm(h, G_DWLIN2, D[DLIN2], F[DROP2], DW[LINW2], "dWlin2");
+    // dWlin2 waits for the launch of the pair behind it where its tiles fill the rounds of that one
+    PairThird dwlin2;
+    bool dwlin2_later = false;
+    {
+        const GemmPlan& p3 = h.gemm[G_DWLIN2];
+        dwlin2.shape = &p3.shape; dwlin2.A = (const half_t*)D[DLIN2]; dwlin2.B = (const half_t*)F[DROP2];
+        dwlin2.C = (half_t*)DW[LINW2]; dwlin2.alpha = p3.alpha;
+        dwlin2_later = pair_takes_third(h, G_DXLIN1, D[DLIN1], W[LINW1], D[DLIN1_LINW1], nullptr, G_DWLIN1, D[DLIN1], F[SB1],
+                                        DW[LINW1], dwlin2);
+    }
+    if (!dwlin2_later) run_gemm(h, G_DWLIN2, D[DLIN2], F[DROP2], DW[LINW2], "dWlin2");
     if (!fuse_bdrlb) {
         ProfScope ps(h, "bdrlb");
         if (relu_from_output(h))
@@ -1292,14 +1285,9 @@ void backward(Handle& h, const BwdPtrs& t0) {
             op_bdrlb(h, D[DDROP2], h.lb[DDROP2], F[DROP2MASK], h.lf[DROP2MASK], F[LIN1], h.lf[LIN1],
                      D[DLIN1], h.lb[DLIN1], DW[LINB1]);
     }
-    if (pair_weights) {
-        run_gemm(h, G_DXLIN1, D[DLIN1], W[LINW1], D[DLIN1_LINW1], "dXlin1");
-        run_gemm_pair(h, G_DWLIN1, D[DLIN1], F[SB1], DW[LINW1], "dWlin1", nullptr,
-                      G_DWLIN2, D[DLIN2], F[DROP2], DW[LINW2], "dWlin2", "dWlin1+dWlin2");
-    } else {
-        run_gemm_pair(h, G_DXLIN1, D[DLIN1], W[LINW1], D[DLIN1_LINW1], "dXlin1", nullptr,
-                      G_DWLIN1, D[DLIN1], F[SB1], DW[LINW1], "dWlin1", "dXlin1+dWlin1");
-    }
+    run_gemm_pair(h, G_DXLIN1, D[DLIN1], W[LINW1], D[DLIN1_LINW1], "dXlin1", nullptr, G_DWLIN1, D[DLIN1], F[SB1], DW[LINW1],
+                  "dWlin1", dwlin2_later ? "dXlin1+dWlin1+dWlin2" : "dXlin1+dWlin1", nullptr, dwlin2_later ? &dwlin2 : nullptr);
+    if (dwlin2_later && !dwlin2.taken) run_gemm(h, G_DWLIN2, D[DLIN2], F[DROP2], DW[LINW2], "dWlin2");
     fused = false;
     if (h.fuse_ln_backward) {
         ProfScope ps(h, "ebsb+blnrd2+baob");

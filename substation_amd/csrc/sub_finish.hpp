@@ -10,8 +10,9 @@ constexpr int kFinishThreads = 256;      // threads of a workgroup that runs fin
 
 // One workgroup of kFinishThreads threads: 32 features x 8 slices of the partial
 // rows, the slices combined through `red` (8 x 33 floats of LDS).  bx counts the
-// 32-feature groups of job j; groups past its end do nothing.
-__device__ __forceinline__ void finish_block(const FinishJob& j, long bx, float (*red)[33]) {
+// 32-feature groups of job j (a FinishJob, wherever it lies); groups past its end do nothing.
+template <typename Job>
+__device__ __forceinline__ void finish_block(Job& j, long bx, float (*red)[33]) {
     const int fl = threadIdx.x & 31, sl = threadIdx.x >> 5;
     const long idx = bx * 32 + fl;
     const bool ok = idx < (long)j.ns * j.nbatch * j.R;

@@ -245,6 +245,9 @@ struct GemmEpilogue {
     // keep ? gelu'(gate) * x : 0 with `gate` the pre-activation values and gate_bits those keep bits (required).
     int act = ACT_RELU;
     half_t* pre_out = nullptr;
+    // the contraction of a small output may be split in as many parts as is fastest; otherwise their number, and with it the
+    // order of the sums, depends on the shape alone (one unit of the last place of a pre-activation decides a ReLU's gate)
+    bool any_split = false;
 };
 // Work that needs no memory path, offered to a product whose 256x256 tiles leave CUs idle: the
 // keep bits of the attention dropout (attention_keep_word) for the first `tiles_done` key tiles of
@@ -265,11 +268,8 @@ void launch_gemm(const GemmShape& g, const half_t* A, const half_t* B, half_t* C
 // Can launch_gemm apply ep.relu_dropout to this product?  Only the asynchronous kernel with
 // 256x256 tiles does, on a single dense row-major output.
 bool gemm_relu_dropout_ok(const GemmShape& g, const void* A, const void* B, const void* C, const GemmEpilogue& ep);
-// A third product offered to launch_gemm_pair: taken (and `taken` set) when its
-// whole 128x128 tiles fit into the places the pair leaves free on the CUs, it is
-// read the way the pair's second product is and its contraction is no longer
-// than theirs; the launch then takes about as long as without it.  Its
-// contraction is never split.
+// A third product offered to launch_gemm_pair: taken (and `taken` set) when its tiles in that launch are
+// expected to cost less than a launch of its own.
 struct PairThird {
     const GemmShape* shape = nullptr;
     const half_t* A = nullptr;
@@ -278,19 +278,14 @@ struct PairThird {
     float alpha = 1.f;
     bool taken = false;
 };
-// Two independent contractions in one launch, their workgroups interleaved so that
-// every CU works on both at once.  Returns false, having launched nothing, when
-// the pair does not qualify (then call launch_gemm for each).  `tail` (optional):
+// Two independent contractions in one launch, each split as suits it (see GemmEpilogue::any_split).  Returns false,
+// having launched nothing, when the pair does not qualify (then call launch_gemm for each).  `tail` (optional):
 // deferred column sums of EARLIER launches, finished by extra workgroups of this
 // launch; tail->n is set to 0 when they were taken, else it is left as it was.
 bool launch_gemm_pair(const GemmShape& g1, const half_t* A1, const half_t* B1, half_t* C1, float alpha1,
                       const GemmEpilogue& ep1, const GemmShape& g2, const half_t* A2, const half_t* B2,
                       half_t* C2, float alpha2, const GemmEpilogue& ep2, hipStream_t st, float* ws = nullptr,
                       size_t ws_floats = 0, FinishJobs* tail = nullptr, PairThird* third = nullptr);
-// Would launch_gemm_pair take these two products as one launch?
-bool gemm_pair_ok(const GemmShape& g1, const half_t* A1, const half_t* B1, half_t* C1, const GemmEpilogue& ep1,
-                  const GemmShape& g2, const half_t* A2, const half_t* B2, half_t* C2, const GemmEpilogue& ep2,
-                  float* ws, size_t ws_floats);
 // Would launch_gemm_pair with these two products take `third` along?
 bool gemm_pair_takes_third(const GemmShape& g1, const half_t* A1, const half_t* B1, half_t* C1,
                            const GemmEpilogue& ep1, const GemmShape& g2, const half_t* A2, const half_t* B2,

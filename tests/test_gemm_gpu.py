@@ -143,3 +143,50 @@ def test_two_contractions_in_one_call(B, L, H, E, expect_pair):
         d = {k: to_layout(mk(k, 0.5), k, k) for k in ('BJU', 'UI', 'BJI')}
         assert o.einsum_pair((d['BJU'], 'BJU', d['UI'], 'UI', nan('BJI'), 'BJI'),
                              (d['BJU'], 'BJU', d['BJI'], 'BJI', nan('UI'), 'UI'))
+
+
+@pytest.mark.parametrize('L,E,U', [(8, 8, 8), (72, 136, 200), (64, 64, 3072), (1000, 72, 776), (2616, 128, 776), (1928, 72, 2056)])
+def test_tiles_with_remainders(L, E, U):
+    """Every operand orientation on tiles of each size (64 x 64 for few outputs up to 256 x 128 for many), with
+    remainders in m, n and k; a bias row and a whole addend."""
+    from substation_amd.ops import Ops
+    o = Ops(1, L, 1, E, intermediate_size=U)
+    sz = o.sizes
+    rng = np.random.default_rng(L)
+    mk = lambda lay: h16(rng.normal(size=tuple(sz[d] for d in lay)))
+    for las, lbs, lc, bias in ((('BJI', 'IBJ'), ('UI', 'IU'), 'BJU', 'U'), (('BJU', 'UBJ'), ('UI', 'IU'), 'BJI', 'BJI')):
+        for la in las:
+            for lb in lbs:
+                A, Bm, T = mk(la), mk(lb), mk(bias)
+                want = np.einsum(f'{la},{lb}->{lc}'.lower(), A, Bm)
+                C = torch.full(tuple(sz[d] for d in lc), float('nan'), dtype=torch.float16, device='cuda')
+                assert o.handle.classify(la, lb, lc)['kernel'] == 1
+                o.einsum(to_layout(A, la, la), la, to_layout(Bm, lb, lb), lb, C, lc)
+                torch.cuda.synchronize()
+                assert_close(from_layout(C, lc, lc), want, name=f'{la},{lb}->{lc}')
+                o.einsum(to_layout(A, la, la), la, to_layout(Bm, lb, lb), lb, C, lc, addend=to_layout(T, bias, bias), l_addend=bias)
+                torch.cuda.synchronize()
+                assert_close(from_layout(C, lc, lc), want + T, name=f'{la},{lb}->{lc} + {bias}')
+
+
+@pytest.mark.parametrize('B,L,H,E,U', [(1, 72, 3, 192, 776), (2, 1000, 2, 128, 512), (1, 2616, 12, 768, 776), (1, 2616, 12, 768, 3072)])
+def test_products_sharing_a_launch(B, L, H, E, U):
+    """A data gradient with a residual and a weight gradient as one list of tiles: remainders, several
+    batches, contractions of unequal length, and more tiles than the chip takes at once."""
+    from substation_amd.ops import Ops
+    o = Ops(B, L, H, E, intermediate_size=U)
+    sz = o.sizes
+    g = torch.Generator(device='cuda').manual_seed(L)
+    mk = lambda lay: torch.randn(tuple(sz[d] for d in lay), generator=g, device='cuda').half() * 0.5
+    nan = lambda lay: torch.full(tuple(sz[d] for d in lay), float('nan'), dtype=torch.float16, device='cuda')
+    for (la1, lb1, lc1, lt1), (la2, lb2, lc2) in (
+            (('BJU', 'UI', 'BJI', 'BJI'), ('BJU', 'BJI', 'UI')),
+            (('QHPI', 'QBJHP', 'BJI', 'BJI'), ('QBJHP', 'BJI', 'QHPI'))):
+        d = {lay: mk(lay) for lay in {la1, lb1, la2, lb2}}
+        T, C1, C2 = mk(lt1), nan(lc1), nan(lc2)
+        o.einsum_pair((d[la1], la1, d[lb1], lb1, C1, lc1, T, lt1), (d[la2], la2, d[lb2], lb2, C2, lc2))
+        torch.cuda.synchronize()
+        w1 = np.einsum(f'{la1},{lb1}->{lc1}'.lower(), d[la1].double().cpu(), d[lb1].double().cpu(), optimize=True) + T.double().cpu().numpy()
+        w2 = np.einsum(f'{la2},{lb2}->{lc2}'.lower(), d[la2].double().cpu(), d[lb2].double().cpu(), optimize=True)
+        assert_close(C1.double().cpu().numpy(), w1, name=f'{la1},{lb1}->{lc1}')
+        assert_close(C2.double().cpu().numpy(), w2, name=f'{la2},{lb2}->{lc2}')
