@@ -639,16 +639,27 @@ void run_gemm_pair(Handle& h, int id1, const void* A1, const void* B1, void* C1,
     run_gemm(h, id2, A2, B2, C2, name2);
 }
 
-// Would run_gemm_pair with these arguments take `third` into its launch?
-bool pair_takes_third(Handle& h, int id1, const void* A1, const void* B1, void* C1, const void* addend1, int id2,
-                      const void* A2, const void* B2, void* C2, const PairThird& third) {
-    if (!h.pair_products) return false;
+// Where a second weight gradient goes that is ready before a data gradient (1) and its weight gradient (2): into their
+// launch, into one with (2) where (1) shares no launch with either, or into one of its own.  Under weight orders that have
+// every operand of (1) contiguous along k (the shipped configuration of 96 sequences of 128) it never shares one: there
+// dWlin1 + dWlin2 as 256 tiles of 256 x 128 take 172 us where they took 2 x 111 as 256 of 128 x 128 each, dWQKV + dWout 123
+// where dWQKV took 104 and dWout 38 in dXout's launch.
+enum ThirdPlace { THIRD_ALONE, THIRD_IN_PAIR, THIRD_WITH_SECOND };
+ThirdPlace place_third(Handle& h, int id1, const void* A1, const void* B1, void* C1, const void* addend1, int id2,
+                       const void* A2, const void* B2, void* C2, const PairThird& third) {
+    if (!h.pair_products) return THIRD_ALONE;
     const GemmPlan& p1 = h.gemm[id1];
     const GemmPlan& p2 = h.gemm[id2];
     ensure_gws(h, h.gws_need);
-    return gemm_pair_takes_third(p1.shape, (const half_t*)A1, (const half_t*)B1, (half_t*)C1,
-                                 addend_epilogue(p1, addend1), p2.shape, (const half_t*)A2, (const half_t*)B2,
-                                 (half_t*)C2, GemmEpilogue{}, h.gws, h.gws_floats, third);
+    const half_t* a1 = (const half_t*)A1; const half_t* b1 = (const half_t*)B1;
+    const half_t* a2 = (const half_t*)A2; const half_t* b2 = (const half_t*)B2;
+    const GemmEpilogue e1 = addend_epilogue(p1, addend1), e2{};
+    if (gemm_pair_takes_third(p1.shape, a1, b1, (half_t*)C1, e1, p2.shape, a2, b2, (half_t*)C2, e2, h.gws, h.gws_floats, third))
+        return THIRD_IN_PAIR;
+    if (gemm_pair_ok(p1.shape, a1, b1, (half_t*)C1, e1, p2.shape, a2, b2, (half_t*)C2, e2, h.gws, h.gws_floats))
+        return THIRD_ALONE;
+    return gemm_pair_ok(p2.shape, a2, b2, (half_t*)C2, e2, *third.shape, third.A, third.B, third.C, e2, h.gws, h.gws_floats)
+               ? THIRD_WITH_SECOND : THIRD_ALONE;
 }
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -1268,15 +1279,15 @@ void backward(Handle& h, const BwdPtrs& t0) {
     }
     // dWlin2 waits for the launch of the pair behind it where its tiles fill the rounds of that one
     PairThird dwlin2;
-    bool dwlin2_later = false;
+    ThirdPlace dwlin2_at = THIRD_ALONE;
     {
         const GemmPlan& p3 = h.gemm[G_DWLIN2];
         dwlin2.shape = &p3.shape; dwlin2.A = (const half_t*)D[DLIN2]; dwlin2.B = (const half_t*)F[DROP2];
         dwlin2.C = (half_t*)DW[LINW2]; dwlin2.alpha = p3.alpha;
-        dwlin2_later = pair_takes_third(h, G_DXLIN1, D[DLIN1], W[LINW1], D[DLIN1_LINW1], nullptr, G_DWLIN1, D[DLIN1], F[SB1],
-                                        DW[LINW1], dwlin2);
+        dwlin2_at = place_third(h, G_DXLIN1, D[DLIN1], W[LINW1], D[DLIN1_LINW1], nullptr, G_DWLIN1, D[DLIN1], F[SB1],
+                                DW[LINW1], dwlin2);
     }
-    if (!dwlin2_later) run_gemm(h, G_DWLIN2, D[DLIN2], F[DROP2], DW[LINW2], "dWlin2");
+    if (dwlin2_at == THIRD_ALONE) run_gemm(h, G_DWLIN2, D[DLIN2], F[DROP2], DW[LINW2], "dWlin2");
     if (!fuse_bdrlb) {
         ProfScope ps(h, "bdrlb");
         if (relu_from_output(h))
@@ -1285,9 +1296,16 @@ void backward(Handle& h, const BwdPtrs& t0) {
             op_bdrlb(h, D[DDROP2], h.lb[DDROP2], F[DROP2MASK], h.lf[DROP2MASK], F[LIN1], h.lf[LIN1],
                      D[DLIN1], h.lb[DLIN1], DW[LINB1]);
     }
-    run_gemm_pair(h, G_DXLIN1, D[DLIN1], W[LINW1], D[DLIN1_LINW1], "dXlin1", nullptr, G_DWLIN1, D[DLIN1], F[SB1], DW[LINW1],
-                  "dWlin1", dwlin2_later ? "dXlin1+dWlin1+dWlin2" : "dXlin1+dWlin1", nullptr, dwlin2_later ? &dwlin2 : nullptr);
-    if (dwlin2_later && !dwlin2.taken) run_gemm(h, G_DWLIN2, D[DLIN2], F[DROP2], DW[LINW2], "dWlin2");
+    if (dwlin2_at == THIRD_WITH_SECOND) {
+        run_gemm(h, G_DXLIN1, D[DLIN1], W[LINW1], D[DLIN1_LINW1], "dXlin1");
+        run_gemm_pair(h, G_DWLIN1, D[DLIN1], F[SB1], DW[LINW1], "dWlin1", nullptr, G_DWLIN2, D[DLIN2], F[DROP2], DW[LINW2],
+                      "dWlin2", "dWlin1+dWlin2");
+    } else {
+        const bool later = dwlin2_at == THIRD_IN_PAIR;
+        run_gemm_pair(h, G_DXLIN1, D[DLIN1], W[LINW1], D[DLIN1_LINW1], "dXlin1", nullptr, G_DWLIN1, D[DLIN1], F[SB1], DW[LINW1],
+                      "dWlin1", later ? "dXlin1+dWlin1+dWlin2" : "dXlin1+dWlin1", nullptr, later ? &dwlin2 : nullptr);
+        if (later && !dwlin2.taken) run_gemm(h, G_DWLIN2, D[DLIN2], F[DROP2], DW[LINW2], "dWlin2");
+    }
     fused = false;
     if (h.fuse_ln_backward) {
         ProfScope ps(h, "ebsb+blnrd2+baob");
@@ -1319,17 +1337,17 @@ void backward(Handle& h, const BwdPtrs& t0) {
     // when the last pair of products of the pass has room for its tiles it runs there,
     // unsplit, and dXout runs alone here.
     PairThird dwout;
-    bool dwout_later = false;
+    ThirdPlace dwout_at = THIRD_ALONE;
     if (h.finish_in_pair && attn_fused) {
         const GemmPlan& p3 = h.gemm[G_DWOUT];
         dwout.shape = &p3.shape; dwout.A = (const half_t*)F[GAMMA]; dwout.B = (const half_t*)D[DATT];
         dwout.C = (half_t*)DW[WO]; dwout.alpha = p3.alpha;
-        dwout_later = fuse_dx ? pair_takes_third(h, G_DXQKV_RESID, W[WKQV], D[DKKQQVV], t.DX, D[DRESID1], G_DWQKV,
-                                                 t.X, D[DKKQQVV], DW[WKQV], dwout)
-                              : pair_takes_third(h, G_DXQKV, W[WKQV], D[DKKQQVV], D[DXATT], nullptr, G_DWQKV, t.X,
-                                                 D[DKKQQVV], DW[WKQV], dwout);
+        dwout_at = fuse_dx ? place_third(h, G_DXQKV_RESID, W[WKQV], D[DKKQQVV], t.DX, D[DRESID1], G_DWQKV,
+                                         t.X, D[DKKQQVV], DW[WKQV], dwout)
+                           : place_third(h, G_DXQKV, W[WKQV], D[DKKQQVV], D[DXATT], nullptr, G_DWQKV, t.X,
+                                         D[DKKQQVV], DW[WKQV], dwout);
     }
-    if (dwout_later)
+    if (dwout_at != THIRD_ALONE)
         run_gemm(h, G_DXOUT, W[WO], D[DATT], D[DGAMMA], "dXout");
     else
         run_gemm_pair(h, G_DXOUT, W[WO], D[DATT], D[DGAMMA], "dXout", nullptr,
@@ -1386,17 +1404,25 @@ void backward(Handle& h, const BwdPtrs& t0) {
     // their own launch when every producer of those sums has been launched by now
     // (baib below would add one more).
     FinishJobs* tail = h.deferring && attn_bias && h.finish_in_pair ? &h.deferred : nullptr;
-    PairThird* third = dwout_later ? &dwout : nullptr;
-    const char* last_name = dwout_later ? "dXQKV-fused+dWQKV-fused+dWout" : "dXQKV-fused+dWQKV-fused";
-    if (fuse_dx) {
-        // DX = WKQV.DKKQQVV + DRESID1 in one pass; DXATT is not written
-        run_gemm_pair(h, G_DXQKV_RESID, W[WKQV], D[DKKQQVV], t.DX, "dXQKV-fused", D[DRESID1],
-                      G_DWQKV, t.X, D[DKKQQVV], DW[WKQV], "dWQKV-fused", last_name, tail, third);
+    if (dwout_at == THIRD_WITH_SECOND) {
+        run_gemm(h, fuse_dx ? G_DXQKV_RESID : G_DXQKV, W[WKQV], D[DKKQQVV], fuse_dx ? t.DX : D[DXATT], "dXQKV-fused",
+                 fuse_dx ? D[DRESID1] : nullptr);
+        run_gemm_pair(h, G_DWQKV, t.X, D[DKKQQVV], DW[WKQV], "dWQKV-fused", nullptr, G_DWOUT, F[GAMMA], D[DATT], DW[WO], "dWout",
+                      "dWQKV-fused+dWout", tail);
     } else {
-        run_gemm_pair(h, G_DXQKV, W[WKQV], D[DKKQQVV], D[DXATT], "dXQKV-fused", nullptr,
-                      G_DWQKV, t.X, D[DKKQQVV], DW[WKQV], "dWQKV-fused", last_name, tail, third);
+        const bool later = dwout_at == THIRD_IN_PAIR;
+        PairThird* third = later ? &dwout : nullptr;
+        const char* last_name = later ? "dXQKV-fused+dWQKV-fused+dWout" : "dXQKV-fused+dWQKV-fused";
+        if (fuse_dx) {
+            // DX = WKQV.DKKQQVV + DRESID1 in one pass; DXATT is not written
+            run_gemm_pair(h, G_DXQKV_RESID, W[WKQV], D[DKKQQVV], t.DX, "dXQKV-fused", D[DRESID1],
+                          G_DWQKV, t.X, D[DKKQQVV], DW[WKQV], "dWQKV-fused", last_name, tail, third);
+        } else {
+            run_gemm_pair(h, G_DXQKV, W[WKQV], D[DKKQQVV], D[DXATT], "dXQKV-fused", nullptr,
+                          G_DWQKV, t.X, D[DKKQQVV], DW[WKQV], "dWQKV-fused", last_name, tail, third);
+        }
+        if (later && !dwout.taken) run_gemm(h, G_DWOUT, F[GAMMA], D[DATT], DW[WO], "dWout");
     }
-    if (dwout_later && !dwout.taken) run_gemm(h, G_DWOUT, F[GAMMA], D[DATT], DW[WO], "dWout");
     if (!attn_bias) {
         ProfScope ps(h, "baib");
         op_baib(h, D[DKKQQVV], h.lb[DKKQQVV], DW[BKQV], h.lp[BKQV]);

@@ -793,6 +793,15 @@ bool pair_select(const GemmShape* const sh[2], const Canon cin[2], float* ws, si
 
 }  // namespace
 
+bool gemm_pair_ok(const GemmShape& s1, const half_t* A1, const half_t* B1, half_t* C1, const GemmEpilogue& ep1,
+                  const GemmShape& s2, const half_t* A2, const half_t* B2, half_t* C2, const GemmEpilogue& ep2,
+                  float* ws, size_t ws_floats) {
+    const GemmShape* sh[2] = {&s1, &s2};
+    const Canon c[2] = {canonicalise(s1, A1, B1, C1, 1.f, ep1), canonicalise(s2, A2, B2, C2, 1.f, ep2)};
+    PairSel sel;
+    return pair_select(sh, c, ws, ws_floats, nullptr, sel);
+}
+
 bool gemm_pair_takes_third(const GemmShape& s1, const half_t* A1, const half_t* B1, half_t* C1,
                            const GemmEpilogue& ep1, const GemmShape& s2, const half_t* A2, const half_t* B2,
                            half_t* C2, const GemmEpilogue& ep2, float* ws, size_t ws_floats,

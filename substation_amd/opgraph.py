@@ -40,6 +40,7 @@ OPERATORS = [
     # dWlin2 in the same launch where its tiles fill the rounds of that one
     ('dXlin1+dWlin1+dWlin2', 'bwd', ('DLIN1', 'LINW1', 'DLIN1_LINW1', 'SB1', 'DLIN2', 'DROP2', 'LINW2')),
     ('dXlin1', 'bwd', ('DLIN1', 'LINW1', 'DLIN1_LINW1')),
+    ('dWlin1+dWlin2', 'bwd', ('DLIN1', 'SB1', 'LINW1', 'DLIN2', 'DROP2', 'LINW2')),     # where dXlin1 shares no launch
     ('dWlin1', 'bwd', ('DLIN1', 'SB1', 'LINW1')),
     ('ebsb+blnrd2+baob', 'bwd', ('LN1', 'DRESID2', 'DLIN1_LINW1', 'DLIN2', 'DLN1', 'LN1STD', 'LN1DIFF',
                                  'DROP1MASK', 'DRESID1', 'DATT')),
@@ -62,6 +63,7 @@ OPERATORS = [
     ('dXQKV-fused+dWQKV-fused+dWout', 'bwd', ('WKQV', 'DKKQQVV', 'DXATT', 'DRESID1', 'X', 'GAMMA', 'DATT', 'WO')),
     ('dXQKV-fused+dWQKV-fused', 'bwd', ('WKQV', 'DKKQQVV', 'DXATT', 'DRESID1', 'X')),
     ('dXQKV-fused', 'bwd', ('WKQV', 'DKKQQVV', 'DXATT', 'DRESID1', 'X')),
+    ('dWQKV-fused+dWout', 'bwd', ('X', 'DKKQQVV', 'WKQV', 'GAMMA', 'DATT', 'WO')),
     ('dWQKV-fused', 'bwd', ('X', 'DKKQQVV', 'WKQV')),
     ('baib', 'bwd', ('DKKQQVV', 'BKQV')),
     ('bei', 'bwd', ('DXATT', 'DRESID1', 'X')),
@@ -77,11 +79,12 @@ OP_TENSORS = {name: tensors for name, _, tensors in OPERATORS}
 ALTERNATIVES = [
     ('QKV-fused', 'aib'),
     # dWout runs inside the last launch of the pass when that has room for its tiles
-    ('dXQKV-fused+dWQKV-fused+dWout', 'dXQKV-fused+dWQKV-fused', 'dXQKV-fused', 'dWQKV-fused', 'bei',
-     'dXout+dWout', 'dXout', 'dWout', 'colfinish'),
+    ('dXQKV-fused+dWQKV-fused+dWout', 'dXQKV-fused+dWQKV-fused', 'dXQKV-fused',
+     'dWQKV-fused+dWout', 'dWQKV-fused', 'bei', 'dXout+dWout', 'dXout', 'dWout', 'colfinish'),
     ('lin1+bad', 'lin1', 'bad'),
     # (dWlin2 may wait for the launch of the pair behind it)
-    ('dXlin2+bdrlb', 'dXlin2', 'bdrlb', 'dXlin1+dWlin1+dWlin2', 'dXlin1+dWlin1', 'dXlin1', 'dWlin1', 'dWlin2'),
+    ('dXlin2+bdrlb', 'dXlin2', 'bdrlb', 'dXlin1+dWlin1+dWlin2', 'dXlin1+dWlin1', 'dXlin1', 'dWlin1+dWlin2',
+     'dWlin1', 'dWlin2'),
     ('attention', 'QKT+softmax', 'QKT', 'softmax', 'gamma'),
     ('attention-bwd-dQ', 'attention-bwd-dKdV', 'dX2gamma', 'dX1gamma+bs', 'dX1gamma', 'bs', 'dX1QKT', 'dX2QKT',
      'baib'),
