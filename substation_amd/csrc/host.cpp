@@ -2,15 +2,20 @@
 //
 // A training step of a small layer is as long as the host takes to issue it.  Written in Python (a torch.autograd.Function
 // with 37 torch.empty, 130 data_ptr and two ctypes calls per step) that was 240 to 480 us at B=2 L=128 E=768, of which
-// the library's own launches were 75; here a pass is one allocation for its intermediates, the launches, and a node that
-// the engine runs without taking the interpreter's lock.
+// the library's own launches were 75; here a pass is a few allocations for its intermediates, the launches, and a node
+// that the engine runs without taking the interpreter's lock.
+#include <algorithm>
 #include <dlfcn.h>
 
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/autograd/variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/extension.h>
 
 #include "../../include/substation_amd.h"
@@ -65,21 +70,46 @@ void use_current_stream(void* handle, c10::DeviceIndex device) {
     check(lib.set_stream(handle, c10::hip::getCurrentHIPStream(device).stream()), "sub_set_stream");
 }
 
-// Sizes of a list of buffers that live side by side in one allocation, each from a multiple of 256 bytes on.
+// A list of buffers, side by side in allocations of up to 32 MiB (a larger buffer has one of its own), each from a multiple
+// of 256 bytes on.  Not all of them in one: torch's allocator had to ask the device for a block of that size again
+// wherever a program had since put tensors into the one it had given back, 1 ms and more on a layer's first pass at
+// B=8 L=512 E=1024.  Not one for each: 37 per training step took 0.2 ms there where blocks had to be split and joined.
 struct Buffers {
-    std::vector<int64_t> offset;      // in halves
-    int64_t total = 0;
+    static constexpr int64_t kMost = 16 << 20;    // halves
+    std::vector<std::pair<int, int64_t>> where;   // allocation, offset in halves
+    std::vector<int64_t> sizes;                   // of the allocations, in halves
     explicit Buffers(const std::vector<int64_t>& numels) {
         for (int64_t n : numels) {
-            offset.push_back(total);
-            total += (n + 127) / 128 * 128;
+            n = (n + 127) / 128 * 128;
+            if (sizes.empty() || sizes.back() + n > kMost) sizes.push_back(0);
+            where.emplace_back((int)sizes.size() - 1, sizes.back());
+            sizes.back() += n;
         }
     }
-    void pointers(const at::Tensor& flat, std::vector<void*>& out) const {
-        auto* base = static_cast<char*>(flat.data_ptr());
-        for (int64_t o : offset) out.push_back(base + 2 * o);
+    std::vector<at::Tensor> allocate(const at::TensorOptions& opt) const {
+        std::vector<at::Tensor> ts;
+        ts.reserve(sizes.size());
+        for (int64_t n : sizes) ts.push_back(at::empty({n}, opt));
+        return ts;
+    }
+    void pointers(const at::Tensor* ts, std::vector<void*>& out) const {
+        for (const auto& [t, o] : where) out.push_back(static_cast<char*>(ts[t].data_ptr()) + 2 * o);
     }
 };
+
+// What the node below has no answer for and a Python autograd function has (a refusal, a traced call, a rule): tangents of
+// forward-mode differentiation, functorch's transforms, dispatch modes and tensor subclasses, tracing.
+bool has_tangent(const at::Tensor& t) {
+    const auto* m = torch::autograd::impl::get_autograd_meta(t);
+    return m && m->fw_grad_;
+}
+bool plain(const at::Tensor& X, const std::vector<at::Tensor>& params) {
+    if (torch::jit::tracer::isTracing() || c10::impl::TorchDispatchModeTLS::any_modes_set() ||
+        c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode))
+        return false;
+    auto odd = [](const at::Tensor& t) { return has_tangent(t) || t.key_set().has(c10::DispatchKey::Python); };
+    return !odd(X) && std::none_of(params.begin(), params.end(), odd);
+}
 
 struct EncoderLayer : std::enable_shared_from_this<EncoderLayer> {
     void* handle;
@@ -131,19 +161,18 @@ struct EncoderLayer : std::enable_shared_from_this<EncoderLayer> {
         if (list.empty() || list[0].device() != X.device()) list = workspace(which, X).cast<std::vector<at::Tensor>>();
     }
 
-    at::Tensor forward(const at::Tensor& X, const std::vector<at::Tensor>& params);
+    std::optional<at::Tensor> forward(const at::Tensor& X, const std::vector<at::Tensor>& params);
 };
 
 struct EncoderBackward : Node {
     std::shared_ptr<EncoderLayer> layer;
-    std::vector<SavedVariable> saved;         // the parameters as the forward pass read them, then X
-    at::Tensor flat;                          // the forward intermediates (unless the layer keeps its own)
+    // the parameters as the forward pass read them, X, and the forward intermediates (unless the layer keeps its own)
+    std::vector<SavedVariable> saved;
     uint64_t generation = 0;
 
     std::string name() const override { return "EncoderFunctionBackward"; }
     void release_variables() override {
         for (auto& s : saved) s.reset_data();
-        flat.reset();
     }
 
     variable_list apply(variable_list&& grads) override {
@@ -155,7 +184,8 @@ struct EncoderBackward : Node {
         variable_list in;
         in.reserve(saved.size());
         for (auto& s : saved) in.push_back(s.unpack());
-        const at::Tensor& X = in.back();
+        const size_t np = l.param_shapes.size();
+        const at::Tensor& X = in[np];
         const c10::DeviceGuard guard(X.device());
         at::Tensor DY = grads[0].defined() ? grads[0].contiguous() : at::zeros(l.out_shape, X.options());
         variable_list out;
@@ -163,7 +193,7 @@ struct EncoderBackward : Node {
         const auto opt = X.options();
         out.push_back(at::empty(l.in_shape, DY.options()));
         for (const auto& s : l.param_shapes) out.push_back(at::empty(s, opt));
-        at::Tensor scratch;
+        std::vector<at::Tensor> scratch;
         std::vector<void*> p;
         p.reserve(96);
         p.push_back(DY.data_ptr());
@@ -171,12 +201,12 @@ struct EncoderBackward : Node {
         if (l.persistent) {
             for (const auto& t : l.kept_bwd) p.push_back(t.data_ptr());
         } else {
-            scratch = at::empty({l.bwd.total}, opt);
-            l.bwd.pointers(scratch, p);
+            scratch = l.bwd.allocate(opt);
+            l.bwd.pointers(scratch.data(), p);
         }
-        for (size_t i = 0; i + 1 < in.size(); ++i) p.push_back(in[i].data_ptr());
+        for (size_t i = 0; i < np; ++i) p.push_back(in[i].data_ptr());
         if (l.persistent) for (const auto& t : l.kept_fwd) p.push_back(t.data_ptr());
-        else l.fwd.pointers(flat, p);
+        else l.fwd.pointers(in.data() + np + 1, p);
         p.push_back(X.data_ptr());
         p.push_back(out[0].data_ptr());
         use_current_stream(l.handle, X.device().index());
@@ -185,7 +215,9 @@ struct EncoderBackward : Node {
     }
 };
 
-at::Tensor EncoderLayer::forward(const at::Tensor& X_, const std::vector<at::Tensor>& params) {
+// None where the caller is to take the Python function.
+std::optional<at::Tensor> EncoderLayer::forward(const at::Tensor& X_, const std::vector<at::Tensor>& params) {
+    if (!plain(X_, params)) return std::nullopt;
     if (!X_.is_cuda()) raise("Encoder.forward needs a tensor on the GPU", PyExc_RuntimeError);
     if (X_.sizes() != at::IntArrayRef(in_shape)) {
         std::ostringstream m;
@@ -199,8 +231,8 @@ at::Tensor EncoderLayer::forward(const at::Tensor& X_, const std::vector<at::Ten
         grad = X_.requires_grad();
         for (size_t i = 0; !grad && i < params.size(); ++i) grad = params[i].requires_grad();
     }
-    at::Tensor X, Y, flat;
-    std::vector<at::Tensor> w;
+    at::Tensor X, Y;
+    std::vector<at::Tensor> w, interm;
     std::vector<void*> p;
     p.reserve(48);
     {
@@ -217,8 +249,8 @@ at::Tensor EncoderLayer::forward(const at::Tensor& X_, const std::vector<at::Ten
             if (grad) keep(kept_bwd, "backward_interm", X);
             for (const auto& t : kept_fwd) p.push_back(t.data_ptr());
         } else {
-            flat = at::empty({fwd.total}, Y.options());
-            fwd.pointers(flat, p);
+            interm = fwd.allocate(Y.options());
+            fwd.pointers(interm.data(), p);
         }
         p.push_back(Y.data_ptr());
     }
@@ -232,10 +264,10 @@ at::Tensor EncoderLayer::forward(const at::Tensor& X_, const std::vector<at::Ten
         std::shared_ptr<EncoderBackward> node(new EncoderBackward(), torch::autograd::deleteNode);
         node->set_next_edges(torch::autograd::collect_next_edges(X_, params));
         node->layer = shared_from_this();
-        node->saved.reserve(w.size() + 1);
+        node->saved.reserve(w.size() + 1 + interm.size());
         for (const auto& t : w) node->saved.emplace_back(t, false);
         node->saved.emplace_back(X, false);
-        node->flat = flat;
+        for (const auto& t : interm) node->saved.emplace_back(t, false);
         node->generation = generation;
         torch::autograd::set_history(Y, node);
     }
@@ -249,5 +281,8 @@ PYBIND11_MODULE(_host, m) {
     py::class_<EncoderLayer, std::shared_ptr<EncoderLayer>>(m, "EncoderLayer")
         .def(py::init<uintptr_t, py::object, std::vector<int64_t>, std::vector<int64_t>, std::vector<std::vector<int64_t>>,
                       const std::vector<int64_t>&, const std::vector<int64_t>&, bool, bool, bool, py::object>())
+        .def_readwrite("generation", &EncoderLayer::generation)
+        .def("check_compact", &EncoderLayer::check_compact)
+        .def("check_relu_gate", &EncoderLayer::check_relu_gate)
         .def("forward", &EncoderLayer::forward);
 }

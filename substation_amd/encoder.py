@@ -29,57 +29,64 @@ def causal_mask(seq_len, device='cuda', dtype=torch.float16):
     return torch.triu(torch.full((seq_len, seq_len), float('-inf'), dtype=dtype, device=device), diagonal=1)
 
 
-def _debug_function(module, in_shape, out_shape, workspace):
-    """The layer call of ``enable_debug=True``: every named tensor in a buffer of its own, captured after each pass."""
-    handle, lib, layouts = module._handle, module._handle.lib, module.layouts
-    n_params = len(layouts['params'])
+def _python_function(weak, layer, in_shape, out_shape, shapes, workspace):
+    """The layer call as a Python autograd function, with a buffer for every named tensor: ``enable_debug=True``, which
+    captures them after each pass, and the calls that the native node leaves to it (tracing, forward-mode differentiation,
+    functorch, dispatch modes).  ``layer`` is the native layer, or what stands in for it and only counts the passes."""
 
-    def tensors(key, like):
+    def call(module, name, device, args):
+        module._handle.set_stream(torch.cuda.current_stream(device).cuda_stream)
+        ptrs = (ctypes.c_void_p * len(args))(*(t.data_ptr() for t in args))
+        _lib.check(getattr(module._handle.lib, 'sub_' + name)(module._handle.ptr, ptrs, len(args)), name)
+        if module.enable_debug:
+            torch.cuda.synchronize()
+
+    def tensors(module, key, like):
         if module.persistent_workspace:
             return workspace(key, like)
-        return [torch.empty(tuple(module.sizes[s] for s in layout), device=like.device, dtype=module.torch_dtype)
-                for _, layout in layouts[key]]
-
-    def call(fn, device, args, what):
-        handle.set_stream(torch.cuda.current_stream(device).cuda_stream)
-        ptrs = (ctypes.c_void_p * len(args))(*(t.data_ptr() for t in args))
-        _lib.check(fn(handle.ptr, ptrs, len(args)), what)
-        torch.cuda.synchronize()
+        return [torch.empty(shape, device=like.device, dtype=module.torch_dtype) for shape in shapes(key)]
 
     class EncoderFunction(torch.autograd.Function):
         @staticmethod
         def forward(ctx, X, *weights):
+            ctx.module = module = weak()
+            layouts = module.layouts
             if not X.is_cuda:
                 raise RuntimeError('Encoder.forward needs a tensor on the GPU')
             if tuple(X.shape) != in_shape:
                 raise ValueError(f"X has shape {tuple(X.shape)}, the configured input layout "
                                  f"{layouts['input'][1]} needs {in_shape}")
+            layer.check_compact()
             X = X.contiguous()
             Y = torch.empty(out_shape, device=X.device, dtype=X.dtype)
-            interm = tensors('forward_interm', X)
-            module._generation += 1
-            ctx.generation = module._generation
+            interm = tensors(module, 'forward_interm', X)
+            layer.generation += 1
+            ctx.generation = layer.generation
             weights = [t.contiguous() for t in weights]
-            call(lib.sub_encoder_forward, X.device, [X, *weights, *interm, Y], 'encoder_forward')
+            call(module, 'encoder_forward', X.device, [X, *weights, *interm, Y])
             ctx.save_for_backward(*weights, *interm, X)
-            for (name, _), t in zip(list(layouts['forward_interm']) + list(layouts['params']), interm + weights):
-                module.debug[name] = t.detach().cpu().numpy()
+            if module.enable_debug:
+                for (name, _), t in zip(list(layouts['forward_interm']) + list(layouts['params']), interm + weights):
+                    module.debug[name] = t.detach().cpu().numpy()
             return Y
 
         @staticmethod
         def backward(ctx, DY):
-            if module.persistent_workspace and ctx.generation != module._generation:
+            module, layouts = ctx.module, ctx.module.layouts
+            if module.persistent_workspace and ctx.generation != layer.generation:
                 raise RuntimeError('persistent_workspace: forward() ran again before this backward pass; '
                                    'what it had saved has been overwritten')
+            layer.check_relu_gate()
             DY = DY.contiguous()
             DX = torch.empty(in_shape, device=DY.device, dtype=DY.dtype)
-            interm = tensors('backward_interm', DY)
-            grads = [torch.empty_like(t) for t in ctx.saved_tensors[:n_params]]
-            call(lib.sub_encoder_backward, DY.device, [DY, *grads, *interm, *ctx.saved_tensors, DX], 'encoder_backward')
-            for (name, _), t in zip(layouts['backward_interm'], interm):
-                module.debug[name] = t.detach().cpu().numpy()
-            for (name, _), t in zip(layouts['params'], grads):
-                module.debug['D' + name] = t.detach().cpu().numpy()
+            interm = tensors(module, 'backward_interm', DY)
+            grads = [torch.empty_like(t) for t in ctx.saved_tensors[:len(layouts['params'])]]
+            call(module, 'encoder_backward', DY.device, [DY, *grads, *interm, *ctx.saved_tensors, DX])
+            if module.enable_debug:
+                for (name, _), t in zip(layouts['backward_interm'], interm):
+                    module.debug[name] = t.detach().cpu().numpy()
+                for (name, _), t in zip(layouts['params'], grads):
+                    module.debug['D' + name] = t.detach().cpu().numpy()
             return (DX, *grads)
 
     return EncoderFunction
@@ -181,7 +188,6 @@ class Encoder(torch.nn.Module):
             compact.update({'LIN1': 8, 'DROP2MASK': 8})
         self.persistent_workspace = bool(persistent_workspace)
         self.canonical_state_dict = bool(canonical_state_dict)
-        self._generation = 0
         self._workspace = {}           # 'forward_interm' / 'backward_interm' -> tensors, when persistent
         self._shared_backward = None   # set by EncoderStack: one backward workspace for all layers
         handle = self._handle
@@ -205,14 +211,21 @@ class Encoder(torch.nn.Module):
 
         if enable_debug:
             self._layer = None
-            self.encoder_func = _debug_function(self, in_shape, out_shape, _workspace)
+            layer = types.SimpleNamespace(generation=0, check_compact=lambda: None, check_relu_gate=lambda: None)
         else:
-            self._layer = _lib.host().EncoderLayer(
+            self._layer = layer = _lib.host().EncoderLayer(
                 handle.ptr, handle, in_shape, out_shape, _shapes('params'),
                 [math.prod(s) for s in _shapes('forward_interm')], [math.prod(s) for s in _shapes('backward_interm')],
                 self.persistent_workspace, self.compact_attention, self.compact_activation, _workspace)
-            layer = self._layer
-            self.encoder_func = types.SimpleNamespace(apply=lambda X, *weights: layer.forward(X, weights))
+        self._function = None
+        self._function_args = (weak, layer, in_shape, out_shape, _shapes, _workspace)
+
+    @property
+    def encoder_func(self):
+        """The layer call as a torch.autograd.Function (made when first asked for: a class takes 0.1 ms to make)."""
+        if self._function is None:
+            self._function = _python_function(*self._function_args)
+        return self._function
 
     def _canonical_perm(self, name, layout):
         canon = _lay.CANONICAL[name]
@@ -299,7 +312,9 @@ class Encoder(torch.nn.Module):
         """Run the encoder.  X is in ``layouts['input'][1]`` order; the result is
         in ``layouts['output'][1]`` order."""
         if self._layer is not None:
-            return self._layer.forward(X, self.params)
+            Y = self._layer.forward(X, self.params)
+            if Y is not None:
+                return Y
         return self.encoder_func.apply(X, *self.params)
 
 

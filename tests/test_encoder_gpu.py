@@ -1012,3 +1012,68 @@ def test_hip_graph_replays_match_eager_and_draw_new_masks():
         for a, b in zip(replays[r], collect(ref, Yr)):
             assert torch.equal(a, b), f'replay {r} differs from the eager run at step {2 + r}'
     assert not torch.equal(replays[0][0], replays[1][0])     # new masks on every replay
+
+
+def _plain_layer(**more):
+    from substation_amd import Encoder, layouts as L
+    torch.manual_seed(0)
+    enc = Encoder('unused', 2, 64, 2, 128, L.mi355x_layouts(), torch.float16, 0.0, 0.0, 0.0, 0.0, activation='gelu',
+                  seed=SEED, **more).cuda()
+    with torch.no_grad():
+        for q in enc.parameters():
+            q.mul_(0.1)
+    g = torch.Generator().manual_seed(5)
+    return enc, [torch.randn(2, 64, 128, generator=g).half().cuda() for _ in range(2)]
+
+
+def test_saved_tensor_hooks_see_every_intermediate():
+    """Offloading or recomputing what the layer saves (saved_tensors_hooks) covers the forward intermediates too."""
+    enc, (x, dy) = _plain_layer()
+    x.requires_grad_()
+    enc(x).backward(dy)
+    want = [x.grad.clone()] + [q.grad.clone() for q in enc.parameters()]
+    x.grad = None
+    enc.zero_grad(set_to_none=True)
+    packed = []
+
+    def pack(t):
+        packed.append(t.numel())
+        return t.cpu()
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t.cuda()):
+        y = enc(x)
+    # X, the twelve E x E matrices in the weights, and well over ten tensors of X's size among the intermediates
+    assert sum(packed) > x.numel() + 12 * 128 * 128 + 10 * x.numel()
+    y.backward(dy)
+    for a, b in zip(want, [x.grad] + [q.grad for q in enc.parameters()]):
+        assert torch.equal(a, b)
+
+
+def test_calls_that_the_native_node_does_not_know_are_traced_or_refused():
+    """A traced layer is a node of the graph, not a constant; tangents and functorch's transforms are refused, not dropped."""
+    import torch.autograd.forward_ad as fwd
+    enc, (x, x2) = _plain_layer()
+    enc.requires_grad_(False)                    # (a traced graph holds them as constants)
+    with torch.no_grad():
+        traced = torch.jit.trace(lambda t: enc(t), x, check_trace=False)
+        assert torch.equal(traced(x2), enc(x2))
+    with fwd.dual_level(), pytest.raises(RuntimeError):
+        enc(fwd.make_dual(x, x2))
+    with pytest.raises(RuntimeError):
+        torch.func.vmap(enc)(torch.stack([x, x2]))
+    with pytest.raises(RuntimeError):
+        torch.func.grad(lambda t: enc(t).float().sum())(x)
+    assert torch.equal(enc(x), traced(x))        # and the layer still works
+
+
+def test_python_function_gives_the_native_node_bits():
+    enc, (x, dy) = _plain_layer()
+    x.requires_grad_()
+    got = []
+    for call in (enc, lambda t: enc.encoder_func.apply(t, *enc.params)):
+        x.grad = None
+        enc.zero_grad(set_to_none=True)
+        y = call(x)
+        y.backward(dy)
+        got.append([y.detach(), x.grad] + [q.grad for q in enc.parameters()])
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
