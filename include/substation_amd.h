@@ -244,7 +244,9 @@ int sub_set_attention_mask(void* handle, const void* attn_mask, const char* layo
  * bit per element (byte (b*J + j)*I/8 + i/8, bit i%8, canonical order whatever
  * the tensor's layout) in the first B*J*I/8 bytes of the DROP1MASK and DROP3MASK
  * buffers, instead of as 0/1 tensors: 7.5 MiB less to write and to read per mask at
- * B=8, L=512, E=1024.  Same results.  Set it to 0 before the forward call when the
+ * B=8, L=512, E=1024.  The activation's, where that dropout runs as an operator of
+ * its own and its mask is kept, likewise in the first B*J*U/8 bytes of DROP2MASK
+ * (feed-forward size a multiple of 8).  Same results.  Set it to 0 before the forward call when the
  * mask tensors are wanted (debug capture); both calls must see the same value. */
 #define SUB_OPT_PACKED_MASKS 9
 /* SUB_OPT_SKIP_UNREAD (default 1): intermediates that neither call reads

@@ -236,7 +236,7 @@ struct Handle {
     bool relu_from_output = true;     // ReLU: the backward gate is read off DROP2; LIN1 and DROP2MASK are not produced
     int side_jobs = 1;                // bit 0: CUs that the stacked projections' tiles leave idle draw attention keep bits;
                                       // bit 1: workgroups behind the first LayerNorm launch draw lin1's keep bits
-    bool packed_masks = true;         // DROP1MASK / DROP3MASK travel as one bit per element inside their buffers
+    bool packed_masks = true;         // DROP1MASK, DROP2MASK and DROP3MASK travel as one bit per element inside their buffers
     bool skip_unread = true;          // intermediates that neither pass reads are not written (ATT after its bias, LIN2, DLN2, DLN1)
     // where the last forward call's lin1 epilogue left one bit per element of DROP2 (set = positive), or
     // null: the unused SB1_LINW1 buffer of that call.  The backward call reads its gate from there when it
@@ -287,8 +287,9 @@ float* static_scratch() {
     return g_scratch_ptr[dev];
 }
 
-// The two residual dropout masks as bits (SUB_OPT_PACKED_MASKS): rows must be whole 8-packs.
+// Dropout masks as bits (SUB_OPT_PACKED_MASKS), those of the residuals and the activation's: rows must be whole 8-packs.
 bool packed_masks(const Handle& h) { return h.packed_masks && h.sz.n[dI] % 8 == 0; }
+bool packed_act_mask(const Handle& h) { return h.packed_masks && h.sz.n[dU] % 8 == 0; }
 
 PhiloxKey make_key(const Handle& h, uint32_t site, float p) {
     PhiloxKey k;
@@ -722,12 +723,13 @@ void op_blnrd(Handle& h, const void* dout, const Layout& ldout, const void* istd
 
 void op_bad(Handle& h, const void* in, const Layout& lin_, const void* bias, void* lin,
             const Layout& llin, void* mask, const Layout& lmask, void* out, const Layout& lout,
-            float p, uint32_t site, bool out_only = false) {
+            float p, uint32_t site, bool out_only = false, bool packed_mask = false) {
     Space sp = make_space(h.sz, {dB, dJ}, dU);
     View vi = make_view(in, lin_, sp), vl = make_view(lin, llin, sp), vm = make_view(mask, lmask, sp),
          vo = make_view(out, lout, sp);
     flatten(sp.rs, {&vi, &vl, &vm, &vo});
-    launch_bad(sp.rs, vi, vector_view(bias, sp.rs.R), vl, vm, vo, h.act, make_key(h, site, p), h.stream, out_only);
+    launch_bad(sp.rs, vi, vector_view(bias, sp.rs.R), vl, vm, vo, h.act, make_key(h, site, p), h.stream, out_only,
+               packed_mask ? (uint8_t*)mask : nullptr);
 }
 
 void op_bsb(Handle& h, const void* in, const Layout& lin_, const void* scale, const void* dout,
@@ -752,11 +754,12 @@ void op_ebsb(Handle& h, const void* in, const Layout& lin_, const void* scale, c
 }
 
 void op_bdrlb(Handle& h, const void* ddrop, const Layout& ld, const void* mask, const Layout& lm,
-              const void* lin, const Layout& ll, void* dlinear, const Layout& lo, void* dbias) {
+              const void* lin, const Layout& ll, void* dlinear, const Layout& lo, void* dbias, bool packed_mask = false) {
     Space sp = make_space(h.sz, {dB, dJ}, dU);
     float* ws = take_ws(h, colreduce_ws_floats(sp.rs, 1));
     launch_bdrlb(sp.rs, make_view(ddrop, ld, sp), make_view(mask, lm, sp), make_view(lin, ll, sp),
-                 make_view(dlinear, lo, sp), ColOut{(half_t*)dbias}, h.act, ws, h.stream, defer_of(h));
+                 make_view(dlinear, lo, sp), ColOut{(half_t*)dbias}, h.act, ws, h.stream, defer_of(h),
+                 packed_mask ? (const uint8_t*)mask : nullptr);
 }
 
 // The ReLU layer's bdrlb with the gate taken from the forward output DROP2 = relu(LIN1) * mask, which is
@@ -1156,7 +1159,7 @@ void forward(Handle& h, const FwdPtrs& t0) {
     {
         ProfScope ps(h, "bad");
         op_bad(h, F[SB1_LINW1], h.lf[SB1_LINW1], W[LINB1], F[LIN1], h.lf[LIN1], F[DROP2MASK],
-               h.lf[DROP2MASK], F[DROP2], h.lf[DROP2], h.p_act, SUB_SITE_ACT, relu_from_output(h));
+               h.lf[DROP2MASK], F[DROP2], h.lf[DROP2], h.p_act, SUB_SITE_ACT, relu_from_output(h), packed_act_mask(h));
     }
     }
     run_gemm(h, G_LIN2, F[DROP2], W[LINW2], F[DROP2_LINW2], "lin2");
@@ -1294,7 +1297,7 @@ void backward(Handle& h, const BwdPtrs& t0) {
             op_bdrlb_from_output(h, D[DDROP2], h.lb[DDROP2], F[DROP2], h.lf[DROP2], D[DLIN1], h.lb[DLIN1], DW[LINB1]);
         else
             op_bdrlb(h, D[DDROP2], h.lb[DDROP2], F[DROP2MASK], h.lf[DROP2MASK], F[LIN1], h.lf[LIN1],
-                     D[DLIN1], h.lb[DLIN1], DW[LINB1]);
+                     D[DLIN1], h.lb[DLIN1], DW[LINB1], packed_act_mask(h));
     }
     if (dwlin2_at == THIRD_WITH_SECOND) {
         run_gemm(h, G_DXLIN1, D[DLIN1], W[LINW1], D[DLIN1_LINW1], "dXlin1");

@@ -17,11 +17,12 @@ namespace {
 constexpr int BLOCK = 256;
 constexpr int WPB = BLOCK / WAVE;
 
-enum ColKind { COL_BSB, COL_EBSB, COL_BDRLB, COL_BAOB, COL_BDRLB_OUT };
+enum ColKind { COL_BSB, COL_EBSB, COL_BDRLB, COL_BAOB, COL_BDRLB_OUT, COL_BDRLB_BITS };
 
 struct ColArgs {
     View v[7];
     int act;
+    const uint8_t* mask_bits = nullptr;      // COL_BDRLB_BITS: one bit per element, canonical order, a byte per pack
 };
 
 template <int KIND> struct ColTraits;
@@ -30,6 +31,7 @@ template <> struct ColTraits<COL_EBSB> { static constexpr int NS = 3; };
 template <> struct ColTraits<COL_BDRLB> { static constexpr int NS = 1; };
 template <> struct ColTraits<COL_BAOB> { static constexpr int NS = 1; };
 template <> struct ColTraits<COL_BDRLB_OUT> { static constexpr int NS = 1; };
+template <> struct ColTraits<COL_BDRLB_BITS> { static constexpr int NS = 1; };
 
 template <int KIND> struct ColIn;      // which views are read: count and indices into ColArgs::v
 // `nt`: inputs read here for the last time (saved by the forward pass, or the
@@ -39,6 +41,8 @@ template <> struct ColIn<COL_EBSB> { static constexpr int N = 4; static constexp
 template <> struct ColIn<COL_BDRLB> { static constexpr int N = 3; static constexpr int idx[4] = {0, 1, 2, 0}; static constexpr bool nt[4] = {true, true, true, false}; };
 // the ReLU gate read off the forward pass's output: DROP2 > 0 exactly where the mask kept a positive LIN1
 template <> struct ColIn<COL_BDRLB_OUT> { static constexpr int N = 2; static constexpr int idx[4] = {0, 1, 0, 0}; static constexpr bool nt[4] = {true, false, false, false}; };
+// (bound by memory: the mask as a tensor was a fourth of what it moved)
+template <> struct ColIn<COL_BDRLB_BITS> { static constexpr int N = 2; static constexpr int idx[4] = {0, 2, 0, 0}; static constexpr bool nt[4] = {true, true, false, false}; };
 template <> struct ColIn<COL_BAOB> { static constexpr int N = 1; static constexpr int idx[4] = {0, 0, 0, 0}; static constexpr bool nt[4] = {false, false, false, false}; };
 
 // Raw 128-bit loads of the inputs of one row chunk (inputs T, T+1, ...).
@@ -56,7 +60,7 @@ __device__ __forceinline__ void col_load_raw(const ColArgs& a, const RowIdx& ix,
 // One 8-pack of one row: elementwise output (stored to v[3]) and the running sums.
 template <int KIND>
 __device__ __forceinline__ void col_compute(const ColArgs& a, const RowIdx& ix, int e0, int nv,
-                                            const F8 (&in)[4], const F8& fscale,
+                                            const F8 (&in)[4], const F8& fscale, uint32_t bits,
                                             float (&acc)[ColTraits<KIND>::NS][8]) {
     if (KIND == COL_BSB) {
         // in0 IN (normed), in1 DOUT -> DIN
@@ -80,13 +84,14 @@ __device__ __forceinline__ void col_compute(const ColArgs& a, const RowIdx& ix, 
             acc[2][i] += in[3].v[i];
         }
         store8h(a.v[3], view_offset(a.v[3], ix), e0, nv, o);
-    } else if (KIND == COL_BDRLB) {
-        // in0 DDROP, in1 MASK, in2 LIN -> DLINEAR
+    } else if (KIND == COL_BDRLB || KIND == COL_BDRLB_BITS) {
+        // in0 DDROP, in1 MASK (unless it comes as `bits`), in2 LIN -> DLINEAR
+        constexpr int LIN = KIND == COL_BDRLB ? 2 : 1;
         h8 oh;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            float d = in[0].v[i] * in[1].v[i];
-            float g = a.act == ACT_GELU ? gelu_bwd(in[2].v[i], d) : (in[2].v[i] > 0.f ? d : 0.f);
+            float d = in[0].v[i] * (KIND == COL_BDRLB ? in[1].v[i] : (float)((bits >> i) & 1u));
+            float g = a.act == ACT_GELU ? gelu_bwd(in[LIN].v[i], d) : (in[LIN].v[i] > 0.f ? d : 0.f);
             oh[i] = (half_t)g;
         }
         oh = pin(oh);
@@ -140,6 +145,7 @@ __global__ __launch_bounds__(BLOCK) void k_colreduce(RowSpace rs, ColArgs a, flo
             h8 raw[U][NIN];
             F8 gen[4];
             int nvu[U];
+            uint32_t bits[U] = {};
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 unsigned r = row + u * stride;
@@ -147,6 +153,7 @@ __global__ __launch_bounds__(BLOCK) void k_colreduce(RowSpace rs, ColArgs a, flo
                 r = nvu[u] ? r : row;
                 ix[u].i0 = i0; ix[u].i1 = i1;
                 ix[u].i2 = r / n3; ix[u].i3 = r - ix[u].i2 * n3;
+                if (KIND == COL_BDRLB_BITS) bits[u] = a.mask_bits[(size_t)r * ((unsigned)rs.R >> 3) + ((unsigned)e0 >> 3)];
                 if (FAST) {
                     col_load_raw<KIND, 0>(a, ix[u], e0, nvu[u], raw[u]);
                 } else {
@@ -166,7 +173,7 @@ __global__ __launch_bounds__(BLOCK) void k_colreduce(RowSpace rs, ColArgs a, flo
 #pragma unroll
                         for (int i = 0; i < 8; ++i) gen[t].v[i] = (float)raw[u][t][i];
                 }
-                col_compute<KIND>(a, ix[u], e0, nvu[u], gen, fscale, acc);
+                col_compute<KIND>(a, ix[u], e0, nvu[u], gen, fscale, bits[u], acc);
             }
         }
     }
@@ -306,10 +313,17 @@ void launch_ebsb(const RowSpace& rs, View in, View dout1, View dout2, View dline
 }
 
 void launch_bdrlb(const RowSpace& rs, View ddrop, View mask, View lin, View dlinear, ColOut dbias,
-                  int act, float* ws, hipStream_t st, FinishJobs* defer) {
+                  int act, float* ws, hipStream_t st, FinishJobs* defer, const uint8_t* mask_bits) {
     ColArgs a{}; a.v[0] = ddrop; a.v[1] = mask; a.v[2] = lin; a.v[3] = dlinear; a.act = act;
     FinishArgs fo{{dbias.p, nullptr, nullptr}, 0, 0, 1, 1};
-    run_col<COL_BDRLB>(rs, a, fo, ws, st, "backward dropout-activation-bias", defer);
+    const char* const what = "backward dropout-activation-bias";
+    if (mask_bits) {
+        if (rs.R % 8 || rs.n0 != 1 || rs.n1 != 1) fail(std::string(what) + ": a bit mask needs rows of whole 8-packs");
+        a.mask_bits = mask_bits;
+        run_col<COL_BDRLB_BITS>(rs, a, fo, ws, st, what, defer);
+    } else {
+        run_col<COL_BDRLB>(rs, a, fo, ws, st, what, defer);
+    }
 }
 
 void launch_bdrlb_from_output(const RowSpace& rs, View ddrop, View out, View dlinear, ColOut dbias, float* ws,

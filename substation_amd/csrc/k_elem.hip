@@ -32,10 +32,12 @@ __device__ __forceinline__ Chunk chunk_of(const RowSpace& rs, unsigned idx, unsi
 
 // ACT, FLAT: the activation and a flat row space as compile-time facts (a choice of activation per element
 // is a branch per element; a strided row space three divisions per pack of 8).
+// mask_bits: the mask as one bit per element (a byte per pack, canonical order) instead of the tensor: memory is what
+// bounds this, and a fourth of it was the mask.
 template <bool FAST, int ACT = -1, bool FLAT = false>
 __global__ __launch_bounds__(BLOCK) void k_bad(RowSpace rs, View in, View bias, View lin, View mask,
                                                View out, int act, PhiloxKey key_, unsigned nchunks,
-                                               unsigned cpr, int out_only) {
+                                               unsigned cpr, int out_only, uint8_t* mask_bits) {
     const PhiloxKey key = resolved(key_);
     const unsigned stride = gridDim.x * BLOCK;
     for (unsigned base = blockIdx.x * BLOCK + threadIdx.x; base < nchunks; base += stride * UNROLL) {
@@ -63,7 +65,8 @@ __global__ __launch_bounds__(BLOCK) void k_bad(RowSpace rs, View in, View bias, 
             }
             if (!out_only) {
                 st8h<FAST, true>(lin, view_offset_of<FLAT>(lin, c[u].ix), c[u].e0, c[u].nv, lh);
-                st8h<FAST, true>(mask, view_offset_of<FLAT>(mask, c[u].ix), c[u].e0, c[u].nv, mask_h8(bits));
+                if (mask_bits) mask_bits[(size_t)c[u].row * cpr + (c[u].e0 >> 3)] = (uint8_t)bits;
+                else st8h<FAST, true>(mask, view_offset_of<FLAT>(mask, c[u].ix), c[u].e0, c[u].nv, mask_h8(bits));
             }
             st8h<FAST>(out, view_offset_of<FLAT>(out, c[u].ix), c[u].e0, c[u].nv, oh);
         }
@@ -110,13 +113,14 @@ inline unsigned check_chunks(long nchunks, const char* what) {
 }  // namespace
 
 void launch_bad(const RowSpace& rs, View in, View bias, View lin, View mask, View out, int act,
-                PhiloxKey key, hipStream_t st, bool out_only) {
+                PhiloxKey key, hipStream_t st, bool out_only, uint8_t* mask_bits) {
+    if (mask_bits && rs.R % 8) fail("bias-activation-dropout: a bit mask needs rows of whole 8-packs");
     unsigned cpr = (unsigned)((rs.R + 7) / 8);
     unsigned nchunks = check_chunks(rs.rows() * cpr, "bias-activation-dropout");
     if (nchunks == 0) return;
-    const bool fast = in.vec && bias.vec && lin.vec && mask.vec && out.vec;
+    const bool fast = in.vec && bias.vec && lin.vec && (mask.vec || mask_bits) && out.vec;
 #define SUB_BAD(...) hipLaunchKernelGGL((k_bad<__VA_ARGS__>), dim3(elem_grid(nchunks)), dim3(BLOCK), 0, st, rs, in, bias, lin, \
-                                        mask, out, act, key, nchunks, cpr, out_only ? 1 : 0)
+                                        mask, out, act, key, nchunks, cpr, out_only ? 1 : 0, mask_bits)
     if (fast && rs.flat && act == ACT_GELU) SUB_BAD(true, ACT_GELU, true);
     else if (fast && rs.flat) SUB_BAD(true, ACT_RELU, true);
     else if (fast && act == ACT_GELU) SUB_BAD(true, ACT_GELU, false);
@@ -124,7 +128,7 @@ void launch_bad(const RowSpace& rs, View in, View bias, View lin, View mask, Vie
 #undef SUB_BAD
     else
         hipLaunchKernelGGL(k_bad<false>, dim3(elem_grid(nchunks)), dim3(BLOCK), 0, st, rs, in, bias, lin,
-                           mask, out, act, key, nchunks, cpr, out_only ? 1 : 0);
+                           mask, out, act, key, nchunks, cpr, out_only ? 1 : 0, mask_bits);
     check_launch("bias-activation-dropout");
 }
 
