@@ -121,7 +121,9 @@ __global__ __launch_bounds__(BLOCK) void k_colreduce(RowSpace rs, ColArgs a, flo
                                                      long rows_per_block, long nrows) {
     constexpr int NS = ColTraits<KIND>::NS;
     constexpr int NIN = ColIn<KIND>::N;
-    constexpr int U = FAST ? 2 : 1;                    // rows in flight per lane
+    // Rows in flight per lane: four of two inputs, which is all the rows a lane has in a grid of 2048 workgroups over
+    // 4000 rows, so its loads take one round trip instead of two.
+    constexpr int U = !FAST ? 1 : NIN <= 2 ? 4 : 2;
     __shared__ float red[BLOCK][9];          // +1 pad: conflict-free column reads
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int lpr = 1 << lpr_log2, rpw = WAVE >> lpr_log2;
@@ -184,15 +186,12 @@ __global__ __launch_bounds__(BLOCK) void k_colreduce(RowSpace rs, ColArgs a, flo
 #pragma unroll
         for (int i = 0; i < 8; ++i) red[tid][i] = acc[s][i];
         __syncthreads();
-        if (tid < lpr && nv > 0) {
-            float tot[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) tot[i] = 0.f;
-            for (int t = tid; t < BLOCK; t += lpr)
-#pragma unroll
-                for (int i = 0; i < 8; ++i) tot[i] += red[t][i];
-            float* dst = ws + (((long)s * gridDim.z + blockIdx.z) * ntc + blockIdx.y) * rs.R + e0;
-            for (int i = 0; i < nv; ++i) dst[i] = tot[i];
+        // (a thread per feature: with the lanes that had loaded it, 8 features each, this was a chain of 128 reads)
+        const int f = blockIdx.x * lpr * 8 + tid;
+        if (tid < lpr * 8 && f < rs.R) {
+            float tot = 0.f;
+            for (int t = tid >> 3; t < BLOCK; t += lpr) tot += red[t][tid & 7];
+            ws[(((long)s * gridDim.z + blockIdx.z) * ntc + blockIdx.y) * rs.R + f] = tot;
         }
     }
 }
