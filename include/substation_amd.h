@@ -253,7 +253,8 @@ int sub_set_attention_mask(void* handle, const void* attn_mask, const char* layo
  * afterwards are not written: ATT keeps the product without its bias (the bias
  * is added in registers, encoder.cu:134-135 writes it back in place), LIN2 is
  * left alone, and where the LayerNorm backward runs as one launch DLN2 and DLN1
- * are left alone.  8 MiB less to write in each of four launches at B=8, L=512,
+ * are left alone, and so are ATT and DROP2_LINW2 where their products were split
+ * along k and go into the launch behind them as partial sums.  8 MiB less to write in each of four launches at B=8, L=512,
  * E=1024; outputs and gradients are bit-identical.  Set it to 0 (debug capture
  * does) when those tensors are wanted. */
 #define SUB_OPT_SKIP_UNREAD 10

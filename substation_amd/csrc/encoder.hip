@@ -597,11 +597,12 @@ void ensure_gws(Handle& h, size_t floats) {
 }
 
 void run_gemm(Handle& h, int id, const void* A, const void* B, void* C, const char* name,
-              const void* addend = nullptr, GemmSideJob* side = nullptr) {
+              const void* addend = nullptr, GemmSideJob* side = nullptr, SplitSums* sums = nullptr) {
     ProfScope ps(h, name);
     const GemmPlan& p = h.gemm[id];
     GemmEpilogue ep;
     ep.any_split = id >= G_DXLIN2 || id == G_DXQKV_RESID;      // the backward pass
+    ep.sums = sums;
     if (addend) {
         ep.bias = (const half_t*)addend; ep.sbM = p.sM; ep.sbN = p.sN;
         for (int i = 0; i < 3; ++i) ep.sbb[i] = p.sb[i];
@@ -699,7 +700,7 @@ void op_bdrln(Handle& h, const void* in, const Layout& lin_, const void* resid, 
               const Layout& llin, void* mask, const Layout& lmask, void* diff, const Layout& ldiff,
               void* normed, const Layout& lnorm, void* out, const Layout& lout, void* istd,
               const Layout& listd, float p, uint32_t site, bool packed_mask = false, bool write_lin = true,
-              KeepWordsJob* side = nullptr) {
+              KeepWordsJob* side = nullptr, SplitSums sums = SplitSums{}) {
     Space sp = make_space(h.sz, {dB, dJ}, dI);
     int R = sp.rs.R;
     View vi = make_view(in, lin_, sp), vr = make_view(resid, lres, sp), vl = make_view(lin, llin, sp),
@@ -708,7 +709,7 @@ void op_bdrln(Handle& h, const void* in, const Layout& lin_, const void* resid, 
     flatten(sp.rs, {&vi, &vr, &vl, &vm, &vd, &vn, &vo, &vs});
     launch_bdrln(sp.rs, vi, vr, vector_view(linear_bias, R), vector_view(scale, R), vector_view(bias, R),
                  vl, vm, vd, vn, vo, vs, make_key(h, site, p), h.eps, h.stream, packed_mask ? (uint8_t*)mask : nullptr,
-                 write_lin, side);
+                 write_lin, side, sums);
 }
 
 void op_blnrd(Handle& h, const void* dout, const Layout& ldout, const void* istd, const Layout& listd,
@@ -1119,7 +1120,11 @@ void forward(Handle& h, const FwdPtrs& t0) {
         h.mask_plan_built = false;          // the backward pass makes its plan from the mask as it is now
     }
     if (!fused_attention) run_gemm(h, G_GAMMA, VV, F[ATTN_DROP], F[GAMMA], "gamma");
-    run_gemm(h, G_OUT, W[WO], F[GAMMA], F[ATT], "out");
+    // Small products go into the LayerNorm launch behind them as the sums of their splits (ATT and DROP2_LINW2, which
+    // nothing else reads, are not written then), where their rows are the tokens in order.
+    SplitSums out_sums, lin2_sums;
+    auto as_sums = [&](int tensor, SplitSums& s) { return h.skip_unread && h.lf[tensor].str() == "BJI" ? &s : nullptr; };
+    run_gemm(h, G_OUT, W[WO], F[GAMMA], F[ATT], "out", nullptr, nullptr, as_sums(ATT, out_sums));
     const bool lin1_gelu = lin1_takes_gelu_epilogue(h, W, F);
     const bool lin1_bad = lin1_gelu || (relu_from_output(h) && h.fuse_epilogues && h.gemm[G_LIN1_BAD].ok &&
                                         aligned16(W[LINB1]) && aligned16(F[DROP2]) && aligned16(F[SB1]) && aligned16(W[LINW1]));
@@ -1139,7 +1144,7 @@ void forward(Handle& h, const FwdPtrs& t0) {
         op_bdrln(h, F[ATT], h.lf[ATT], t.X, h.lX, W[BO], W[S1], W[B1], F[ATT], h.lf[ATT],
                  F[DROP1MASK], h.lf[DROP1MASK], F[LN1DIFF], h.lf[LN1DIFF], F[LN1], h.lf[LN1],
                  F[SB1], h.lf[SB1], F[LN1STD], h.lf[LN1STD], h.p_resid1, SUB_SITE_RESID1, packed_masks(h), !h.skip_unread,
-                 &keep_job);
+                 &keep_job, out_sums);
     }
     if (lin1_bad) {
         // product, bias, activation and dropout in one launch: SB1_LINW1 and DROP2MASK (ReLU: and LIN1) are not produced
@@ -1162,12 +1167,13 @@ void forward(Handle& h, const FwdPtrs& t0) {
                h.lf[DROP2MASK], F[DROP2], h.lf[DROP2], h.p_act, SUB_SITE_ACT, relu_from_output(h), packed_act_mask(h));
     }
     }
-    run_gemm(h, G_LIN2, F[DROP2], W[LINW2], F[DROP2_LINW2], "lin2");
+    run_gemm(h, G_LIN2, F[DROP2], W[LINW2], F[DROP2_LINW2], "lin2", nullptr, nullptr, as_sums(DROP2_LINW2, lin2_sums));
     {
         ProfScope ps(h, "bdrln2");
         op_bdrln(h, F[DROP2_LINW2], h.lf[DROP2_LINW2], F[SB1], h.lf[SB1], W[LINB2], W[S2], W[B2],
                  F[LIN2], h.lf[LIN2], F[DROP3MASK], h.lf[DROP3MASK], F[LN2DIFF], h.lf[LN2DIFF],
-                 F[LN2], h.lf[LN2], t.Y, h.lY, F[LN2STD], h.lf[LN2STD], h.p_resid2, SUB_SITE_RESID2, packed_masks(h), !h.skip_unread);
+                 F[LN2], h.lf[LN2], t.Y, h.lY, F[LN2STD], h.lf[LN2STD], h.p_resid2, SUB_SITE_RESID2, packed_masks(h), !h.skip_unread,
+                 nullptr, lin2_sums);
     }
     if (h.staging && h.stage_y) {
         ProfScope ps(h, "relayout-out");

@@ -833,6 +833,14 @@ bool launch_gemm_pair(const GemmShape& s1, const half_t* A1, const half_t* B1, h
     return true;
 }
 
+void launch_split_sums(const SplitSums& sums, half_t* C, long rows, long row, hipStream_t st) {
+    GemmArgs a{};
+    a.C = C; a.M = (int)rows; a.N = (int)row; a.sCM = row; a.sCN = 1; a.nb1 = a.nb2 = 1; a.nbatch = 1;
+    a.alpha = sums.alpha; a.splits = sums.splits; a.partial = const_cast<float*>(sums.p);
+    launch_splitk_reduce(a, st);
+    check_launch("gemm split sums");
+}
+
 void launch_gemm(const GemmShape& s, const half_t* A, const half_t* B, half_t* C, float alpha,
                  const GemmEpilogue& ep, hipStream_t st, float* ws, size_t ws_floats, GemmSideJob* side) {
     long batch = s.batch();
@@ -877,7 +885,12 @@ void launch_gemm(const GemmShape& s, const half_t* A, const half_t* B, half_t* C
             tp.a.splits = choice.splits;
             if (tp.a.splits > 1) tp.a.partial = ws;
             launch_tiles(&tp, 1, choice.form, nullptr, st);
-            if (tp.a.splits > 1) launch_splitk_reduce(tp.a, st);
+            if (tp.a.splits > 1) {
+                if (ep.sums && batch == 1 && !tp.a.bias && tp.a.sCM == tp.a.N)
+                    *ep.sums = SplitSums{ws, tp.a.splits, (long)tp.a.M * tp.a.N, alpha};
+                else
+                    launch_splitk_reduce(tp.a, st);
+            }
         }
     } else {
         if (ep.relu_dropout || ep.gate) fail("gemm: the ReLU-dropout epilogue needs the MFMA kernel");

@@ -344,11 +344,17 @@ __global__ __launch_bounds__(BLOCK) void k_bdrln(RowSpace rs, View in, View resi
 // SIMD taking turns on them; the launch was bound by that, not by memory).  Here a chunk is
 // inside the row or outside it, the row's loads are issued first, together with the lane's
 // columns of the three per-feature vectors, and the keep bits are drawn while they travel.
-template <int VPL>
+//
+// SUMS: `in` is a product's fp32 sums over up to 8 splits of k, added up here in the order of the launch that would have
+// written them as fp16 (the same bits): a launch and its gap, 4 us of the 87 that a forward pass of 1848 x 768 takes.
+// Rows of at most 1024 (VPL 2): 128 registers for the sums on their way; longer ones take that launch.
+template <int VPL, bool SUMS>
 __global__ __launch_bounds__(BLOCK) void k_bdrln_flat(int R, unsigned nrows, View in, View resid, View lin_bias,
                                                       View scale, View bias, View lin, View mask, View diff,
                                                       View normed, View out, View istd, PhiloxKey key_, float eps,
-                                                      uint8_t* mask_bits, bool write_lin, KeepWordsJob side) {
+                                                      uint8_t* mask_bits, bool write_lin, KeepWordsJob side,
+                                                      SplitSums sums) {
+    if (SUMS) fetch_args_now(sums.p, sums.splits, sums.slab, sums.alpha);
     fetch_args_now(R, nrows, in.p, in.s3, resid.p, resid.s3, lin_bias.p, scale.p, bias.p, lin.p, lin.s3, mask.p, mask.s3,
                    diff.p, diff.s3, normed.p, normed.s3, out.p, out.s3, istd.p, istd.s3, key_.k0, key_.k1, key_.site,
                    key_.step, key_.thr, key_.step_dev, eps, mask_bits, write_lin, side.blocks);
@@ -388,9 +394,20 @@ __global__ __launch_bounds__(BLOCK) void k_bdrln_flat(int R, unsigned nrows, Vie
     auto masked = [&](h8 v, int c) { return __builtin_bit_cast(h8, __builtin_bit_cast(i4v, v) & keep_all[c]); };
     for (unsigned row = blockIdx.x * WPB + (threadIdx.x >> 6); row < nrows; row += row_blocks * WPB) {
         h8 vi[VPL], vr[VPL];
+        float4 part[SUMS ? VPL : 1][8][2];
 #pragma unroll
         for (int c = 0; c < VPL; ++c) {
-            vi[c] = ldg8<true>(in.p + (long)row * in.s3 + e0[c]);
+            if constexpr (SUMS) {
+                const float* p = sums.p + (long)row * R + e0[c];
+#pragma unroll
+                for (int t = 0; t < 8; ++t) {
+                    const float* q = p + (t < sums.splits ? t : 0) * sums.slab;
+                    part[c][t][0] = *reinterpret_cast<const float4*>(q);
+                    part[c][t][1] = *reinterpret_cast<const float4*>(q + 4);
+                }
+            } else {
+                vi[c] = ldg8<true>(in.p + (long)row * in.s3 + e0[c]);
+            }
             vr[c] = ldg8<false>(resid.p + (long)row * resid.s3 + e0[c]);
         }
         // the keep bits are drawn while the loads travel: nothing that waits for one may move up here
@@ -407,6 +424,23 @@ __global__ __launch_bounds__(BLOCK) void k_bdrln_flat(int R, unsigned nrows, Vie
         for (int c = 0; c < VPL; ++c)
             bits[c] = keep_pack<true>(key, (uint64_t)row * (uint64_t)R + (uint64_t)((c * WAVE + lane) * 8));
         __builtin_amdgcn_sched_barrier(0);
+        if constexpr (SUMS) {
+#pragma unroll
+            for (int c = 0; c < VPL; ++c) {
+                float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
+#pragma unroll
+                for (int t = 0; t < 8; ++t) {
+                    const bool on = t < sums.splits;
+                    a.x += on ? part[c][t][0].x : 0.f; a.y += on ? part[c][t][0].y : 0.f;
+                    a.z += on ? part[c][t][0].z : 0.f; a.w += on ? part[c][t][0].w : 0.f;
+                    b.x += on ? part[c][t][1].x : 0.f; b.y += on ? part[c][t][1].y : 0.f;
+                    b.z += on ? part[c][t][1].z : 0.f; b.w += on ? part[c][t][1].w : 0.f;
+                }
+                vi[c] = h8{(half_t)(a.x * sums.alpha), (half_t)(a.y * sums.alpha), (half_t)(a.z * sums.alpha), (half_t)(a.w * sums.alpha),
+                           (half_t)(b.x * sums.alpha), (half_t)(b.y * sums.alpha), (half_t)(b.z * sums.alpha), (half_t)(b.w * sums.alpha)};
+                vi[c] = pin(vi[c]);
+            }
+        }
         float x[VPL][8];
         float s = 0.f;
 #pragma unroll
@@ -717,7 +751,7 @@ void launch_bs(const RowSpace& rs, View alpha, View mask, View ddrop, View dbeta
 
 void launch_bdrln(const RowSpace& rs, View in, View resid, View lin_bias, View scale, View bias,
                   View lin, View mask, View diff, View normed, View out, View istd, PhiloxKey key,
-                  float eps, hipStream_t st, uint8_t* mask_bits, bool write_lin, KeepWordsJob* side) {
+                  float eps, hipStream_t st, uint8_t* mask_bits, bool write_lin, KeepWordsJob* side, SplitSums sums) {
     if (mask_bits && rs.R % 8) fail("bias-dropout-residual-layernorm: a bit mask needs rows of whole 8-packs");
     unsigned nrows = check_rows(rs, "bias-dropout-residual-layernorm");
     if (nrows == 0) return;
@@ -736,15 +770,23 @@ void launch_bdrln(const RowSpace& rs, View in, View resid, View lin_bias, View s
         side->blocks = 0;
     }
     const unsigned extra_blocks = job.blocks;
-    if (fast && rs.flat && (mask.p || mask_bits) && (lin.p || !write_lin)) {
+    const bool flat = fast && rs.flat && (mask.p || mask_bits) && (lin.p || !write_lin);
+    if (sums.p && !(flat && vpl <= 2)) {
+        // (rows as long as they lie apart: whoever leaves a product as sums has seen to that)
+        launch_split_sums(sums, in.p, nrows, rs.R, st);
+        sums.p = nullptr;
+    }
+    if (flat) {
         const dim3 grid(row_grid(nrows, 1) + extra_blocks);
-#define SUB_BDRLN_FLAT(V) hipLaunchKernelGGL((k_bdrln_flat<V>), grid, dim3(BLOCK), 0, st, rs.R, nrows, in, resid, lin_bias, \
-                                             scale, bias, lin, mask, diff, normed, out, istd, key, eps, mask_bits, write_lin, job)
-        switch (vpl) {
-            case 1: SUB_BDRLN_FLAT(1); break;
-            case 2: SUB_BDRLN_FLAT(2); break;
-            case 4: SUB_BDRLN_FLAT(4); break;
-            default: SUB_BDRLN_FLAT(8); break;
+#define SUB_BDRLN_FLAT(V, S) hipLaunchKernelGGL((k_bdrln_flat<V, S>), grid, dim3(BLOCK), 0, st, rs.R, nrows, in, resid, lin_bias, \
+                                             scale, bias, lin, mask, diff, normed, out, istd, key, eps, mask_bits, write_lin, job, sums)
+        if (sums.p && vpl == 1) SUB_BDRLN_FLAT(1, true);
+        else if (sums.p) SUB_BDRLN_FLAT(2, true);
+        else switch (vpl) {
+            case 1: SUB_BDRLN_FLAT(1, false); break;
+            case 2: SUB_BDRLN_FLAT(2, false); break;
+            case 4: SUB_BDRLN_FLAT(4, false); break;
+            default: SUB_BDRLN_FLAT(8, false); break;
         }
 #undef SUB_BDRLN_FLAT
         check_launch("bias-dropout-residual-layernorm");

@@ -28,6 +28,13 @@ void launch_bs(const RowSpace& rs, View alpha, View mask, View ddrop, View dbeta
 // workgroups behind those of the rows draw the keep words of the ReLU-dropout epilogue
 // (relu_dropout_keep_words) of a later product with a dense [M][N] output in 256x256 tiles, word
 // quadruple ((tile_m * N/256 + tile_n) * 8 + wave) * 64 + lane of `out` (M * N / 8 bytes).
+// A product of dense rows left as the fp32 sums of its k splits: fp16(alpha * their sum) is its output, wherever that is read.
+struct SplitSums {
+    const float* p = nullptr;    // [splits][rows][row]; null: the output itself was written
+    int splits = 0;              // at most 8
+    long slab = 0;
+    float alpha = 1.f;
+};
 struct KeepWordsJob {
     PhiloxKey key;
     uint32_t* out = nullptr;
@@ -41,7 +48,7 @@ struct KeepWordsJob {
 void launch_bdrln(const RowSpace& rs, View in, View resid, View lin_bias, View scale, View bias,
                   View lin, View mask, View diff, View normed, View out, View istd, PhiloxKey key,
                   float eps, hipStream_t st, uint8_t* mask_bits = nullptr, bool write_lin = true,
-                  KeepWordsJob* side = nullptr);
+                  KeepWordsJob* side = nullptr, SplitSums sums = SplitSums{});
 void launch_blnrd(const RowSpace& rs, View dout, View istd, View diff, View mask, View d_ln_in,
                   View d_drop_in, hipStream_t st, const uint8_t* mask_bits = nullptr);
 
@@ -248,6 +255,8 @@ struct GemmEpilogue {
     // the contraction of a small output may be split in as many parts as is fastest; otherwise their number, and with it the
     // order of the sums, depends on the shape alone (one unit of the last place of a pre-activation decides a ReLU's gate)
     bool any_split = false;
+    // where given, and the product is split, has dense rows and no addend: it is left as the sums of its splits
+    SplitSums* sums = nullptr;
 };
 // Work that needs no memory path, offered to a product whose 256x256 tiles leave CUs idle: the
 // keep bits of the attention dropout (attention_keep_word) for the first `tiles_done` key tiles of
@@ -295,6 +304,8 @@ bool gemm_pair_takes_third(const GemmShape& g1, const half_t* A1, const half_t* 
                            const GemmEpilogue& ep1, const GemmShape& g2, const half_t* A2, const half_t* B2,
                            half_t* C2, const GemmEpilogue& ep2, float* ws, size_t ws_floats,
                            const PairThird& third);
+// Writes the output of a product that was left as the sums of its splits.
+void launch_split_sums(const SplitSums& sums, half_t* C, long rows, long row, hipStream_t st);
 // Scratch (in floats) that launch_gemm can make use of for this shape; 0 if none.
 size_t gemm_splitk_ws_floats(const GemmShape& g);
 // Which kernel launch_gemm would pick: 0 = scalar fallback, 1 = MFMA.
