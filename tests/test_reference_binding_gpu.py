@@ -80,7 +80,6 @@ def test_positional_exports_through_the_reference_binding(which):
                               *(t.data_ptr() for t in fwd), X.data_ptr(), DX.data_ptr())
     assert rc == 0, lib.sub_last_error()
     torch.cuda.synchronize()
-    lib.destroy(handle)
 
     got = {'SB2': from_layout(Y, 'BJI', ly), 'DX': from_layout(DX, 'BJI', lx)}
     for (name, layout), g in zip(lay['params'], grads):
@@ -96,6 +95,7 @@ def test_positional_exports_through_the_reference_binding(which):
     held = ctypes.create_string_buffer(16)
     lib.sub_tensor_layout.argtypes = [ctypes.c_void_p, ctypes.c_char_p, ctypes.c_char_p]
     assert lib.sub_tensor_layout(handle, b'DROP2', held) == 0, lib.sub_last_error()
+    lib.destroy(handle)
     held = held.value.decode()
     assert held == ('BJU' if which != 'mi355x' else layouts_f['DROP2'])
     drop2 = from_layout(fwd[names.index('DROP2')].reshape(-1).view([sizes[d] for d in held]), 'BJU', held)
