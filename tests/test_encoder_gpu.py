@@ -1014,6 +1014,36 @@ def test_hip_graph_replays_match_eager_and_draw_new_masks():
     assert not torch.equal(replays[0][0], replays[1][0])     # new masks on every replay
 
 
+@pytest.mark.parametrize('dims,act', [((1, 64, 12, 768), 'gelu'),     # feed-forward product in splits, rows of two packs a lane
+                                      ((3, 40, 8, 512), 'relu'),      # rows of one
+                                      ((1, 16, 16, 1024), 'gelu'),    # the attention output's product in splits as well
+                                      ((2, 24, 16, 2048), 'gelu'),    # longer rows: a launch writes the output
+                                      ((1, 1, 8, 512), 'gelu')])
+def test_products_left_as_sums_and_masks_as_bits_change_no_bit(dims, act):
+    """Options 9 and 10 off write every mask as a tensor and every split product's output; nothing else may change."""
+    from substation_amd import Encoder, layouts as L
+    B, Ls, H, E = dims
+    got = []
+    for on in (1, 0):
+        torch.manual_seed(0)
+        enc = Encoder('unused', B, Ls, H, E, L.mi355x_layouts(), torch.float16, 0.1, 0.1, 0.1, 0.1, activation=act,
+                      seed=SEED).cuda()
+        with torch.no_grad():
+            for q in enc.parameters():
+                q.mul_(0.05)
+        enc.set_rng(SEED, 3)
+        for option in (9, 10):
+            enc._handle.set_option(option, on)
+        g = torch.Generator().manual_seed(5)
+        x = torch.randn(B, Ls, E, generator=g).half().cuda().requires_grad_(True)
+        y = enc(x)
+        y.backward(torch.randn(B, Ls, E, generator=g).half().cuda())
+        got.append([y.detach(), x.grad] + [q.grad for q in enc.parameters()])
+    for a, b in zip(*got):
+        assert torch.isfinite(a.float()).all()
+        assert torch.equal(a, b)
+
+
 def _plain_layer(**more):
     from substation_amd import Encoder, layouts as L
     torch.manual_seed(0)
