@@ -164,9 +164,10 @@ int sub_set_attention_mask(void* handle, const void* attn_mask, const char* layo
  * ATTN_DROP_MASK buffer one keep bit per score instead (both buffers must be
  * the ones handed to the matching backward call, as in the reference).  The
  * dropout mask is the same counter-based one as in the separate operators.
- * Needs head size 64 or 128, sequence lengths that are multiples of 128,
- * and feature-contiguous projections (an attention mask set with
- * sub_set_attention_mask is added to the score tiles); otherwise, or with 0,
+ * Needs head size 64 or 128 and feature-contiguous projections (an attention
+ * mask set with sub_set_attention_mask is added to the score tiles; a ReLU layer
+ * whose sequence length is not a multiple of 128 keeps the operators in its
+ * forward pass and takes the kernels in its backward pass); otherwise, or with 0,
  * the operators run separately (results then agree to fp16 rounding, not bit
  * for bit, because probabilities are no longer rounded before the weighted sum).
  * Set the option before the forward call and leave it until after the matching
@@ -174,8 +175,8 @@ int sub_set_attention_mask(void* handle, const void* attn_mask, const char* layo
  * than fall back: a caller that has asked sub_attention_in_registers() and got
  * 1 may then pass token allocations (any non-null pointer) for the four tensors
  * that are neither written nor read -- BETA, ATTN_DROP, DATTN_DROP, DBETA --
- * and needs only 8 bytes per score row behind ALPHA and K/8 bytes per score
- * row behind ATTN_DROP_MASK (both 16-byte aligned). */
+ * and needs only 8 bytes per score row behind ALPHA and K/8 bytes (K rounded up
+ * to a multiple of 128) per score row behind ATTN_DROP_MASK (both 16-byte aligned). */
 #define SUB_OPT_FUSE_ATTENTION 4
 #define SUB_FUSE_REQUIRED 2
 /* SUB_OPT_PAIR_PRODUCTS (default 1): in encoder_backward a data-gradient product

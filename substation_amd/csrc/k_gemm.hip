@@ -205,7 +205,7 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_dma(GemmArgs g) {
         }
         if ((nblocks & 7) == 0) lid = (lid & 7u) * (nblocks >> 3) + (lid >> 3);
     }
-    // (32-bit arithmetic, as in the register-staged kernel)
+    // (32-bit arithmetic)
     const unsigned per_batch = (unsigned)(tiles_m * tiles_n);
     const unsigned bz = lid / per_batch;
     int r = (int)(lid - bz * per_batch);
