@@ -122,11 +122,12 @@ const char* sub_last_error(void);
  * attention scores (fp16 device tensor owned by the caller, layout "JK" or
  * "KJ"; -inf above the diagonal for a causal layer).  As in
  * substation/attention.py:65-68 the mask is added to the raw scores, before the
- * 1/sqrt(P) scaling.  encoder_forward uses it until it is cleared with NULL;
- * encoder_backward needs nothing (masked positions have zero probability).
- * The mask's contents are read by every encoder_forward call (also to find the
- * tiles that are -inf throughout, which the attention kernels pass over) and
- * must stay unchanged until the matching encoder_backward has been issued.
+ * 1/sqrt(P) scaling.  encoder_forward uses it until it is cleared with NULL.
+ * Its contents are read by every encoder_forward call (also to find the tiles
+ * that are -inf throughout, which the attention kernels pass over) and, where
+ * self-attention runs with the scores in registers, by encoder_backward, which
+ * forms the scores again: the mask has to stay set, allocated and unchanged until
+ * the matching encoder_backward has been issued (and, for its memory, has run).
  * Allocates a small table: not to be called during a graph capture. */
 int sub_set_attention_mask(void* handle, const void* attn_mask, const char* layout);
 

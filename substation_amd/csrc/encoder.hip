@@ -1870,11 +1870,9 @@ int sub_op_attention_backward_biases(void* handle, int n_queries, int n_keys, co
 int sub_set_attention_mask(void* handle, const void* attn_mask, const char* layout) {
     return guarded([&] {
         Handle& h = as_handle(handle); need_cfg(h);
-        h.mask_plan_built = false;
-        if (!attn_mask) { h.attn_mask = nullptr; return; }
+        if (!attn_mask) { h.attn_mask = nullptr; h.mask_plan_built = false; return; }
         Layout l = L(h, layout);
         if (l.rank != 2 || !l.has[dJ] || !l.has[dK]) fail("sub_set_attention_mask: layout must be JK or KJ");
-        h.attn_mask = attn_mask; h.l_attn_mask = l;
         const Sizes& z = h.sz;
         if (mha_shape_ok(z.n[dH], z.n[dB], z.n[dJ], z.n[dK], z.n[dP]) && !h.mask_plan) {
             hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -1884,6 +1882,8 @@ int sub_set_attention_mask(void* handle, const void* attn_mask, const char* layo
             hip_check(hipMalloc(&h.mask_plan, bytes), "hipMalloc(mask plan)");
             h.mask_plan_bytes = bytes;
         }
+        h.mask_plan_built = false;
+        h.attn_mask = attn_mask; h.l_attn_mask = l;       // last: a call that fails leaves the mask of before
     });
 }
 

@@ -33,6 +33,8 @@ struct Lib {
     decltype(&sub_set_stream) set_stream = nullptr;
     decltype(&sub_get_option) get_option = nullptr;
     decltype(&sub_attention_in_registers) attention_in_registers = nullptr;
+    decltype(&sub_set_attention_mask) set_attention_mask = nullptr;
+    decltype(&sub_set_rng_counter) set_rng_counter = nullptr;
     decltype(&sub_encoder_forward) encoder_forward = nullptr;
     decltype(&sub_encoder_backward) encoder_backward = nullptr;
 } lib;
@@ -49,6 +51,8 @@ void load(const std::string& path, py::object error) {
     get(lib.set_stream, "sub_set_stream");
     get(lib.get_option, "sub_get_option");
     get(lib.attention_in_registers, "sub_attention_in_registers");
+    get(lib.set_attention_mask, "sub_set_attention_mask");
+    get(lib.set_rng_counter, "sub_set_rng_counter");
     get(lib.encoder_forward, "sub_encoder_forward");
     get(lib.encoder_backward, "sub_encoder_backward");
     g_error = error.release().ptr();
@@ -111,6 +115,12 @@ bool plain(const at::Tensor& X, const std::vector<at::Tensor>& params) {
     return !odd(X) && std::none_of(params.begin(), params.end(), odd);
 }
 
+// An additive attention mask and the order of its dims.
+struct Mask {
+    at::Tensor values;
+    std::string layout;
+};
+
 struct EncoderLayer : std::enable_shared_from_this<EncoderLayer> {
     void* handle;
     py::object keep_alive;            // the Python object that owns `handle`
@@ -122,6 +132,10 @@ struct EncoderLayer : std::enable_shared_from_this<EncoderLayer> {
     py::object workspace;
     std::vector<at::Tensor> kept_fwd, kept_bwd;
     uint64_t generation = 0;
+    // What `handle` holds a bare pointer to from one call to the next.  Kept here and not on the module: a backward pass
+    // that runs after its module is gone keeps this object, and its kernels read the mask.
+    std::shared_ptr<Mask> mask;
+    std::optional<at::Tensor> step_counter;
 
     EncoderLayer(uintptr_t handle_, py::object owner, std::vector<int64_t> in, std::vector<int64_t> out,
                  std::vector<std::vector<int64_t>> params, const std::vector<int64_t>& fwd_numels,
@@ -156,6 +170,18 @@ struct EncoderLayer : std::enable_shared_from_this<EncoderLayer> {
         if (!v)
             raise("this Encoder was built with compact_activation=True but the ReLU gate from the dropout output (option 6) "
                   "is switched off: LIN1 and DROP2MASK would be written through 8-element buffers", PyExc_RuntimeError);
+    }
+    // (the old tensor is let go only once the handle points to the new one)
+    void set_attention_mask(const std::optional<at::Tensor>& values, const std::string& layout) {
+        std::shared_ptr<Mask> m;
+        if (values) m = std::make_shared<Mask>(Mask{*values, layout});
+        check(lib.set_attention_mask(handle, m ? m->values.data_ptr() : nullptr, layout.c_str()), "sub_set_attention_mask");
+        mask = std::move(m);
+    }
+    void set_step_counter(const std::optional<at::Tensor>& counter) {
+        check(lib.set_rng_counter(handle, counter ? static_cast<uint32_t*>(counter->data_ptr()) : nullptr),
+              "sub_set_rng_counter");
+        step_counter = counter;
     }
     void keep(std::vector<at::Tensor>& list, const char* which, const at::Tensor& X) {
         if (list.empty() || list[0].device() != X.device()) list = workspace(which, X).cast<std::vector<at::Tensor>>();
@@ -284,5 +310,7 @@ PYBIND11_MODULE(_host, m) {
         .def_readwrite("generation", &EncoderLayer::generation)
         .def("check_compact", &EncoderLayer::check_compact)
         .def("check_relu_gate", &EncoderLayer::check_relu_gate)
+        .def("set_attention_mask", &EncoderLayer::set_attention_mask)
+        .def("set_step_counter", &EncoderLayer::set_step_counter)
         .def("forward", &EncoderLayer::forward);
 }

@@ -13,7 +13,6 @@ the caller's current stream, and keyword-only extras exist: ``activation``
 """
 import ctypes
 import math
-import types
 import weakref
 
 import torch
@@ -32,7 +31,7 @@ def causal_mask(seq_len, device='cuda', dtype=torch.float16):
 def _python_function(weak, layer, in_shape, out_shape, shapes, workspace):
     """The layer call as a Python autograd function, with a buffer for every named tensor: ``enable_debug=True``, which
     captures them after each pass, and the calls that the native node leaves to it (tracing, forward-mode differentiation,
-    functorch, dispatch modes).  ``layer`` is the native layer, or what stands in for it and only counts the passes."""
+    functorch, dispatch modes).  ``layer`` is the native layer."""
 
     def call(module, name, device, args):
         module._handle.set_stream(torch.cuda.current_stream(device).cuda_stream)
@@ -209,14 +208,11 @@ class Encoder(torch.nn.Module):
                 store[key] = [torch.empty(shape, device=like.device, dtype=torch_dtype) for shape in _shapes(key)]
             return store[key]
 
-        if enable_debug:
-            self._layer = None
-            layer = types.SimpleNamespace(generation=0, check_compact=lambda: None, check_relu_gate=lambda: None)
-        else:
-            self._layer = layer = _lib.host().EncoderLayer(
-                handle.ptr, handle, in_shape, out_shape, _shapes('params'),
-                [math.prod(s) for s in _shapes('forward_interm')], [math.prod(s) for s in _shapes('backward_interm')],
-                self.persistent_workspace, self.compact_attention, self.compact_activation, _workspace)
+        self._layer = layer = _lib.host().EncoderLayer(
+            handle.ptr, handle, in_shape, out_shape, _shapes('params'),
+            [math.prod(s) for s in _shapes('forward_interm')], [math.prod(s) for s in _shapes('backward_interm')],
+            self.persistent_workspace, self.compact_attention, self.compact_activation, _workspace)
+        self._native_calls = not enable_debug
         self._function = None
         self._function_args = (weak, layer, in_shape, out_shape, _shapes, _workspace)
 
@@ -273,16 +269,11 @@ class Encoder(torch.nn.Module):
         tensor over (query, key) positions, e.g. ``causal_mask(L)``; ``None``
         clears it.  It is added to the raw scores, before the 1/sqrt(P) scaling
         (substation/attention.py:65-68)."""
-        if mask is None:
-            self._attn_mask = None
-            self._handle.set_attention_mask(0)
-            return
         L = self.max_seq_len
-        if not (mask.is_cuda and mask.dtype == self.torch_dtype and tuple(mask.shape) == (L, L)
-                and mask.is_contiguous()):
+        if mask is not None and not (
+                mask.is_cuda and mask.dtype == self.torch_dtype and tuple(mask.shape) == (L, L) and mask.is_contiguous()):
             raise ValueError(f'the attention mask is a contiguous [{L}, {L}] fp16 CUDA tensor')
-        self._attn_mask = mask                 # keeps the memory alive
-        self._handle.set_attention_mask(mask.data_ptr(), layout)
+        self._layer.set_attention_mask(mask, layout)
 
     def use_device_step(self, counter=None):
         """Keeps the dropout step in device memory (a one-element int32 CUDA tensor,
@@ -291,15 +282,13 @@ class Encoder(torch.nn.Module):
         step of ``set_rng`` plus this counter, which every forward advances on
         the stream.  Returns the tensor; ``use_device_step(False)`` switches back."""
         if counter is False:
-            self._step_counter = None
-            self._handle.set_rng_counter(0)
+            self._layer.set_step_counter(None)
             return None
         if counter is None:
             counter = torch.zeros(1, dtype=torch.int32, device='cuda')
         if not (counter.is_cuda and counter.dtype == torch.int32 and counter.numel() == 1):
             raise ValueError('the step counter is a one-element int32 CUDA tensor')
-        self._step_counter = counter          # keeps the memory alive
-        self._handle.set_rng_counter(counter.data_ptr())
+        self._layer.set_step_counter(counter)
         return counter
 
     def profile(self):
@@ -311,7 +300,7 @@ class Encoder(torch.nn.Module):
     def forward(self, X):
         """Run the encoder.  X is in ``layouts['input'][1]`` order; the result is
         in ``layouts['output'][1]`` order."""
-        if self._layer is not None:
+        if self._native_calls:
             Y = self._layer.forward(X, self.params)
             if Y is not None:
                 return Y

@@ -1,6 +1,8 @@
 """GPU parity of the whole layer (module API -> C ABI -> HIP kernels) against the
 oracle, tensor by tensor, with the device's own seeded dropout masks fed to the
 oracle.  Tolerance: 1e-2 relative on fp16 outputs and gradients; masks exact."""
+import gc
+
 import numpy as np
 import pytest
 import torch
@@ -1107,3 +1109,48 @@ def test_python_function_gives_the_native_node_bits():
         got.append([y.detach(), x.grad] + [q.grad for q in enc.parameters()])
     for a, b in zip(*got):
         assert torch.equal(a, b)
+
+
+def _masked_layer(act, L=256):
+    """A layer, its input and output gradient, and two masks whose 32 x 32 blocks are visible, masked out and mixed."""
+    from substation_amd import Encoder, causal_mask, layouts as lay
+    torch.manual_seed(0)
+    enc = Encoder('unused', 2, L, 2, 128, lay.mi355x_layouts(), torch.float16, 0.1, 0.1, 0.1, 0.1, activation=act,
+                  seed=SEED).cuda()
+    with torch.no_grad():
+        for q in enc.parameters():
+            q.mul_(0.1)
+    g = torch.Generator().manual_seed(5)
+    x, dy = (torch.randn(2, L, 128, generator=g).half().cuda() for _ in range(2))
+    causal = causal_mask(L)
+    other = torch.flip(causal, (0, 1)) + 2.0 * torch.randn(L, L, generator=g).half().cuda()
+    return enc, x.requires_grad_(), dy, causal, other
+
+
+def _pass(enc, x, dy, mask):
+    x.grad = None
+    enc.zero_grad(set_to_none=True)
+    enc.set_rng(SEED, 0)
+    enc.set_attention_mask(mask)
+    enc(x).backward(dy)
+    return [x.grad] + [q.grad for q in enc.parameters()]
+
+
+def test_backward_pass_of_a_masked_layer_that_is_gone():
+    """The mask belongs to what the backward pass keeps: the memory of a module dropped between the passes is not reused."""
+    enc, x, dy, mask, other = _masked_layer('gelu')
+    want = [t.clone() for t in _pass(enc, x, dy, other)]
+    x.grad = None
+    enc.zero_grad(set_to_none=True)
+    enc.set_rng(SEED, 0)
+    enc.set_attention_mask(other.clone())
+    params = list(enc.parameters())
+    y = enc(x)
+    del enc
+    gc.collect()
+    taken = [torch.full_like(mask, -3.0) for _ in range(16)]        # what the allocator would hand out again
+    y.backward(dy)
+    for a, b in zip(want, [x.grad] + [q.grad for q in params]):
+        assert torch.isfinite(a.float()).all()
+        assert torch.equal(a, b)
+    del taken

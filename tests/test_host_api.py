@@ -5,15 +5,18 @@ exports every symbol include/substation_amd.h declares, layout -> stride algebra
 host twin of the device mask generator against the oracle, configuration errors,
 and the layouts schema.  No GPU call is made."""
 import ctypes
+import gc
 import itertools
 import os
 import re
+import weakref
 
 import numpy as np
 import pytest
+import torch
 
 from oracle import philox_ref as ph
-from substation_amd import _lib, layouts as L
+from substation_amd import Encoder, _lib, layouts as L
 from tests.einsums import EINSUMS, operand_layouts
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -222,3 +225,41 @@ def test_einsum_with_addend_rejects_an_addend_that_is_no_sub_block_of_the_output
     # a null addend
     rc = lib.sub_op_einsum_add(h.ptr, one, s('BJI'), one, s('HPI'), None, s('HP'), one, s('BJHP'), 1.0)
     assert rc < 0 and b'null addend' in lib.sub_last_error()
+
+
+class _CalledCuda(torch.Tensor):
+    """A host tensor that passes for one on the GPU where only its kind and its address are looked at."""
+    is_cuda = True
+
+
+@pytest.mark.parametrize('debug', [False, True])
+def test_what_the_handle_points_to_outlives_the_module(debug):
+    """The native layer, all that a backward pass keeps, owns the attention mask and the step counter; one that takes
+    another's place lets it go, and a call that fails does not."""
+    def owned(dtype, *shape):
+        array = np.zeros(shape, dtype=dtype)
+        return weakref.ref(array), torch.from_numpy(array).as_subclass(_CalledCuda)
+
+    def enc():
+        return Encoder('unused', 1, 8, 2, 32, L.mi355x_layouts(), torch.float16, 0., 0., 0., 0., enable_debug=debug)
+    module = enc()
+    memory = []
+    for call, dtype, shape in ((module.set_attention_mask, np.float16, (8, 8)), (module.use_device_step, np.int32, (1,))):
+        for _ in range(2):
+            ref, t = owned(dtype, *shape)
+            call(t)
+            memory.append(ref)
+            del t
+    ref, t = owned(np.float16, 8, 8)
+    with pytest.raises(_lib.SubstationError):
+        module.set_attention_mask(t, 'JI')
+    del t, call
+    gc.collect()
+    assert [r() is not None for r in memory] == [False, True, False, True] and ref() is None
+    layer = module._layer
+    del module
+    gc.collect()
+    assert [r() is not None for r in memory] == [False, True, False, True]
+    del layer
+    gc.collect()
+    assert all(r() is None for r in memory)
