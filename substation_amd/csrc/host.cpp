@@ -133,7 +133,7 @@ struct EncoderLayer : std::enable_shared_from_this<EncoderLayer> {
     std::vector<at::Tensor> kept_fwd, kept_bwd;
     uint64_t generation = 0;
     // What `handle` holds a bare pointer to from one call to the next.  Kept here and not on the module: a backward pass
-    // that runs after its module is gone keeps this object, and its kernels read the mask.
+    // that runs after its module is gone keeps this object.
     std::shared_ptr<Mask> mask;
     std::optional<at::Tensor> step_counter;
 
@@ -172,11 +172,14 @@ struct EncoderLayer : std::enable_shared_from_this<EncoderLayer> {
                   "is switched off: LIN1 and DROP2MASK would be written through 8-element buffers", PyExc_RuntimeError);
     }
     // (the old tensor is let go only once the handle points to the new one)
-    void set_attention_mask(const std::optional<at::Tensor>& values, const std::string& layout) {
-        std::shared_ptr<Mask> m;
-        if (values) m = std::make_shared<Mask>(Mask{*values, layout});
-        check(lib.set_attention_mask(handle, m ? m->values.data_ptr() : nullptr, layout.c_str()), "sub_set_attention_mask");
+    void use_mask(std::shared_ptr<Mask> m) {
+        if (m == mask) return;
+        check(lib.set_attention_mask(handle, m ? m->values.data_ptr() : nullptr, m ? m->layout.c_str() : "JK"),
+              "sub_set_attention_mask");
         mask = std::move(m);
+    }
+    void set_attention_mask(const std::optional<at::Tensor>& values, const std::string& layout) {
+        use_mask(values ? std::make_shared<Mask>(Mask{*values, layout}) : nullptr);
     }
     void set_step_counter(const std::optional<at::Tensor>& counter) {
         check(lib.set_rng_counter(handle, counter ? static_cast<uint32_t*>(counter->data_ptr()) : nullptr),
@@ -190,8 +193,19 @@ struct EncoderLayer : std::enable_shared_from_this<EncoderLayer> {
     std::optional<at::Tensor> forward(const at::Tensor& X, const std::vector<at::Tensor>& params);
 };
 
+// A backward pass under the mask of its forward pass, whatever has been set since.
+struct MaskScope {
+    EncoderLayer& layer;
+    const std::shared_ptr<Mask> now;
+    MaskScope(EncoderLayer& l, const std::shared_ptr<Mask>& m) : layer(l), now(l.mask) { layer.use_mask(m); }
+    ~MaskScope() {
+        try { layer.use_mask(now); } catch (...) {}   // (one that the handle has taken before)
+    }
+};
+
 struct EncoderBackward : Node {
     std::shared_ptr<EncoderLayer> layer;
+    std::shared_ptr<Mask> mask;          // of the forward pass
     // the parameters as the forward pass read them, X, and the forward intermediates (unless the layer keeps its own)
     std::vector<SavedVariable> saved;
     uint64_t generation = 0;
@@ -236,6 +250,7 @@ struct EncoderBackward : Node {
         p.push_back(X.data_ptr());
         p.push_back(out[0].data_ptr());
         use_current_stream(l.handle, X.device().index());
+        const MaskScope own(l, mask);
         check(lib.encoder_backward(l.handle, p.data(), (int)p.size()), "encoder_backward");
         return out;
     }
@@ -290,6 +305,7 @@ std::optional<at::Tensor> EncoderLayer::forward(const at::Tensor& X_, const std:
         std::shared_ptr<EncoderBackward> node(new EncoderBackward(), torch::autograd::deleteNode);
         node->set_next_edges(torch::autograd::collect_next_edges(X_, params));
         node->layer = shared_from_this();
+        node->mask = mask;
         node->saved.reserve(w.size() + 1 + interm.size());
         for (const auto& t : w) node->saved.emplace_back(t, false);
         node->saved.emplace_back(X, false);
@@ -304,6 +320,7 @@ std::optional<at::Tensor> EncoderLayer::forward(const at::Tensor& X_, const std:
 
 PYBIND11_MODULE(_host, m) {
     m.def("load", &load);
+    py::class_<Mask, std::shared_ptr<Mask>>(m, "Mask");
     py::class_<EncoderLayer, std::shared_ptr<EncoderLayer>>(m, "EncoderLayer")
         .def(py::init<uintptr_t, py::object, std::vector<int64_t>, std::vector<int64_t>, std::vector<std::vector<int64_t>>,
                       const std::vector<int64_t>&, const std::vector<int64_t>&, bool, bool, bool, py::object>())
@@ -311,6 +328,7 @@ PYBIND11_MODULE(_host, m) {
         .def("check_compact", &EncoderLayer::check_compact)
         .def("check_relu_gate", &EncoderLayer::check_relu_gate)
         .def("set_attention_mask", &EncoderLayer::set_attention_mask)
+        .def_property("mask", [](const EncoderLayer& l) { return l.mask; }, &EncoderLayer::use_mask)
         .def("set_step_counter", &EncoderLayer::set_step_counter)
         .def("forward", &EncoderLayer::forward);
 }

@@ -61,6 +61,7 @@ def _python_function(weak, layer, in_shape, out_shape, shapes, workspace):
             interm = tensors(module, 'forward_interm', X)
             layer.generation += 1
             ctx.generation = layer.generation
+            ctx.mask = layer.mask
             weights = [t.contiguous() for t in weights]
             call(module, 'encoder_forward', X.device, [X, *weights, *interm, Y])
             ctx.save_for_backward(*weights, *interm, X)
@@ -80,7 +81,11 @@ def _python_function(weak, layer, in_shape, out_shape, shapes, workspace):
             DX = torch.empty(in_shape, device=DY.device, dtype=DY.dtype)
             interm = tensors(module, 'backward_interm', DY)
             grads = [torch.empty_like(t) for t in ctx.saved_tensors[:len(layouts['params'])]]
-            call(module, 'encoder_backward', DY.device, [DY, *grads, *interm, *ctx.saved_tensors, DX])
+            now, layer.mask = layer.mask, ctx.mask
+            try:
+                call(module, 'encoder_backward', DY.device, [DY, *grads, *interm, *ctx.saved_tensors, DX])
+            finally:
+                layer.mask = now
             if module.enable_debug:
                 for (name, _), t in zip(layouts['backward_interm'], interm):
                     module.debug[name] = t.detach().cpu().numpy()
@@ -268,7 +273,8 @@ class Encoder(torch.nn.Module):
         substation/transformer.py:443-546): ``mask`` is an additive [L, L] fp16 CUDA
         tensor over (query, key) positions, e.g. ``causal_mask(L)``; ``None``
         clears it.  It is added to the raw scores, before the 1/sqrt(P) scaling
-        (substation/attention.py:65-68)."""
+        (substation/attention.py:65-68).  It holds for the forward passes that
+        follow; a backward pass runs under the mask of its own forward pass."""
         L = self.max_seq_len
         if mask is not None and not (
                 mask.is_cuda and mask.dtype == self.torch_dtype and tuple(mask.shape) == (L, L) and mask.is_contiguous()):

@@ -1127,12 +1127,14 @@ def _masked_layer(act, L=256):
     return enc, x.requires_grad_(), dy, causal, other
 
 
-def _pass(enc, x, dy, mask):
+def _pass(enc, x, dy, mask, between=lambda: None, call=None):
     x.grad = None
     enc.zero_grad(set_to_none=True)
     enc.set_rng(SEED, 0)
     enc.set_attention_mask(mask)
-    enc(x).backward(dy)
+    y = (call or enc)(x)
+    between()
+    y.backward(dy)
     return [x.grad] + [q.grad for q in enc.parameters()]
 
 
@@ -1154,3 +1156,27 @@ def test_backward_pass_of_a_masked_layer_that_is_gone():
         assert torch.isfinite(a.float()).all()
         assert torch.equal(a, b)
     del taken
+
+
+@pytest.mark.parametrize('python', [False, True])
+def test_backward_pass_runs_under_the_mask_of_its_forward_pass(python):
+    """A mask that is replaced or cleared between the passes holds from the next forward pass on."""
+    enc, x, dy, causal, other = _masked_layer('gelu')
+    call = (lambda t: enc.encoder_func.apply(t, *enc.params)) if python else enc
+    want = {id(m): [t.clone() for t in _pass(enc, x, dy, m, call=call)] for m in (causal, other, None)}
+    for first, then in ((causal, other), (other, causal), (other, None), (None, causal)):
+        got = _pass(enc, x, dy, first, lambda: enc.set_attention_mask(then), call)
+        for a, b in zip(want[id(first)], got):
+            assert torch.equal(a, b)
+        # two forward passes under different masks, backward in either order; then what is set now still holds
+        ys = []
+        for m in (first, then):
+            enc.set_attention_mask(m)
+            enc.set_rng(SEED, 0)
+            ys.append(call(x))
+        for y, m in ((ys[0], first), (ys[1], then)):
+            got = torch.autograd.grad(y, [x, *enc.params], dy)
+            for a, b in zip(want[id(m)], got):
+                assert torch.equal(a, b)
+        enc.set_rng(SEED, 0)
+        assert torch.equal(call(x), ys[1])
