@@ -206,7 +206,8 @@ struct MaskScope {
 struct EncoderBackward : Node {
     std::shared_ptr<EncoderLayer> layer;
     std::shared_ptr<Mask> mask;          // of the forward pass
-    // the parameters as the forward pass read them, X, and the forward intermediates (unless the layer keeps its own)
+    // the parameters as the forward pass read them, X, and the forward intermediates (those of a layer that keeps its own
+    // too: what hooks on saved tensors see does not depend on who holds the memory)
     std::vector<SavedVariable> saved;
     uint64_t generation = 0;
 
@@ -245,7 +246,7 @@ struct EncoderBackward : Node {
             l.bwd.pointers(scratch.data(), p);
         }
         for (size_t i = 0; i < np; ++i) p.push_back(in[i].data_ptr());
-        if (l.persistent) for (const auto& t : l.kept_fwd) p.push_back(t.data_ptr());
+        if (l.persistent) for (size_t i = np + 1; i < in.size(); ++i) p.push_back(in[i].data_ptr());
         else l.fwd.pointers(in.data() + np + 1, p);
         p.push_back(X.data_ptr());
         p.push_back(out[0].data_ptr());
@@ -306,10 +307,11 @@ std::optional<at::Tensor> EncoderLayer::forward(const at::Tensor& X_, const std:
         node->set_next_edges(torch::autograd::collect_next_edges(X_, params));
         node->layer = shared_from_this();
         node->mask = mask;
-        node->saved.reserve(w.size() + 1 + interm.size());
+        const std::vector<at::Tensor>& held = persistent ? kept_fwd : interm;
+        node->saved.reserve(w.size() + 1 + held.size());
         for (const auto& t : w) node->saved.emplace_back(t, false);
         node->saved.emplace_back(X, false);
-        for (const auto& t : interm) node->saved.emplace_back(t, false);
+        for (const auto& t : held) node->saved.emplace_back(t, false);
         node->generation = generation;
         torch::autograd::set_history(Y, node);
     }

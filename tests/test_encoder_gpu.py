@@ -1180,3 +1180,28 @@ def test_backward_pass_runs_under_the_mask_of_its_forward_pass(python):
                 assert torch.equal(a, b)
         enc.set_rng(SEED, 0)
         assert torch.equal(call(x), ys[1])
+
+
+def test_saved_tensor_hooks_see_the_intermediates_of_a_persistent_workspace():
+    """The same where the layer keeps its buffers: the backward pass reads what the hooks hand back, not the workspace."""
+    enc, (x, dy) = _plain_layer(persistent_workspace=True)
+    x.requires_grad_()
+    enc(x).backward(dy)
+    want = [x.grad.clone()] + [q.grad.clone() for q in enc.parameters()]
+    x.grad = None
+    enc.zero_grad(set_to_none=True)
+    packed = []
+
+    def pack(t):
+        packed.append(tuple(t.shape))
+        return t.cpu()
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t.cuda()):
+        y = enc(x)
+    workspace = enc._workspace['forward_interm']
+    assert len(packed) == 12 + 1 + len(workspace)
+    assert packed[13:] == [tuple(t.shape) for t in workspace]
+    for t in workspace:
+        t.fill_(float('nan'))
+    y.backward(dy)
+    for a, b in zip(want, [x.grad] + [q.grad for q in enc.parameters()]):
+        assert torch.equal(a, b)
