@@ -246,17 +246,14 @@ int sub_set_attention_mask(void* handle, const void* attn_mask, const char* layo
  * bit per element (byte (b*J + j)*I/8 + i/8, bit i%8, canonical order whatever
  * the tensor's layout) in the first B*J*I/8 bytes of the DROP1MASK and DROP3MASK
  * buffers, instead of as 0/1 tensors: 7.5 MiB less to write and to read per mask at
- * B=8, L=512, E=1024.  The activation's, where that dropout runs as an operator of
- * its own and its mask is kept, likewise in the first B*J*U/8 bytes of DROP2MASK
- * (feed-forward size a multiple of 8).  Same results.  Set it to 0 before the forward call when the
+ * B=8, L=512, E=1024.  Same results.  Set it to 0 before the forward call when the
  * mask tensors are wanted (debug capture); both calls must see the same value. */
 #define SUB_OPT_PACKED_MASKS 9
 /* SUB_OPT_SKIP_UNREAD (default 1): intermediates that neither call reads
  * afterwards are not written: ATT keeps the product without its bias (the bias
  * is added in registers, encoder.cu:134-135 writes it back in place), LIN2 is
  * left alone, and where the LayerNorm backward runs as one launch DLN2 and DLN1
- * are left alone, and so are ATT and DROP2_LINW2 where their products were split
- * along k and go into the launch behind them as partial sums.  8 MiB less to write in each of four launches at B=8, L=512,
+ * are left alone.  8 MiB less to write in each of four launches at B=8, L=512,
  * E=1024; outputs and gradients are bit-identical.  Set it to 0 (debug capture
  * does) when those tensors are wanted. */
 #define SUB_OPT_SKIP_UNREAD 10
@@ -277,6 +274,12 @@ int sub_set_attention_mask(void* handle, const void* attn_mask, const char* layo
  * tensor in the configured order, through strided kernels where it must be (what debug capture and
  * a layout search need).  The operator entry points sub_op_* always take the layouts they are given. */
 #define SUB_OPT_PRIVATE_LAYOUTS 11
+/* SUB_OPT_OPAQUE_INTERMEDIATES (default 0; the Python module sets it): the caller hands the intermediates from
+ * encoder_forward to encoder_backward and looks into none of them.  Option 9 then also covers DROP2MASK where the
+ * activation's dropout runs as an operator of its own and its mask is kept (bits in the first B*J*U/8 bytes, feed-forward
+ * size a multiple of 8), and option 10 also ATT and DROP2_LINW2 where their products were split along k and go into the
+ * launch behind them as partial sums.  Same results.  Both calls must see the same value. */
+#define SUB_OPT_OPAQUE_INTERMEDIATES 12
 /* *planned = 1 when, with the handle's sizes, layouts and options as they are
  * now, self-attention runs with the scores in registers
  * (given 16-byte aligned tensors).  No counterpart in the reference. */

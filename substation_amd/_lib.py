@@ -25,6 +25,7 @@ OPT_SIDE_JOBS = 8
 OPT_PACKED_MASKS = 9
 OPT_SKIP_UNREAD = 10
 OPT_PRIVATE_LAYOUTS = 11
+OPT_OPAQUE_INTERMEDIATES = 12
 FUSE_REQUIRED = 2
 
 

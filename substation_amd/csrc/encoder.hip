@@ -237,8 +237,9 @@ struct Handle {
     bool relu_from_output = true;     // ReLU: the backward gate is read off DROP2; LIN1 and DROP2MASK are not produced
     int side_jobs = 1;                // bit 0: CUs that the stacked projections' tiles leave idle draw attention keep bits;
                                       // bit 1: workgroups behind the first LayerNorm launch draw lin1's keep bits
-    bool packed_masks = true;         // DROP1MASK, DROP2MASK and DROP3MASK travel as one bit per element inside their buffers
+    bool packed_masks = true;         // DROP1MASK and DROP3MASK travel as one bit per element inside their buffers
     bool skip_unread = true;          // intermediates that neither pass reads are not written (ATT after its bias, LIN2, DLN2, DLN1)
+    bool opaque = false;              // nobody looks into DROP2MASK (bits as well), ATT and DROP2_LINW2 (left alone as well)
     // where the last forward call's lin1 epilogue left one bit per element of DROP2 (set = positive), or
     // null: the unused SB1_LINW1 buffer of that call.  The backward call reads its gate from there when it
     // is handed the same buffer, and from DROP2 itself otherwise.
@@ -289,7 +290,7 @@ float* static_scratch() {
 
 // Dropout masks as bits (SUB_OPT_PACKED_MASKS), those of the residuals and the activation's: rows must be whole 8-packs.
 bool packed_masks(const Handle& h) { return h.packed_masks && h.sz.n[dI] % 8 == 0; }
-bool packed_act_mask(const Handle& h) { return h.packed_masks && h.sz.n[dU] % 8 == 0; }
+bool packed_act_mask(const Handle& h) { return h.packed_masks && h.opaque && h.sz.n[dU] % 8 == 0; }
 
 PhiloxKey make_key(const Handle& h, uint32_t site, float p) {
     PhiloxKey k;
@@ -1136,7 +1137,7 @@ void forward(Handle& h, const FwdPtrs& t0) {
     // Small products go into the LayerNorm launch behind them as the sums of their splits (ATT and DROP2_LINW2, which
     // nothing else reads, are not written then), where their rows are the tokens in order.
     SplitSums out_sums, lin2_sums;
-    auto as_sums = [&](int tensor, SplitSums& s) { return h.skip_unread && h.lf[tensor].str() == "BJI" ? &s : nullptr; };
+    auto as_sums = [&](int tensor, SplitSums& s) { return h.skip_unread && h.opaque && h.lf[tensor].str() == "BJI" ? &s : nullptr; };
     run_gemm(h, G_OUT, W[WO], F[GAMMA], F[ATT], "out", nullptr, nullptr, as_sums(ATT, out_sums));
     const bool lin1_gelu = lin1_takes_gelu_epilogue(h, W, F);
     const bool lin1_bad = lin1_gelu || (relu_from_output(h) && h.fuse_epilogues && h.gemm[G_LIN1_BAD].ok &&
@@ -1637,6 +1638,7 @@ int sub_get_option(void* handle, int option, int* value) {
         else if (option == SUB_OPT_PACKED_MASKS) *value = h.packed_masks;
         else if (option == SUB_OPT_SKIP_UNREAD) *value = h.skip_unread;
         else if (option == SUB_OPT_PRIVATE_LAYOUTS) *value = h.private_layouts;
+        else if (option == SUB_OPT_OPAQUE_INTERMEDIATES) *value = h.opaque;
         else fail("sub_get_option: unknown option");
     });
 }
@@ -1653,6 +1655,7 @@ int sub_set_option(void* handle, int option, int value) {
         else if (option == SUB_OPT_SIDE_JOBS) h.side_jobs = value & 3;
         else if (option == SUB_OPT_PACKED_MASKS) h.packed_masks = value != 0;
         else if (option == SUB_OPT_SKIP_UNREAD) h.skip_unread = value != 0;
+        else if (option == SUB_OPT_OPAQUE_INTERMEDIATES) h.opaque = value != 0;
         else if (option == SUB_OPT_PRIVATE_LAYOUTS) {
             h.private_layouts = value != 0;
             if (h.configured) plan_layouts(h, h.private_layouts);

@@ -169,6 +169,8 @@ class Encoder(torch.nn.Module):
             self._handle.set_option(_lib.OPT_PACKED_MASKS, 0)
             self._handle.set_option(_lib.OPT_SKIP_UNREAD, 0)
             self._handle.set_option(_lib.OPT_PRIVATE_LAYOUTS, 0)
+        else:
+            self._handle.set_option(_lib.OPT_OPAQUE_INTERMEDIATES, 1)
         # compact_attention: when self-attention runs with the scores in registers,
         # four of the six score-sized tensors ([H,B,J,K]) are never touched and the
         # other two only hold 8 resp. K/8 (K rounded up to 128) bytes per score row; allocate just that

@@ -96,6 +96,7 @@ class LayerTimer:
         # every tensor in the order under test (by default the library would run a configuration with
         # feature-major activations in its own orders and copy at the boundary)
         handle.set_option(self._lib.OPT_PRIVATE_LAYOUTS, 0)
+        handle.set_option(self._lib.OPT_OPAQUE_INTERMEDIATES, 1)       # the launches of the module
         handle.set_stream(self.torch.cuda.current_stream().cuda_stream)
         if profiling:
             handle.profile_enable(True)

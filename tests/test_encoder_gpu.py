@@ -1205,3 +1205,47 @@ def test_saved_tensor_hooks_see_the_intermediates_of_a_persistent_workspace():
     y.backward(dy)
     for a, b in zip(want, [x.grad] + [q.grad for q in enc.parameters()]):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize('dims,split', [((1, 64, 12, 768), ('DROP2_LINW2',)), ((1, 16, 16, 1024), ('ATT', 'DROP2_LINW2'))])
+def test_a_caller_that_looks_into_the_intermediates_finds_them(dims, split):
+    """Without option 12 (a C caller's default) the activation's mask is a 0/1 tensor and the outputs of products that are
+    split along k are written; output and gradients are the same bits as with it.  Sums of 768 (1024) to 4096 products of
+    fp16 values in fp32, rounded once: half a step of fp16, and as much again for the order of the sum."""
+    from substation_amd import Encoder, layouts as L
+    B, Ls, H, E = dims
+    P, U = E // H, 4 * E
+    got, held = [], []
+    for opaque in (1, 0):
+        torch.manual_seed(0)
+        enc = Encoder('unused', B, Ls, H, E, L.mi355x_layouts(), torch.float16, 0.1, 0.1, 0.1, 0.1, activation='gelu',
+                      seed=SEED, persistent_workspace=True).cuda()
+        with torch.no_grad():
+            for q in enc.parameters():
+                q.mul_(0.05)
+        enc.set_rng(SEED, 3)
+        assert enc._handle.get_option(12) == 1
+        enc._handle.set_option(12, opaque)
+        g = torch.Generator().manual_seed(5)
+        x = torch.randn(B, Ls, E, generator=g).half().cuda().requires_grad_(True)
+        enc(x)                                                       # (allocates the workspace)
+        workspace = dict(zip((n for n, _ in enc.layouts['forward_interm']), enc._workspace['forward_interm']))
+        for t in workspace.values():
+            t.fill_(float('nan'))
+        enc.set_rng(SEED, 3)
+        y = enc(x)
+        held.append({n: t.clone() for n, t in workspace.items()})
+        y.backward(torch.randn(B, Ls, E, generator=g).half().cuda())
+        got.append([y.detach(), x.grad] + [q.grad for q in enc.parameters()])
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+    opaque, shown = held
+    assert not torch.isfinite(opaque['DROP2MASK'].float()).all()
+    for name in ('ATT', 'DROP2_LINW2'):
+        assert torch.isnan(opaque[name].float()).all() == (name in split)
+    keep = ph.dropout_mask((B, Ls, U), 0.1, SEED, 2, step=3, dtype=np.float32)
+    assert np.array_equal(shown['DROP2MASK'].float().cpu().numpy(), keep)
+    w = {n: q.detach().double() for n, q in enc.named_parameters()}
+    for name, want in (('ATT', shown['GAMMA'].double().reshape(B * Ls, E) @ w['WO'].reshape(E, H * P).t()),
+                       ('DROP2_LINW2', shown['DROP2'].double().reshape(B * Ls, U) @ w['LINW2'].t())):
+        assert_close(shown[name].reshape(B * Ls, E).float().cpu().numpy(), want.cpu().numpy(), tol=1e-3, name=name)

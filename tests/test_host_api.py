@@ -263,3 +263,11 @@ def test_what_the_handle_points_to_outlives_the_module(debug):
     del layer
     gc.collect()
     assert all(r() is None for r in memory)
+
+
+def test_intermediates_are_opaque_to_the_module_and_open_to_a_c_caller():
+    def enc(debug):
+        return Encoder('unused', 1, 8, 2, 32, L.mi355x_layouts(), torch.float16, 0., 0., 0., 0., enable_debug=debug)
+    assert _handle().get_option(_lib.OPT_OPAQUE_INTERMEDIATES) == 0
+    assert enc(False)._handle.get_option(_lib.OPT_OPAQUE_INTERMEDIATES) == 1
+    assert enc(True)._handle.get_option(_lib.OPT_OPAQUE_INTERMEDIATES) == 0
