@@ -274,6 +274,10 @@ int sub_set_attention_mask(void* handle, const void* attn_mask, const char* layo
  * tensor in the configured order, through strided kernels where it must be (what debug capture and
  * a layout search need).  The operator entry points sub_op_* always take the layouts they are given. */
 #define SUB_OPT_PRIVATE_LAYOUTS 11
+/* encoder_backward takes the staged copies of the input and the weights that the handle made last for those of its own
+ * forward call where they were made from the same addresses.  A caller whose tensors may have come and gone at those
+ * addresses since (saved tensors that are dropped and restored, say) calls this first: the copies are made again. */
+int sub_forget_staged(void* handle);
 /* SUB_OPT_OPAQUE_INTERMEDIATES (default 0; the Python module sets it): the caller hands the intermediates from
  * encoder_forward to encoder_backward and looks into none of them.  Option 9 then also covers DROP2MASK where the
  * activation's dropout runs as an operator of its own and its mask is kept (bits in the first B*J*U/8 bytes, feed-forward

@@ -204,7 +204,7 @@ struct Handle {
     half_t* sX = nullptr; half_t* sY = nullptr; half_t* sDY = nullptr; half_t* sDX = nullptr;
     half_t* sW[SUB_N_PARAMS] = {}; half_t* sDW[SUB_N_PARAMS] = {};
     half_t* staged_fwd = nullptr; half_t* staged_bwd = nullptr;      // the allocations that sX, sY, sW and sDX, sDY, sDW lie in
-    // what the last forward call made sX / sW from (the backward call after it reuses them for the same pointers)
+    // what sX / sW were last made from (a backward call reuses them for the same pointers; see sub_forget_staged)
     const void* staged_x_from = nullptr; const void* staged_w_from[SUB_N_PARAMS] = {};
     int pos_p[SUB_N_PARAMS], pos_f[SUB_N_FWD], pos_b[SUB_N_BWD];   // internal id -> caller position
     Layout lKK, lQQ, lDKK, lDQQ, lWsub, lBsub;
@@ -1567,6 +1567,14 @@ int sub_set_rng(void* handle, uint64_t seed, uint32_t step) {
 
 int sub_set_rng_counter(void* handle, uint32_t* device_step) {
     return guarded([&] { as_handle(handle).step_dev = device_step; });
+}
+
+int sub_forget_staged(void* handle) {
+    return guarded([&] {
+        Handle& h = as_handle(handle);
+        h.staged_x_from = nullptr;
+        for (const void*& w : h.staged_w_from) w = nullptr;
+    });
 }
 
 int sub_encoder_forward(void* handle, void* const* ptrs, int n) {

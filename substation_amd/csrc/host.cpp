@@ -35,6 +35,7 @@ struct Lib {
     decltype(&sub_attention_in_registers) attention_in_registers = nullptr;
     decltype(&sub_set_attention_mask) set_attention_mask = nullptr;
     decltype(&sub_set_rng_counter) set_rng_counter = nullptr;
+    decltype(&sub_forget_staged) forget_staged = nullptr;
     decltype(&sub_encoder_forward) encoder_forward = nullptr;
     decltype(&sub_encoder_backward) encoder_backward = nullptr;
 } lib;
@@ -53,6 +54,7 @@ void load(const std::string& path, py::object error) {
     get(lib.attention_in_registers, "sub_attention_in_registers");
     get(lib.set_attention_mask, "sub_set_attention_mask");
     get(lib.set_rng_counter, "sub_set_rng_counter");
+    get(lib.forget_staged, "sub_forget_staged");
     get(lib.encoder_forward, "sub_encoder_forward");
     get(lib.encoder_backward, "sub_encoder_backward");
     g_error = error.release().ptr();
@@ -132,6 +134,7 @@ struct EncoderLayer : std::enable_shared_from_this<EncoderLayer> {
     py::object workspace;
     std::vector<at::Tensor> kept_fwd, kept_bwd;
     uint64_t generation = 0;
+    uint64_t passes = 0;              // forward and backward passes begun
     // What `handle` holds a bare pointer to from one call to the next.  Kept here and not on the module: a backward pass
     // that runs after its module is gone keeps this object.
     std::shared_ptr<Mask> mask;
@@ -186,6 +189,12 @@ struct EncoderLayer : std::enable_shared_from_this<EncoderLayer> {
               "sub_set_rng_counter");
         step_counter = counter;
     }
+    // Only the pass right behind its forward pass (number `forward` of them all) can know the handle's staged copies by the
+    // addresses they were made from: hooks may have dropped and restored the saved tensors, at addresses of others' by now.
+    void begin_backward(uint64_t forward) {
+        if (passes != forward) check(lib.forget_staged(handle), "sub_forget_staged");
+        ++passes;
+    }
     void keep(std::vector<at::Tensor>& list, const char* which, const at::Tensor& X) {
         if (list.empty() || list[0].device() != X.device()) list = workspace(which, X).cast<std::vector<at::Tensor>>();
     }
@@ -209,7 +218,7 @@ struct EncoderBackward : Node {
     // the parameters as the forward pass read them, X, and the forward intermediates (those of a layer that keeps its own
     // too: what hooks on saved tensors see does not depend on who holds the memory)
     std::vector<SavedVariable> saved;
-    uint64_t generation = 0;
+    uint64_t generation = 0, pass = 0;
 
     std::string name() const override { return "EncoderFunctionBackward"; }
     void release_variables() override {
@@ -252,6 +261,7 @@ struct EncoderBackward : Node {
         p.push_back(out[0].data_ptr());
         use_current_stream(l.handle, X.device().index());
         const MaskScope own(l, mask);
+        l.begin_backward(pass);
         check(lib.encoder_backward(l.handle, p.data(), (int)p.size()), "encoder_backward");
         return out;
     }
@@ -297,6 +307,7 @@ std::optional<at::Tensor> EncoderLayer::forward(const at::Tensor& X_, const std:
         p.push_back(Y.data_ptr());
     }
     ++generation;
+    ++passes;
     {
         py::gil_scoped_release nogil;
         use_current_stream(handle, X.device().index());
@@ -313,6 +324,7 @@ std::optional<at::Tensor> EncoderLayer::forward(const at::Tensor& X_, const std:
         node->saved.emplace_back(X, false);
         for (const auto& t : held) node->saved.emplace_back(t, false);
         node->generation = generation;
+        node->pass = passes;
         torch::autograd::set_history(Y, node);
     }
     return Y;
@@ -327,6 +339,8 @@ PYBIND11_MODULE(_host, m) {
         .def(py::init<uintptr_t, py::object, std::vector<int64_t>, std::vector<int64_t>, std::vector<std::vector<int64_t>>,
                       const std::vector<int64_t>&, const std::vector<int64_t>&, bool, bool, bool, py::object>())
         .def_readwrite("generation", &EncoderLayer::generation)
+        .def_readwrite("passes", &EncoderLayer::passes)
+        .def("begin_backward", &EncoderLayer::begin_backward)
         .def("check_compact", &EncoderLayer::check_compact)
         .def("check_relu_gate", &EncoderLayer::check_relu_gate)
         .def("set_attention_mask", &EncoderLayer::set_attention_mask)

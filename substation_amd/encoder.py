@@ -60,7 +60,8 @@ def _python_function(weak, layer, in_shape, out_shape, shapes, workspace):
             Y = torch.empty(out_shape, device=X.device, dtype=X.dtype)
             interm = tensors(module, 'forward_interm', X)
             layer.generation += 1
-            ctx.generation = layer.generation
+            layer.passes += 1
+            ctx.generation, ctx.pass_number = layer.generation, layer.passes
             ctx.mask = layer.mask
             weights = [t.contiguous() for t in weights]
             call(module, 'encoder_forward', X.device, [X, *weights, *interm, Y])
@@ -83,6 +84,7 @@ def _python_function(weak, layer, in_shape, out_shape, shapes, workspace):
             grads = [torch.empty_like(t) for t in ctx.saved_tensors[:len(layouts['params'])]]
             now, layer.mask = layer.mask, ctx.mask
             try:
+                layer.begin_backward(ctx.pass_number)
                 call(module, 'encoder_backward', DY.device, [DY, *grads, *interm, *ctx.saved_tensors, DX])
             finally:
                 layer.mask = now

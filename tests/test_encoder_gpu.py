@@ -1249,3 +1249,46 @@ def test_a_caller_that_looks_into_the_intermediates_finds_them(dims, split):
     for name, want in (('ATT', shown['GAMMA'].double().reshape(B * Ls, E) @ w['WO'].reshape(E, H * P).t()),
                        ('DROP2_LINW2', shown['DROP2'].double().reshape(B * Ls, U) @ w['LINW2'].t())):
         assert_close(shown[name].reshape(B * Ls, E).float().cpu().numpy(), want.cpu().numpy(), tol=1e-3, name=name)
+
+
+@pytest.mark.parametrize('python', [False, True])
+def test_restored_tensors_are_not_taken_for_what_lay_at_their_addresses(python):
+    """Hooks drop what two forward passes save and restore it for the backward passes, one after the other at the same
+    addresses; under a configuration whose input and weights the layer holds copies of, each pass reads its own."""
+    from substation_amd import Encoder, layouts as L
+    lay = L.reference_layouts('bert-b8-l512-h16-e1024')
+    torch.manual_seed(0)
+    enc = Encoder('unused', 2, 128, 2, 128, lay, torch.float16, 0.0, 0.0, 0.0, 0.0, activation='gelu', seed=SEED).cuda()
+    with torch.no_grad():
+        for q in enc.parameters():
+            q.mul_(0.1)
+    call = (lambda t: enc.encoder_func.apply(t, *enc.params)) if python else enc
+    shape = tuple(enc.sizes[d] for d in lay['input'][1])
+    g = torch.Generator().manual_seed(5)
+    host = [torch.randn(shape, generator=g).half() for _ in range(2)]
+    dy = torch.randn(tuple(enc.sizes[d] for d in lay['output'][1]), generator=g).half().cuda()
+    want = []
+    for t in host:
+        y = call(t.cuda())
+        want.append([q.clone() for q in torch.autograd.grad(y, enc.params, dy)])
+    addresses = []
+
+    def restore(t):
+        t = t.cuda()
+        if t.shape == shape:
+            addresses.append(t.data_ptr())
+        return t
+    for order in ((1, 0), (0, 1)):
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), restore):
+            ys = [call(t.cuda()) for t in host]
+        for i in order:
+            for a, b in zip(want[i], torch.autograd.grad(ys[i], enc.params, dy)):
+                assert torch.equal(a, b)
+        # a forward pass of another input in between, that leaves its address to the restored one
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), restore):
+            y = call(host[0].cuda())
+        with torch.no_grad():
+            call(host[1].cuda())
+        for a, b in zip(want[0], torch.autograd.grad(y, enc.params, dy)):
+            assert torch.equal(a, b)
+    assert len(set(addresses)) < len(addresses)          # otherwise nothing was tested
