@@ -1,14 +1,18 @@
 // Contractions in a ring of LDS stages with waves of their own for the fetching; one launch takes up to three products.
 //
-// What bounds a product here is how fast a CU draws its operands: about 35 bytes a cycle of whatever it is that the
-// L2s do not hold, whether all CUs draw or half of them.  A wave that issues an asynchronous load waits until the memory
-// path has taken it, so when the multiplying waves fetched as well, a step of 64 k of a 128 x 128 tile took the 640
-// cycles that its 32 KiB take plus the 512 of its matrix instructions.  Here four waves only fetch and the others
+// What bounds a product here is how fast a CU draws its operands: 51 bytes a cycle of lines that its L2 has, 12 of lines
+// that it has not, so about 31 where a fifth is missing (4096 x 1024 x 4096: 512 MiB drawn, 104 of them from beyond the L2s;
+// its 36 us are what the fetch alone takes at those two rates).  A wave that issues an asynchronous load waits until the
+// memory path has taken it, so when the multiplying waves fetched as well, a step of 64 k of a 128 x 128 tile took the
+// cycles that its 32 KiB take (640 at best) plus the 512 of its matrix instructions.  Here four waves only fetch and the others
 // only multiply, and a workgroup stays on its CU: while it writes one tile, the first stages of its next one are on their way.
 // Tiles with remainders are read and written through range-checked buffers, so a 128 x 128 tile at the edge costs what
 // one inside does (the kernel before predicated every load of such a product).  M = 2613 rows, us before and now:
 // 768 x 3072 (n x k) 35 -> 21, 3072 x 768 21 -> 18.5, its weight gradient 42 -> 20.5; 64 rows x 768 x 768: 14 -> 6.4; 4096 x 1024 x
-// 4096: 43 -> 35 (990 TFLOP/s).  Of the 12 us that 4096 x 1024 x 1024 takes, 2 are the way to the first step, 1.2 the tile's way out.
+// 4096: 43 -> 35-37 (930 to 990 TFLOP/s, box to box).  4096 x 1024 x 1024, one tile of 16 steps per CU, takes 15 to 17 us.
+// Registers: 72 to 168 a lane up to 128 x 128 tiles, 242 to 256 at 256 x 128, where the instance of two orientations (two
+// loop bodies) spills two of them (12 bytes of scratch); the instances of one product hold its arguments in scalar
+// registers and spill 25 to 36 of those, the ones of several products none.
 #include <algorithm>
 #include <type_traits>
 
@@ -542,7 +546,8 @@ TileChoice choose_tiles(const TileProduct* p, int n, unsigned forms, size_t ws_f
     int order[kMaxProducts] = {0, 1, 2};
     std::sort(order, order + n, [&](int x, int y) { return steps_of(p[x].a, p[x].a.splits) > steps_of(p[y].a, p[y].a.splits); });
     const GemmArgs& longest = p[order[0]].a;
-    // The longest contraction in parts: a reduction follows (about 3 us and a pass over the partial sums).
+    // The longest contraction in parts: a reduction follows (about 3 us and a pass over the partial sums; charged as well
+    // where the LayerNorm launch behind takes the parts themselves and none runs, so such products are split less than pays).
     const bool free_split = ws_floats > 0 && longest.splits == 1 && longest.N % 4 == 0;
     for (int s = 1; s <= (free_split ? 8 : 1); ++s) {
         const size_t partial = (size_t)longest.nbatch * longest.M * longest.N * s;
