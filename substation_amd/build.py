@@ -18,7 +18,8 @@ LIB_DIR = os.path.join(HERE, 'lib')
 LIB = os.path.join(LIB_DIR, 'libsubstation_amd.so')
 HOST_LIB = os.path.join(LIB_DIR, '_host.so')       # the host side of a layer call (torch extension module)
 SOURCES = ['encoder.hip', 'k_rows.hip', 'k_elem.hip', 'k_cols.hip', 'k_lnbwd.hip', 'k_attn.hip', 'k_mha.hip', 'k_relayout.hip', 'k_probe.hip', 'k_gemm.hip',
-           'k_gemm_tiles.hip']
+           'k_gemm_tiles.hip', 'k_gemm_wide.hip',
+           *(('k_gemm_wide_act.hip', f'-DSUB_EPI={epi}') for epi in range(1, 6))]
 FLAGS = ['--offload-arch=gfx950', '-O3', '-std=c++17', '-fPIC', '-Wall', '-Wno-unused-function',
          # packed-fp32 VALU forms are switched off for every kernel of this library
          '-Xclang', '-target-feature', '-Xclang', '-packed-fp32-ops']
@@ -63,8 +64,9 @@ def build(verbose=False, jobs=8):
     hipcc = _hipcc()
 
     def compile_one(src):
-        obj = os.path.join(OBJ, src.replace('.hip', '.o'))
-        out = _run([hipcc, *FLAGS, *EXTRA_FLAGS.get(src, []), '-c', os.path.join(CSRC, src), '-o', obj])
+        src, *defines = [src] if isinstance(src, str) else src
+        obj = os.path.join(OBJ, src.replace('.hip', ''.join(defines) + '.o'))
+        out = _run([hipcc, *FLAGS, *EXTRA_FLAGS.get(src, []), *defines, '-c', os.path.join(CSRC, src), '-o', obj])
         if verbose and out.strip():
             print(out)
         return obj

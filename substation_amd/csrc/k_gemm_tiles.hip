@@ -13,49 +13,11 @@
 // Registers: 72 to 168 a lane up to 128 x 128 tiles, 242 to 256 at 256 x 128, where the instance of two orientations (two
 // loop bodies) spills two of them (12 bytes of scratch); the instances of one product hold its arguments in scalar
 // registers and spill 25 to 36 of those, the ones of several products none.
-#include <algorithm>
-#include <type_traits>
-
-#include "sub_finish.hpp"
-#include "sub_gemm.hpp"
+#include "sub_tiles.hpp"
 
 namespace sub {
 
 namespace {
-
-typedef uint32_t u4v __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ unsigned lds_addr(const void* p) {
-    return (unsigned)(uintptr_t)(__attribute__((address_space(3))) const void*)p;
-}
-// What lies behind `at` in LDS may have changed.
-__device__ __forceinline__ void lds_fence(unsigned at) { asm volatile("" ::"v"(at) : "memory"); }
-
-// 16 bytes per lane from buffer `r` into LDS at `lds` + 16 * lane; zeros from beyond the buffer's end.  Spelled out
-// because of what the compiler makes of its own form of it: a transposing read from LDS, which it cannot tell from
-// a read of bytes on their way, then waits for every load in flight, so that a step takes a round trip to memory
-// (1100 cycles for 64 k of a 64 x 64 tile, where 500 do).  The waits that are needed stand in the loops.
-__device__ __forceinline__ void load_to_lds(unsigned lds, unsigned voff, u4v r) {
-    // (all but voff are the same in every lane; m0 holds nothing else in these kernels)
-    auto u = [](uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); };
-    const u4v ru = {u(r[0]), u(r[1]), u(r[2]), u(r[3])};
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-                 ::"s"(u(lds)), "v"(voff), "s"(ru));
-}
-
-// Logical index of workgroup b of n such that the ones that the eight XCDs get in turn are consecutive on one XCD.
-__device__ __forceinline__ unsigned xcd_order(unsigned b, unsigned n) {
-    const unsigned q = n >> 3, r = n & 7u, x = b & 7u;
-    return x * q + (x < r ? x : r) + (b >> 3);
-}
-
-template <typename T>
-__device__ __forceinline__ T* uniform(T* p) {
-    const uint64_t v = reinterpret_cast<uint64_t>(p);
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
-    const uint32_t up = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
-    return reinterpret_cast<T*>(((uint64_t)up << 32) | lo);
-}
 
 // NM matrix instructions with NR reads from LDS dealt out evenly in front of them (and NV vector instructions behind each).
 template <int m, int NM, int NR, int NV = 0>
@@ -69,27 +31,16 @@ __device__ __forceinline__ void deal_reads() {
     }
 }
 
-struct NoJobs { int n = 0; };
-template <int NP>
-struct TileGroup {
-    GemmArgs g[NP];
-    unsigned end[NP];                 // products' tiles in the launch's list: those of product p end at end[p]
-    unsigned second[NP];              // operands read the way of K2 (see k_gemm_ring)
-    unsigned n = 0, workers = 0;      // products; workgroups that take tiles
-    unsigned tail_groups = 0;
-    typename std::conditional<NP == 1, NoJobs, FinishJobs>::type tail;     // column sums of earlier launches, finished by the workgroups behind those
-};
-
-// (the launch's arguments where they lie: an index into them that is not a constant would otherwise have them copied
-// into scratch memory)
-typedef const __attribute__((address_space(4))) GemmArgs Args;
-
 // 32 TM WM x 32 TN WN outputs per tile, WM x WN waves that multiply, NL that fetch, S stages of 64 k.
 // K1, K2: which operands are contiguous along k (bit 0: A, bit 1: B), of products with `second` clear and set.
 template <int TM, int TN, int WM, int WN, int NL, int S, int NP, int K1, int K2>
-struct Ring {
-    typedef const __attribute__((address_space(4))) TileGroup<NP> Group;
-    static constexpr int NC = WM * WN, BM = 32 * TM * WM, BN = 32 * TN * WN, STAGE = (BM + BN) * BK;
+struct Ring : TileList<32 * TM * WM, 32 * TN * WN, NP> {
+    static constexpr int NC = WM * WN, BM = 32 * TM * WM, BN = 32 * TN * WN;
+    typedef TileList<BM, BN, NP> List;
+    typedef typename List::Group Group;
+    typedef typename List::Tile Tile;
+    using List::tile_of;
+    static constexpr int STAGE = (BM + BN) * BK;
     static constexpr int PITCH = 32 * TN + 8, SLAB = 16 * PITCH;      // a wave's slab of 16 output rows
     static constexpr int HALVES = S * STAGE + NC * SLAB;
     static constexpr int LPR = 4 * TN, RPI = 64 / LPR;                // lanes per output row, rows per store
@@ -98,55 +49,6 @@ struct Ring {
     using TBK = DTile<BN, true, NL>;
     using TBF = DTile<BN, false, NL>;
     static constexpr int LA = TAK::NV, LB = TBK::NV, L = LA + LB;     // loads per fetching wave and stage
-
-    // One tile of the list.
-    struct Tile {
-        int p;                        // product
-        int m0, n0, kt_begin, nkt;
-        unsigned split, bz;
-        long b0, b1, b2;
-    };
-    static __device__ __forceinline__ void locate(Group& G, unsigned id, Tile& t) {
-        t.p = 0;
-        unsigned first = 0;
-        if constexpr (NP > 1) {
-            if (G.n > 1 && id >= G.end[0]) { t.p = 1; first = G.end[0]; }
-            if (G.n > 2 && id >= G.end[1]) { t.p = 2; first = G.end[1]; }
-        }
-        Args& g = G.g[t.p];
-        id -= first;
-        // (a division is some 30 instructions in front of a workgroup's first load: those of the common product are left out)
-        const unsigned tiles_m = (unsigned)(g.M + BM - 1) / BM, tiles_n = (unsigned)(g.N + BN - 1) / BN;
-        t.split = 0; t.kt_begin = 0;
-        t.nkt = g.K0 * ((g.K1 + BK - 1) / BK);
-        if (g.splits > 1) {
-            const unsigned ns = (unsigned)g.splits, nkt = (unsigned)t.nkt, rest = id / ns;       // k-splits of one tile sit next to each other
-            t.split = id - rest * ns; id = rest;
-            t.kt_begin = (int)(nkt * t.split / ns);
-            t.nkt = (int)(nkt * (t.split + 1) / ns) - t.kt_begin;
-        }
-        t.bz = 0; t.b0 = t.b1 = t.b2 = 0;
-        if (g.nbatch > 1) {
-            const unsigned per_batch = tiles_m * tiles_n;
-            t.bz = id / per_batch;
-            id -= t.bz * per_batch;
-            const unsigned tq = t.bz / (unsigned)g.nb2;
-            t.b2 = t.bz - tq * (unsigned)g.nb2; t.b0 = tq / (unsigned)g.nb1; t.b1 = tq - (unsigned)t.b0 * (unsigned)g.nb1;
-        }
-        // tiles that run together on an XCD share operand panels: groups of GM tile rows
-        constexpr unsigned GM = BM > BN ? 4 : 8;
-        const unsigned grp = tiles_m <= GM ? 0 : id / (GM * tiles_n), first_m = grp * GM, gsz = min(tiles_m - first_m, GM);
-        const unsigned rr = id - grp * GM * tiles_n, col = gsz == GM ? rr / GM : rr / gsz;
-        t.m0 = (int)((first_m + rr - col * gsz) * BM); t.n0 = (int)(col * BN);
-    }
-    // The r-th tile of logical workgroup l of n: rounds of n; what is left of the last one goes to the workgroups from the
-    // other end (the list starts with the longest contractions).
-    static __device__ __forceinline__ bool tile_of(Group& G, unsigned l, unsigned n, unsigned r, Tile& t) {
-        const unsigned total = NP == 1 ? G.end[0] : G.end[G.n - 1], id = r * n + ((r + 1) * n <= total ? l : n - 1 - l);
-        if (id >= total) return false;
-        locate(G, id, t);
-        return true;
-    }
 
     // ---- the fetching waves ---------------------------------------------------------------------------------------
     // One operand of the product at hand.
@@ -485,30 +387,15 @@ __global__ __launch_bounds__((WM * WN + NL) * 64) void k_gemm_ring(TileGroup<NP>
 
 // The tiles there are, and what they take (us): a step of 64 k with few workgroups, with one on every second CU (two
 // share a CU: on every CU), and in every place; a launch with the way into and out of its first tile; a tile's way out
-// where all CUs are on theirs.  From products of 64 .. 8192 rows with 1 .. 256 steps.  256 x 256 is k_gemm_dma.
+// where all CUs are on theirs.  From products of 64 .. 8192 rows with 1 .. 256 steps.  256 x 256 is k_gemm_wide.
 struct Form { int bm, bn, per_cu; double few, half, full, once, out; };
 constexpr Form kForms[TILE_FORMS] = {
     {64, 64, 2, 0.20, 0.20, 0.38, 3.6, 1.6},
     {128, 64, 2, 0.29, 0.33, 0.59, 3.8, 2.0},
     {128, 128, 1, 0.33, 0.37, 0.47, 4.4, 2.0},
     {256, 128, 1, 0.52, 0.54, 0.83, 5.9, 2.0},
-    {256, 256, 1, 0.90, 1.00, 1.68, 5.0, 3.5},
+    {256, 256, 1, 1.00, 1.00, 1.42, 5.5, 4.3},
 };
-
-long tiles_of(const GemmArgs& a, int splits, const Form& f) {
-    return ((a.M + f.bm - 1) / f.bm) * (long)((a.N + f.bn - 1) / f.bn) * a.nbatch * splits;
-}
-long steps_of(const GemmArgs& a, int splits) { return ((long)a.K0 * ((a.K1 + BK - 1) / BK) + splits - 1) / splits; }
-
-// Products of one launch may be read in one way, or in the two of which an instance exists.
-bool orientations(const TileProduct* p, int n, int& k1, int& k2) {
-    int seen = 0;
-    for (int i = 0; i < n; ++i) seen |= 1 << ((p[i].akc ? 1 : 0) | (p[i].bkc ? 2 : 0));
-    for (int k = 0; k < 4; ++k)
-        if (seen == 1 << k) { k1 = k2 = k; return true; }
-    k1 = 1; k2 = 0;
-    return seen == 3;
-}
 
 // The launch's rounds: its list has the longest contractions in front, and a round lasts as long as its longest tile.
 double launch_us(const long* len, const long* cnt, int n, const Form& F) {
@@ -560,7 +447,7 @@ TileChoice choose_tiles(const TileProduct* p, int n, unsigned forms, size_t ws_f
                 const GemmArgs& a = p[order[i]].a;
                 const int splits = i == 0 && s > 1 ? s : a.splits;
                 len[i] = steps_of(a, splits);
-                cnt[i] = tiles_of(a, splits, kForms[f]);
+                cnt[i] = tiles_of(a, splits, kForms[f].bm, kForms[f].bn);
             }
             for (int i = 0; i + 1 < n && len[i] < len[i + 1]; ++i) { std::swap(len[i], len[i + 1]); std::swap(cnt[i], cnt[i + 1]); }
             const double t = launch_us(len, cnt, n, kForms[f]) + reduce;
@@ -573,26 +460,8 @@ TileChoice choose_tiles(const TileProduct* p, int n, unsigned forms, size_t ws_f
 template <int NP>
 static void launch_tiles_n(const TileProduct* p, int n, int form, FinishJobs* tail, hipStream_t st) {
     TileGroup<NP> G;
-    int k1 = 0, k2 = 0, order[kMaxProducts] = {0, 1, 2};
-    if (n < 1 || n > NP || !orientations(p, n, k1, k2)) fail("gemm: these products do not share a launch");
-    std::sort(order, order + n, [&](int x, int y) { return steps_of(p[x].a, p[x].a.splits) > steps_of(p[y].a, p[y].a.splits); });
-    const Form& F = kForms[form];
-    long total = 0;
-    for (int i = 0; i < n; ++i) {
-        const TileProduct& q = p[order[i]];
-        G.g[i] = q.a;
-        G.second[i] = ((q.akc ? 1 : 0) | (q.bkc ? 2 : 0)) != k1;
-        total += tiles_of(q.a, q.a.splits, F);
-        if (total > 0x7fffffffL) fail("gemm: too many tiles");
-        G.end[i] = (unsigned)total;
-    }
-    G.n = (unsigned)n;
-    G.workers = (unsigned)std::min(total, 256L * F.per_cu);
-    if constexpr (NP > 1)
-        if (tail && tail->n > 0) {
-            const long groups = finish_groups(*tail);
-            if (groups * tail->n <= 4096) { G.tail = *tail; G.tail_groups = (unsigned)groups; tail->n = 0; }
-        }
+    int k1, k2;
+    list_tiles<NP>(G, p, n, kForms[form].bm, kForms[form].bn, 256L * kForms[form].per_cu, tail, k1, k2);
     const dim3 grid(G.workers + (unsigned)G.tail.n * G.tail_groups), block(512);
 #define SUB_RING(...)                                                                                                        \
     do {                                                                                                                     \
@@ -613,6 +482,7 @@ static void launch_tiles_n(const TileProduct* p, int n, int form, FinishJobs* ta
 }
 
 void launch_tiles(const TileProduct* p, int n, int form, FinishJobs* tail, hipStream_t st) {
+    if (form == TILE_256x256) { launch_wide(p, n, tail, 0, st); return; }
     if (n == 1 && !(tail && tail->n)) launch_tiles_n<1>(p, n, form, tail, st);
     else launch_tiles_n<kMaxProducts>(p, n, form, tail, st);
 }

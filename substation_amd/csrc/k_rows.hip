@@ -209,7 +209,7 @@ __global__ __launch_bounds__(BLOCK) void k_bdrln(RowSpace rs, View in, View resi
         const uint32_t tiles_n = side.N / 256, items = (side.M / 256) * tiles_n * 512;
         for (uint32_t id = (blockIdx.x - row_blocks) * BLOCK + threadIdx.x; id < items; id += side.blocks * BLOCK) {
             const uint32_t tile = id >> 9, tm = tile / tiles_n;
-            const KeepWords k = relu_dropout_keep_words(skey, side.N, tm, tile - tm * tiles_n, (id >> 6) & 7, id & 63);
+            const KeepWords k = relu_dropout_keep_words(skey, side.N, tm, tile - tm * tiles_n, (id >> 7) & 3, (id >> 6) & 1, id & 63);
             reinterpret_cast<uint4*>(side.out)[id] = make_uint4(k.w[0], k.w[1], k.w[2], k.w[3]);
         }
         return;
@@ -364,7 +364,7 @@ __global__ __launch_bounds__(BLOCK) void k_bdrln_flat(int R, unsigned nrows, Vie
         const uint32_t tiles_n = side.N / 256, items = (side.M / 256) * tiles_n * 512;
         for (uint32_t id = (blockIdx.x - row_blocks) * BLOCK + threadIdx.x; id < items; id += side.blocks * BLOCK) {
             const uint32_t tile = id >> 9, tm = tile / tiles_n;
-            const KeepWords k = relu_dropout_keep_words(skey, side.N, tm, tile - tm * tiles_n, (id >> 6) & 7, id & 63);
+            const KeepWords k = relu_dropout_keep_words(skey, side.N, tm, tile - tm * tiles_n, (id >> 7) & 3, (id >> 6) & 1, id & 63);
             reinterpret_cast<uint4*>(side.out)[id] = make_uint4(k.w[0], k.w[1], k.w[2], k.w[3]);
         }
         return;

@@ -22,7 +22,7 @@ struct GemmArgs {
     int splits;                   // > 1: the k range is split, fp32 partial tiles go to `partial`
     float* partial;               // [split][batch][M][N]
     long nbatch = 1;              // batches in all
-    int relu_dropout = 0;         // epilogue of the asynchronous kernel: ReLU and dropout after the addend
+    int relu_dropout = 0;         // epilogue of the 256 x 256 tiles: ReLU and dropout after the addend
     PhiloxKey key;
     const half_t* gate = nullptr; // or: zero where gate <= 0 (strides of `bias`), column sums per 128-row slab
     float* colsum = nullptr;
@@ -31,7 +31,7 @@ struct GemmArgs {
     const uint32_t* gate_bits = nullptr;   // gate: those bits instead of the values of `gate`
     int act = ACT_RELU;                    // the activation of relu_dropout / gate (GemmEpilogue::act)
     half_t* pre_out = nullptr;             // GELU with dropout: where the rounded sum before the activation goes
-    // GemmSideJob of the eight-wave asynchronous kernel: workgroups side_first .. gridDim.x - 1 draw
+    // GemmSideJob of the 256 x 256 kernel: workgroups side_first .. gridDim.x - 1 draw
     // the attention keep words of key tiles 0 .. side_tiles_done - 1 of side_rows score rows
     unsigned side_first = 0, side_blocks = 0;
     PhiloxKey side_key;
@@ -102,13 +102,7 @@ struct DTile {
     // idx-th 32-row block below row0 at k-step ks lies at
     //   (base ^ ((2 ks ^ 4 (idx & 1)) * 8)) + idx * 32 * BK
     // (32 rows further the swizzle flips bit 2 of the slot, a k-step further the slot moves
-    // by 2, and neither carries).  The eight-wave kernel computes that inside its loop from a
-    // value the compiler cannot see through: left to itself it keeps all 24 addresses of a
-    // wave in registers across the loop and spills other things.  (The four-wave kernel has
-    // the registers and got slower with it: 40 -> 43 us at M = 4096, N = 1024, K = 4096.)
-    static __device__ __forceinline__ int frag_base(int row0, int lane) {
-        return kc_off(row0 + (lane & 31), lane >> 5);
-    }
+    // by 2, and neither carries).
     static __device__ __forceinline__ h8 frag_at(const half_t* lds, int base, int idx, int ks) {
         return *reinterpret_cast<const h8*>(lds + ((base ^ (((2 * ks) ^ (4 * (idx & 1))) * 8)) + idx * 32 * BK));
     }
@@ -151,6 +145,10 @@ bool tiles_take(const TileProduct& p);                        // within the rang
 // The best of `forms` (a bit each).  ws_floats > 0: the longest contraction may be split over that much scratch.
 TileChoice choose_tiles(const TileProduct* p, int n, unsigned forms, size_t ws_floats);
 // `tail`: column sums of earlier launches, finished by workgroups behind the tiles (tail->n = 0 then).
+// k_gemm_wide.hip: 256 x 256 tiles, the ones that carry an activation in their epilogue among them (of a single product).
+bool wide_takes(const TileProduct& p);
+// side_blocks: workgroups behind the tiles, for GemmArgs::side_*
+void launch_wide(const TileProduct* p, int n, FinishJobs* tail, unsigned side_blocks, hipStream_t st);
 void launch_tiles(const TileProduct* p, int n, int form, FinishJobs* tail, hipStream_t st);
 
 }  // namespace sub

@@ -27,7 +27,7 @@ void launch_bs(const RowSpace& rs, View alpha, View mask, View ddrop, View dbeta
 // Side job of launch_bdrln (a launch that waits for memory with its vector units idle): `blocks`
 // workgroups behind those of the rows draw the keep words of the ReLU-dropout epilogue
 // (relu_dropout_keep_words) of a later product with a dense [M][N] output in 256x256 tiles, word
-// quadruple ((tile_m * N/256 + tile_n) * 8 + wave) * 64 + lane of `out` (M * N / 8 bytes).
+// quadruple (((tile_m * N/256 + tile_n) * 4 + wave) * 2 + half) * 64 + lane of `out` (M * N / 8 bytes).
 // A product of dense rows left as the fp32 sums of its k splits: fp16(alpha * their sum) is its output, wherever that is read.
 struct SplitSums {
     const float* p = nullptr;    // [splits][rows][row]; null: the output itself was written
@@ -274,7 +274,7 @@ struct GemmSideJob {
 void launch_gemm(const GemmShape& g, const half_t* A, const half_t* B, half_t* C, float alpha,
                  const GemmEpilogue& ep, hipStream_t st, float* ws = nullptr, size_t ws_floats = 0,
                  GemmSideJob* side = nullptr);
-// Can launch_gemm apply ep.relu_dropout to this product?  Only the asynchronous kernel with
+// Can launch_gemm apply ep.relu_dropout to this product?  Only the kernel with
 // 256x256 tiles does, on a single dense row-major output.
 bool gemm_relu_dropout_ok(const GemmShape& g, const void* A, const void* B, const void* C, const GemmEpilogue& ep);
 // A third product offered to launch_gemm_pair: taken (and `taken` set) when its tiles in that launch are

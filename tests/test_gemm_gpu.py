@@ -68,9 +68,8 @@ def test_k_remainder_and_tile_edges():
 
 @pytest.mark.parametrize('E,H', [(192, 3), (64, 1), (128, 2)])
 def test_wide_tiles_every_operand_orientation(E, H):
-    """4096 x 4096 outputs take the 256 x 256 tiles of the asynchronous kernel with
-    eight waves: each operand k-contiguous or not, with an odd number of 64-deep
-    k-tiles (three, one) and an even one."""
+    """4096 x 4096 outputs take 256 x 256 tiles: each operand k-contiguous or not, with
+    an odd number of 64-deep k-tiles (three, one) and an even one."""
     from substation_amd.ops import Ops
     o = Ops(8, 512, H, E, intermediate_size=4096)
     sz = o.sizes
@@ -190,3 +189,50 @@ def test_products_sharing_a_launch(B, L, H, E, U):
         w2 = np.einsum(f'{la2},{lb2}->{lc2}'.lower(), d[la2].double().cpu(), d[lb2].double().cpu(), optimize=True)
         assert_close(C1.double().cpu().numpy(), w1, name=f'{la1},{lb1}->{lc1}')
         assert_close(C2.double().cpu().numpy(), w2, name=f'{la2},{lb2}->{lc2}')
+
+
+@pytest.mark.parametrize('B,L,E,U', [(1, 4104, 1024, 4104), (4, 1000, 1032, 4096), (13, 208, 2048, 8192)])
+def test_wide_tiles_with_remainders(B, L, E, U):
+    """256 x 256 tiles whose last row and column of tiles are not whole, a contraction that is not a multiple of 64 where
+    neither operand lies along it, an outer and an inner contraction, several tiles per workgroup, a scale, a bias row and
+    a whole addend, and a data gradient beside a weight gradient (the two ways of reading A in one launch).  fp16
+    operands, fp32 sums, one rounding: 2^-11 of the value, and sums of up to 8192 terms to 1e-5 of their rms."""
+    from substation_amd.ops import Ops
+    o = Ops(B, L, 8, E, intermediate_size=U)
+    sz = o.sizes
+    g = torch.Generator(device='cuda').manual_seed(E)
+    mk = lambda lay: torch.randn(tuple(sz[d] for d in lay), generator=g, device='cuda').half()
+    nan = lambda lay: torch.full(tuple(sz[d] for d in lay), float('nan'), dtype=torch.float16, device='cuda')
+
+    def want(la, A, lb, Bm, lc, alpha=1.0, T=None, lt=None):
+        k = [d for d in la if d in lb and d not in lc]
+        ma, nb = [d for d in la if d in lc], [d for d in lb if d in lc]
+        mat = lambda X, l, r, c: X.double().permute([l.index(d) for d in r + c]).reshape(int(np.prod([sz[d] for d in r])), -1)
+        W = (alpha * torch.mm(mat(A, la, ma, k), mat(Bm, lb, k, nb))).half()
+        W = W.reshape([sz[d] for d in ma + nb]).permute([(ma + nb).index(d) for d in lc])
+        if T is None:
+            return W.double()
+        return W.double() + T.double().reshape([sz[d] if d in lt else 1 for d in lc])
+
+    def check(C, W, name):
+        err = (C.double() - W).abs() - 2.0 ** -10 * W.abs()
+        assert float(err.max()) <= 2e-3 * float(W.pow(2).mean().sqrt()), name
+
+    ways = [('BJI', 'UI'), ('BJI', 'IU'), ('IBJ', 'IU'), ('IBJ', 'UI')]
+    for la, lb in ways if E % 64 == 0 else ways[2:3]:
+        A, Bm, bias, T = mk(la), mk(lb), mk('U'), mk('BJU')
+        for alpha, t, lt in ((1.0, None, None), (0.125, None, None), (1.0, bias, 'U'), (1.0, T, 'BJU')):
+            C = nan('BJU')
+            o.einsum(A, la, Bm, lb, C, 'BJU', alpha=alpha, addend=t, l_addend=lt)
+            torch.cuda.synchronize()
+            check(C, want(la, A, lb, Bm, 'BJU', alpha, t, lt), f'{la},{lb}->BJU alpha {alpha} + {lt}')
+    if E == 2048:
+        for (la1, lb1, lc1, lt1), (la2, lb2, lc2) in (
+                (('BJU', 'UI', 'BJI', 'BJI'), ('BJU', 'BJI', 'UI')),
+                (('QHPI', 'QBJHP', 'BJI', 'BJI'), ('QBJHP', 'BJI', 'QHPI'))):
+            d = {lay: mk(lay) for lay in {la1, lb1, la2, lb2}}
+            T, C1, C2 = mk(lt1), nan(lc1), nan(lc2)
+            o.einsum_pair((d[la1], la1, d[lb1], lb1, C1, lc1, T, lt1), (d[la2], la2, d[lb2], lb2, C2, lc2))
+            torch.cuda.synchronize()
+            check(C1, want(la1, d[la1], lb1, d[lb1], lc1, 1.0, T, lt1), f'{la1},{lb1}->{lc1}')
+            check(C2, want(la2, d[la2], lb2, d[lb2], lc2), f'{la2},{lb2}->{lc2}')
