@@ -239,6 +239,7 @@ struct Handle {
                                       // bit 1: workgroups behind the first LayerNorm launch draw lin1's keep bits
     bool packed_masks = true;         // DROP1MASK and DROP3MASK travel as one bit per element inside their buffers
     bool skip_unread = true;          // intermediates that neither pass reads are not written (ATT after its bias, LIN2, DLN2, DLN1)
+    bool act_whole = false;           // the feed-forward block's outputs are whole 256 x 256 tiles, and enough of them
     bool opaque = false;              // nobody looks into DROP2MASK (bits as well), ATT and DROP2_LINW2 (left alone as well)
     // where the last forward call's lin1 epilogue left one bit per element of DROP2 (set = positive), or
     // null: the unused SB1_LINW1 buffer of that call.  The backward call reads its gate from there when it
@@ -556,6 +557,11 @@ void plan_layouts(Handle& h, bool own) {
         p.ok = p.sb[0] == 0 && gemm_relu_dropout_ok(p.shape, (const void*)16, (const void*)16, (const void*)16, ep);
     }
 
+    {
+        const GemmShape& s = h.gemm[G_LIN1_BAD].shape;
+        const long tiles = (s.M / 256) * (s.N / 256);
+        h.act_whole = s.M % 256 == 0 && s.N % 256 == 0 && s.K1 % 64 == 0 && tiles * 10 >= (tiles + 255) / 256 * 256 * 9;
+    }
     {   // scratch of the five column reductions of one backward pass, side by side
         Space si = make_space(sz, {dB, dJ}, dI), su = make_space(sz, {dB, dJ}, dU);
         Space sq = make_space(sz, {dQ, dH, dB, dJ}, dP);
@@ -572,8 +578,17 @@ void plan_layouts(Handle& h, bool own) {
         // the attention kernels' partial sums for the projection-bias gradient stand in for baib's
         const size_t attn_bias = (size_t)(3 * sz.n[dH] * sz.n[dB] * ((sz.n[dJ] + 127) / 128) * sz.n[dP]);
         if (attn_bias > (baib > baib2 ? baib : baib2)) h.ws_need_bwd += attn_bias;
-        // the partial column sums of dXlin2's epilogue (one row per 128 tokens)
-        h.ws_need_bwd += (size_t)((sz.n[dB] * sz.n[dJ] + 127) / 128) * sz.n[dU] + 64;
+        // the partial column sums of dXlin2's epilogue
+        if (h.gemm[G_DXLIN2_BDRLB].ok) {
+            const GemmPlan& p = h.gemm[G_DXLIN2_BDRLB];
+            GemmEpilogue ep; ep.gate = (const half_t*)16; ep.colsum = (float*)16; ep.sbM = p.sM; ep.sbN = p.sN;
+            int rows = 0;
+            for (int act : {ACT_RELU, ACT_GELU}) {
+                ep.act = act; ep.gate_bits = (const uint32_t*)16;
+                rows = std::max(rows, gemm_colsum_rows(p.shape, (const void*)16, (const void*)16, (const void*)16, ep));
+            }
+            h.ws_need_bwd += (size_t)rows * sz.n[dU] + 64;
+        }
     }
     h.gws_need = 0;
     for (int i = 0; i < G_COUNT; ++i) {
@@ -779,9 +794,12 @@ bool relu_from_output(const Handle& h) { return h.relu_from_output && h.act == A
 // GELU: lin1 with bias, activation and dropout in its epilogue (LIN1 and DROP2 written, the keep bits left in the
 // SB1_LINW1 buffer instead of a DROP2MASK tensor) and dXlin2 with the backward of that in its epilogue.  Both or
 // neither: without DROP2MASK the separate backward operator has nothing to read.
+bool act_epilogues(const Handle& h) {
+    // (at the sizes where the products have always done it, also where somebody looks into the intermediates)
+    return h.relu_from_output && h.fuse_epilogues && h.gemm[G_LIN1_BAD].ok && (h.opaque || h.act_whole);
+}
 bool gelu_epilogues(const Handle& h) {
-    return h.relu_from_output && h.act == ACT_GELU && h.fuse_epilogues && h.gemm[G_LIN1_BAD].ok &&
-           h.gemm[G_DXLIN2_BDRLB].ok && h.lf[LIN1].str() == "BJU";
+    return act_epilogues(h) && h.act == ACT_GELU && h.gemm[G_DXLIN2_BDRLB].ok && h.lf[LIN1].str() == "BJU";
 }
 // What the forward call adds to that from the tensors it is handed.  The backward call is handed the same ones and
 // asks the same question: it knows from the handle's options and these pointers alone whether the keep bits of
@@ -1143,7 +1161,7 @@ void forward(Handle& h, const FwdPtrs& t0) {
     auto as_sums = [&](int tensor, SplitSums& s) { return h.skip_unread && h.opaque && h.lf[tensor].str() == "BJI" ? &s : nullptr; };
     run_gemm(h, G_OUT, W[WO], F[GAMMA], F[ATT], "out", nullptr, nullptr, as_sums(ATT, out_sums));
     const bool lin1_gelu = lin1_takes_gelu_epilogue(h, W, F);
-    const bool lin1_bad = lin1_gelu || (relu_from_output(h) && h.fuse_epilogues && h.gemm[G_LIN1_BAD].ok &&
+    const bool lin1_bad = lin1_gelu || (relu_from_output(h) && act_epilogues(h) &&
                                         aligned16(W[LINB1]) && aligned16(F[DROP2]) && aligned16(F[SB1]) && aligned16(W[LINW1]));
     // The keep bits of lin1's ReLU-dropout epilogue depend on nothing but seed, step and position:
     // workgroups behind those of bdrln1, a launch that waits for memory with its vector units idle,
@@ -1282,7 +1300,8 @@ void backward(Handle& h, const BwdPtrs& t0) {
                            h.gemm[G_LIN1_BAD].shape.M == h.gemm[G_DXLIN2_BDRLB].shape.M &&
                            h.gemm[G_LIN1_BAD].shape.N == h.gemm[G_DXLIN2_BDRLB].shape.N;
     const bool bdrlb_gelu = lin1_takes_gelu_epilogue(h, W, F);       // the forward call's own test: its keep bits lie in SB1_LINW1
-    const bool fuse_bdrlb = ((relu_from_output(h) && h.fuse_epilogues && h.gemm[G_DXLIN2_BDRLB].ok && aligned16(F[DROP2])) ||
+    const bool fuse_bdrlb = ((relu_from_output(h) && h.fuse_epilogues && h.gemm[G_DXLIN2_BDRLB].ok && (h.opaque || h.act_whole) &&
+                              aligned16(F[DROP2])) ||
                              bdrlb_gelu) &&
                             aligned16(D[DLIN1]) && aligned16(D[DLIN2]) && aligned16(W[LINW2]);
     if (bdrlb_gelu && !fuse_bdrlb)
@@ -1292,12 +1311,12 @@ void backward(Handle& h, const BwdPtrs& t0) {
         // product, gate and the column sums of the result in one launch: DDROP2 is not produced
         ProfScope ps(h, "dXlin2+bdrlb");
         const GemmPlan& p = h.gemm[G_DXLIN2_BDRLB];
-        const int ntc = (int)(p.shape.M / 128), U = (int)p.shape.N;
-        float* ws = take_ws(h, (size_t)ntc * U);
         GemmEpilogue ep;
-        ep.gate = (const half_t*)(bdrlb_gelu ? F[LIN1] : F[DROP2]); ep.sbM = p.sM; ep.sbN = p.sN; ep.colsum = ws;
+        ep.gate = (const half_t*)(bdrlb_gelu ? F[LIN1] : F[DROP2]); ep.sbM = p.sM; ep.sbN = p.sN; ep.colsum = (float*)16;
         if (bits_here || bdrlb_gelu) ep.gate_bits = (const uint32_t*)F[SB1_LINW1];
         if (bdrlb_gelu) ep.act = ACT_GELU;
+        const int ntc = gemm_colsum_rows(p.shape, D[DLIN2], W[LINW2], D[DLIN1], ep), U = (int)p.shape.N;
+        float* ws = ep.colsum = take_ws(h, (size_t)ntc * U);
         launch_gemm(p.shape, (const half_t*)D[DLIN2], (const half_t*)W[LINW2], (half_t*)D[DLIN1], p.alpha, ep, h.stream);
         FinishJob job{ws, FinishArgs{{(half_t*)DW[LINB1], nullptr, nullptr, nullptr}, 0, 0, 1, 1}, 1, 1, ntc, U};
         finish_or_defer(defer_of(h), job, h.stream);
@@ -2191,6 +2210,10 @@ int sub_op_einsum_pair(void* handle, const void* A1, const char* l_A1, const voi
     });
 }
 
+// Operator calls: products of a quarter of the chip in 256 x 256 tiles and more.  (With fewer a launch is a few us, and the
+// caller's way of many calls bounds it; it keeps the mask as a tensor that can be looked at.)
+static bool worth_an_epilogue(const GemmShape& g) { return ((g.M + 255) / 256) * ((g.N + 255) / 256) >= 64; }
+
 int sub_op_einsum_bad(void* handle, const void* A, const char* l_A, const void* B, const char* l_B, const void* bias,
                       const char* l_bias, void* lin, void* out, const char* l_out, void* bits, float p, uint32_t site,
                       int* applied) {
@@ -2209,7 +2232,7 @@ int sub_op_einsum_bad(void* handle, const void* A, const char* l_A, const void* 
         // the keep bits are indexed by the offset into the output: it has to be dense in canonical order
         if (lc.str() != "BJU" || ((uintptr_t)bits & 3) || !aligned16(bias) || !aligned16(out) || !aligned16(A) ||
             !aligned16(B) || (h.act == ACT_GELU && (!lin || !aligned16(lin))) ||
-            !gemm_relu_dropout_ok(g, A, B, out, ep))
+            !worth_an_epilogue(g) || !gemm_relu_dropout_ok(g, A, B, out, ep))
             return;
         launch_gemm(g, (const half_t*)A, (const half_t*)B, (half_t*)out, 1.f, ep, h.stream);
         *applied = 1;
@@ -2230,11 +2253,10 @@ int sub_op_einsum_bdrlb(void* handle, const void* A, const char* l_A, const void
         ep.gate = (const half_t*)gate; ep.gate_bits = (const uint32_t*)bits; ep.colsum = (float*)16;
         if (h.act == ACT_GELU) ep.act = ACT_GELU;
         if (lc.str() != "BJU" || ep.sbb[0] != 0 || ((uintptr_t)bits & 3) || !aligned16(gate) || !aligned16(dlinear) ||
-            !aligned16(A) || !aligned16(B) || !gemm_relu_dropout_ok(g, A, B, dlinear, ep))
+            !aligned16(A) || !aligned16(B) || !worth_an_epilogue(g) || !gemm_relu_dropout_ok(g, A, B, dlinear, ep))
             return;
-        const int ntc = (int)(g.M / 128), U = (int)g.N;
-        float* ws = take_ws(h, (size_t)ntc * U);
-        ep.colsum = ws;
+        const int ntc = gemm_colsum_rows(g, A, B, dlinear, ep), U = (int)g.N;
+        float* ws = ep.colsum = take_ws(h, (size_t)ntc * U);
         launch_gemm(g, (const half_t*)A, (const half_t*)B, (half_t*)dlinear, 1.f, ep, h.stream);
         FinishJob job{ws, FinishArgs{{(half_t*)dbias, nullptr, nullptr, nullptr}, 0, 0, 1, 1}, 1, 1, ntc, U};
         finish_or_defer(defer_of(h), job, h.stream);

@@ -201,18 +201,6 @@ int pick_kind(const Canon& c, bool& akc, bool& bkc) {
     return ok && tiles_take(TileProduct{a, akc, bkc}) ? 1 : 0;
 }
 
-// Whole 256 x 256 tiles: what an epilogue with an activation works on.
-bool whole_256(const GemmArgs& a) { return a.M % 256 == 0 && a.N % 256 == 0 && a.K1 % BK == 0 && a.splits == 1; }
-
-// Do these tiles keep the CUs busy?  Asked for the products with an activation in their epilogue, which other tiles do not have.
-// With an operand that is read through the slower LDS transpose path the bar is higher: three quarters of a round
-// is not enough then (measured).
-bool fills_256(const GemmArgs& a, long batch, bool akc, bool bkc) {
-    const long tiles = (long)(a.M / 256) * (a.N / 256) * batch;
-    const double fill = (double)tiles / (double)((tiles + 255) / 256 * 256);
-    return whole_256(a) && fill >= (akc && bkc ? 0.7 : 0.9);
-}
-
 void launch_splitk_reduce(const GemmArgs& a, hipStream_t st) {
     const long n = a.nbatch * (long)a.M * (a.N / 4);
     hipLaunchKernelGGL(k_gemm_splitk_reduce, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a, a.nbatch);
@@ -245,12 +233,29 @@ int gemm_kernel_kind(const GemmShape& s, const void* A, const void* B, const voi
     return pick_kind(c, akc, bkc);
 }
 
+// The tiles that a product with an activation in its epilogue runs in, -1 if it does not.
+static int act_form(const GemmShape& s, const void* A, const void* B, const void* C, const GemmEpilogue& ep) {
+    if (s.batch() != 1 || s.sCN != 1 || s.sCM != s.N || s.N % 32 != 0) return -1;       // one dense row-major output
+    TileProduct p;
+    Canon c = canonicalise(s, (const half_t*)A, (const half_t*)B, (half_t*)C, 1.f, ep);
+    if (pick_kind(c, p.akc, p.bkc) != 1) return -1;
+    p.a = c.a; p.a.nbatch = 1;
+    // A small output whose contraction a forward pass splits keeps the order of its sums, with or without an activation behind
+    // it: split, and the operators.
+    if ((size_t)s.M * s.N <= kSplitMaxOut && pick_splits(c.a, 1, SIZE_MAX) > 1) return -1;
+    return choose_act_form(p);
+}
+
 bool gemm_relu_dropout_ok(const GemmShape& s, const void* A, const void* B, const void* C,
                           const GemmEpilogue& ep) {
-    if (s.batch() != 1 || s.sCN != 1 || s.sCM != s.N) return false;       // one dense row-major output
-    Canon c = canonicalise(s, (const half_t*)A, (const half_t*)B, (half_t*)C, 1.f, ep);
-    bool akc, bkc;
-    return pick_kind(c, akc, bkc) == 1 && fills_256(c.a, 1, akc, bkc);
+    return act_form(s, A, B, C, ep) >= 0;
+}
+
+int gemm_colsum_rows(const GemmShape& s, const void* A, const void* B, const void* C, const GemmEpilogue& ep) {
+    const int form = act_form(s, A, B, C, ep);
+    if (form < 0) fail("gemm: no activation in this product's epilogue (see gemm_relu_dropout_ok)");
+    const long bm = tile_form(form).bm;
+    return (int)(2 * ((s.M + bm - 1) / bm));             // two rows of waves
 }
 
 size_t gemm_splitk_ws_floats(const GemmShape& s) {
@@ -374,17 +379,19 @@ void launch_gemm(const GemmShape& s, const half_t* A, const half_t* B, half_t* C
     if (kind == 1) {
         TileProduct tp{c.a, akc, bkc};
         tp.a.nbatch = batch;
-        const bool in_epilogue = ep.relu_dropout || ep.gate;
-        if (in_epilogue && (!fills_256(c.a, batch, akc, bkc) || batch != 1 || s.sCN != 1 || s.sCM != s.N))
-            fail("gemm: the ReLU-dropout epilogue needs the 256x256 kernel (see gemm_relu_dropout_ok)");
+        if (ep.relu_dropout || ep.gate) {
+            const int form = act_form(s, A, B, C, ep);
+            if (form < 0 || alpha != 1.0f) fail("gemm: no activation in this product's epilogue (see gemm_relu_dropout_ok)");
+            launch_tiles_act(tp, form, st);
+            check_launch("gemm");
+            return;
+        }
         // A forward pass sums in an order that depends on the product's shape alone (pick_splits), whatever the tile.
-        const bool small = ws && (size_t)batch * c.a.M * c.a.N <= kSplitMaxOut && !in_epilogue;
+        const bool small = ws && (size_t)batch * c.a.M * c.a.N <= kSplitMaxOut;
         if (small && !ep.any_split) tp.a.splits = pick_splits(c.a, batch, ws_floats);
-        TileChoice choice;
-        choice.form = TILE_256x256;
-        if (!in_epilogue) choice = choose_single(tp, small && ep.any_split ? ws_floats : 0);
+        const TileChoice choice = choose_single(tp, small && ep.any_split ? ws_floats : 0);
         if (side) side->tiles_done = 0;
-        if (side && side->keep && side->key.thr && choice.form == TILE_256x256 && choice.splits == 1 && !in_epilogue) {
+        if (side && side->keep && side->key.thr && choice.form == TILE_256x256 && choice.splits == 1) {
             // CUs the tiles leave idle draw attention keep bits meanwhile: what fits into the time the
             // product takes (about 9 us + 1.5 us per k-tile; the rate per CU and us is the measured break-even:
             // 12 of the 16 key tiles of the bench workload cost the launch 0.3 us, 14 cost it 2.5, all 16 6 us)
@@ -403,7 +410,7 @@ void launch_gemm(const GemmShape& s, const half_t* A, const half_t* B, half_t* C
             }
         }
         tp.a = c.a; tp.a.nbatch = batch;
-        if (c.a.side_blocks || in_epilogue) {
+        if (c.a.side_blocks) {
             launch_wide(&tp, 1, nullptr, c.a.side_blocks, st);
         } else {
             tp.a.splits = choice.splits;

@@ -24,11 +24,7 @@ bool wide_takes(const TileProduct& p) {
 }
 
 void launch_wide(const TileProduct* p, int n, FinishJobs* tail, unsigned side_blocks, hipStream_t st) {
-    const GemmArgs& a = p->a;
-    if (n == 1 && a.gate) a.act == ACT_GELU ? launch_wide_act<EPI_GELU_GATE_COLSUM>(*p, st) : launch_wide_act<EPI_GATE_COLSUM>(*p, st);
-    else if (n == 1 && a.relu_dropout && a.act == ACT_GELU) launch_wide_act<EPI_GELU_DROPOUT>(*p, st);
-    else if (n == 1 && a.relu_dropout) a.keep_words ? launch_wide_act<EPI_RELU_DROPOUT_PRE>(*p, st) : launch_wide_act<EPI_RELU_DROPOUT>(*p, st);
-    else if (n == 1 && !(tail && tail->n)) launch_plain<1>(p, n, tail, side_blocks, st);
+    if (n == 1 && !(tail && tail->n)) launch_plain<1>(p, n, tail, side_blocks, st);
     else if (side_blocks) fail("gemm: a side job has its product to itself");
     else launch_plain<kMaxProducts>(p, n, tail, 0, st);
 }

@@ -206,10 +206,9 @@ __global__ __launch_bounds__(BLOCK) void k_bdrln(RowSpace rs, View in, View resi
     const unsigned row_blocks = gridDim.x - side.blocks;
     if (blockIdx.x >= row_blocks) {
         const PhiloxKey skey = resolved(side.key);
-        const uint32_t tiles_n = side.N / 256, items = (side.M / 256) * tiles_n * 512;
+        const uint32_t items = (uint32_t)((uint64_t)side.M * side.N / 128);
         for (uint32_t id = (blockIdx.x - row_blocks) * BLOCK + threadIdx.x; id < items; id += side.blocks * BLOCK) {
-            const uint32_t tile = id >> 9, tm = tile / tiles_n;
-            const KeepWords k = relu_dropout_keep_words(skey, side.N, tm, tile - tm * tiles_n, (id >> 7) & 3, (id >> 6) & 1, id & 63);
+            const KeepWords k = keep_words128(skey, id);
             reinterpret_cast<uint4*>(side.out)[id] = make_uint4(k.w[0], k.w[1], k.w[2], k.w[3]);
         }
         return;
@@ -361,10 +360,9 @@ __global__ __launch_bounds__(BLOCK) void k_bdrln_flat(int R, unsigned nrows, Vie
     const unsigned row_blocks = gridDim.x - side.blocks;
     if (blockIdx.x >= row_blocks) {
         const PhiloxKey skey = resolved(side.key);
-        const uint32_t tiles_n = side.N / 256, items = (side.M / 256) * tiles_n * 512;
+        const uint32_t items = (uint32_t)((uint64_t)side.M * side.N / 128);
         for (uint32_t id = (blockIdx.x - row_blocks) * BLOCK + threadIdx.x; id < items; id += side.blocks * BLOCK) {
-            const uint32_t tile = id >> 9, tm = tile / tiles_n;
-            const KeepWords k = relu_dropout_keep_words(skey, side.N, tm, tile - tm * tiles_n, (id >> 7) & 3, (id >> 6) & 1, id & 63);
+            const KeepWords k = keep_words128(skey, id);
             reinterpret_cast<uint4*>(side.out)[id] = make_uint4(k.w[0], k.w[1], k.w[2], k.w[3]);
         }
         return;
@@ -760,10 +758,10 @@ void launch_bdrln(const RowSpace& rs, View in, View resid, View lin_bias, View s
                 diff.vec && normed.vec && out.vec;
     // the side job: as many workgroups as draw one lane's words per thread, at most four per CU
     KeepWordsJob job;
-    if (side && side->out && side->key.thr && side->M % 256 == 0 && side->N % 256 == 0 && side->M > 0 && side->N > 0 &&
-        (uint64_t)side->M * side->N / 8 / 16 <= 0x7fffffffu) {
+    if (side && side->out && side->key.thr && side->M > 0 && side->N > 0 && (uint64_t)side->M * side->N % 128 == 0 &&
+        (uint64_t)side->M * side->N / 128 <= 0x7fffffffu) {
         job = *side;
-        const uint64_t items = (uint64_t)side->M / 256 * (side->N / 256) * 512;
+        const uint64_t items = (uint64_t)side->M * side->N / 128;
         job.blocks = (uint32_t)((items + BLOCK - 1) / BLOCK < 1024 ? (items + BLOCK - 1) / BLOCK : 1024);
         side->blocks = job.blocks;
     } else if (side) {

@@ -288,26 +288,15 @@ __device__ __forceinline__ uint32_t attention_keep_word(const PhiloxKey& key, ui
            (keep8(philox_group_dev(key, g0 + 2), key.thr) << 16) | (keep8(philox_group_dev(key, g0 + 3), key.thr) << 24);
 }
 
-// The ReLU-dropout epilogue of the 256x256 contraction kernel walks its tile so that lane `lane` of wave `wave` (of 4: 2 x 2)
-// stores 32 packs of 8 outputs, pack c at
-//   row = 256 tile_m + 128 (c / 16) + 64 (wave / 2) + 16 (c / 2 % 4) + 8 (c % 2) + lane / 8,
-//   column = 256 tile_n + 128 (c / 8 % 2) + 64 (wave % 2) + 8 (lane % 8)
-// of the dense [M][N] output.  Its keep bits are 256 bits per lane, pack c in byte c.  This draws the four words of packs
-// 16 h .. 16 h + 15 for one lane.
+// Keep bits of 128 consecutive canonical elements, number 128 id on: bit e of the row of words is element e's.
 struct KeepWords { uint32_t w[4]; };
-__device__ __forceinline__ KeepWords relu_dropout_keep_words(const PhiloxKey& key, uint32_t N, uint32_t tile_m,
-                                                             uint32_t tile_n, uint32_t wave, uint32_t h, uint32_t lane) {
-    const uint64_t row0 = (uint64_t)tile_m * 256 + h * 128 + (wave >> 1) * 64 + (lane >> 3);
-    const uint64_t g0 = (row0 * N + (uint64_t)tile_n * 256 + (wave & 1) * 64 + (lane & 7) * 8) >> 3;
+__device__ __forceinline__ KeepWords keep_words128(const PhiloxKey& key, uint64_t id) {
     KeepWords k;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         uint32_t w = 0;
 #pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            const int c = 4 * j + b, row = ((c >> 1) & 3) * 16 + (c & 1) * 8;
-            w |= keep8(philox_group_dev(key, g0 + (uint64_t)row * (N >> 3) + (uint64_t)((c >> 3) * 16)), key.thr) << (8 * b);
-        }
+        for (int b = 0; b < 4; ++b) w |= keep8(philox_group_dev(key, id * 16 + (uint64_t)(4 * j + b)), key.thr) << (8 * b);
         k.w[j] = w;
     }
     return k;
@@ -420,10 +409,12 @@ __device__ __forceinline__ GeluTerms gelu_terms(float x, float x2) {
 
 // (The results pass through a register as fp32: a conversion to fp16 that follows rounds that value,
 // whereas fused with the last multiplication into one instruction it would round the exact product.)
+// (s as 1 / (1 + e^-2u): one that needs no bound, e^-2u may become infinite.)
 __device__ __forceinline__ float gelu_fwd(float x) {
 #pragma clang fp contract(off)
-    float g = x * gelu_terms(x, x * x).s;
-    asm volatile("" : "+v"(g));
+    const float w = x * __builtin_fmaf(x * x, -0.1029432395800235f, -2.302208198144325f);      // -2u log2(e)
+    float g = x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(w));
+    asm("" : "+v"(g));
     return g;
 }
 
@@ -435,7 +426,7 @@ __device__ __forceinline__ float gelu_bwd(float x, float d) {
     const float zp = __builtin_fmaf(x2, 0.21406444881780073f, 1.5957691216057308f);   // d(2u)/dx
     const float q = (x * zp) * t.r;
     float g = __builtin_fmaf(t.s, q, t.s) * d;
-    asm volatile("" : "+v"(g));
+    asm("" : "+v"(g));
     return g;
 }
 

@@ -145,7 +145,13 @@ bool tiles_take(const TileProduct& p);                        // within the rang
 // The best of `forms` (a bit each).  ws_floats > 0: the longest contraction may be split over that much scratch.
 TileChoice choose_tiles(const TileProduct* p, int n, unsigned forms, size_t ws_floats);
 // `tail`: column sums of earlier launches, finished by workgroups behind the tiles (tail->n = 0 then).
-// k_gemm_wide.hip: 256 x 256 tiles, the ones that carry an activation in their epilogue among them (of a single product).
+// Outputs of a tile of form f, and workgroups of that form on a CU.
+struct TileForm { int bm, bn, per_cu; };
+TileForm tile_form(int form);
+// The best form for a product with an activation in its epilogue (-1: none), and its launch.
+int choose_act_form(const TileProduct& p);
+void launch_tiles_act(const TileProduct& p, int form, hipStream_t st);
+// k_gemm_wide.hip: 256 x 256 tiles.
 bool wide_takes(const TileProduct& p);
 // side_blocks: workgroups behind the tiles, for GemmArgs::side_*
 void launch_wide(const TileProduct* p, int n, FinishJobs* tail, unsigned side_blocks, hipStream_t st);

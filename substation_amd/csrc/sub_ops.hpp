@@ -25,9 +25,8 @@ void launch_softmax(const RowSpace& rs, View beta, View alpha, View mask, View d
 void launch_bs(const RowSpace& rs, View alpha, View mask, View ddrop, View dbeta, float scale,
                hipStream_t st);
 // Side job of launch_bdrln (a launch that waits for memory with its vector units idle): `blocks`
-// workgroups behind those of the rows draw the keep words of the ReLU-dropout epilogue
-// (relu_dropout_keep_words) of a later product with a dense [M][N] output in 256x256 tiles, word
-// quadruple (((tile_m * N/256 + tile_n) * 4 + wave) * 2 + half) * 64 + lane of `out` (M * N / 8 bytes).
+// workgroups behind those of the rows draw the keep bits of the ReLU-dropout epilogue of a later product
+// with a dense [M][N] output, one bit per output in canonical order, to `out` (M * N / 8 bytes, M * N a multiple of 128).
 // A product of dense rows left as the fp32 sums of its k splits: fp16(alpha * their sum) is its output, wherever that is read.
 struct SplitSums {
     const float* p = nullptr;    // [splits][rows][row]; null: the output itself was written
@@ -234,12 +233,12 @@ struct GemmEpilogue {
     bool relu_dropout = false;
     PhiloxKey key;
     // or: out = gate > 0 ? x : 0 with `gate` laid out like an addend (strides sbM, sbN, sbb), and the
-    // column sums of out over the rows of every 128-row slab as fp32 rows of `colsum` ([M / 128][N]);
+    // column sums of out as fp32 partial sums, `colsum` ([gemm_colsum_rows][N]);
     // same conditions as relu_dropout (gemm_relu_dropout_ok)
     const half_t* gate = nullptr;
     float* colsum = nullptr;
-    // relu_dropout: also writes one bit per output (set = positive), M * N / 8 bytes in the kernel's
-    // own order; gate: reads those bits, written by a product of the same output shape, instead of
+    // relu_dropout: also writes one bit per output (set = positive), M * N / 8 bytes in canonical order (bit
+    // m N + n); gate: reads those bits, written by a product of the same output shape, instead of
     // the values of `gate` (which must still be given)
     uint32_t* gate_bits_out = nullptr;
     const uint32_t* gate_bits = nullptr;
@@ -274,9 +273,11 @@ struct GemmSideJob {
 void launch_gemm(const GemmShape& g, const half_t* A, const half_t* B, half_t* C, float alpha,
                  const GemmEpilogue& ep, hipStream_t st, float* ws = nullptr, size_t ws_floats = 0,
                  GemmSideJob* side = nullptr);
-// Can launch_gemm apply ep.relu_dropout to this product?  Only the kernel with
-// 256x256 tiles does, on a single dense row-major output.
+// Can launch_gemm apply ep.relu_dropout or ep.gate to this product?  A single dense row-major output, rows of whole
+// 32-bit words of keep bits.
 bool gemm_relu_dropout_ok(const GemmShape& g, const void* A, const void* B, const void* C, const GemmEpilogue& ep);
+// Rows of partial column sums that launch_gemm leaves with ep.gate (for a product that is ok).
+int gemm_colsum_rows(const GemmShape& g, const void* A, const void* B, const void* C, const GemmEpilogue& ep);
 // A third product offered to launch_gemm_pair: taken (and `taken` set) when its tiles in that launch are
 // expected to cost less than a launch of its own.
 struct PairThird {

@@ -14,6 +14,15 @@ namespace {
 
 typedef uint32_t u4v __attribute__((ext_vector_type(4)));
 
+// f(0), f(1) .. f(N - 1), the index a constant of the type.
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void each(const F& f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        each<N, I + 1>(f);
+    }
+}
+
 __device__ __forceinline__ unsigned lds_addr(const void* p) {
     return (unsigned)(uintptr_t)(__attribute__((address_space(3))) const void*)p;
 }
@@ -39,6 +48,95 @@ __device__ __forceinline__ void load_to_lds(unsigned lds, unsigned voff, u4v r) 
     const u4v ru = {u(r[0]), u(r[1]), u(r[2]), u(r[3])};
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
                  ::"s"(u(lds)), "v"(voff), "s"(ru));
+}
+
+// What the epilogue does after the scaling and the optional addend.
+// EPI_RELU_DROPOUT_PRE: EPI_RELU_DROPOUT with the keep bits drawn ahead of the launch (GemmEpilogue::keep_words)
+// EPI_GELU_DROPOUT: as EPI_RELU_DROPOUT with GELU; also stores the rounded sum before the activation
+// (GemmArgs::pre_out, which the backward pass needs) and leaves the keep bits where the ReLU form leaves its gate bits.
+// EPI_GELU_GATE_COLSUM: the backward counterpart: out = keep bit ? gelu'(pre-activation) * product : 0, and column sums.
+enum { EPI_PLAIN = 0, EPI_RELU_DROPOUT = 1, EPI_GATE_COLSUM = 2, EPI_RELU_DROPOUT_PRE = 3, EPI_GELU_DROPOUT = 4,
+       EPI_GELU_GATE_COLSUM = 5 };
+
+template <typename Key>
+__device__ __forceinline__ PhiloxKey key_of(Key& from) {
+    PhiloxKey k;
+    k.k0 = from.k0; k.k1 = from.k1; k.site = from.site; k.step = from.step; k.thr = from.thr; k.step_dev = from.step_dev;
+    return resolved(k);
+}
+
+// Eight halves (non-negative, or zero) where the bits of w's low byte are set, else zero; and the bits of those that are not zero.
+__device__ __forceinline__ h8 keep8_of(h8 v, uint32_t w) {
+    // bits 2 p and 2 p + 1 side by side, 16 apart, for every pair p; 0 - bit is a half's mask
+    const uint32_t x = (w & 0xffu) | (w << 15);
+    u4v r = __builtin_bit_cast(u4v, v);
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+        const uint32_t b = (x >> (2 * p)) & 0x10001u;
+        uint32_t m;
+        asm("v_pk_sub_u16 %0, 0, %1" : "=v"(m) : "v"(b));
+        r[p] &= m;
+    }
+    return __builtin_bit_cast(h8, r);
+}
+__device__ __forceinline__ uint32_t nonzero8(h8 v) {
+    const u4v r = __builtin_bit_cast(u4v, v);
+    uint32_t d = 0;
+#pragma unroll
+    for (int p = 3; p >= 0; --p) {
+        uint32_t b;
+        asm("v_pk_min_u16 %0, %1, %2" : "=v"(b) : "v"(r[p]), "v"(0x10001u));
+        d = (d << 2) | b;
+    }
+    return (d | (d >> 15)) & 0xffu;
+}
+
+// One bit per output travels in canonical order (bit m N + n), N a multiple of 32.  Four lanes next to one another hold the 32
+// columns of a word, each the byte of its 8 (a pack); of four packs, lane j of the four writes and reads the word of pack j.
+__device__ __forceinline__ uint32_t quad_word(uint32_t byte, int lane) {
+    uint32_t x = (byte & 0xffu) << (8 * (lane & 3));
+    x |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xF, 0xF, true);      // the lane next to this one
+    x |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x4E, 0xF, 0xF, true);      // the other two
+    return x;
+}
+// Byte of pack j (its word is in lane j of the four).
+template <int j>
+__device__ __forceinline__ uint32_t quad_byte(uint32_t word, int lane) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)word, j * 0x55, 0xF, 0xF, true) >> (8 * (lane & 3));
+}
+
+// A pack of rounded sums through the activation; `keep`: its keep bits, on return the bits to leave for the backward pass.
+// GELU: the keep bits themselves; ReLU: set where the result is positive.
+template <int EPI>
+__device__ __forceinline__ h8 act_forward(h8 v, uint32_t& keep) {
+    if constexpr (EPI == EPI_GELU_DROPOUT) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = (half_t)gelu_fwd((float)v[e]);       // for every element, then selected: no branches
+        return keep8_of(v, keep);
+    } else {
+        // what the bias-activation-dropout operator does to the rounded sum
+        v = keep8_of(__builtin_elementwise_max(v, (h8)(half_t)0.0f), keep);     // ReLU, packed
+        keep = nonzero8(v);
+        return v;
+    }
+}
+// A pack of the incoming gradient through the activation's backward pass, added to the column sums.  saved: GELU's
+// pre-activation values; ReLU without bits: its output.
+template <int EPI, bool BITS>
+__device__ __forceinline__ h8 act_backward(h8 v, h8 saved, uint32_t bits, float (&colsum)[8]) {
+    if constexpr (EPI == EPI_GELU_GATE_COLSUM) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = (half_t)gelu_bwd((float)saved[e], (float)v[e]);
+    }
+    if constexpr (BITS) {
+        v = keep8_of(v, bits);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = (float)saved[e] > 0.f ? v[e] : (half_t)0.0f;
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) colsum[e] += (float)v[e];
+    return v;
 }
 
 // Logical index of workgroup b of n such that the ones that the eight XCDs get in turn are consecutive on one XCD.
@@ -165,5 +263,9 @@ void list_tiles(TileGroup<NP>& G, const TileProduct* p, int n, int bm, int bn, l
 }
 
 }  // namespace
+
+// One product with activation EPI in its epilogue, in tiles of form `form` (k_gemm_act.hip, compiled once for each EPI).
+template <int EPI>
+void launch_act(const TileProduct& p, int form, hipStream_t st);
 
 }  // namespace sub

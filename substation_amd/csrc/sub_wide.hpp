@@ -35,23 +35,6 @@ namespace {
 
 typedef float f4v __attribute__((ext_vector_type(4)));
 
-// f(0), f(1) .. f(N - 1), the index a constant of the type.
-template <int N, int I = 0, typename F>
-__device__ __forceinline__ void each(const F& f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        each<N, I + 1>(f);
-    }
-}
-
-// What the epilogue does after the scaling and the optional addend.
-// EPI_RELU_DROPOUT_PRE: EPI_RELU_DROPOUT with the keep bits drawn ahead of the launch (GemmEpilogue::keep_words)
-// EPI_GELU_DROPOUT: as EPI_RELU_DROPOUT with GELU; also stores the rounded sum before the activation
-// (GemmArgs::pre_out, which the backward pass needs) and leaves the keep bits where the ReLU form leaves its gate bits.
-// EPI_GELU_GATE_COLSUM: the backward counterpart: out = keep bit ? gelu'(pre-activation) * product : 0, and column sums.
-enum { EPI_PLAIN = 0, EPI_RELU_DROPOUT = 1, EPI_GATE_COLSUM = 2, EPI_RELU_DROPOUT_PRE = 3, EPI_GELU_DROPOUT = 4,
-       EPI_GELU_GATE_COLSUM = 5 };
-
 // acc += b^T a, 16 x 16 outputs, 32 k.  Spelled out so that the accumulators stay in the accumulation registers (left to
 // itself the compiler moves a quarter of them back and forth every step).  What it then does not know of: the wait between
 // the last of these and the first read of an accumulator (Wide::settle).
@@ -59,41 +42,14 @@ __device__ __forceinline__ void mul(f4v& acc, h8 b, h8 a) {
     asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(acc) : "v"(b), "v"(a));
 }
 
+// One of them, read where it is used: left to itself the compiler reads all 256 ahead, and spills them.
+__device__ __forceinline__ float accumulator(float a) {
+    float x;
+    asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(x) : "a"(a));
+    return x;
+}
 __device__ __forceinline__ void mul_first(f4v& acc, h8 b, h8 a) {
     asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, 0" : "=a"(acc) : "v"(b), "v"(a));
-}
-
-template <typename Key>
-__device__ __forceinline__ PhiloxKey key_of(Key& from) {
-    PhiloxKey k;
-    k.k0 = from.k0; k.k1 = from.k1; k.site = from.site; k.step = from.step; k.thr = from.thr; k.step_dev = from.step_dev;
-    return resolved(k);
-}
-
-// Eight halves (non-negative, or zero) where the bits of w's low byte are set, else zero; and the bits of those that are not zero.
-__device__ __forceinline__ h8 keep8_of(h8 v, uint32_t w) {
-    // bits 2 p and 2 p + 1 side by side, 16 apart, for every pair p; 0 - bit is a half's mask
-    const uint32_t x = (w & 0xffu) | (w << 15);
-    u4v r = __builtin_bit_cast(u4v, v);
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-        const uint32_t b = (x >> (2 * p)) & 0x10001u;
-        uint32_t m;
-        asm("v_pk_sub_u16 %0, 0, %1" : "=v"(m) : "v"(b));
-        r[p] &= m;
-    }
-    return __builtin_bit_cast(h8, r);
-}
-__device__ __forceinline__ uint32_t nonzero8(h8 v) {
-    const u4v r = __builtin_bit_cast(u4v, v);
-    uint32_t d = 0;
-#pragma unroll
-    for (int p = 3; p >= 0; --p) {
-        uint32_t b;
-        asm("v_pk_min_u16 %0, %1, %2" : "=v"(b) : "v"(r[p]), "v"(0x10001u));
-        d = (d << 2) | b;
-    }
-    return (d | (d >> 15)) & 0xffu;
 }
 
 // A workgroup that multiplies nothing (see GemmSideJob): workgroup sb of nsb.
@@ -170,7 +126,8 @@ struct Wide : TileList<4 * QM, 4 * QN, NP> {
     static constexpr int PACKS = 4 * TA * NI;                          // packs of 8 outputs that a lane stores
     static constexpr bool DRAWS = EPI == EPI_RELU_DROPOUT || EPI == EPI_GELU_DROPOUT;
     static constexpr bool GATED = EPI == EPI_GATE_COLSUM || EPI == EPI_GELU_GATE_COLSUM;
-    static_assert(EPI == EPI_PLAIN || PACKS == 32, "32 packs of keep bits per lane");
+    static constexpr bool READS = GATED || EPI == EPI_RELU_DROPOUT_PRE;          // bits of the outputs, as another launch left them
+    static_assert(EPI == EPI_PLAIN || (PACKS == 32 && LPR == 8 && TA == 4), "32 packs of keep bits per lane, in the order of Epilogue::bits_part");
 
     // ---- what is fetched: the tiles' steps one after the other -----------------------------------------------------
     // (All of it in scalar registers but the offsets, and next to nothing to be computed from step to step: with one wave
@@ -400,7 +357,8 @@ struct Wide : TileList<4 * QM, 4 * QN, NP> {
             step(std::true_type{}, std::false_type{});
             int kt = 1;
             if constexpr (DRAWS) {
-                for (; kt < t.nkt - PACKS / 2; ++kt) step(std::false_type{}, std::false_type{});
+                const int from = e.draw.c ? t.nkt : t.nkt - PACKS / 2;
+                for (; kt < from; ++kt) step(std::false_type{}, std::false_type{});
                 for (; kt < t.nkt; ++kt) step(std::false_type{}, std::true_type{});
                 while (e.draw.c < PACKS) e.draw.one();        // a contraction shorter than that
             } else {
@@ -422,29 +380,48 @@ struct Wide : TileList<4 * QM, 4 * QN, NP> {
     struct Epilogue {
         Draw draw;
         h8 bias8[2];                  // a bias row's 8 columns of this lane, in both halves of B
-        uint32_t bits[GATED || EPI == EPI_RELU_DROPOUT_PRE ? 8 : 1];
-        long bits_at = 0;
+        uint32_t bits[READS ? 8 : 1];          // words of 4 packs each (quad_word)
+
+        // The bits of a tile's outputs from the wave's first row and column on, and the lane's place in them: of 4 packs,
+        // pack lane % 4 (two slabs of 16 rows, 8 rows at a time), the word of its columns.
+        static __device__ __forceinline__ __amdgpu_buffer_rsrc_t bits_of(Args& g, const Tile& t, const uint32_t* p, int wm, int wn, int lane,
+                                                                         unsigned (&at)[2]) {
+            const int m_wave = t.m0 + wm * QM, n_wave = t.n0 + wn * QN, rows = g.M - m_wave, cols = g.N - n_wave, q = lane & 3;
+            const uint64_t first = reinterpret_cast<uint64_t>(uniform(p)) + (uint64_t)(((long)m_wave * g.N + n_wave) >> 3);
+            const long bytes = p && rows > 0 && cols > 0 ? ((long)(rows - 1) * g.N + cols) >> 3 : 0;
+            auto u = [](uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); };
+#pragma unroll
+            for (int hb = 0; hb < 2; ++hb)
+                at[hb] = (unsigned)(((q >> 1) * 16 + (q & 1) * RPI + lane / LPR) * (g.N >> 3) + (lane % LPR >> 2) * 4) |
+                         ((lane % LPR >> 2) * 32 + hb * HN < cols ? 0u : 1u << 31);
+            return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(first), 0, (int)u((uint32_t)(bytes < 0x7fffffffL ? bytes : 0x7fffffffL)), 0x00020000);
+        }
+        // word k: packs 4 k .. 4 k + 3
+        static __device__ __forceinline__ unsigned bits_part(Args& g, int k) {
+            return (unsigned)((k >> 2) * HM + (k & 1) * 32) * (unsigned)(g.N >> 3) + (unsigned)((k >> 1 & 1) * (HN >> 3));
+        }
 
         // What it reads besides the accumulators, asked for ahead of the contraction.
         __device__ __forceinline__ void open(Args& g, const Tile& t, int wm, int wn, int wave, int lane) {
             if constexpr (EPI != EPI_PLAIN) {
-                const long tiles_n = (g.N + BN - 1) / BN;
-                // two quadruples of words per lane
-                bits_at = (((long)(t.m0 / BM) * tiles_n + t.n0 / BN) * NW + wave) * 128 + lane;
-                const uint4* from = reinterpret_cast<const uint4*>(GATED ? g.gate_bits : g.keep_words);
-                if ((GATED && g.gate_bits) || EPI == EPI_RELU_DROPOUT_PRE) {
+                if (READS && (EPI != EPI_GATE_COLSUM || g.gate_bits)) {
+                    unsigned at[2];
+                    const __amdgpu_buffer_rsrc_t r = bits_of(g, t, GATED ? g.gate_bits : g.keep_words, wm, wn, lane, at);
 #pragma unroll
-                    for (int i = 0; i < 2; ++i) {
-                        const uint4 w = from[bits_at + i * 64];
-                        bits[i * 4] = w.x; bits[i * 4 + 1] = w.y; bits[i * 4 + 2] = w.z; bits[i * 4 + 3] = w.w;
-                    }
+                    for (int k = 0; k < 8; ++k)
+                        bits[k] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, (int)at[k >> 1 & 1], (int)bits_part(g, k), 0);
                 }
                 if constexpr (DRAWS) {
                     draw.key = key_of(g.key);
                     const uint64_t row = (uint64_t)(t.m0 + wm * QM + lane / LPR);
                     draw.group0 = (row * (uint64_t)g.sCM + (uint64_t)(t.n0 + wn * QN + (lane % LPR) * 8)) >> 3;
                     draw.stride = g.sCM >> 3;
-                    draw.c = 0;
+                    if (!draw.key.thr) {
+                        // nothing is dropped
+                        draw.c = PACKS;
+#pragma unroll
+                        for (int k = 0; k < 8; ++k) draw.kb[k] = ~0u;
+                    }
                 }
             }
         }
@@ -486,7 +463,10 @@ struct Wide : TileList<4 * QM, 4 * QN, NP> {
             for (int hb = 0; hb < 2; ++hb)
 #pragma unroll
                 for (int e = 0; e < 8; ++e) colsum[hb][e] = 0.f;
-            uint32_t out_bits[8];
+            uint32_t out_word = 0;
+            unsigned at_o[2] = {0, 0};
+            __amdgpu_buffer_rsrc_t ro = rc;
+            if constexpr (EPI != EPI_PLAIN && !GATED) ro = bits_of(g, t, g.gate_bits_out, wm, wn, lane, at_o);     // (null: none)
             auto tile = [&](auto kind) __attribute__((always_inline)) {
                 constexpr int ADD = decltype(kind)::value;          // 0 no addend, 1 a row, 2 a tensor, 3 the gate's values
                 __amdgpu_buffer_rsrc_t rb = rc, rl = rc;
@@ -508,13 +488,12 @@ struct Wide : TileList<4 * QM, 4 * QN, NP> {
                 // the row's index, so that neither the writes (16 rows of 8 bytes) nor the reads (8 rows of 128) meet in a bank.
                 auto fill = [&](auto sl_) __attribute__((always_inline)) {
                     constexpr int sl = decltype(sl_)::value, h = sl / (2 * TA), hb = sl / TA % 2, i = sl % TA;
-                    f4v x[TB];
+                    float x[TB][4];
 #pragma unroll
-                    for (int j = 0; j < TB; ++j) {
-                        x[j] = acc[h][hb][i][j];
-                        asm volatile("" : "+v"(x[j]));        // (read here: the compiler would read all of them ahead, and spill them)
-                    }
-                    if (alpha != 1.0f) {
+                    for (int j = 0; j < TB; ++j)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) x[j][e] = accumulator(acc[h][hb][i][j][e]);
+                    if (EPI == EPI_PLAIN && alpha != 1.0f) {
 #pragma unroll
                         for (int j = 0; j < TB; ++j)
 #pragma unroll
@@ -541,59 +520,34 @@ struct Wide : TileList<4 * QM, 4 * QN, NP> {
                     for (int it = 0; it < NI; ++it) vals[it] = *reinterpret_cast<const h8*>(slab + (sl % SLABS) * SLAB + it * RPI * QN + (from ^ (it * RPI / 2 * 8)));
                     if constexpr (sl + 2 < 4 * TA) fill(std::integral_constant<int, sl + 2>{});
                     {
-#pragma unroll
-                        for (int it = 0; it < NI; ++it) {
-                            const int c = sl * NI + it;
+                        each<NI>([&](auto it_) __attribute__((always_inline)) {
+                            constexpr int it = decltype(it_)::value, c = sl * NI + it;
                             const unsigned at = at_c[hb], uni = wave_part(g.sCM, h, hb, i, it);
                             h8 val = vals[it];
                             // (packed half add: the same single rounding as through fp32)
                             if (ADD == 1) val = val + one[hb];
                             if (ADD == 2) val = val + ad[sl % 4][it];
-                            if constexpr (EPI == EPI_GATE_COLSUM) {
-                                // the ReLU layer's backward-dropout-activation: zero where the forward output was not positive
-                                if constexpr (ADD == 3) {
-#pragma unroll
-                                    for (int e = 0; e < 8; ++e) val[e] = (float)ad[sl % 4][it][e] > 0.f ? val[e] : (half_t)0.0f;
-                                } else {
-                                    val = keep8_of(val, bits[c >> 2] >> (8 * (c & 3)));
-                                }
-#pragma unroll
-                                for (int e = 0; e < 8; ++e) colsum[hb][e] += (float)val[e];
+                            if constexpr (GATED) {
+                                uint32_t w = 0;
+                                if constexpr (ADD == 0 || EPI == EPI_GELU_GATE_COLSUM) w = quad_byte<c & 3>(bits[c >> 2], lane);
+                                // (rows beyond the last: nothing in the column sums; without bits, what is read there is zero)
+                                w = h * HM + i * 16 + it * RPI + row < rows ? w : 0u;
+                                val = act_backward<EPI, ADD == 0 || EPI == EPI_GELU_GATE_COLSUM>(val, ad[sl % 4][it], w, colsum[hb]);
                             }
-                            if constexpr (EPI == EPI_GELU_GATE_COLSUM) {
-                                // the GELU layer's backward-dropout-activation, as the operator computes it
-                                const uint32_t w = bits[c >> 2] >> (8 * (c & 3));
-#pragma unroll
-                                for (int e = 0; e < 8; ++e) {
-                                    // (computed for every element and then selected: no branch per element)
-                                    val[e] = (half_t)gelu_bwd((float)ad[sl % 4][it][e], (float)val[e]);
-                                }
-                                val = keep8_of(val, w);
-#pragma unroll
-                                for (int e = 0; e < 8; ++e) colsum[hb][e] += (float)val[e];
-                            }
-                            if constexpr (EPI == EPI_GELU_DROPOUT) {
-                                put(rl, at, uni, val);                       // the pre-activation, for the backward pass
-                                const uint32_t w = draw.kb[c >> 2] >> (8 * (c & 3));
-#pragma unroll
-                                for (int e = 0; e < 8; ++e) {
-                                    val[e] = (half_t)gelu_fwd((float)val[e]);      // for every element, then selected: no branches
-                                }
-                                val = keep8_of(val, w);
-                            }
-                            if constexpr (EPI == EPI_RELU_DROPOUT || EPI == EPI_RELU_DROPOUT_PRE) {
-                                // what the bias-activation-dropout operator does to the rounded sum, with the same keep
-                                // bits (the element index is the offset into the dense output)
-                                const uint32_t w = (EPI == EPI_RELU_DROPOUT ? draw.kb[c >> 2] : bits[EPI == EPI_RELU_DROPOUT ? 0 : c >> 2]) >> (8 * (c & 3));
-                                val = keep8_of(__builtin_elementwise_max(val, (h8)(half_t)0.0f), w);       // ReLU, packed
-                                const uint32_t positive = nonzero8(val);
-                                out_bits[c >> 2] = (c & 3) ? out_bits[c >> 2] | (positive << (8 * (c & 3))) : positive;
+                            if constexpr (EPI == EPI_GELU_DROPOUT) put(rl, at, uni, val);          // the pre-activation, for the backward pass
+                            if constexpr (DRAWS || EPI == EPI_RELU_DROPOUT_PRE) {
+                                uint32_t keep;
+                                if constexpr (DRAWS) keep = draw.kb[c >> 2] >> (8 * (c & 3));
+                                else keep = quad_byte<c & 3>(bits[c >> 2], lane);
+                                val = act_forward<EPI>(val, keep);
+                                const uint32_t word = quad_word(keep, lane);
+                                out_word = (lane & 3) == (c & 3) ? word : out_word;
+                                if constexpr ((c & 3) == 3)
+                                    __builtin_amdgcn_raw_buffer_store_b32(out_word, ro, (int)at_o[c >> 3 & 1], (int)bits_part(g, c >> 2), 0);
                             }
                             put(rc, at, uni, val);
-                        }
+                        });
                     }
-                    // (a slab's arithmetic is not spread over the next ones': registers)
-                    if (EPI == EPI_GELU_GATE_COLSUM) __builtin_amdgcn_sched_barrier(0);
                     if constexpr (ADD >= 2 && sl + 4 < 4 * TA) addends(std::integral_constant<int, sl + 4>{});
                 });
             };
@@ -605,21 +559,9 @@ struct Wide : TileList<4 * QM, 4 * QN, NP> {
                 else if (g.sbM == 0) tile(std::integral_constant<int, 1>{});
                 else tile(std::integral_constant<int, 2>{});
             }
-            if constexpr (EPI == EPI_RELU_DROPOUT || EPI == EPI_RELU_DROPOUT_PRE || EPI == EPI_GELU_DROPOUT) {
-                if (g.gate_bits_out) {
-                    // one bit per output (ReLU: set = positive; GELU: the keep bits) in the order in which this kernel walks a
-                    // tile: the gate of a product with the same output shape reads 1/16 of what the outputs themselves would cost it
-                    uint4* to = reinterpret_cast<uint4*>(g.gate_bits_out);
-#pragma unroll
-                    for (int i = 0; i < 2; ++i)
-                        to[bits_at + i * 64] = EPI == EPI_GELU_DROPOUT
-                            ? make_uint4(draw.kb[i * 4], draw.kb[i * 4 + 1], draw.kb[i * 4 + 2], draw.kb[i * 4 + 3])
-                            : make_uint4(out_bits[i * 4], out_bits[i * 4 + 1], out_bits[i * 4 + 2], out_bits[i * 4 + 3]);
-                }
-            }
             if constexpr (GATED) {
                 // lanes LPR apart hold the same 8 columns for other rows: add them up, then one fp32 row of partial sums
-                // per 128 rows of the output (a finishing launch adds them up)
+                // per wave (a finishing launch adds them up)
 #pragma unroll
                 for (int o = LPR; o < 64; o <<= 1)
 #pragma unroll
@@ -629,6 +571,7 @@ struct Wide : TileList<4 * QM, 4 * QN, NP> {
                 if (lane < LPR) {
 #pragma unroll
                     for (int hb = 0; hb < 2; ++hb) {
+                        if (hb * HN + nl >= cols) continue;
                         float* dst = g.colsum + ((long)(t.m0 / BM) * 2 + wm) * g.N + n_wave + hb * HN + lane * 8;
 #pragma unroll
                         for (int e = 0; e < 8; ++e) dst[e] = colsum[hb][e];
@@ -690,9 +633,5 @@ void launch_wide_as(const TileGroup<NP>& G, int k1, int k2, unsigned blocks, hip
 }
 
 }  // namespace
-
-// One product with activation EPI in its epilogue (k_gemm_wide_act.hip, compiled once for each of them).
-template <int EPI>
-void launch_wide_act(const TileProduct& p, hipStream_t st);
 
 }  // namespace sub

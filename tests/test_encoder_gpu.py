@@ -1292,3 +1292,45 @@ def test_restored_tensors_are_not_taken_for_what_lay_at_their_addresses(python):
         for a, b in zip(want[0], torch.autograd.grad(y, enc.params, dy)):
             assert torch.equal(a, b)
     assert len(set(addresses)) < len(addresses)          # otherwise nothing was tested
+
+
+@pytest.mark.parametrize('dims', [(1, 64, 12, 768, 3072), (1, 16, 4, 256, 800), (5, 72, 4, 512, 1056), (13, 201, 12, 768, 3072),
+                                  (24, 77, 12, 768, 3072), (3, 1000, 8, 1024, 4128)])
+@pytest.mark.parametrize('activation', ['relu', 'gelu'])
+@pytest.mark.parametrize('p', [0.1, 0.0])
+def test_activation_epilogues_on_tiles_of_every_size_equal_the_operators(dims, activation, p):
+    """Bias, activation and dropout in the epilogue of the product before them, and their backward pass, on tiles from
+    64 x 64 (few tokens) to 256 x 256 (3000 of them), with rows and columns of tiles that are not whole (U = 800, 1056,
+    4128 end inside a tile of each size) and without dropout: output and every gradient bit for bit those of the
+    operators, the bias gradient (the same terms in another order) to rounding.  Twice, as the bits that the
+    forward pass leaves lie in a buffer that is used again."""
+    from substation_amd import Encoder, layouts as L
+    B, Ls, H, E, U = dims
+    outs = []
+    for from_output in (0, 1):
+        torch.manual_seed(0)
+        enc = Encoder('unused', B, Ls, H, E, L.mi355x_layouts(), torch.float16, p, p, p, p, seed=SEED, intermediate_size=U,
+                      activation=activation).cuda()
+        enc._handle.set_option(6, from_output)
+        g = torch.Generator().manual_seed(5)
+        with torch.no_grad():
+            for q in enc.parameters():
+                q.mul_(0.1)
+        got = []
+        for step in range(2):
+            X = (0.5 * torch.randn(B, Ls, E, generator=g)).half().cuda().requires_grad_(True)
+            DY = torch.randn(B, Ls, E, generator=g).half().cuda()
+            enc.set_rng(SEED, step)
+            enc.zero_grad()
+            Y = enc(X)
+            Y.backward(DY)
+            torch.cuda.synchronize()
+            got += [('Y', Y.detach().clone()), ('DX', X.grad.clone())] + [('D' + n, q.grad.clone()) for n, q in enc.named_parameters()]
+        outs.append(got)
+    for (name, a), (_, b) in zip(*outs):
+        assert torch.isfinite(b.float()).all() and float(b.float().abs().max()) > 0, name
+        if name == 'DLINB1':
+            # sums of up to 3000 fp32 terms in another order, rounded to fp16 once: 2^-11 and 3000 2^-24 of the terms' size
+            assert_close(b.float().cpu().numpy(), a.float().cpu().numpy(), tol=2e-3, name=name)
+        else:
+            assert torch.equal(a, b), name
