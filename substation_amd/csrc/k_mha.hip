@@ -697,10 +697,41 @@ struct KvStage {
     uint32_t keep[4][32];         // [wave's key tile][query]
 };
 
+// acc += a b with acc in the accumulation registers, where the 128 of dK and dV at head size 128 leave the ordinary ones
+// to everything that vector instructions work on.  The compiler does not see what this is: the two wait states that an
+// operand written by a vector instruction needs are spelled out, and settle() stands between the last product and the
+// first read of acc.
+__device__ __forceinline__ void add_product(f16v& acc, h8 a, h8 b) {
+    asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+}
+// acc = a b and acc += a b with b in the accumulation registers and acc in the ordinary ones; nothing may read acc within
+// the 18 wait states that follow.
+__device__ __forceinline__ void set_product(f16v& acc, h8 a, h8 b) {
+    asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_f16 %0, %1, %2, 0" : "=&v"(acc) : "v"(a), "a"(b));
+}
+__device__ __forceinline__ void add_product_v(f16v& acc, h8 a, h8 b) {
+    asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "a"(b));
+}
+template <int N>
+__device__ __forceinline__ void settle(f16v (&acc)[N]) {
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < N; ++i) asm volatile("" : "+a"(acc[i]));
+}
+
 template <int P, bool MASKED, bool RAGGED>
 __global__ __launch_bounds__(256, (P == 64 && MASKED) ? 2 : 1) void k_mha_bwd_dkv(AttnArgs a) {
     using G = Geo<P>;
-    __shared__ __attribute__((aligned(16))) KvStage<P> stage[RING];
+    // Head size 128 has one wave per SIMD, in which the vector work on a tile and the products around it wait for one another
+    // (4400 cycles a tile, of which the matrix pipe works 1024).  There the scores of a tile are formed during the vector
+    // work on the one before it, a product for each element, dV and dK behind them; the fragments come from LDS a few
+    // products ahead of their use, the tiles of queries from memory four tiles ahead.  The registers allow it with dK,
+    // dV and the wave's own K and V in the accumulation half.  H 32, P 128, 4 x 2048: 1048 -> 759 us, of which 145 us lie
+    // before and behind the tiles.  (Fragments all read a tile ahead: 44 loads a tile from scratch.  Tiles fetched
+    // five ahead: 787 us.  With a mask the tiles are taken from a list and begin from mask values: as for head size 64,
+    // where two waves per SIMD fill each other's gaps.)
+    constexpr bool AHEAD = P == 128 && !MASKED;
+    __shared__ __attribute__((aligned(16))) KvStage<P> stage[AHEAD ? 4 : RING];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, hi = lane >> 5;
     const unsigned kblocks = RAGGED ? (a.K + QB - 1) / QB : a.K / QB;
     const unsigned lb = logical_block();
@@ -747,6 +778,153 @@ __global__ __launch_bounds__(256, (P == 64 && MASKED) ? 2 : 1) void k_mha_bwd_dk
     };
     InFlight fl;
     fl.stat = 0.f; fl.kw = make_uint4(0, 0, 0, 0);
+    f16v dk[G::NPT], dv[G::NPT];
+#pragma unroll
+    for (int pt = 0; pt < G::NPT; ++pt)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) { dk[pt][v] = 0.f; dv[pt][v] = 0.f; }
+    if constexpr (AHEAD) {
+        // The tiles in turn, by addresses that move along (worked out for each tile they are a dozen 64-bit products in the
+        // open), the last one again behind it.  Each lane brings one word besides: the lower half of wave w the keep words of
+        // its keys, the upper halves the statistics, so that no branch has a load on its way kept until its end.
+        const half_t* pq = a.q.p + (long)h * a.q.sh + (long)b * a.q.sb + (long)(tid / (P / 8)) * a.q.sr + tid % (P / 8) * 8;
+        const half_t* pd_o = a.d_o.p + (long)h * a.d_o.sh + (long)b * a.d_o.sb + (long)(tid / (P / 8)) * a.d_o.sr + tid % (P / 8) * 8;
+        const uint32_t* small = hi ? reinterpret_cast<const uint32_t*>(wave & 1 ? a.dsum : a.lse) + row0
+                                   : a.keep + (size_t)row0 * nkt + kb * 4 + wave;
+        const long small_row = hi ? 1 : nkt;
+        if (!RAGGED) small += l32 * small_row;
+        uint32_t* const small_to = hi ? reinterpret_cast<uint32_t*>(wave & 1 ? stage[0].dsum : stage[0].lse) + l32 : stage[0].keep[wave] + l32;
+        unsigned upto = 0;
+        struct Tile { h8 q[2], d_o[2]; uint32_t w; };
+        auto bring = [&](Tile& f) __attribute__((always_inline)) {
+            if (RAGGED) {
+                const unsigned q = upto * 32 + l32, last = (unsigned)a.J - 1;
+                tile_fetch<P, RAGGED>(a.q, h, b, upto * 32, a.J, tid, f.q);
+                tile_fetch<P, RAGGED>(a.d_o, h, b, upto * 32, a.J, tid, f.d_o);
+                f.w = small[min(q, last) * small_row];
+                ++upto;
+            } else {
+                f.q[0] = *reinterpret_cast<const h8*>(pq);
+                f.q[1] = *reinterpret_cast<const h8*>(pq + 16 * a.q.sr);
+                f.d_o[0] = *reinterpret_cast<const h8*>(pd_o);
+                f.d_o[1] = *reinterpret_cast<const h8*>(pd_o + 16 * a.d_o.sr);
+                f.w = *small;
+                const long on = ++upto < n ? 32 : 0;
+                pq += on * a.q.sr;
+                pd_o += on * a.d_o.sr;
+                small += on * small_row;
+            }
+        };
+        // Tile t into its stage.
+        auto lay = [&](unsigned t, const Tile& f) __attribute__((always_inline)) {
+            KvStage<P>& sg = stage[t & 3];
+            tile_put<P>(sg.q, tid, f.q);
+            tile_put<P>(sg.d_o, tid, f.d_o);
+            // (a log-sum-exp of +inf: the probabilities of a query past the end are zero)
+            const bool beyond = RAGGED && hi && !(wave & 1) && t * 32 + l32 >= (unsigned)a.J;
+            small_to[(t & 3) * (sizeof(KvStage<P>) / 4)] = beyond ? 0x7F800000u : f.w;
+        };
+        Tile way;
+        {
+            Tile f1, f2;
+            bring(way);
+            bring(f1);
+            bring(f2);
+            row_frags<P>(a.k, h, b, kpos, hi, fk);
+            row_frags<P>(a.v, h, b, kpos, hi, fv);
+            lay(0, way);
+            lay(1, f1);
+            lay(2, f2);
+        }
+        __syncthreads();
+        wait_loads();
+#pragma unroll
+        for (int ks = 0; ks < G::NKS; ++ks) asm volatile("" : "+a"(fk[ks]), "+a"(fv[ks]));
+        bring(way);
+        constexpr int NS = 4, NT = 5;
+        h8 rq[NS], rd[NS], tr[8];       // fragments on their way: NS slices of the features, NT transposed ones
+        auto slice = [&](const KvStage<P>& sg, int ks) __attribute__((always_inline)) {
+            rq[ks % NS] = *reinterpret_cast<const h8*>(sg.q + Geo<P>::at(l32, 2 * ks + hi));
+            rd[ks % NS] = *reinterpret_cast<const h8*>(sg.d_o + Geo<P>::at(l32, 2 * ks + hi));
+        };
+        // fragment f of the sixteen that dV and dK take: dO and Q in turn, feature tile f / 2 % NPT, half f / 8 of the queries
+        auto turned = [&](const KvStage<P>& sg, int f) __attribute__((always_inline)) {
+            tr[f & 7] = tr_frag<P>(f & 1 ? sg.q : sg.d_o, (f / 2 % G::NPT) * 32, f / (2 * G::NPT), lane);
+        };
+        f16v s0, dp0, s1, dp1;
+        auto scores = [&](const KvStage<P>& next, auto V, f16v& sn, f16v& dpn) __attribute__((always_inline)) {      // product V
+            constexpr int ks = V / 2;
+            if constexpr (V == 0) set_product(sn, rq[0], fk[0]);
+            else if constexpr (V == 1) set_product(dpn, rd[0], fv[0]);
+            else if constexpr (V % 2 == 0) add_product_v(sn, rq[ks % NS], fk[ks]);
+            else add_product_v(dpn, rd[ks % NS], fv[ks]);
+            if constexpr (V % 2 == 1 && ks + NS < G::NKS) slice(next, ks + NS);
+        };
+        each<NS>([&](auto S) __attribute__((always_inline)) { slice(stage[0], S); });
+        each<2 * G::NKS>([&](auto V) __attribute__((always_inline)) { scores(stage[0], V, s0, dp0); });
+        each<NS>([&](auto S) __attribute__((always_inline)) { slice(stage[1], S); });
+        asm volatile("s_nop 15\n\ts_nop 15" : "+v"(s0), "+v"(dp0));
+        // Tile i, whose scores are (s, dp); those of tile i + 1 into (sn, dpn) (behind the last tile: of what lies there, unused).
+        auto tile = [&](unsigned i, const f16v& s, const f16v& dp, f16v& sn, f16v& dpn) __attribute__((always_inline)) {
+            const KvStage<P>&sg = stage[i & 3], &next = stage[(i + 1) & 3], &after = stage[(i + 2) & 3];
+            if (working) {
+                h8 pd[2], ds[2];
+                float4 ls[2], dd[2];
+                uint4 w[2];
+                auto stats = [&](int q) __attribute__((always_inline)) {
+                    ls[q & 1] = *reinterpret_cast<const float4*>(sg.lse + q * 8 + hi * 4);
+                    dd[q & 1] = *reinterpret_cast<const float4*>(sg.dsum + q * 8 + hi * 4);
+                    w[q & 1] = *reinterpret_cast<const uint4*>(sg.keep[wave] + q * 8 + hi * 4);
+                };
+                stats(0);
+                float p[2];
+                int keep[2];
+                auto second = [&](auto V) __attribute__((always_inline)) {       // of element V: what follows its exponential
+                    constexpr int v = V, q = v / 4, e = v % 4;
+                    const float ddv = e == 0 ? dd[q & 1].x : e == 1 ? dd[q & 1].y : e == 2 ? dd[q & 1].z : dd[q & 1].w;
+                    pd[v >> 3][v & 7] = (half_t)__int_as_float(__float_as_int(p[v & 1]) & keep[v & 1]);
+                    ds[v >> 3][v & 7] = (half_t)(p[v & 1] * (__int_as_float(__float_as_int(dp[v]) & keep[v & 1]) - ddv));
+                };
+                each<16>([&](auto V) __attribute__((always_inline)) {
+                    constexpr int v = V, q = v / 4, e = v % 4;
+                    scores(next, V, sn, dpn);
+                    if constexpr (e == 1 && q < 3) stats(q + 1);
+                    if constexpr (v >= 16 - NT) turned(sg, v - 16 + NT);
+                    if constexpr (v > 0) second(std::integral_constant<int, v - 1>{});
+                    const float lsv = e == 0 ? ls[q & 1].x : e == 1 ? ls[q & 1].y : e == 2 ? ls[q & 1].z : ls[q & 1].w;
+                    const uint32_t wv = e == 0 ? w[q & 1].x : e == 1 ? w[q & 1].y : e == 2 ? w[q & 1].z : w[q & 1].w;
+                    p[v & 1] = __builtin_amdgcn_exp2f(fmaf(s[v], c, -lsv));
+                    keep[v & 1] = __builtin_amdgcn_sbfe((int)wv, l32, 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                });
+                second(std::integral_constant<int, 15>{});
+                each<4 * G::NPT>([&](auto F) __attribute__((always_inline)) {
+                    constexpr int f = F, st = f / (2 * G::NPT), pt = f / 2 % G::NPT;
+                    if constexpr (f + NT < 4 * G::NPT) turned(sg, f + NT);
+                    if constexpr (f >= 2 && f % 2 == 0 && f / 2 <= NS) slice(after, f / 2 - 1);
+                    if constexpr (f == 7) lay(i + 3, way);
+                    if constexpr (f == 9) bring(way);
+                    if constexpr (f & 1) add_product(dk[pt], tr[f & 7], ds[st]);
+                    else add_product(dv[pt], tr[f & 7], pd[st]);
+                    __builtin_amdgcn_sched_barrier(0);
+                });
+                asm volatile("" : "+v"(sn), "+v"(dpn));      // (theirs until the products have arrived, also where unused)
+            }
+            if (!working) {
+                lay(i + 3, way);
+                bring(way);
+            }
+            __syncthreads();
+        };
+        unsigned i = 0;
+        do {
+            tile(i, s0, dp0, s1, dp1);
+            if (i + 1 < n) tile(i + 1, s1, dp1, s0, dp0);
+            i += 2;
+        } while (i < n);
+        settle(dk);
+        settle(dv);
+    } else {
     {
         InFlight f1;
         f1.stat = 0.f; f1.kw = make_uint4(0, 0, 0, 0);
@@ -761,11 +939,6 @@ __global__ __launch_bounds__(256, (P == 64 && MASKED) ? 2 : 1) void k_mha_bwd_dk
     row_frags_lds<P>(stage[0].q, l32, hi, fq);
     row_frags_lds<P>(stage[0].d_o, l32, hi, fdo);
 
-    f16v dk[G::NPT], dv[G::NPT];
-#pragma unroll
-    for (int pt = 0; pt < G::NPT; ++pt)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) { dk[pt][v] = 0.f; dv[pt][v] = 0.f; }
     int cur = 0, nxt = 1, nn = 2;
     MaskRegs mk = {};
     if (MASKED && n > 0 && entry_class(e0, wave) != BLOCK_CLEAR) load_mask<false, RAGGED>(a, kpos, entry_tile(e0) * 32, hi, mk);
@@ -827,6 +1000,7 @@ __global__ __launch_bounds__(256, (P == 64 && MASKED) ? 2 : 1) void k_mha_bwd_dk
         __syncthreads();
         const int x = cur; cur = nxt; nxt = nn; nn = x;
         e0 = e1; e1 = e2; e2 = e3;
+    }
     }
     if (mine_) {
         store_rows<P>(a.dk, h, b, kpos, hi, dk, a.alpha);

@@ -5,6 +5,7 @@
 
 #include <hip/hip_runtime.h>
 #include <cstdint>
+#include <type_traits>
 
 #include "sub_philox.hpp"
 
@@ -16,6 +17,15 @@ typedef _Float16 h4 __attribute__((ext_vector_type(4)));
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 
 constexpr int WAVE = 64;
+
+// f(0), f(1) .. f(N - 1), the index a constant of the type.
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void each(const F& f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        each<N, I + 1>(f);
+    }
+}
 
 // Row space: up to four outer dimensions (canonical order) times a row of R
 // elements.  The canonical element index of (row r, column e) is r*R + e.

@@ -14,15 +14,6 @@ namespace {
 
 typedef uint32_t u4v __attribute__((ext_vector_type(4)));
 
-// f(0), f(1) .. f(N - 1), the index a constant of the type.
-template <int N, int I = 0, typename F>
-__device__ __forceinline__ void each(const F& f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        each<N, I + 1>(f);
-    }
-}
-
 __device__ __forceinline__ unsigned lds_addr(const void* p) {
     return (unsigned)(uintptr_t)(__attribute__((address_space(3))) const void*)p;
 }

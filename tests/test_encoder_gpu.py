@@ -232,6 +232,16 @@ def test_attention_in_registers_at_any_sequence_length(dims, masked, compact):
     _compare(want, got, names=OUTPUTS)
 
 
+# one to six query tiles, and the multiples of 128: the pipeline's stages are filled before it knows how many it needs
+@pytest.mark.parametrize('L', [8, 33, 65, 100, 128, 130, 161, 256, 384])
+def test_attention_backward_at_head_size_128_for_few_and_odd_query_tiles(L):
+    """Without a mask, head size 128 forms the scores of a query tile during the work on the one before it."""
+    launches = []
+    want, got = run_layer_default(2, L, 2, 256, 0.1, seed_data=L, launches=launches)
+    assert 'attention-bwd-dKdV' in launches and 'attention-bwd-dQ' in launches, launches
+    _compare(want, got, names=OUTPUTS)
+
+
 @pytest.mark.parametrize('dims,masked', [((3, 8, 2, 128), False), ((2, 77, 2, 128), False), ((2, 72, 2, 256), True),
                                          ((1, 519, 2, 128), True), ((1, 1030, 1, 64), False)])
 def test_relu_forward_in_operators_backward_in_registers(dims, masked):
