@@ -122,11 +122,19 @@ __device__ __forceinline__ unsigned logical_block() {
 // Position (within a tile of 32) that accumulator register v of a lane holds.
 __device__ __forceinline__ constexpr int reg_pos(int v, int hi) { return (v >> 2) * 8 + hi * 4 + (v & 3); }
 
-// Output rows: D[feature, position] accumulators -> t[position][feature], 8-byte pieces.
-template <int P>
-__device__ __forceinline__ void store_rows(const AttnSide& t, unsigned h, unsigned b, unsigned pos, int hi,
-                                           const f16v (&acc)[P / 32], float scale) {
-    half_t* p = const_cast<half_t*>(t.p) + (long)h * t.sh + (long)b * t.sb + (long)pos * t.sr + hi * 4;
+// Output rows: D[feature, position] accumulators of a wave -> t[position][feature] for its 32 positions from pos0 on,
+// those below `limit`, by way of LDS (`tile`: 32 * P halves, the wave's own): an accumulator holds a position per lane, so
+// that straight from the registers an instruction writes 16 bytes to each of 32 rows, and from LDS whole rows.  On the way
+// the columns of what is stored are summed, into `sums` (of the wave: 4 rows of P floats, one for each 16 lanes; or null).
+// Straight from the registers 6 of the 35 us of dK and dV at H 16, P 64, 8 x 512 were the stores and 1 the sums (9
+// instructions a value), at 96 x 128 17 and 1 of 48.  This way: 8 x 512: dK and dV 35.3 -> 32.4 us, forward 26.3 -> 25.7;
+// 96 x 128: dK and dV 48.5 -> 38.3, dQ 41.9 -> 38.3, forward 31.5 -> 28.0.
+template <int P, bool RAGGED>
+__device__ __forceinline__ void store_rows(const AttnSide& t, unsigned h, unsigned b, unsigned pos0, unsigned limit, int lane,
+                                           const f16v (&acc)[P / 32], float scale, half_t* tile, float* sums) {
+    constexpr int PER = P / 8, ROWS = WAVE / PER;      // 16-byte words of a row, rows of an instruction
+    const int l32 = lane & 31, hi = lane >> 5, row = lane / PER, chunk = lane % PER;
+    __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int pt = 0; pt < P / 32; ++pt)
 #pragma unroll
@@ -134,8 +142,40 @@ __device__ __forceinline__ void store_rows(const AttnSide& t, unsigned h, unsign
             h4 w;
 #pragma unroll
             for (int e = 0; e < 4; ++e) w[e] = (half_t)(acc[pt][q * 4 + e] * scale);
-            *reinterpret_cast<h4*>(p + pt * 32 + q * 8) = w;
+            *reinterpret_cast<h4*>(tile + Geo<P>::at(l32, pt * 4 + q) + hi * 4) = w;
         }
+    __builtin_amdgcn_wave_barrier();
+    half_t* p = const_cast<half_t*>(t.p) + (long)h * t.sh + (long)b * t.sb + (long)(pos0 + row) * t.sr + chunk * 8;
+    h8 w[32 / ROWS];
+#pragma unroll
+    for (int i = 0; i < 32 / ROWS; ++i) w[i] = *reinterpret_cast<const h8*>(tile + Geo<P>::at(i * ROWS + row, chunk));
+#pragma unroll
+    for (int i = 0; i < 32 / ROWS; ++i)
+        if (!RAGGED || pos0 + i * ROWS + row < limit) *reinterpret_cast<h8*>(p + (long)(i * ROWS) * t.sr) = w[i];
+    if (!sums) return;
+    float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < 32 / ROWS; ++i) {
+        const bool in = !RAGGED || pos0 + i * ROWS + row < limit;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] += in ? (float)w[i][e] : 0.f;
+    }
+    if (P == 64) {          // two rows in 16 lanes
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] += dpp<0x128>(x[e]);
+        if (lane & 8) return;
+    }
+#pragma unroll
+    for (int e = 0; e < 8; e += 4)
+        *reinterpret_cast<float4*>(sums + (lane >> 4) * P + chunk * 8 + e) = make_float4(x[e], x[e + 1], x[e + 2], x[e + 3]);
+}
+// One value per feature of what four waves have left in `sums`; behind a barrier.
+template <int P>
+__device__ __forceinline__ float column_sum(const float* sums, int feature) {
+    float x[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < 16; ++i) x[i & 3] += sums[i * P + feature];
+    return (x[0] + x[1]) + (x[2] + x[3]);
 }
 
 // x where bit `pos` of `bits` is set, else +0.0
@@ -152,41 +192,6 @@ __device__ __forceinline__ void drop_past_end(f16v& s, unsigned tile0, unsigned 
 
 // Words of keep bits per score row: one per 32 keys, in whole groups of four (mha_keep_pitch).
 __device__ __forceinline__ unsigned keep_pitch(unsigned K) { return (K + QB - 1) / QB * 4; }
-
-// Sums over the 128 positions of a workgroup of the rows store_rows() writes
-// (same rounding), one value per feature: 32 lanes hold the positions of a
-// wave, the four waves meet in LDS (`red`: 4 * P floats, free to use).
-template <int P>
-__device__ __forceinline__ void column_sums(const f16v (&acc)[P / 32], float scale, float* red, float* out,
-                                            int tid) {
-    const int lane = tid & 63, wave = tid >> 6, l32 = lane & 31, hi = lane >> 5;
-    // Five DPP steps per value and no trip through LDS: four total each row of 16 lanes, the fifth
-    // (row_bcast15 into rows 1 and 3) adds the row below, so that lanes 16..31 (48..63) hold the total
-    // of lanes 0..31 (32..63).  All values first and then the store: the chains are independent and
-    // fill each other's wait states.  (With a ds_bpermute as the last step the 32 values of a lane went
-    // through LDS one after the other, 2 to 3 us at the end of every workgroup.)
-    float x[P / 32][16];
-#pragma unroll
-    for (int pt = 0; pt < P / 32; ++pt)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            float t = (float)(half_t)(acc[pt][v] * scale);
-            t += dpp<0xB1>(t);
-            t += dpp<0x4E>(t);
-            t += dpp<0x141>(t);
-            t += dpp<0x140>(t);
-            t += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(t), 0x142, 0xA, 0xF, false));
-            x[pt][v] = t;
-        }
-    if (l32 == 16) {
-#pragma unroll
-        for (int pt = 0; pt < P / 32; ++pt)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) red[wave * P + pt * 32 + reg_pos(v, hi)] = x[pt][v];
-    }
-    __syncthreads();
-    if (tid < P) out[tid] = (red[tid] + red[P + tid]) + (red[2 * P + tid] + red[3 * P + tid]);
-}
 
 // Additive attention mask (substation/attention.py:65-68: added to the raw scores,
 // before the scaling) for the 16 scores of a lane.  QUERY_LANES: the lane holds
@@ -519,9 +524,8 @@ __global__ __launch_bounds__(256) void k_mha_fwd(AttnArgs a, PhiloxKey key_) {
         e0 = e1; e1 = e2; e2 = e3;
     }
     const float l_tot = l_run + __shfl_xor(l_run, 32);
-    if (!mine_) return;
-    store_rows<P>(a.o, h, b, j, hi, o, 1.0f / l_tot);
-    if (hi == 0) a.lse[row] = m_ref * c + __builtin_amdgcn_logf(l_tot);
+    store_rows<P, RAGGED>(a.o, h, b, qb * QB + wave * 32, a.J, lane, o, 1.0f / l_tot, wave < 2 ? kt[wave] : vt[wave - 2], nullptr);
+    if (mine_ && hi == 0) a.lse[row] = m_ref * c + __builtin_amdgcn_logf(l_tot);
 }
 
 // ---------------------------------------------------------------------------
@@ -671,16 +675,12 @@ __global__ __launch_bounds__(256, !MASKED ? (P == 128 ? 2 : 3) : 1) void k_mha_b
         const int x = cur; cur = nxt; nxt = nn; nn = x;
         e0 = e1; e1 = e2; e2 = e3;
     }
-    if (mine_) store_rows<P>(a.dq, h, b, j, hi, dq, a.alpha);
-    if (RAGGED && !mine_) {       // nothing to the column sums
-#pragma unroll
-        for (int pt = 0; pt < G::NPT; ++pt)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) dq[pt][v] = 0.f;
-    }
-    if (a.bias_q)
-        column_sums<P>(dq, a.alpha, reinterpret_cast<float*>(&kt[0][0]),
-                       a.bias_q + ((size_t)h * (a.B * qblocks) + b * qblocks + qb) * P, tid);
+    float* const sums = a.bias_q ? reinterpret_cast<float*>(kt[2]) : nullptr;       // (of 4 waves 64 * P bytes, a tile's)
+    store_rows<P, RAGGED>(a.dq, h, b, qb * QB + wave * 32, a.J, lane, dq, a.alpha, wave < 2 ? kt[wave] : vt[wave - 2],
+                          sums ? sums + wave * 4 * P : nullptr);
+    if (!sums) return;
+    __syncthreads();
+    if (tid < P) a.bias_q[((size_t)h * (a.B * qblocks) + b * qblocks + qb) * P + tid] = column_sum<P>(sums, tid);
 }
 
 // ---------------------------------------------------------------------------
@@ -740,7 +740,6 @@ __global__ __launch_bounds__(256, (P == 64 && MASKED) ? 2 : 1) void k_mha_bwd_dk
     if (MASKED) masked_order(a.klist, kblocks, nq, a.H * a.B, lb, kb, hb);
     const unsigned b = hb % a.B, h = hb / a.B;
     const unsigned kpos_ = kb * QB + wave * 32 + l32;                // this lane's key
-    const bool mine_ = !RAGGED || kpos_ < (unsigned)a.K;
     const unsigned kpos = RAGGED ? min(kpos_, (unsigned)a.K - 1) : kpos_;
     const bool working = !RAGGED || __builtin_amdgcn_readfirstlane((int)(kb * QB + wave * 32)) < a.K;
     const unsigned row0 = (h * a.B + b) * a.J;                       // score row of query 0
@@ -1002,21 +1001,15 @@ __global__ __launch_bounds__(256, (P == 64 && MASKED) ? 2 : 1) void k_mha_bwd_dk
         e0 = e1; e1 = e2; e2 = e3;
     }
     }
-    if (mine_) {
-        store_rows<P>(a.dk, h, b, kpos, hi, dk, a.alpha);
-        store_rows<P>(a.dv, h, b, kpos, hi, dv, 1.0f);
-    } else if (RAGGED) {          // nothing to the column sums
-#pragma unroll
-        for (int pt = 0; pt < G::NPT; ++pt)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) { dk[pt][v] = 0.f; dv[pt][v] = 0.f; }
-    }
-    if (a.bias_kv) {
-        const size_t ntc = (size_t)a.B * kblocks, part = (size_t)h * ntc + b * kblocks + kb;
-        float* red = reinterpret_cast<float*>(&stage[0]);
-        column_sums<P>(dk, a.alpha, red, a.bias_kv + part * P, tid);
-        column_sums<P>(dv, 1.0f, red + 4 * P, a.bias_kv + ((size_t)a.H * ntc + part) * P, tid);
-    }
+    half_t* const tile = wave < 2 ? stage[wave].q : stage[wave - 2].d_o;
+    float* const sums_k = reinterpret_cast<float*>(stage[2].q);         // (of 4 waves 64 * P bytes, a tile's)
+    float* const sums_v = reinterpret_cast<float*>(stage[2].d_o);
+    store_rows<P, RAGGED>(a.dk, h, b, kb * QB + wave * 32, a.K, lane, dk, a.alpha, tile, a.bias_kv ? sums_k + wave * 4 * P : nullptr);
+    store_rows<P, RAGGED>(a.dv, h, b, kb * QB + wave * 32, a.K, lane, dv, 1.0f, tile, a.bias_kv ? sums_v + wave * 4 * P : nullptr);
+    if (!a.bias_kv) return;
+    __syncthreads();
+    const size_t ntc = (size_t)a.B * kblocks, part = (size_t)h * ntc + b * kblocks + kb;
+    if (tid < 2 * P) a.bias_kv[((tid < P ? 0 : (size_t)a.H * ntc) + part) * P + tid % P] = column_sum<P>(tid < P ? sums_k : sums_v, tid % P);
 }
 
 // Whether the kernels have to watch the ends of the sequences.
