@@ -477,8 +477,9 @@ void plan_layouts(Handle& h, bool own) {
         h.lX = make_layout("BJI", sz); h.lY = make_layout("BJI", sz);
         h.stage_x = h.xX.str() != "BJI"; h.stage_y = h.xY.str() != "BJI";
         for (int i = 0; i < SUB_N_PARAMS; ++i) {
-            h.lp[i] = make_layout(kOwnP[i], sz);
-            h.stage_p[i] = h.xp[i].str() != kOwnP[i];
+            // (the feed-forward weights as they lie: the contraction kernels read and write both orders at the same rate)
+            h.lp[i] = i == LINW1 || i == LINW2 ? h.xp[i] : make_layout(kOwnP[i], sz);
+            h.stage_p[i] = h.xp[i].str() != h.lp[i].str();
         }
         for (int i = 0; i < SUB_N_FWD; ++i) h.lf[i] = make_layout(kOwnF[i], sz);
         for (int i = 0; i < SUB_N_BWD; ++i) h.lb[i] = make_layout(kOwnB[i], sz);

@@ -1261,6 +1261,21 @@ def test_a_caller_that_looks_into_the_intermediates_finds_them(dims, split):
         assert_close(shown[name].reshape(B * Ls, E).float().cpu().numpy(), want.cpu().numpy(), tol=1e-3, name=name)
 
 
+@pytest.mark.parametrize('dims,act', [((2, 40, 2, 128), 'gelu'), ((3, 77, 2, 128), 'relu'), ((4, 256, 8, 512), 'relu'),
+                                      ((4, 256, 8, 512), 'gelu')])
+@pytest.mark.parametrize('w1,w2', [('IU', 'UI'), ('IU', 'IU'), ('UI', 'UI'), ('UI', 'IU')])
+def test_feed_forward_weights_of_feature_major_layouts_as_they_lie(dims, act, w1, w2):
+    """Under a configuration that the layer runs in its own orders, LINW1 and LINW2 and their gradients are read and
+    written in the caller's: every order of the two, tiles with and without an activation in their epilogue."""
+    from substation_amd import layouts as L
+    lay = dict(L.reference_layouts('bert-b8-l512-h16-e1024'))
+    lay['params'] = [(n, {'LINW1': w1, 'LINW2': w2}.get(n, o)) for n, o in lay['params']]
+    launches = []
+    want, got = run_layer_default(*dims, 0.1, seed_data=dims[1], w_std=0.02, act=act, which=lay, launches=launches)
+    assert 'relayout-in' in launches, launches
+    _compare(want, got, names=OUTPUTS)
+
+
 @pytest.mark.parametrize('python', [False, True])
 def test_restored_tensors_are_not_taken_for_what_lay_at_their_addresses(python):
     """Hooks drop what two forward passes save and restore it for the backward passes, one after the other at the same
