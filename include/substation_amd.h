@@ -264,7 +264,7 @@ int sub_set_attention_mask(void* handle, const void* attn_mask, const char* layo
  * (pytorch_module/layouts-bert-*.pickle) -- encoder_forward / encoder_backward run the whole layer in those
  * orders: every intermediate lies in the library's order inside the caller's buffer (same number of
  * elements), and the tensors that cross the boundary in another order (input, output, their gradients,
- * weights, weight gradients; weights WKQV QHPI, BKQV QHP, WO IHP, LINW1 UI, LINW2 IU) are copied into it
+ * weights, weight gradients; weights WKQV QHPI, BKQV QHP, WO IHP; LINW1 and LINW2 are used as they lie) are copied into it
  * and back by a tiled transposing kernel (entries `relayout-in`, `relayout-out`, `relayout-in-bwd`,
  * `relayout-out-bwd` of the per-launch timing).
  * Outputs and gradients are the same to rounding; saved intermediates are NOT in the configured order

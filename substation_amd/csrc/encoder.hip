@@ -452,7 +452,8 @@ void configure(Handle& h, const sub_config* c) {
 // feature dim contiguous; the reference's shipped configurations are feature-major -- every intermediate
 // lives in the library's own order inside the caller's buffer (same number of elements), and the tensors that
 // cross the boundary (input, output, their gradients, weights, weight gradients) are copied into that order and
-// back by k_relayout.  A configuration whose activations are all in the library's orders runs as it is, with
+// back by k_relayout, all but LINW1, LINW2 and their gradients (16 of 25 MB of weights at E 1024; copied, the
+// relayout launches took 46 us of a pass at 8 x 512, now 35, and the layer 0.528 -> 0.516 ms).  A configuration whose activations are all in the library's orders runs as it is, with
 // its own weight orders.
 void plan_layouts(Handle& h, bool own) {
     const Sizes& sz = h.sz;
@@ -477,7 +478,7 @@ void plan_layouts(Handle& h, bool own) {
         h.lX = make_layout("BJI", sz); h.lY = make_layout("BJI", sz);
         h.stage_x = h.xX.str() != "BJI"; h.stage_y = h.xY.str() != "BJI";
         for (int i = 0; i < SUB_N_PARAMS; ++i) {
-            // (the feed-forward weights as they lie: the contraction kernels read and write both orders at the same rate)
+            // (the contraction kernels read and write both orders of a matrix at the same rate)
             h.lp[i] = i == LINW1 || i == LINW2 ? h.xp[i] : make_layout(kOwnP[i], sz);
             h.stage_p[i] = h.xp[i].str() != h.lp[i].str();
         }
