@@ -209,7 +209,8 @@ int sub_set_attention_mask(void* handle, const void* attn_mask, const char* layo
  * epilogue of lin1, which writes LIN1 (the backward pass needs it) and DROP2 and
  * leaves the keep bits of the dropout, one per element, in the first B*J*U/8 bytes
  * of SB1_LINW1 in place of the DROP2MASK tensor; encoder_backward runs bdrlb
- * (block_bdrlb.cuh:13-146) in the epilogue of dXlin2 from LIN1 and those bits.
+ * (block_bdrlb.cuh:13-146) in the epilogue of dXlin2 from LIN1 and those bits, or,
+ * where DLIN1, DLIN2 or LINW2 is no multiple of 16, as a launch of its own on them.
  * DROP2MASK, SB1_LINW1 and DDROP2 are not written; results are bit-identical
  * (DLINB1 to rounding).  encoder_backward knows from the options and the pointers
  * it is handed, which are the forward call's, that the bits lie in SB1_LINW1:

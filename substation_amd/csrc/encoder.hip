@@ -794,8 +794,8 @@ void op_bdrlb_from_output(Handle& h, const void* ddrop, const Layout& ld, const 
 // Both passes decide this from the handle alone, so they agree.
 bool relu_from_output(const Handle& h) { return h.relu_from_output && h.act == ACT_RELU; }
 // GELU: lin1 with bias, activation and dropout in its epilogue (LIN1 and DROP2 written, the keep bits left in the
-// SB1_LINW1 buffer instead of a DROP2MASK tensor) and dXlin2 with the backward of that in its epilogue.  Both or
-// neither: without DROP2MASK the separate backward operator has nothing to read.
+// SB1_LINW1 buffer, a byte per pack in canonical order, instead of a DROP2MASK tensor) and the backward of that in
+// dXlin2's epilogue, or, where that finds a tensor misaligned, in the operator of its own on those bits.
 bool act_epilogues(const Handle& h) {
     // (at the sizes where the products have always done it, also where somebody looks into the intermediates)
     return h.relu_from_output && h.fuse_epilogues && h.gemm[G_LIN1_BAD].ok && (h.opaque || h.act_whole);
@@ -1306,9 +1306,6 @@ void backward(Handle& h, const BwdPtrs& t0) {
                               aligned16(F[DROP2])) ||
                              bdrlb_gelu) &&
                             aligned16(D[DLIN1]) && aligned16(D[DLIN2]) && aligned16(W[LINW2]);
-    if (bdrlb_gelu && !fuse_bdrlb)
-        fail("encoder_backward: the forward call ran lin1 with the GELU epilogue (no DROP2MASK was written), and its "
-             "backward epilogue needs 16-byte aligned DLIN1, DLIN2 and LINW2");
     if (fuse_bdrlb) {
         // product, gate and the column sums of the result in one launch: DDROP2 is not produced
         ProfScope ps(h, "dXlin2+bdrlb");
@@ -1340,6 +1337,9 @@ void backward(Handle& h, const BwdPtrs& t0) {
         ProfScope ps(h, "bdrlb");
         if (relu_from_output(h))
             op_bdrlb_from_output(h, D[DDROP2], h.lb[DDROP2], F[DROP2], h.lf[DROP2], D[DLIN1], h.lb[DLIN1], DW[LINB1]);
+        else if (bdrlb_gelu)
+            op_bdrlb(h, D[DDROP2], h.lb[DDROP2], F[SB1_LINW1], h.lf[SB1_LINW1], F[LIN1], h.lf[LIN1], D[DLIN1], h.lb[DLIN1],
+                     DW[LINB1], true);
         else
             op_bdrlb(h, D[DDROP2], h.lb[DDROP2], F[DROP2MASK], h.lf[DROP2MASK], F[LIN1], h.lf[LIN1],
                      D[DLIN1], h.lb[DLIN1], DW[LINB1], packed_act_mask(h));
