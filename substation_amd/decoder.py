@@ -174,6 +174,8 @@ def _make_function(m):
         @staticmethod
         def backward(ctx, dy):
             x, enc, *params = ctx.saved_tensors
+            # (the epilogues of the backward pass need whole 16-byte words, wherever a parameter lies or was restored to)
+            params = [t if t.data_ptr() % 16 == 0 else t.clone() for t in params]
             w = dict(zip(names, params))
             s = ctx.saved
             dy = dy.contiguous()
@@ -197,7 +199,7 @@ def _make_function(m):
                                                        dlin1, 'BJU', g['linear1_b']):
                 if s['mask3'] is None:
                     raise RuntimeError('DecoderLayer: the forward pass ran linear1 with its activation epilogue, the '
-                                       'backward pass cannot (tensors not 16-byte aligned?)')
+                                       'backward pass cannot')
                 dff1 = e('BJU')
                 o.einsum(dff, 'BJI', w['linear2_w'], 'IU', dff1, 'BJU')
                 o.bdrlb(dff1, 'BJU', s['mask3'], 'BJU', s['lin1'], 'BJU', dlin1, 'BJU', g['linear1_b'])
