@@ -213,7 +213,8 @@ int sub_set_attention_mask(void* handle, const void* attn_mask, const char* layo
  * where DLIN1, DLIN2 or LINW2 is no multiple of 16, as a launch of its own on them.
  * DROP2MASK, SB1_LINW1 and DDROP2 are not written; results are bit-identical
  * (DLINB1 to rounding).  encoder_backward knows from the options and the pointers
- * it is handed, which are the forward call's, that the bits lie in SB1_LINW1:
+ * it is handed, which are the forward call's, that the bits lie in SB1_LINW1 (or
+ * is told, see sub_forward_form):
  * the option must not change between a forward call and its backward call.
  * Set it to 0 before the forward call when LIN1, DROP2MASK, SB1_LINW1 or
  * DDROP2 are wanted (debug capture). */
@@ -279,6 +280,14 @@ int sub_set_attention_mask(void* handle, const void* attn_mask, const char* layo
  * forward call where they were made from the same addresses.  A caller whose tensors may have come and gone at those
  * addresses since (saved tensors that are dropped and restored, say) calls this first: the copies are made again. */
 int sub_forget_staged(void* handle);
+/* encoder_backward works out from its options and from the tensors it is handed, which it takes to lie where its forward
+ * call found them, whether that call ran attention with the scores in registers and lin1 with the activation in its
+ * epilogue: both want 16-byte aligned tensors.  A caller whose tensors may lie elsewhere by then (saved tensors that are
+ * dropped and restored, say) asks for the number *form behind the forward call and says it in front of the backward call
+ * that belongs to it; it holds for that one call.  Tensors that the forward call found 16-byte aligned must be so again
+ * where attention ran in registers (the call fails otherwise). */
+int sub_forward_form(void* handle, int* form);
+int sub_set_forward_form(void* handle, int form);
 /* SUB_OPT_OPAQUE_INTERMEDIATES (default 0; the Python module sets it): the caller hands the intermediates from
  * encoder_forward to encoder_backward and looks into none of them.  Option 9 then also covers DROP2MASK where the
  * activation's dropout runs as an operator of its own and its mask is kept (bits in the first B*J*U/8 bytes, feed-forward

@@ -245,6 +245,8 @@ struct Handle {
     // null: the unused SB1_LINW1 buffer of that call.  The backward call reads its gate from there when it
     // is handed the same buffer, and from DROP2 itself otherwise.
     const void* gate_bits_at = nullptr;
+    int form = 0;                     // what the last forward call left (FORM_*); see sub_forward_form
+    int form_given = -1;              // the same of the forward call that the next backward call belongs to, if it was said
     std::vector<ProfEntry> prof;
     size_t prof_used = 0;
     size_t prof_forward = 0;          // entries of the last forward call, kept by the backward call after it
@@ -803,9 +805,9 @@ bool act_epilogues(const Handle& h) {
 bool gelu_epilogues(const Handle& h) {
     return act_epilogues(h) && h.act == ACT_GELU && h.gemm[G_DXLIN2_BDRLB].ok && h.lf[LIN1].str() == "BJU";
 }
-// What the forward call adds to that from the tensors it is handed.  The backward call is handed the same ones and
-// asks the same question: it knows from the handle's options and these pointers alone whether the keep bits of
-// the forward call it belongs to lie in SB1_LINW1 (whichever forward call of the handle that was).
+// What the forward call adds to that from the tensors it is handed.  A backward call that was not told the form of its
+// forward call is taken to be handed the same ones and asks the same question: it then knows from the handle's options and
+// these pointers alone whether the keep bits lie in SB1_LINW1 (whichever forward call of the handle that was).
 bool lin1_takes_gelu_epilogue(const Handle& h, void* const* W, void* const* F) {
     return gelu_epilogues(h) && aligned16(F[LIN1]) && F[SB1_LINW1] && ((uintptr_t)F[SB1_LINW1] & 3) == 0 &&
            aligned16(W[LINB1]) && aligned16(F[DROP2]) && aligned16(F[SB1]) && aligned16(W[LINW1]);
@@ -1027,6 +1029,9 @@ void op_bei(Handle& h, const void* a, const Layout& la, const void* b, const Lay
 // ---------------------------------------------------------------------------
 // The two operator sequences
 // ---------------------------------------------------------------------------
+// What a forward call has left for its backward call where that depends on the tensors it was handed.
+enum { FORM_BITS = 1,            // bits of lin1's epilogue (ReLU: gate, GELU: keep) in SB1_LINW1
+       FORM_REGISTERS = 2 };     // statistics and keep bits of the attention in registers, no score-sized tensors
 struct FwdPtrs {
     void* X; void* W[SUB_N_PARAMS]; void* F[SUB_N_FWD]; void* Y;
 };
@@ -1120,6 +1125,7 @@ void forward(Handle& h, const FwdPtrs& t0) {
     // (registers: the backward pass runs its attention in registers and reads what this pass leaves for it)
     const bool registers = attention_fused(h, F, at);
     const bool fused_attention = registers && !forward_in_operators(h);
+    h.form = registers ? FORM_REGISTERS : 0;
     if (h.fuse_epilogues && h.gemm[G_QKV_BIAS].ok && aligned16(W[BKQV]) && aligned16(F[KKQQVV])) {
         // projection + bias in one pass; WKKWQQWVV (the pre-bias copy) is not written.  The CUs its tiles
         // leave idle draw part of the attention's dropout bits, which depend on nothing but the seed.
@@ -1193,6 +1199,7 @@ void forward(Handle& h, const FwdPtrs& t0) {
         if (keep_job.blocks) ep.keep_words = keep_job.out;
         if (F[SB1_LINW1] && ((uintptr_t)F[SB1_LINW1] & 3) == 0) ep.gate_bits_out = (uint32_t*)F[SB1_LINW1];
         h.gate_bits_at = ep.gate_bits_out;
+        if (ep.gate_bits_out) h.form |= FORM_BITS;
         if (lin1_gelu) { ep.act = ACT_GELU; ep.pre_out = (half_t*)F[LIN1]; }
         launch_gemm(p.shape, (const half_t*)F[SB1], (const half_t*)W[LINW1], (half_t*)F[DROP2], p.alpha, ep, h.stream);
     } else {
@@ -1228,9 +1235,17 @@ void forward(Handle& h, const FwdPtrs& t0) {
 
 void backward(Handle& h, const BwdPtrs& t0) {
     if (!h.configured) fail("encoder_backward: handle is not configured");
+    const int form = h.form_given;
+    h.form_given = -1;
     // the first backward call after a forward call keeps that call's entries in front of its own
     h.prof_used = h.prof_forward;
     h.prof_forward = 0;
+    AttnArgs at;
+    bool attn_fused = attention_fused(h, t0.F, at);
+    if (form >= 0 && !attn_fused && (form & FORM_REGISTERS))
+        fail("encoder_backward: the forward call ran attention with the scores in registers, and what it left for the backward "
+             "call is not 16-byte aligned any more (or an option has changed since)");
+    attn_fused = attn_fused && (form < 0 || (form & FORM_REGISTERS));
     BwdPtrs t = t0;
     if (h.staging) {
         const void* xs = nullptr;
@@ -1298,13 +1313,13 @@ void backward(Handle& h, const BwdPtrs& t0) {
                      F[DROP3MASK], h.lf[DROP3MASK], D[DRESID2], h.lb[DRESID2], D[DLIN2], h.lb[DLIN2], packed_masks(h));
         }
     }
-    const bool bits_here = h.gate_bits_at && h.gate_bits_at == F[SB1_LINW1] &&
+    const bool bits_here = (form < 0 ? h.gate_bits_at && h.gate_bits_at == F[SB1_LINW1] : (form & FORM_BITS) != 0) &&
                            h.gemm[G_LIN1_BAD].shape.M == h.gemm[G_DXLIN2_BDRLB].shape.M &&
                            h.gemm[G_LIN1_BAD].shape.N == h.gemm[G_DXLIN2_BDRLB].shape.N;
-    const bool bdrlb_gelu = lin1_takes_gelu_epilogue(h, W, F);       // the forward call's own test: its keep bits lie in SB1_LINW1
+    const bool bdrlb_gelu = h.act == ACT_GELU && (form < 0 ? lin1_takes_gelu_epilogue(h, W, F) : (form & FORM_BITS) != 0);
     const bool fuse_bdrlb = ((relu_from_output(h) && h.fuse_epilogues && h.gemm[G_DXLIN2_BDRLB].ok && (h.opaque || h.act_whole) &&
                               aligned16(F[DROP2])) ||
-                             bdrlb_gelu) &&
+                             (bdrlb_gelu && aligned16(F[LIN1]) && ((uintptr_t)F[SB1_LINW1] & 3) == 0)) &&
                             aligned16(D[DLIN1]) && aligned16(D[DLIN2]) && aligned16(W[LINW2]);
     if (fuse_bdrlb) {
         // product, gate and the column sums of the result in one launch: DDROP2 is not produced
@@ -1312,7 +1327,7 @@ void backward(Handle& h, const BwdPtrs& t0) {
         const GemmPlan& p = h.gemm[G_DXLIN2_BDRLB];
         GemmEpilogue ep;
         ep.gate = (const half_t*)(bdrlb_gelu ? F[LIN1] : F[DROP2]); ep.sbM = p.sM; ep.sbN = p.sN; ep.colsum = (float*)16;
-        if (bits_here || bdrlb_gelu) ep.gate_bits = (const uint32_t*)F[SB1_LINW1];
+        if ((bits_here && ((uintptr_t)F[SB1_LINW1] & 3) == 0) || bdrlb_gelu) ep.gate_bits = (const uint32_t*)F[SB1_LINW1];
         if (bdrlb_gelu) ep.act = ACT_GELU;
         const int ntc = gemm_colsum_rows(p.shape, D[DLIN2], W[LINW2], D[DLIN1], ep), U = (int)p.shape.N;
         float* ws = ep.colsum = take_ws(h, (size_t)ntc * U);
@@ -1376,8 +1391,6 @@ void backward(Handle& h, const BwdPtrs& t0) {
             op_baob(h, D[DATT], h.lb[DATT], DW[BO]);
         }
     }
-    AttnArgs at;
-    const bool attn_fused = attention_fused(h, F, at);
     const bool fuse_dx = h.fuse_epilogues && h.gemm[G_DXQKV_RESID].ok && aligned16(D[DRESID1]) &&
                          aligned16(t.DX);
     // dWout (64 tiles of 128 x 128 at the bench workload, too few for a launch of its
@@ -1698,6 +1711,17 @@ int sub_set_option(void* handle, int option, int value) {
         }
         else fail("sub_set_option: unknown option");
     });
+}
+
+int sub_forward_form(void* handle, int* form) {
+    return guarded([&] {
+        if (!form) fail("sub_forward_form: null result pointer");
+        *form = as_handle(handle).form;
+    });
+}
+
+int sub_set_forward_form(void* handle, int form) {
+    return guarded([&] { as_handle(handle).form_given = form < 0 ? -1 : form; });
 }
 
 int sub_tensor_layout(void* handle, const char* name, char out[16]) {

@@ -36,6 +36,8 @@ struct Lib {
     decltype(&sub_set_attention_mask) set_attention_mask = nullptr;
     decltype(&sub_set_rng_counter) set_rng_counter = nullptr;
     decltype(&sub_forget_staged) forget_staged = nullptr;
+    decltype(&sub_forward_form) forward_form = nullptr;
+    decltype(&sub_set_forward_form) set_forward_form = nullptr;
     decltype(&sub_encoder_forward) encoder_forward = nullptr;
     decltype(&sub_encoder_backward) encoder_backward = nullptr;
 } lib;
@@ -55,6 +57,8 @@ void load(const std::string& path, py::object error) {
     get(lib.set_attention_mask, "sub_set_attention_mask");
     get(lib.set_rng_counter, "sub_set_rng_counter");
     get(lib.forget_staged, "sub_forget_staged");
+    get(lib.forward_form, "sub_forward_form");
+    get(lib.set_forward_form, "sub_set_forward_form");
     get(lib.encoder_forward, "sub_encoder_forward");
     get(lib.encoder_backward, "sub_encoder_backward");
     g_error = error.release().ptr();
@@ -115,6 +119,15 @@ bool plain(const at::Tensor& X, const std::vector<at::Tensor>& params) {
         return false;
     auto odd = [](const at::Tensor& t) { return has_tangent(t) || t.key_set().has(c10::DispatchKey::Python); };
     return !odd(X) && std::none_of(params.begin(), params.end(), odd);
+}
+
+// A saved tensor as the backward pass needs it: dense, and 16-byte aligned where the forward pass found it so.  (A hook may
+// restore it as a slice of a larger buffer, or with other strides.)
+bool misaligned(const at::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) & 15; }
+at::Tensor as_saved(at::Tensor t, bool was_misaligned) {
+    at::NoGradGuard no_grad;
+    t = t.contiguous();
+    return misaligned(t) && !was_misaligned ? t.clone() : t;
 }
 
 // An additive attention mask and the order of its dims.
@@ -191,9 +204,16 @@ struct EncoderLayer : std::enable_shared_from_this<EncoderLayer> {
     }
     // Only the pass right behind its forward pass (number `forward` of them all) can know the handle's staged copies by the
     // addresses they were made from: hooks may have dropped and restored the saved tensors, at addresses of others' by now.
-    void begin_backward(uint64_t forward) {
+    void begin_backward(uint64_t forward, int form) {
         if (passes != forward) check(lib.forget_staged(handle), "sub_forget_staged");
+        check(lib.set_forward_form(handle, form), "sub_set_forward_form");
         ++passes;
+    }
+    // What the forward pass that has just run left (see sub_forward_form).
+    int form() const {
+        int v = 0;
+        check(lib.forward_form(handle, &v), "sub_forward_form");
+        return v;
     }
     void keep(std::vector<at::Tensor>& list, const char* which, const at::Tensor& X) {
         if (list.empty() || list[0].device() != X.device()) list = workspace(which, X).cast<std::vector<at::Tensor>>();
@@ -218,7 +238,14 @@ struct EncoderBackward : Node {
     // the parameters as the forward pass read them, X, and the forward intermediates (those of a layer that keeps its own
     // too: what hooks on saved tensors see does not depend on who holds the memory)
     std::vector<SavedVariable> saved;
+    std::vector<bool> misaligned;        // of those
+    int form = 0;                        // what the forward pass left (sub_forward_form)
     uint64_t generation = 0, pass = 0;
+
+    void save(const at::Tensor& t) {
+        saved.emplace_back(t, false);
+        misaligned.push_back(::misaligned(t));
+    }
 
     std::string name() const override { return "EncoderFunctionBackward"; }
     void release_variables() override {
@@ -233,7 +260,7 @@ struct EncoderBackward : Node {
         l.check_relu_gate();
         variable_list in;
         in.reserve(saved.size());
-        for (auto& s : saved) in.push_back(s.unpack());
+        for (size_t i = 0; i < saved.size(); ++i) in.push_back(as_saved(saved[i].unpack(), misaligned[i]));
         const size_t np = l.param_shapes.size();
         const at::Tensor& X = in[np];
         const c10::DeviceGuard guard(X.device());
@@ -261,7 +288,7 @@ struct EncoderBackward : Node {
         p.push_back(out[0].data_ptr());
         use_current_stream(l.handle, X.device().index());
         const MaskScope own(l, mask);
-        l.begin_backward(pass);
+        l.begin_backward(pass, form);
         check(lib.encoder_backward(l.handle, p.data(), (int)p.size()), "encoder_backward");
         return out;
     }
@@ -320,9 +347,10 @@ std::optional<at::Tensor> EncoderLayer::forward(const at::Tensor& X_, const std:
         node->mask = mask;
         const std::vector<at::Tensor>& held = persistent ? kept_fwd : interm;
         node->saved.reserve(w.size() + 1 + held.size());
-        for (const auto& t : w) node->saved.emplace_back(t, false);
-        node->saved.emplace_back(X, false);
-        for (const auto& t : held) node->saved.emplace_back(t, false);
+        for (const auto& t : w) node->save(t);
+        node->save(X);
+        for (const auto& t : held) node->save(t);
+        node->form = form();
         node->generation = generation;
         node->pass = passes;
         torch::autograd::set_history(Y, node);
@@ -341,6 +369,7 @@ PYBIND11_MODULE(_host, m) {
         .def_readwrite("generation", &EncoderLayer::generation)
         .def_readwrite("passes", &EncoderLayer::passes)
         .def("begin_backward", &EncoderLayer::begin_backward)
+        .def("form", &EncoderLayer::form)
         .def("check_compact", &EncoderLayer::check_compact)
         .def("check_relu_gate", &EncoderLayer::check_relu_gate)
         .def("set_attention_mask", &EncoderLayer::set_attention_mask)

@@ -40,6 +40,9 @@ def _python_function(weak, layer, in_shape, out_shape, shapes, workspace):
         if module.enable_debug:
             torch.cuda.synchronize()
 
+    def misaligned(t):
+        return t.data_ptr() % 16 != 0
+
     def tensors(module, key, like):
         if module.persistent_workspace:
             return workspace(key, like)
@@ -65,7 +68,9 @@ def _python_function(weak, layer, in_shape, out_shape, shapes, workspace):
             ctx.mask = layer.mask
             weights = [t.contiguous() for t in weights]
             call(module, 'encoder_forward', X.device, [X, *weights, *interm, Y])
+            ctx.form = layer.form()
             ctx.save_for_backward(*weights, *interm, X)
+            ctx.misaligned = [misaligned(t) for t in (*weights, *interm, X)]
             if module.enable_debug:
                 for (name, _), t in zip(list(layouts['forward_interm']) + list(layouts['params']), interm + weights):
                     module.debug[name] = t.detach().cpu().numpy()
@@ -81,11 +86,14 @@ def _python_function(weak, layer, in_shape, out_shape, shapes, workspace):
             DY = DY.contiguous()
             DX = torch.empty(in_shape, device=DY.device, dtype=DY.dtype)
             interm = tensors(module, 'backward_interm', DY)
-            grads = [torch.empty_like(t) for t in ctx.saved_tensors[:len(layouts['params'])]]
+            # dense, and 16-byte aligned where the forward pass found them so, whatever hooks have restored
+            saved = [t.contiguous() for t in ctx.saved_tensors]
+            saved = [t.clone() if misaligned(t) and not was else t for t, was in zip(saved, ctx.misaligned)]
+            grads = [torch.empty_like(t) for t in saved[:len(layouts['params'])]]
             now, layer.mask = layer.mask, ctx.mask
             try:
-                layer.begin_backward(ctx.pass_number)
-                call(module, 'encoder_backward', DY.device, [DY, *grads, *interm, *ctx.saved_tensors, DX])
+                layer.begin_backward(ctx.pass_number, ctx.form)
+                call(module, 'encoder_backward', DY.device, [DY, *grads, *interm, *saved, DX])
             finally:
                 layer.mask = now
             if module.enable_debug:

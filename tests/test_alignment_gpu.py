@@ -40,7 +40,7 @@ def _pass(enc, x, dy, call=None, hooks=None):
     return dict([('SB2', y.detach()), ('DX', x.grad)] + [('D' + n, q.grad) for n, q in enc.named_parameters()])
 
 
-def _c_pass(enc, x, dy, odd):
+def _c_pass(enc, x, dy, odd, between=lambda: None):
     """Both passes as a C caller makes them, with the named buffers (parameters, intermediates, 'D' + parameter) at odd
     addresses; intermediates start as NaN."""
     handle, lay = enc._handle, enc.layouts
@@ -58,6 +58,7 @@ def _c_pass(enc, x, dy, odd):
     y, dx = torch.empty_like(dy), torch.empty_like(x)
     enc.set_rng(SEED, 0)
     call('forward', [x, *params, *fwd, y])
+    between()
     call('backward', [dy, *grads, *bwd, *params, *fwd, x, dx])
     return dict([('SB2', y), ('DX', dx)] + [('D' + n, t) for (n, _), t in zip(lay['params'], grads)])
 
@@ -98,3 +99,56 @@ def test_decoder_layer_whose_second_feed_forward_weight_is_misaligned():
         y.backward(dy)
         got.append(dict([('y', y.detach())] + [(n, q.grad) for n, q in layer.named_parameters()]))
     _close(got[1], got[0])
+
+
+@pytest.mark.parametrize('act', ['relu', 'gelu'])
+@pytest.mark.parametrize('python', [False, True])
+@pytest.mark.parametrize('persistent', [False, True])
+@pytest.mark.parametrize('what', ['LINW1', 'all', 'strided'])
+def test_saved_tensors_that_hooks_restore_elsewhere(act, python, persistent, what):
+    """Restored to addresses that are no multiple of 16, or with other strides: the backward pass takes what its forward pass
+    left for it, bit for bit as without hooks (at 2 x 128 x 768 the two passes run with activation epilogues)."""
+    enc, x, dy = _encoder((2, 128, 12, 768), act, persistent_workspace=persistent)
+    call = (lambda t: enc.encoder_func.apply(t, *enc.params)) if python else enc
+    want = {n: t.clone() for n, t in _pass(enc, x, dy, call).items()}
+
+    def restore(t):
+        if what == 'strided':
+            return t.t().contiguous().t() if t.dim() == 2 else t
+        return _odd(t) if what == 'all' or t.shape == enc.LINW1.shape else t
+    got = _pass(enc, x, dy, call, torch.autograd.graph.saved_tensors_hooks(lambda t: t, restore))
+    for n, t in want.items():
+        assert torch.equal(got[n], t), n
+
+
+@pytest.mark.parametrize('act', ['relu', 'gelu'])
+@pytest.mark.parametrize('python', [False, True])
+def test_saved_tensors_restored_aligned_that_were_not(act, python):
+    """The other way round: the forward pass finds LINW1 misaligned and runs bias, activation and dropout as an operator; a
+    hook restores it aligned."""
+    enc, x, dy = _encoder((2, 128, 12, 768), act)
+    call = (lambda t: enc.encoder_func.apply(t, *enc.params)) if python else enc
+    enc.LINW1.data = _odd(enc.LINW1.data)
+    assert enc.LINW1.data_ptr() % 16
+    want = _pass(enc, x, dy, call)
+    _close(_pass(enc, x, dy, call, torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t.clone())), want)
+
+
+def test_backward_call_that_cannot_take_what_its_forward_call_left_refuses():
+    """A C caller says what its forward call left; without attention in registers (switched off in between, which is also
+    what a tensor at an odd address does) there is no backward pass for that, and none is begun."""
+    from substation_amd import _lib
+    enc, x, dy = _encoder((2, 128, 2, 128), 'gelu')
+    form = ctypes.c_int(-1)
+
+    def say():
+        _lib.check(enc._handle.lib.sub_forward_form(enc._handle.ptr, ctypes.byref(form)))
+        _lib.check(enc._handle.lib.sub_set_forward_form(enc._handle.ptr, form))
+    want = _c_pass(enc, x.detach(), dy, ())
+    got = _c_pass(enc, x.detach(), dy, (), say)
+    assert form.value > 0
+    with pytest.raises(_lib.SubstationError):
+        _c_pass(enc, x.detach(), dy, (), lambda: (say(), enc._handle.set_option(4, 0)))
+    _c_pass(enc, x.detach(), dy, ())              # said for that one call only
+    for n, t in want.items():
+        assert torch.equal(got[n], t), n
