@@ -204,6 +204,7 @@ struct Handle {
     half_t* sX = nullptr; half_t* sY = nullptr; half_t* sDY = nullptr; half_t* sDX = nullptr;
     half_t* sW[SUB_N_PARAMS] = {}; half_t* sDW[SUB_N_PARAMS] = {};
     half_t* staged_fwd = nullptr; half_t* staged_bwd = nullptr;      // the allocations that sX, sY, sW and sDX, sDY, sDW lie in
+    half_t* staged_lin[2][2] = {};    // copies of LINW1, LINW2 and of their gradients where the caller's are misaligned
     // what sX / sW were last made from (a backward call reuses them for the same pointers; see sub_forget_staged)
     const void* staged_x_from = nullptr; const void* staged_w_from[SUB_N_PARAMS] = {};
     int pos_p[SUB_N_PARAMS], pos_f[SUB_N_FWD], pos_b[SUB_N_BWD];   // internal id -> caller position
@@ -261,7 +262,8 @@ struct Handle {
         if (gws) (void)hipFree(gws);
         if (mask_plan) (void)hipFree(mask_plan);
         if (clock_buf) (void)hipFree(clock_buf);
-        for (half_t* q : {staged_fwd, staged_bwd}) if (q) (void)hipFree(q);
+        for (half_t* q : {staged_fwd, staged_bwd, staged_lin[0][0], staged_lin[0][1], staged_lin[1][0], staged_lin[1][1]})
+            if (q) (void)hipFree(q);
         for (auto& e : prof) (void)hipEventDestroy(e.a);
         if (swapped) (void)hipThreadExchangeStreamCaptureMode(&mode);
     }
@@ -454,7 +456,7 @@ void configure(Handle& h, const sub_config* c) {
 // feature dim contiguous; the reference's shipped configurations are feature-major -- every intermediate
 // lives in the library's own order inside the caller's buffer (same number of elements), and the tensors that
 // cross the boundary (input, output, their gradients, weights, weight gradients) are copied into that order and
-// back by k_relayout, all but LINW1, LINW2 and their gradients (16 of 25 MB of weights at E 1024; copied, the
+// back by k_relayout, all but aligned LINW1, LINW2 and their gradients (16 of 25 MB of weights at E 1024; copied, the
 // relayout launches took 46 us of a pass at 8 x 512, now 35, and the layer 0.528 -> 0.516 ms).  A configuration whose activations are all in the library's orders runs as it is, with
 // its own weight orders.
 void plan_layouts(Handle& h, bool own) {
@@ -1070,11 +1072,31 @@ void allocate_staged(Handle& h, bool backward) {
 }
 
 void drop_staged(Handle& h) {
-    if (!h.staged_fwd && !h.staged_bwd) return;
-    refuse_capture(h, "sub_configure");
-    for (half_t** q : {&h.staged_fwd, &h.staged_bwd}) if (*q) { hip_check(hipFree(*q), "hipFree(staged tensors)"); *q = nullptr; }
+    half_t** const all[] = {&h.staged_fwd, &h.staged_bwd, &h.staged_lin[0][0], &h.staged_lin[0][1], &h.staged_lin[1][0], &h.staged_lin[1][1]};
+    for (half_t** q : all) {
+        if (!*q) continue;
+        refuse_capture(h, "sub_configure");
+        hip_check(hipFree(*q), "hipFree(staged tensors)");
+        *q = nullptr;
+    }
     h.sX = h.sY = h.sDX = h.sDY = nullptr;
     for (int i = 0; i < SUB_N_PARAMS; ++i) h.sW[i] = h.sDW[i] = nullptr;
+}
+
+// Is parameter i (or its gradient), at p, read and written by way of a copy?  LINW1 and LINW2 are at addresses that are no
+// multiple of 16: their products would go to the scalar kernel (forward and backward at 8 x 512, E 1024: 4520 us, this way 577;
+// aligned 548).
+bool staged_param(const Handle& h, int i, const void* p) {
+    return h.stage_p[i] || (h.staging && (i == LINW1 || i == LINW2) && !aligned16(p));
+}
+half_t* staged_copy(Handle& h, int i, bool gradient) {
+    if (h.stage_p[i]) return gradient ? h.sDW[i] : h.sW[i];
+    half_t*& q = h.staged_lin[gradient][i == LINW2];
+    if (!q) {
+        refuse_capture(h, "hipMalloc(staged weight)");
+        hip_check(hipMalloc((void**)&q, (size_t)h.lp[i].numel * sizeof(half_t)), "hipMalloc(staged weight)");
+    }
+    return q;
 }
 
 // The input and the weights in the library's orders: copied when `fresh`, or when the copies at hand were made
@@ -1083,7 +1105,7 @@ void stage_inputs(Handle& h, const void* X, void* const* W, const void*& Xs, voi
     Xs = X;
     for (int i = 0; i < SUB_N_PARAMS; ++i) Ws[i] = W[i];
     bool any = h.stage_x;
-    for (int i = 0; i < SUB_N_PARAMS; ++i) any = any || h.stage_p[i];
+    for (int i = 0; i < SUB_N_PARAMS; ++i) any = any || staged_param(h, i, W[i]);
     if (!any) return;
     allocate_staged(h, false);
     ProfScope ps(h, name);
@@ -1097,10 +1119,11 @@ void stage_inputs(Handle& h, const void* X, void* const* W, const void*& Xs, voi
         }
     }
     for (int i = 0; i < SUB_N_PARAMS; ++i) {
-        if (!h.stage_p[i]) continue;
-        Ws[i] = h.sW[i];
+        if (!staged_param(h, i, W[i])) continue;
+        half_t* const copy = staged_copy(h, i, false);
+        Ws[i] = copy;
         if (fresh || h.staged_w_from[i] != W[i]) {
-            jobs[n++] = RelayoutJob{h.xp[i], h.lp[i], (const half_t*)W[i], h.sW[i]};
+            jobs[n++] = RelayoutJob{h.xp[i], h.lp[i], (const half_t*)W[i], copy};
             h.staged_w_from[i] = W[i];
         }
     }
@@ -1259,7 +1282,7 @@ void backward(Handle& h, const BwdPtrs& t0) {
         }
         if (h.stage_x) t.DX = h.sDX;
         for (int i = 0; i < SUB_N_PARAMS; ++i)
-            if (h.stage_p[i]) t.DW[i] = h.sDW[i];
+            if (staged_param(h, i, t0.DW[i])) t.DW[i] = staged_copy(h, i, true);
     }
     // The five bias / scale gradients are only consumed by the caller: their
     // reductions leave fp32 partials in separate scratch regions and one launch
@@ -1498,14 +1521,14 @@ void backward(Handle& h, const BwdPtrs& t0) {
     }
     if (h.staging) {
         bool any = h.stage_x;
-        for (int i = 0; i < SUB_N_PARAMS; ++i) any = any || h.stage_p[i];
+        for (int i = 0; i < SUB_N_PARAMS; ++i) any = any || staged_param(h, i, t0.DW[i]);
         if (any) {
             ProfScope ps(h, "relayout-out-bwd");
             RelayoutJob jobs[1 + SUB_N_PARAMS];
             int n = 0;
             if (h.stage_x) jobs[n++] = RelayoutJob{h.lX, h.xX, (const half_t*)t.DX, (half_t*)t0.DX};
             for (int i = 0; i < SUB_N_PARAMS; ++i)
-                if (h.stage_p[i]) jobs[n++] = RelayoutJob{h.lp[i], h.xp[i], (const half_t*)t.DW[i], (half_t*)t0.DW[i]};
+                if (staged_param(h, i, t0.DW[i])) jobs[n++] = RelayoutJob{h.lp[i], h.xp[i], (const half_t*)t.DW[i], (half_t*)t0.DW[i]};
             launch_relayout_batch(jobs, n, h.stream);
         }
     }

@@ -152,3 +152,24 @@ def test_backward_call_that_cannot_take_what_its_forward_call_left_refuses():
     _c_pass(enc, x.detach(), dy, ())              # said for that one call only
     for n, t in want.items():
         assert torch.equal(got[n], t), n
+
+
+@pytest.mark.parametrize('odd', [('LINW1',), ('LINW2',), ('LINW1', 'LINW2', 'DLINW1', 'DLINW2')])
+@pytest.mark.parametrize('act', ['relu', 'gelu'])
+def test_misaligned_feed_forward_weights_of_feature_major_layouts(odd, act):
+    """Under a configuration that the layer runs in its own orders, LINW1 and LINW2 are read and written as they lie; where
+    they lie misaligned, by way of copies, like the other weights: the launches and the bits are those of aligned ones."""
+    enc, x, dy = _encoder((2, 128, 12, 768), act, 'bert-b8-l512-h16-e1024')
+    enc._handle.profile_enable(True)
+    want = _c_pass(enc, x.detach(), dy, ())
+    launches = [n for n, _ in enc._handle.profile_read()]
+    got = _c_pass(enc, x.detach(), dy, odd)
+    assert [n for n, _ in enc._handle.profile_read()] == launches and 'lin1+bad' in launches and 'dXlin2+bdrlb' in launches
+    for n, t in want.items():
+        assert torch.equal(got[n], t), n
+    # and with saved tensors and other addresses in every pass
+    for n in ('LINW1', 'LINW2'):
+        if n in odd:
+            getattr(enc, n).data = _odd(getattr(enc, n).data)
+    for n, t in _pass(enc, x, dy).items():
+        assert torch.equal(want[n], t), n
