@@ -240,7 +240,8 @@ struct Handle {
                                       // bit 1: workgroups behind the first LayerNorm launch draw lin1's keep bits
     bool packed_masks = true;         // DROP1MASK and DROP3MASK travel as one bit per element inside their buffers
     bool skip_unread = true;          // intermediates that neither pass reads are not written (ATT after its bias, LIN2, DLN2, DLN1)
-    bool act_whole = false;           // the feed-forward block's outputs are whole 256 x 256 tiles, and enough of them
+    // lin1's (dXlin2's) outputs are whole 256 x 256 tiles, and enough of them: see whole_round
+    bool lin1_whole = false, dxlin2_whole = false;
     bool opaque = false;              // nobody looks into DROP2MASK (bits as well), ATT and DROP2_LINW2 (left alone as well)
     // where the last forward call's lin1 epilogue left one bit per element of DROP2 (set = positive), or
     // null: the unused SB1_LINW1 buffer of that call.  The backward call reads its gate from there when it
@@ -450,6 +451,14 @@ void configure(Handle& h, const sub_config* c) {
     h.configured = true;
 }
 
+// Whole 256 x 256 tiles that fill their rounds of 256: to 0.7 where both operands lie along k, else to 0.9.  At these sizes the
+// activation runs in the product's epilogue also where a caller may look into the intermediates (lin1 with bias, ReLU and
+// dropout at 3072 x 4096 x 1024, three quarters of a round: 42 us, in two launches 32 + 15).
+bool whole_round(const GemmShape& s) {
+    const long tiles = (s.M / 256) * (s.N / 256), rounds = (tiles + 255) / 256;
+    return s.M % 256 == 0 && s.N % 256 == 0 && s.K1 % 64 == 0 && tiles * 10 >= rounds * 256 * (s.sAK1 == 1 && s.sBK1 == 1 ? 7 : 9);
+}
+
 // The dimension orders the launches run in, and everything that follows from them (contraction plans,
 // scratch sizes).  own = false: the caller's.  own = true (SUB_OPT_PRIVATE_LAYOUTS): when an activation of the
 // caller's configuration is not in the order the fused paths of this library need -- token-major rows with the
@@ -563,11 +572,8 @@ void plan_layouts(Handle& h, bool own) {
         p.ok = p.sb[0] == 0 && gemm_relu_dropout_ok(p.shape, (const void*)16, (const void*)16, (const void*)16, ep);
     }
 
-    {
-        const GemmShape& s = h.gemm[G_LIN1_BAD].shape;
-        const long tiles = (s.M / 256) * (s.N / 256);
-        h.act_whole = s.M % 256 == 0 && s.N % 256 == 0 && s.K1 % 64 == 0 && tiles * 10 >= (tiles + 255) / 256 * 256 * 9;
-    }
+    h.lin1_whole = whole_round(h.gemm[G_LIN1_BAD].shape);
+    h.dxlin2_whole = whole_round(h.gemm[G_DXLIN2_BDRLB].shape);
     {   // scratch of the five column reductions of one backward pass, side by side
         Space si = make_space(sz, {dB, dJ}, dI), su = make_space(sz, {dB, dJ}, dU);
         Space sq = make_space(sz, {dQ, dH, dB, dJ}, dP);
@@ -801,11 +807,11 @@ bool relu_from_output(const Handle& h) { return h.relu_from_output && h.act == A
 // SB1_LINW1 buffer, a byte per pack in canonical order, instead of a DROP2MASK tensor) and the backward of that in
 // dXlin2's epilogue, or, where that finds a tensor misaligned, in the operator of its own on those bits.
 bool act_epilogues(const Handle& h) {
-    // (at the sizes where the products have always done it, also where somebody looks into the intermediates)
-    return h.relu_from_output && h.fuse_epilogues && h.gemm[G_LIN1_BAD].ok && (h.opaque || h.act_whole);
+    return h.relu_from_output && h.fuse_epilogues && h.gemm[G_LIN1_BAD].ok && (h.opaque || h.lin1_whole);
 }
 bool gelu_epilogues(const Handle& h) {
-    return act_epilogues(h) && h.act == ACT_GELU && h.gemm[G_DXLIN2_BDRLB].ok && h.lf[LIN1].str() == "BJU";
+    return act_epilogues(h) && h.act == ACT_GELU && h.gemm[G_DXLIN2_BDRLB].ok && (h.opaque || h.dxlin2_whole) &&
+           h.lf[LIN1].str() == "BJU";
 }
 // What the forward call adds to that from the tensors it is handed.  A backward call that was not told the form of its
 // forward call is taken to be handed the same ones and asks the same question: it then knows from the handle's options and
@@ -1340,7 +1346,7 @@ void backward(Handle& h, const BwdPtrs& t0) {
                            h.gemm[G_LIN1_BAD].shape.M == h.gemm[G_DXLIN2_BDRLB].shape.M &&
                            h.gemm[G_LIN1_BAD].shape.N == h.gemm[G_DXLIN2_BDRLB].shape.N;
     const bool bdrlb_gelu = h.act == ACT_GELU && (form < 0 ? lin1_takes_gelu_epilogue(h, W, F) : (form & FORM_BITS) != 0);
-    const bool fuse_bdrlb = ((relu_from_output(h) && h.fuse_epilogues && h.gemm[G_DXLIN2_BDRLB].ok && (h.opaque || h.act_whole) &&
+    const bool fuse_bdrlb = ((relu_from_output(h) && h.fuse_epilogues && h.gemm[G_DXLIN2_BDRLB].ok && (h.opaque || h.dxlin2_whole) &&
                               aligned16(F[DROP2])) ||
                              (bdrlb_gelu && aligned16(F[LIN1]) && ((uintptr_t)F[SB1_LINW1] & 3) == 0)) &&
                             aligned16(D[DLIN1]) && aligned16(D[DLIN2]) && aligned16(W[LINW2]);

@@ -1359,3 +1359,18 @@ def test_activation_epilogues_on_tiles_of_every_size_equal_the_operators(dims, a
             assert_close(b.float().cpu().numpy(), a.float().cpu().numpy(), tol=2e-3, name=name)
         else:
             assert torch.equal(a, b), name
+
+
+@pytest.mark.parametrize('batch,act,fused', [(4, 'relu', ()), (6, 'relu', ('lin1+bad',)), (6, 'gelu', ()),
+                                             (8, 'relu', ('lin1+bad', 'dXlin2+bdrlb')), (8, 'gelu', ('lin1+bad', 'dXlin2+bdrlb'))])
+def test_activation_epilogues_where_a_caller_may_look_into_the_intermediates(batch, act, fused):
+    """Without option 12 (a C caller's default): from 0.7 of a round of 256 x 256 tiles on where both operands lie along k
+    (lin1 in the default orders), from 0.9 on elsewhere (dXlin2).  Batches of 4, 6 and 8 have 128, 192 and 256 tiles."""
+    from substation_amd import Encoder, layouts as L
+    enc = Encoder('unused', batch, 512, 16, 1024, L.mi355x_layouts(), torch.float16, 0.1, 0.1, 0.1, 0.1, activation=act,
+                  seed=SEED, profiling=True).cuda()
+    enc._handle.set_option(12, 0)
+    x = torch.randn(batch, 512, 1024).half().cuda().requires_grad_()
+    enc(x).backward(torch.ones_like(x))
+    launches = [n for n, _ in enc.profile()]
+    assert tuple(n for n in launches if n in ('lin1+bad', 'dXlin2+bdrlb')) == fused, launches
