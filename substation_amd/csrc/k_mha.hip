@@ -145,10 +145,14 @@ __device__ __forceinline__ constexpr int reg_pos(int v, int hi) { return (v >> 2
 // Straight from the registers 6 of the 35 us of dK and dV at H 16, P 64, 8 x 512 were the stores and 1 the sums (9
 // instructions a value), at 96 x 128 17 and 1 of 48.  This way: 8 x 512: dK and dV 35.3 -> 32.4 us, forward 26.3 -> 25.7;
 // 96 x 128: dK and dV 48.5 -> 38.3, dQ 41.9 -> 38.3, forward 31.5 -> 28.0.
+// (Nothing of the addresses below is to be kept in registers while the tiles are worked on: the lane's index is made anew
+// here, and the callers' wave index is a scalar.  Without that a lane needed 4 to 20 registers more, one wave per SIMD
+// instead of two in the forward kernel of head size 128 at odd lengths: 4 x 1000, H 16, P 128: 104 us, with it 76.6.)
 template <int P, bool RAGGED>
 __device__ __forceinline__ void store_rows(const AttnSide& t, unsigned h, unsigned b, unsigned pos0, unsigned limit, int lane,
                                            const f16v (&acc)[P / 32], float scale, half_t* tile, float* sums) {
     constexpr int PER = P / 8, ROWS = WAVE / PER;      // 16-byte words of a row, rows of an instruction
+    asm volatile("" : "+v"(lane));
     const int l32 = lane & 31, hi = lane >> 5, row = lane / PER, chunk = lane % PER;
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
@@ -541,7 +545,8 @@ __global__ __launch_bounds__(256) void k_mha_fwd(AttnArgs a, PhiloxKey key_) {
         e0 = e1; e1 = e2; e2 = e3;
     }
     const float l_tot = l_run + __shfl_xor(l_run, 32);
-    store_rows<P, RAGGED>(a.o, h, b, qb * QB + wave * 32, a.J, lane, o, 1.0f / l_tot, wave < 2 ? kt[wave] : vt[wave - 2], nullptr);
+    const int w = __builtin_amdgcn_readfirstlane(wave);
+    store_rows<P, RAGGED>(a.o, h, b, qb * QB + w * 32, a.J, lane, o, 1.0f / l_tot, w < 2 ? kt[w] : vt[w - 2], nullptr);
     if (mine_ && hi == 0) a.lse[row] = m_ref * c + __builtin_amdgcn_logf(l_tot);
 }
 
@@ -694,8 +699,9 @@ __global__ __launch_bounds__(256, !MASKED ? (P == 128 ? 2 : 3) : 1) void k_mha_b
         e0 = e1; e1 = e2; e2 = e3;
     }
     float* const sums = a.bias_q ? reinterpret_cast<float*>(kt[2]) : nullptr;       // (of 4 waves 64 * P bytes, a tile's)
-    store_rows<P, RAGGED>(a.dq, h, b, qb * QB + wave * 32, a.J, lane, dq, a.alpha, wave < 2 ? kt[wave] : vt[wave - 2],
-                          sums ? sums + wave * 4 * P : nullptr);
+    const int w = __builtin_amdgcn_readfirstlane(wave);
+    store_rows<P, RAGGED>(a.dq, h, b, qb * QB + w * 32, a.J, lane, dq, a.alpha, w < 2 ? kt[w] : vt[w - 2],
+                          sums ? sums + w * 4 * P : nullptr);
     if (!sums) return;
     __syncthreads();
     if (tid < P) a.bias_q[((size_t)h * (a.B * qblocks) + b * qblocks + qb) * P + tid] = column_sum<P>(sums, tid);
@@ -1020,11 +1026,12 @@ __global__ __launch_bounds__(256, (P == 64 && MASKED) ? 2 : 1) void k_mha_bwd_dk
         e0 = e1; e1 = e2; e2 = e3;
     }
     }
-    half_t* const tile = wave < 2 ? stage[wave].q : stage[wave - 2].d_o;
+    const int w = __builtin_amdgcn_readfirstlane(wave);
+    half_t* const tile = w < 2 ? stage[w].q : stage[w - 2].d_o;
     float* const sums_k = reinterpret_cast<float*>(stage[2].q);         // (of 4 waves 64 * P bytes, a tile's)
     float* const sums_v = reinterpret_cast<float*>(stage[2].d_o);
-    store_rows<P, RAGGED>(a.dk, h, b, kb * QB + wave * 32, a.K, lane, dk, a.alpha, tile, a.bias_kv ? sums_k + wave * 4 * P : nullptr);
-    store_rows<P, RAGGED>(a.dv, h, b, kb * QB + wave * 32, a.K, lane, dv, 1.0f, tile, a.bias_kv ? sums_v + wave * 4 * P : nullptr);
+    store_rows<P, RAGGED>(a.dk, h, b, kb * QB + w * 32, a.K, lane, dk, a.alpha, tile, a.bias_kv ? sums_k + w * 4 * P : nullptr);
+    store_rows<P, RAGGED>(a.dv, h, b, kb * QB + w * 32, a.K, lane, dv, 1.0f, tile, a.bias_kv ? sums_v + w * 4 * P : nullptr);
     if (!a.bias_kv) return;
     __syncthreads();
     const size_t ntc = (size_t)a.B * kblocks, part = (size_t)h * ntc + b * kblocks + kb;
