@@ -174,9 +174,11 @@ def _make_function(m):
         @staticmethod
         def backward(ctx, dy):
             x, enc, *params = ctx.saved_tensors
-            # (the epilogues of the backward pass need whole 16-byte words, wherever a parameter lies or was restored to)
-            params = [t if t.data_ptr() % 16 == 0 else t.clone() for t in params]
             w = dict(zip(names, params))
+            # (the products with an epilogue need whole 16-byte words, wherever a parameter lies or was restored to)
+            for n in ('linear2_w', 'edattn_wv', 'sattn_wkqv'):
+                if w[n].data_ptr() % 16:
+                    w[n] = w[n].clone()
             s = ctx.saved
             dy = dy.contiguous()
             # the second stage of every column sum of the pass (eight bias / scale gradients) in one launch at its end

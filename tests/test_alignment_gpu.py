@@ -82,23 +82,26 @@ def test_gelu_layer_whose_backward_epilogue_finds_a_misaligned_tensor(dims, odd)
         _close(_pass(enc, x, dy), want)
 
 
-def test_decoder_layer_whose_second_feed_forward_weight_is_misaligned():
-    """2048 x 4096 feed-forward outputs: 128 tiles of 256 x 256, so linear1 carries its activation."""
+def test_decoder_layer_whose_parameters_are_misaligned():
+    """2048 x 4096 feed-forward outputs: 128 tiles of 256 x 256, so linear1 carries its activation.  The second feed-forward
+    weight at an odd address in both passes; every parameter restored to one for the backward pass."""
     from substation_amd import DecoderLayer
     torch.manual_seed(0)
     layer = DecoderLayer(8, 256, 128, 4, 256, 0.1, 0.1, 0.1, 0.1, activation='gelu', seed=SEED, intermediate_size=4096).cuda()
     x, src, dy = (torch.randn(8, n, 256).half().cuda() for n in (256, 128, 256))
-    got = []
-    for odd in (False, True):
-        if odd:
-            layer.linear2_w.data = _odd(layer.linear2_w.data)
+
+    def both_passes(restore=lambda t: t):
         layer.zero_grad(set_to_none=True)
         layer.set_rng(SEED, 1)
-        y = layer(x, src)
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, restore):
+            y = layer(x, src)
         assert layer.ffn_in_epilogues
         y.backward(dy)
-        got.append(dict([('y', y.detach())] + [(n, q.grad) for n, q in layer.named_parameters()]))
-    _close(got[1], got[0])
+        return dict([('y', y.detach())] + [(n, q.grad) for n, q in layer.named_parameters()])
+    want = both_passes()
+    _close(both_passes(_odd), want)
+    layer.linear2_w.data = _odd(layer.linear2_w.data)
+    _close(both_passes(), want)
 
 
 @pytest.mark.parametrize('act', ['relu', 'gelu'])
