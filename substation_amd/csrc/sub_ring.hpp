@@ -313,7 +313,7 @@ struct Ring : TileList<32 * TM * WM, 32 * TN * WN, NP> {
             if (from_bits) {
                 const __amdgpu_buffer_rsrc_t r = bits_rsrc(p);
 #pragma unroll
-                for (int k = 0; k < WORDS; ++k) bits[k] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, (int)bits_at, (int)(k * bits_step), 0);
+                for (int k = 0; k < WORDS; ++k) bits[k] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, (int)(bits_at + k * bits_step), 0, 0);
             }
         }
         uint32_t kb[WORDS];                                                // FORWARD: keep bits of the lane's packs, a byte each
@@ -398,7 +398,7 @@ struct Ring : TileList<32 * TM * WM, 32 * TN * WN, NP> {
                         const uint32_t word = quad_word(keep, lane);
                         out_word = q == (c & 3) ? word : out_word;
                         if constexpr ((c & 3) == 3 || c == PACKS - 1)
-                            __builtin_amdgcn_raw_buffer_store_b32(out_word, ro, (int)bits_at, (int)((c >> 2) * bits_step), 0);
+                            __builtin_amdgcn_raw_buffer_store_b32(out_word, ro, (int)(bits_at + (c >> 2) * bits_step), 0, 0);
                     }
                     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4v, val), rc, (int)c_at, 0, 0);
                     c_at += c_step;

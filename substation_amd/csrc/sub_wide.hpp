@@ -141,13 +141,16 @@ struct Wide : TileList<4 * QM, 4 * QN, NP> {
         unsigned round = 0;
         unsigned oa[LA], ob[LB];      // bytes from a half's first element to the lane's words
     };
-    static __device__ __forceinline__ void aim(u4v (&r)[2], const half_t* first, long bytes, long half) {
+    // (The range check takes a load's scalar offset, the place in k, from the half's size: that offset is never larger than it.  So
+    // a second half that lies past the operand's last row is not one of no bytes: its rows are read as those of the first, and
+    // multiplied into outputs that there are none of.)
+    static __device__ __forceinline__ void aim(u4v (&r)[2], const half_t* first, long bytes, long half, bool second) {
         auto u = [](uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); };
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            const uint64_t p = reinterpret_cast<uint64_t>(first) + (uint64_t)(h * half);
-            const long n = bytes - h * half;
-            r[h] = u4v{u((uint32_t)p), u((uint32_t)(p >> 32)), u(n > 0 ? (uint32_t)n : 0u), 0x00020000u};
+            const long at = h && second ? half : 0;
+            const uint64_t p = reinterpret_cast<uint64_t>(first) + (uint64_t)at;
+            r[h] = u4v{u((uint32_t)p), u((uint32_t)(p >> 32)), u((uint32_t)(bytes - at)), 0x00020000u};
         }
     }
     static __device__ __forceinline__ void open(Group& G, Stream& s, unsigned l, unsigned n, int wave, int lane) {
@@ -168,9 +171,9 @@ struct Wide : TileList<4 * QM, 4 * QN, NP> {
         s.ka = s.step_a * (unsigned)kin; s.kb = s.step_b * (unsigned)kin;
         const int rows = min(g.M - t.m0, BM), cols = min(g.N - t.n0, BN);
         aim(s.ra, g.A + t.b0 * g.sAb[0] + t.b1 * g.sAb[1] + t.b2 * g.sAb[2] + (long)t.m0 * g.sAM + outer * g.sAK0,
-            2 * ((long)(rows - 1) * g.sAM + (long)(g.K1 - 1) * g.sAK1 + 1), 2 * HM * g.sAM);
+            2 * ((long)(rows - 1) * g.sAM + (long)(g.K1 - 1) * g.sAK1 + 1), 2 * HM * g.sAM, rows > HM);
         aim(s.rb, g.B + t.b0 * g.sBb[0] + t.b1 * g.sBb[1] + t.b2 * g.sBb[2] + (long)t.n0 * g.sBN + outer * g.sBK0,
-            2 * ((long)(cols - 1) * g.sBN + (long)(g.K1 - 1) * g.sBK1 + 1), 2 * HN * g.sBN);
+            2 * ((long)(cols - 1) * g.sBN + (long)(g.K1 - 1) * g.sBK1 + 1), 2 * HN * g.sBN, cols > HN);
         if (kc & 1) DTile<HM, true, NW>::offsets(s.oa, g.sAM, g.sAK1, wave, lane);
         else DTile<HM, false, NW>::offsets(s.oa, g.sAM, g.sAK1, wave, lane);
         if (kc & 2) DTile<HN, true, NW>::offsets(s.ob, g.sBN, g.sBK1, wave, lane);
@@ -409,7 +412,7 @@ struct Wide : TileList<4 * QM, 4 * QN, NP> {
                     const __amdgpu_buffer_rsrc_t r = bits_of(g, t, GATED ? g.gate_bits : g.keep_words, wm, wn, lane, at);
 #pragma unroll
                     for (int k = 0; k < 8; ++k)
-                        bits[k] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, (int)at[k >> 1 & 1], (int)bits_part(g, k), 0);
+                        bits[k] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, (int)(at[k >> 1 & 1] + bits_part(g, k)), 0, 0);
                 }
                 if constexpr (DRAWS) {
                     draw.key = key_of(g.key);
@@ -438,12 +441,13 @@ struct Wide : TileList<4 * QM, 4 * QN, NP> {
                 auto u = [](uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); };
                 return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(at), 0, (int)u((uint32_t)(bytes < 0x7fffffffL ? bytes : 0x7fffffffL)), 0x00020000);
             };
-            // (at: the lane's part of a word's place, `uni` the wave's)
+            // (at: the lane's part of a word's place, `uni` the wave's.  Their sum is the vector offset, which alone is certain to
+            // be checked: `uni` may lie beyond the buffer's size, and as a scalar offset would be taken from that.)
             auto get = [](__amdgpu_buffer_rsrc_t r, unsigned at, unsigned uni) __attribute__((always_inline)) {
-                return __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(r, (int)at, (int)uni, 0));
+                return __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(r, (int)(at + uni), 0, 0));
             };
             auto put = [](__amdgpu_buffer_rsrc_t r, unsigned at, unsigned uni, h8 v) __attribute__((always_inline)) {
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4v, v), r, (int)at, (int)uni, 0);
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4v, v), r, (int)(at + uni), 0, 0);
             };
             const long c_first = t.b0 * g.sCb[0] + t.b1 * g.sCb[1] + t.b2 * g.sCb[2];
             const __amdgpu_buffer_rsrc_t rc = buffer(g.C + c_first, g.sCM);
@@ -543,7 +547,7 @@ struct Wide : TileList<4 * QM, 4 * QN, NP> {
                                 const uint32_t word = quad_word(keep, lane);
                                 out_word = (lane & 3) == (c & 3) ? word : out_word;
                                 if constexpr ((c & 3) == 3)
-                                    __builtin_amdgcn_raw_buffer_store_b32(out_word, ro, (int)at_o[c >> 3 & 1], (int)bits_part(g, c >> 2), 0);
+                                    __builtin_amdgcn_raw_buffer_store_b32(out_word, ro, (int)(at_o[c >> 3 & 1] + bits_part(g, c >> 2)), 0, 0);
                             }
                             put(rc, at, uni, val);
                         });

@@ -236,3 +236,79 @@ def test_wide_tiles_with_remainders(B, L, E, U):
             torch.cuda.synchronize()
             check(C1, want(la1, d[la1], lb1, d[lb1], lc1, 1.0, T, lt1), f'{la1},{lb1}->{lc1}')
             check(C2, want(la2, d[la2], lb2, d[lb2], lc2), f'{la2},{lb2}->{lc2}')
+
+
+class _Guarded:
+    """Tensors in the middle of allocations of their own: 4 MiB of a pattern on both sides, more than a tile of 256 rows of the
+    outputs below, which no kernel may write and whose values (NaN as halves) no output may show."""
+    GUARD = 4 << 20
+
+    def __init__(self):
+        self.held = []
+
+    def place(self, shape, dtype=torch.float16, values=None):
+        n = int(np.prod(shape)) * torch.empty(0, dtype=dtype).element_size()
+        flat = torch.full((n + 2 * self.GUARD,), 0x7E, dtype=torch.uint8, device='cuda')
+        self.held.append(flat)
+        t = flat[self.GUARD:self.GUARD + n].view(dtype).view(shape)
+        return t if values is None else t.copy_(values)
+
+    def check(self, name):
+        torch.cuda.synchronize()
+        for i, flat in enumerate(self.held):
+            assert bool((flat[:self.GUARD] == 0x7E).all()) and bool((flat[-self.GUARD:] == 0x7E).all()), (name, i)
+
+
+@pytest.mark.parametrize('L,E,U', [(4104, 1024, 4104),     # 256 x 256 tiles whose last row and column have 8 of 256
+                                   (4296, 1032, 4240),     # 200 rows, 144 columns; a contraction with a remainder
+                                   (2616, 128, 776), (1928, 72, 2056), (72, 136, 200)])
+def test_nothing_behind_an_output_is_written_and_nothing_behind_an_operand_read(L, E, U):
+    """Rows and columns of tiles that the output has not: every way of reading the operands, alone, with a bias row and with
+    a whole addend."""
+    from substation_amd.ops import Ops
+    o = Ops(1, L, 1, E, intermediate_size=U)
+    sz = o.sizes
+    g = torch.Generator(device='cuda').manual_seed(L)
+    for la in ('BJI', 'IBJ'):
+        for lb in ('UI', 'IU'):
+            mem = _Guarded()
+            mk = lambda lay: mem.place([sz[d] for d in lay], values=torch.randn([sz[d] for d in lay], generator=g, device='cuda'))
+            A, Bm, bias, T = mk(la), mk(lb), mk('U'), mk('BJU')
+            mat = lambda X, lay: X.float().reshape(L, E) if lay == 'BJI' else X.float().reshape(E, -1).t() if lay == 'IBJ' else \
+                X.float() if lay == 'IU' else X.float().t()
+            want = mat(A, la) @ mat(Bm, lb)
+            for t, lt in ((None, None), (bias, 'U'), (T, 'BJU')):
+                C = mem.place([sz[d] for d in 'BJU'])
+                o.einsum(A, la, Bm, lb, C, 'BJU', addend=t, l_addend=lt)
+                name = f'{la},{lb} + {lt}'
+                mem.check(name)
+                w = want if t is None else want + t.float().reshape(-1, U)
+                # fp16 outputs of sums of up to 1032 terms: half a step, twice with an addend, and the sums' order
+                assert float((C.float().reshape(L, U) - w).abs().max()) <= 2.0 ** -10 * float(w.abs().max()), name
+
+
+@pytest.mark.parametrize('L,E,U', [(4104, 1024, 4128), (2616, 768, 3104), (1000, 512, 4128)])
+@pytest.mark.parametrize('act', ['relu', 'gelu'])
+def test_nothing_behind_what_an_activation_epilogue_leaves_is_written(L, E, U, act):
+    """The output, the pre-activation, the bits and the gradient of tiles that are not whole."""
+    from substation_amd.ops import Ops
+    o = Ops(1, L, E // 64, E, intermediate_size=U, activation=act, seed=7)
+    sz = o.sizes
+    g = torch.Generator(device='cuda').manual_seed(L)
+    mem = _Guarded()
+    mk = lambda lay, s=1.0: mem.place([sz[d] for d in lay], values=s * torch.randn([sz[d] for d in lay], generator=g, device='cuda'))
+    x, w1, bias, dy, w2 = mk('BJI'), mk('UI', 0.05), mk('U'), mk('BJI'), mk('IU', 0.05)
+    out, lin, dlin = (mem.place([sz[d] for d in 'BJU']) for _ in range(3))
+    bits, dbias = mem.place([L * U // 8], torch.uint8), mem.place([U])
+    assert o.einsum_bad(x, 'BJI', w1, 'UI', bias, 'U', lin if act == 'gelu' else None, out, 'BJU', bits, p=0.1)
+    mem.check('forward')
+    assert o.einsum_bdrlb(dy, 'BJI', w2, 'IU', lin if act == 'gelu' else out, 'BJU', bits, dlin, 'BJU', dbias)
+    mem.check('backward')
+    # and the values are those of the operators, the bias gradient to rounding (up to 4104 terms in another order)
+    sb, mask, lin2, out2, dlin2, dbias2 = (torch.empty(shape, dtype=torch.float16, device='cuda') for shape in [out.shape] * 5 + [[U]])
+    o.einsum(x, 'BJI', w1, 'UI', sb, 'BJU')
+    o.bad(sb, 'BJU', bias, lin2, 'BJU', mask, 'BJU', out2, 'BJU', p=0.1)
+    o.einsum(dy, 'BJI', w2, 'IU', sb, 'BJU')
+    o.bdrlb(sb, 'BJU', mask, 'BJU', lin2, 'BJU', dlin2, 'BJU', dbias2)
+    assert torch.equal(out, out2) and torch.equal(dlin, dlin2) and float(dlin.float().abs().max()) > 0
+    assert_close(dbias.float().cpu().numpy(), dbias2.float().cpu().numpy(), tol=2e-3, name='dbias')
