@@ -198,7 +198,7 @@ int sub_set_attention_mask(void* handle, const void* attn_mask, const char* layo
  * and DROP2 in BJU order, bias, ReLU and dropout then run in the epilogue of the
  * lin1 product (profiling name `lin1+bad`) and SB1_LINW1 is not written either:
  * the first B*J*U/8 bytes of that buffer then hold one bit per element of DROP2
- * (set where it is positive), in the kernel's own order.  In encoder_backward
+ * (set where it is positive), in canonical order (bit (b*J + j)*U + u).  In encoder_backward
  * bdrlb runs in the epilogue of the dXlin2 product (`dXlin2+bdrlb`), which takes
  * its gate from those bits when it is handed the SB1_LINW1 buffer that the
  * handle's latest encoder_forward call wrote and from DROP2 itself otherwise
@@ -506,16 +506,16 @@ int sub_op_einsum(void* handle, const void* A, const char* l_A, const void* B, c
  * sub_op_einsum_bad: out = dropout(act(einsum(A, B) + bias)) (gemm.cuh:134-147 followed
  * by block_bad.cuh:28-145) with the handle's activation and the keep bits of (seed,
  * step, site, p); `out` in BJU order; `bits` receives B*J*U/8 bytes (ReLU: one bit per
- * output, set where it is positive; GELU: the keep bits) in the kernel's own order, for
- * sub_op_einsum_bdrlb only; GELU also stores the pre-activation to `lin`, laid out like
+ * output, set where it is positive; GELU: the keep bits) in the order of the output, for
+ * sub_op_einsum_bdrlb; GELU also stores the pre-activation to `lin`, laid out like
  * `out` (ReLU: ignored, may be null).
  * sub_op_einsum_bdrlb: dlinear = act'(.) * keep * einsum(A, B) and dbias = its sum over
  * the tokens (gemm.cuh:134-147 followed by block_bdrlb.cuh:13-146); `gate` is the forward
  * output (ReLU) or the pre-activation (GELU), laid out like `dlinear` (BJU), `bits`
  * what sub_op_einsum_bad left.
  * *applied = 0 and nothing launched when the product does not qualify for the kernel
- * that carries these epilogues (whole 256 x 256 tiles for most of the CUs, 16-byte
- * aligned tensors): the caller then runs the product and the operator one after the other. */
+ * that carries these epilogues (from 64 tiles of 256 x 256 outputs on, whole or not; U a
+ * multiple of 32; 16-byte aligned tensors): the caller then runs the product and the operator one after the other. */
 int sub_op_einsum_bad(void* handle, const void* A, const char* l_A, const void* B, const char* l_B, const void* bias,
                       const char* l_bias, void* lin, void* out, const char* l_out, void* bits, float p, uint32_t site,
                       int* applied);

@@ -2265,8 +2265,11 @@ int sub_op_einsum_pair(void* handle, const void* A1, const char* l_A1, const voi
     });
 }
 
-// Operator calls: products of a quarter of the chip in 256 x 256 tiles and more.  (With fewer a launch is a few us, and the
-// caller's way of many calls bounds it; it keeps the mask as a tensor that can be looked at.)
+// Operator calls: products of a quarter of the chip in 256 x 256 tiles and more.  Below that the caller keeps a mask tensor that
+// can be looked at, which is the only reason for the line: one launch is faster than two at every size.  us of one launch (two),
+// p = 0.1, ReLU forward, backward, GELU forward, backward; 256 rows x 3072 x 768 (12 tiles): 8.9 (10.9), 10.1 (14.4), 8.9 (11.1),
+// 10.6 (14.4); 1024 x 3072 x 768 (48): 13.1 (17.9), 13.6 (21.7), 15.6 (18.1), 16.2 (22.0); 1024 x 4096 x 1024 (64): 16.9 (23.2),
+// 17.7 (26.4), 20.0 (23.5), 20.6 (27.4); 3072 x 4096 x 1024 (192): 38.3 (45.8), 34.8 (52.8), 42.6 (45.1), 40.9 (52.2).
 static bool worth_an_epilogue(const GemmShape& g) { return ((g.M + 255) / 256) * ((g.N + 255) / 256) >= 64; }
 
 int sub_op_einsum_bad(void* handle, const void* A, const char* l_A, const void* B, const char* l_B, const void* bias,

@@ -390,11 +390,13 @@ void launch_gemm(const GemmShape& s, const half_t* A, const half_t* B, half_t* C
         const bool small = ws && (size_t)batch * c.a.M * c.a.N <= kSplitMaxOut;
         if (small && !ep.any_split) tp.a.splits = pick_splits(c.a, batch, ws_floats);
         const TileChoice choice = choose_single(tp, small && ep.any_split ? ws_floats : 0);
+        unsigned side_blocks = 0;
         if (side) side->tiles_done = 0;
         if (side && side->keep && side->key.thr && choice.form == TILE_256x256 && choice.splits == 1) {
             // CUs the tiles leave idle draw attention keep bits meanwhile: what fits into the time the
-            // product takes (about 9 us + 1.5 us per k-tile; the rate per CU and us is the measured break-even:
-            // 12 of the 16 key tiles of the bench workload cost the launch 0.3 us, 14 cost it 2.5, all 16 6 us)
+            // product takes (about 9 us + 1.5 us per k-tile; the rate per CU and us is the measured break-even.  At 8 x 512, E 1024,
+            // us of this launch and of the attention behind it with 10 of the 16 key tiles drawn here: 32.5 and 23.5, 11: 32.5 and
+            // 23.1, 12 (what the rule gives): 32.5 and 22.7, 14: 34.7 and 22.0, all 16: 38.3 and 20.9)
             const long tiles = (long)((c.a.M + 255) / 256) * ((c.a.N + 255) / 256) * batch;
             const long idle = 256 - tiles, nkt = (long)c.a.K0 * ((c.a.K1 + BK - 1) / BK);
             if (tiles >= 128 && idle >= 32 && side->nk % 32 == 0) {
@@ -402,7 +404,7 @@ void launch_gemm(const GemmShape& s, const half_t* A, const half_t* B, half_t* C
                 long td = (long)(groups / (4.0 * (double)side->rows));
                 if (td > side->nk / 32) td = side->nk / 32;
                 if (td > 0) {
-                    c.a.side_first = (unsigned)tiles; c.a.side_blocks = (unsigned)idle;
+                    side_blocks = (unsigned)idle;
                     c.a.side_key = side->key; c.a.side_keep = side->keep;
                     c.a.side_rows = side->rows; c.a.side_nk = side->nk; c.a.side_tiles_done = (uint32_t)td;
                     side->tiles_done = (uint32_t)td;
@@ -410,8 +412,8 @@ void launch_gemm(const GemmShape& s, const half_t* A, const half_t* B, half_t* C
             }
         }
         tp.a = c.a; tp.a.nbatch = batch;
-        if (c.a.side_blocks) {
-            launch_wide(&tp, 1, nullptr, c.a.side_blocks, st);
+        if (side_blocks) {
+            launch_wide(&tp, 1, nullptr, side_blocks, st);
         } else {
             tp.a.splits = choice.splits;
             if (tp.a.splits > 1) tp.a.partial = ws;

@@ -22,18 +22,17 @@ struct GemmArgs {
     int splits;                   // > 1: the k range is split, fp32 partial tiles go to `partial`
     float* partial;               // [split][batch][M][N]
     long nbatch = 1;              // batches in all
-    int relu_dropout = 0;         // epilogue of the 256 x 256 tiles: ReLU and dropout after the addend
+    int relu_dropout = 0;         // the activation and dropout after the addend
     PhiloxKey key;
-    const half_t* gate = nullptr; // or: zero where gate <= 0 (strides of `bias`), column sums per 128-row slab
+    const half_t* gate = nullptr; // or: the activation's backward pass (strides of `bias`), with column sums per row of waves
     float* colsum = nullptr;
     const uint32_t* keep_words = nullptr;  // relu_dropout: the keep bits, drawn ahead (relu_dropout_keep_words)
     uint32_t* gate_bits_out = nullptr;     // relu_dropout: one bit per output, set where it is positive
     const uint32_t* gate_bits = nullptr;   // gate: those bits instead of the values of `gate`
     int act = ACT_RELU;                    // the activation of relu_dropout / gate (GemmEpilogue::act)
     half_t* pre_out = nullptr;             // GELU with dropout: where the rounded sum before the activation goes
-    // GemmSideJob of the 256 x 256 kernel: workgroups side_first .. gridDim.x - 1 draw
+    // GemmSideJob of the 256 x 256 kernel: the workgroups behind those of the tiles draw
     // the attention keep words of key tiles 0 .. side_tiles_done - 1 of side_rows score rows
-    unsigned side_first = 0, side_blocks = 0;
     PhiloxKey side_key;
     uint32_t* side_keep = nullptr;
     uint32_t side_rows = 0, side_nk = 0, side_tiles_done = 0;

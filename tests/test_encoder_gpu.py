@@ -1374,3 +1374,36 @@ def test_activation_epilogues_where_a_caller_may_look_into_the_intermediates(bat
     enc(x).backward(torch.ones_like(x))
     launches = [n for n, _ in enc.profile()]
     assert tuple(n for n in launches if n in ('lin1+bad', 'dXlin2+bdrlb')) == fused, launches
+
+
+@pytest.mark.parametrize('dims', [(2, 128, 12, 768, 3072), (5, 72, 4, 512, 1056), (13, 201, 12, 768, 3072), (24, 77, 12, 768, 3072)])
+def test_keep_bits_drawn_ahead_for_tiles_of_every_size(dims):
+    """Option 8, bit 1: the first LayerNorm launch draws the keep bits of lin1's ReLU epilogue, which reads them on tiles of
+    four sizes; the words are those of the seeded mask, and no bit of output or gradients changes."""
+    from substation_amd import Encoder, layouts as L
+    B, Ls, H, E, U = dims
+    got = []
+    for jobs in (3, 0):
+        torch.manual_seed(0)
+        enc = Encoder('unused', B, Ls, H, E, L.mi355x_layouts(), torch.float16, 0.1, 0.1, 0.1, 0.1, seed=SEED,
+                      intermediate_size=U, persistent_workspace=True, profiling=True).cuda()
+        with torch.no_grad():
+            for q in enc.parameters():
+                q.mul_(0.1)
+        enc._handle.set_option(8, jobs)
+        g = torch.Generator().manual_seed(5)
+        x = torch.randn(B, Ls, E, generator=g).half().cuda().requires_grad_(True)
+        dy = torch.randn(B, Ls, E, generator=g).half().cuda()
+        enc.set_rng(SEED, 3)
+        y = enc(x)
+        held = dict(zip((n for n, _ in enc.layouts['forward_interm']), enc._workspace['forward_interm']))['SB1_LINW1'].clone()
+        y.backward(dy)
+        assert 'lin1+bad' in [n for n, _ in enc.profile()]
+        got.append([y.detach().clone(), x.grad.clone()] + [q.grad.clone() for q in enc.parameters()])
+        if jobs:
+            n = B * Ls * U // 8
+            words = held.reshape(-1).view(torch.uint8)[n:2 * n].cpu().numpy()
+            keep = ph.dropout_mask((B, Ls, U), 0.1, SEED, 2, step=3, dtype=np.uint8)
+            assert np.array_equal(words, np.packbits(keep.reshape(-1), bitorder='little'))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
