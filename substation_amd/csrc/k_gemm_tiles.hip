@@ -81,17 +81,27 @@ TileChoice choose_tiles(const TileProduct* p, int n, unsigned forms, size_t ws_f
 
 TileForm tile_form(int form) { return TileForm{kForms[form].bm, kForms[form].bn, kForms[form].per_cu}; }
 
-// What the activation adds to a tile (us): per pack of 8 outputs that a lane stores, its arithmetic and, but for the 256 x 256
-// tiles, which draw them between their matrix instructions, its keep bits.
+// What the activation adds to a tile (us): for each pack of 8 outputs that a lane stores, its arithmetic (0.1, GELU 0.25) and,
+// forward, its keep bits: 0.2, and 0.13 on 256 x 256 tiles, which draw them between their matrix instructions, but not for nothing
+// (taken as free, a ReLU layer of 2613 x 3072 x 768 went to those tiles: 35.2 us, now 27.9 on 128 x 128).  Measured, the difference
+// to the plain product of the same tiles, 1848 and 2613 x 3072 x 768 and 4096 x 4096 x 1024, p = 0.1 (in brackets without dropout):
+//              64 x 64             128 x 64            128 x 128           256 x 128           256 x 256
+//   ReLU       .15-.16 (.05-.12)   .06-.16 (.04-.08)   .21-.29 (.08-.19)   .23-.26 (.12-.15)   .18-.24 (.06-.09)
+//   GELU       .20-.32 (.14-.28)   .24-.34 (.20-.32)   .49-.65 (.35-.52)   .39-.46 (.28-.35)   .29-.37 (.20-.27)
+//   ReLU back  .26-.32             .18-.32             .23-.34             .45-.58             .13-.18
+//   GELU back  .51-.60             .71-.79             .62-.68             .75-.88             .36-.42
+// With these numbers per form in place of the four, the same tiles come out at these sizes but for GELU at 2613 (128 x 64: 29.5
+// for 30.2 alone, 32.6 for 31.6 within the layer) and ReLU's backward at 2560 x 2048 x 512 (24.4 for 22.2): the four stay.  Against
+// the best tiles in brackets this takes at 1848 rows 20.2 (20.2), 23.3 (23.3), 23.7 (23.0), 28.1 (28.1) us in the order of the
+// rows, at 2613 24.4 (24.4), 30.2 (29.5), 24.5 (24.5), 30.0 (30.0).
 int choose_act_form(const TileProduct& p) {
     int best = -1;
     double best_us = 0.;
     for (int f = 0; f < TILE_FORMS; ++f) {
-        const bool wide = f == TILE_256x256;
-        if (wide ? !wide_takes(p) : !p.akc) continue;
+        if (f == TILE_256x256 ? !wide_takes(p) : !p.akc) continue;
         const Form& F = kForms[f];
         const long len = steps_of(p.a, 1), cnt = tiles_of(p.a, 1, F.bm, F.bn);
-        const double packs = (double)F.bm * F.bn / (4 * 64 * 8) * F.per_cu, draw = p.a.gate || wide ? 0. : 0.2;
+        const double packs = (double)F.bm * F.bn / (4 * 64 * 8) * F.per_cu, draw = p.a.gate ? 0. : f == TILE_256x256 ? 0.13 : 0.2;
         const double rounds = (double)((cnt + 256L * F.per_cu - 1) / (256L * F.per_cu));
         const double us = launch_us(&len, &cnt, 1, F) + rounds * packs * ((p.a.act == ACT_GELU ? 0.25 : 0.1) + draw);
         if (best < 0 || us < best_us) { best = f; best_us = us; }
