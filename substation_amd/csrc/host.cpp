@@ -125,6 +125,7 @@ bool plain(const at::Tensor& X, const std::vector<at::Tensor>& params) {
 // restore it as a slice of a larger buffer, or with other strides.)
 bool misaligned(const at::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) & 15; }
 at::Tensor as_saved(at::Tensor t, bool was_misaligned) {
+    if (t.is_contiguous() && (was_misaligned || !misaligned(t))) return t;
     at::NoGradGuard no_grad;
     t = t.contiguous();
     return misaligned(t) && !was_misaligned ? t.clone() : t;
