@@ -291,7 +291,9 @@ int sub_set_forward_form(void* handle, int form);
 /* SUB_OPT_OPAQUE_INTERMEDIATES (default 0; the Python module sets it): the caller hands the intermediates from
  * encoder_forward to encoder_backward and looks into none of them.  Option 9 then also covers DROP2MASK where the
  * activation's dropout runs as an operator of its own and its mask is kept (bits in the first B*J*U/8 bytes, feed-forward
- * size a multiple of 8), and option 10 also ATT and DROP2_LINW2 where their products were split along k and go into the
+ * size a multiple of 8), option 6's epilogues run at any size (without it only where the outputs of lin1 resp. dXlin2 are
+ * whole 256 x 256 tiles that fill their rounds of 256 to 0.7, or to 0.9 where an operand does not lie along k; GELU: both), and
+ * option 10 also ATT and DROP2_LINW2 where their products were split along k and go into the
  * launch behind them as partial sums.  Same results.  Both calls must see the same value. */
 #define SUB_OPT_OPAQUE_INTERMEDIATES 12
 /* *planned = 1 when, with the handle's sizes, layouts and options as they are

@@ -10,9 +10,12 @@
 // one inside does (the kernel before predicated every load of such a product).  M = 2613 rows, us before and now:
 // 768 x 3072 (n x k) 35 -> 21, 3072 x 768 21 -> 18.5, its weight gradient 42 -> 20.5; 64 rows x 768 x 768: 14 -> 6.4; 4096 x 1024 x
 // 4096: 43 -> 35-37 (930 to 990 TFLOP/s, box to box).  4096 x 1024 x 1024, one tile of 16 steps per CU, takes 15 to 17 us.
-// Registers: 72 to 168 a lane up to 128 x 128 tiles, 242 to 256 at 256 x 128, where the instance of two orientations (two
-// loop bodies) spills two of them (12 bytes of scratch); the instances of one product hold its arguments in scalar
-// registers and spill 25 to 36 of those, the ones of several products none.
+// Registers without an activation: 72 to 168 a lane up to 128 x 128 tiles, 242 to 256 at 256 x 128, where the instance of two
+// orientations (two loop bodies) spills two of them (12 bytes of scratch) and that of one product with both operands across k one;
+// the instances of one product hold its arguments in scalar registers and spill 26 to 36 of those, the ones of several
+// products none.  With one: 85 to 212 up to 128 x 128 (128 x 64 with GELU: 20 bytes of scratch), 253 to 256 at 256 x 128, where
+// GELU spills 2 to 7 (12 to 32 bytes), ReLU's gate 44 to 50 (180 to 204), GELU's backward form 56 to 61 (228 to 248), all in the
+// epilogue; 27 to 39 scalar registers backward, 90 to 125 forward (the keys and constants of the draws).
 #pragma once
 
 #include "sub_tiles.hpp"
