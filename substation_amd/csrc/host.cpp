@@ -123,13 +123,25 @@ bool plain(const at::Tensor& X, const std::vector<at::Tensor>& params) {
 
 // A saved tensor as the backward pass needs it: dense, and 16-byte aligned where the forward pass found it so.  (A hook may
 // restore it as a slice of a larger buffer, or with other strides.)
+// What it cannot be is on another device, of another type or size: the kernels are handed bare pointers.
 bool misaligned(const at::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) & 15; }
-at::Tensor as_saved(at::Tensor t, bool was_misaligned) {
-    if (t.is_contiguous() && (was_misaligned || !misaligned(t))) return t;
-    at::NoGradGuard no_grad;
-    t = t.contiguous();
-    return misaligned(t) && !was_misaligned ? t.clone() : t;
-}
+struct Saved {
+    SavedVariable variable;
+    at::Device device;
+    int64_t numel;
+    bool was_misaligned;
+    explicit Saved(const at::Tensor& t) : variable(t, false), device(t.device()), numel(t.numel()), was_misaligned(misaligned(t)) {}
+    at::Tensor unpack() const {
+        at::Tensor t = variable.unpack();
+        if (t.device() != device || t.scalar_type() != at::kHalf || t.numel() != numel)
+            raise("a tensor that the forward pass has saved was restored on another device, with another type or another size",
+                  PyExc_RuntimeError);
+        if (t.is_contiguous() && (was_misaligned || !misaligned(t))) return t;
+        at::NoGradGuard no_grad;
+        t = t.contiguous();
+        return misaligned(t) && !was_misaligned ? t.clone() : t;
+    }
+};
 
 // An additive attention mask and the order of its dims.
 struct Mask {
@@ -238,19 +250,13 @@ struct EncoderBackward : Node {
     std::shared_ptr<Mask> mask;          // of the forward pass
     // the parameters as the forward pass read them, X, and the forward intermediates (those of a layer that keeps its own
     // too: what hooks on saved tensors see does not depend on who holds the memory)
-    std::vector<SavedVariable> saved;
-    std::vector<bool> misaligned;        // of those
+    std::vector<Saved> saved;
     int form = 0;                        // what the forward pass left (sub_forward_form)
     uint64_t generation = 0, pass = 0;
 
-    void save(const at::Tensor& t) {
-        saved.emplace_back(t, false);
-        misaligned.push_back(::misaligned(t));
-    }
-
     std::string name() const override { return "EncoderFunctionBackward"; }
     void release_variables() override {
-        for (auto& s : saved) s.reset_data();
+        for (auto& s : saved) s.variable.reset_data();
     }
 
     variable_list apply(variable_list&& grads) override {
@@ -261,7 +267,7 @@ struct EncoderBackward : Node {
         l.check_relu_gate();
         variable_list in;
         in.reserve(saved.size());
-        for (size_t i = 0; i < saved.size(); ++i) in.push_back(as_saved(saved[i].unpack(), misaligned[i]));
+        for (const auto& s : saved) in.push_back(s.unpack());
         const size_t np = l.param_shapes.size();
         const at::Tensor& X = in[np];
         const c10::DeviceGuard guard(X.device());
@@ -348,9 +354,9 @@ std::optional<at::Tensor> EncoderLayer::forward(const at::Tensor& X_, const std:
         node->mask = mask;
         const std::vector<at::Tensor>& held = persistent ? kept_fwd : interm;
         node->saved.reserve(w.size() + 1 + held.size());
-        for (const auto& t : w) node->save(t);
-        node->save(X);
-        for (const auto& t : held) node->save(t);
+        for (const auto& t : w) node->saved.emplace_back(t);
+        node->saved.emplace_back(X);
+        for (const auto& t : held) node->saved.emplace_back(t);
         node->form = form();
         node->generation = generation;
         node->pass = passes;

@@ -176,3 +176,16 @@ def test_misaligned_feed_forward_weights_of_feature_major_layouts(odd, act):
             getattr(enc, n).data = _odd(getattr(enc, n).data)
     for n, t in _pass(enc, x, dy).items():
         assert torch.equal(want[n], t), n
+
+
+@pytest.mark.parametrize('python', [False, True])
+@pytest.mark.parametrize('restore', [lambda t: t.cpu(), lambda t: t.float(), lambda t: t.reshape(-1)[:8]])
+def test_saved_tensors_that_hooks_restore_as_something_else_are_refused(python, restore):
+    """On another device, with another type or size: an error in front of the first launch, not bare pointers to it."""
+    enc, x, dy = _encoder((2, 128, 2, 128), 'gelu')
+    call = (lambda t: enc.encoder_func.apply(t, *enc.params)) if python else enc
+    want = _pass(enc, x, dy, call)
+    with pytest.raises(RuntimeError, match='restored'):
+        _pass(enc, x, dy, call, torch.autograd.graph.saved_tensors_hooks(lambda t: t, restore))
+    for n, t in _pass(enc, x, dy, call, torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t.reshape(-1))).items():
+        assert torch.equal(want[n], t.reshape(want[n].shape)), n
