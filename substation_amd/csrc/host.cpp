@@ -121,19 +121,21 @@ bool plain(const at::Tensor& X, const std::vector<at::Tensor>& params) {
     return !odd(X) && std::none_of(params.begin(), params.end(), odd);
 }
 
-// A saved tensor as the backward pass needs it: dense, and 16-byte aligned where the forward pass found it so.  (A hook may
-// restore it as a slice of a larger buffer, or with other strides.)
-// What it cannot be is on another device, of another type or size: the kernels are handed bare pointers.
+// A saved tensor as the backward pass needs it: dense, and 16-byte aligned where the forward pass found it so (a hook may
+// restore it as a slice of a larger buffer, or with other strides).  On another device, of another type or size it is
+// refused: the kernels are handed bare pointers.
 bool misaligned(const at::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) & 15; }
 struct Saved {
     SavedVariable variable;
     at::Device device;
+    at::ScalarType type;
     int64_t numel;
     bool was_misaligned;
-    explicit Saved(const at::Tensor& t) : variable(t, false), device(t.device()), numel(t.numel()), was_misaligned(misaligned(t)) {}
+    explicit Saved(const at::Tensor& t)
+        : variable(t, false), device(t.device()), type(t.scalar_type()), numel(t.numel()), was_misaligned(misaligned(t)) {}
     at::Tensor unpack() const {
         at::Tensor t = variable.unpack();
-        if (t.device() != device || t.scalar_type() != at::kHalf || t.numel() != numel)
+        if (t.device() != device || t.scalar_type() != type || t.numel() != numel)
             raise("a tensor that the forward pass has saved was restored on another device, with another type or another size",
                   PyExc_RuntimeError);
         if (t.is_contiguous() && (was_misaligned || !misaligned(t))) return t;

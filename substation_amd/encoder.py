@@ -70,7 +70,7 @@ def _python_function(weak, layer, in_shape, out_shape, shapes, workspace):
             call(module, 'encoder_forward', X.device, [X, *weights, *interm, Y])
             ctx.form = layer.form()
             ctx.save_for_backward(*weights, *interm, X)
-            ctx.saved_as = [(t.device, t.numel(), misaligned(t)) for t in (*weights, *interm, X)]
+            ctx.saved_as = [(t.device, t.dtype, t.numel(), misaligned(t)) for t in (*weights, *interm, X)]
             if module.enable_debug:
                 for (name, _), t in zip(list(layouts['forward_interm']) + list(layouts['params']), interm + weights):
                     module.debug[name] = t.detach().cpu().numpy()
@@ -88,13 +88,13 @@ def _python_function(weak, layer, in_shape, out_shape, shapes, workspace):
             interm = tensors(module, 'backward_interm', DY)
             # dense, and 16-byte aligned where the forward pass found them so, whatever hooks have restored
             saved = []
-            for t, (device, numel, was_misaligned) in zip(ctx.saved_tensors, ctx.saved_as):
-                if t.device != device or t.dtype != module.torch_dtype or t.numel() != numel:
+            for t, (device, dtype, numel, was_misaligned) in zip(ctx.saved_tensors, ctx.saved_as):
+                if t.device != device or t.dtype != dtype or t.numel() != numel:
                     raise RuntimeError('a tensor that the forward pass has saved was restored on another device, with '
                                        'another type or another size')
                 t = t.contiguous()
                 saved.append(t.clone() if misaligned(t) and not was_misaligned else t)
-            grads = [torch.empty(shape, device=DY.device, dtype=module.torch_dtype) for shape in shapes('params')]
+            grads = [torch.empty(shape, device=t.device, dtype=t.dtype) for shape, t in zip(shapes('params'), saved)]
             now, layer.mask = layer.mask, ctx.mask
             try:
                 layer.begin_backward(ctx.pass_number, ctx.form)
