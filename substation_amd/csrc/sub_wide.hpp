@@ -78,16 +78,17 @@ template <int ROWS, int ALONG_K>
 struct Fragments {
     typedef __attribute__((address_space(3))) const h8* lds_h8;
     typedef s4v __attribute__((address_space(3))) * lds_s4;
-    // ALONG_K: the swizzle of a row 16 rows further differs in bit 1 of the slot, 32 rows further in bit 2, and a slice of
-    // 32 k further the slot differs in bit 2: four addresses, everything else is a constant behind one of them.
-    // Else: rows 16 i further the address differs in bits 5 and 6.
+    // ALONG_K: the order within a row is the same 16 rows further, and a slice of 32 k further the slot differs in bit 2: two
+    // addresses, everything else is a constant behind one of them.  Else: rows 16 i further the address differs in bits 5 and 6.
+    using Along = DTile<ROWS, true, 4, 16>;
+    using Across = DTile<ROWS, false, 4, 16>;
     unsigned at[4];
     __device__ __forceinline__ void open(unsigned lds, int row0, int lane) {
         const int l = lane & 15, k = 8 * (lane >> 4) + (l >> 2), m = row0 + 4 * (l & 3);
-        const unsigned b = 2u * (unsigned)(ALONG_K ? DTile<ROWS, true, 4>::kc_off(row0 + l, lane >> 4)
-                                                   : k * ROWS + (((m >> 3) ^ DTile<ROWS, false, 4>::mc_swz(k)) << 3) + (m & 7));
+        const unsigned b = 2u * (unsigned)(ALONG_K ? Along::kc_off(row0 + l, lane >> 4)
+                                                   : k * ROWS + (((m >> 3) ^ Across::mc_swz(k)) << 3) + (m & 7));
 #pragma unroll
-        for (int x = 0; x < 4; ++x) at[x] = lds + (b ^ (unsigned)(x * 32));
+        for (int x = 0; x < 4; ++x) at[x] = lds + (b ^ (unsigned)(x * (ALONG_K ? 64 : 32)));
     }
     __device__ __forceinline__ void move(unsigned by) {
 #pragma unroll
@@ -96,7 +97,7 @@ struct Fragments {
     // rows 16 i .. of the wave's, k-slice ks (0, 1), of the half `half` bytes behind the first
     __device__ __forceinline__ void read(h8& f, int i, int ks, unsigned half) const {
         if (ALONG_K) {
-            f = *(lds_h8)(uintptr_t)(at[(i ^ (2 * ks)) & 3] + half + (unsigned)(i * 16 * BK * 2));
+            f = *(lds_h8)(uintptr_t)(at[ks] + half + (unsigned)(i * 16 * BK * 2));
         } else {
             typedef short s8 __attribute__((ext_vector_type(8)));
             const unsigned p = at[i] + half + (unsigned)(ks * 32 * ROWS * 2);
@@ -177,10 +178,10 @@ struct Wide : TileList<4 * QM, 4 * QN, NP> {
             2 * ((long)(rows - 1) * g.sAM + (long)(g.K1 - 1) * g.sAK1 + 1), 2 * HM * g.sAM, rows > HM);
         aim(s.rb, g.B + t.b0 * g.sBb[0] + t.b1 * g.sBb[1] + t.b2 * g.sBb[2] + (long)t.n0 * g.sBN + outer * g.sBK0,
             2 * ((long)(cols - 1) * g.sBN + (long)(g.K1 - 1) * g.sBK1 + 1), 2 * HN * g.sBN, cols > HN);
-        if (kc & 1) DTile<HM, true, NW>::offsets(s.oa, g.sAM, g.sAK1, wave, lane);
-        else DTile<HM, false, NW>::offsets(s.oa, g.sAM, g.sAK1, wave, lane);
-        if (kc & 2) DTile<HN, true, NW>::offsets(s.ob, g.sBN, g.sBK1, wave, lane);
-        else DTile<HN, false, NW>::offsets(s.ob, g.sBN, g.sBK1, wave, lane);
+        if (kc & 1) DTile<HM, true, NW, 16>::offsets(s.oa, g.sAM, g.sAK1, wave, lane);
+        else DTile<HM, false, NW, 16>::offsets(s.oa, g.sAM, g.sAK1, wave, lane);
+        if (kc & 2) DTile<HN, true, NW, 16>::offsets(s.ob, g.sBN, g.sBK1, wave, lane);
+        else DTile<HN, false, NW, 16>::offsets(s.ob, g.sBN, g.sBK1, wave, lane);
 #pragma unroll
         for (int i = 0; i < LA; ++i) s.oa[i] *= 2;
 #pragma unroll
