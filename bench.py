@@ -19,6 +19,7 @@ and its backward at [H=16,B=8,J=512,K=512], and every other memory-bound
 operator at the default workload's shapes) and prints their line instead.
 """
 import argparse
+import itertools
 import json
 import os
 import statistics
@@ -150,14 +151,6 @@ def algorithmic_work(B, L, H, E, relu_from_output=True, packed_masks=True, skip_
     w['attention'] = ('mfma', 2 * attn[0], 2 * 4 * bji + hbjk // 8, 2 * attn[0])
     w['attention-bwd-dQ'] = ('mfma', 3 * attn[0], 2 * 6 * bji + hbjk // 8, 2 * attn[0])
     w['attention-bwd-dKdV'] = ('mfma', 4 * attn[0], 2 * 6 * bji + hbjk // 8, 2 * attn[0])
-    # two products in one launch
-    w['dXlin1+dWlin1'] = ('mfma', 2 * ffn[0], 2 * ffn[1])
-    w['dXlin1+dWlin1+dWlin2'] = ('mfma', 3 * ffn[0], 3 * ffn[1])
-    w['dWlin1+dWlin2'] = ('mfma', 2 * ffn[0], 2 * ffn[1])
-    w['dXQKV-fused+dWQKV-fused'] = ('mfma', 2 * proj[0], 2 * proj[1])
-    w['dXout+dWout'] = ('mfma', 2 * outp[0], 2 * outp[1])
-    # the last launch of the backward pass with dWout's tiles in the places it leaves free
-    w['dXQKV-fused+dWQKV-fused+dWout'] = ('mfma', 2 * proj[0] + outp[0], 2 * proj[1] + outp[1])
     # lin1 with bias, ReLU and dropout in its epilogue: the product's flops, SB1 and LINW1 in, DROP2 out
     # the ReLU gate travels as one bit per element of DROP2: written by lin1's epilogue, read by dXlin2's
     w['lin1+bad'] = ('mfma', ffn[0], ffn[1] + tok * U // 8)
@@ -166,6 +159,13 @@ def algorithmic_work(B, L, H, E, relu_from_output=True, packed_masks=True, skip_
         w[n] = ('mfma',) + outp
     for n in ('lin1', 'lin2', 'dXlin2', 'dWlin2', 'dXlin1', 'dWlin1'):
         w[n] = ('mfma',) + ffn
+    # the products of the backward pass that may share a launch
+    for data, weights in (('dXlin1', ('dWlin1', 'dWlin2')), ('dXout', ('dWout', 'dWlin1', 'dWlin2')),
+                          ('dXQKV-fused', ('dWQKV-fused', 'dWout', 'dWlin1', 'dWlin2'))):
+        for n in range(1, len(weights) + 1):
+            for some in itertools.combinations(weights, n):
+                for members in ((data, *some), some):
+                    w['+'.join(members)] = ('mfma', sum(w[m][1] for m in members), sum(w[m][2] for m in members))
     return w
 
 

@@ -184,9 +184,11 @@ int sub_set_attention_mask(void* handle, const void* attn_mask, const char* layo
  * and the weight-gradient product next to it (encoder.cu:205-216 DLIN1_LINW1 and
  * DLINW1; :262-276 DXATT and DWKQV), which do not depend on one another, run as
  * one launch, their tiles in one list, where that is expected to be faster than a
- * launch each; a third product joins them on the same terms.  Results are unchanged
- * to rounding.  Profiling names: `dXlin1+dWlin1`, `dXlin1+dWlin1+dWlin2`,
- * `dXQKV-fused+dWQKV-fused`. */
+ * launch each.  Up to four weight gradients join a data gradient on the same terms,
+ * or wait for a later one: they feed nothing in this pass.  Results are unchanged
+ * to rounding.  Profiling names: the members', in the order dXlin1 | dXout |
+ * dXQKV-fused, dWQKV-fused, dWout, dWlin1, dWlin2 (`dXlin1+dWlin1`,
+ * `dXQKV-fused+dWQKV-fused+dWout+dWlin1+dWlin2`). */
 #define SUB_OPT_PAIR_PRODUCTS 5
 /* SUB_OPT_RELU_FROM_OUTPUT (default 1).  ReLU layers: the backward pass reads
  * the gate of dropout and ReLU off the forward output DROP2 = relu(LIN1) * mask,
@@ -224,11 +226,9 @@ int sub_set_attention_mask(void* handle, const void* attn_mask, const char* layo
  * LayerNorm-parameter gradients) runs in extra workgroups of the last pair of
  * products of the pass, in the places its tiles leave free on the CUs (two
  * workgroups each), instead of in a launch of its own (same code, same order of
- * additions: bit-identical).  Where that launch also has room for the tiles of
- * the dWout product, dWout runs there with its contraction in one piece and
- * dXout runs alone (DWO then sums its terms in another order than with the
- * option off: equal to rounding).  Profiling names: `dXout`,
- * `dXQKV-fused+dWQKV-fused+dWout`.  Needs SUB_OPT_PAIR_PRODUCTS and the
+ * additions: bit-identical).  dWout, where it would run there, is launched next to
+ * dXout with the option off (DWO then sums its terms in another order: equal to
+ * rounding).  Needs SUB_OPT_PAIR_PRODUCTS and the
  * in-register attention (whose kernels produce the DBKQV partials). */
 #define SUB_OPT_FINISH_IN_PAIR 7
 /* SUB_OPT_SIDE_JOBS (bit mask, default 1).  Bit 0: where the 256x256 tiles of

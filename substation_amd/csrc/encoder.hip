@@ -9,6 +9,7 @@
 #include <map>
 #include <algorithm>
 #include <mutex>
+#include <set>
 #include <string>
 #include <vector>
 
@@ -249,6 +250,9 @@ struct Handle {
     const void* gate_bits_at = nullptr;
     int form = 0;                     // what the last forward call left (FORM_*); see sub_forward_form
     int form_given = -1;              // the same of the forward call that the next backward call belongs to, if it was said
+    BackwardPlan plan;                // see backward_plan()
+    uint64_t plan_key = 0;
+    size_t plan_ws = 0;
     std::vector<ProfEntry> prof;
     size_t prof_used = 0;
     size_t prof_forward = 0;          // entries of the last forward call, kept by the backward call after it
@@ -422,6 +426,7 @@ void configure(Handle& h, const sub_config* c) {
     const float ps[4] = {c->p_softmax, c->p_resid1, c->p_act, c->p_resid2};
     for (float p : ps) if (!(p >= 0.f && p <= 1.f)) fail("sub_configure: dropout probability outside [0,1]");
     h.configured = false;
+    h.plan_key = 0;
     // a handle that is configured again forgets the attention mask of its old sizes
     // (the table of what the mask leaves to do was sized for them)
     if (h.mask_plan) {
@@ -651,45 +656,78 @@ GemmEpilogue addend_epilogue(const GemmPlan& p, const void* addend) {
     return e;
 }
 
-void run_gemm_pair(Handle& h, int id1, const void* A1, const void* B1, void* C1, const char* name1,
-                   const void* addend1, int id2, const void* A2, const void* B2, void* C2, const char* name2,
-                   const char* pair_name, FinishJobs* tail = nullptr, PairThird* third = nullptr) {
-    if (h.pair_products) {
-        ProfScope ps(h, pair_name);
-        const GemmPlan& p1 = h.gemm[id1];
-        const GemmPlan& p2 = h.gemm[id2];
-        ensure_gws(h, h.gws_need);
-        if (launch_gemm_pair(p1.shape, (const half_t*)A1, (const half_t*)B1, (half_t*)C1, p1.alpha,
-                             addend_epilogue(p1, addend1), p2.shape, (const half_t*)A2, (const half_t*)B2,
-                             (half_t*)C2, p2.alpha, GemmEpilogue{}, h.stream, h.gws, h.gws_floats, tail, third))
-            return;
-        ps.cancel();
-    }
-    run_gemm(h, id1, A1, B1, C1, name1, addend1);
-    run_gemm(h, id2, A2, B2, C2, name2);
+// The profiling name of a launch of several products (kept for the life of the process: a handful of them).
+const char* launch_name(const GemmJob* jobs, const GemmLaunch& l) {
+    static std::mutex lock;
+    static std::set<std::string> names;
+    std::string name;
+    for (int i = 0; i < l.n; ++i) name += (i ? "+" : "") + std::string(jobs[l.job[i]].name);
+    std::lock_guard<std::mutex> hold(lock);
+    return names.insert(name).first->c_str();
 }
 
-// Where a second weight gradient goes that is ready before a data gradient (1) and its weight gradient (2): into their
-// launch, into one with (2) where (1) shares no launch with either, or into one of its own.  Under weight orders that have
-// every operand of (1) contiguous along k (the shipped configuration of 96 sequences of 128) it never shares one: there
-// dWlin1 + dWlin2 as 256 tiles of 256 x 128 take 172 us where they took 2 x 111 as 256 of 128 x 128 each, dWQKV + dWout 123
-// where dWQKV took 104 and dWout 38 in dXout's launch.
-enum ThirdPlace { THIRD_ALONE, THIRD_IN_PAIR, THIRD_WITH_SECOND };
-ThirdPlace place_third(Handle& h, int id1, const void* A1, const void* B1, void* C1, const void* addend1, int id2,
-                       const void* A2, const void* B2, void* C2, const PairThird& third) {
-    if (!h.pair_products) return THIRD_ALONE;
-    const GemmPlan& p1 = h.gemm[id1];
-    const GemmPlan& p2 = h.gemm[id2];
+GemmJob gemm_job(Handle& h, int id, const void* A, const void* B, void* C, const char* name, const void* addend = nullptr) {
+    GemmJob j;
+    j.name = name; j.shape = &h.gemm[id].shape; j.alpha = h.gemm[id].alpha;
+    j.A = (const half_t*)A; j.B = (const half_t*)B; j.C = (half_t*)C;
+    j.ep = addend_epilogue(h.gemm[id], addend);
+    j.ep.any_split = true;
+    return j;
+}
+
+// The products of one place of the backward pass, as planned.
+void run_stage(Handle& h, const GemmJob* jobs, const GemmStage& s, FinishJobs* tail) {
+    for (int i = 0; i < s.n; ++i) {
+        const GemmLaunch& l = s.launch[i];
+        ProfScope ps(h, h.profiling ? launch_name(jobs, l) : nullptr);
+        if (l.form >= 0) {
+            launch_gemm_together(jobs, l, h.stream, h.gws, h.gws_floats, i + 1 == s.n ? tail : nullptr);
+        } else {
+            const GemmJob& j = jobs[l.job[0]];
+            launch_gemm(*j.shape, j.A, j.B, j.C, j.alpha, j.ep, h.stream, h.gws, h.gws_floats);
+        }
+    }
+}
+
+// The plan for these products, kept as long as what it was made from stays the same: the configuration, the options, which
+// operands are 16-byte aligned, and the scratch at hand.  (Making it takes 30 to 110 us.)
+const BackwardPlan& backward_plan(Handle& h, const GemmJob (&jobs)[7], bool late, bool fuse_dx) {
     ensure_gws(h, h.gws_need);
-    const half_t* a1 = (const half_t*)A1; const half_t* b1 = (const half_t*)B1;
-    const half_t* a2 = (const half_t*)A2; const half_t* b2 = (const half_t*)B2;
-    const GemmEpilogue e1 = addend_epilogue(p1, addend1), e2{};
-    if (gemm_pair_takes_third(p1.shape, a1, b1, (half_t*)C1, e1, p2.shape, a2, b2, (half_t*)C2, e2, h.gws, h.gws_floats, third))
-        return THIRD_IN_PAIR;
-    if (gemm_pair_ok(p1.shape, a1, b1, (half_t*)C1, e1, p2.shape, a2, b2, (half_t*)C2, e2, h.gws, h.gws_floats))
-        return THIRD_ALONE;
-    return gemm_pair_ok(p2.shape, a2, b2, (half_t*)C2, e2, *third.shape, third.A, third.B, third.C, e2, h.gws, h.gws_floats)
-               ? THIRD_WITH_SECOND : THIRD_ALONE;
+    uint64_t key = 1u | (h.pair_products ? 2u : 0u) | (late ? 4u : 0u) | (h.finish_in_pair ? 8u : 0u) | (fuse_dx ? 16u : 0u);
+    for (int i = 0; i < 7; ++i) {
+        const void* operand[4] = {jobs[i].A, jobs[i].B, jobs[i].C, jobs[i].ep.bias};
+        for (int k = 0; k < 4; ++k) key |= (reinterpret_cast<uintptr_t>(operand[k]) & 15 ? 1ull : 0ull) << (8 + 4 * i + k);
+    }
+    if (key == h.plan_key && h.gws_floats == h.plan_ws) return h.plan;
+    plan_backward_products(jobs, h.pair_products, late, h.gws_floats, h.plan);
+    if (!h.finish_in_pair) {
+        // dWout next to dXout (the others where and as they are with that option, so that they stay the same bit for bit)
+        bool was_late = false;
+        GemmStage& last = h.plan.stage[2];
+        for (int i = 0; i < last.n; ++i)
+            for (int k = 0; k < last.launch[i].n; ++k)
+                if (last.launch[i].job[k] == 4) {
+                    was_late = true;
+                    last.launch[i].drop(4);
+                    if (last.launch[i].n == 0) {
+                        for (--last.n; i < last.n; ++i) last.launch[i] = last.launch[i + 1];
+                        break;
+                    }
+                }
+        GemmStage& mid = h.plan.stage[1];
+        const int both[2] = {3, 4};
+        if (was_late && mid.n == 1 && mid.launch[0].n == 1) {
+            plan_gemm_stage(jobs, both, 2, h.pair_products, h.gws_floats, mid);
+        } else if (was_late) {
+            if (mid.n == kMaxProducts) fail("encoder_backward: too many launches");
+            mid.launch[mid.n] = GemmLaunch{};
+            mid.launch[mid.n].n = 1; mid.launch[mid.n].job[0] = 4;
+            ++mid.n;
+        }
+    }
+    h.plan_key = key;
+    h.plan_ws = h.gws_floats;
+    return h.plan;
 }
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -1303,6 +1341,23 @@ void backward(Handle& h, const BwdPtrs& t0) {
     struct Reset { Handle& h; ~Reset() { h.deferring = false; } } reset{h};
     void* const* W = t.W; void* const* F = t.F; void* const* D = t.Bk; void* const* DW = t.DW;
     bool fused = false;
+    // The products whose place is open.  A weight gradient feeds nothing in this pass: it runs next to a data gradient whose launch
+    // has room for it, or with the others at the end, where five products share one.  At 8 x 512, E 1024 (4096 rows) dXlin1 alone
+    // and one round of 256 tiles of 256 x 256 for all but dXout take 37 + 110 us, where dXlin1 with the two weight gradients of the
+    // feed-forward block (192 such tiles) took 98 and the rest (256 x 128) 71; at 96 x 128 90 + 36 + 297 for 94 + 36 + 171 + 121.
+    // DX = WKQV.DKKQQVV + DRESID1 in one pass where possible; DXATT is not written then
+    const bool fuse_dx = h.fuse_epilogues && h.gemm[G_DXQKV_RESID].ok && aligned16(D[DRESID1]) && aligned16(t.DX);
+    const GemmJob jobs[7] = {
+        gemm_job(h, G_DXLIN1, D[DLIN1], W[LINW1], D[DLIN1_LINW1], "dXlin1"),
+        gemm_job(h, G_DWLIN1, D[DLIN1], F[SB1], DW[LINW1], "dWlin1"),
+        gemm_job(h, G_DWLIN2, D[DLIN2], F[DROP2], DW[LINW2], "dWlin2"),
+        gemm_job(h, G_DXOUT, W[WO], D[DATT], D[DGAMMA], "dXout"),
+        gemm_job(h, G_DWOUT, F[GAMMA], D[DATT], DW[WO], "dWout"),
+        fuse_dx ? gemm_job(h, G_DXQKV_RESID, W[WKQV], D[DKKQQVV], t.DX, "dXQKV-fused", D[DRESID1])
+                : gemm_job(h, G_DXQKV, W[WKQV], D[DKKQQVV], D[DXATT], "dXQKV-fused"),
+        gemm_job(h, G_DWQKV, t.X, D[DKKQQVV], DW[WKQV], "dWQKV-fused"),
+    };
+    const BackwardPlan& plan = backward_plan(h, jobs, attn_fused, fuse_dx);
     // the backward passes around the two LayerNorms, each as one launch where possible
     auto ln2_backward = [&](LnBwdMode m) {
         return op_lnbwd(h, false, F[LN2], h.lf[LN2], W[S2], t.DY, h.lY, nullptr, h.lY, nullptr, h.lY,
@@ -1366,17 +1421,6 @@ void backward(Handle& h, const BwdPtrs& t0) {
     } else {
         run_gemm(h, G_DXLIN2, D[DLIN2], W[LINW2], D[DDROP2], "dXlin2");
     }
-    // dWlin2 waits for the launch of the pair behind it where its tiles fill the rounds of that one
-    PairThird dwlin2;
-    ThirdPlace dwlin2_at = THIRD_ALONE;
-    {
-        const GemmPlan& p3 = h.gemm[G_DWLIN2];
-        dwlin2.shape = &p3.shape; dwlin2.A = (const half_t*)D[DLIN2]; dwlin2.B = (const half_t*)F[DROP2];
-        dwlin2.C = (half_t*)DW[LINW2]; dwlin2.alpha = p3.alpha;
-        dwlin2_at = place_third(h, G_DXLIN1, D[DLIN1], W[LINW1], D[DLIN1_LINW1], nullptr, G_DWLIN1, D[DLIN1], F[SB1],
-                                DW[LINW1], dwlin2);
-    }
-    if (dwlin2_at == THIRD_ALONE) run_gemm(h, G_DWLIN2, D[DLIN2], F[DROP2], DW[LINW2], "dWlin2");
     if (!fuse_bdrlb) {
         ProfScope ps(h, "bdrlb");
         if (relu_from_output(h))
@@ -1388,16 +1432,7 @@ void backward(Handle& h, const BwdPtrs& t0) {
             op_bdrlb(h, D[DDROP2], h.lb[DDROP2], F[DROP2MASK], h.lf[DROP2MASK], F[LIN1], h.lf[LIN1],
                      D[DLIN1], h.lb[DLIN1], DW[LINB1], packed_act_mask(h));
     }
-    if (dwlin2_at == THIRD_WITH_SECOND) {
-        run_gemm(h, G_DXLIN1, D[DLIN1], W[LINW1], D[DLIN1_LINW1], "dXlin1");
-        run_gemm_pair(h, G_DWLIN1, D[DLIN1], F[SB1], DW[LINW1], "dWlin1", nullptr, G_DWLIN2, D[DLIN2], F[DROP2], DW[LINW2],
-                      "dWlin2", "dWlin1+dWlin2");
-    } else {
-        const bool later = dwlin2_at == THIRD_IN_PAIR;
-        run_gemm_pair(h, G_DXLIN1, D[DLIN1], W[LINW1], D[DLIN1_LINW1], "dXlin1", nullptr, G_DWLIN1, D[DLIN1], F[SB1], DW[LINW1],
-                      "dWlin1", later ? "dXlin1+dWlin1+dWlin2" : "dXlin1+dWlin1", nullptr, later ? &dwlin2 : nullptr);
-        if (later && !dwlin2.taken) run_gemm(h, G_DWLIN2, D[DLIN2], F[DROP2], DW[LINW2], "dWlin2");
-    }
+    run_stage(h, jobs, plan.stage[0], nullptr);
     fused = false;
     if (h.fuse_ln_backward) {
         ProfScope ps(h, "ebsb+blnrd2+baob");
@@ -1420,28 +1455,7 @@ void backward(Handle& h, const BwdPtrs& t0) {
             op_baob(h, D[DATT], h.lb[DATT], DW[BO]);
         }
     }
-    const bool fuse_dx = h.fuse_epilogues && h.gemm[G_DXQKV_RESID].ok && aligned16(D[DRESID1]) &&
-                         aligned16(t.DX);
-    // dWout (64 tiles of 128 x 128 at the bench workload, too few for a launch of its
-    // own without splitting its contraction) needs nothing but DATT and feeds nothing:
-    // when the last pair of products of the pass has room for its tiles it runs there,
-    // unsplit, and dXout runs alone here.
-    PairThird dwout;
-    ThirdPlace dwout_at = THIRD_ALONE;
-    if (h.finish_in_pair && attn_fused) {
-        const GemmPlan& p3 = h.gemm[G_DWOUT];
-        dwout.shape = &p3.shape; dwout.A = (const half_t*)F[GAMMA]; dwout.B = (const half_t*)D[DATT];
-        dwout.C = (half_t*)DW[WO]; dwout.alpha = p3.alpha;
-        dwout_at = fuse_dx ? place_third(h, G_DXQKV_RESID, W[WKQV], D[DKKQQVV], t.DX, D[DRESID1], G_DWQKV,
-                                         t.X, D[DKKQQVV], DW[WKQV], dwout)
-                           : place_third(h, G_DXQKV, W[WKQV], D[DKKQQVV], D[DXATT], nullptr, G_DWQKV, t.X,
-                                         D[DKKQQVV], DW[WKQV], dwout);
-    }
-    if (dwout_at != THIRD_ALONE)
-        run_gemm(h, G_DXOUT, W[WO], D[DATT], D[DGAMMA], "dXout");
-    else
-        run_gemm_pair(h, G_DXOUT, W[WO], D[DATT], D[DGAMMA], "dXout", nullptr,
-                      G_DWOUT, F[GAMMA], D[DATT], DW[WO], "dWout", "dXout+dWout");
+    run_stage(h, jobs, plan.stage[1], nullptr);
     half_t* KK = sub_q(F[KKQQVV], h, 0); half_t* QQ = sub_q(F[KKQQVV], h, 1); half_t* VV = sub_q(F[KKQQVV], h, 2);
     half_t* DKK = sub_q(D[DKKQQVV], h, 0); half_t* DQQ = sub_q(D[DKKQQVV], h, 1); half_t* DVV = sub_q(D[DKKQQVV], h, 2);
     bool attn_bias = false;
@@ -1494,25 +1508,7 @@ void backward(Handle& h, const BwdPtrs& t0) {
     // their own launch when every producer of those sums has been launched by now
     // (baib below would add one more).
     FinishJobs* tail = h.deferring && attn_bias && h.finish_in_pair ? &h.deferred : nullptr;
-    if (dwout_at == THIRD_WITH_SECOND) {
-        run_gemm(h, fuse_dx ? G_DXQKV_RESID : G_DXQKV, W[WKQV], D[DKKQQVV], fuse_dx ? t.DX : D[DXATT], "dXQKV-fused",
-                 fuse_dx ? D[DRESID1] : nullptr);
-        run_gemm_pair(h, G_DWQKV, t.X, D[DKKQQVV], DW[WKQV], "dWQKV-fused", nullptr, G_DWOUT, F[GAMMA], D[DATT], DW[WO], "dWout",
-                      "dWQKV-fused+dWout", tail);
-    } else {
-        const bool later = dwout_at == THIRD_IN_PAIR;
-        PairThird* third = later ? &dwout : nullptr;
-        const char* last_name = later ? "dXQKV-fused+dWQKV-fused+dWout" : "dXQKV-fused+dWQKV-fused";
-        if (fuse_dx) {
-            // DX = WKQV.DKKQQVV + DRESID1 in one pass; DXATT is not written
-            run_gemm_pair(h, G_DXQKV_RESID, W[WKQV], D[DKKQQVV], t.DX, "dXQKV-fused", D[DRESID1],
-                          G_DWQKV, t.X, D[DKKQQVV], DW[WKQV], "dWQKV-fused", last_name, tail, third);
-        } else {
-            run_gemm_pair(h, G_DXQKV, W[WKQV], D[DKKQQVV], D[DXATT], "dXQKV-fused", nullptr,
-                          G_DWQKV, t.X, D[DKKQQVV], DW[WKQV], "dWQKV-fused", last_name, tail, third);
-        }
-        if (later && !dwout.taken) run_gemm(h, G_DWOUT, F[GAMMA], D[DATT], DW[WO], "dWout");
-    }
+    run_stage(h, jobs, plan.stage[2], tail);
     if (!attn_bias) {
         ProfScope ps(h, "baib");
         op_baib(h, D[DKKQQVV], h.lb[DKKQQVV], DW[BKQV], h.lp[BKQV]);
@@ -2252,14 +2248,20 @@ int sub_op_einsum_pair(void* handle, const void* A1, const char* l_A1, const voi
         }
         size_t need = gemm_splitk_ws_floats(g1), need2 = gemm_splitk_ws_floats(g2);
         ensure_gws(h, need > need2 ? need : need2);
-        bool done = h.pair_products &&
-                    launch_gemm_pair(g1, (const half_t*)A1, (const half_t*)B1, (half_t*)C1, alpha1, ep1, g2,
-                                     (const half_t*)A2, (const half_t*)B2, (half_t*)C2, alpha2, GemmEpilogue{},
-                                     h.stream, h.gws, h.gws_floats);
-        if (!done) {
-            launch_gemm(g1, (const half_t*)A1, (const half_t*)B1, (half_t*)C1, alpha1, ep1, h.stream, h.gws, h.gws_floats);
-            launch_gemm(g2, (const half_t*)A2, (const half_t*)B2, (half_t*)C2, alpha2, GemmEpilogue{}, h.stream, h.gws,
-                        h.gws_floats);
+        GemmJob jobs[2];
+        jobs[0].shape = &g1; jobs[0].A = (const half_t*)A1; jobs[0].B = (const half_t*)B1; jobs[0].C = (half_t*)C1;
+        jobs[0].alpha = alpha1; jobs[0].ep = ep1;
+        jobs[1].shape = &g2; jobs[1].A = (const half_t*)A2; jobs[1].B = (const half_t*)B2; jobs[1].C = (half_t*)C2;
+        jobs[1].alpha = alpha2;
+        const int both[2] = {0, 1};
+        GemmStage plan;
+        plan_gemm_stage(jobs, both, 2, h.pair_products, h.gws_floats, plan);
+        const bool done = plan.n == 1;
+        if (done) {
+            launch_gemm_together(jobs, plan.launch[0], h.stream, h.gws, h.gws_floats, nullptr);
+        } else {
+            for (const GemmJob& j : jobs)
+                launch_gemm(*j.shape, j.A, j.B, j.C, j.alpha, j.ep, h.stream, h.gws, h.gws_floats);
         }
         if (paired) *paired = done ? 1 : 0;
     });

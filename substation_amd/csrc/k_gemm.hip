@@ -271,14 +271,6 @@ size_t gemm_splitk_ws_floats(const GemmShape& s) {
 
 namespace {
 
-// What launch_gemm_pair would launch: the two products as the kernel takes them and, when one is offered and
-// its place in the launch costs less than a launch of its own, a third one.
-struct PairSel {
-    TileProduct p[3];
-    TileChoice c;
-    int n = 0;
-};
-
 unsigned forms_for(const TileProduct* p, int n) {
     unsigned forms = kRingForms | 1u << TILE_256x256;
     for (int i = 0; i < n; ++i)
@@ -291,74 +283,119 @@ TileChoice choose_single(const TileProduct& p, size_t ws_floats) {
     return choose_tiles(&p, 1, forms_for(&p, 1), ws_floats);
 }
 
-bool pair_select(const GemmShape* const sh[2], const Canon cin[2], float* ws, size_t ws_floats, const PairThird* third,
-                 PairSel& out) {
-    constexpr double gap = 1.5;                          // between two launches (us)
-    auto take = [&](int i, const Canon& c, const GemmShape& s) {
-        out.p[i].a = c.a;
-        out.p[i].a.nbatch = s.batch();
-        return s.batch() > 0 && pick_kind(c, out.p[i].akc, out.p[i].bkc) == 1;
-    };
-    double alone = gap;
-    for (int i = 0; i < 2; ++i) {
-        if (!take(i, cin[i], *sh[i])) return false;
-        alone += choose_single(out.p[i], ws_floats).us;
-    }
-    out.n = 2;
-    out.c = choose_tiles(out.p, 2, forms_for(out.p, 2), ws_floats);
-    if (out.c.form < 0 || out.c.us > alone) return false;
-    if (third && third->shape &&
-        take(2, canonicalise(*third->shape, third->A, third->B, third->C, third->alpha, GemmEpilogue{}), *third->shape)) {
-        const TileChoice all = choose_tiles(out.p, 3, forms_for(out.p, 3), ws_floats);
-        if (all.form >= 0 && all.us < out.c.us + gap + choose_single(out.p[2], ws_floats).us) { out.n = 3; out.c = all; }
-    }
-    if (out.c.splits > 1) {
-        out.p[out.c.split].a.splits = out.c.splits;
-        out.p[out.c.split].a.partial = ws;
-    }
-    return true;
+constexpr double kGap = 1.5;                             // between two launches (us)
+
+// A job as the kernel takes it.
+bool take(const GemmJob& j, TileProduct& p) {
+    if (j.shape->batch() == 0 || j.shape->M == 0 || j.shape->N == 0) return false;
+    const Canon c = canonicalise(*j.shape, j.A, j.B, j.C, j.alpha, j.ep);
+    p.a = c.a;
+    p.a.nbatch = j.shape->batch();
+    return pick_kind(c, p.akc, p.bkc) == 1;
 }
 
 }  // namespace
 
-bool gemm_pair_ok(const GemmShape& s1, const half_t* A1, const half_t* B1, half_t* C1, const GemmEpilogue& ep1,
-                  const GemmShape& s2, const half_t* A2, const half_t* B2, half_t* C2, const GemmEpilogue& ep2,
-                  float* ws, size_t ws_floats) {
-    const GemmShape* sh[2] = {&s1, &s2};
-    const Canon c[2] = {canonicalise(s1, A1, B1, C1, 1.f, ep1), canonicalise(s2, A2, B2, C2, 1.f, ep2)};
-    PairSel sel;
-    return pair_select(sh, c, ws, ws_floats, nullptr, sel);
+void GemmLaunch::drop(int j) {
+    for (int i = 0; i < n; ++i)
+        if (job[i] == j) {
+            if (split == i) splits = 1;
+            if (split >= i && split > 0) --split;
+            for (--n; i < n; ++i) job[i] = job[i + 1];
+            return;
+        }
 }
 
-bool gemm_pair_takes_third(const GemmShape& s1, const half_t* A1, const half_t* B1, half_t* C1,
-                           const GemmEpilogue& ep1, const GemmShape& s2, const half_t* A2, const half_t* B2,
-                           half_t* C2, const GemmEpilogue& ep2, float* ws, size_t ws_floats,
-                           const PairThird& third) {
-    const GemmShape* sh[2] = {&s1, &s2};
-    const Canon c[2] = {canonicalise(s1, A1, B1, C1, 1.f, ep1), canonicalise(s2, A2, B2, C2, 1.f, ep2)};
-    PairSel sel;
-    return pair_select(sh, c, ws, ws_floats, &third, sel) && sel.n == 3;
-}
-
-// Two or three products in one launch.  What it gains over launches of their own: the last round of the one is filled with
+// Several products in one launch.  What it gains over launches of their own: the last round of the one is filled with
 // tiles of the next, and a workgroup's way into a tile overlaps with the one before (dXlin1 + dWlin1 at 4096 x 1024 x 4096
 // each: 78 -> 65 us against the launch of register-staged 256 x 128 tiles before, 75 for the two alone; at 2613 x 768 x 3072
-// 77 -> 36 us).  Returns false, having launched nothing, where the products do not share a launch or are expected to be
-// faster alone; the caller then launches them one after the other.
-bool launch_gemm_pair(const GemmShape& s1, const half_t* A1, const half_t* B1, half_t* C1, float alpha1,
-                      const GemmEpilogue& ep1, const GemmShape& s2, const half_t* A2, const half_t* B2,
-                      half_t* C2, float alpha2, const GemmEpilogue& ep2, hipStream_t st, float* ws,
-                      size_t ws_floats, FinishJobs* tail, PairThird* third) {
-    const GemmShape* sh[2] = {&s1, &s2};
-    const Canon cin[2] = {canonicalise(s1, A1, B1, C1, alpha1, ep1), canonicalise(s2, A2, B2, C2, alpha2, ep2)};
-    PairSel sel;
-    if (!pair_select(sh, cin, ws, ws_floats, third, sel)) return false;
+// 77 -> 36 us).
+double plan_gemm_stage(const GemmJob* jobs, const int* ids, int n, bool together, size_t ws_floats, GemmStage& out) {
+    TileProduct p[kMaxProducts];
+    bool ok[kMaxProducts], all = n > 1 && n <= kMaxProducts && together;
+    double alone[kMaxProducts], sum = 0.;
+    for (int i = 0; i < n; ++i) {
+        ok[i] = take(jobs[ids[i]], p[i]);
+        all = all && ok[i];
+        const bool small = ok[i] && (size_t)p[i].a.nbatch * p[i].a.M * p[i].a.N <= kSplitMaxOut;
+        alone[i] = ok[i] ? choose_single(p[i], small ? ws_floats : 0).us : 0.;
+        sum += alone[i] + (i ? kGap : 0.);
+    }
+    double best = sum;
+    out.n = n;
+    for (int i = 0; i < n; ++i) {
+        out.launch[i] = GemmLaunch{};
+        out.launch[i].n = 1; out.launch[i].job[0] = ids[i];
+    }
+    // jobs `from` .. of the list in one launch, those in front of it alone
+    auto share = [&](int from) {
+        const TileChoice c = choose_tiles(p + from, n - from, forms_for(p + from, n - from), ws_floats);
+        const double us = c.us + (from ? alone[0] + kGap : 0.);
+        if (c.form < 0 || us >= best) return;
+        best = us;
+        out.n = from + 1;
+        GemmLaunch& l = out.launch[from];
+        l.n = n - from;
+        for (int i = from; i < n; ++i) l.job[i - from] = ids[i];
+        l.form = c.form; l.split = c.split; l.splits = c.splits;
+    };
+    if (n > 2) {
+        bool rest = together;
+        for (int i = 1; i < n; ++i) rest = rest && ok[i];
+        if (rest) share(1);
+    }
+    if (all) {
+        const GemmStage before = out;
+        const double was = best;
+        out.launch[0] = GemmLaunch{};
+        share(0);
+        if (best == was) out = before;
+    }
+    return best;
+}
+
+void plan_backward_products(const GemmJob (&jobs)[7], bool together, bool late, size_t ws_floats, BackwardPlan& out) {
+    // what every place takes with every set of the weight gradients that may wait (bits 0, 1, 2: jobs 1, 2, 4)
+    GemmStage plan[3][8];
+    double us[3][8];
+    for (int at = 0; at < 3; ++at)
+        for (int set = 0; set < (at ? 8 : 4); ++set) {
+            if (!together && set != (at == 0 ? 3 : at == 1 ? 4 : 0)) continue;
+            int ids[kMaxProducts], n = 0;
+            ids[n++] = at == 0 ? 0 : at == 1 ? 3 : 5;
+            if (at == 2) ids[n++] = 6;
+            if (set & 4) ids[n++] = 4;
+            if (set & 1) ids[n++] = 1;
+            if (set & 2) ids[n++] = 2;
+            us[at][set] = plan_gemm_stage(jobs, ids, n, together, ws_floats, plan[at][set]);
+        }
+    double best = -1.;
+    for (int w1 = 0; w1 < (together ? 3 : 1); ++w1)
+        for (int w2 = 0; w2 < (together ? 3 : 1); ++w2)
+            for (int wo = 1; wo < (together && late ? 3 : 2); ++wo) {
+                int set[3] = {0, 0, 0};
+                set[w1] |= 1; set[w2] |= 2; set[wo] |= 4;
+                const double t = us[0][set[0]] + us[1][set[1]] + us[2][set[2]];
+                if (best >= 0. && t >= best) continue;
+                best = t;
+                for (int at = 0; at < 3; ++at) out.stage[at] = plan[at][set[at]];
+            }
+}
+
+void launch_gemm_together(const GemmJob* jobs, const GemmLaunch& l, hipStream_t st, float* ws, size_t ws_floats, FinishJobs* tail) {
+    TileProduct p[kMaxProducts];
+    for (int i = 0; i < l.n; ++i) {
+        if (!take(jobs[l.job[i]], p[i])) fail("gemm: these products do not share a launch");
+        if (l.splits > 1 && l.split == i) {
+            if ((size_t)p[i].a.nbatch * p[i].a.M * p[i].a.N * l.splits > ws_floats) fail("gemm: no room for the sums of a split product");
+            p[i].a.splits = l.splits;
+            p[i].a.partial = ws;
+        }
+    }
     // (none of the column sums in `tail` may be one that this launch itself contributes to)
-    launch_tiles(sel.p, sel.n, sel.c.form, tail, st);
-    if (sel.n == 3) third->taken = true;
-    if (sel.c.splits > 1) launch_splitk_reduce(sel.p[sel.c.split].a, st);
-    check_launch("gemm pair");
-    return true;
+    launch_tiles(p, l.n, l.form, tail, st);
+    if (l.splits > 1) launch_splitk_reduce(p[l.split].a, st);
+    check_launch("gemm group");
 }
 
 void launch_split_sums(const SplitSums& sums, half_t* C, long rows, long row, hipStream_t st) {

@@ -9,17 +9,21 @@ namespace {
 
 // The tiles there are, and what they take (us): a step of 64 k with few workgroups, with one on every second CU (two
 // share a CU: on every CU), and in every place; a launch with the way into and out of its first tile; a tile's way out
-// where all CUs are on theirs.  From products of 64 .. 8192 rows with 1 .. 256 steps.  256 x 256 is k_gemm_wide.
+// where all CUs are on theirs.  From products of 64 .. 12288 rows with 1 .. 256 steps, alone and up to five in a launch, on operands of
+// normal distribution that are used in turn.  256 x 256 is k_gemm_wide.
 struct Form { int bm, bn, per_cu; double few, half, full, once, out; };
 constexpr Form kForms[TILE_FORMS] = {
     {64, 64, 2, 0.20, 0.20, 0.38, 3.6, 1.6},
     {128, 64, 2, 0.29, 0.33, 0.59, 3.8, 2.0},
     {128, 128, 1, 0.33, 0.37, 0.47, 4.4, 2.0},
-    {256, 128, 1, 0.52, 0.54, 0.83, 5.9, 2.0},
-    {256, 256, 1, 1.00, 1.00, 1.42, 5.5, 4.3},
+    {256, 128, 1, 0.56, 0.62, 0.92, 5.9, 2.0},
+    {256, 256, 1, 1.02, 1.25, 1.47, 5.5, 4.3},
 };
+// Several products of more than a round of the smaller tiles: the workgroups drift apart, and share fewer lines of their L2
+// (4096 x 1024 x 4096 twice in tiles of 128 x 128: 75.5 us, 3 times 117 and once 38.5).
+constexpr double kDrift = 1.12;
 
-// The launch's rounds: its list has the longest contractions in front, and a round lasts as long as its longest tile.
+// One launch: its busiest workgroup.
 double launch_us(const long* len, const long* cnt, int n, const Form& F) {
     long total = 0;
     for (int i = 0; i < n; ++i) total += cnt[i];
@@ -27,17 +31,90 @@ double launch_us(const long* len, const long* cnt, int n, const Form& F) {
     const double x = (double)total / (128.0 * F.per_cu);
     const double step = x <= 1.0 ? F.few + (F.half - F.few) * x : F.per_cu > 1 || x >= 2.0 ? F.full : F.half + (F.full - F.half) * (x - 1.0);
     const double out = F.out * (total < places ? (double)total / (double)places : 1.0);
-    double t = F.once;
-    for (long id = 0; id < total; id += places) {
-        long at = id;
-        int i = 0;
-        while (at >= cnt[i]) at -= cnt[i++];
-        t += (double)len[i] * step + out;
-    }
-    return t;
+    if (n == 1) return F.once + (double)((total + places - 1) / places) * ((double)len[0] * step + out);
+    Schedule s;
+    const double drift = total > places && F.bm * F.bn <= 128 * 128 ? kDrift : 1.0;
+    return F.once + step * drift * schedule_tiles(len, cnt, n, std::min(total, places), out / step, s);
 }
 
 }  // namespace
+
+// The longest tiles first, each to the workgroups that have least to do.  Workgroups with as much to do as their neighbours are one
+// run, so that tiles next to each other in the list, which share operands, go to workgroups next to each other.  Up to the last
+// three rounds, or four, all of them take a tile in turn.  Four weight gradients of 192 tiles and 192 steps and a data gradient of 192
+// tiles and 48 steps (96 sequences of 128, E 1024) so end at step 192; with the rounds and the way back for the last of them that
+// were here before, a quarter of the workgroups had 192 + 48 to do.
+double schedule_tiles(const long* len, const long* cnt, int n, long workers, double out_steps, Schedule& s) {
+    struct Run { long worker, count, load; };                  // (loads in sixteenths of a step)
+    constexpr int kMaxRuns = 64;
+    Run run[kMaxRuns];
+    int runs = 1;
+    run[0] = Run{0, workers, 0};
+    auto cut = [&](int i, long count) {                        // run i behind its first `count` workgroups
+        if (count <= 0 || count >= run[i].count) return;
+        for (int k = runs++; k > i; --k) run[k] = run[k - 1];
+        run[i].count = count;
+        run[i + 1].worker += count; run[i + 1].count -= count;
+    };
+    auto give = [&](int i, long count, long load) {            // to the first `count` workgroups of run i
+        cut(i, count);
+        run[i].load += load;
+        int m = 0;
+        for (int k = 1; k < runs; ++k)
+            if (run[k].load == run[m].load) run[m].count += run[k].count;
+            else run[++m] = run[k];
+        runs = m + 1;
+    };
+    long total = 0;
+    for (int i = 0; i < n; ++i) total += cnt[i];
+    // lengths so mixed that this takes more parts than fit: whole rounds, what is left of the last one to the workgroups from the
+    // other end, each round as long as its longest tile
+    auto in_turn = [&]() {
+        s.rounds = (unsigned)(total / workers);
+        const unsigned rest = (unsigned)(total % workers);
+        s.n = rest ? 1 : 0;
+        s.part[0] = SchedulePart{(unsigned)workers - rest, (unsigned)(total - rest), rest};
+        double steps = 0.;
+        for (long id = 0; id < total; id += workers) {
+            long in = id;
+            int i = 0;
+            while (in >= cnt[i]) in -= cnt[i++];
+            steps += (double)len[i] + out_steps;
+        }
+        return steps;
+    };
+    s.rounds = (unsigned)std::max(0L, total / workers - 3);
+    s.n = 0;
+    long in_rounds = s.rounds * workers, at = 0, worker = 0;
+    for (int i = 0; i < n; ++i) {
+        const long load = 16 * len[i] + (long)(16. * out_steps);
+        long left = cnt[i];
+        while (left > 0) {
+            int r = 0;
+            if (in_rounds > 0) {
+                while (run[r].worker + run[r].count <= worker) ++r;
+                cut(r, worker - run[r].worker);
+                if (run[r].worker < worker) ++r;
+            } else {
+                for (int k = 1; k < runs; ++k)
+                    if (run[k].load < run[r].load) r = k;
+            }
+            const long c = std::min(left, run[r].count);
+            if (in_rounds > 0) {
+                in_rounds -= c;
+                worker = (worker + c) % workers;
+            } else {
+                if (s.n == kMaxParts || runs > kMaxRuns - 4) return in_turn();
+                s.part[s.n++] = SchedulePart{(unsigned)run[r].worker, (unsigned)at, (unsigned)c};
+            }
+            give(r, c, load);
+            left -= c; at += c;
+        }
+    }
+    long longest = 0;
+    for (int r = 0; r < runs; ++r) longest = std::max(longest, run[r].load);
+    return (double)longest / 16.;
+}
 
 bool tiles_take(const TileProduct& p) {
     const GemmArgs& a = p.a;
@@ -52,8 +129,8 @@ TileChoice choose_tiles(const TileProduct* p, int n, unsigned forms, size_t ws_f
     int k1, k2;
     if (n < 1 || n > kMaxProducts || !orientations(p, n, k1, k2)) return best;
     // the order of the launch's list: longest contraction first
-    int order[kMaxProducts] = {0, 1, 2};
-    std::sort(order, order + n, [&](int x, int y) { return steps_of(p[x].a, p[x].a.splits) > steps_of(p[y].a, p[y].a.splits); });
+    int order[kMaxProducts];
+    longest_first(p, n, order);
     const GemmArgs& longest = p[order[0]].a;
     // The longest contraction in parts: a reduction follows (about 3 us and a pass over the partial sums; charged as well
     // where the LayerNorm launch behind takes the parts themselves and none runs, so such products are split less than pays).
@@ -79,7 +156,10 @@ TileChoice choose_tiles(const TileProduct* p, int n, unsigned forms, size_t ws_f
     return best;
 }
 
-TileForm tile_form(int form) { return TileForm{kForms[form].bm, kForms[form].bn, kForms[form].per_cu}; }
+TileForm tile_form(int form) {
+    const Form& F = kForms[form];
+    return TileForm{F.bm, F.bn, F.per_cu, F.out / F.full};
+}
 
 // What the activation adds to a tile (us): for each pack of 8 outputs that a lane stores, its arithmetic (0.1, GELU 0.25) and,
 // forward, its keep bits: 0.2, and 0.13 on 256 x 256 tiles, which draw them between their matrix instructions, but not for nothing
@@ -120,7 +200,7 @@ template <int NP>
 static void launch_tiles_n(const TileProduct* p, int n, int form, FinishJobs* tail, hipStream_t st) {
     TileGroup<NP> G;
     int k1, k2;
-    list_tiles<NP>(G, p, n, kForms[form].bm, kForms[form].bn, 256L * kForms[form].per_cu, tail, k1, k2);
+    list_tiles<NP>(G, p, n, form, tail, k1, k2);
     launch_ring_as<NP, EPI_PLAIN>(G, form, k1, k2, G.workers + (unsigned)G.tail.n * G.tail_groups, st);
 }
 

@@ -9,7 +9,7 @@ template <int NP>
 void launch_plain(const TileProduct* p, int n, FinishJobs* tail, unsigned side_blocks, hipStream_t st) {
     TileGroup<NP> G;
     int k1, k2;
-    list_tiles<NP>(G, p, n, 256, 256, 256, tail, k1, k2);
+    list_tiles<NP>(G, p, n, TILE_256x256, tail, k1, k2);
     launch_wide_as<NP, EPI_PLAIN>(G, k1, k2, G.workers + (unsigned)G.tail.n * G.tail_groups + side_blocks, st);
 }
 

@@ -136,14 +136,21 @@ struct DTile {
 };
 
 
-// k_gemm_tiles.hip: products in tiles of four sizes, up to three in one launch.
+// k_gemm_tiles.hip: products in tiles of five sizes, up to five in one launch.
 enum { TILE_64x64 = 0, TILE_128x64, TILE_128x128, TILE_256x128, TILE_256x256, TILE_FORMS };
 constexpr unsigned kRingForms = (1u << TILE_256x256) - 1;
-constexpr int kMaxProducts = 3;
 struct TileProduct {
     GemmArgs a;                   // with splits (and, if more than one, partial) and nbatch set
     bool akc, bkc;                // operands contiguous along k
 };
+// Which workgroup takes which tiles of a launch's list (tiles of the same length next to each other, the longest in front):
+// `rounds` rounds of all workgroups, tile r n + l to workgroup l, then parts of the list that go to neighbouring workgroups.
+struct SchedulePart { unsigned worker, tile, count; };
+constexpr int kMaxParts = 12;
+struct Schedule { unsigned rounds = 0, n = 0; SchedulePart part[kMaxParts]; };
+// The schedule of cnt[i] tiles of len[i] steps, i < n, for `workers` workgroups, and the steps of the one that takes longest (a tile's
+// way out counted as out_steps of them).
+double schedule_tiles(const long* len, const long* cnt, int n, long workers, double out_steps, Schedule& s);
 struct TileChoice {
     int form = -1;                // none where the orientations do not share a launch
     double us = 0.;               // what the launch is expected to take
@@ -154,7 +161,8 @@ bool tiles_take(const TileProduct& p);                        // within the rang
 TileChoice choose_tiles(const TileProduct* p, int n, unsigned forms, size_t ws_floats);
 // `tail`: column sums of earlier launches, finished by workgroups behind the tiles (tail->n = 0 then).
 // Outputs of a tile of form f, and workgroups of that form on a CU.
-struct TileForm { int bm, bn, per_cu; };
+// out_steps: the way out of a tile in steps of it.
+struct TileForm { int bm, bn, per_cu; double out_steps; };
 TileForm tile_form(int form);
 // The best form for a product with an activation in its epilogue (-1: none), and its launch.
 int choose_act_form(const TileProduct& p);

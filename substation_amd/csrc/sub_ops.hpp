@@ -278,33 +278,39 @@ void launch_gemm(const GemmShape& g, const half_t* A, const half_t* B, half_t* C
 bool gemm_relu_dropout_ok(const GemmShape& g, const void* A, const void* B, const void* C, const GemmEpilogue& ep);
 // Rows of partial column sums that launch_gemm leaves with ep.gate (for a product that is ok).
 int gemm_colsum_rows(const GemmShape& g, const void* A, const void* B, const void* C, const GemmEpilogue& ep);
-// A third product offered to launch_gemm_pair: taken (and `taken` set) when its tiles in that launch are
-// expected to cost less than a launch of its own.
-struct PairThird {
+// A product that may share a launch with others.  None of them reads what another one writes.
+struct GemmJob {
+    const char* name = "";
     const GemmShape* shape = nullptr;
     const half_t* A = nullptr;
     const half_t* B = nullptr;
     half_t* C = nullptr;
     float alpha = 1.f;
-    bool taken = false;
+    GemmEpilogue ep;             // (an addend at most)
 };
-// Two independent contractions in one launch, each split as suits it (see GemmEpilogue::any_split).  Returns false,
-// having launched nothing, when the pair does not qualify (then call launch_gemm for each).  `tail` (optional):
-// deferred column sums of EARLIER launches, finished by extra workgroups of this
-// launch; tail->n is set to 0 when they were taken, else it is left as it was.
-bool launch_gemm_pair(const GemmShape& g1, const half_t* A1, const half_t* B1, half_t* C1, float alpha1,
-                      const GemmEpilogue& ep1, const GemmShape& g2, const half_t* A2, const half_t* B2,
-                      half_t* C2, float alpha2, const GemmEpilogue& ep2, hipStream_t st, float* ws = nullptr,
-                      size_t ws_floats = 0, FinishJobs* tail = nullptr, PairThird* third = nullptr);
-// Would launch_gemm_pair launch these two products as one?
-bool gemm_pair_ok(const GemmShape& g1, const half_t* A1, const half_t* B1, half_t* C1, const GemmEpilogue& ep1,
-                  const GemmShape& g2, const half_t* A2, const half_t* B2, half_t* C2, const GemmEpilogue& ep2,
-                  float* ws, size_t ws_floats);
-// Would launch_gemm_pair with these two products take `third` along?
-bool gemm_pair_takes_third(const GemmShape& g1, const half_t* A1, const half_t* B1, half_t* C1,
-                           const GemmEpilogue& ep1, const GemmShape& g2, const half_t* A2, const half_t* B2,
-                           half_t* C2, const GemmEpilogue& ep2, float* ws, size_t ws_floats,
-                           const PairThird& third);
+constexpr int kMaxProducts = 5;  // of one launch
+// Jobs of one launch: their tiles of form `form`, the contraction of member `split` in `splits` parts.  form < 0: one job, launched
+// by launch_gemm.
+struct GemmLaunch {
+    int n = 0, job[kMaxProducts] = {0, 0, 0, 0, 0};
+    int form = -1, split = 0, splits = 1;
+    void drop(int j);            // without job j (the others as they were)
+};
+struct GemmStage {
+    int n = 0;
+    GemmLaunch launch[kMaxProducts];
+};
+// The fastest of: jobs ids[0 .. n - 1] in one launch, the first apart from the rest, each of them alone.  What it is expected
+// to take (us).  together: whether any may share a launch at all.
+double plan_gemm_stage(const GemmJob* jobs, const int* ids, int n, bool together, size_t ws_floats, GemmStage& out);
+// One launch of more than one product, or of one whose form is set.  `tail` (optional): deferred column sums of EARLIER launches,
+// finished by extra workgroups of this launch; tail->n is set to 0 when they were taken, else it is left as it was.
+void launch_gemm_together(const GemmJob* jobs, const GemmLaunch& l, hipStream_t st, float* ws, size_t ws_floats, FinishJobs* tail);
+// Seven products of a backward pass, in three places between which other operators stand: a data gradient opens each of them
+// (jobs 0, 3, 5), and the weight gradients run where that is expected to be fastest, from the place on where their operands are
+// there: jobs 1 and 2 in any, job 4 in the second or (late) the third, job 6 in the third.
+struct BackwardPlan { GemmStage stage[3]; };
+void plan_backward_products(const GemmJob (&jobs)[7], bool together, bool late, size_t ws_floats, BackwardPlan& out);
 // Writes the output of a product that was left as the sums of its splits.
 void launch_split_sums(const SplitSums& sums, half_t* C, long rows, long row, hipStream_t st);
 // Scratch (in floats) that launch_gemm can make use of for this shape; 0 if none.

@@ -108,7 +108,8 @@ struct Ring : TileList<32 * TM * WM, 32 * TN * WN, NP> {
         unsigned round = 0, steps = 0;
         auto next_tile = [&]() {
             Tile t;
-            more = tile_of(G, l, n, round++, t);
+            more = tile_of(G, l, n, round, t);
+            ++round;
             if (!more) { oa.left = oa.step = ob.left = ob.step = full_a = full_b = 0; left = 0x7fffffff; return; }
             Args& g = G.g[t.p];
             per_k1 = (g.K1 + BK - 1) / BK;
@@ -451,7 +452,7 @@ struct Ring : TileList<32 * TM * WM, 32 * TN * WN, NP> {
         unsigned r = 0;
         int stage = 0;
         Tile t;
-        bool any = tile_of(G, l, n, 0, t);
+        bool any = tile_of(G, l, n, r, t);
         lds_fence(ring_at);
         __builtin_amdgcn_s_barrier();
         lds_fence(ring_at);
@@ -473,6 +474,7 @@ __global__ __launch_bounds__((WM * WN + NL) * 64) void k_gemm_ring(TileGroup<NP>
 #define SUB_RING(...)                                                                                                        \
     do {                                                                                                                     \
         if constexpr (NP > 1) if (k1 == 1 && k2 == 0) { hipLaunchKernelGGL((k_gemm_ring<__VA_ARGS__, NP, 1, 0, EPI>), grid, block, 0, st, G); break; } \
+        if constexpr (NP > 1) if (k1 == 3 && k2 == 0) { hipLaunchKernelGGL((k_gemm_ring<__VA_ARGS__, NP, 3, 0, EPI>), grid, block, 0, st, G); break; } \
         if (k1 == 3) hipLaunchKernelGGL((k_gemm_ring<__VA_ARGS__, NP, 3, 3, EPI>), grid, block, 0, st, G);                    \
         else if (k1 == 1) hipLaunchKernelGGL((k_gemm_ring<__VA_ARGS__, NP, 1, 1, EPI>), grid, block, 0, st, G);               \
         else if constexpr (EPI == EPI_PLAIN) {                                                                               \

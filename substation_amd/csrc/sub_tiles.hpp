@@ -151,6 +151,7 @@ struct TileGroup {
     unsigned end[NP];                 // products' tiles in the launch's list: those of product p end at end[p]
     unsigned second[NP];              // operands read the way of K2 (see k_gemm_ring)
     unsigned n = 0, workers = 0;      // products; workgroups that take tiles
+    Schedule when;                    // (of several products)
     unsigned tail_groups = 0;
     typename std::conditional<NP == 1, NoJobs, FinishJobs>::type tail;     // column sums of earlier launches, finished by the workgroups behind those
 };
@@ -174,8 +175,9 @@ struct TileList {
         t.p = 0;
         unsigned first = 0;
         if constexpr (NP > 1) {
-            if (G.n > 1 && id >= G.end[0]) { t.p = 1; first = G.end[0]; }
-            if (G.n > 2 && id >= G.end[1]) { t.p = 2; first = G.end[1]; }
+#pragma unroll
+            for (unsigned i = 1; i < NP; ++i)
+                if (G.n > i && id >= G.end[i - 1]) { t.p = (int)i; first = G.end[i - 1]; }
         }
         Args& g = G.g[t.p];
         id -= first;
@@ -203,11 +205,24 @@ struct TileList {
         const unsigned rr = id - grp * GM * tiles_n, col = gsz == GM ? rr / GM : rr / gsz;
         t.m0 = (int)((first_m + rr - col * gsz) * BM); t.n0 = (int)(col * BN);
     }
-    // The r-th tile of logical workgroup l of n: rounds of n; what is left of the last one goes to the workgroups from the
-    // other end (the list starts with the longest contractions).
-    static __device__ __forceinline__ bool tile_of(Group& G, unsigned l, unsigned n, unsigned r, Tile& t) {
-        const unsigned total = NP == 1 ? G.end[0] : G.end[G.n - 1], id = r * n + ((r + 1) * n <= total ? l : n - 1 - l);
-        if (id >= total) return false;
+    // The tile of logical workgroup l of n in entry r of the launch's schedule, or in the next one that has any for it (r is moved
+    // there).  One product: rounds of n, what is left of the last one goes to the workgroups from the other end.
+    static __device__ __forceinline__ bool tile_of(Group& G, unsigned l, unsigned n, unsigned& r, Tile& t) {
+        unsigned id;
+        if constexpr (NP == 1) {
+            const unsigned total = G.end[0];
+            id = r * n + ((r + 1) * n <= total ? l : n - 1 - l);
+            if (id >= total) return false;
+        } else if (r < G.when.rounds) {
+            id = r * n + l;
+        } else {
+            for (;; ++r) {
+                const unsigned s = r - G.when.rounds;
+                if (s >= G.when.n) return false;
+                const unsigned j = l - G.when.part[s].worker;         // (wraps around below the first)
+                if (j < G.when.part[s].count) { id = G.when.part[s].tile + j; break; }
+            }
+        }
         locate(G, id, t);
         return true;
     }
@@ -225,27 +240,38 @@ inline bool orientations(const TileProduct* p, int n, int& k1, int& k2) {
     for (int i = 0; i < n; ++i) seen |= 1 << ((p[i].akc ? 1 : 0) | (p[i].bkc ? 2 : 0));
     for (int k = 0; k < 4; ++k)
         if (seen == 1 << k) { k1 = k2 = k; return true; }
-    k1 = 1; k2 = 0;
-    return seen == 3;
+    k1 = seen == 9 ? 3 : 1; k2 = 0;
+    return seen == 3 || seen == 9;
 }
 
-// The list of a launch in tiles of bm x bn for `places` workgroups, longest contractions first; `tail`: see launch_tiles.
+// The indices of n products, longest contraction first.
+inline void longest_first(const TileProduct* p, int n, int (&order)[kMaxProducts]) {
+    for (int i = 0; i < n; ++i) order[i] = i;
+    std::stable_sort(order, order + n, [&](int x, int y) { return steps_of(p[x].a, p[x].a.splits) > steps_of(p[y].a, p[y].a.splits); });
+}
+
+// The list of a launch in tiles of form `form`, longest contractions first; `tail`: see launch_tiles.
 template <int NP>
-void list_tiles(TileGroup<NP>& G, const TileProduct* p, int n, int bm, int bn, long places, FinishJobs* tail, int& k1, int& k2) {
-    int order[kMaxProducts] = {0, 1, 2};
+void list_tiles(TileGroup<NP>& G, const TileProduct* p, int n, int form, FinishJobs* tail, int& k1, int& k2) {
+    const TileForm f = tile_form(form);
+    const int bm = f.bm, bn = f.bn;
+    const long places = 256L * f.per_cu;
+    int order[kMaxProducts];
     if (n < 1 || n > NP || !orientations(p, n, k1, k2)) fail("gemm: these products do not share a launch");
-    std::sort(order, order + n, [&](int x, int y) { return steps_of(p[x].a, p[x].a.splits) > steps_of(p[y].a, p[y].a.splits); });
-    long total = 0;
+    longest_first(p, n, order);
+    long total = 0, len[NP], cnt[NP];
     for (int i = 0; i < n; ++i) {
         const TileProduct& q = p[order[i]];
         G.g[i] = q.a;
         G.second[i] = ((q.akc ? 1 : 0) | (q.bkc ? 2 : 0)) != k1;
-        total += tiles_of(q.a, q.a.splits, bm, bn);
+        len[i] = steps_of(q.a, q.a.splits);
+        total += cnt[i] = tiles_of(q.a, q.a.splits, bm, bn);
         if (total > 0x7fffffffL) fail("gemm: too many tiles");
         G.end[i] = (unsigned)total;
     }
     G.n = (unsigned)n;
     G.workers = (unsigned)std::min(total, places);
+    if constexpr (NP > 1) schedule_tiles(len, cnt, n, G.workers, f.out_steps, G.when);
     if constexpr (NP > 1)
         if (tail && tail->n > 0) {
             const long groups = finish_groups(*tail);

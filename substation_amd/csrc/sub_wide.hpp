@@ -160,7 +160,9 @@ struct Wide : TileList<4 * QM, 4 * QN, NP> {
     static __device__ __forceinline__ void open(Group& G, Stream& s, unsigned l, unsigned n, int wave, int lane) {
         Tile t;
         s.ka = s.kb = 0;
-        if (!tile_of(G, l, n, s.round++, t)) {
+        const bool more = tile_of(G, l, n, s.round, t);
+        ++s.round;
+        if (!more) {
             // nothing more: loads out of range, so that the count of loads in flight goes on
             s.ra[0][2] = s.ra[1][2] = s.rb[0][2] = s.rb[1][2] = 0u;
             s.step_a = s.step_b = 0;
@@ -614,7 +616,7 @@ struct Wide : TileList<4 * QM, 4 * QN, NP> {
         __builtin_amdgcn_s_barrier();
         Tile t;
         unsigned r = 0, set = 0;
-        bool landed = false, any = tile_of(G, l, n, 0, t);
+        bool landed = false, any = tile_of(G, l, n, r, t);
         while (any) {
             if (K1 == K2 || !G.second[t.p]) any = consume<K1 & 1, (K1 >> 1)>(G, s, l, n, r, t, set, landed, lds, slab, wave, lane);
             else any = consume<K2 & 1, (K2 >> 1)>(G, s, l, n, r, t, set, landed, lds, slab, wave, lane);
@@ -634,6 +636,7 @@ template <int NP, int EPI>
 void launch_wide_as(const TileGroup<NP>& G, int k1, int k2, unsigned blocks, hipStream_t st) {
     const dim3 grid(blocks), block(256);
     if constexpr (NP > 1) if (k1 == 1 && k2 == 0) { hipLaunchKernelGGL((k_gemm_wide<64, 64, NP, 1, 0, EPI>), grid, block, 0, st, G); return; }
+    if constexpr (NP > 1) if (k1 == 3 && k2 == 0) { hipLaunchKernelGGL((k_gemm_wide<64, 64, NP, 3, 0, EPI>), grid, block, 0, st, G); return; }
     if (k1 == 3) hipLaunchKernelGGL((k_gemm_wide<64, 64, NP, 3, 3, EPI>), grid, block, 0, st, G);
     else if (k1 == 2) hipLaunchKernelGGL((k_gemm_wide<64, 64, NP, 2, 2, EPI>), grid, block, 0, st, G);
     else if (k1 == 1) hipLaunchKernelGGL((k_gemm_wide<64, 64, NP, 1, 1, EPI>), grid, block, 0, st, G);

@@ -139,8 +139,12 @@ class LayerTimer:
                 self._lib.check(lib.sub_encoder_backward(handle.ptr, bp, nb), 'encoder_backward')
                 prof = handle.profile_read()      # both passes; no host wait between them
                 if it >= self.warmup:
+                    step = {}
                     for name, ms in prof:
-                        times.setdefault(name, []).append(ms * 1e-3)
+                        op = _og.operator_of(name)
+                        step[op] = step.get(op, 0.0) + ms * 1e-3
+                    for op, sec in step.items():
+                        times.setdefault(op, []).append(sec)
         finally:
             handle.close()
         self.measurements += 1

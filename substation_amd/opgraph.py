@@ -78,12 +78,11 @@ OP_TENSORS = {name: tensors for name, _, tensors in OPERATORS}
 #: which of them run depends on the layouts of the whole group's tensors.
 ALTERNATIVES = [
     ('QKV-fused', 'aib'),
-    # dWout runs inside the last launch of the pass when that has room for its tiles
-    ('dXQKV-fused+dWQKV-fused+dWout', 'dXQKV-fused+dWQKV-fused', 'dXQKV-fused',
-     'dWQKV-fused+dWout', 'dWQKV-fused', 'bei', 'dXout+dWout', 'dXout', 'dWout', 'colfinish'),
     ('lin1+bad', 'lin1', 'bad'),
-    # (dWlin2 may wait for the launch of the pair behind it)
-    ('dXlin2+bdrlb', 'dXlin2', 'bdrlb', 'dXlin1+dWlin1+dWlin2', 'dXlin1+dWlin1', 'dXlin1', 'dWlin1+dWlin2',
+    # (the weight gradients run in the launch of a data gradient that has room for them, or together in the last one)
+    ('dXQKV-fused+dWQKV-fused+dWout', 'dXQKV-fused+dWQKV-fused', 'dXQKV-fused',
+     'dWQKV-fused+dWout', 'dWQKV-fused', 'bei', 'dXout+dWout', 'dXout', 'dWout', 'colfinish',
+     'dXlin2+bdrlb', 'dXlin2', 'bdrlb', 'dXlin1+dWlin1+dWlin2', 'dXlin1+dWlin1', 'dXlin1', 'dWlin1+dWlin2',
      'dWlin1', 'dWlin2'),
     ('attention', 'QKT+softmax', 'QKT', 'softmax', 'gamma'),
     ('attention-bwd-dQ', 'attention-bwd-dKdV', 'dX2gamma', 'dX1gamma+bs', 'dX1gamma', 'bs', 'dX1QKT', 'dX2QKT',
@@ -103,6 +102,13 @@ GROUP_ALSO_DEPENDS = {
     'attention-bwd-dQ': _ATTENTION_DECIDERS,
     'dXQKV-fused+dWQKV-fused+dWout': _ATTENTION_DECIDERS + ('BKQV',),
 }
+
+
+def operator_of(launch):
+    """The operator that a launch is timed as.  Of the launches of several products only some are operators of their own; the others
+    count as their first member, whose group has the rest in it."""
+    return launch if launch in OP_TENSORS else launch.split('+')[0]
+
 
 #: the 18 contractions (pytorch_module/encoder.cu:90-276; canonical list
 #: tc_profiling/einsum_perms.py:367-394): name -> (A, B, C) operand names, where

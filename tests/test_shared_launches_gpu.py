@@ -1,0 +1,52 @@
+"""Launches of several products: tiles of up to five of them in one schedule, against the products launched one by one."""
+import pytest
+import torch
+
+from tests.helpers import assert_close
+
+pytestmark = pytest.mark.gpu
+
+ALL = 'dXQKV-fused+dWQKV-fused+dWout+dWlin1+dWlin2'
+
+
+# (B, L, H, E), layouts, a launch that has to be among them (None: whichever)
+CASES = [
+    ((1, 16, 2, 128), None, None),                   # fewer tiles than one product's
+    ((3, 43, 4, 256), None, None),                   # rows that are a multiple of nothing
+    ((5, 201, 12, 768), None, None),                 # remainders of every tile size
+    ((4, 512, 16, 1024), None, ALL),
+    ((8, 512, 16, 1024), None, ALL),                 # 256 x 256 tiles, a round of them exactly
+    ((48, 128, 16, 1024), 'bert-b96-l128-h16-e1024', ALL),     # data gradients with both operands along k
+    ((2, 1024, 32, 2048), None, None),               # several rounds
+    ((1, 2048, 32, 4096), None, None),               # whole rounds in front of the parts of the schedule
+]
+
+
+@pytest.mark.parametrize('dims,which,launch', CASES)
+def test_products_that_share_a_launch_give_what_they_give_alone(dims, which, launch):
+    from substation_amd import Encoder, layouts as L
+    B, Ls, H, E = dims
+    lay = L.mi355x_layouts(which)
+    g = torch.Generator('cuda').manual_seed(3)
+    sizes = L.sizes_map(B, Ls, H, E)
+    X, DY = (torch.randn(L.shape_of(lay[k][1], sizes), generator=g, device='cuda').half() for k in ('input', 'output'))
+    grads = []
+    for shared in (0, 1):
+        torch.manual_seed(0)
+        with torch.device('cuda'):
+            enc = Encoder('unused', B, Ls, H, E, lay, torch.float16, 0.1, 0.1, 0.1, 0.1, seed=7, activation='gelu', profiling=True)
+        with torch.no_grad():
+            for q in enc.parameters():
+                q.mul_(0.1)
+        enc._handle.set_option(5, shared)
+        enc.set_rng(7, 0)
+        x = X.clone().requires_grad_()
+        enc(x).backward(DY)
+        torch.cuda.synchronize()
+        names = [n for n, _ in enc.profile()]
+        assert shared or not any('+dW' in n for n in names)
+        assert not (shared and launch) or launch in names, names
+        grads.append({'X': x.grad, **{n: q.grad for n, q in enc.named_parameters()}})
+    for name, alone in grads[0].items():
+        # (sums in another order, rounded to fp16, and what follows from them: within the bound of any product here)
+        assert_close(grads[1][name].float().cpu().numpy(), alone.float().cpu().numpy(), tol=1e-2, name=name)
