@@ -209,19 +209,36 @@ void launch_splitk_reduce(const GemmArgs& a, hipStream_t st) {
 constexpr size_t kSplitMaxOut = 2u << 20;     // largest output (elements) whose contraction is split
 constexpr long kSplitTarget = 256;            // workgroups a split product aims for (the CUs of the device)
 
-// How many ways to split k so that a small output still fills the chip: the
-// weight-gradient products have few output tiles and a long contraction.
-int pick_splits(const GemmArgs& a, long batch, size_t ws_floats) {
-    const long tiles = (long)((a.M + 127) / 128) * ((a.N + 127) / 128) * batch;
-    const int nkt = a.K0 * ((a.K1 + BK - 1) / BK);
-    // one workgroup per CU: a second, partly filled round costs more than it gains
-    int splits = (int)(kSplitTarget / tiles);
-    if (splits > 8) splits = 8;
-    while (splits > 1 && nkt / splits < 8) --splits;
-    const size_t need = (size_t)batch * a.M * a.N;          // floats per split
-    while (splits > 1 && need * splits > ws_floats) --splits;
-    if (a.N % 4 != 0) splits = 1;
-    return splits < 1 ? 1 : splits;
+// Scratch (floats) for the sums of a product's splits.  Only small outputs are split (measured: beyond ~2M elements the fp32
+// partial traffic costs more than the extra workgroups gain).
+size_t split_floats(long M, long N, long batch) {
+    const size_t per = (size_t)batch * M * N;
+    const long tiles = ((M + 127) / 128) * ((N + 127) / 128) * batch;
+    if (tiles > kSplitTarget / 2 || per > kSplitMaxOut) return 0;
+    return per * (size_t)std::min(kSplitTarget / tiles, 8L);
+}
+
+unsigned forms_for(const TileProduct* p, int n) {
+    unsigned forms = kRingForms | 1u << TILE_256x256;
+    for (int i = 0; i < n; ++i)
+        if (!wide_takes(p[i])) forms = kRingForms;
+    return forms;
+}
+
+// What a product takes in a launch of its own.
+TileChoice choose_single(const TileProduct& p, size_t ws_floats, double reduce_us = kReduceLaunch) {
+    return choose_tiles(&p, 1, forms_for(&p, 1), ws_floats, reduce_us);
+}
+
+// In how many parts a forward pass sums a product, by its shape and the order of its operands alone: as is fastest, within the
+// scratch that every caller brings.  A product that does not widen its rows has a LayerNorm behind it in the layers, which takes the
+// parts in place of their sum (3.9 us without, 5.7 with six parts of 64 x 768, 0.6 of that for their bytes).  (Splits to fill the CUs as far as 8 steps each were left of it, which was the rule here before,
+// cost more than they gave where the fp32 sums are many: us of lin2 and the LayerNorm behind it, 2613 x 768 x 3072 in two parts
+// 32 and in one 29, 1024 x 768 x 3072 in five 21.4 and in one 19.9; and a product of 512 x 4096 x 1024 in two parts had no activation
+// in its epilogue, 28 with its activation and now 14.)
+int forward_splits(const TileProduct& p) {
+    const bool widens = p.a.N > (long)p.a.K0 * p.a.K1;
+    return choose_single(p, split_floats(p.a.M, p.a.N, p.a.nbatch), widens ? kReduceLaunch : 1.4).splits;
 }
 
 }  // namespace
@@ -242,7 +259,7 @@ static int act_form(const GemmShape& s, const void* A, const void* B, const void
     p.a = c.a; p.a.nbatch = 1;
     // A small output whose contraction a forward pass splits keeps the order of its sums, with or without an activation behind
     // it: split, and the operators.
-    if ((size_t)s.M * s.N <= kSplitMaxOut && pick_splits(c.a, 1, SIZE_MAX) > 1) return -1;
+    if (forward_splits(p) > 1) return -1;
     return choose_act_form(p);
 }
 
@@ -259,29 +276,10 @@ int gemm_colsum_rows(const GemmShape& s, const void* A, const void* B, const voi
 }
 
 size_t gemm_splitk_ws_floats(const GemmShape& s) {
-    // only small outputs are split (measured: beyond ~2M elements the fp32 partial
-    // traffic costs more than the extra workgroups gain)
-    size_t per = (size_t)s.batch() * s.M * s.N;
-    long tiles = ((s.M + 127) / 128) * ((s.N + 127) / 128) * s.batch();
-    if (tiles > kSplitTarget / 2 || per > kSplitMaxOut) return 0;
-    size_t splits = kSplitTarget / tiles;
-    if (splits > 8) splits = 8;
-    return per * splits;
+    return split_floats(s.M, s.N, s.batch());
 }
 
 namespace {
-
-unsigned forms_for(const TileProduct* p, int n) {
-    unsigned forms = kRingForms | 1u << TILE_256x256;
-    for (int i = 0; i < n; ++i)
-        if (!wide_takes(p[i])) forms = kRingForms;
-    return forms;
-}
-
-// What a product takes in a launch of its own.
-TileChoice choose_single(const TileProduct& p, size_t ws_floats) {
-    return choose_tiles(&p, 1, forms_for(&p, 1), ws_floats);
-}
 
 constexpr double kGap = 1.5;                             // between two launches (us)
 
@@ -423,9 +421,8 @@ void launch_gemm(const GemmShape& s, const half_t* A, const half_t* B, half_t* C
             check_launch("gemm");
             return;
         }
-        // A forward pass sums in an order that depends on the product's shape alone (pick_splits), whatever the tile.
         const bool small = ws && (size_t)batch * c.a.M * c.a.N <= kSplitMaxOut;
-        if (small && !ep.any_split) tp.a.splits = pick_splits(c.a, batch, ws_floats);
+        if (small && !ep.any_split) tp.a.splits = forward_splits(tp);
         const TileChoice choice = choose_single(tp, small && ep.any_split ? ws_floats : 0);
         unsigned side_blocks = 0;
         if (side) side->tiles_done = 0;

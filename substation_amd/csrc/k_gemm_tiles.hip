@@ -124,7 +124,7 @@ bool tiles_take(const TileProduct& p) {
     return la < (1L << 30) && lb < (1L << 30) && lc < (1L << 30) && lt < (1L << 30);
 }
 
-TileChoice choose_tiles(const TileProduct* p, int n, unsigned forms, size_t ws_floats) {
+TileChoice choose_tiles(const TileProduct* p, int n, unsigned forms, size_t ws_floats, double reduce_us) {
     TileChoice best;
     int k1, k2;
     if (n < 1 || n > kMaxProducts || !orientations(p, n, k1, k2)) return best;
@@ -132,13 +132,13 @@ TileChoice choose_tiles(const TileProduct* p, int n, unsigned forms, size_t ws_f
     int order[kMaxProducts];
     longest_first(p, n, order);
     const GemmArgs& longest = p[order[0]].a;
-    // The longest contraction in parts: a reduction follows (about 3 us and a pass over the partial sums; charged as well
-    // where the LayerNorm launch behind takes the parts themselves and none runs, so such products are split less than pays).
+    // The longest contraction in parts: a reduction follows (a launch of about 3 us, or less in a launch that takes the parts
+    // themselves, and a pass over the partial sums).
     const bool free_split = ws_floats > 0 && longest.splits == 1 && longest.N % 4 == 0;
     for (int s = 1; s <= (free_split ? 8 : 1); ++s) {
         const size_t partial = (size_t)longest.nbatch * longest.M * longest.N * s;
         if (s > 1 && (steps_of(longest, s) < 4 || partial > ws_floats)) break;
-        const double reduce = s > 1 || longest.splits > 1 ? 3.0 + (double)partial * 8.0 / 4e6 : 0.0;
+        const double reduce = s > 1 || longest.splits > 1 ? reduce_us + (double)partial * 8.0 / 4e6 : 0.0;
         for (int f = 0; f < TILE_FORMS; ++f) {
             if (!(forms >> f & 1u) || (f == TILE_256x256 && s > 1)) continue;
             long len[kMaxProducts], cnt[kMaxProducts];

@@ -157,8 +157,10 @@ struct TileChoice {
     int split = 0, splits = 1;    // product `split` in `splits` parts
 };
 bool tiles_take(const TileProduct& p);                        // within the range of the loads' offsets
-// The best of `forms` (a bit each).  ws_floats > 0: the longest contraction may be split over that much scratch.
-TileChoice choose_tiles(const TileProduct* p, int n, unsigned forms, size_t ws_floats);
+// The best of `forms` (a bit each).  ws_floats > 0: the longest contraction may be split over that much scratch; reduce_us: what
+// adding up the parts takes besides a pass over them.
+constexpr double kReduceLaunch = 3.0;
+TileChoice choose_tiles(const TileProduct* p, int n, unsigned forms, size_t ws_floats, double reduce_us = kReduceLaunch);
 // `tail`: column sums of earlier launches, finished by workgroups behind the tiles (tail->n = 0 then).
 // Outputs of a tile of form f, and workgroups of that form on a CU.
 // out_steps: the way out of a tile in steps of it.
