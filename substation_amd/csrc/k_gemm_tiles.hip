@@ -124,10 +124,51 @@ bool tiles_take(const TileProduct& p) {
     return la < (1L << 30) && lb < (1L << 30) && lc < (1L << 30) && lt < (1L << 30);
 }
 
+// The launches a thread has last asked about, by everything that the choice depends on (choosing takes 1 to 8 us, a layer's pass
+// of some 15 products as much as a few launches; a decoder layer's operator calls make 25 such choices).
+namespace {
+struct Asked {
+    struct Product { int M, N, K1, K0, splits, order; long nbatch; };
+    long n = 0, forms = 0;
+    size_t ws_floats = 0;
+    double reduce_us = 0.;
+    Product p[kMaxProducts] = {};
+};
+struct Answer { Asked asked; TileChoice choice; };
+thread_local Answer answers[64];
+
+TileChoice choose_anew(const TileProduct* p, int n, unsigned forms, size_t ws_floats, double reduce_us);
+}  // namespace
+
 TileChoice choose_tiles(const TileProduct* p, int n, unsigned forms, size_t ws_floats, double reduce_us) {
+    if (n < 1 || n > kMaxProducts) return TileChoice{};
+    Asked q;
+    q.n = n; q.forms = forms; q.ws_floats = ws_floats; q.reduce_us = reduce_us;
+    uint64_t h = (uint64_t)ws_floats * 31 + forms;
+    for (int i = 0; i < n; ++i) {
+        const GemmArgs& a = p[i].a;
+        q.p[i] = Asked::Product{a.M, a.N, a.K1, a.K0, a.splits, (p[i].akc ? 1 : 0) | (p[i].bkc ? 2 : 0), a.nbatch};
+        for (uint64_t x : {(uint64_t)a.M, (uint64_t)a.N, (uint64_t)a.K1, (uint64_t)a.nbatch}) h = (h ^ x) * 0x9E3779B97F4A7C15ull;
+    }
+    Answer& at = answers[(h >> 40) % 64];
+    const Asked& was = at.asked;
+    bool same = was.n == q.n && was.forms == q.forms && was.ws_floats == q.ws_floats && was.reduce_us == q.reduce_us;
+    for (int i = 0; same && i < n; ++i) {
+        const Asked::Product &x = was.p[i], &y = q.p[i];
+        same = x.M == y.M && x.N == y.N && x.K1 == y.K1 && x.K0 == y.K0 && x.splits == y.splits && x.order == y.order && x.nbatch == y.nbatch;
+    }
+    if (!same) {
+        at.choice = choose_anew(p, n, forms, ws_floats, reduce_us);
+        at.asked = q;
+    }
+    return at.choice;
+}
+
+namespace {
+TileChoice choose_anew(const TileProduct* p, int n, unsigned forms, size_t ws_floats, double reduce_us) {
     TileChoice best;
     int k1, k2;
-    if (n < 1 || n > kMaxProducts || !orientations(p, n, k1, k2)) return best;
+    if (!orientations(p, n, k1, k2)) return best;
     // the order of the launch's list: longest contraction first
     int order[kMaxProducts];
     longest_first(p, n, order);
@@ -155,6 +196,7 @@ TileChoice choose_tiles(const TileProduct* p, int n, unsigned forms, size_t ws_f
     }
     return best;
 }
+}  // namespace
 
 TileForm tile_form(int form) {
     const Form& F = kForms[form];
