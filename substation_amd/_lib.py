@@ -64,6 +64,7 @@ SIGNATURES = {
     'sub_forget_staged': (_I, [_VP]),
     'sub_forward_form': (_I, [_VP, ctypes.POINTER(_I)]),
     'sub_set_forward_form': (_I, [_VP, _I]),
+    'sub_forward_alone': (_I, [_VP]),
     'sub_set_rng': (_I, [_VP, _U64, _U32]),
     'sub_set_rng_counter': (_I, [_VP, _VP]),
     'sub_last_error': (_CP, []),

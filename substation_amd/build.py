@@ -19,7 +19,7 @@ LIB = os.path.join(LIB_DIR, 'libsubstation_amd.so')
 HOST_LIB = os.path.join(LIB_DIR, '_host.so')       # the host side of a layer call (torch extension module)
 SOURCES = ['encoder.hip', 'k_rows.hip', 'k_elem.hip', 'k_cols.hip', 'k_lnbwd.hip', 'k_attn.hip', 'k_mha.hip', 'k_relayout.hip', 'k_probe.hip', 'k_gemm.hip',
            'k_gemm_tiles.hip', 'k_gemm_wide.hip',
-           *(('k_gemm_act.hip', f'-DSUB_EPI={epi}') for epi in range(1, 6))]
+           *(('k_gemm_act.hip', f'-DSUB_EPI={epi}') for epi in range(1, 7))]
 FLAGS = ['--offload-arch=gfx950', '-O3', '-std=c++17', '-fPIC', '-Wall', '-Wno-unused-function',
          # packed-fp32 VALU forms are switched off for every kernel of this library
          '-Xclang', '-target-feature', '-Xclang', '-packed-fp32-ops']

@@ -249,6 +249,8 @@ struct Handle {
     // is handed the same buffer, and from DROP2 itself otherwise.
     const void* gate_bits_at = nullptr;
     int form = 0;                     // what the last forward call left (FORM_*); see sub_forward_form
+    bool alone_next = false;          // no backward call will follow the next forward call (sub_forward_alone)
+    bool left_nothing = false;        // and none can follow the latest one
     int form_given = -1;              // the same of the forward call that the next backward call belongs to, if it was said
     BackwardPlan plan;                // see backward_plan()
     uint64_t plan_key = 0;
@@ -766,7 +768,7 @@ void op_bdrln(Handle& h, const void* in, const Layout& lin_, const void* resid, 
               const Layout& llin, void* mask, const Layout& lmask, void* diff, const Layout& ldiff,
               void* normed, const Layout& lnorm, void* out, const Layout& lout, void* istd,
               const Layout& listd, float p, uint32_t site, bool packed_mask = false, bool write_lin = true,
-              KeepWordsJob* side = nullptr, SplitSums sums = SplitSums{}) {
+              KeepWordsJob* side = nullptr, SplitSums sums = SplitSums{}, bool saves = true) {
     Space sp = make_space(h.sz, {dB, dJ}, dI);
     int R = sp.rs.R;
     View vi = make_view(in, lin_, sp), vr = make_view(resid, lres, sp), vl = make_view(lin, llin, sp),
@@ -775,7 +777,7 @@ void op_bdrln(Handle& h, const void* in, const Layout& lin_, const void* resid, 
     flatten(sp.rs, {&vi, &vr, &vl, &vm, &vd, &vn, &vo, &vs});
     launch_bdrln(sp.rs, vi, vr, vector_view(linear_bias, R), vector_view(scale, R), vector_view(bias, R),
                  vl, vm, vd, vn, vo, vs, make_key(h, site, p), h.eps, h.stream, packed_mask ? (uint8_t*)mask : nullptr,
-                 write_lin, side, sums);
+                 write_lin, side, sums, saves);
 }
 
 void op_blnrd(Handle& h, const void* dout, const Layout& ldout, const void* istd, const Layout& listd,
@@ -1176,7 +1178,10 @@ void stage_inputs(Handle& h, const void* X, void* const* W, const void*& Xs, voi
 }
 
 void forward(Handle& h, const FwdPtrs& t0) {
+    const bool alone = h.alone_next && h.opaque;
+    h.alone_next = false;
     if (!h.configured) fail("encoder_forward: handle is not configured");
+    h.left_nothing = alone;
     h.prof_used = 0;
     h.prof_forward = 0;
     FwdPtrs t = t0;
@@ -1254,7 +1259,7 @@ void forward(Handle& h, const FwdPtrs& t0) {
         op_bdrln(h, F[ATT], h.lf[ATT], t.X, h.lX, W[BO], W[S1], W[B1], F[ATT], h.lf[ATT],
                  F[DROP1MASK], h.lf[DROP1MASK], F[LN1DIFF], h.lf[LN1DIFF], F[LN1], h.lf[LN1],
                  F[SB1], h.lf[SB1], F[LN1STD], h.lf[LN1STD], h.p_resid1, SUB_SITE_RESID1, packed_masks(h), !h.skip_unread,
-                 &keep_job, out_sums);
+                 &keep_job, out_sums, !alone);
     }
     if (lin1_bad) {
         // product, bias, activation and dropout in one launch: SB1_LINW1 and DROP2MASK (ReLU: and LIN1) are not produced
@@ -1264,7 +1269,8 @@ void forward(Handle& h, const FwdPtrs& t0) {
         ep.bias = (const half_t*)W[LINB1]; ep.sbM = p.sM; ep.sbN = p.sN;
         ep.relu_dropout = true; ep.key = make_key(h, SUB_SITE_ACT, h.p_act);
         if (keep_job.blocks) ep.keep_words = keep_job.out;
-        if (F[SB1_LINW1] && ((uintptr_t)F[SB1_LINW1] & 3) == 0) ep.gate_bits_out = (uint32_t*)F[SB1_LINW1];
+        ep.alone = alone;
+        if (!alone && F[SB1_LINW1] && ((uintptr_t)F[SB1_LINW1] & 3) == 0) ep.gate_bits_out = (uint32_t*)F[SB1_LINW1];
         h.gate_bits_at = ep.gate_bits_out;
         if (ep.gate_bits_out) h.form |= FORM_BITS;
         if (lin1_gelu) { ep.act = ACT_GELU; ep.pre_out = (half_t*)F[LIN1]; }
@@ -1284,7 +1290,7 @@ void forward(Handle& h, const FwdPtrs& t0) {
         op_bdrln(h, F[DROP2_LINW2], h.lf[DROP2_LINW2], F[SB1], h.lf[SB1], W[LINB2], W[S2], W[B2],
                  F[LIN2], h.lf[LIN2], F[DROP3MASK], h.lf[DROP3MASK], F[LN2DIFF], h.lf[LN2DIFF],
                  F[LN2], h.lf[LN2], t.Y, h.lY, F[LN2STD], h.lf[LN2STD], h.p_resid2, SUB_SITE_RESID2, packed_masks(h), !h.skip_unread,
-                 nullptr, lin2_sums);
+                 nullptr, lin2_sums, !alone);
     }
     if (h.staging && h.stage_y) {
         ProfScope ps(h, "relayout-out");
@@ -1304,6 +1310,7 @@ void backward(Handle& h, const BwdPtrs& t0) {
     if (!h.configured) fail("encoder_backward: handle is not configured");
     const int form = h.form_given;
     h.form_given = -1;
+    if (form < 0 && h.left_nothing) fail("encoder_backward: the latest forward call left nothing for it (sub_forward_alone)");
     // the first backward call after a forward call keeps that call's entries in front of its own
     h.prof_used = h.prof_forward;
     h.prof_forward = 0;
@@ -1642,10 +1649,13 @@ int sub_forget_staged(void* handle) {
 int sub_encoder_forward(void* handle, void* const* ptrs, int n) {
     return guarded([&] {
         Handle& h = as_handle(handle);
+        const bool alone = h.alone_next;
+        h.alone_next = false;         // (a call that is refused is the one it was said of)
         if (n != 1 + SUB_N_PARAMS + SUB_N_FWD + 1) fail("sub_encoder_forward: expected 37 pointers");
         need_cfg(h);
         for (int i = 0; i < n; ++i) if (!ptrs[i]) fail("sub_encoder_forward: null tensor pointer");
         FwdPtrs t; unpack_forward(h, ptrs, t);
+        h.alone_next = alone;
         forward(h, t);
     });
 }
@@ -1743,6 +1753,10 @@ int sub_forward_form(void* handle, int* form) {
         if (!form) fail("sub_forward_form: null result pointer");
         *form = as_handle(handle).form;
     });
+}
+
+int sub_forward_alone(void* handle) {
+    return guarded([&] { as_handle(handle).alone_next = true; });
 }
 
 int sub_set_forward_form(void* handle, int form) {

@@ -38,6 +38,7 @@ struct Lib {
     decltype(&sub_forget_staged) forget_staged = nullptr;
     decltype(&sub_forward_form) forward_form = nullptr;
     decltype(&sub_set_forward_form) set_forward_form = nullptr;
+    decltype(&sub_forward_alone) forward_alone = nullptr;
     decltype(&sub_encoder_forward) encoder_forward = nullptr;
     decltype(&sub_encoder_backward) encoder_backward = nullptr;
 } lib;
@@ -59,6 +60,7 @@ void load(const std::string& path, py::object error) {
     get(lib.forget_staged, "sub_forget_staged");
     get(lib.forward_form, "sub_forward_form");
     get(lib.set_forward_form, "sub_set_forward_form");
+    get(lib.forward_alone, "sub_forward_alone");
     get(lib.encoder_forward, "sub_encoder_forward");
     get(lib.encoder_backward, "sub_encoder_backward");
     g_error = error.release().ptr();
@@ -347,6 +349,8 @@ std::optional<at::Tensor> EncoderLayer::forward(const at::Tensor& X_, const std:
     {
         py::gil_scoped_release nogil;
         use_current_stream(handle, X.device().index());
+        // (a workspace that stays with the module can be looked at, these intermediates are gone when this returns)
+        if (!grad && !persistent) check(lib.forward_alone(handle), "sub_forward_alone");
         check(lib.encoder_forward(handle, p.data(), (int)p.size()), "encoder_forward");
     }
     if (grad) {

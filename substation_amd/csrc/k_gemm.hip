@@ -169,7 +169,8 @@ Canon canonicalise(const GemmShape& s, const half_t* A, const half_t* B, half_t*
     a.alpha = alpha; a.bias = ep.bias;
     a.relu_dropout = ep.relu_dropout ? 1 : 0; a.key = ep.key;
     a.gate = ep.gate; a.colsum = ep.colsum; a.gate_bits_out = ep.gate_bits_out; a.gate_bits = ep.gate_bits;
-    a.keep_words = ep.keep_words; a.act = ep.act; a.pre_out = ep.pre_out;
+    a.keep_words = ep.keep_words; a.act = ep.act; a.pre_out = ep.pre_out; a.alone = ep.alone ? 1 : 0;
+    if (ep.alone) a.gate_bits_out = nullptr;
     a.splits = 1; a.partial = nullptr;
     c.ok_c = a.sCN == 1;
     return c;
@@ -191,7 +192,7 @@ int pick_kind(const Canon& c, bool& akc, bool& bkc) {
     if (a.gate && !(a.sbN == 1 && mult8(a.sbM) && al16(a.gate) && !a.bias && a.colsum)) return 0;
     // GELU: the backward form needs the keep bits, the forward form a place for the pre-activation and for those bits
     if (a.act == ACT_GELU && a.gate && !a.gate_bits) return 0;
-    if (a.act == ACT_GELU && a.relu_dropout && !(a.pre_out && al16(a.pre_out) && a.gate_bits_out && !a.keep_words)) return 0;
+    if (a.act == ACT_GELU && a.relu_dropout && !(a.pre_out && al16(a.pre_out) && (a.gate_bits_out || a.alone) && !a.keep_words)) return 0;
     // every 16-byte access must be aligned and whole
     bool ok = mult8(a.N) && mult8(a.sCM) && mult8(a.sCb[0]) && mult8(a.sCb[1]) && mult8(a.sCb[2]);
     ok = ok && mult8(a.sAK0) && mult8(a.sAb[0]) && mult8(a.sAb[1]) && mult8(a.sAb[2]);

@@ -1,4 +1,4 @@
-// The contraction kernels with activation SUB_EPI (1 .. 5) in their epilogue.
+// The contraction kernels with activation SUB_EPI (1 .. 6) in their epilogue.
 #include "sub_ring.hpp"
 #include "sub_wide.hpp"
 

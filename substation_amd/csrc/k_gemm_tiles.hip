@@ -234,7 +234,7 @@ int choose_act_form(const TileProduct& p) {
 void launch_tiles_act(const TileProduct& p, int form, hipStream_t st) {
     const GemmArgs& a = p.a;
     if (a.gate) a.act == ACT_GELU ? launch_act<EPI_GELU_GATE_COLSUM>(p, form, st) : launch_act<EPI_GATE_COLSUM>(p, form, st);
-    else if (a.act == ACT_GELU) launch_act<EPI_GELU_DROPOUT>(p, form, st);
+    else if (a.act == ACT_GELU) a.alone ? launch_act<EPI_GELU_ALONE>(p, form, st) : launch_act<EPI_GELU_DROPOUT>(p, form, st);
     else a.keep_words ? launch_act<EPI_RELU_DROPOUT_PRE>(p, form, st) : launch_act<EPI_RELU_DROPOUT>(p, form, st);
 }
 

@@ -352,11 +352,11 @@ __global__ __launch_bounds__(BLOCK) void k_bdrln_flat(int R, unsigned nrows, Vie
                                                       View scale, View bias, View lin, View mask, View diff,
                                                       View normed, View out, View istd, PhiloxKey key_, float eps,
                                                       uint8_t* mask_bits, bool write_lin, KeepWordsJob side,
-                                                      SplitSums sums) {
+                                                      SplitSums sums, bool saves) {
     if (SUMS) fetch_args_now(sums.p, sums.splits, sums.slab, sums.alpha);
     fetch_args_now(R, nrows, in.p, in.s3, resid.p, resid.s3, lin_bias.p, scale.p, bias.p, lin.p, lin.s3, mask.p, mask.s3,
                    diff.p, diff.s3, normed.p, normed.s3, out.p, out.s3, istd.p, istd.s3, key_.k0, key_.k1, key_.site,
-                   key_.step, key_.thr, key_.step_dev, eps, mask_bits, write_lin, side.blocks);
+                   key_.step, key_.thr, key_.step_dev, eps, mask_bits, write_lin, side.blocks, saves);
     const unsigned row_blocks = gridDim.x - side.blocks;
     if (blockIdx.x >= row_blocks) {
         const PhiloxKey skey = resolved(side.key);
@@ -456,7 +456,7 @@ __global__ __launch_bounds__(BLOCK) void k_bdrln_flat(int R, unsigned nrows, Vie
                 x[c][i] = kept + (float)re8[i];
                 s += x[c][i];
             }
-            if (inside[c]) {
+            if (inside[c] && saves) {
                 if (write_lin) stg8<true>(lin.p + (long)row * lin.s3 + e0[c], lh);
                 if (mask_bits) mask_bits[(size_t)row * (R >> 3) + (c * WAVE + lane)] = (uint8_t)bits[c];
                 else stg8<true>(mask.p + (long)row * mask.s3 + e0[c], mask_h8(bits[c]));
@@ -472,7 +472,7 @@ __global__ __launch_bounds__(BLOCK) void k_bdrln_flat(int R, unsigned nrows, Vie
                 q += x[c][i] * x[c][i];
             }
         const float is = rsqrtf(wave_sum(q) * invn + eps);       // 1/std
-        if (lane == 0) istd.p[(long)row * istd.s3] = (half_t)is;
+        if (lane == 0 && saves) istd.p[(long)row * istd.s3] = (half_t)is;
 #pragma unroll
         for (int c = 0; c < VPL; ++c) {
             if (!inside[c]) continue;
@@ -485,8 +485,10 @@ __global__ __launch_bounds__(BLOCK) void k_bdrln_flat(int R, unsigned nrows, Vie
                 n[i] = (half_t)nn;
                 o[i] = (half_t)(nn * (float)s8[i] + (float)b8[i]);
             }
-            stg8<true>(diff.p + (long)row * diff.s3 + e0[c], d);
-            stg8<true>(normed.p + (long)row * normed.s3 + e0[c], n);
+            if (saves) {
+                stg8<true>(diff.p + (long)row * diff.s3 + e0[c], d);
+                stg8<true>(normed.p + (long)row * normed.s3 + e0[c], n);
+            }
             stg8<false>(out.p + (long)row * out.s3 + e0[c], o);
         }
     }
@@ -749,7 +751,7 @@ void launch_bs(const RowSpace& rs, View alpha, View mask, View ddrop, View dbeta
 
 void launch_bdrln(const RowSpace& rs, View in, View resid, View lin_bias, View scale, View bias,
                   View lin, View mask, View diff, View normed, View out, View istd, PhiloxKey key,
-                  float eps, hipStream_t st, uint8_t* mask_bits, bool write_lin, KeepWordsJob* side, SplitSums sums) {
+                  float eps, hipStream_t st, uint8_t* mask_bits, bool write_lin, KeepWordsJob* side, SplitSums sums, bool saves) {
     if (mask_bits && rs.R % 8) fail("bias-dropout-residual-layernorm: a bit mask needs rows of whole 8-packs");
     unsigned nrows = check_rows(rs, "bias-dropout-residual-layernorm");
     if (nrows == 0) return;
@@ -777,7 +779,7 @@ void launch_bdrln(const RowSpace& rs, View in, View resid, View lin_bias, View s
     if (flat) {
         const dim3 grid(row_grid(nrows, 1) + extra_blocks);
 #define SUB_BDRLN_FLAT(V, S) hipLaunchKernelGGL((k_bdrln_flat<V, S>), grid, dim3(BLOCK), 0, st, rs.R, nrows, in, resid, lin_bias, \
-                                             scale, bias, lin, mask, diff, normed, out, istd, key, eps, mask_bits, write_lin, job, sums)
+                                             scale, bias, lin, mask, diff, normed, out, istd, key, eps, mask_bits, write_lin, job, sums, saves)
         if (sums.p && vpl == 1) SUB_BDRLN_FLAT(1, true);
         else if (sums.p) SUB_BDRLN_FLAT(2, true);
         else switch (vpl) {

@@ -31,6 +31,7 @@ struct GemmArgs {
     const uint32_t* gate_bits = nullptr;   // gate: those bits instead of the values of `gate`
     int act = ACT_RELU;                    // the activation of relu_dropout / gate (GemmEpilogue::act)
     half_t* pre_out = nullptr;             // GELU with dropout: where the rounded sum before the activation goes
+    int alone = 0;                         // no backward pass follows (GemmEpilogue::alone)
     // GemmSideJob of the 256 x 256 kernel: the workgroups behind those of the tiles draw
     // the attention keep words of key tiles 0 .. side_tiles_done - 1 of side_rows score rows
     PhiloxKey side_key;

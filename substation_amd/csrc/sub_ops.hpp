@@ -47,7 +47,8 @@ struct KeepWordsJob {
 void launch_bdrln(const RowSpace& rs, View in, View resid, View lin_bias, View scale, View bias,
                   View lin, View mask, View diff, View normed, View out, View istd, PhiloxKey key,
                   float eps, hipStream_t st, uint8_t* mask_bits = nullptr, bool write_lin = true,
-                  KeepWordsJob* side = nullptr, SplitSums sums = SplitSums{});
+                  KeepWordsJob* side = nullptr, SplitSums sums = SplitSums{},
+                  bool saves = true);
 void launch_blnrd(const RowSpace& rs, View dout, View istd, View diff, View mask, View d_ln_in,
                   View d_drop_in, hipStream_t st, const uint8_t* mask_bits = nullptr);
 
@@ -251,6 +252,7 @@ struct GemmEpilogue {
     // keep ? gelu'(gate) * x : 0 with `gate` the pre-activation values and gate_bits those keep bits (required).
     int act = ACT_RELU;
     half_t* pre_out = nullptr;
+    bool alone = false;          // relu_dropout: no backward pass follows; pre_out and gate_bits_out are not written
     // the contraction of a small output may be split in as many parts as is fastest; otherwise their number, and with it the
     // order of the sums, depends on the shape alone (one unit of the last place of a pre-activation decides a ReLU's gate)
     bool any_split = false;

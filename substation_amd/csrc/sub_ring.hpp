@@ -399,9 +399,11 @@ struct Ring : TileList<32 * TM * WM, 32 * TN * WN, NP> {
                         uint32_t keep = kb[c >> 2] >> (8 * (c & 3));
                         if (from_bits) keep = quad_byte<c & 3>(bits[c >> 2], lane);
                         val = act_forward<EPI>(val, keep);
-                        const uint32_t word = quad_word(keep, lane);
-                        out_word = q == (c & 3) ? word : out_word;
-                        if constexpr ((c & 3) == 3 || c == PACKS - 1)
+                        if constexpr (EPI != EPI_GELU_ALONE) {
+                            const uint32_t word = quad_word(keep, lane);
+                            out_word = q == (c & 3) ? word : out_word;
+                        }
+                        if constexpr (EPI != EPI_GELU_ALONE && ((c & 3) == 3 || c == PACKS - 1))
                             __builtin_amdgcn_raw_buffer_store_b32(out_word, ro, (int)(bits_at + (c >> 2) * bits_step), 0, 0);
                     }
                     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4v, val), rc, (int)c_at, 0, 0);

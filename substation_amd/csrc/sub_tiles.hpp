@@ -45,9 +45,10 @@ __device__ __forceinline__ void load_to_lds(unsigned lds, unsigned voff, u4v r) 
 // EPI_RELU_DROPOUT_PRE: EPI_RELU_DROPOUT with the keep bits drawn ahead of the launch (GemmEpilogue::keep_words)
 // EPI_GELU_DROPOUT: as EPI_RELU_DROPOUT with GELU; also stores the rounded sum before the activation
 // (GemmArgs::pre_out, which the backward pass needs) and leaves the keep bits where the ReLU form leaves its gate bits.
+// EPI_GELU_ALONE: without either, where no backward pass follows.
 // EPI_GELU_GATE_COLSUM: the backward counterpart: out = keep bit ? gelu'(pre-activation) * product : 0, and column sums.
 enum { EPI_PLAIN = 0, EPI_RELU_DROPOUT = 1, EPI_GATE_COLSUM = 2, EPI_RELU_DROPOUT_PRE = 3, EPI_GELU_DROPOUT = 4,
-       EPI_GELU_GATE_COLSUM = 5 };
+       EPI_GELU_GATE_COLSUM = 5, EPI_GELU_ALONE = 6 };
 
 template <typename Key>
 __device__ __forceinline__ PhiloxKey key_of(Key& from) {
@@ -100,7 +101,7 @@ __device__ __forceinline__ uint32_t quad_byte(uint32_t word, int lane) {
 // GELU: the keep bits themselves; ReLU: set where the result is positive.
 template <int EPI>
 __device__ __forceinline__ h8 act_forward(h8 v, uint32_t& keep) {
-    if constexpr (EPI == EPI_GELU_DROPOUT) {
+    if constexpr (EPI == EPI_GELU_DROPOUT || EPI == EPI_GELU_ALONE) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = (half_t)gelu_fwd((float)v[e]);       // for every element, then selected: no branches
         return keep8_of(v, keep);

@@ -128,7 +128,7 @@ struct Wide : TileList<4 * QM, 4 * QN, NP> {
     static constexpr int LATE = TB / 2;                                // fragments of B0 read in the quarter that uses them
     static constexpr int LPR = QN / 8, RPI = 64 / LPR, NI = 16 / RPI;  // lanes per output row, rows per store, stores per slab
     static constexpr int PACKS = 4 * TA * NI;                          // packs of 8 outputs that a lane stores
-    static constexpr bool DRAWS = EPI == EPI_RELU_DROPOUT || EPI == EPI_GELU_DROPOUT;
+    static constexpr bool DRAWS = EPI == EPI_RELU_DROPOUT || EPI == EPI_GELU_DROPOUT || EPI == EPI_GELU_ALONE;
     static constexpr bool GATED = EPI == EPI_GATE_COLSUM || EPI == EPI_GELU_GATE_COLSUM;
     static constexpr bool READS = GATED || EPI == EPI_RELU_DROPOUT_PRE;          // bits of the outputs, as another launch left them
     static_assert(EPI == EPI_PLAIN || (PACKS == 32 && LPR == 8 && TA == 4), "32 packs of keep bits per lane, in the order of Epilogue::bits_part");
@@ -550,9 +550,11 @@ struct Wide : TileList<4 * QM, 4 * QN, NP> {
                                 if constexpr (DRAWS) keep = draw.kb[c >> 2] >> (8 * (c & 3));
                                 else keep = quad_byte<c & 3>(bits[c >> 2], lane);
                                 val = act_forward<EPI>(val, keep);
-                                const uint32_t word = quad_word(keep, lane);
-                                out_word = (lane & 3) == (c & 3) ? word : out_word;
-                                if constexpr ((c & 3) == 3)
+                                if constexpr (EPI != EPI_GELU_ALONE) {
+                                    const uint32_t word = quad_word(keep, lane);
+                                    out_word = (lane & 3) == (c & 3) ? word : out_word;
+                                }
+                                if constexpr (EPI != EPI_GELU_ALONE && (c & 3) == 3)
                                     __builtin_amdgcn_raw_buffer_store_b32(out_word, ro, (int)(at_o[c >> 3 & 1] + bits_part(g, c >> 2)), 0, 0);
                             }
                             put(rc, at, uni, val);
