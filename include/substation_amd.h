@@ -539,6 +539,18 @@ int sub_op_einsum_pair(void* handle, const void* A1, const char* l_A1, const voi
                        const void* T1, const char* l_T1, void* C1, const char* l_C1, float alpha1,
                        const void* A2, const char* l_A2, const void* B2, const char* l_B2, void* C2,
                        const char* l_C2, float alpha2, int* paired);
+/* Up to fourteen independent contractions, each with an optional addend as in sub_op_einsum_add, in as few launches as is
+ * fastest: weight gradients that nothing waits for fill each other's last rounds of tiles (encoder_backward does the same with
+ * its own).  sizes: the handle whose sizes the layouts mean (null: `handle`).  No output may be another product's input. */
+typedef struct {
+    void* sizes;
+    const void* A; const char* l_A;
+    const void* B; const char* l_B;
+    const void* T; const char* l_T;
+    void* C; const char* l_C;
+    float alpha;
+} SubEinsum;
+int sub_op_einsum_group(void* handle, const SubEinsum* products, int n);
 int sub_op_einsum_add(void* handle, const void* A, const char* l_A, const void* B, const char* l_B,
                       const void* T, const char* l_T, void* C, const char* l_C, float alpha);
 

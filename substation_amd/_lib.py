@@ -46,6 +46,13 @@ class SubConfig(ctypes.Structure):
     ]
 
 
+class Einsum(ctypes.Structure):
+    """A product of sub_op_einsum_group."""
+    _fields_ = [('sizes', ctypes.c_void_p), ('A', ctypes.c_void_p), ('l_A', ctypes.c_char_p),
+                ('B', ctypes.c_void_p), ('l_B', ctypes.c_char_p), ('T', ctypes.c_void_p), ('l_T', ctypes.c_char_p),
+                ('C', ctypes.c_void_p), ('l_C', ctypes.c_char_p), ('alpha', ctypes.c_float)]
+
+
 _lib = None
 _host = None
 
@@ -112,6 +119,7 @@ SIGNATURES = {
                                ctypes.POINTER(ctypes.c_int)]),
     'sub_op_einsum_bdrlb': (_I, [_VP, _VP, _CP, _VP, _CP, _VP, _CP, _VP, _VP, _CP, _VP,
                                  ctypes.POINTER(ctypes.c_int)]),
+    'sub_op_einsum_group': (_I, [_VP, ctypes.POINTER(Einsum), _I]),
     'sub_op_einsum_pair': (_I, [_VP, _VP, _CP, _VP, _CP, _VP, _CP, _VP, _CP, _F,
                                 _VP, _CP, _VP, _CP, _VP, _CP, _F, ctypes.POINTER(ctypes.c_int)]),
     'sub_layout_strides': (_I, [_VP, _CP, ctypes.POINTER(ctypes.c_int64)]),

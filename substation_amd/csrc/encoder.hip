@@ -2281,6 +2281,55 @@ int sub_op_einsum_pair(void* handle, const void* A1, const char* l_A1, const voi
     });
 }
 
+int sub_op_einsum_group(void* handle, const SubEinsum* p, int n) {
+    return guarded([&] {
+        Handle& h = as_handle(handle); need_cfg(h);
+        if (n < 0 || n > 2 * kMaxProducts) fail("sub_op_einsum_group: at most " + std::to_string(2 * kMaxProducts) + " products");
+        std::vector<GemmShape> shape(n);
+        std::vector<GemmJob> jobs(n);
+        size_t need = 0;
+        for (int i = 0; i < n; ++i) {
+            const SubEinsum& q = p[i];
+            if (!q.A || !q.B || !q.C || !q.l_A || !q.l_B || !q.l_C) fail("sub_op_einsum_group: null tensor or layout");
+            Handle& sz = q.sizes ? as_handle(q.sizes) : h;
+            need_cfg(sz);
+            const Layout lc = L(sz, q.l_C);
+            shape[i] = classify_einsum(L(sz, q.l_A), L(sz, q.l_B), lc);
+            GemmJob& j = jobs[i];
+            j.name = "einsum"; j.shape = &shape[i]; j.alpha = q.alpha;
+            j.A = (const half_t*)q.A; j.B = (const half_t*)q.B; j.C = (half_t*)q.C;
+            if (q.T) {
+                if (!q.l_T || !addend_strides(shape[i], L(sz, q.l_T), lc, j.ep.sbM, j.ep.sbN, j.ep.sbb))
+                    fail(std::string("sub_op_einsum_group: the dims of the addend are not free or batch dims of ") + q.l_C +
+                         " in one dense run each");
+                j.ep.bias = (const half_t*)q.T;
+                if (gemm_kernel_kind(shape[i], q.A, q.B, q.C, j.ep) != 1)
+                    fail("sub_op_einsum_group: these layouts go to the kernel without an epilogue (addend and output "
+                         "must be contiguous along the same free dims)");
+            }
+            need = std::max(need, gemm_splitk_ws_floats(shape[i]));
+        }
+        if (n == 0) return;
+        ensure_gws(h, need);
+        // the longest contractions first, in one launch or, from some place of that order on, in another
+        std::vector<int> order(n);
+        for (int i = 0; i < n; ++i) order[i] = i;
+        std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return shape[x].K() > shape[y].K(); });
+        GemmStage best[2], tried[2];
+        double us = -1.;
+        for (int cut = std::max(1, n - kMaxProducts); cut <= std::min(n, kMaxProducts); ++cut) {
+            double t = plan_gemm_stage(jobs.data(), order.data(), cut, h.pair_products, h.gws_floats, tried[0]);
+            tried[1].n = 0;
+            if (cut < n) t += 1.5 + plan_gemm_stage(jobs.data(), order.data() + cut, n - cut, h.pair_products, h.gws_floats, tried[1]);
+            if (us >= 0. && t >= us) continue;
+            us = t;
+            best[0] = tried[0]; best[1] = tried[1];
+        }
+        run_stage(h, jobs.data(), best[0], nullptr);
+        run_stage(h, jobs.data(), best[1], nullptr);
+    });
+}
+
 // Operator calls: products of a quarter of the chip in 256 x 256 tiles and more.  Below that the caller keeps a mask tensor that
 // can be looked at, which is the only reason for the line: one launch is faster than two at every size.  us of one launch (two),
 // p = 0.1, ReLU forward, backward, GELU forward, backward; 256 rows x 3072 x 768 (12 tiles): 8.9 (10.9), 10.1 (14.4), 8.9 (11.1),

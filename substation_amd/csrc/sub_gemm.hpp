@@ -137,7 +137,7 @@ struct DTile {
 };
 
 
-// k_gemm_tiles.hip: products in tiles of five sizes, up to five in one launch.
+// k_gemm_tiles.hip: products in tiles of five sizes, up to kMaxProducts in one launch.
 enum { TILE_64x64 = 0, TILE_128x64, TILE_128x128, TILE_256x128, TILE_256x256, TILE_FORMS };
 constexpr unsigned kRingForms = (1u << TILE_256x256) - 1;
 struct TileProduct {

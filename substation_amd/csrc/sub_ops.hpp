@@ -290,11 +290,11 @@ struct GemmJob {
     float alpha = 1.f;
     GemmEpilogue ep;             // (an addend at most)
 };
-constexpr int kMaxProducts = 5;  // of one launch
+constexpr int kMaxProducts = 7;  // of one launch (their arguments stay below 4 KiB)
 // Jobs of one launch: their tiles of form `form`, the contraction of member `split` in `splits` parts.  form < 0: one job, launched
 // by launch_gemm.
 struct GemmLaunch {
-    int n = 0, job[kMaxProducts] = {0, 0, 0, 0, 0};
+    int n = 0, job[kMaxProducts] = {};
     int form = -1, split = 0, splits = 1;
     void drop(int j);            // without job j (the others as they were)
 };

@@ -214,6 +214,20 @@ class Ops:
             _p(a2), _s(la2), _p(b2), _s(lb2), _p(c2), _s(lc2), 1.0, ctypes.byref(paired)), 'einsum_pair')
         return bool(paired.value)
 
+    def einsum_group(self, products):
+        """Independent contractions (up to fourteen) in as few launches as is fastest.  Each is (a, l_a, b, l_b, c, l_c),
+        or with (addend, l_addend) appended; an Ops in front of that says whose sizes its layouts mean."""
+        group = (_lib.Einsum * len(products))()
+        for q, product in zip(group, products):
+            if isinstance(product[0], Ops):
+                q.sizes = product[0].handle.ptr
+                product = product[1:]
+            a, l_a, b, l_b, c, l_c = product[:6]
+            q.A, q.l_A, q.B, q.l_B, q.C, q.l_C, q.alpha = _p(a), _s(l_a), _p(b), _s(l_b), _p(c), _s(l_c), 1.0
+            if len(product) > 6:
+                q.T, q.l_T = _p(product[6]), _s(product[7])
+        _lib.check(self.lib.sub_op_einsum_group(self._pre(), group, len(products)), 'einsum_group')
+
     def einsum(self, a, l_a, b, l_b, c, l_c, alpha=1.0, addend=None, l_addend=None):
         """c = alpha * einsum(a, b) [+ addend, broadcast over the dims it lacks]."""
         if addend is not None:

@@ -50,3 +50,34 @@ def test_products_that_share_a_launch_give_what_they_give_alone(dims, which, lau
     for name, alone in grads[0].items():
         # (sums in another order, rounded to fp16, and what follows from them: within the bound of any product here)
         assert_close(grads[1][name].float().cpu().numpy(), alone.float().cpu().numpy(), tol=1e-2, name=name)
+
+
+@pytest.mark.parametrize('dims,source', [((2, 128, 2, 128), 256), ((3, 40, 4, 256), 72), ((4, 384, 16, 1024), 128)])
+def test_group_of_contractions_gives_what_each_of_them_gives(dims, source):
+    """Ten products of two sizes in one call, one of them added to its own output, against single calls."""
+    from substation_amd.ops import Ops
+    B, Ls, H, E = dims
+    o, os_ = Ops(B, Ls, H, E), Ops(B, source, H, E)
+    g = torch.Generator('cuda').manual_seed(1)
+
+    def tensor(ops, layout):
+        return (0.3 * torch.randn(ops.empty(layout).shape, generator=g, device='cuda')).half()
+
+    products, alone = [], []
+    for ops, la, lb, lc, lt in [(o, 'QHPI', 'QBJHP', 'BJI', 'BJI'), (os_, 'BKHP', 'HPI', 'BKI', 'BKI'), (os_, 'BKHP', 'BKI', 'HPI', None),
+                                (os_, 'BKHP', 'BKI', 'HPI', None), (o, 'QBJHP', 'BJI', 'QHPI', None), (o, 'BJI', 'BJHP', 'IHP', None),
+                                (o, 'BJHP', 'BJI', 'HPI', None), (o, 'BJI', 'BJHP', 'IHP', None), (o, 'BJU', 'BJI', 'UI', None),
+                                (o, 'BJI', 'BJU', 'IU', None)]:
+        a, b, c = tensor(ops, la), tensor(ops, lb), tensor(ops, lc)
+        want = ops.empty(lc)
+        if lt:
+            ops.einsum(a, la, b, lb, want, lc, addend=c, l_addend=lt)
+            products.append((ops, a, la, b, lb, c, lc, c, lt))
+        else:
+            ops.einsum(a, la, b, lb, want, lc)
+            products.append((ops, a, la, b, lb, c, lc))
+        alone.append(want)
+    o.einsum_group(products)
+    for (_, _, la, _, lb, c, lc, *_), want in zip(products, alone):
+        # fp32 sums in another order, rounded once
+        assert_close(c.float().cpu().numpy(), want.float().cpu().numpy(), tol=2e-3, name=f'{la},{lb}->{lc}')
