@@ -300,6 +300,8 @@ float* static_scratch() {
     return g_scratch_ptr[dev];
 }
 
+// Forward products of a ReLU layer (see GemmEpilogue::same_order).
+bool before_relu(const Handle& h) { return h.act == ACT_RELU; }
 // Dropout masks as bits (SUB_OPT_PACKED_MASKS), those of the residuals and the activation's: rows must be whole 8-packs.
 bool packed_masks(const Handle& h) { return h.packed_masks && h.sz.n[dI] % 8 == 0; }
 bool packed_act_mask(const Handle& h) { return h.packed_masks && h.opaque && h.sz.n[dU] % 8 == 0; }
@@ -566,6 +568,7 @@ void plan_layouts(Handle& h, bool own) {
     if (h.gemm[G_LIN1_BAD].ok) {
         GemmPlan& p = h.gemm[G_LIN1_BAD];
         GemmEpilogue ep; ep.bias = (const half_t*)16; ep.sbM = p.sM; ep.sbN = p.sN; ep.relu_dropout = true;
+        ep.same_order = before_relu(h);
         p.ok = h.lf[DROP2].str() == "BJU" &&
                gemm_relu_dropout_ok(p.shape, (const void*)16, (const void*)16, (const void*)16, ep);
     }
@@ -637,6 +640,7 @@ void run_gemm(Handle& h, int id, const void* A, const void* B, void* C, const ch
     const GemmPlan& p = h.gemm[id];
     GemmEpilogue ep;
     ep.any_split = id >= G_DXLIN2 || id == G_DXQKV_RESID;      // the backward pass
+    ep.same_order = before_relu(h) && !ep.any_split && id != G_LIN2;
     ep.sums = sums;
     if (addend) {
         ep.bias = (const half_t*)addend; ep.sbM = p.sM; ep.sbN = p.sN;
@@ -1270,6 +1274,7 @@ void forward(Handle& h, const FwdPtrs& t0) {
         ep.relu_dropout = true; ep.key = make_key(h, SUB_SITE_ACT, h.p_act);
         if (keep_job.blocks) ep.keep_words = keep_job.out;
         ep.alone = alone;
+        ep.same_order = before_relu(h);
         if (!alone && F[SB1_LINW1] && ((uintptr_t)F[SB1_LINW1] & 3) == 0) ep.gate_bits_out = (uint32_t*)F[SB1_LINW1];
         h.gate_bits_at = ep.gate_bits_out;
         if (ep.gate_bits_out) h.form |= FORM_BITS;
@@ -2216,6 +2221,7 @@ int sub_op_einsum(void* handle, const void* A, const char* l_A, const void* B, c
         Handle& h = as_handle(handle); need_cfg(h);
         GemmShape g = classify_einsum(L(h, l_A), L(h, l_B), L(h, l_C));
         GemmEpilogue ep;
+        ep.same_order = before_relu(h);
         ensure_gws(h, gemm_splitk_ws_floats(g));
         launch_gemm(g, (const half_t*)A, (const half_t*)B, (half_t*)C, alpha, ep, h.stream, h.gws, h.gws_floats);
     });
@@ -2228,6 +2234,7 @@ int sub_op_einsum_add(void* handle, const void* A, const char* l_A, const void* 
         const Layout lc = L(h, l_C), lt = L(h, l_T);
         GemmShape g = classify_einsum(L(h, l_A), L(h, l_B), lc);
         GemmEpilogue ep;
+        ep.same_order = before_relu(h);
         if (!T) fail("sub_op_einsum_add: null addend");
         if (!addend_strides(g, lt, lc, ep.sbM, ep.sbN, ep.sbb))
             fail(std::string("sub_op_einsum_add: the dims of ") + l_T + " are not free or batch dims of " + l_C +
@@ -2351,6 +2358,7 @@ int sub_op_einsum_bad(void* handle, const void* A, const char* l_A, const void* 
         ep.bias = (const half_t*)bias;
         ep.relu_dropout = true; ep.key = make_key(h, site, p);
         ep.gate_bits_out = (uint32_t*)bits;
+        ep.same_order = before_relu(h);
         if (h.act == ACT_GELU) { ep.act = ACT_GELU; ep.pre_out = (half_t*)lin; }
         // the keep bits are indexed by the offset into the output: it has to be dense in canonical order
         if (lc.str() != "BJU" || ((uintptr_t)bits & 3) || !aligned16(bias) || !aligned16(out) || !aligned16(A) ||

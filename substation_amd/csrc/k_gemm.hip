@@ -169,7 +169,7 @@ Canon canonicalise(const GemmShape& s, const half_t* A, const half_t* B, half_t*
     a.alpha = alpha; a.bias = ep.bias;
     a.relu_dropout = ep.relu_dropout ? 1 : 0; a.key = ep.key;
     a.gate = ep.gate; a.colsum = ep.colsum; a.gate_bits_out = ep.gate_bits_out; a.gate_bits = ep.gate_bits;
-    a.keep_words = ep.keep_words; a.act = ep.act; a.pre_out = ep.pre_out; a.alone = ep.alone ? 1 : 0;
+    a.keep_words = ep.keep_words; a.act = ep.act; a.pre_out = ep.pre_out; a.alone = ep.alone ? 1 : 0; a.same_order = ep.same_order ? 1 : 0;
     if (ep.alone) a.gate_bits_out = nullptr;
     a.splits = 1; a.partial = nullptr;
     c.ok_c = a.sCN == 1;
@@ -237,7 +237,15 @@ TileChoice choose_single(const TileProduct& p, size_t ws_floats, double reduce_u
 // cost more than they gave where the fp32 sums are many: us of lin2 and the LayerNorm behind it, 2613 x 768 x 3072 in two parts
 // 32 and in one 29, 1024 x 768 x 3072 in five 21.4 and in one 19.9; and a product of 512 x 4096 x 1024 in two parts had no activation
 // in its epilogue, 28 with its activation and now 14.)
+// In front of a ReLU the rule is that of old, which fills the CUs as long as eight steps a part are left of it.
 int forward_splits(const TileProduct& p) {
+    if (p.a.same_order) {
+        const long tiles = (long)((p.a.M + 127) / 128) * ((p.a.N + 127) / 128) * p.a.nbatch;
+        const int nkt = p.a.K0 * ((p.a.K1 + BK - 1) / BK);
+        int splits = (int)std::min(kSplitTarget / tiles, 8L);
+        while (splits > 1 && nkt / splits < 8) --splits;
+        return p.a.N % 4 != 0 || (size_t)p.a.nbatch * p.a.M * p.a.N > kSplitMaxOut ? 1 : std::max(splits, 1);
+    }
     const bool widens = p.a.N > (long)p.a.K0 * p.a.K1;
     return choose_single(p, split_floats(p.a.M, p.a.N, p.a.nbatch), widens ? kReduceLaunch : 1.4).splits;
 }
@@ -424,7 +432,8 @@ void launch_gemm(const GemmShape& s, const half_t* A, const half_t* B, half_t* C
         }
         const bool small = ws && (size_t)batch * c.a.M * c.a.N <= kSplitMaxOut;
         if (small && !ep.any_split) tp.a.splits = forward_splits(tp);
-        const TileChoice choice = choose_single(tp, small && ep.any_split ? ws_floats : 0);
+        const unsigned forms = !tp.a.same_order ? forms_for(&tp, 1) : summed_wide(tp) ? 1u << TILE_256x256 : kRingForms;
+        const TileChoice choice = choose_tiles(&tp, 1, forms, small && ep.any_split ? ws_floats : 0);
         unsigned side_blocks = 0;
         if (side) side->tiles_done = 0;
         if (side && side->keep && side->key.thr && choice.form == TILE_256x256 && choice.splits == 1) {

@@ -19,6 +19,13 @@ constexpr Form kForms[TILE_FORMS] = {
     {256, 128, 1, 0.56, 0.62, 0.92, 5.9, 2.0},
     {256, 256, 1, 1.02, 1.25, 1.47, 5.5, 4.3},
 };
+// The last two as they were when the order of the sums in front of a ReLU was fixed (GemmEpilogue::same_order): which products go into
+// 256 x 256 tiles is decided by these there.
+constexpr Form kOrderForms[2] = {
+    {256, 128, 1, 0.52, 0.54, 0.83, 5.9, 2.0},
+    {256, 256, 1, 1.00, 1.00, 1.42, 5.5, 4.3},
+};
+inline const Form& form_of(int f, bool order) { return order && f >= TILE_256x128 ? kOrderForms[f - TILE_256x128] : kForms[f]; }
 // Several products of more than a round of the smaller tiles: the workgroups drift apart, and share fewer lines of their L2
 // (4096 x 1024 x 4096 twice in tiles of 128 x 128: 75.5 us, 3 times 117 and once 38.5).
 constexpr double kDrift = 1.12;
@@ -216,12 +223,12 @@ TileForm tile_form(int form) {
 // for 30.2 alone, 32.6 for 31.6 within the layer) and ReLU's backward at 2560 x 2048 x 512 (24.4 for 22.2): the four stay.  Against
 // the best tiles in brackets this takes at 1848 rows 20.2 (20.2), 23.3 (23.3), 23.7 (23.0), 28.1 (28.1) us in the order of the
 // rows, at 2613 24.4 (24.4), 30.2 (29.5), 24.5 (24.5), 30.0 (30.0).
-int choose_act_form(const TileProduct& p) {
+static int best_act_form(const TileProduct& p, unsigned forms, bool order) {
     int best = -1;
     double best_us = 0.;
     for (int f = 0; f < TILE_FORMS; ++f) {
-        if (f == TILE_256x256 ? !wide_takes(p) : !p.akc) continue;
-        const Form& F = kForms[f];
+        if (!(forms >> f & 1u) || (f == TILE_256x256 ? !wide_takes(p) : !p.akc)) continue;
+        const Form& F = form_of(f, order);
         const long len = steps_of(p.a, 1), cnt = tiles_of(p.a, 1, F.bm, F.bn);
         const double packs = (double)F.bm * F.bn / (4 * 64 * 8) * F.per_cu, draw = p.a.gate ? 0. : f == TILE_256x256 ? 0.13 : 0.2;
         const double rounds = (double)((cnt + 256L * F.per_cu - 1) / (256L * F.per_cu));
@@ -229,6 +236,24 @@ int choose_act_form(const TileProduct& p) {
         if (best < 0 || us < best_us) { best = f; best_us = us; }
     }
     return best;
+}
+
+int choose_act_form(const TileProduct& p) {
+    constexpr unsigned all = kRingForms | 1u << TILE_256x256;
+    if (!p.a.same_order) return best_act_form(p, all, false);
+    const int form = best_act_form(p, all, true);
+    return form == TILE_256x256 || form < 0 ? form : best_act_form(p, kRingForms, false);
+}
+
+bool summed_wide(const TileProduct& p) {
+    if (!wide_takes(p)) return false;
+    double us[TILE_FORMS];
+    for (int f = 0; f < TILE_FORMS; ++f) {
+        const Form& F = form_of(f, true);
+        const long len = steps_of(p.a, p.a.splits), cnt = tiles_of(p.a, p.a.splits, F.bm, F.bn);
+        us[f] = launch_us(&len, &cnt, 1, F);
+    }
+    return us[TILE_256x256] < *std::min_element(us, us + TILE_256x256);
 }
 
 void launch_tiles_act(const TileProduct& p, int form, hipStream_t st) {

@@ -31,6 +31,7 @@ struct GemmArgs {
     const uint32_t* gate_bits = nullptr;   // gate: those bits instead of the values of `gate`
     int act = ACT_RELU;                    // the activation of relu_dropout / gate (GemmEpilogue::act)
     half_t* pre_out = nullptr;             // GELU with dropout: where the rounded sum before the activation goes
+    int same_order = 0;                    // GemmEpilogue::same_order
     int alone = 0;                         // no backward pass follows (GemmEpilogue::alone)
     // GemmSideJob of the 256 x 256 kernel: the workgroups behind those of the tiles draw
     // the attention keep words of key tiles 0 .. side_tiles_done - 1 of side_rows score rows
@@ -169,6 +170,8 @@ struct TileForm { int bm, bn, per_cu; double out_steps; };
 TileForm tile_form(int form);
 // The best form for a product with an activation in its epilogue (-1: none), and its launch.
 int choose_act_form(const TileProduct& p);
+// With same_order: whether the product is summed in the order of 256 x 256 tiles (k slices of 32; the others': 16).
+bool summed_wide(const TileProduct& p);
 void launch_tiles_act(const TileProduct& p, int form, hipStream_t st);
 // k_gemm_wide.hip: 256 x 256 tiles.
 bool wide_takes(const TileProduct& p);

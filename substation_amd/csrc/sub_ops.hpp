@@ -253,9 +253,11 @@ struct GemmEpilogue {
     int act = ACT_RELU;
     half_t* pre_out = nullptr;
     bool alone = false;          // relu_dropout: no backward pass follows; pre_out and gate_bits_out are not written
-    // the contraction of a small output may be split in as many parts as is fastest; otherwise their number, and with it the
-    // order of the sums, depends on the shape alone (one unit of the last place of a pre-activation decides a ReLU's gate)
+    // the contraction of a small output may be split in as many parts as is fastest within the scratch at hand
     bool any_split = false;
+    // in front of a ReLU: the order of the sums is a fixed function of the shape, whatever is fastest (one unit of the last place
+    // of a pre-activation decides a gate, and a gate moves whole rows of gradients)
+    bool same_order = false;
     // where given, and the product is split, has dense rows and no addend: it is left as the sums of its splits
     SplitSums* sums = nullptr;
 };
