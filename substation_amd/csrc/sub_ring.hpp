@@ -1,4 +1,4 @@
-// Contractions in a ring of LDS stages with waves of their own for the fetching; one launch takes up to three products.
+// Contractions in a ring of LDS stages with waves of their own for the fetching; one launch takes up to kMaxProducts products.
 //
 // What bounds a product here is how fast a CU draws its operands: 51 bytes a cycle of lines that its L2 has, 12 of lines
 // that it has not, so about 31 where a fifth is missing (4096 x 1024 x 4096: 512 MiB drawn, 104 of them from beyond the L2s;
@@ -10,12 +10,13 @@
 // one inside does (the kernel before predicated every load of such a product).  M = 2613 rows, us before and now:
 // 768 x 3072 (n x k) 35 -> 21, 3072 x 768 21 -> 18.5, its weight gradient 42 -> 20.5; 64 rows x 768 x 768: 14 -> 6.4; 4096 x 1024 x
 // 4096: 43 -> 35-37 (930 to 990 TFLOP/s, box to box).  4096 x 1024 x 1024, one tile of 16 steps per CU, takes 15 to 17 us.
-// Registers without an activation: 72 to 168 a lane up to 128 x 128 tiles, 242 to 256 at 256 x 128, where the instance of two
-// orientations (two loop bodies) spills two of them (12 bytes of scratch) and that of one product with both operands across k one;
+// Registers without an activation: 72 to 168 a lane up to 128 x 128 tiles, 242 to 256 at 256 x 128, where the instance of data and weight
+// gradients (two loop bodies) spills two of them (12 bytes of scratch) and that of one product with both operands across k one;
 // the instances of one product hold its arguments in scalar registers and spill 26 to 36 of those, the ones of several
-// products none.  With one: 85 to 212 up to 128 x 128 (128 x 64 with GELU: 20 bytes of scratch), 253 to 256 at 256 x 128, where
-// GELU spills 2 to 7 (12 to 32 bytes), ReLU's gate 44 to 50 (180 to 204), GELU's backward form 56 to 61 (228 to 248), all in the
-// epilogue; 27 to 39 scalar registers backward, 90 to 125 forward (the keys and constants of the draws).
+// products none.  With one: 85 to 212 up to 128 x 128 (128 x 64 with GELU, and 64 x 64 with GELU where no gradient is wanted: 20 bytes of
+// scratch), 251 to 256 at 256 x 128, where GELU spills 2 to 7 (12 to 32 bytes; none where no gradient is wanted), ReLU's gate 44 to 50
+// (180 to 204), GELU's backward form 56 to 61 (228 to 248), all in the epilogue; 27 to 39 scalar registers backward, 76 to 125 forward
+// (the keys and constants of the draws).
 #pragma once
 
 #include "sub_tiles.hpp"

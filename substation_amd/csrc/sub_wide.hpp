@@ -25,9 +25,9 @@
 // half's resource is fixed for a tile and a step is one scalar offset), a branch around the wait at each quarter, and the
 // epilogue's slab written and read in turn (now four of them, two ahead).
 // 256 x 128 tiles in this manner take 60 us for 4096 x 2048 x 4096, as those of k_gemm_ring do: the operand fetch bounds them.
-// Registers: 171 to 193 and the 256 accumulation registers, 192 to 206 with an activation, none of them spilled.  The instances of one
+// Registers: 163 to 191 and the 256 accumulation registers, 188 to 206 with an activation, none of them spilled.  The instances of one
 // product hold its arguments in scalar registers and spill 84 to 96 of those (to lanes of vector registers), with an activation
-// 105 to 213, on the way into and out of a tile; those of several products 0, of two orientations 49.
+// 105 to 217, on the way into and out of a tile; those of several products 0, of two orientations 65 or 66.
 #pragma once
 
 #include "sub_tiles.hpp"
