@@ -253,7 +253,7 @@ struct Handle {
     bool left_nothing = false;        // and none can follow the latest one
     int form_given = -1;              // the same of the forward call that the next backward call belongs to, if it was said
     BackwardPlan plan;                // see backward_plan()
-    uint64_t plan_key = 0;
+    uint64_t plan_key = 0;            // 0: none (plan_layouts, which every change of sizes or orders goes through, drops it)
     size_t plan_ws = 0;
     std::vector<ProfEntry> prof;
     size_t prof_used = 0;
@@ -430,7 +430,6 @@ void configure(Handle& h, const sub_config* c) {
     const float ps[4] = {c->p_softmax, c->p_resid1, c->p_act, c->p_resid2};
     for (float p : ps) if (!(p >= 0.f && p <= 1.f)) fail("sub_configure: dropout probability outside [0,1]");
     h.configured = false;
-    h.plan_key = 0;
     // a handle that is configured again forgets the attention mask of its old sizes
     // (the table of what the mask leaves to do was sized for them)
     if (h.mask_plan) {
@@ -479,6 +478,7 @@ bool whole_round(const GemmShape& s) {
 // its own weight orders.
 void plan_layouts(Handle& h, bool own) {
     const Sizes& sz = h.sz;
+    h.plan_key = 0;                   // (what was planned for the orders of before)
     static const char* const kOwnP[SUB_N_PARAMS] = {"QHPI", "QHP", "IHP", "I", "I", "I", "U", "UI", "I", "I", "I", "IU"};
     static const char* const kOwnF[SUB_N_FWD] = {
         "QBJHP", "QBJHP", "HBJK", "HBJK", "HBJK", "HBJK", "BJHP", "BJI", "BJI", "BJI", "BJU", "BJU", "BJU",
@@ -695,8 +695,8 @@ void run_stage(Handle& h, const GemmJob* jobs, const GemmStage& s, FinishJobs* t
     }
 }
 
-// The plan for these products, kept as long as what it was made from stays the same: the configuration, the options, which
-// operands are 16-byte aligned, and the scratch at hand.  (Making it takes 30 to 110 us.)
+// The plan for these products, kept as long as what it was made from stays the same: sizes and dimension orders (plan_layouts), the
+// options, which operands are 16-byte aligned, and the scratch at hand.  (Making it takes 30 to 110 us.)
 const BackwardPlan& backward_plan(Handle& h, const GemmJob (&jobs)[7], bool late, bool fuse_dx) {
     ensure_gws(h, h.gws_need);
     uint64_t key = 1u | (h.pair_products ? 2u : 0u) | (late ? 4u : 0u) | (h.finish_in_pair ? 8u : 0u) | (fuse_dx ? 16u : 0u);
@@ -705,6 +705,7 @@ const BackwardPlan& backward_plan(Handle& h, const GemmJob (&jobs)[7], bool late
         for (int k = 0; k < 4; ++k) key |= (reinterpret_cast<uintptr_t>(operand[k]) & 15 ? 1ull : 0ull) << (8 + 4 * i + k);
     }
     if (key == h.plan_key && h.gws_floats == h.plan_ws) return h.plan;
+    h.plan_key = 0;
     plan_backward_products(jobs, h.pair_products, late, h.gws_floats, h.plan);
     if (!h.finish_in_pair) {
         // dWout next to dXout (the others where and as they are with that option, so that they stay the same bit for bit)

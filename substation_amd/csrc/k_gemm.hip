@@ -391,13 +391,23 @@ void plan_backward_products(const GemmJob (&jobs)[7], bool together, bool late, 
 
 void launch_gemm_together(const GemmJob* jobs, const GemmLaunch& l, hipStream_t st, float* ws, size_t ws_floats, FinishJobs* tail) {
     TileProduct p[kMaxProducts];
+    int k1, k2;
+    bool fits = l.form >= 0 && l.form < TILE_FORMS;
     for (int i = 0; i < l.n; ++i) {
-        if (!take(jobs[l.job[i]], p[i])) fail("gemm: these products do not share a launch");
-        if (l.splits > 1 && l.split == i) {
-            if ((size_t)p[i].a.nbatch * p[i].a.M * p[i].a.N * l.splits > ws_floats) fail("gemm: no room for the sums of a split product");
+        fits = fits && take(jobs[l.job[i]], p[i]) && (l.form != TILE_256x256 || (l.splits == 1 && wide_takes(p[i])));
+        if (fits && l.splits > 1 && l.split == i) {
+            fits = p[i].a.N % 4 == 0 && (size_t)p[i].a.nbatch * p[i].a.M * p[i].a.N * l.splits <= ws_floats;
             p[i].a.splits = l.splits;
             p[i].a.partial = ws;
         }
+    }
+    if (!fits || !orientations(p, l.n, k1, k2)) {
+        // (a plan that is not one for these products: none that is kept should be)
+        for (int i = 0; i < l.n; ++i) {
+            const GemmJob& j = jobs[l.job[i]];
+            launch_gemm(*j.shape, j.A, j.B, j.C, j.alpha, j.ep, st, ws, ws_floats);
+        }
+        return;
     }
     // (none of the column sums in `tail` may be one that this launch itself contributes to)
     launch_tiles(p, l.n, l.form, tail, st);

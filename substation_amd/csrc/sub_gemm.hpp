@@ -145,6 +145,15 @@ struct TileProduct {
     GemmArgs a;                   // with splits (and, if more than one, partial) and nbatch set
     bool akc, bkc;                // operands contiguous along k
 };
+// Products of one launch may be read in one way, or in the two of which an instance exists.
+inline bool orientations(const TileProduct* p, int n, int& k1, int& k2) {
+    int seen = 0;
+    for (int i = 0; i < n; ++i) seen |= 1 << ((p[i].akc ? 1 : 0) | (p[i].bkc ? 2 : 0));
+    for (int k = 0; k < 4; ++k)
+        if (seen == 1 << k) { k1 = k2 = k; return true; }
+    k1 = seen == 9 ? 3 : 1; k2 = 0;
+    return seen == 3 || seen == 9;
+}
 // Which workgroup takes which tiles of a launch's list (tiles of the same length next to each other, the longest in front):
 // `rounds` rounds of all workgroups, tile r n + l to workgroup l, then parts of the list that go to neighbouring workgroups.
 struct SchedulePart { unsigned worker, tile, count; };

@@ -235,16 +235,6 @@ inline long tiles_of(const GemmArgs& a, int splits, int bm, int bn) {
 }
 inline long steps_of(const GemmArgs& a, int splits) { return ((long)a.K0 * ((a.K1 + BK - 1) / BK) + splits - 1) / splits; }
 
-// Products of one launch may be read in one way, or in the two of which an instance exists.
-inline bool orientations(const TileProduct* p, int n, int& k1, int& k2) {
-    int seen = 0;
-    for (int i = 0; i < n; ++i) seen |= 1 << ((p[i].akc ? 1 : 0) | (p[i].bkc ? 2 : 0));
-    for (int k = 0; k < 4; ++k)
-        if (seen == 1 << k) { k1 = k2 = k; return true; }
-    k1 = seen == 9 ? 3 : 1; k2 = 0;
-    return seen == 3 || seen == 9;
-}
-
 // The indices of n products, longest contraction first.
 inline void longest_first(const TileProduct* p, int n, int (&order)[kMaxProducts]) {
     for (int i = 0; i < n; ++i) order[i] = i;

@@ -1,0 +1,60 @@
+"""Which launches a call makes, and that what is kept from one call to the next does not change them (on the CPU: tests/launches.py)."""
+import copy
+import ctypes
+import itertools
+
+import pytest
+
+import tests.launches as launches
+
+
+def _pointers(addresses):
+    return (ctypes.c_void_p * len(addresses))(*addresses), len(addresses)
+
+
+def _pass(lib, check, handle):
+    """The launches of a forward and a backward call (layer calls with 37 and 64 tensors, all of them aligned)."""
+    forward = launches.tensors(37)
+    backward = launches.tensors(64, first=64)
+    return launches.launched(lambda: (check(lib.sub_encoder_forward(handle.ptr, *_pointers(forward))),
+                                      check(lib.sub_encoder_backward(handle.ptr, *_pointers(backward)))))
+
+
+def _orders(L, which):
+    lay = copy.deepcopy(L.mi355x_layouts() if which == 'own' or which == 'token-contiguous'
+                        else L.reference_layouts('bert-b8-l512-h16-e1024'))
+    # feed-forward tensors with the tokens contiguous: weight gradients whose operands both lie along their contraction
+    other = {'token-contiguous': dict(DLIN1='UBJ', DROP2='UBJ', LIN1='UBJ', SB1='IBJ', DLIN2='IBJ', WKQV='QIHP'),
+             'reference-but-LINW1': dict(LINW1='UI')}.get(which, {})
+    for group in ('params', 'forward_interm', 'backward_interm'):
+        lay[group] = [(name, other.get(name, order)) for name, order in lay[group]]
+    return lay
+
+
+def _options_between_passes():
+    from substation_amd import _lib, layouts as L
+    lib = _lib.load()
+    # (weight gradients over 4096 tokens, over 4000, which is no multiple of 64, and over 215, which is none of 8)
+    for which, (B, S, H, E) in itertools.product(('own', 'reference', 'reference-but-LINW1', 'token-contiguous'),
+                                                 ((8, 512, 16, 1024), (8, 500, 16, 1024), (5, 43, 4, 256))):
+        for option, value in ((11, 0), (11, 1), (5, 0), (7, 0), (3, 0), (1, 0), (2, 0), (4, 0), (12, 1)):
+            def handle():
+                return _lib.Handle(_lib.make_config(B, S, H, E, _orders(L, which), 0.1, 0.1, 0.1, 0.1, activation='gelu'))
+            fresh, used = handle(), handle()
+            if (option, value) == (11, 1):
+                used.set_option(11, 0)
+            _pass(lib, _lib.check, used)
+            used.set_option(option, value)
+            fresh.set_option(option, value)
+            try:
+                got, want = _pass(lib, _lib.check, used), _pass(lib, _lib.check, fresh)
+                at = next((i for i, (a, b) in enumerate(itertools.zip_longest(got, want)) if a != b), None)
+                print('same' if at is None else f'{which} {B}x{S} option {option}={value}: {got[at:at + 1]} for {want[at:at + 1]}')
+            except _lib.SubstationError as e:
+                print(f'{which} {B}x{S} option {option}={value}: {e}')
+
+
+def test_options_that_change_between_passes(tmp_path):
+    """A handle whose options change after a pass launches what one does that had them from the start."""
+    lines = launches.run(_options_between_passes, tmp_path)
+    assert len(lines) == 4 * 3 * 9 and set(lines) == {'same'}, [l for l in lines if l != 'same']

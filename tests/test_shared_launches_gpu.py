@@ -81,3 +81,35 @@ def test_group_of_contractions_gives_what_each_of_them_gives(dims, source):
     for (_, _, la, _, lb, c, lc, *_), want in zip(products, alone):
         # fp32 sums in another order, rounded once
         assert_close(c.float().cpu().numpy(), want.float().cpu().numpy(), tol=2e-3, name=f'{la},{lb}->{lc}')
+
+
+@pytest.mark.parametrize('dims', [(8, 500, 16, 1024), (5, 43, 4, 256)])
+def test_products_after_a_change_of_dimension_orders(dims):
+    """Gradients of a layer whose tensors are no longer kept in the library's own orders (option 11) after a pass in them, against one
+    that never was in them: tokens contiguous in the feed-forward block, 4000 of them, which is no multiple of 64, and 215."""
+    from substation_amd import Encoder, layouts as L
+    B, Ls, H, E = dims
+    lay = dict(L.mi355x_layouts())
+    other = dict(DLIN1='UBJ', DROP2='UBJ', LIN1='UBJ', SB1='IBJ', DLIN2='IBJ', WKQV='QIHP')
+    for group in ('params', 'forward_interm', 'backward_interm'):
+        lay[group] = [(name, other.get(name, order)) for name, order in lay[group]]
+    g = torch.Generator('cuda').manual_seed(3)
+    X, DY = (torch.randn(B, Ls, E, generator=g, device='cuda').half() for _ in range(2))
+    grads = []
+    for before in (False, True):
+        torch.manual_seed(0)
+        with torch.device('cuda'):
+            enc = Encoder('unused', B, Ls, H, E, lay, torch.float16, 0.1, 0.1, 0.1, 0.1, seed=7, activation='gelu')
+        with torch.no_grad():
+            for q in enc.parameters():
+                q.mul_(0.1)
+        if before:
+            enc(X.clone().requires_grad_()).backward(DY)
+            enc.zero_grad(set_to_none=True)
+        enc._handle.set_option(11, 0)
+        enc.set_rng(7, 0)
+        x = X.clone().requires_grad_()
+        enc(x).backward(DY)
+        grads.append([x.grad] + [q.grad for q in enc.parameters()])
+    for a, b in zip(*grads):
+        assert torch.equal(a, b)
