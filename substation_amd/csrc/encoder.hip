@@ -2293,6 +2293,7 @@ int sub_op_einsum_group(void* handle, const SubEinsum* p, int n) {
     return guarded([&] {
         Handle& h = as_handle(handle); need_cfg(h);
         if (n < 0 || n > 2 * kMaxProducts) fail("sub_op_einsum_group: at most " + std::to_string(2 * kMaxProducts) + " products");
+        if (n > 0 && !p) fail("sub_op_einsum_group: null products");
         std::vector<GemmShape> shape(n);
         std::vector<GemmJob> jobs(n);
         size_t need = 0;

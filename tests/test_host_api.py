@@ -271,3 +271,11 @@ def test_intermediates_are_opaque_to_the_module_and_open_to_a_c_caller():
     assert _handle().get_option(_lib.OPT_OPAQUE_INTERMEDIATES) == 0
     assert enc(False)._handle.get_option(_lib.OPT_OPAQUE_INTERMEDIATES) == 1
     assert enc(True)._handle.get_option(_lib.OPT_OPAQUE_INTERMEDIATES) == 0
+
+
+def test_a_group_of_contractions_without_its_products_is_refused():
+    h = _handle()
+    for n in (1, 14):
+        with pytest.raises(_lib.SubstationError, match='null products'):
+            _lib.check(h.lib.sub_op_einsum_group(h.ptr, None, n))
+    _lib.check(h.lib.sub_op_einsum_group(h.ptr, None, 0))
