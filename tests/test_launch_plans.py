@@ -58,3 +58,50 @@ def test_options_that_change_between_passes(tmp_path):
     """A handle whose options change after a pass launches what one does that had them from the start."""
     lines = launches.run(_options_between_passes, tmp_path)
     assert len(lines) == 4 * 3 * 9 and set(lines) == {'same'}, [l for l in lines if l != 'same']
+
+
+# the ten products that a decoder layer has at the end of its backward pass: layouts of A, B, C and of an addend; which of its two
+# sequence lengths they are over
+GROUP = [('QHPI', 'QBJHP', 'BJI', 'BJI', 0), ('BKHP', 'HPI', 'BKI', 'BKI', 1), ('BKHP', 'BKI', 'HPI', None, 1),
+         ('BKHP', 'BKI', 'HPI', None, 1), ('QBJHP', 'BJI', 'QHPI', None, 0), ('BJI', 'BJHP', 'IHP', None, 0),
+         ('BJHP', 'BJI', 'HPI', None, 0), ('BJI', 'BJHP', 'IHP', None, 0), ('BJU', 'BJI', 'UI', None, 0), ('BJI', 'BJU', 'IU', None, 0)]
+
+
+class Group:
+    """GROUP as a call on a handle of one size, some of the products by another handle's."""
+
+    def __init__(self, B=8, S=256, H=16, E=1024, source=512, options=()):
+        from substation_amd import _lib, layouts as L
+        self.l, self.lib = _lib, _lib.load()
+        self.handles = [_lib.Handle(_lib.make_config(B, s, H, E, L.mi355x_layouts())) for s in (S, source)]
+        for option, value in options:
+            self.handles[0].set_option(option, value)
+        self.products = (_lib.Einsum * len(GROUP))()
+        at = itertools.count(1)
+        for q, (la, lb, lc, lt, which) in zip(self.products, GROUP):
+            q.sizes = self.handles[which].ptr
+            q.A, q.B, q.C = (next(at) << 36 for _ in range(3))
+            q.l_A, q.l_B, q.l_C = la.encode(), lb.encode(), lc.encode()
+            if lt:
+                q.T, q.l_T = q.C, lt.encode()
+            q.alpha = 1.0
+
+    def launched(self):
+        return launches.launched(
+            lambda: self.l.check(self.lib.sub_op_einsum_group(self.handles[0].ptr, self.products, len(self.products))))
+
+
+def _timed_operator_calls():
+    from substation_amd import _lib
+    g = Group()
+    g.handles[0].profile_enable()
+    for _ in range(5):
+        g.launched()
+        a, b = launches.tensors(2)
+        _lib.check(g.lib.sub_op_relayout(g.handles[0].ptr, a, b'BJI', b, b'IBJ'))
+    print(launches.recorder.recorder_events())
+
+
+def test_operator_calls_leave_nothing_in_a_handles_timing(tmp_path):
+    """Entries of the per-launch timing are begun anew by the next layer call; a handle that operator calls are made on has none."""
+    assert launches.run(_timed_operator_calls, tmp_path) == ['0']
