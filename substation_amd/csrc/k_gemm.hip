@@ -319,44 +319,42 @@ void GemmLaunch::drop(int j) {
 // 77 -> 36 us).
 double plan_gemm_stage(const GemmJob* jobs, const int* ids, int n, bool together, size_t ws_floats, GemmStage& out) {
     TileProduct p[kMaxProducts];
-    bool ok[kMaxProducts], all = n > 1 && n <= kMaxProducts && together;
+    int id[kMaxProducts], m = 0;                         // the jobs that tiles take
     double alone[kMaxProducts], sum = 0.;
-    for (int i = 0; i < n; ++i) {
-        ok[i] = take(jobs[ids[i]], p[i]);
-        all = all && ok[i];
-        const bool small = ok[i] && (size_t)p[i].a.nbatch * p[i].a.M * p[i].a.N <= kSplitMaxOut;
-        alone[i] = ok[i] ? choose_single(p[i], small ? ws_floats : 0).us : 0.;
-        sum += alone[i] + (i ? kGap : 0.);
-    }
-    double best = sum;
-    out.n = n;
-    for (int i = 0; i < n; ++i) {
-        out.launch[i] = GemmLaunch{};
-        out.launch[i].n = 1; out.launch[i].job[0] = ids[i];
-    }
-    // jobs `from` .. of the list in one launch, those in front of it alone
-    auto share = [&](int from) {
-        const TileChoice c = choose_tiles(p + from, n - from, forms_for(p + from, n - from), ws_floats);
-        const double us = c.us + (from ? alone[0] + kGap : 0.);
-        if (c.form < 0 || us >= best) return;
-        best = us;
-        out.n = from + 1;
-        GemmLaunch& l = out.launch[from];
-        l.n = n - from;
-        for (int i = from; i < n; ++i) l.job[i - from] = ids[i];
-        l.form = c.form; l.split = c.split; l.splits = c.splits;
+    out.n = 0;
+    auto launch = [&](const int* job, int count) -> GemmLaunch& {
+        GemmLaunch& l = out.launch[out.n++];
+        l = GemmLaunch{};
+        l.n = count;
+        for (int i = 0; i < count; ++i) l.job[i] = job[i];
+        return l;
     };
-    if (n > 2) {
-        bool rest = together;
-        for (int i = 1; i < n; ++i) rest = rest && ok[i];
-        if (rest) share(1);
+    for (int i = 0; i < n; ++i) {
+        sum += i ? kGap : 0.;
+        if (!take(jobs[ids[i]], p[m])) {                 // (misaligned, say: by itself, and the others without it)
+            launch(ids + i, 1);
+            continue;
+        }
+        const bool small = (size_t)p[m].a.nbatch * p[m].a.M * p[m].a.N <= kSplitMaxOut;
+        alone[m] = choose_single(p[m], small ? ws_floats : 0).us;
+        sum += alone[m];
+        id[m++] = ids[i];
     }
-    if (all) {
-        const GemmStage before = out;
-        const double was = best;
-        out.launch[0] = GemmLaunch{};
-        share(0);
-        if (best == was) out = before;
+    const double in_front = kGap * out.n;
+    double best = sum;
+    TileChoice how;
+    int from = m;                                        // jobs `from` .. of the list in one launch, those in front of it alone
+    for (int f : {1, 0}) {
+        if (!together || m - f < 2) continue;
+        const TileChoice c = choose_tiles(p + f, m - f, forms_for(p + f, m - f), ws_floats);
+        const double us = in_front + c.us + (f ? alone[0] + kGap : 0.);
+        if (c.form < 0 || us >= best) continue;
+        best = us; how = c; from = f;
+    }
+    for (int i = 0; i < from; ++i) launch(id + i, 1);
+    if (from < m) {
+        GemmLaunch& l = launch(id + from, m - from);
+        l.form = how.form; l.split = how.split; l.splits = how.splits;
     }
     return best;
 }

@@ -304,8 +304,8 @@ struct GemmStage {
     int n = 0;
     GemmLaunch launch[kMaxProducts];
 };
-// The fastest of: jobs ids[0 .. n - 1] in one launch, the first apart from the rest, each of them alone.  What it is expected
-// to take (us).  together: whether any may share a launch at all.
+// The fastest of: jobs ids[0 .. n - 1] in one launch, the first apart from the rest, each of them alone (as those that the tiles do
+// not take are in any case).  What it is expected to take (us).  together: whether any may share a launch at all.
 double plan_gemm_stage(const GemmJob* jobs, const int* ids, int n, bool together, size_t ws_floats, GemmStage& out);
 // One launch of more than one product, or of one whose form is set.  `tail` (optional): deferred column sums of EARLIER launches,
 // finished by extra workgroups of this launch; tail->n is set to 0 when they were taken, else it is left as it was.

@@ -105,3 +105,21 @@ def _timed_operator_calls():
 def test_operator_calls_leave_nothing_in_a_handles_timing(tmp_path):
     """Entries of the per-launch timing are begun anew by the next layer call; a handle that operator calls are made on has none."""
     assert launches.run(_timed_operator_calls, tmp_path) == ['0']
+
+
+def _misaligned_members():
+    for odd in (None, 2, 4, 9):          # (those without an addend: it is refused with one)
+        g = Group()
+        if odd is not None:
+            g.products[odd].B += 2
+        names = [name for name, _ in g.launched()]
+        print(sum('k_gemm_fma' in n for n in names), sum('ILi7E' in n or 'Li7ELi' in n for n in names), len(names))
+
+
+def test_a_misaligned_member_of_a_group_runs_alone(tmp_path):
+    """One product that the tiles do not take (an operand that is an odd slice of a buffer): a launch more, and no others'."""
+    lines = [tuple(int(x) for x in l.split()) for l in launches.run(_misaligned_members, tmp_path)]
+    whole, *rest = lines
+    assert whole[0] == 0 and whole[1] >= 1
+    for scalar, shared, total in rest:
+        assert scalar == 1 and shared >= 1 and total <= whole[2] + 1
