@@ -184,6 +184,13 @@ __global__ void k_clock_sample(unsigned long long* slot) {
     slot[2 * blockIdx.x + 1] = wall_clock64();
 }
 
+// The launches of a group of contractions, by all that they depend on.
+struct GroupPlan {
+    std::vector<int64_t> asked;
+    GemmStage stage[2];
+};
+constexpr size_t kMaxGroups = 8;
+
 struct Handle {
     bool configured = false;
     Sizes sz;
@@ -255,6 +262,8 @@ struct Handle {
     BackwardPlan plan;                // see backward_plan()
     uint64_t plan_key = 0;            // 0: none (plan_layouts, which every change of sizes or orders goes through, drops it)
     size_t plan_ws = 0;
+    std::vector<GroupPlan> groups;    // see group_plan()
+    size_t group_next = 0;            // the one that makes room
     std::vector<ProfEntry> prof;
     size_t prof_used = 0;
     size_t prof_forward = 0;          // entries of the last forward call, kept by the backward call after it
@@ -738,6 +747,51 @@ const BackwardPlan& backward_plan(Handle& h, const GemmJob (&jobs)[7], bool late
     h.plan_key = key;
     h.plan_ws = h.gws_floats;
     return h.plan;
+}
+
+// The launches of a group of contractions: the longest first, in one launch or, from some place of that order on, in another.  Kept for the
+// last groups asked for (a decoder layer's backward pass has two): shapes, strides, alignments, the option and the scratch are all that
+// they depend on.  Ten products of 8 x 256 on 512, E 1024: a call that
+// makes its plan takes the host 31 us with every choice of tiles at hand and 130 without, one that finds it 14, and a decoder layer of that
+// size waits for its host.
+const GroupPlan& group_plan(Handle& h, const std::vector<GemmJob>& jobs) {
+    const int n = (int)jobs.size();
+    GroupPlan q;
+    q.asked.reserve(2 + 33 * jobs.size());
+    q.asked.push_back(h.pair_products);
+    q.asked.push_back((int64_t)h.gws_floats);
+    for (const GemmJob& j : jobs) {
+        const GemmShape& s = *j.shape;
+        const GemmEpilogue& e = j.ep;
+        for (int64_t v : {s.M, s.N, s.K0, s.K1, s.sAM, s.sAK1, s.sAK0, s.sBN, s.sBK1, s.sBK0, s.sCM, s.sCN, e.sbM, e.sbN}) q.asked.push_back(v);
+        for (int i = 0; i < 3; ++i)
+            for (int64_t v : {s.nb[i], s.sAb[i], s.sBb[i], s.sCb[i], e.sbb[i]}) q.asked.push_back(v);
+        int64_t bits = e.bias ? 1 : 0;
+        for (const void* p : {(const void*)j.A, (const void*)j.B, (const void*)j.C, (const void*)e.bias})
+            bits = 2 * bits + (reinterpret_cast<uintptr_t>(p) & 15 ? 1 : 0);
+        q.asked.push_back(bits);
+    }
+    for (const GroupPlan& g : h.groups)
+        if (g.asked == q.asked) return g;
+    std::vector<int> order(n);
+    for (int i = 0; i < n; ++i) order[i] = i;
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return jobs[x].shape->K() > jobs[y].shape->K(); });
+    double us = -1.;
+    for (int cut = std::max(1, n - kMaxProducts); cut <= std::min(n, kMaxProducts); ++cut) {
+        GemmStage tried[2];
+        double t = plan_gemm_stage(jobs.data(), order.data(), cut, h.pair_products, h.gws_floats, tried[0]);
+        if (cut < n) t += 1.5 + plan_gemm_stage(jobs.data(), order.data() + cut, n - cut, h.pair_products, h.gws_floats, tried[1]);
+        if (us >= 0. && t >= us) continue;
+        us = t;
+        q.stage[0] = tried[0]; q.stage[1] = tried[1];
+    }
+    if (h.groups.size() < kMaxGroups) {
+        h.groups.push_back(std::move(q));
+        return h.groups.back();
+    }
+    GroupPlan& at = h.groups[h.group_next++ % kMaxGroups];
+    at = std::move(q);
+    return at;
 }
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -2322,22 +2376,8 @@ int sub_op_einsum_group(void* handle, const SubEinsum* p, int n) {
         }
         if (n == 0) return;
         ensure_gws(h, need);
-        // the longest contractions first, in one launch or, from some place of that order on, in another
-        std::vector<int> order(n);
-        for (int i = 0; i < n; ++i) order[i] = i;
-        std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return shape[x].K() > shape[y].K(); });
-        GemmStage best[2], tried[2];
-        double us = -1.;
-        for (int cut = std::max(1, n - kMaxProducts); cut <= std::min(n, kMaxProducts); ++cut) {
-            double t = plan_gemm_stage(jobs.data(), order.data(), cut, h.pair_products, h.gws_floats, tried[0]);
-            tried[1].n = 0;
-            if (cut < n) t += 1.5 + plan_gemm_stage(jobs.data(), order.data() + cut, n - cut, h.pair_products, h.gws_floats, tried[1]);
-            if (us >= 0. && t >= us) continue;
-            us = t;
-            best[0] = tried[0]; best[1] = tried[1];
-        }
         // (entries of the per-launch timing are a layer call's: nothing would take an operator call's away again)
-        for (const GemmStage& stage : best)
+        for (const GemmStage& stage : group_plan(h, jobs).stage)
             for (int i = 0; i < stage.n; ++i) run_launch(h, jobs.data(), stage.launch[i], nullptr);
     });
 }

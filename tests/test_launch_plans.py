@@ -86,9 +86,10 @@ class Group:
                 q.T, q.l_T = q.C, lt.encode()
             q.alpha = 1.0
 
-    def launched(self):
-        return launches.launched(
-            lambda: self.l.check(self.lib.sub_op_einsum_group(self.handles[0].ptr, self.products, len(self.products))))
+    def launched(self, on=None):
+        """By its own handle or by the one of another group (the sizes stay its own)."""
+        handle = (on or self).handles[0].ptr
+        return launches.launched(lambda: self.l.check(self.lib.sub_op_einsum_group(handle, self.products, len(self.products))))
 
 
 def _timed_operator_calls():
@@ -123,3 +124,28 @@ def test_a_misaligned_member_of_a_group_runs_alone(tmp_path):
     assert whole[0] == 0 and whole[1] >= 1
     for scalar, shared, total in rest:
         assert scalar == 1 and shared >= 1 and total <= whole[2] + 1
+
+
+def _groups_in_turn():
+    def groups():
+        for dims in ((8, 256, 16, 1024, 512), (2, 128, 12, 768, 128), (3, 40, 4, 256, 72), (16, 384, 12, 768, 256), (4, 1000, 16, 1024, 96)):
+            for odd in (None, 4):
+                g = Group(*dims)
+                if odd is not None:
+                    g.products[odd].B += 2
+                yield g
+    want = [g.launched() for g in groups()]
+    one = Group()
+    for on in (1, 0, 1):
+        one.handles[0].set_option(5, on)
+        for turn in range(2):
+            for g, w in zip(groups(), want):
+                got = g.launched(one)
+                alone = all('Li7E' not in name for name, _ in got)
+                print('same' if (got == w if on else alone) else (on, turn, got, w))
+
+
+def test_groups_that_a_handle_has_seen_before(tmp_path):
+    """More groups than a handle keeps plans of, by sizes, alignments and the option, over and over: what a new handle launches."""
+    lines = launches.run(_groups_in_turn, tmp_path)
+    assert len(lines) == 60 and set(lines) == {'same'}, [l for l in lines if l != 'same'][:2]
