@@ -8,9 +8,11 @@
 #include <cmath>
 #include <map>
 #include <algorithm>
+#include <atomic>
 #include <mutex>
 #include <set>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/substation_amd.h"
@@ -256,7 +258,7 @@ struct Handle {
     // is handed the same buffer, and from DROP2 itself otherwise.
     const void* gate_bits_at = nullptr;
     int form = 0;                     // what the last forward call left (FORM_*); see sub_forward_form
-    bool alone_next = false;          // no backward call will follow the next forward call (sub_forward_alone)
+    std::atomic<std::thread::id> alone_next{};   // no backward call will follow this thread's next forward call (sub_forward_alone)
     bool left_nothing = false;        // and none can follow the latest one
     int form_given = -1;              // the same of the forward call that the next backward call belongs to, if it was said
     BackwardPlan plan;                // see backward_plan()
@@ -1239,9 +1241,7 @@ void stage_inputs(Handle& h, const void* X, void* const* W, const void*& Xs, voi
     else ps.cancel();
 }
 
-void forward(Handle& h, const FwdPtrs& t0) {
-    const bool alone = h.alone_next && h.opaque;
-    h.alone_next = false;
+void forward(Handle& h, const FwdPtrs& t0, bool alone) {
     if (!h.configured) fail("encoder_forward: handle is not configured");
     h.left_nothing = alone;
     h.prof_used = 0;
@@ -1712,14 +1712,14 @@ int sub_forget_staged(void* handle) {
 int sub_encoder_forward(void* handle, void* const* ptrs, int n) {
     return guarded([&] {
         Handle& h = as_handle(handle);
-        const bool alone = h.alone_next;
-        h.alone_next = false;         // (a call that is refused is the one it was said of)
+        // (a call that is refused is the one it was said of; one of another thread, which may be in between, is not)
+        std::thread::id me = std::this_thread::get_id();
+        const bool alone = h.alone_next.compare_exchange_strong(me, std::thread::id{}) && h.opaque;
         if (n != 1 + SUB_N_PARAMS + SUB_N_FWD + 1) fail("sub_encoder_forward: expected 37 pointers");
         need_cfg(h);
         for (int i = 0; i < n; ++i) if (!ptrs[i]) fail("sub_encoder_forward: null tensor pointer");
         FwdPtrs t; unpack_forward(h, ptrs, t);
-        h.alone_next = alone;
-        forward(h, t);
+        forward(h, t, alone);
     });
 }
 
@@ -1819,7 +1819,7 @@ int sub_forward_form(void* handle, int* form) {
 }
 
 int sub_forward_alone(void* handle) {
-    return guarded([&] { as_handle(handle).alone_next = true; });
+    return guarded([&] { as_handle(handle).alone_next = std::this_thread::get_id(); });
 }
 
 int sub_set_forward_form(void* handle, int form) {

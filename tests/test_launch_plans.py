@@ -149,3 +149,35 @@ def test_groups_that_a_handle_has_seen_before(tmp_path):
     """More groups than a handle keeps plans of, by sizes, alignments and the option, over and over: what a new handle launches."""
     lines = launches.run(_groups_in_turn, tmp_path)
     assert len(lines) == 60 and set(lines) == {'same'}, [l for l in lines if l != 'same'][:2]
+
+
+def _two_threads():
+    import threading
+    from substation_amd import _lib, layouts as L
+    lib = _lib.load()
+    h = _lib.Handle(_lib.make_config(2, 128, 4, 256, L.mi355x_layouts(), 0.1, 0.1, 0.1, 0.1, activation='gelu'))
+    h.set_option(12, 1)
+    forward, backward = _pointers(launches.tensors(37)), _pointers(launches.tensors(64, first=64))
+    said, done = threading.Event(), threading.Event()
+    refused = []
+
+    def without_gradients():
+        _lib.check(lib.sub_forward_alone(h.ptr))
+        said.set()
+        done.wait()
+        _lib.check(lib.sub_encoder_forward(h.ptr, *forward))
+        refused.append(lib.sub_encoder_backward(h.ptr, *backward) < 0)
+
+    other = threading.Thread(target=without_gradients)
+    other.start()
+    said.wait()
+    _lib.check(lib.sub_encoder_forward(h.ptr, *forward))
+    print(lib.sub_encoder_backward(h.ptr, *backward) == 0)
+    done.set()
+    other.join()
+    print(refused == [True])
+
+
+def test_a_forward_pass_of_another_thread_keeps_what_its_backward_pass_reads(tmp_path):
+    """That no backward call follows is said of the calling thread's next forward call, whatever another one calls in between."""
+    assert launches.run(_two_threads, tmp_path) == ['True', 'True']
