@@ -311,7 +311,11 @@ float* static_scratch() {
     return g_scratch_ptr[dev];
 }
 
-// Forward products of a ReLU layer (see GemmEpilogue::same_order).
+// Forward products that a ReLU stands behind (see GemmEpilogue::same_order): those of a ReLU layer up to lin1.  lin2, behind the layer's
+// own gates, is summed as is fastest; a layer above it in a stack has gates that follow from it, which may fall otherwise where the
+// fastest way is another one (they did at 4 x 256, E 768, where lin2 in five parts became one in one).  Operator calls do not say
+// what stands behind them: all single products of a handle with ReLU are held to that order, a decoder layer's data gradients
+// (sub_op_einsum) among them, as they always were.
 bool before_relu(const Handle& h) { return h.act == ACT_RELU; }
 // Dropout masks as bits (SUB_OPT_PACKED_MASKS), those of the residuals and the activation's: rows must be whole 8-packs.
 bool packed_masks(const Handle& h) { return h.packed_masks && h.sz.n[dI] % 8 == 0; }

@@ -232,11 +232,12 @@ TileChoice choose_single(const TileProduct& p, size_t ws_floats, double reduce_u
 }
 
 // In how many parts a forward pass sums a product, by its shape and the order of its operands alone: as is fastest, within the
-// scratch that every caller brings.  A product that does not widen its rows has a LayerNorm behind it in the layers, which takes the
-// parts in place of their sum (3.9 us without, 5.7 with six parts of 64 x 768, 0.6 of that for their bytes).  (Splits to fill the CUs as far as 8 steps each were left of it, which was the rule here before,
-// cost more than they gave where the fp32 sums are many: us of lin2 and the LayerNorm behind it, 2613 x 768 x 3072 in two parts
-// 32 and in one 29, 1024 x 768 x 3072 in five 21.4 and in one 19.9; and a product of 512 x 4096 x 1024 in two parts had no activation
-// in its epilogue, 28 with its activation and now 14.)
+// scratch that every caller brings.  A product that does not widen its rows has a LayerNorm behind it in the layers, which takes
+// the parts in place of their sum (3.9 us without, 5.7 with six parts of 64 x 768, 0.6 of that for their bytes).  (Splits to fill
+// the CUs as far as 8 steps each were left of it, which was the rule here before, cost more than they gave where the fp32 sums are
+// many: us of lin2 and the LayerNorm behind it, 2613 x 768 x 3072 in two parts 32 and in one 29, 1024 x 768 x 3072 in five 21.4
+// and in one 19.9; and a product of 512 x 4096 x 1024 in two parts had no activation in its epilogue, 28 with its activation and
+// now 14.)
 // In front of a ReLU the rule is that of old, which fills the CUs as long as eight steps a part are left of it.
 int forward_splits(const TileProduct& p) {
     if (p.a.same_order) {

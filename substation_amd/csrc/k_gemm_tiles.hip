@@ -9,8 +9,8 @@ namespace {
 
 // The tiles there are, and what they take (us): a step of 64 k with few workgroups, with one on every second CU (two
 // share a CU: on every CU), and in every place; a launch with the way into and out of its first tile; a tile's way out
-// where all CUs are on theirs.  From products of 64 .. 12288 rows with 1 .. 256 steps, alone and up to five in a launch, on operands of
-// normal distribution that are used in turn.  256 x 256 is k_gemm_wide.
+// where all CUs are on theirs.  From products of 64 .. 12288 rows with 1 .. 256 steps, alone and two to five in a launch (which takes up to
+// kMaxProducts), on operands of normal distribution that are used in turn.  256 x 256 is k_gemm_wide.
 struct Form { int bm, bn, per_cu; double few, half, full, once, out; };
 constexpr Form kForms[TILE_FORMS] = {
     {64, 64, 2, 0.20, 0.20, 0.38, 3.6, 1.6},
@@ -19,13 +19,16 @@ constexpr Form kForms[TILE_FORMS] = {
     {256, 128, 1, 0.56, 0.62, 0.92, 5.9, 2.0},
     {256, 256, 1, 1.02, 1.25, 1.47, 5.5, 4.3},
 };
-// The last two as they were when the order of the sums in front of a ReLU was fixed (GemmEpilogue::same_order): which products go into
-// 256 x 256 tiles is decided by these there.
-constexpr Form kOrderForms[2] = {
+// As they were when the order of the sums in front of a ReLU was fixed (GemmEpilogue::same_order): whether such a product goes into
+// 256 x 256 tiles is decided by these and by nothing that is fitted anew, so they are never changed.
+constexpr Form kOrderForms[TILE_FORMS] = {
+    {64, 64, 2, 0.20, 0.20, 0.38, 3.6, 1.6},
+    {128, 64, 2, 0.29, 0.33, 0.59, 3.8, 2.0},
+    {128, 128, 1, 0.33, 0.37, 0.47, 4.4, 2.0},
     {256, 128, 1, 0.52, 0.54, 0.83, 5.9, 2.0},
     {256, 256, 1, 1.00, 1.00, 1.42, 5.5, 4.3},
 };
-inline const Form& form_of(int f, bool order) { return order && f >= TILE_256x128 ? kOrderForms[f - TILE_256x128] : kForms[f]; }
+inline const Form& form_of(int f, bool order) { return order ? kOrderForms[f] : kForms[f]; }
 // Several products of more than a round of the smaller tiles: the workgroups drift apart, and share fewer lines of their L2
 // (4096 x 1024 x 4096 twice in tiles of 128 x 128: 75.5 us, 3 times 117 and once 38.5).
 constexpr double kDrift = 1.12;

@@ -2,6 +2,7 @@
 import copy
 import ctypes
 import itertools
+import re
 
 import pytest
 
@@ -181,3 +182,48 @@ def _two_threads():
 def test_a_forward_pass_of_another_thread_keeps_what_its_backward_pass_reads(tmp_path):
     """That no backward call follows is said of the calling thread's next forward call, whatever another one calls in between."""
     assert launches.run(_two_threads, tmp_path) == ['True', 'True']
+
+
+# (B, L, H, E): how the four forward products of a ReLU layer are summed (projections, out, lin1, lin2): in 256 x 256 tiles, whose k slices
+# are twice as long (W), or in others (R), and in how many parts; and lin1 with its activation, which products in parts do not have
+ORDERS = {
+    (1, 16, 8, 512): 'R1 R1 R1 R4 R', (1, 64, 12, 768): 'R1 R1 R1 R6 R', (1, 64, 16, 1024): 'R2 R2 R2 R8 -',
+    (2, 128, 12, 768): 'R1 R1 R1 R6 R', (4, 256, 12, 768): 'R1 R1 R1 R5 R', (24, 77, 12, 768): 'R1 R1 R1 R2 R',
+    (13, 201, 12, 768): 'R1 R1 R1 R2 R', (8, 500, 16, 1024): 'W1 R1 W1 R1 W', (8, 512, 16, 1024): 'W1 R1 W1 R1 W',
+    (10, 512, 16, 1024): 'W1 R1 R1 R1 R', (12, 512, 16, 1024): 'R1 R1 R1 R1 R', (16, 512, 16, 1024): 'R1 R1 W1 R1 W',
+    (96, 128, 16, 1024): 'R1 W1 W1 W1 W', (1, 512, 16, 1024): 'R2 R2 R2 R8 -', (2, 512, 16, 1024): 'R1 R2 R1 R4 R',
+    (1, 128, 32, 4096): 'R2 R8 R2 R8 -', (1, 512, 32, 4096): 'R1 R2 R1 R2 R', (2, 1024, 16, 2048): 'W1 R1 W1 R1 W',
+    (4, 2048, 32, 4096): 'W1 W1 W1 W1 W', (7, 640, 16, 2048): 'W1 W1 R1 W1 R', (9, 333, 12, 768): 'R1 R1 W1 R1 W',
+    (5, 1000, 16, 1024): 'W1 R1 R1 R1 R', (40, 200, 8, 512): 'W1 R1 W1 R1 W',
+}
+
+
+def _orders_in_front_of_a_relu():
+    from substation_amd import _lib, layouts as L
+    lib = _lib.load()
+    for B, S, H, E in ORDERS:
+        h = _lib.Handle(_lib.make_config(B, S, H, E, L.mi355x_layouts(), 0.1, 0.1, 0.1, 0.1, activation='relu'))
+        h.set_option(12, 1)
+        row = []
+        for la, lb, lc in (('BJI', 'QHPI', 'QBJHP'), ('IHP', 'BJHP', 'BJI'), ('BJI', 'UI', 'BJU'), ('BJU', 'IU', 'BJI')):
+            a, b, c = launches.tensors(3)
+            (name, grid), *reduction = launches.launched(lambda: _lib.check(
+                lib.sub_op_einsum(h.ptr, a, la.encode(), b, lb.encode(), c, lc.encode(), 1.0)))
+            wide = 'k_gemm_wide' in name
+            parts = 1
+            if reduction:                                   # (a workgroup for each part of a tile)
+                tm, tn, wm, wn = (int(x) for x in re.findall(r'Li(\d+)E', name)[:4])
+                shape = h.classify(la, lb, lc)
+                tiles = -(-shape['M'] // (32 * tm * wm)) * -(-shape['N'] // (32 * tn * wn)) * shape['batch']
+                assert grid[0] % tiles == 0
+                parts = grid[0] // tiles
+            row.append('RW'[wide] + str(parts))
+        forward = launches.launched(lambda: _lib.check(lib.sub_encoder_forward(h.ptr, *_pointers(launches.tensors(37)))))
+        act = ['RW'['k_gemm_wide' in n] for n, _ in forward if re.search(r'k_gemm_(ring|wide).*Li[13]EEEv', n)]
+        print(' '.join(row + (act or ['-'])))
+
+
+def test_order_of_the_sums_in_front_of_a_relu(tmp_path):
+    """It is a fixed function of the shape: another one moves gates, and with them whole rows of gradients."""
+    lines = launches.run(_orders_in_front_of_a_relu, tmp_path)
+    assert dict(zip(ORDERS, lines)) == ORDERS
