@@ -276,6 +276,9 @@ static void launch_tiles_n(const TileProduct* p, int n, int form, FinishJobs* ta
 
 void launch_tiles(const TileProduct* p, int n, int form, FinishJobs* tail, hipStream_t st) {
     if (form == TILE_256x256) { launch_wide(p, n, tail, 0, st); return; }
+    // One instance for two to seven products.  With another for up to three, and 2.0 KB of arguments in place of 3.7, a data and a weight
+    // gradient (64 rows of E 512; 256, 1024 and 2613 of 768; 4096 of 1024; 8192 of 4096) take 9.28 us for 9.32, 15.1 for 15.2, 25.9 for 25.9,
+    // 35.5 for 35.7, 65.6 for 64.9, 1586 for 1597: nothing either way.
     if (n == 1 && !(tail && tail->n)) launch_tiles_n<1>(p, n, form, tail, st);
     else launch_tiles_n<kMaxProducts>(p, n, form, tail, st);
 }

@@ -293,7 +293,7 @@ struct GemmJob {
     float alpha = 1.f;
     GemmEpilogue ep;             // (an addend at most)
 };
-constexpr int kMaxProducts = 7;  // of one launch (their arguments stay below 4 KiB)
+constexpr int kMaxProducts = 7;  // of one launch (their arguments stay below 4 KiB: see TileGroup)
 // Jobs of one launch: their tiles of form `form`, the contraction of member `split` in `splits` parts.  form < 0: one job, launched
 // by launch_gemm.
 struct GemmLaunch {

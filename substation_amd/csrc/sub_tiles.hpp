@@ -154,8 +154,10 @@ struct TileGroup {
     unsigned n = 0, workers = 0;      // products; workgroups that take tiles
     Schedule when;                    // (of several products)
     unsigned tail_groups = 0;
-    typename std::conditional<NP == 1, NoJobs, FinishJobs>::type tail;     // column sums of earlier launches, finished by the workgroups behind those
+    // column sums of earlier launches, finished by the workgroups behind those
+    typename std::conditional<NP == 1, NoJobs, FinishJobs>::type tail;
 };
+static_assert(sizeof(TileGroup<kMaxProducts>) <= 4096, "a kernel's arguments");
 
 // (the launch's arguments where they lie: an index into them that is not a constant would otherwise have them copied
 // into scratch memory)
