@@ -206,7 +206,7 @@ def _make_function(m):
                 o.einsum(dff, 'BJI', w['linear2_w'], 'IU', dff1, 'BJU')
                 o.bdrlb(dff1, 'BJU', s['mask3'], 'BJU', s['lin1'], 'BJU', dlin1, 'BJU', g['linear1_b'])
             # (weight gradients feed nothing: all of them run at the end, where their tiles fill each other's rounds.  Kernels of
-            # 8 x 256 on 512, E 1024: 569 us, 685 with each next to its data gradient; 8 x 512 on 512: a pass 1004 -> 873)
+            # 8 x 256 on 512, E 1024: 526 us, 639 with each next to its data gradient; 8 x 512 on 512: a pass 1004 -> 873)
             dnormed2_linear = e('BJI')
             o.einsum(dlin1, 'BJU', w['linear1_w'], 'UI', dnormed2_linear, 'BJI')
             # norm2, residual, encoder-decoder attention              transformer.py:396-413

@@ -1,4 +1,4 @@
-"""Launches of several products: tiles of up to five of them in one schedule, against the products launched one by one."""
+"""Launches of several products: tiles of up to seven of them in one schedule, against the products launched one by one."""
 import pytest
 import torch
 
