@@ -440,7 +440,11 @@ void launch_gemm(const GemmShape& s, const half_t* A, const half_t* B, half_t* C
             return;
         }
         const bool small = ws && (size_t)batch * c.a.M * c.a.N <= kSplitMaxOut;
-        if (small && !ep.any_split) tp.a.splits = forward_splits(tp);
+        if (small && !ep.any_split) {
+            tp.a.splits = forward_splits(tp);
+            if (tp.a.splits > 1 && (size_t)batch * c.a.M * c.a.N * tp.a.splits > ws_floats)
+                fail("gemm: scratch for the sums of a split product is smaller than gemm_splitk_ws_floats");
+        }
         const unsigned forms = !tp.a.same_order ? forms_for(&tp, 1) : summed_wide(tp) ? 1u << TILE_256x256 : kRingForms;
         const TileChoice choice = choose_tiles(&tp, 1, forms, small && ep.any_split ? ws_floats : 0);
         unsigned side_blocks = 0;
