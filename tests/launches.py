@@ -14,7 +14,7 @@ def run(body, tmp_path):
     so = os.path.join(str(tmp_path), 'launch_recorder.so')
     subprocess.run(['gcc', '-O1', '-shared', '-fPIC', os.path.join(ROOT, 'tests', 'launch_recorder.c'), '-o', so], check=True)
     code = f'import tests.launches as l\nl.begin({so!r})\nimport importlib\nimportlib.import_module({body.__module__!r}).{body.__name__}()'
-    env = dict(os.environ, PYTHONPATH=ROOT)
+    env = dict(os.environ, PYTHONPATH=os.pathsep.join([ROOT] + os.environ.get('PYTHONPATH', '').split(os.pathsep)).rstrip(os.pathsep))
     r = subprocess.run([sys.executable, '-c', code], cwd=ROOT, env=env, stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True,
                        timeout=120)
     assert r.returncode == 0, r.stderr
