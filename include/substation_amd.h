@@ -291,7 +291,8 @@ int sub_set_forward_form(void* handle, int form);
 /* No encoder_backward call will follow the calling thread's next encoder_forward call on this handle (another thread's call in
  * between is not meant): under SUB_OPT_OPAQUE_INTERMEDIATES it then leaves out what only that would read (LIN1 and the bits in
  * SB1_LINW1 of a layer whose activation runs in the epilogue of lin1; DROP1MASK, LN1DIFF, LN1, LN1STD, DROP3MASK, LN2DIFF,
- * LN2 and LN2STD where their rows are the tokens in order).  The output is the same.  A backward call that would take its intermediates to be that call's is refused. */
+ * LN2 and LN2STD where their rows are the tokens in order).  The output is the same.  A backward call that would take its
+ * intermediates to be that call's is refused. */
 int sub_forward_alone(void* handle);
 /* SUB_OPT_OPAQUE_INTERMEDIATES (default 0; the Python module sets it): the caller hands the intermediates from
  * encoder_forward to encoder_backward and looks into none of them.  Option 9 then also covers DROP2MASK where the

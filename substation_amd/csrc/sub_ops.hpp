@@ -256,8 +256,8 @@ struct GemmEpilogue {
     // the contraction of a small output may be split in as many parts as is fastest within the scratch at hand
     bool any_split = false;
     // in front of a ReLU: the order of the sums is a fixed function of the shape, whatever is fastest (one unit of the last place
-    // of a pre-activation decides a gate, and a gate moves whole rows of gradients).  It is the one that layers of this library have
-    // always had: another fixed order would be no better and would move the gates of every model once more.
+    // of a pre-activation decides a gate, and a gate moves whole rows of gradients).  It is the one that the layers
+    // had when the rule was made: another fixed order would be no better and would move their gates once more.
     bool same_order = false;
     // where given, and the product is split, has dense rows and no addend: it is left as the sums of its splits
     SplitSums* sums = nullptr;
