@@ -6,6 +6,7 @@
 // that the engine runs without taking the interpreter's lock.
 #include <algorithm>
 #include <dlfcn.h>
+#include <mutex>
 
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
@@ -41,6 +42,19 @@ struct Lib {
     decltype(&sub_forward_alone) forward_alone = nullptr;
     decltype(&sub_encoder_forward) encoder_forward = nullptr;
     decltype(&sub_encoder_backward) encoder_backward = nullptr;
+    decltype(&sub_set_rng) set_rng = nullptr;
+    decltype(&sub_ops_defer) ops_defer = nullptr;
+    decltype(&sub_op_einsum) einsum = nullptr;
+    decltype(&sub_op_einsum_add) einsum_add = nullptr;
+    decltype(&sub_op_einsum_bad) einsum_bad = nullptr;
+    decltype(&sub_op_einsum_bdrlb) einsum_bdrlb = nullptr;
+    decltype(&sub_op_einsum_group) einsum_group = nullptr;
+    decltype(&sub_op_attention_forward) attention_forward = nullptr;
+    decltype(&sub_op_attention_backward_biases) attention_backward = nullptr;
+    decltype(&sub_op_bdrln) bdrln = nullptr;
+    decltype(&sub_op_bad) bad = nullptr;
+    decltype(&sub_op_bdrlb) bdrlb = nullptr;
+    decltype(&sub_op_ln_backward) ln_backward = nullptr;
 } lib;
 PyObject* g_error = nullptr;          // substation_amd._lib.SubstationError
 
@@ -63,6 +77,19 @@ void load(const std::string& path, py::object error) {
     get(lib.forward_alone, "sub_forward_alone");
     get(lib.encoder_forward, "sub_encoder_forward");
     get(lib.encoder_backward, "sub_encoder_backward");
+    get(lib.set_rng, "sub_set_rng");
+    get(lib.ops_defer, "sub_ops_defer");
+    get(lib.einsum, "sub_op_einsum");
+    get(lib.einsum_add, "sub_op_einsum_add");
+    get(lib.einsum_bad, "sub_op_einsum_bad");
+    get(lib.einsum_bdrlb, "sub_op_einsum_bdrlb");
+    get(lib.einsum_group, "sub_op_einsum_group");
+    get(lib.attention_forward, "sub_op_attention_forward");
+    get(lib.attention_backward, "sub_op_attention_backward_biases");
+    get(lib.bdrln, "sub_op_bdrln");
+    get(lib.bad, "sub_op_bad");
+    get(lib.bdrlb, "sub_op_bdrlb");
+    get(lib.ln_backward, "sub_op_ln_backward");
     g_error = error.release().ptr();
 }
 
@@ -371,6 +398,252 @@ std::optional<at::Tensor> EncoderLayer::forward(const at::Tensor& X_, const std:
     return Y;
 }
 
+// The operators of a decoder layer's two passes (substation_amd/decoder.py), in the order of the reference's statements
+// (substation/transformer.py:288-441).  Issued from Python (some 55 ctypes calls and 60 torch.empty) they kept the host for 717 us at
+// B=8, lengths 256 and 512, E 1024, where their kernels take 530; from here a pass takes 540, which is those kernels.
+struct DecoderPasses {
+    enum Parameter { SATTN_WKQV, SATTN_IN_B, SATTN_WO, SATTN_OUT_B, EDATTN_WQ, EDATTN_WK, EDATTN_WV, EDATTN_IN_B, EDATTN_WO, EDATTN_OUT_B,
+                     NORM1_SCALE, NORM1_BIAS, NORM2_SCALE, NORM2_BIAS, NORM3_SCALE, NORM3_BIAS, LINEAR1_W, LINEAR1_B, LINEAR2_W, LINEAR2_B,
+                     PARAMETERS };
+    // what a forward pass leaves for its backward pass
+    enum Kept { KQV, STATS1, KEEP1, GAMMA1, MASK1, DIFF1, LN1, NORMED1, ISTD1, Q2, K2, V2, STATS2, KEEP2, GAMMA2, MASK2, DIFF2, LN2, NORMED2,
+                ISTD2, LIN1, MASK3, FF1, BITS, MASK4, DIFF3, LN3, ISTD3, KEPT };
+    typedef std::optional<at::Tensor> Maybe;
+
+    void* target;                     // the handles of the two sizes
+    void* source;
+    py::object keep_alive;
+    int64_t B, Lt, Ls, H, P, E, U;
+    double p_sattn, p_edattn, p_linear1, p_ff;
+    uint32_t site_sattn, site_edattn, site_linear1, site_ff;
+    bool relu;
+    float scale;
+    std::mutex busy;                  // a pass is a sequence of calls on the same two handles
+
+    DecoderPasses(uintptr_t target_, uintptr_t source_, py::object owner, const std::vector<int64_t>& sizes,
+                  const std::vector<double>& probs, const std::vector<uint32_t>& sites, bool relu_, double scale_)
+        : target(reinterpret_cast<void*>(target_)), source(reinterpret_cast<void*>(source_)), keep_alive(std::move(owner)),
+          B(sizes.at(0)), Lt(sizes.at(1)), Ls(sizes.at(2)), H(sizes.at(3)), P(sizes.at(4)), E(sizes.at(5)), U(sizes.at(6)),
+          p_sattn(probs.at(0)), p_edattn(probs.at(1)), p_linear1(probs.at(2)), p_ff(probs.at(3)),
+          site_sattn(sites.at(0)), site_edattn(sites.at(1)), site_linear1(sites.at(2)), site_ff(sites.at(3)),
+          relu(relu_), scale((float)scale_) {}
+    ~DecoderPasses() {
+        if (!Py_IsInitialized()) { keep_alive.release(); return; }
+        py::gil_scoped_acquire gil;
+        keep_alive = py::object();
+    }
+
+    static void* at_(const at::Tensor& t) {
+        if (!(t.is_cuda() && t.scalar_type() == at::kHalf && t.is_contiguous()))
+            raise("operators take contiguous fp16 CUDA tensors", PyExc_ValueError);
+        return t.data_ptr();
+    }
+    static void* at_(const Maybe& t) { return t ? at_(*t) : nullptr; }
+    static char* part(const at::Tensor& t, int64_t i, int64_t of) { return static_cast<char*>(at_(t)) + 2 * (t.numel() / of) * i; }
+
+    // A pass: the current device's stream, tensors on that device.
+    struct Place {
+        at::TensorOptions half;
+        explicit Place(DecoderPasses& d) {
+            const c10::DeviceIndex device = c10::hip::current_device();
+            half = at::TensorOptions().dtype(at::kHalf).device(c10::Device(c10::kCUDA, device));
+            use_current_stream(d.target, device);
+            if (d.source != d.target) use_current_stream(d.source, device);
+        }
+        at::Tensor operator()(at::IntArrayRef shape) const { return at::empty(shape, half); }
+        at::Tensor operator()(at::IntArrayRef shape, at::ScalarType type) const { return at::empty(shape, half.dtype(type)); }
+    };
+
+    std::vector<Maybe> forward(const at::Tensor& x, const at::Tensor& enc, const std::vector<at::Tensor>& w, const Maybe& mask, uint64_t seed,
+                               uint32_t step, bool epilogues) {
+        py::gil_scoped_release nogil;
+        const std::lock_guard<std::mutex> one(busy);
+        const Place e(*this);
+        check(lib.set_rng(target, seed, step), "sub_set_rng");
+        check(lib.set_rng(source, seed, step), "sub_set_rng");
+        std::vector<Maybe> k(KEPT + 1);                      // and the output
+        std::vector<void*> wp;
+        wp.reserve(PARAMETERS);
+        if (w.size() != PARAMETERS) raise("DecoderLayer: 20 parameters", PyExc_ValueError);
+        for (const auto& t : w) wp.push_back(at_(t));
+        const auto make = [&](Kept i, at::IntArrayRef shape) { k[i] = e(shape); return k[i]->data_ptr(); };
+        const std::initializer_list<int64_t> bji = {B, Lt, E}, bj = {B, Lt}, bjhp = {B, Lt, H, P}, bkhp = {B, Ls, H, P}, bju = {B, Lt, U};
+        // masked self-attention, residual, norm1
+        make(KQV, {3, B, Lt, H, P});
+        check(lib.einsum_add(target, at_(x), "BJI", wp[SATTN_WKQV], "QHPI", wp[SATTN_IN_B], "QHP", at_(k[KQV]), "QBJHP", 1.f), "einsum_add");
+        const auto workspace = [&](Kept stats, Kept keep, int64_t keys) {
+            k[stats] = e({2 * H * B * Lt}, at::kFloat);
+            k[keep] = e({H * B * Lt * (keys / 32)}, at::kInt);
+        };
+        workspace(STATS1, KEEP1, Lt);
+        make(GAMMA1, bjhp);
+        check(lib.attention_forward(target, (int)Lt, (int)Lt, part(*k[KQV], 1, 3), "BJHP", part(*k[KQV], 0, 3), part(*k[KQV], 2, 3), "BKHP",
+                                    at_(k[GAMMA1]), "BJHP", k[STATS1]->data_ptr(), k[KEEP1]->data_ptr(), at_(mask), "JK", scale, 0.f, 0),
+              "attention_forward");
+        const at::Tensor att1 = e(bji);
+        check(lib.einsum(target, wp[SATTN_WO], "IHP", at_(k[GAMMA1]), "BJHP", at_(att1), "BJI", 1.f), "einsum");
+        const auto norm = [&](const at::Tensor& in, const at::Tensor& residual, Parameter b, Parameter s, Kept m, Kept diff, Kept ln, int normed,
+                              Kept istd, double p, uint32_t site) {
+            make(m, bji); make(diff, bji); make(ln, bji); make(istd, bj);
+            k[normed] = e(bji);
+            check(lib.bdrln(target, at_(in), "BJI", at_(residual), "BJI", wp[b], wp[s], wp[s + 1], at_(in), "BJI", at_(k[m]), "BJI",
+                            at_(k[diff]), "BJI", at_(k[ln]), "BJI", at_(k[normed]), "BJI", at_(k[istd]), "BJ", (float)p, site), "bdrln");
+        };
+        norm(att1, x, SATTN_OUT_B, NORM1_SCALE, MASK1, DIFF1, LN1, NORMED1, ISTD1, p_sattn, site_sattn);
+        // encoder-decoder attention, residual, norm2
+        make(Q2, bjhp); make(K2, bkhp); make(V2, bkhp);
+        const at::Tensor& in_b = w[EDATTN_IN_B];
+        check(lib.einsum_add(target, at_(k[NORMED1]), "BJI", wp[EDATTN_WQ], "HPI", part(in_b, 0, 3), "HP", at_(k[Q2]), "BJHP", 1.f), "einsum_add");
+        check(lib.einsum_add(source, at_(enc), "BKI", wp[EDATTN_WK], "HPI", part(in_b, 1, 3), "HP", at_(k[K2]), "BKHP", 1.f), "einsum_add");
+        check(lib.einsum_add(source, at_(enc), "BKI", wp[EDATTN_WV], "HPI", part(in_b, 2, 3), "HP", at_(k[V2]), "BKHP", 1.f), "einsum_add");
+        workspace(STATS2, KEEP2, Ls);
+        make(GAMMA2, bjhp);
+        check(lib.attention_forward(target, (int)Lt, (int)Ls, at_(k[Q2]), "BJHP", at_(k[K2]), at_(k[V2]), "BKHP", at_(k[GAMMA2]), "BJHP",
+                                    k[STATS2]->data_ptr(), k[KEEP2]->data_ptr(), nullptr, "JK", scale, 0.f, 0), "attention_forward");
+        const at::Tensor att2 = e(bji);
+        check(lib.einsum(target, wp[EDATTN_WO], "IHP", at_(k[GAMMA2]), "BJHP", at_(att2), "BJI", 1.f), "einsum");
+        norm(att2, *k[NORMED1], EDATTN_OUT_B, NORM2_SCALE, MASK2, DIFF2, LN2, NORMED2, ISTD2, p_edattn, site_edattn);
+        // feed-forward, residual, norm3: linear1 with bias, activation and dropout in its epilogue where the product qualifies (the keep
+        // bits then travel as bits, no mask tensor; ReLU needs no pre-activation either); else operator by operator
+        make(FF1, bju);
+        if (!relu) make(LIN1, bju);
+        int applied = 0;
+        if (epilogues) {
+            k[BITS] = e({B * Lt * U / 8}, at::kByte);
+            check(lib.einsum_bad(target, at_(k[NORMED2]), "BJI", wp[LINEAR1_W], "UI", wp[LINEAR1_B], "U", at_(k[LIN1]), at_(k[FF1]), "BJU",
+                                 k[BITS]->data_ptr(), (float)p_linear1, site_linear1, &applied), "einsum_bad");
+        }
+        if (!applied) {
+            k[BITS].reset();
+            make(LIN1, bju); make(MASK3, bju);
+            check(lib.einsum(target, at_(k[NORMED2]), "BJI", wp[LINEAR1_W], "UI", at_(k[LIN1]), "BJU", 1.f), "einsum");
+            check(lib.bad(target, at_(k[LIN1]), "BJU", wp[LINEAR1_B], at_(k[LIN1]), "BJU", at_(k[MASK3]), "BJU", at_(k[FF1]), "BJU",
+                          (float)p_linear1, site_linear1), "bad");
+        }
+        const at::Tensor ff = e(bji);
+        check(lib.einsum(target, at_(k[FF1]), "BJU", wp[LINEAR2_W], "IU", at_(ff), "BJI", 1.f), "einsum");
+        norm(ff, *k[NORMED2], LINEAR2_B, NORM3_SCALE, MASK4, DIFF3, LN3, KEPT, ISTD3, p_ff, site_ff);
+        return k;
+    }
+
+    // The second stage of every column sum of a pass in one launch at its end (whatever becomes of the pass).
+    struct Deferred {
+        std::vector<void*> handles;
+        explicit Deferred(const DecoderPasses& d) {
+            for (void* h : {d.target, d.source}) {
+                if (std::find(handles.begin(), handles.end(), h) != handles.end()) continue;
+                check(lib.ops_defer(h, 1), "sub_ops_defer");
+                handles.push_back(h);
+            }
+        }
+        void finish() {
+            while (!handles.empty()) {
+                void* h = handles.back();
+                handles.pop_back();
+                check(lib.ops_defer(h, 0), "sub_ops_defer");
+            }
+        }
+        ~Deferred() {
+            for (; !handles.empty(); handles.pop_back()) lib.ops_defer(handles.back(), 0);
+        }
+    };
+
+    // The gradients of x, of the encoder's output and of the parameters.
+    std::vector<at::Tensor> backward(const at::Tensor& x, const at::Tensor& enc, std::vector<at::Tensor> w, const std::vector<Maybe>& k,
+                                     const at::Tensor& dy, const Maybe& mask) {
+        py::gil_scoped_release nogil;
+        const std::lock_guard<std::mutex> one(busy);
+        if (w.size() != PARAMETERS || k.size() < KEPT) raise("DecoderLayer: not what a forward pass has saved", PyExc_ValueError);
+        // (the products with an epilogue need whole 16-byte words, wherever a parameter lies or was restored to)
+        for (const Parameter i : {LINEAR2_W, EDATTN_WV, SATTN_WKQV})
+            if (misaligned(w[i])) w[i] = w[i].clone();
+        const Place e(*this);
+        Deferred deferred(*this);
+        std::vector<at::Tensor> out(2);                      // dx and d(encoder output), then the parameters'
+        std::vector<void*> wp, g;
+        wp.reserve(PARAMETERS); g.reserve(PARAMETERS);
+        for (const auto& t : w) {
+            wp.push_back(at_(t));
+            out.push_back(at::empty_like(t));
+            g.push_back(at_(out.back()));
+        }
+        const std::initializer_list<int64_t> bji = {B, Lt, E}, bjhp = {B, Lt, H, P}, bkhp = {B, Ls, H, P}, bju = {B, Lt, U};
+        // a LayerNorm's backward pass, its dropout's and (second: with a second gradient) the sums next to it
+        struct Norm { at::Tensor dln, dres, ddrop; };
+        const auto norm = [&](Kept ln, Parameter s, const at::Tensor& dout, Kept istd, Kept diff, Kept m, const at::Tensor* dout2,
+                              const at::Tensor* dlinear, void* dlinear_bias, void* dout_bias) {
+            Norm n{e(bji), e(bji), e(bji)};
+            check(lib.ln_backward(target, dout2 ? 1 : 0, at_(k[ln]), "BJI", wp[s], at_(dout), "BJI", dout2 ? at_(*dout2) : nullptr, "BJI",
+                                  dlinear ? at_(*dlinear) : nullptr, "BJI", at_(k[istd]), "BJ", at_(k[diff]), "BJI", at_(k[m]), "BJI",
+                                  at_(n.dln), "BJI", at_(n.dres), "BJI", at_(n.ddrop), "BJI", g[s], g[s + 1], dlinear_bias, dout_bias),
+                  "ln_backward");
+            return n;
+        };
+        // norm3, residual, feed-forward
+        const Norm n3 = norm(LN3, NORM3_SCALE, dy, ISTD3, DIFF3, MASK4, nullptr, nullptr, nullptr, nullptr);
+        const at::Tensor& dff = n3.ddrop;
+        const at::Tensor dlin1 = e(bju);
+        int applied = 0;
+        if (k[BITS])
+            check(lib.einsum_bdrlb(target, at_(dff), "BJI", wp[LINEAR2_W], "IU", at_(k[relu ? FF1 : LIN1]), "BJU", k[BITS]->data_ptr(), at_(dlin1),
+                                   "BJU", g[LINEAR1_B], &applied), "einsum_bdrlb");
+        if (!applied) {
+            if (!k[MASK3])
+                raise("DecoderLayer: the forward pass ran linear1 with its activation epilogue, the backward pass cannot", PyExc_RuntimeError);
+            const at::Tensor dff1 = e(bju);
+            check(lib.einsum(target, at_(dff), "BJI", wp[LINEAR2_W], "IU", at_(dff1), "BJU", 1.f), "einsum");
+            check(lib.bdrlb(target, at_(dff1), "BJU", at_(k[MASK3]), "BJU", at_(k[LIN1]), "BJU", at_(dlin1), "BJU", g[LINEAR1_B]), "bdrlb");
+        }
+        // (weight gradients feed nothing: all of them run at the end, where their tiles fill each other's rounds.  Kernels of
+        // 8 x 256 on 512, E 1024: 526 us, 639 with each next to its data gradient; 8 x 512 on 512: a pass 1004 -> 873)
+        const at::Tensor dnormed2 = e(bji);
+        check(lib.einsum(target, at_(dlin1), "BJU", wp[LINEAR1_W], "UI", at_(dnormed2), "BJI", 1.f), "einsum");
+        // norm2, residual, encoder-decoder attention
+        const Norm n2 = norm(LN2, NORM2_SCALE, n3.dres, ISTD2, DIFF2, MASK2, &dnormed2, &dff, g[LINEAR2_B], g[EDATTN_OUT_B]);
+        const at::Tensor& datt2 = n2.ddrop;
+        const at::Tensor dgamma2 = e(bjhp);
+        check(lib.einsum(target, wp[EDATTN_WO], "IHP", at_(datt2), "BJI", at_(dgamma2), "BJHP", 1.f), "einsum");
+        const at::Tensor dq2 = e(bjhp), dk2 = e(bkhp), dv2 = e(bkhp);
+        const at::Tensor& d_in_b = out[2 + EDATTN_IN_B];
+        check(lib.attention_backward(target, (int)Lt, (int)Ls, at_(k[Q2]), "BJHP", at_(k[K2]), at_(k[V2]), "BKHP", at_(k[GAMMA2]), "BJHP",
+                                     at_(dgamma2), "BJHP", k[STATS2]->data_ptr(), k[KEEP2]->data_ptr(), at_(dq2), "BJHP", at_(dk2), at_(dv2), "BKHP",
+                                     nullptr, "JK", scale, part(d_in_b, 0, 3), part(d_in_b, 1, 3), part(d_in_b, 2, 3)), "attention_backward");
+        const at::Tensor dnormed1 = e(bji);
+        out[1] = e({B, Ls, E});
+        void* const denc = at_(out[1]);
+        const auto group = [&](std::initializer_list<SubEinsum> products) {
+            check(lib.einsum_group(target, products.begin(), (int)products.size()), "einsum_group");
+        };
+        group({{nullptr, at_(dq2), "BJHP", wp[EDATTN_WQ], "HPI", nullptr, nullptr, at_(dnormed1), "BJI", 1.f},
+               {source, at_(dk2), "BKHP", wp[EDATTN_WK], "HPI", nullptr, nullptr, denc, "BKI", 1.f}});
+        // norm1, residual, self-attention
+        const at::Tensor unused = at::empty_like(out[2 + SATTN_OUT_B]);      // the column sums of the third input are not needed here
+        const Norm n1 = norm(LN1, NORM1_SCALE, n2.dres, ISTD1, DIFF1, MASK1, &dnormed1, &datt2, at_(unused), g[SATTN_OUT_B]);
+        const at::Tensor& datt1 = n1.ddrop;
+        const at::Tensor dgamma1 = e(bjhp);
+        check(lib.einsum(target, wp[SATTN_WO], "IHP", at_(datt1), "BJI", at_(dgamma1), "BJHP", 1.f), "einsum");
+        const at::Tensor dkqv = e({3, B, Lt, H, P});
+        const at::Tensor &kqv = *k[KQV], &ds_in_b = out[2 + SATTN_IN_B];
+        check(lib.attention_backward(target, (int)Lt, (int)Lt, part(kqv, 1, 3), "BJHP", part(kqv, 0, 3), part(kqv, 2, 3), "BKHP", at_(k[GAMMA1]),
+                                     "BJHP", at_(dgamma1), "BJHP", k[STATS1]->data_ptr(), k[KEEP1]->data_ptr(), part(dkqv, 1, 3), "BJHP",
+                                     part(dkqv, 0, 3), part(dkqv, 2, 3), "BKHP", at_(mask), "JK", scale, part(ds_in_b, 1, 3), part(ds_in_b, 0, 3),
+                                     part(ds_in_b, 2, 3)), "attention_backward");
+        out[0] = e(bji);
+        group({{nullptr, wp[SATTN_WKQV], "QHPI", at_(dkqv), "QBJHP", at_(n1.dres), "BJI", at_(out[0]), "BJI", 1.f},
+               {source, at_(dv2), "BKHP", wp[EDATTN_WV], "HPI", denc, "BKI", denc, "BKI", 1.f},
+               {source, at_(dv2), "BKHP", at_(enc), "BKI", nullptr, nullptr, g[EDATTN_WV], "HPI", 1.f},
+               {source, at_(dk2), "BKHP", at_(enc), "BKI", nullptr, nullptr, g[EDATTN_WK], "HPI", 1.f},
+               {nullptr, at_(dkqv), "QBJHP", at_(x), "BJI", nullptr, nullptr, g[SATTN_WKQV], "QHPI", 1.f},
+               {nullptr, at_(datt1), "BJI", at_(k[GAMMA1]), "BJHP", nullptr, nullptr, g[SATTN_WO], "IHP", 1.f},
+               {nullptr, at_(dq2), "BJHP", at_(k[NORMED1]), "BJI", nullptr, nullptr, g[EDATTN_WQ], "HPI", 1.f},
+               {nullptr, at_(datt2), "BJI", at_(k[GAMMA2]), "BJHP", nullptr, nullptr, g[EDATTN_WO], "IHP", 1.f},
+               {nullptr, at_(dlin1), "BJU", at_(k[NORMED2]), "BJI", nullptr, nullptr, g[LINEAR1_W], "UI", 1.f},
+               {nullptr, at_(dff), "BJI", at_(k[FF1]), "BJU", nullptr, nullptr, g[LINEAR2_W], "IU", 1.f}});
+        deferred.finish();
+        return out;
+    }
+};
+
 }  // namespace
 
 PYBIND11_MODULE(_host, m) {
@@ -389,4 +662,9 @@ PYBIND11_MODULE(_host, m) {
         .def_property("mask", [](const EncoderLayer& l) { return l.mask; }, &EncoderLayer::use_mask)
         .def("set_step_counter", &EncoderLayer::set_step_counter)
         .def("forward", &EncoderLayer::forward);
+    py::class_<DecoderPasses>(m, "DecoderPasses")
+        .def(py::init<uintptr_t, uintptr_t, py::object, const std::vector<int64_t>&, const std::vector<double>&, const std::vector<uint32_t>&, bool,
+                      double>())
+        .def("forward", &DecoderPasses::forward)
+        .def("backward", &DecoderPasses::backward);
 }

@@ -161,3 +161,31 @@ def test_decoder_activation_epilogues_match_the_operators(activation):
             assert_close(_f64(a), _f64(b), tol=2e-3, name=name)
         else:
             assert torch.equal(a, b), name
+
+
+@pytest.mark.parametrize('lengths', [(128, 256), (128, 128)])
+def test_decoder_layer_refuses_a_tensor_of_another_type_and_goes_on(lengths):
+    """In either pass; any integer is a seed, those a multiple of 2**64 apart the same one."""
+    from substation_amd import DecoderLayer, _lib
+    Lt, Ls = lengths
+    layer = DecoderLayer(2, Lt, Ls, 2, 128, activation='gelu').cuda()
+    x = torch.randn(2, Lt, 128).half().cuda()
+    enc = torch.randn(2, Ls, 128).half().cuda()
+    dy = torch.randn(2, Lt, 128).half().cuda()
+
+    def run(seed=-3):
+        layer.set_rng(seed, 7)
+        layer.zero_grad(set_to_none=True)
+        y = layer(x, enc)
+        y.backward(dy)
+        return [y.detach()] + [p.grad for p in layer.parameters()]
+
+    want = run()
+    with pytest.raises(ValueError, match='contiguous fp16'):
+        layer(x, enc.float())
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t.float()):
+        y = layer(x, enc)
+    with pytest.raises(ValueError, match='contiguous fp16'):
+        y.backward(dy)
+    for a, b in zip(run(2 ** 64 - 3), want):
+        assert torch.equal(a, b)
