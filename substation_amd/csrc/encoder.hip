@@ -390,8 +390,9 @@ float* take_ws(Handle& h, size_t floats) {
         if (h.deferred.n > 0) launch_colfinish(h.deferred, h.stream);
         h.deferred.n = 0;
         h.ws_cursor = 0;
-        // twice the size as well: after a few calls the buffer holds every reduction of a block of calls
-        ensure_ws(h, floats > 2 * h.ws_floats ? floats : 2 * h.ws_floats);
+        // twice the size as well, and no less than two backward passes of the layer take: a new handle's first block of calls
+        // asks the device for memory once, where it went on doubling (each time a wait for all that runs)
+        ensure_ws(h, std::max({floats, 2 * h.ws_floats, 2 * h.ws_need_bwd}));
     }
     float* p = h.ws + h.ws_cursor;
     h.ws_cursor += (floats + 63) & ~(size_t)63;

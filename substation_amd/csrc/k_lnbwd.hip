@@ -175,20 +175,18 @@ __global__ __launch_bounds__(LN_BLOCK) void k_lnbwd(RowSpace rs, LnBwdArgs a, fl
 // (a lane still owns 16 columns, so the column sums stay in registers); the two sums over the row that
 // the LayerNorm backward needs meet in LDS, in wave order, behind one barrier per pass -- which is why
 // every wave then makes the same number of passes, a wave without a row walking row 0 and keeping nothing.
-constexpr int LNF_BLOCK = 1024;
-constexpr int LNF_WPB = LNF_BLOCK / WAVE;
-
-template <int VPL, bool EXT, bool PACKED, bool MOVE, int SEG = 1>
-__global__ __launch_bounds__(LNF_BLOCK) void k_lnbwd_flat(int R, LnBwdArgs a, float* ws, unsigned nrows) {
-    static_assert(SEG == 1 || VPL == 2, "a segment is 1024 features: two packs per lane");
-    constexpr int ROWS = LNF_WPB / SEG;           // rows per workgroup and pass
-    __shared__ float stat[2][LNF_WPB][2];         // SEG > 1: the waves' shares of the two row sums, by pass parity
+// WAVES: of a workgroup, sixteen where there are rows for all CUs (see lnbwd_waves).
+template <int VPL, bool EXT, bool PACKED, bool MOVE, int SEG = 1, int WAVES = 16>
+__global__ __launch_bounds__(WAVES * WAVE) void k_lnbwd_flat(int R, LnBwdArgs a, float* ws, unsigned nrows) {
+    static_assert(SEG == 1 || (VPL == 2 && WAVES == 16), "a segment is 1024 features: two packs per lane");
+    constexpr int ROWS = WAVES / SEG;             // rows per workgroup and pass
+    __shared__ float stat[2][WAVES][2];           // SEG > 1: the waves' shares of the two row sums, by pass parity
     constexpr int NS = MOVE ? 3 : (EXT ? 4 : 2);
     constexpr int S_DROP = MOVE ? 2 : 3;          // which sum takes d_drop_in
     constexpr bool DROP_SUM = EXT || MOVE;
     constexpr int NR = DROP_SUM ? NS - 1 : NS;    // sums kept in registers
-    __shared__ float red[LNF_WPB][VPL * WAVE * 8];
-    __shared__ float red2[LNF_WPB][VPL * WAVE * 8];     // a second set of slabs: two sums per reduction pass
+    __shared__ float red[WAVES][VPL * WAVE * 8];
+    __shared__ float red2[WAVES][VPL * WAVE * 8];     // a second set of slabs: two sums per reduction pass
     typedef int i4v __attribute__((ext_vector_type(4)));
     fetch_args_now(R, nrows, a.in.p, a.in.s3, a.d1.p, a.d1.s3, a.diff.p, a.diff.s3, a.istd.p, a.istd.s3, a.scale.p, a.g.p,
                    a.g.s3, a.d_ln_in.p, a.d_ln_in.s3, a.d_drop_in.p, a.d_drop_in.s3, a.write_g, ws);
@@ -342,7 +340,7 @@ __global__ __launch_bounds__(LNF_BLOCK) void k_lnbwd_flat(int R, LnBwdArgs a, fl
     };
     // (feature f lies in the slabs of the waves of its segment)
     auto reduce = [&](const float (*from)[VPL * WAVE * 8], int s) {
-        for (int f = threadIdx.x; f < R; f += LNF_BLOCK) {
+        for (int f = threadIdx.x; f < R; f += WAVES * WAVE) {
             const int sg = SEG > 1 ? f / (VPL * WAVE * 8) : 0, fl = SEG > 1 ? f % (VPL * WAVE * 8) : f;
             float t = 0.f;
 #pragma unroll
@@ -377,6 +375,22 @@ inline int lnbwd_blocks(long nrows) {
     return (int)blocks;
 }
 
+// Waves of a workgroup of k_lnbwd_flat for rows of up to 1024 features, a row each: as few as leave no more than 256 partial rows, one
+// workgroup per CU.  A CU draws 33 KB a us of what is not in its L2, however few of them do: with sixteen, 1024 rows were
+// read by 64 CUs.  us of the two launches of a layer, E 768, with sixteen waves and now: 256 rows 7.9 and 7.4, 5.7 and 5.1; 1024 rows 9.2 and
+// 7.7, 6.8 and 5.6.  2048 rows of 1024, mask as a tensor, 12.3 and (four sums, in the kernel above) 14.9, 10.0 and 10.4.  Beyond that
+// two workgroups of eight waves to a CU take what one of sixteen does (2613 and 4096 rows: 0.7 us either way), and the launch that adds
+// up 512 partial rows 1.5 us more.
+inline int lnbwd_waves(long nrows) { return nrows <= 1024 ? 4 : nrows <= 2048 ? 8 : 16; }
+inline int lnbwd_flat_blocks(long nrows) {
+    const int waves = lnbwd_waves(nrows);
+    return waves == 16 ? lnbwd_blocks(nrows) : (int)((nrows + waves - 1) / waves);
+}
+// (the extended form with its four sums does not fit the 128 registers of sixteen waves)
+inline bool lnbwd_flat(const RowSpace& rs, const LnBwdArgs& a, bool ext) {
+    return rs.flat && !(ext && !a.move_sum && lnbwd_waves(rs.rows()) == 16);
+}
+
 }  // namespace
 
 bool lnbwd_supported(const RowSpace& rs, const LnBwdArgs& a, bool ext) {
@@ -391,7 +405,8 @@ bool lnbwd_supported(const RowSpace& rs, const LnBwdArgs& a, bool ext) {
 }
 
 size_t lnbwd_ws_floats(const RowSpace& rs, bool ext) {
-    return (size_t)(ext ? 4 : 3) * lnbwd_blocks(rs.rows()) * rs.R;      // (3: the plain form with move_sum)
+    const int blocks = rs.R <= 1024 ? std::max(lnbwd_blocks(rs.rows()), lnbwd_flat_blocks(rs.rows())) : lnbwd_blocks(rs.rows());
+    return (size_t)(ext ? 4 : 3) * blocks * rs.R;      // (3: the plain form with move_sum)
 }
 
 void launch_lnbwd(const RowSpace& rs, const LnBwdArgs& a, bool ext, half_t* const sums[4], float* ws,
@@ -399,16 +414,17 @@ void launch_lnbwd(const RowSpace& rs, const LnBwdArgs& a, bool ext, half_t* cons
     if (!lnbwd_supported(rs, a, ext)) fail("fused LayerNorm backward: unsupported shape or layout");
     if (!ws) fail("fused LayerNorm backward: no reduction workspace");
     const unsigned nrows = (unsigned)rs.rows();
-    const int blocks = lnbwd_blocks(nrows);
+    const bool flat = rs.R <= 1024 && lnbwd_flat(rs, a, ext);
+    const int blocks = flat ? lnbwd_flat_blocks(nrows) : lnbwd_blocks(nrows);
     const int vpl = rs.R <= 512 ? 1 : 2;
     if (rs.R > 1024) {
         // (lnbwd_supported has ruled out the extended form without move_sum: MOVE_ is EXT_ || move_sum)
 #define SUB_LNBWD_WIDE(EXT_, MOVE_, SEG_)                                                                         \
     do {                                                                                                          \
         if (a.mask_bits)                                                                                          \
-            hipLaunchKernelGGL((k_lnbwd_flat<2, EXT_, true, MOVE_, SEG_>), dim3(blocks), dim3(LNF_BLOCK), 0, st, rs.R, a, ws, nrows); \
+            hipLaunchKernelGGL((k_lnbwd_flat<2, EXT_, true, MOVE_, SEG_>), dim3(blocks), dim3(16 * WAVE), 0, st, rs.R, a, ws, nrows); \
         else                                                                                                      \
-            hipLaunchKernelGGL((k_lnbwd_flat<2, EXT_, false, MOVE_, SEG_>), dim3(blocks), dim3(LNF_BLOCK), 0, st, rs.R, a, ws, nrows); \
+            hipLaunchKernelGGL((k_lnbwd_flat<2, EXT_, false, MOVE_, SEG_>), dim3(blocks), dim3(16 * WAVE), 0, st, rs.R, a, ws, nrows); \
     } while (0)
 #define SUB_LNBWD_WIDE_SEG(SEG_)                                                                                  \
     do {                                                                                                          \
@@ -421,22 +437,24 @@ void launch_lnbwd(const RowSpace& rs, const LnBwdArgs& a, bool ext, half_t* cons
 #undef SUB_LNBWD_WIDE_SEG
 #undef SUB_LNBWD_WIDE
     } else {
-#define SUB_LNBWD_K(KERNEL_, BLOCK_, FIRST_, VPL_, EXT_)                                                          \
+#define SUB_LNBWD_K(VPL_, EXT_, BITS_, MOVE_)                                                                     \
     do {                                                                                                          \
-        if (a.mask_bits && a.move_sum)                                                                            \
-            hipLaunchKernelGGL((KERNEL_<VPL_, EXT_, true, true>), dim3(blocks), dim3(BLOCK_), 0, st, FIRST_, a, ws, nrows);  \
-        else if (a.mask_bits)                                                                                     \
-            hipLaunchKernelGGL((KERNEL_<VPL_, EXT_, true, false>), dim3(blocks), dim3(BLOCK_), 0, st, FIRST_, a, ws, nrows); \
-        else if (a.move_sum)                                                                                      \
-            hipLaunchKernelGGL((KERNEL_<VPL_, EXT_, false, true>), dim3(blocks), dim3(BLOCK_), 0, st, FIRST_, a, ws, nrows); \
-        else                                                                                                      \
-            hipLaunchKernelGGL((KERNEL_<VPL_, EXT_, false, false>), dim3(blocks), dim3(BLOCK_), 0, st, FIRST_, a, ws, nrows); \
+        const dim3 grid(blocks);                                                                                  \
+        if (!flat) hipLaunchKernelGGL((k_lnbwd<VPL_, EXT_, BITS_, MOVE_>), grid, dim3(LN_BLOCK), 0, st, rs, a, ws, nrows);       \
+        else switch (lnbwd_waves(nrows)) {                                                                        \
+            case 4: hipLaunchKernelGGL((k_lnbwd_flat<VPL_, EXT_, BITS_, MOVE_, 1, 4>), grid, dim3(4 * WAVE), 0, st, rs.R, a, ws, nrows); break; \
+            case 8: hipLaunchKernelGGL((k_lnbwd_flat<VPL_, EXT_, BITS_, MOVE_, 1, 8>), grid, dim3(8 * WAVE), 0, st, rs.R, a, ws, nrows); break; \
+            default:                                                                                              \
+                if constexpr (!EXT_ || MOVE_)                                                                     \
+                    hipLaunchKernelGGL((k_lnbwd_flat<VPL_, EXT_, BITS_, MOVE_>), grid, dim3(16 * WAVE), 0, st, rs.R, a, ws, nrows); \
+        }                                                                                                         \
     } while (0)
-    // (the extended form with its four sums does not fit the sixteen-wave kernel's registers)
 #define SUB_LNBWD(VPL_, EXT_)                                                                                     \
     do {                                                                                                          \
-        if (rs.flat && !(EXT_ && !a.move_sum)) SUB_LNBWD_K(k_lnbwd_flat, LNF_BLOCK, rs.R, VPL_, EXT_);            \
-        else SUB_LNBWD_K(k_lnbwd, LN_BLOCK, rs, VPL_, EXT_);                                                      \
+        if (a.mask_bits && a.move_sum) SUB_LNBWD_K(VPL_, EXT_, true, true);                                       \
+        else if (a.mask_bits) SUB_LNBWD_K(VPL_, EXT_, true, false);                                               \
+        else if (a.move_sum) SUB_LNBWD_K(VPL_, EXT_, false, true);                                                \
+        else SUB_LNBWD_K(VPL_, EXT_, false, false);                                                               \
     } while (0)
     if (ext) {
         if (vpl == 1) SUB_LNBWD(1, true);

@@ -406,6 +406,21 @@ def test_ln_backward_one_launch_or_separate(B, L, H, E, extended):
             assert_close(dlb.float().cpu().numpy(), w[3], name='DLINEAR_BIAS')
             assert_close(dob.float().cpu().numpy(), ref.op_baob(from_layout(o2, 'BJI', lay)), name='DOUT_BIAS')
 
+# (where the number of waves of a workgroup changes: 1024 and 2048 rows, a last workgroup of one row; one, two packs a lane)
+@pytest.mark.parametrize('B,L,E', [(1, 1, 1024), (1, 5, 520), (1, 1024, 512), (5, 205, 776), (2, 1024, 1024), (3, 683, 512)])
+@pytest.mark.parametrize('extended', [False, True])
+def test_ln_backward_in_workgroups_of_every_size(B, L, E, extended):
+    test_ln_backward_one_launch_or_separate(B, L, 1, E, extended)
+
+
+@pytest.mark.parametrize('dims', [(1, 4, 2, 128), (1, 513, 1, 64), (9, 128, 2, 128), (2, 512, 12, 768), (9, 233, 1, 64)])
+def test_layer_norm_passes_of_few_rows_match_the_oracle(dims):
+    """Bias-dropout-residual-LayerNorm and its backward pass as the layer launches them, masks as bits: 4 rows, a row and two rows to a
+    workgroup forward (513: the last one has one row), four, eight and sixteen waves backward."""
+    from tests.test_encoder_gpu import OUTPUTS, _compare, run_layer_default
+    want, got = run_layer_default(*dims, 0.1, act='gelu', seed_data=3)
+    _compare(want, got, names=OUTPUTS)
+
 
 @pytest.mark.parametrize('dims', [(2, 64, 2, 128), (3, 40, 3, 120), (2, 5, 1, 20), (8, 512, 16, 1024)])
 def test_relayout_is_a_permutation_of_the_same_tensor(dims):
