@@ -352,11 +352,11 @@ __global__ __launch_bounds__(BLOCK) void k_bdrln_flat(int R, unsigned nrows, Vie
                                                       View scale, View bias, View lin, View mask, View diff,
                                                       View normed, View out, View istd, PhiloxKey key_, float eps,
                                                       uint8_t* mask_bits, bool write_lin, KeepWordsJob side,
-                                                      SplitSums sums, bool saves) {
+                                                      SplitSums sums, bool saves, unsigned waves) {
     if (SUMS) fetch_args_now(sums.p, sums.splits, sums.slab, sums.alpha);
     fetch_args_now(R, nrows, in.p, in.s3, resid.p, resid.s3, lin_bias.p, scale.p, bias.p, lin.p, lin.s3, mask.p, mask.s3,
                    diff.p, diff.s3, normed.p, normed.s3, out.p, out.s3, istd.p, istd.s3, key_.k0, key_.k1, key_.site,
-                   key_.step, key_.thr, key_.step_dev, eps, mask_bits, write_lin, side.blocks, saves);
+                   key_.step, key_.thr, key_.step_dev, eps, mask_bits, write_lin, side.blocks, saves, waves);
     const unsigned row_blocks = gridDim.x - side.blocks;
     if (blockIdx.x >= row_blocks) {
         const PhiloxKey skey = resolved(side.key);
@@ -390,7 +390,7 @@ __global__ __launch_bounds__(BLOCK) void k_bdrln_flat(int R, unsigned nrows, Vie
         bi8[c] = ldg8<false>(bias.p + e0[c]);
     }
     auto masked = [&](h8 v, int c) { return __builtin_bit_cast(h8, __builtin_bit_cast(i4v, v) & keep_all[c]); };
-    for (unsigned row = blockIdx.x * WPB + (threadIdx.x >> 6); row < nrows; row += row_blocks * WPB) {
+    for (unsigned row = blockIdx.x * waves + (threadIdx.x >> 6); row < nrows; row += row_blocks * waves) {
         h8 vi[VPL], vr[VPL];
         float4 part[SUMS ? VPL : 1][8][2];
 #pragma unroll
@@ -777,9 +777,12 @@ void launch_bdrln(const RowSpace& rs, View in, View resid, View lin_bias, View s
         sums.p = nullptr;
     }
     if (flat) {
-        const dim3 grid(row_grid(nrows, 1) + extra_blocks);
-#define SUB_BDRLN_FLAT(V, S) hipLaunchKernelGGL((k_bdrln_flat<V, S>), grid, dim3(BLOCK), 0, st, rs.R, nrows, in, resid, lin_bias, \
-                                             scale, bias, lin, mask, diff, normed, out, istd, key, eps, mask_bits, write_lin, job, sums, saves)
+        // Few rows: each in a workgroup of its own, since a CU draws 33 KB a us of what is not in its L2, however few CUs do (64 rows of 768,
+        // us with four rows to a workgroup and now: 3.9 and 3.7, with the parts of a split sum 5.3 and 4.5; 256 rows: no difference).
+        const unsigned waves = extra_blocks || nrows >= 256 ? WPB : 1;
+        const dim3 grid(waves == WPB ? row_grid(nrows, 1) + extra_blocks : nrows), block(waves * WAVE);
+#define SUB_BDRLN_FLAT(V, S) hipLaunchKernelGGL((k_bdrln_flat<V, S>), grid, block, 0, st, rs.R, nrows, in, resid, lin_bias, \
+                                             scale, bias, lin, mask, diff, normed, out, istd, key, eps, mask_bits, write_lin, job, sums, saves, waves)
         if (sums.p && vpl == 1) SUB_BDRLN_FLAT(1, true);
         else if (sums.p) SUB_BDRLN_FLAT(2, true);
         else switch (vpl) {
