@@ -428,7 +428,8 @@ int sub_op_baob(void* handle, const void* datt, const char* l_datt, void* dbo);
  * encoder_backward does for its own (encoder.cu:158-299 has one kernel per
  * reduction; no counterpart there).  The gradient vectors are complete only after
  * that call; same bits as without.  When the list (6 entries) or the scratch buffer
- * is full, what is on the list is finished early.  encoder_backward refuses to run
+ * is full, what is on the list is finished early, and so it is by a group of contractions
+ * (sub_op_einsum_group), whose last launch has room for it.  encoder_backward refuses to run
  * in between. */
 int sub_ops_defer(void* handle, int on);
 /* block_aib.cuh:64-155, on the Q-stacked tensors */

@@ -4,6 +4,7 @@ C ABI.  Inputs are rounded to fp16 first, so the only difference left is the
 device's fp32-internal arithmetic and one fp16 rounding per output: tolerance
 1e-2 relative (pytorch_module/benchmark.py:294-302 uses atol=rtol=1e-2).
 Dropout masks are compared bit-exactly with oracle/philox_ref.py."""
+import contextlib
 import itertools
 
 import numpy as np
@@ -240,6 +241,39 @@ def test_deferred_column_sums_give_the_same_bits():
     o.baob(tensors[0][1], 'BJI', dbo)
     torch.cuda.synchronize()
     assert torch.equal(dbo, plain[3])
+
+
+@pytest.mark.parametrize('E', [64, 192, 1024])
+@pytest.mark.parametrize('finish_in_group', [0, 1])
+def test_deferred_column_sums_finished_by_a_group_of_contractions(E, finish_in_group):
+    """Put off, and finished in the last launch of a group of products (option 7) or behind it: the bits of neither."""
+    from substation_amd import _lib
+    B, L = 3, 72
+    o = _ops(B, L, 1, E)
+    o.handle.set_option(_lib.OPT_FINISH_IN_PAIR, finish_in_group)
+    g = torch.Generator(device='cuda').manual_seed(7)
+    rand = lambda layout: torch.randn(o.empty(layout).shape, generator=g, device='cuda').half()
+    a, b, w, d = rand('BJI'), rand('BJI'), rand('UI'), rand('BJU')
+
+    def run(deferred, group):
+        sums = [torch.zeros(E, dtype=torch.float16, device='cuda') for _ in range(8)]
+        big, dw = o.empty('BJU'), o.empty('UI')
+        with o.deferred_column_sums() if deferred else contextlib.nullcontext():
+            for s in sums[:4]:
+                o.baob(a, 'BJI', s)
+            if group:
+                o.einsum_group([(a, 'BJI', w, 'UI', big, 'BJU'), (d, 'BJU', b, 'BJI', dw, 'UI')])
+            for s in sums[4:]:
+                o.baob(b, 'BJI', s)
+            if group:
+                o.einsum_group([(a, 'BJI', w, 'UI', big, 'BJU')])
+        torch.cuda.synchronize()
+        return sums
+
+    want = run(False, False)
+    for got in (run(True, True), run(True, False)):
+        for x, y in zip(got, want):
+            assert torch.equal(x, y)
 
 
 @pytest.mark.parametrize('B,L,H,E', SIZES + [(2, 3, 1, 20), (4, 64, 1, 1024), (2, 8, 1, 4096)])
