@@ -614,7 +614,7 @@ void plan_layouts(Handle& h, bool own) {
                        colreduce_ws_floats(su.rs, 1) + (baib > baib2 ? baib : baib2) + 8 * 64;
         if (fused > h.ws_need_bwd) h.ws_need_bwd = fused;
         // the attention kernels' partial sums for the projection-bias gradient stand in for baib's
-        const size_t attn_bias = (size_t)(3 * sz.n[dH] * sz.n[dB] * ((sz.n[dJ] + 127) / 128) * sz.n[dP]);
+        const size_t attn_bias = mha_bias_floats(sz.n[dH], sz.n[dB], sz.n[dJ], sz.n[dJ], sz.n[dP]);
         if (attn_bias > (baib > baib2 ? baib : baib2)) h.ws_need_bwd += attn_bias;
         // the partial column sums of dXlin2's epilogue
         if (h.gemm[G_DXLIN2_BDRLB].ok) {
@@ -1283,7 +1283,7 @@ void forward(Handle& h, const FwdPtrs& t0, bool alone) {
     if (fused_attention) {
         ProfScope ps(h, "attention");
         mask_plan(h, at, true);
-        launch_mha_forward(at, (int)h.sz.n[dP], make_key(h, SUB_SITE_SOFTMAX, h.p_softmax), h.stream);
+        launch_mha_forward(at, (int)h.sz.n[dP], make_key(h, SUB_SITE_SOFTMAX, h.p_softmax), h.act == ACT_RELU, h.stream);
     }
     bool fused_scores = fused_attention;
     if (!registers && h.fuse_scores) {
@@ -1542,7 +1542,7 @@ void backward(Handle& h, const BwdPtrs& t0) {
         const Layout& lbias = h.lp[BKQV];
         attn_bias = lbias.has[dQ] && lbias.has[dH] && lbias.has[dP];
         const int P = (int)h.sz.n[dP], H = (int)h.sz.n[dH];
-        const int ntq = at.B * ((at.J + 127) / 128), ntk = at.B * ((at.K + 127) / 128);
+        const int ntq = (int)mha_bias_rows_q(at, P), ntk = (int)mha_bias_rows_kv(at, P);
         half_t* dbias = (half_t*)DW[BKQV];
         auto finish = [&](float* ws, int ns, int ntc, half_t* o0, half_t* o1) {
             FinishJob job{ws, FinishArgs{{o0, o1, nullptr, nullptr}, 0, lbias.stride[dH], lbias.stride[dP], H}, ns, H,
@@ -1982,7 +1982,7 @@ int sub_op_attention_forward(void* handle, int n_queries, int n_keys, const void
         AttnArgs a;
         op_attention_args(h, n_queries, n_keys, q, l_q, k, v, l_kv, out, l_out, stats, keep, attn_mask,
                           l_attn_mask, scale, a);
-        launch_mha_forward(a, (int)h.sz.n[dP], make_key(h, site, p), h.stream);
+        launch_mha_forward(a, (int)h.sz.n[dP], make_key(h, site, p), h.act == ACT_RELU, h.stream);
     });
 }
 
@@ -2015,10 +2015,10 @@ int sub_op_attention_backward_biases(void* handle, int n_queries, int n_keys, co
             !attn_side(dk, make_layout(l_dkv, z), dK, a.dk) || !attn_side(dv, make_layout(l_dkv, z), dK, a.dv))
             fail("attention backward: d_out and dq take a layout over B, J, H, P and dk, dv one over B, K, H, P, "
                  "P innermost");
-        // the sums over (sample, position) of dq, dk, dv start in these launches (one partial row per block of
-        // 128 positions) and end in the finishing stage of the column sums, deferred or not
+        // the sums over (sample, position) of dq, dk, dv start in these launches (partial rows for blocks of
+        // positions) and end in the finishing stage of the column sums, deferred or not
         const int P = (int)h.sz.n[dP], H = (int)h.sz.n[dH];
-        const int ntq = a.B * (a.J / 128), ntk = a.B * (a.K / 128);
+        const int ntq = (int)mha_bias_rows_q(a, P), ntk = (int)mha_bias_rows_kv(a, P);
         auto finish = [&](float* ws, int ns, int ntc, void* o0, void* o1) {
             FinishJob job{ws, FinishArgs{{(half_t*)o0, (half_t*)o1, nullptr, nullptr}, 0, P, 1, H}, ns, H, ntc, P};
             finish_or_defer(defer_of(h), job, h.stream);

@@ -42,7 +42,7 @@ struct Geo {
     static constexpr int NKS = P / 16;             // k-steps of a contraction over the features
     static constexpr int NPT = P / 32;             // 32-wide tiles of the feature dim
     static constexpr int TILE = 32 * P;            // halves of an LDS tile of 32 positions
-    static constexpr int VL = (32 * (P / 8)) / 256; // 16-byte words per thread and tile
+    static constexpr int VL = (32 * (P / 8)) / 256; // 16-byte words per thread and tile (of 256 threads)
 
     // LDS tiles are [position][feature] without padding; the index of a 16-byte
     // chunk within its row is xor-ed with a function of the row chosen so that both
@@ -76,12 +76,13 @@ __device__ __forceinline__ void row_frags_lds(const half_t* tile, int l32, int h
 
 // A tile of 32 positions x P features: global -> registers -> LDS, all threads.  RAGGED: positions from `limit` on
 // read the last one that there is (their scores are taken out where they would count).
-template <int P, bool RAGGED>
+// PARTS: by 256 / PARTS threads.
+template <int P, bool RAGGED, int PARTS = 1>
 __device__ __forceinline__ void tile_fetch(const AttnSide& t, unsigned h, unsigned b, unsigned pos0, unsigned limit, int tid,
-                                           h8 (&r)[Geo<P>::VL]) {
+                                           h8 (&r)[Geo<P>::VL * PARTS]) {
 #pragma unroll
-    for (int i = 0; i < Geo<P>::VL; ++i) {
-        const int id = tid + i * 256, row = id / (P / 8), c = id % (P / 8);
+    for (int i = 0; i < Geo<P>::VL * PARTS; ++i) {
+        const int id = tid + i * (256 / PARTS), row = id / (P / 8), c = id % (P / 8);
         const unsigned pos = RAGGED ? min(pos0 + row, limit - 1) : pos0 + row;
         r[i] = *reinterpret_cast<const h8*>(t.p + (long)h * t.sh + (long)b * t.sb + (long)pos * t.sr + c * 8);
     }
@@ -90,23 +91,24 @@ __device__ __forceinline__ void tile_fetch(const AttnSide& t, unsigned h, unsign
 // along; else wherever they lie, by a 64-bit product for each row (four to eight quarter-rate multiplications a tile among
 // vector work that bounds these kernels: H 16, P 64, 8 x 512 forward 24.8 -> 24.2 us, dK and dV 31.2 -> 30.6; H 32, P 128,
 // 4 x 2048 forward 497 -> 487, dQ 528 -> 509).
-template <int P, bool WALK, bool RAGGED>
+template <int P, bool WALK, bool RAGGED, int PARTS>
 struct Tiles {
     const half_t* p;
-    __device__ __forceinline__ Tiles(const AttnSide& t, unsigned h, unsigned b, int tid)
-        : p(t.p + (long)h * t.sh + (long)b * t.sb + (long)(tid / (P / 8)) * t.sr + tid % (P / 8) * 8) {}
-    __device__ __forceinline__ void fetch(const AttnSide& t, unsigned h, unsigned b, unsigned tile, unsigned limit, int tid, h8 (&r)[Geo<P>::VL]) {
-        if (!WALK) { tile_fetch<P, RAGGED>(t, h, b, tile * 32, limit, tid, r); return; }
+    __device__ __forceinline__ Tiles(const AttnSide& t, unsigned h, unsigned b, unsigned first, int tid)
+        : p(t.p + (long)h * t.sh + (long)b * t.sb + (long)(first * 32 + tid / (P / 8)) * t.sr + tid % (P / 8) * 8) {}
+    __device__ __forceinline__ void fetch(const AttnSide& t, unsigned h, unsigned b, unsigned tile, unsigned limit, int tid,
+                                          h8 (&r)[Geo<P>::VL * PARTS]) {
+        if (!WALK) { tile_fetch<P, RAGGED, PARTS>(t, h, b, tile * 32, limit, tid, r); return; }
 #pragma unroll
-        for (int i = 0; i < Geo<P>::VL; ++i) r[i] = *reinterpret_cast<const h8*>(p + i * (256 / (P / 8)) * t.sr);
+        for (int i = 0; i < Geo<P>::VL * PARTS; ++i) r[i] = *reinterpret_cast<const h8*>(p + i * (256 / PARTS / (P / 8)) * t.sr);
         p += 32 * t.sr;
     }
 };
-template <int P>
-__device__ __forceinline__ void tile_put(half_t* tile, int tid, const h8 (&r)[Geo<P>::VL]) {
+template <int P, int PARTS = 1>
+__device__ __forceinline__ void tile_put(half_t* tile, int tid, const h8 (&r)[Geo<P>::VL * PARTS]) {
 #pragma unroll
-    for (int i = 0; i < Geo<P>::VL; ++i) {
-        const int id = tid + i * 256, row = id / (P / 8), c = id % (P / 8);
+    for (int i = 0; i < Geo<P>::VL * PARTS; ++i) {
+        const int id = tid + i * (256 / PARTS), row = id / (P / 8), c = id % (P / 8);
         *reinterpret_cast<h8*>(tile + Geo<P>::at(row, c)) = r[i];
     }
 }
@@ -189,12 +191,12 @@ __device__ __forceinline__ void store_rows(const AttnSide& t, unsigned h, unsign
     for (int e = 0; e < 8; e += 4)
         *reinterpret_cast<float4*>(sums + (lane >> 4) * P + chunk * 8 + e) = make_float4(x[e], x[e + 1], x[e + 2], x[e + 3]);
 }
-// One value per feature of what four waves have left in `sums`; behind a barrier.
-template <int P>
+// One value per feature of what WAVES waves have left in `sums`; behind a barrier.
+template <int P, int WAVES>
 __device__ __forceinline__ float column_sum(const float* sums, int feature) {
     float x[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int i = 0; i < 16; ++i) x[i & 3] += sums[i * P + feature];
+    for (int i = 0; i < 4 * WAVES; ++i) x[i & 3] += sums[i * P + feature];
     return (x[0] + x[1]) + (x[2] + x[3]);
 }
 
@@ -254,12 +256,12 @@ __device__ __forceinline__ void start_from_mask(const MaskRegs& mk, f16v& s) {
 // kernel) a list names the tiles of the other side that are not dead for all
 // four waves; the kernels walk that list instead of all tiles.
 //   row of a list: [0] = number of entries, then the entries, then padding that
-//   reads as "tile 0, dead for all waves" (the kernels read up to 3 past the end).
+//   reads as "tile 0, dead for all waves" (the kernels read up to 4 past the end).
 //   entry: bits 0..15 tile index, bits 16+2w.. the class of the block for wave w.
 // ---------------------------------------------------------------------------
 enum : uint32_t { BLOCK_MIXED = 0, BLOCK_DEAD = 1, BLOCK_CLEAR = 2 };
 constexpr uint32_t kAllDead = BLOCK_DEAD * 0x55u << 16;
-constexpr int kListPad = 4;       // the count and three entries of padding
+constexpr int kListPad = 5;       // the count and four entries of padding
 
 // One wave per 32x32 block of the mask.
 __global__ __launch_bounds__(64) void k_mha_mask_classes(const half_t* mask, long sj, long sk, int J, int K, uint8_t* cls) {
@@ -347,8 +349,45 @@ __device__ __forceinline__ uint32_t entry_class(uint32_t e, int wave) {
 // buffers: while tile t is worked on, tile t+1 already lies in LDS (its row
 // fragments are read ahead, during the vector work on tile t) and tile t+2 is on
 // its way from memory in registers.  One barrier per tile.
+//
+// PARTS = 2 (head size 64): two waves of 32 positions and, for each, two waves that walk a half of the other side's tiles
+// each, through a ring of their own.  What they have come to is added up at the end, by way of LDS.  Twice the workgroups
+// with half the tiles each, where there are few (see parts).
 // ---------------------------------------------------------------------------
 constexpr int RING = 3;
+constexpr long kFewBlocks = 128;  // workgroups of a launch without (see parts)
+
+// The place of a wave: of `blocks` of QB positions, in PARTS pieces each.
+template <int PARTS>
+struct Place {
+    static constexpr int WAVES = 4 / PARTS;          // of 32 positions
+    int tid, lane, wave, half;                       // (tid, wave: within the half)
+    __device__ __forceinline__ Place() : tid(threadIdx.x % (256 / PARTS)), lane(threadIdx.x & 63), wave((threadIdx.x >> 6) % WAVES),
+                                         half(PARTS > 1 ? threadIdx.x / (256 / PARTS) : 0) {}
+};
+
+// A wave's accumulators to the other half's wave and back: 16 N words of 64 lanes.
+template <int N>
+__device__ __forceinline__ void leave(float* to, int lane, const f16v (&acc)[N]) {
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; v += 4)
+            *reinterpret_cast<float4*>(to + ((i * 4 + v / 4) * 64 + lane) * 4) = make_float4(acc[i][v], acc[i][v + 1], acc[i][v + 2], acc[i][v + 3]);
+}
+// acc = acc * mine + (what is left there) * theirs; what lay there is no longer needed.
+template <int N>
+__device__ __forceinline__ void collect(const float* from, int lane, f16v (&acc)[N], float mine, float theirs) {
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; v += 4) {
+            const float4 x = *reinterpret_cast<const float4*>(from + ((i * 4 + v / 4) * 64 + lane) * 4);
+            acc[i][v] = acc[i][v] * mine + x.x * theirs; acc[i][v + 1] = acc[i][v + 1] * mine + x.y * theirs;
+            acc[i][v + 2] = acc[i][v + 2] * mine + x.z * theirs; acc[i][v + 3] = acc[i][v + 3] * mine + x.w * theirs;
+        }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // (halves are written there next, which the compiler takes for other memory)
+}
 
 // Every load issued so far has arrived.  Placed before a main loop: a load of the
 // prologue whose first use is inside the loop would otherwise put its wait there,
@@ -363,44 +402,50 @@ __device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0F70
 // one by one, with the score-sized tensors in memory and, for lengths that are not multiples of 8, products
 // through the scalar kernel: the layer's forward and backward at B=13 L=201 E=768 took 3990 us.
 // ---------------------------------------------------------------------------
-template <int P, bool MASKED, bool RAGGED>
-__global__ __launch_bounds__(256) void k_mha_fwd(AttnArgs a, PhiloxKey key_) {
+template <int P, bool MASKED, bool RAGGED, int PARTS>
+__device__ __forceinline__ void mha_fwd(const AttnArgs& a, const PhiloxKey& key_) {
     using G = Geo<P>;
-    __shared__ __attribute__((aligned(16))) half_t kt[RING][G::TILE];
-    __shared__ __attribute__((aligned(16))) half_t vt[RING][G::TILE];
+    __shared__ __attribute__((aligned(16))) half_t kt_[PARTS][RING][G::TILE];
+    __shared__ __attribute__((aligned(16))) half_t vt_[PARTS][RING][G::TILE];
     const PhiloxKey key = resolved(key_);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, hi = lane >> 5;
+    const Place<PARTS> at;
+    const int tid = at.tid, lane = at.lane, wave = at.wave, l32 = lane & 31, hi = lane >> 5;
+    half_t (*const kt)[G::TILE] = kt_[at.half];
+    half_t (*const vt)[G::TILE] = vt_[at.half];
     const unsigned qblocks = RAGGED ? (a.J + QB - 1) / QB : a.J / QB;
-    const unsigned lb = logical_block();
+    const unsigned lb = logical_block() / PARTS;
     const unsigned nt = RAGGED ? (a.K + 31) / 32 : a.K / 32, pitch = RAGGED ? keep_pitch(a.K) : nt;
     unsigned qb = lb % qblocks, hb = lb / qblocks;
     if (MASKED) masked_order(a.qlist, qblocks, nt, a.H * a.B, lb, qb, hb);
     const unsigned b = hb % a.B, h = hb / a.B;
-    const unsigned j_ = qb * QB + wave * 32 + l32;                   // this lane's query
+    const int piece = PARTS > 1 ? (int)(logical_block() % PARTS) * Place<PARTS>::WAVES : 0;      // its first wave's, of the block's four
+    const unsigned j_ = qb * QB + (piece + wave) * 32 + l32;                   // this lane's query
     const bool mine_ = !RAGGED || j_ < (unsigned)a.J;                // (RAGGED: lanes past the end follow the last query)
     const unsigned j = RAGGED ? min(j_, (unsigned)a.J - 1) : j_;
     // waves whose queries all lie past the end only help with the tiles
-    const bool working = !RAGGED || __builtin_amdgcn_readfirstlane((int)(qb * QB + wave * 32)) < a.J;
+    const bool working = !RAGGED || __builtin_amdgcn_readfirstlane((int)(qb * QB + (piece + wave) * 32)) < a.J;
     const unsigned row = (h * a.B + b) * a.J + j;                    // its score row
     const float c = a.alpha * LOG2E;
     // the key tiles to walk: all of them, or those a mask leaves for these 128 queries
     const uint32_t* live = (MASKED && a.qlist) ? a.qlist + (size_t)qb * (nt + kListPad) : nullptr;
-    const unsigned n = live ? live[0] : nt;
-    uint32_t e0 = live_entry<MASKED>(live, 0), e1 = live_entry<MASKED>(live, 1), e2 = live_entry<MASKED>(live, 2);
+    const unsigned all = live ? live[0] : nt, longest = (all + PARTS - 1) / PARTS;
+    // (the second half's begin behind the first's; of an odd number it has one less)
+    const unsigned begin = at.half ? longest : 0, n = at.half ? all - longest : longest;
+    uint32_t e0 = live_entry<MASKED>(live, begin), e1 = live_entry<MASKED>(live, begin + 1), e2 = live_entry<MASKED>(live, begin + 2);
 
-    h8 fq[G::NKS], fk[G::NKS], kr[G::VL], vr[G::VL];
-    Tiles<P, !MASKED && !RAGGED, RAGGED> tiles_k(a.k, h, b, tid), tiles_v(a.v, h, b, tid);
+    h8 fq[G::NKS], fk[G::NKS], kr[G::VL * PARTS], vr[G::VL * PARTS];
+    Tiles<P, !MASKED && !RAGGED, RAGGED, PARTS> tiles_k(a.k, h, b, begin, tid), tiles_v(a.v, h, b, begin, tid);
     {   // the first two tiles and the query rows: all loads in flight together
-        h8 kr1[G::VL], vr1[G::VL];
+        h8 kr1[G::VL * PARTS], vr1[G::VL * PARTS];
         tiles_k.fetch(a.k, h, b, entry_tile(e0), a.K, tid, kr);
         tiles_v.fetch(a.v, h, b, entry_tile(e0), a.K, tid, vr);
         tiles_k.fetch(a.k, h, b, entry_tile(e1), a.K, tid, kr1);
         tiles_v.fetch(a.v, h, b, entry_tile(e1), a.K, tid, vr1);
         row_frags<P>(a.q, h, b, j, hi, fq);
-        tile_put<P>(kt[0], tid, kr);
-        tile_put<P>(vt[0], tid, vr);
-        tile_put<P>(kt[1], tid, kr1);
-        tile_put<P>(vt[1], tid, vr1);
+        tile_put<P, PARTS>(kt[0], tid, kr);
+        tile_put<P, PARTS>(vt[0], tid, vr);
+        tile_put<P, PARTS>(kt[1], tid, kr1);
+        tile_put<P, PARTS>(vt[1], tid, vr1);
     }
     __syncthreads();
     row_frags_lds<P>(kt[0], l32, hi, fk);
@@ -414,7 +459,7 @@ __global__ __launch_bounds__(256) void k_mha_fwd(AttnArgs a, PhiloxKey key_) {
     const float slack = RESCALE_SLACK / c;
     int cur = 0, nxt = 1, nn = 2;
     MaskRegs mk = {};
-    if (MASKED && n > 0 && entry_class(e0, wave) != BLOCK_CLEAR) load_mask<true, RAGGED>(a, j, entry_tile(e0) * 32, hi, mk);
+    if (MASKED && n > 0 && entry_class(e0, piece + wave) != BLOCK_CLEAR) load_mask<true, RAGGED>(a, j, entry_tile(e0) * 32, hi, mk);
     // keep words drawn ahead of this launch are fetched a tile early: at the place of their
     // use the load would stand between the scores and their exponentials
     uint32_t word_ahead = 0;
@@ -426,10 +471,10 @@ __global__ __launch_bounds__(256) void k_mha_fwd(AttnArgs a, PhiloxKey key_) {
     uint32_t carry = 0, carry_tile = ~0u;
     wait_loads();
 
-    for (unsigned i = 0; i < n; ++i) {
-        const uint32_t e3 = live_entry<MASKED>(live, i + 3);
+    for (unsigned i = 0; i < longest; ++i) {
+        const uint32_t e3 = live_entry<MASKED>(live, begin + i + 3);
         const unsigned t = entry_tile(e0);
-        const bool from_mask = MASKED && entry_class(e0, wave) != BLOCK_CLEAR;
+        const bool from_mask = MASKED && entry_class(e0, piece + wave) != BLOCK_CLEAR;
         const bool fetch = i + 2 < n;
         const uint32_t word_ready = word_ahead;
         if (key.thr && i + 1 < n && entry_tile(e1) < a.keep_tiles_ready)
@@ -438,12 +483,12 @@ __global__ __launch_bounds__(256) void k_mha_fwd(AttnArgs a, PhiloxKey key_) {
             tiles_k.fetch(a.k, h, b, entry_tile(e2), a.K, tid, kr);
             tiles_v.fetch(a.v, h, b, entry_tile(e2), a.K, tid, vr);
         }
-        if (working) {
+        if (working && (PARTS == 1 || i < n)) {
         f16v s;
 #pragma unroll
         for (int v = 0; v < 16; ++v) s[v] = 0.f;
         if (from_mask) start_from_mask(mk, s);
-        if (MASKED && i + 1 < n && entry_class(e1, wave) != BLOCK_CLEAR) load_mask<true, RAGGED>(a, j, entry_tile(e1) * 32, hi, mk);
+        if (MASKED && i + 1 < n && entry_class(e1, piece + wave) != BLOCK_CLEAR) load_mask<true, RAGGED>(a, j, entry_tile(e1) * 32, hi, mk);
 #pragma unroll
         for (int ks = 0; ks < G::NKS; ++ks) s = __builtin_amdgcn_mfma_f32_32x32x16_f16(fk[ks], fq[ks], s, 0, 0, 0);
         // fragments for the second product of this tile and the first of the next
@@ -537,55 +582,91 @@ __global__ __launch_bounds__(256) void k_mha_fwd(AttnArgs a, PhiloxKey key_) {
                 o[pt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[st][pt], pb[st], o[pt], 0, 0, 0);
         }
         if (fetch) {
-            tile_put<P>(kt[nn], tid, kr);
-            tile_put<P>(vt[nn], tid, vr);
+            tile_put<P, PARTS>(kt[nn], tid, kr);
+            tile_put<P, PARTS>(vt[nn], tid, vr);
         }
         __syncthreads();
         const int x = cur; cur = nxt; nxt = nn; nn = x;
         e0 = e1; e1 = e2; e2 = e3;
     }
-    const float l_tot = l_run + __shfl_xor(l_run, 32);
     const int w = __builtin_amdgcn_readfirstlane(wave);
-    store_rows<P, RAGGED>(a.o, h, b, qb * QB + w * 32, a.J, lane, o, 1.0f / l_tot, w < 2 ? kt[w] : vt[w - 2], nullptr);
+    half_t* out = w < 2 ? kt[w] : vt[w - 2];
+    if constexpr (PARTS > 1) {
+        // (the tiles' places are free)
+        static_assert(Place<PARTS>::WAVES * G::NPT * 16 * 64 * sizeof(float) <= sizeof(kt_), "two waves' accumulators");
+        float* const left = reinterpret_cast<float*>(kt_) + wave * (G::NPT * 16 * 64);
+        float* const stats = reinterpret_cast<float*>(vt_) + wave * 128;
+        if (at.half) {
+            leave(left, lane, o);
+            stats[lane] = m_ref;
+            stats[64 + lane] = l_run;
+        }
+        __syncthreads();
+        if (at.half) return;
+        const float m1 = stats[lane], m_new = fmaxf(m_ref, m1);
+        // (a half that has seen no key of this query has nothing, and no reference)
+        const float mine = m_ref == -INFINITY ? (m_new == -INFINITY ? 1.f : 0.f) : __builtin_amdgcn_exp2f((m_ref - m_new) * c);
+        const float theirs = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m1 - m_new) * c);
+        l_run = l_run * mine + stats[64 + lane] * theirs;
+        collect(left, lane, o, mine, theirs);
+        m_ref = m_new;
+        out = reinterpret_cast<half_t*>(left);
+    }
+    const float l_tot = l_run + __shfl_xor(l_run, 32);
+    store_rows<P, RAGGED>(a.o, h, b, qb * QB + (piece + w) * 32, a.J, lane, o, 1.0f / l_tot, out, nullptr);
     if (mine_ && hi == 0) a.lse[row] = m_ref * c + __builtin_amdgcn_logf(l_tot);
+}
+template <int P, bool MASKED, bool RAGGED>
+__global__ __launch_bounds__(256) void k_mha_fwd(AttnArgs a, PhiloxKey key_) {
+    mha_fwd<P, MASKED, RAGGED, 1>(a, key_);
+}
+template <int P, bool MASKED, bool RAGGED>
+__global__ __launch_bounds__(256) void k_mha_fwd_halves(AttnArgs a, PhiloxKey key_) {
+    mha_fwd<P, MASKED, RAGGED, 2>(a, key_);
 }
 
 // ---------------------------------------------------------------------------
 // backward, dQ.  grid = H * B * ceil(J / 128); wave = 32 queries.
 // ---------------------------------------------------------------------------
-template <int P, bool MASKED, bool RAGGED>
-__global__ __launch_bounds__(256, !MASKED ? (P == 128 ? 2 : 3) : 1) void k_mha_bwd_dq(AttnArgs a) {
+template <int P, bool MASKED, bool RAGGED, int PARTS>
+__device__ __forceinline__ void mha_bwd_dq(const AttnArgs& a) {
     using G = Geo<P>;
     // Head size 128: with the key and value fragments of a whole tile in registers a tile ahead the kernel
     // needs 300 registers per lane and runs one wave per SIMD; read two k-slices ahead of their use instead,
     // it fits 256 and two waves share a SIMD.
     constexpr bool JIT = !MASKED;
-    __shared__ __attribute__((aligned(16))) half_t kt[RING][G::TILE];
-    __shared__ __attribute__((aligned(16))) half_t vt[RING][G::TILE];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, hi = lane >> 5;
+    __shared__ __attribute__((aligned(16))) half_t kt_[PARTS][RING][G::TILE];
+    __shared__ __attribute__((aligned(16))) half_t vt_[PARTS][RING][G::TILE];
+    const Place<PARTS> at;
+    const int tid = at.tid, lane = at.lane, wave = at.wave, l32 = lane & 31, hi = lane >> 5;
+    half_t (*const kt)[G::TILE] = kt_[at.half];
+    half_t (*const vt)[G::TILE] = vt_[at.half];
     const unsigned qblocks = RAGGED ? (a.J + QB - 1) / QB : a.J / QB;
-    const unsigned lb = logical_block();
+    const unsigned lb = logical_block() / PARTS;
     const unsigned nt = RAGGED ? (a.K + 31) / 32 : a.K / 32, pitch = RAGGED ? keep_pitch(a.K) : nt;
     unsigned qb = lb % qblocks, hb = lb / qblocks;
     if (MASKED) masked_order(a.qlist, qblocks, nt, a.H * a.B, lb, qb, hb);
     const unsigned b = hb % a.B, h = hb / a.B;
-    const unsigned j_ = qb * QB + wave * 32 + l32;
+    const int piece = PARTS > 1 ? (int)(logical_block() % PARTS) * Place<PARTS>::WAVES : 0;      // its first wave's, of the block's four
+    const unsigned j_ = qb * QB + (piece + wave) * 32 + l32;
     const bool mine_ = !RAGGED || j_ < (unsigned)a.J;
     const unsigned j = RAGGED ? min(j_, (unsigned)a.J - 1) : j_;
-    const bool working = !RAGGED || __builtin_amdgcn_readfirstlane((int)(qb * QB + wave * 32)) < a.J;
+    const bool working = !RAGGED || __builtin_amdgcn_readfirstlane((int)(qb * QB + (piece + wave) * 32)) < a.J;
     const unsigned row = (h * a.B + b) * a.J + j;
     const float c = a.alpha * LOG2E;
     const uint32_t* live = (MASKED && a.qlist) ? a.qlist + (size_t)qb * (nt + kListPad) : nullptr;
-    const unsigned n = live ? live[0] : nt;
-    uint32_t e0 = live_entry<MASKED>(live, 0), e1 = live_entry<MASKED>(live, 1), e2 = live_entry<MASKED>(live, 2);
+    const unsigned all = live ? live[0] : nt, longest = (all + PARTS - 1) / PARTS;
+    // (the second half's begin behind the first's; of an odd number it has one less)
+    const unsigned begin = at.half ? longest : 0, n = at.half ? all - longest : longest;
+    uint32_t e0 = live_entry<MASKED>(live, begin), e1 = live_entry<MASKED>(live, begin + 1), e2 = live_entry<MASKED>(live, begin + 2);
 
-    h8 fq[G::NKS], fdo[G::NKS], fk[G::NKS], fv[G::NKS], kr[G::VL], vr[G::VL];
+    h8 fq[G::NKS], fdo[G::NKS], fk[G::NKS], fv[G::NKS], kr[G::VL * PARTS], vr[G::VL * PARTS];
     float dsum, lse;
     uint32_t word;
-    Tiles<P, !MASKED && !RAGGED, RAGGED> tiles_k(a.k, h, b, tid), tiles_v(a.v, h, b, tid);
+    Tiles<P, !MASKED && !RAGGED, RAGGED, PARTS> tiles_k(a.k, h, b, begin, tid), tiles_v(a.v, h, b, begin, tid);
     {   // the first two tiles, the rows of this lane's query and its statistics: all
         // loads in flight together
-        h8 kr1[G::VL], vr1[G::VL], fo[G::NKS];
+        h8 kr1[G::VL * PARTS], vr1[G::VL * PARTS], fo[G::NKS];
         tiles_k.fetch(a.k, h, b, entry_tile(e0), a.K, tid, kr);
         tiles_v.fetch(a.v, h, b, entry_tile(e0), a.K, tid, vr);
         tiles_k.fetch(a.k, h, b, entry_tile(e1), a.K, tid, kr1);
@@ -595,17 +676,17 @@ __global__ __launch_bounds__(256, !MASKED ? (P == 128 ? 2 : 3) : 1) void k_mha_b
         row_frags<P>(a.o, h, b, j, hi, fo);
         lse = a.lse[row];
         word = a.keep[(size_t)row * pitch + entry_tile(e0)];
-        tile_put<P>(kt[0], tid, kr);
-        tile_put<P>(vt[0], tid, vr);
-        tile_put<P>(kt[1], tid, kr1);
-        tile_put<P>(vt[1], tid, vr1);
+        tile_put<P, PARTS>(kt[0], tid, kr);
+        tile_put<P, PARTS>(vt[0], tid, vr);
+        tile_put<P, PARTS>(kt[1], tid, kr1);
+        tile_put<P, PARTS>(vt[1], tid, vr1);
         float part = 0.f;
 #pragma unroll
         for (int ks = 0; ks < G::NKS; ++ks)
 #pragma unroll
             for (int i = 0; i < 8; ++i) part += (float)fdo[ks][i] * (float)fo[ks][i];
         dsum = part + __shfl_xor(part, 32);
-        if (hi == 0 && mine_) a.dsum[row] = dsum;
+        if (hi == 0 && mine_ && !at.half) a.dsum[row] = dsum;
     }
     __syncthreads();
     if constexpr (!JIT) {
@@ -620,24 +701,24 @@ __global__ __launch_bounds__(256, !MASKED ? (P == 128 ? 2 : 3) : 1) void k_mha_b
         for (int v = 0; v < 16; ++v) dq[pt][v] = 0.f;
     int cur = 0, nxt = 1, nn = 2;
     MaskRegs mk = {};
-    if (MASKED && n > 0 && entry_class(e0, wave) != BLOCK_CLEAR) load_mask<true, RAGGED>(a, j, entry_tile(e0) * 32, hi, mk);
+    if (MASKED && n > 0 && entry_class(e0, piece + wave) != BLOCK_CLEAR) load_mask<true, RAGGED>(a, j, entry_tile(e0) * 32, hi, mk);
     wait_loads();
 
-    for (unsigned i = 0; i < n; ++i) {
-        const uint32_t e3 = live_entry<MASKED>(live, i + 3);
-        const bool from_mask = MASKED && entry_class(e0, wave) != BLOCK_CLEAR;
+    for (unsigned i = 0; i < longest; ++i) {
+        const uint32_t e3 = live_entry<MASKED>(live, begin + i + 3);
+        const bool from_mask = MASKED && entry_class(e0, piece + wave) != BLOCK_CLEAR;
         const bool fetch = i + 2 < n;
         if (fetch) {
             tiles_k.fetch(a.k, h, b, entry_tile(e2), a.K, tid, kr);
             tiles_v.fetch(a.v, h, b, entry_tile(e2), a.K, tid, vr);
         }
         const uint32_t wordn = i + 1 < n ? a.keep[(size_t)row * pitch + entry_tile(e1)] : 0u;
-        if (working) {
+        if (working && (PARTS == 1 || i < n)) {
         f16v s, dp;
 #pragma unroll
         for (int v = 0; v < 16; ++v) { s[v] = 0.f; dp[v] = 0.f; }
         if (from_mask) start_from_mask(mk, s);
-        if (MASKED && i + 1 < n && entry_class(e1, wave) != BLOCK_CLEAR) load_mask<true, RAGGED>(a, j, entry_tile(e1) * 32, hi, mk);
+        if (MASKED && i + 1 < n && entry_class(e1, piece + wave) != BLOCK_CLEAR) load_mask<true, RAGGED>(a, j, entry_tile(e1) * 32, hi, mk);
         if constexpr (JIT) {
             h8 ck[2], cv[2];
             ck[0] = *reinterpret_cast<const h8*>(kt[cur] + G::at(l32, hi));
@@ -690,21 +771,41 @@ __global__ __launch_bounds__(256, !MASKED ? (P == 128 ? 2 : 3) : 1) void k_mha_b
                 dq[pt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka[st][pt], ds[st], dq[pt], 0, 0, 0);
         }
         if (fetch) {
-            tile_put<P>(kt[nn], tid, kr);
-            tile_put<P>(vt[nn], tid, vr);
+            tile_put<P, PARTS>(kt[nn], tid, kr);
+            tile_put<P, PARTS>(vt[nn], tid, vr);
         }
         word = wordn;
         __syncthreads();
         const int x = cur; cur = nxt; nxt = nn; nn = x;
         e0 = e1; e1 = e2; e2 = e3;
     }
-    float* const sums = a.bias_q ? reinterpret_cast<float*>(kt[2]) : nullptr;       // (of 4 waves 64 * P bytes, a tile's)
     const int w = __builtin_amdgcn_readfirstlane(wave);
-    store_rows<P, RAGGED>(a.dq, h, b, qb * QB + w * 32, a.J, lane, dq, a.alpha, w < 2 ? kt[w] : vt[w - 2],
-                          sums ? sums + w * 4 * P : nullptr);
+    half_t* out = w < 2 ? kt[w] : vt[w - 2];
+    float* const sums = a.bias_q ? reinterpret_cast<float*>(PARTS > 1 ? vt_[0][2] : kt_[0][2]) : nullptr;       // (of 4 waves 64 * P bytes, a tile's)
+    if constexpr (PARTS > 1) {
+        // (the tiles' places are free)
+        static_assert(Place<PARTS>::WAVES * G::NPT * 16 * 64 * sizeof(float) <= sizeof(kt_), "two waves' accumulators");
+        float* const left = reinterpret_cast<float*>(kt_) + w * (G::NPT * 16 * 64);
+        if (at.half) leave(left, lane, dq);
+        __syncthreads();
+        if (!at.half) collect(left, lane, dq, 1.f, 1.f);
+        out = reinterpret_cast<half_t*>(left);
+    }
+    if (!at.half)
+        store_rows<P, RAGGED>(a.dq, h, b, qb * QB + (piece + w) * 32, a.J, lane, dq, a.alpha, out,
+                              sums ? sums + w * 4 * P : nullptr);
     if (!sums) return;
     __syncthreads();
-    if (tid < P) a.bias_q[((size_t)h * (a.B * qblocks) + b * qblocks + qb) * P + tid] = column_sum<P>(sums, tid);
+    const unsigned part = (b * qblocks + qb) * PARTS + piece / Place<PARTS>::WAVES;
+    if (threadIdx.x < P) a.bias_q[((size_t)h * (a.B * qblocks * PARTS) + part) * P + threadIdx.x] = column_sum<P, Place<PARTS>::WAVES>(sums, threadIdx.x);
+}
+template <int P, bool MASKED, bool RAGGED>
+__global__ __launch_bounds__(256, !MASKED ? (P == 128 ? 2 : 3) : 1) void k_mha_bwd_dq(AttnArgs a) {
+    mha_bwd_dq<P, MASKED, RAGGED, 1>(a);
+}
+template <int P, bool MASKED, bool RAGGED>
+__global__ __launch_bounds__(256) void k_mha_bwd_dq_halves(AttnArgs a) {
+    mha_bwd_dq<P, MASKED, RAGGED, 2>(a);
 }
 
 // ---------------------------------------------------------------------------
@@ -743,8 +844,8 @@ __device__ __forceinline__ void settle(f16v (&acc)[N]) {
     for (int i = 0; i < N; ++i) asm volatile("" : "+a"(acc[i]));
 }
 
-template <int P, bool MASKED, bool RAGGED>
-__global__ __launch_bounds__(256, (P == 64 && MASKED) ? 2 : 1) void k_mha_bwd_dkv(AttnArgs a) {
+template <int P, bool MASKED, bool RAGGED, int PARTS>
+__device__ __forceinline__ void mha_bwd_dkv(const AttnArgs& a) {
     using G = Geo<P>;
     // Head size 128 has one wave per SIMD, in which the vector work on a tile and the products around it wait for one another
     // (4400 cycles a tile, of which the matrix pipe works 1024).  There the scores of a tile are formed during the vector
@@ -755,10 +856,15 @@ __global__ __launch_bounds__(256, (P == 64 && MASKED) ? 2 : 1) void k_mha_bwd_dk
     // five ahead: 787 us.  With a mask the tiles are taken from a list and begin from mask values: as for head size 64,
     // where two waves per SIMD fill each other's gaps.)
     constexpr bool AHEAD = P == 128 && !MASKED;
-    __shared__ __attribute__((aligned(16))) KvStage<P> stage[AHEAD ? 4 : RING];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, hi = lane >> 5;
+    static_assert(PARTS == 1 || P == 64, "head size 128 has the registers of a whole SIMD");
+    __shared__ __attribute__((aligned(16))) KvStage<P> stage_[PARTS][AHEAD ? 4 : RING];
+    const Place<PARTS> at;
+    const int tid = at.tid, lane = at.lane, l32 = lane & 31, hi = lane >> 5;
+    const int piece = PARTS > 1 ? (int)(logical_block() % PARTS) * Place<PARTS>::WAVES : 0;      // its first wave's, of the block's four
+    const int wave = piece + at.wave;                                // (of the block)
+    KvStage<P>* const stage = stage_[at.half];
     const unsigned kblocks = RAGGED ? (a.K + QB - 1) / QB : a.K / QB;
-    const unsigned lb = logical_block();
+    const unsigned lb = logical_block() / PARTS;
     const unsigned nq = RAGGED ? (a.J + 31) / 32 : a.J / 32, nkt = RAGGED ? keep_pitch(a.K) : a.K / 32;
     unsigned kb = lb % kblocks, hb = lb / kblocks;
     if (MASKED) masked_order(a.klist, kblocks, nq, a.H * a.B, lb, kb, hb);
@@ -770,16 +876,17 @@ __global__ __launch_bounds__(256, (P == 64 && MASKED) ? 2 : 1) void k_mha_bwd_dk
     const float c = a.alpha * LOG2E;
     // the query tiles to walk: all of them, or those a mask leaves for these 128 keys
     const uint32_t* live = (MASKED && a.klist) ? a.klist + (size_t)kb * (nq + kListPad) : nullptr;
-    const unsigned n = live ? live[0] : nq;
-    uint32_t e0 = live_entry<MASKED>(live, 0), e1 = live_entry<MASKED>(live, 1), e2 = live_entry<MASKED>(live, 2);
+    const unsigned all = live ? live[0] : nq, longest = (all + PARTS - 1) / PARTS;
+    const unsigned begin = at.half ? longest : 0, n = at.half ? all - longest : longest;
+    uint32_t e0 = live_entry<MASKED>(live, begin), e1 = live_entry<MASKED>(live, begin + 1), e2 = live_entry<MASKED>(live, begin + 2);
 
     h8 fk[G::NKS], fv[G::NKS], fq[G::NKS], fdo[G::NKS];
     struct InFlight {             // one tile of queries on its way from memory
-        h8 q[G::VL], d_o[G::VL];
+        h8 q[G::VL * PARTS], d_o[G::VL * PARTS];
         float stat;
         uint4 kw;
     };
-    Tiles<P, !MASKED && !RAGGED, RAGGED> tiles_q(a.q, h, b, tid), tiles_do(a.d_o, h, b, tid);
+    Tiles<P, !MASKED && !RAGGED, RAGGED, PARTS> tiles_q(a.q, h, b, begin, tid), tiles_do(a.d_o, h, b, begin, tid);
     auto fetch = [&](unsigned qt, InFlight& f) {
         tiles_q.fetch(a.q, h, b, qt, a.J, tid, f.q);
         tiles_do.fetch(a.d_o, h, b, qt, a.J, tid, f.d_o);
@@ -791,8 +898,8 @@ __global__ __launch_bounds__(256, (P == 64 && MASKED) ? 2 : 1) void k_mha_bwd_dk
         else if (tid < 96) f.kw = *reinterpret_cast<const uint4*>(a.keep + (size_t)r * nkt + kb * 4);
     };
     auto put = [&](KvStage<P>& sg, const InFlight& f) {
-        tile_put<P>(sg.q, tid, f.q);
-        tile_put<P>(sg.d_o, tid, f.d_o);
+        tile_put<P, PARTS>(sg.q, tid, f.q);
+        tile_put<P, PARTS>(sg.d_o, tid, f.d_o);
         if (tid < 32) sg.lse[tid] = f.stat;
         else if (tid < 64) sg.dsum[tid - 32] = f.stat;
         else if (tid < 96) {
@@ -968,13 +1075,13 @@ __global__ __launch_bounds__(256, (P == 64 && MASKED) ? 2 : 1) void k_mha_bwd_dk
     if (MASKED && n > 0 && entry_class(e0, wave) != BLOCK_CLEAR) load_mask<false, RAGGED>(a, kpos, entry_tile(e0) * 32, hi, mk);
     wait_loads();
 
-    for (unsigned i = 0; i < n; ++i) {
-        const uint32_t e3 = live_entry<MASKED>(live, i + 3);
+    for (unsigned i = 0; i < longest; ++i) {
+        const uint32_t e3 = live_entry<MASKED>(live, begin + i + 3);
         const bool from_mask = MASKED && entry_class(e0, wave) != BLOCK_CLEAR;
         const bool more = i + 2 < n;
         if (more) fetch(entry_tile(e2), fl);
         const KvStage<P>& sg = stage[cur];
-        if (working) {
+        if (working && (PARTS == 1 || i < n)) {
         f16v s, dp;
 #pragma unroll
         for (int v = 0; v < 16; ++v) { s[v] = 0.f; dp[v] = 0.f; }
@@ -1026,16 +1133,40 @@ __global__ __launch_bounds__(256, (P == 64 && MASKED) ? 2 : 1) void k_mha_bwd_dk
         e0 = e1; e1 = e2; e2 = e3;
     }
     }
-    const int w = __builtin_amdgcn_readfirstlane(wave);
-    half_t* const tile = w < 2 ? stage[w].q : stage[w - 2].d_o;
-    float* const sums_k = reinterpret_cast<float*>(stage[2].q);         // (of 4 waves 64 * P bytes, a tile's)
-    float* const sums_v = reinterpret_cast<float*>(stage[2].d_o);
-    store_rows<P, RAGGED>(a.dk, h, b, kb * QB + w * 32, a.K, lane, dk, a.alpha, tile, a.bias_kv ? sums_k + w * 4 * P : nullptr);
-    store_rows<P, RAGGED>(a.dv, h, b, kb * QB + w * 32, a.K, lane, dv, 1.0f, tile, a.bias_kv ? sums_v + w * 4 * P : nullptr);
+    const int w = __builtin_amdgcn_readfirstlane(at.wave);
+    half_t* tile = w < 2 ? stage[w].q : stage[w - 2].d_o;
+    float *sums_k = reinterpret_cast<float*>(stage_[0][2].q), *sums_v = reinterpret_cast<float*>(stage_[0][2].d_o);   // (of 4 waves 64 * P bytes, a tile's)
+    if constexpr (PARTS > 1) {
+        // (all stages are free: what the second half leaves lies from the first on, a wave's rows go out by way of its own place
+        // there, and the sums lie behind)
+        constexpr int LEFT = 2 * G::NPT * 16 * 64;
+        static_assert((2 * LEFT + 2 * 16 * P) * sizeof(float) <= sizeof(stage_), "two waves' accumulators and sums");
+        float* const first = reinterpret_cast<float*>(&stage_[0][0]);
+        float* const left = first + w * LEFT;
+        if (at.half) { leave(left, lane, dk); leave(left + LEFT / 2, lane, dv); }
+        __syncthreads();
+        if (!at.half) { collect(left, lane, dk, 1.f, 1.f); collect(left + LEFT / 2, lane, dv, 1.f, 1.f); }
+        tile = reinterpret_cast<half_t*>(left);
+        sums_k = first + 2 * LEFT;
+        sums_v = sums_k + 16 * P;
+    }
+    if (!at.half) {
+        store_rows<P, RAGGED>(a.dk, h, b, kb * QB + (piece + w) * 32, a.K, lane, dk, a.alpha, tile, a.bias_kv ? sums_k + w * 4 * P : nullptr);
+        store_rows<P, RAGGED>(a.dv, h, b, kb * QB + (piece + w) * 32, a.K, lane, dv, 1.0f, tile, a.bias_kv ? sums_v + w * 4 * P : nullptr);
+    }
     if (!a.bias_kv) return;
     __syncthreads();
-    const size_t ntc = (size_t)a.B * kblocks, part = (size_t)h * ntc + b * kblocks + kb;
-    if (tid < 2 * P) a.bias_kv[((tid < P ? 0 : (size_t)a.H * ntc) + part) * P + tid % P] = column_sum<P>(tid < P ? sums_k : sums_v, tid % P);
+    const size_t ntc = (size_t)a.B * kblocks * PARTS, part = (size_t)h * ntc + (b * kblocks + kb) * PARTS + piece / Place<PARTS>::WAVES;
+    const int to = threadIdx.x;
+    if (to < 2 * P) a.bias_kv[((to < P ? 0 : (size_t)a.H * ntc) + part) * P + to % P] = column_sum<P, Place<PARTS>::WAVES>(to < P ? sums_k : sums_v, to % P);
+}
+template <int P, bool MASKED, bool RAGGED>
+__global__ __launch_bounds__(256, (P == 64 && MASKED) ? 2 : 1) void k_mha_bwd_dkv(AttnArgs a) {
+    mha_bwd_dkv<P, MASKED, RAGGED, 1>(a);
+}
+template <int P, bool MASKED, bool RAGGED>
+__global__ __launch_bounds__(256) void k_mha_bwd_dkv_halves(AttnArgs a) {
+    mha_bwd_dkv<P, MASKED, RAGGED, 2>(a);
 }
 
 // Whether the kernels have to watch the ends of the sequences.
@@ -1111,12 +1242,30 @@ void for_variant(int P, const AttnArgs& a, Fn&& fn) {
     if (P == 64) msk(std::integral_constant<int, 64>{});
     else msk(std::integral_constant<int, 128>{});
 }
+
+// A lone wave already keeps its SIMD issuing (1400 cycles a tile, 284 vector instructions), so that the halves give nothing where
+// every CU has a workgroup: they are for launches that leave half of the CUs without one.  us of forward, dQ, and dK and dV with whole
+// blocks and with halves, H 12, P 64: 1 x 1024 (96 blocks) 30.9, 24.0, 31.2 and 21.2, 17.4, 21.6, causal 36.6, 30.6, 41.0 and 24.7, 19.8,
+// 25.1; 4 x 256 causal (96) 13.3, 12.4, 15.1 and 10.3, 9.7, 11.7; 3 x 300 (108) 13.6, 11.8, 15.9 and 10.3, 9.7, 11.8; 8 x 128 (96) 7.0, 7.4,
+// 8.2 and 6.5, 7.1, 7.4.  Beyond: 8 x 256 on 512, H 16 (256) no difference, 13 x 201 (312) 15.0, 14.4, 16.4 and 17.4, 15.5, 20.2.
+// (One workgroup on a CU then: the kernels of halves may take the registers of a whole SIMD.)
+int parts(const AttnArgs& a, int P, long rows, long others) {
+    return P == 64 && a.H * (long)a.B * blocks(rows) <= kFewBlocks && tiles(others) >= 4 ? 2 : 1;
+}
 }  // namespace
 
-void launch_mha_forward(const AttnArgs& a, int P, PhiloxKey key, hipStream_t st) {
+long mha_bias_rows_q(const AttnArgs& a, int P) { return a.B * blocks(a.J) * parts(a, P, a.J, a.K); }
+long mha_bias_rows_kv(const AttnArgs& a, int P) { return a.B * blocks(a.K) * parts(a, P, a.K, a.J); }
+size_t mha_bias_floats(long H, long B, long J, long K, long P) { return (size_t)(2 * H * P * B * (blocks(J) + 2 * blocks(K))); }
+
+void launch_mha_forward(const AttnArgs& a, int P, PhiloxKey key, bool same_order, hipStream_t st) {
     if (!mha_forward_ok(a, P)) fail("attention forward: shape, strides or alignment not supported");
-    dim3 grid((unsigned)(a.H * a.B * blocks(a.J)));
+    const int n = same_order ? 1 : parts(a, P, a.J, a.K);
+    dim3 grid((unsigned)(a.H * a.B * blocks(a.J) * n));
     for_variant(P, a, [&](auto p, auto masked, auto rag) {
+        if constexpr (p() == 64) {
+            if (n == 2) { hipLaunchKernelGGL((k_mha_fwd_halves<p(), masked(), rag()>), grid, dim3(256), 0, st, a, key); return; }
+        }
         hipLaunchKernelGGL((k_mha_fwd<p(), masked(), rag()>), grid, dim3(256), 0, st, a, key);
     });
     check_launch("attention forward");
@@ -1128,8 +1277,12 @@ bool mha_backward_ok(const AttnArgs& a, int P) {
 
 void launch_mha_backward_dq(const AttnArgs& a, int P, hipStream_t st) {
     if (!mha_backward_ok(a, P)) fail("attention backward: shape, strides or alignment not supported");
-    dim3 grid((unsigned)(a.H * a.B * blocks(a.J)));
+    const int n = parts(a, P, a.J, a.K);
+    dim3 grid((unsigned)(a.H * a.B * blocks(a.J) * n));
     for_variant(P, a, [&](auto p, auto masked, auto rag) {
+        if constexpr (p() == 64) {
+            if (n == 2) { hipLaunchKernelGGL((k_mha_bwd_dq_halves<p(), masked(), rag()>), grid, dim3(256), 0, st, a); return; }
+        }
         hipLaunchKernelGGL((k_mha_bwd_dq<p(), masked(), rag()>), grid, dim3(256), 0, st, a);
     });
     check_launch("attention backward (dQ)");
@@ -1137,8 +1290,12 @@ void launch_mha_backward_dq(const AttnArgs& a, int P, hipStream_t st) {
 
 void launch_mha_backward_dkv(const AttnArgs& a, int P, hipStream_t st) {
     if (!mha_backward_ok(a, P)) fail("attention backward: shape, strides or alignment not supported");
-    dim3 grid((unsigned)(a.H * a.B * blocks(a.K)));
+    const int n = parts(a, P, a.K, a.J);
+    dim3 grid((unsigned)(a.H * a.B * blocks(a.K) * n));
     for_variant(P, a, [&](auto p, auto masked, auto rag) {
+        if constexpr (p() == 64) {
+            if (n == 2) { hipLaunchKernelGGL((k_mha_bwd_dkv_halves<p(), masked(), rag()>), grid, dim3(256), 0, st, a); return; }
+        }
         hipLaunchKernelGGL((k_mha_bwd_dkv<p(), masked(), rag()>), grid, dim3(256), 0, st, a);
     });
     check_launch("attention backward (dK, dV)");

@@ -177,8 +177,8 @@ struct AttnArgs {
     int H = 0, B = 0, J = 0, K = 0;
     float alpha = 1.f;         // score scale
     // optional (backward): per-workgroup sums over positions of the rounded dq resp.
-    // dk, dv rows, for the gradient of the projection biases.  bias_q: [H][B*ceil(J/128)][P]
-    // floats, bias_kv: [2][H][B*ceil(K/128)][P] (dk, then dv).
+    // dk, dv rows, for the gradient of the projection biases.  bias_q: [H][mha_bias_rows_q][P]
+    // floats, bias_kv: [2][H][mha_bias_rows_kv][P] (dk, then dv).
     float* bias_q = nullptr;
     float* bias_kv = nullptr;
     const half_t* amask = nullptr;   // optional additive mask over (query, key), added before the scaling
@@ -198,12 +198,18 @@ size_t mha_stat_bytes(long H, long B, long J);          // lse followed by dsum
 size_t mha_keep_bytes(long H, long B, long J, long K);
 bool mha_forward_ok(const AttnArgs& a, int head_size);
 bool mha_backward_ok(const AttnArgs& a, int head_size);
-void launch_mha_forward(const AttnArgs& a, int head_size, PhiloxKey key, hipStream_t st);
+// same_order: in front of a ReLU, where another order of the sums moves gates
+void launch_mha_forward(const AttnArgs& a, int head_size, PhiloxKey key, bool same_order, hipStream_t st);
 // skip[J/32][K/32] = 1 where mask[j][k] is -inf for every (j, k) of the block
 // Device bytes of the plan of a [J, K] mask, and the launches that fill it (rebuild)
 // and point the arguments at it.
 size_t mha_mask_plan_bytes(long J, long K);
 void launch_mha_mask_plan(AttnArgs& a, void* plan, bool rebuild, hipStream_t st);
+// Partial rows of P floats that the backward launches leave in bias_q and, for each of dK and dV, in bias_kv, per head; what both take
+// together at most (floats).
+long mha_bias_rows_q(const AttnArgs& a, int head_size);
+long mha_bias_rows_kv(const AttnArgs& a, int head_size);
+size_t mha_bias_floats(long H, long B, long J, long K, long P);
 void launch_mha_backward_dq(const AttnArgs& a, int head_size, hipStream_t st);
 void launch_mha_backward_dkv(const AttnArgs& a, int head_size, hipStream_t st);
 

@@ -6,6 +6,7 @@ device's fp32-internal arithmetic and one fp16 rounding per output: tolerance
 Dropout masks are compared bit-exactly with oracle/philox_ref.py."""
 import contextlib
 import itertools
+import math
 
 import numpy as np
 import pytest
@@ -392,6 +393,78 @@ def test_attention_operator_forward_and_backward(B, H, P, J, K, p, masked, l_q, 
     assert_close(from_layout(dq, 'BJHP', l_q), want_dq, name='dq')
     assert_close(from_layout(dk, 'BKHP', l_kv), want_dk, name='dk')
     assert_close(from_layout(dv, 'BKHP', l_kv), want_dv, name='dv')
+
+
+@pytest.mark.parametrize('J,K', [(128, 128), (256, 128), (128, 384), (512, 512), (384, 1024)])
+@pytest.mark.parametrize('p,mask', [(0.1, None), (0.25, 'causal'), (0.0, 'holes')])
+def test_attention_by_halves_of_the_other_side_equals_the_whole(J, K, p, mask):
+    """Where there are few blocks of 128 positions two waves share a block's other side (4 to 32 tiles of it here).  Forward against the handle of a ReLU layer, which never does: the same keep bits, outputs and
+    log-sum-exps equal but for the order of the sums (fp32, rounded to fp16 once: 2 ** -10 of a row's largest).  Backward, without
+    dropout, against the same samples among so many that a block has its four waves: the gradients, fp16 products of fp16 values
+    summed in another order (2 ** -9 of a tensor's largest)."""
+    from substation_amd.ops import Ops
+    B, H, P = 2, 2, 64
+    g = torch.Generator(device='cuda').manual_seed(J + K)
+    many = 40                                                # samples: more than 128 blocks
+    full = lambda n: torch.randn((many, n, H, P), generator=g, device='cuda').half()
+    q, k, v, d_out = full(J), full(K), full(K), full(J)
+    am = None
+    if mask:
+        am = torch.zeros(J, K, dtype=torch.float16, device='cuda')
+        if mask == 'causal':
+            am[torch.ones(J, K, device='cuda').triu(1).bool()] = -math.inf
+        else:                                                # whole tiles of keys gone for some queries, one row of queries sees one key
+            am[:J // 2, 32:] = -math.inf
+            am[J // 2:, :64] = -math.inf
+            am[J - 1, :K - 1] = -math.inf
+
+    def run(n, act, prob):
+        o = Ops(n, 128, H, H * P, activation=act, seed=SEED)
+        rows = H * n * J
+        stats = torch.empty(2 * rows, dtype=torch.float32, device='cuda')
+        keep = torch.zeros(rows * ((K + 127) // 128 * 4), dtype=torch.int32, device='cuda')
+        out, dq, dk, dv = (torch.empty_like(t[:n]) for t in (q, q, k, v))
+        o.attention_forward(q[:n], 'BJHP', k[:n], v[:n], 'BKHP', out, 'BJHP', stats, keep, 0.125, p=prob, site=ph.SITE_SOFTMAX,
+                            attn_mask=am)
+        lse = stats[:rows].clone()
+        o.attention_backward(q[:n], 'BJHP', k[:n], v[:n], 'BKHP', out, 'BJHP', d_out[:n], 'BJHP', stats, keep, dq, 'BJHP', dk, dv, 'BKHP',
+                             0.125, attn_mask=am)
+        torch.cuda.synchronize()
+        return out, lse, keep, dq, dk, dv
+
+    halves, whole = run(B, 'gelu', p), run(B, 'relu', p)
+    assert torch.equal(halves[2], whole[2])
+    close = lambda a, b, tol: float((a.float() - b.float()).abs().max()) <= tol * float(b.float().abs().max())
+    assert close(halves[0], whole[0], 2 ** -10) and close(halves[1], whole[1], 2 ** -18)
+    few, among = run(B, 'gelu', 0.0), run(many, 'gelu', 0.0)
+    for a, b in zip((few[0],) + few[3:], (among[0],) + among[3:]):
+        assert bool(torch.isfinite(a).all()) and close(a, b[:B], 2 ** -9)
+
+
+@pytest.mark.parametrize('L', [97, 130, 160, 201, 333])
+@pytest.mark.parametrize('causal', [False, True])
+def test_attention_by_halves_at_any_length(L, causal):
+    """4, 5, 7 and 11 tiles with an end inside, 0 to 4 of them in the list of a mask: a layer's two samples alone (few blocks) and in
+    front of 68 others, without dropout.  The outputs pass through the same operators and sums in another order: a fraction of the
+    1e-2 that parity allows."""
+    from substation_amd import Encoder, causal_mask, mi355x_layouts
+    many, few, H, E = 70, 2, 2, 128
+    g = torch.Generator(device='cuda').manual_seed(L)
+    x = torch.randn(many, L, E, generator=g, device='cuda').half()
+    dy = torch.randn(many, L, E, generator=g, device='cuda').half()
+    got = []
+    for n in (few, many):
+        torch.manual_seed(5)
+        enc = Encoder('unused', n, L, H, E, mi355x_layouts(), torch.float16, 0.0, 0.0, 0.0, 0.0, activation='gelu', seed=SEED).cuda()
+        if causal:
+            enc.set_attention_mask(causal_mask(L))
+        X = x[:n].clone().requires_grad_(True)
+        y = enc(X)
+        y.backward(dy[:n])
+        torch.cuda.synchronize()
+        got.append((y.detach()[:few].float(), X.grad[:few].float()))
+    for a, b in zip(*got):
+        assert float((a - b).norm()) <= 3e-3 * float(b.norm())
 
 
 # (1000, 776: rows that end inside a lane's second pack; 5000 rows of 64: more rows than the launch has waves;
