@@ -25,79 +25,136 @@ namespace sub {
 namespace {
 
 // ---------------------------------------------------------------------------
-// Any strides, any sizes: what the matrix-core kernels do not take (mostly rows that are not whole 16-byte words: the
-// score-sized products of sequence lengths that are not multiples of 8).  64 x 64 outputs per workgroup, 4 x 4 per
-// thread, operands converted into LDS 32 k at a time; every output is one fp32 chain of fused multiply-adds in the
-// order of k.  (One thread per output, straight from memory, before: 750 us for the scores of B=8 L=197 H=12, 0.5 GFLOP,
-// bound by the latency of that chain's single-element loads.)
+// Any strides, any sizes: what the half-precision matrix instructions do not take (mostly rows that are not whole 16-byte words: the
+// score-sized products of sequence lengths that are not multiples of 8).  128 x 64 outputs per workgroup, 32 x 64 per wave, 32 k of
+// both operands in LDS at a time, the next 32 on their way meanwhile.  Every output is one fp32 chain of fused multiply-adds in the
+// order of k, which is what v_mfma_f32_32x32x2_f32 does with its two k (204800 sums of 256 compared with fmaf, bit for bit; k past the
+// end are zeros in both operands, which leave a sum as it is).  With v_fma_f32, 4 x 4 outputs per thread, the same bits took half the
+// rate at best, and eight times the reads from LDS.  us of the scores and of the product with V, before and now, H 12, P 64: 13 x 201
+// 41 and 52, 24 and 30; 24 x 77 21 and 23, 14 and 15; 3 x 300 22 and 67, 15 and 30; 2 x 1500, H 16: 215 and 321, 109 and 172 (a third
+// of that instruction's rate: the single elements of a row that starts anywhere).
 // ---------------------------------------------------------------------------
-constexpr int FB = 64, FK = 32, FPITCH = FB + 4;
+constexpr int FM = 128, FN = 64, FK = 32, FPITCH = FK + 8;
+typedef float f16v __attribute__((ext_vector_type(16)));
+enum : int { FMA_SINGLE = 0, FMA_ALONG_K = 1, FMA_ALONG_ROWS = 2 };       // how an operand is read: whole 16-byte words or not
 
-// One operand's 64 x 32 elements into LDS as [k][row].  vec: whole 16-byte words along k.
-__device__ __forceinline__ void fma_tile(float (*dst)[FPITCH], const half_t* p, long s_row, long s_k, int rows, int ks, bool vec,
-                                         int tid) {
-    if (vec) {
-        const int row = tid >> 2, k = (tid & 3) * 8;
-        h8 v = (h8)(half_t)0.0f;
-        if (row < rows && k < ks) v = *reinterpret_cast<const h8*>(p + (long)row * s_row + k);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) dst[k + i][row] = (float)v[i];
-        return;
+// What a thread brings of an operand's ROWS x 32 elements: words, or elements that lie side by side over the threads along k or
+// along the rows.  What lies outside is read from a place that there is, and put down as zero where it is a k: no branch around a
+// load, where the wait for it would go.  Single elements are kept apart: of two in a register, the second's load waits for the first's.
+// In LDS [row][k], as half values: 16 bytes are four steps of a matrix instruction.
+template <int ROWS, int HOW>
+struct FmaPart {
+    static constexpr int N = ROWS * FK / 256, WORDS = N / 8, L = HOW == FMA_SINGLE ? N : WORDS;
+    int row, k, drow, dk;                    // of the first, and on to the next
+    h8 word[WORDS];
+    uint16_t one[N];
+    __device__ __forceinline__ FmaPart(bool k_first, int tid) {
+        if (HOW == FMA_ALONG_K) { row = tid >> 2; k = (tid & 3) * 8; drow = 64; dk = 0; }
+        else if (HOW == FMA_ALONG_ROWS) { row = tid % (ROWS / 8) * 8; k = tid / (ROWS / 8); drow = 0; dk = 256 / (ROWS / 8); }
+        else if (k_first) { row = tid / FK; k = tid % FK; drow = 256 / FK; dk = 0; }
+        else { row = tid % ROWS; k = tid / ROWS; drow = 0; dk = 256 / ROWS; }
     }
-    half_t v[8];
+    // (p: the step's first element, of which there are rows x ks.  Spelled out as memory that is not LDS.)
+    __device__ __forceinline__ void fetch(const half_t* p, long s_row, long s_k, int rows, int ks) {
+        const long first = row < rows && k < ks ? (long)row * s_row + (long)k * s_k : 0, step = (long)drow * s_row + (long)dk * s_k;
+        const __attribute__((address_space(1))) half_t* const q = (const __attribute__((address_space(1))) half_t*)p + first;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int e = tid + i * 256, row = s_k == 1 ? e / FK : e % FB, k = s_k == 1 ? e % FK : e / FB;
-        v[i] = row < rows && k < ks ? p[(long)row * s_row + (long)k * s_k] : (half_t)0.0f;
+        for (int i = 0; i < L; ++i) {
+            const bool in = row + i * drow < rows && k + i * dk < ks;
+            const auto at = q + (in ? i * step : 0);
+            if constexpr (HOW == FMA_SINGLE) one[i] = *(const __attribute__((address_space(1))) uint16_t*)at;
+            else word[i] = *(const __attribute__((address_space(1))) h8*)at;
+        }
     }
+    __device__ __forceinline__ void put(half_t (*to)[FPITCH], int ks) const {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int e = tid + i * 256, row = s_k == 1 ? e / FK : e % FB, k = s_k == 1 ? e % FK : e / FB;
-        dst[k][row] = (float)v[i];
+        for (int i = 0; i < L; ++i) {
+            const bool in = k + i * dk < ks;
+            if constexpr (HOW == FMA_SINGLE) to[row + i * drow][k + i * dk] = in ? __builtin_bit_cast(half_t, one[i]) : (half_t)0.0f;
+            else {
+                const h8 v = in ? word[i] : (h8)(half_t)0.0f;
+                if constexpr (HOW == FMA_ALONG_K) *reinterpret_cast<h8*>(&to[row + i * drow][k]) = v;
+                else
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) to[row + e][k + i * dk] = v[e];
+            }
+        }
     }
-}
+};
 
-__global__ __launch_bounds__(256) void k_gemm_fma(GemmArgs g, bool vec_a, bool vec_b) {
-    __shared__ __attribute__((aligned(16))) float ta[FK][FPITCH], tb[FK][FPITCH];
-    const int tid = threadIdx.x, tm = (tid >> 4) * 4, tn = (tid & 15) * 4;
-    const unsigned tiles_m = (g.M + FB - 1) / FB, tiles_n = (g.N + FB - 1) / FB;
+template <int HOW_A, int HOW_B>
+__global__ __launch_bounds__(256, 4) void k_gemm_fma(GemmArgs g) {
+    __shared__ __attribute__((aligned(16))) half_t ta[2][FM][FPITCH], tb[2][FN][FPITCH];
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hi = lane >> 5;
+    const int wm = __builtin_amdgcn_readfirstlane(tid >> 6) * 32;
+    const unsigned tiles_m = (g.M + FM - 1) / FM, tiles_n = (g.N + FN - 1) / FN;
     unsigned id = blockIdx.x;
-    const unsigned n0 = id % tiles_n * FB; id /= tiles_n;
-    const unsigned m0 = id % tiles_m * FB; id /= tiles_m;
+    const unsigned n0 = id % tiles_n * FN; id /= tiles_n;
+    const unsigned m0 = id % tiles_m * FM; id /= tiles_m;
     const long b2 = id % g.nb2; id /= g.nb2;
     const long b1 = id % g.nb1, b0 = id / g.nb1;
-    const half_t* a = g.A + b0 * g.sAb[0] + b1 * g.sAb[1] + b2 * g.sAb[2] + (long)m0 * g.sAM;
-    const half_t* b = g.B + b0 * g.sBb[0] + b1 * g.sBb[1] + b2 * g.sBb[2] + (long)n0 * g.sBN;
-    float acc[4][4] = {};
+    const half_t* const a = g.A + b0 * g.sAb[0] + b1 * g.sAb[1] + b2 * g.sAb[2] + (long)m0 * g.sAM;
+    const half_t* const b = g.B + b0 * g.sBb[0] + b1 * g.sBb[1] + b2 * g.sBb[2] + (long)n0 * g.sBN;
+    const int rows = min(g.M - (int)m0, FM), cols = min(g.N - (int)n0, FN);
+    FmaPart<FM, HOW_A> pa(g.sAK1 == 1, tid);
+    FmaPart<FN, HOW_B> pb(g.sBK1 == 1, tid);
+    const bool working = wm < rows;                          // (a wave whose outputs all lie outside only helps with the operands)
+    f16v acc[2];
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[0][v] = acc[1][v] = 0.f;
+    auto fetch = [&](int k0, int k) __attribute__((always_inline)) {
+        pa.fetch(a + (long)k0 * g.sAK0 + (long)k * g.sAK1, g.sAM, g.sAK1, rows, g.K1 - k);
+        pb.fetch(b + (long)k0 * g.sBK0 + (long)k * g.sBK1, g.sBN, g.sBK1, cols, g.K1 - k);
+    };
+    fetch(0, 0);
+    int buf = 0;
     for (int k0 = 0; k0 < g.K0; ++k0)
         for (int k = 0; k < g.K1; k += FK) {
             const int ks = min(FK, g.K1 - k);
-            __syncthreads();
-            fma_tile(ta, a + (long)k0 * g.sAK0 + (long)k * g.sAK1, g.sAM, g.sAK1, g.M - (int)m0, ks, vec_a, tid);
-            fma_tile(tb, b + (long)k0 * g.sBK0 + (long)k * g.sBK1, g.sBN, g.sBK1, g.N - (int)n0, ks, vec_b, tid);
-            __syncthreads();
-#pragma unroll 8
-            for (int i = 0; i < ks; ++i) {
-                const float4 x = *reinterpret_cast<const float4*>(&ta[i][tm]), y = *reinterpret_cast<const float4*>(&tb[i][tn]);
-                const float xv[4] = {x.x, x.y, x.z, x.w}, yv[4] = {y.x, y.y, y.z, y.w};
+            pa.put(ta[buf], ks);
+            pb.put(tb[buf], ks);
+            __syncthreads();                                 // (the other buffer is free as well: every wave is done with the step before)
+            const bool same = k + FK < g.K1;
+            if (same || k0 + 1 < g.K0) fetch(same ? k0 : k0 + 1, same ? k + FK : 0);
+            if (working) {
+                // (the halves of the wave take the k of a pair: half a register each)
+                auto value = [&](uint32_t pair) __attribute__((always_inline)) {
+                    return (float)__builtin_bit_cast(half_t, (uint16_t)(pair >> (16 * hi)));
+                };
+                typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+                auto read = [&](const half_t* p) __attribute__((always_inline)) { return *reinterpret_cast<const u4*>(p); };
+                const half_t *const x = ta[buf][wm + l32], *const y0 = tb[buf][l32], *const y1 = tb[buf][32 + l32];
+                for (int i = 0; i < ks; i += 16) {
+                    const u4 fx[2] = {read(x + i), read(x + i + 8)}, f0[2] = {read(y0 + i), read(y0 + i + 8)}, f1[2] = {read(y1 + i), read(y1 + i + 8)};
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) acc[r][c] = __builtin_fmaf(xv[r], yv[c], acc[r][c]);
+                    for (int p = 0; p < 8; ++p) {
+                        const float xv = value(fx[p >> 2][p & 3]);
+                        acc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(xv, value(f0[p >> 2][p & 3]), acc[0], 0, 0, 0);
+                        acc[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(xv, value(f1[p >> 2][p & 3]), acc[1], 0, 0, 0);
+                    }
+                }
             }
+            buf ^= 1;
         }
+    if (!working) return;
+    // register v of a lane: row 8 (v / 4) + 4 hi + v % 4 of the wave's, column l32 of 32.  The halves of the wave trade, so that a lane has
+    // column `lane` of rows 8 (v / 4) + v % 4 and of those 4 further: rows of 128 bytes for an instruction.
+    const int n = (int)n0 + lane;
+    half_t* const c = g.C + b0 * g.sCb[0] + b1 * g.sCb[1] + b2 * g.sCb[2] + (long)n * g.sCN;
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
+    for (int v = 0; v < 16; ++v) {
+        const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[0][v]), __float_as_uint(acc[1][v]), false, false);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const int m = (int)m0 + tm + r, n = (int)n0 + tn + c;
+        for (int q = 0; q < 2; ++q) {
+            const int m = (int)m0 + wm + (v >> 2) * 8 + q * 4 + (v & 3);
             if (m >= g.M || n >= g.N) continue;
-            half_t out = (half_t)(acc[r][c] * g.alpha);
+            half_t out = (half_t)(__uint_as_float(both[q]) * g.alpha);
             if (g.bias)     // same two roundings as the product followed by a separate add
                 out = (half_t)((float)out + (float)g.bias[b0 * g.sbb[0] + b1 * g.sbb[1] + b2 * g.sbb[2] +
                                                           (long)m * g.sbM + (long)n * g.sbN]);
-            g.C[b0 * g.sCb[0] + b1 * g.sCb[1] + b2 * g.sCb[2] + (long)m * g.sCM + (long)n * g.sCN] = out;
+            c[(long)m * g.sCM] = out;
         }
+    }
 }
 
 // Adds the k-split partials: C[b,m,n] = fp16(alpha * sum_s P[s][b][m][n]) (+ addend).
@@ -484,13 +541,24 @@ void launch_gemm(const GemmShape& s, const half_t* A, const half_t* B, half_t* C
         }
     } else {
         if (ep.relu_dropout || ep.gate) fail("gemm: the ReLU-dropout epilogue needs the MFMA kernel");
-        const long blocks = batch * ((c.a.M + FB - 1) / FB) * ((c.a.N + FB - 1) / FB);
+        const long blocks = batch * ((c.a.M + FM - 1) / FM) * ((c.a.N + FN - 1) / FN);
         if (blocks > 0x7fffffffL) fail("gemm: problem too large for the scalar kernel");
-        auto words = [&](const half_t* p, long s_row, long s_k, long s_k0, const long (&sb)[3]) {
-            return s_k == 1 && al16(p) && mult8(s_row) && mult8(c.a.K1) && mult8(s_k0) && mult8(sb[0]) && mult8(sb[1]) && mult8(sb[2]);
+        // whole 16-byte words along k, or else along the operand's rows (of the output: m resp. n)
+        auto how = [&](const half_t* p, long rows, long s_row, long s_k, long s_k0, const long (&sb)[3]) {
+            const bool apart = al16(p) && mult8(s_k0) && mult8(sb[0]) && mult8(sb[1]) && mult8(sb[2]);
+            if (apart && s_k == 1 && mult8(s_row) && mult8(c.a.K1)) return FMA_ALONG_K;
+            return apart && s_row == 1 && mult8(s_k) && mult8(rows) ? FMA_ALONG_ROWS : FMA_SINGLE;
         };
-        hipLaunchKernelGGL(k_gemm_fma, dim3((unsigned)blocks), dim3(256), 0, st, c.a,
-                           words(c.a.A, c.a.sAM, c.a.sAK1, c.a.sAK0, c.a.sAb), words(c.a.B, c.a.sBN, c.a.sBK1, c.a.sBK0, c.a.sBb));
+        const int how_a = how(c.a.A, c.a.M, c.a.sAM, c.a.sAK1, c.a.sAK0, c.a.sAb), how_b = how(c.a.B, c.a.N, c.a.sBN, c.a.sBK1, c.a.sBK0, c.a.sBb);
+        auto run = [&](auto ha) {
+            auto with = [&](auto hb) { hipLaunchKernelGGL((k_gemm_fma<ha(), hb()>), dim3((unsigned)blocks), dim3(256), 0, st, c.a); };
+            if (how_b == FMA_ALONG_K) with(std::integral_constant<int, FMA_ALONG_K>{});
+            else if (how_b == FMA_ALONG_ROWS) with(std::integral_constant<int, FMA_ALONG_ROWS>{});
+            else with(std::integral_constant<int, FMA_SINGLE>{});
+        };
+        if (how_a == FMA_ALONG_K) run(std::integral_constant<int, FMA_ALONG_K>{});
+        else if (how_a == FMA_ALONG_ROWS) run(std::integral_constant<int, FMA_ALONG_ROWS>{});
+        else run(std::integral_constant<int, FMA_SINGLE>{});
     }
     check_launch("gemm");
 }

@@ -312,3 +312,32 @@ def test_nothing_behind_what_an_activation_epilogue_leaves_is_written(L, E, U, a
     o.bdrlb(sb, 'BJU', mask, 'BJU', lin2, 'BJU', dlin2, 'BJU', dbias2)
     assert torch.equal(out, out2) and torch.equal(dlin, dlin2) and float(dlin.float().abs().max()) > 0
     assert_close(dbias.float().cpu().numpy(), dbias2.float().cpu().numpy(), tol=2e-3, name='dbias')
+
+
+# (orders: words along k, along the rows and neither, of either operand; an output that is contiguous along m; steps of 32 k with one, 31 and no
+# k left over, tiles of 128 x 64 with 1, 32, 33 and 64 columns in the last one)
+@pytest.mark.parametrize('la,lb,lc', [('BJHP', 'BKHP', 'HBJK'), ('HBJK', 'BKHP', 'BJHP'), ('HBKJ', 'KBHP', 'BJHP'), ('HPBJ', 'BKHP', 'BHKJ'),
+                                      ('BHJP', 'HBPK', 'JBHK'), ('BHJK', 'BJHP', 'HBPK')])
+@pytest.mark.parametrize('dims', [(2, 33, 2, 24), (1, 97, 1, 64), (1, 129, 3, 192), (3, 65, 1, 31), (1, 255, 1, 8)])
+def test_sums_without_whole_words_are_one_chain_of_fused_multiply_adds(la, lb, lc, dims):
+    """Bit for bit, in the order of k: products of halves are exact in float64, and so are their sums with an fp32 value (here: 11 + 11
+    bits at exponents within 2 ** +-24), so that rounding each sum to float32 is what fmaf does."""
+    from substation_amd.ops import Ops
+    o = Ops(*dims)
+    sz = o.sizes
+    if o.handle.classify(la, lb, lc)['kernel'] == 1:
+        pytest.skip('whole words')
+    rng = np.random.default_rng(len(la) + dims[1])
+    draw = lambda l: h16(np.clip(rng.normal(size=tuple(sz[d] for d in l)), -4, 4)) * (rng.random(size=tuple(sz[d] for d in l)) > 0.1)
+    A, B = draw(la).astype(np.float64), draw(lb).astype(np.float64)
+    k, = set(la) & set(lb) - set(lc)
+    acc = np.zeros(tuple(sz[d] for d in lc), np.float32)
+    for i in range(sz[k]):
+        a, b = np.take(A, i, la.index(k)), np.take(B, i, lb.index(k))
+        term = np.einsum(f'{la.replace(k, "")},{lb.replace(k, "")}->{lc}'.lower(), a, b)
+        acc = (acc.astype(np.float64) + term).astype(np.float32)
+    C = torch.full(tuple(sz[d] for d in lc), float('nan'), dtype=torch.float16, device='cuda')
+    half = lambda x: torch.from_numpy(x.astype(np.float16)).cuda()
+    o.einsum(half(A), la, half(B), lb, C, lc)
+    torch.cuda.synchronize()
+    assert (C.cpu().numpy().view(np.uint16) == acc.astype(np.float16).view(np.uint16)).all()
