@@ -1249,8 +1249,14 @@ void for_variant(int P, const AttnArgs& a, Fn&& fn) {
 // 25.1; 4 x 256 causal (96) 13.3, 12.4, 15.1 and 10.3, 9.7, 11.7; 3 x 300 (108) 13.6, 11.8, 15.9 and 10.3, 9.7, 11.8; 8 x 128 (96) 7.0, 7.4,
 // 8.2 and 6.5, 7.1, 7.4.  Beyond: 8 x 256 on 512, H 16 (256) no difference, 13 x 201 (312) 15.0, 14.4, 16.4 and 17.4, 15.5, 20.2.
 // (One workgroup on a CU then: the kernels of halves may take the registers of a whole SIMD.)
+// With a mask the block with the most to do is what a launch waits for (causal, 32 tiles: 36 us alone, as much as without a mask, where
+// the average has half of it), and a half of that is won wherever there are tiles enough.  us as above, causal: 4 x 512 (192
+// blocks, 16 tiles) 22.7, 19.1, 24.6 and 16.9, 14.7, 21.4; 2 x 1024, H 16 (256, 32) 38.8, 32.4, 43.0 and 27.3, 23.3, 36.1; 3 x 1024 (288, 32)
+// 50.7, 41.6, 52.5 and 34.5, 29.7, 48.0; 2 x 2048 (384, 64) 71.3, 65.6, 85.8 and 54.8, 49.9, 90.4.  But 8 x 384 (288, 12) 22.6, 20.2, 25.0 and
+// 22.1, 20.0, 27.7, 8 x 512 (384, 16) 21.1, 23.0, 29.8 and 22.2, 24.6, 36.4; 8 x 256, H 16 (256, 8) 13.9, 13.6, 16.6 and 15.1, 13.8, 21.5.
 int parts(const AttnArgs& a, int P, long rows, long others) {
-    return P == 64 && a.H * (long)a.B * blocks(rows) <= kFewBlocks && tiles(others) >= 4 ? 2 : 1;
+    const long few = !a.amask || tiles(others) < 12 ? kFewBlocks : tiles(others) < 32 ? 2 * kFewBlocks : 3 * kFewBlocks;
+    return P == 64 && a.H * (long)a.B * blocks(rows) <= few && tiles(others) >= 4 ? 2 : 1;
 }
 }  // namespace
 

@@ -441,14 +441,14 @@ def test_attention_by_halves_of_the_other_side_equals_the_whole(J, K, p, mask):
         assert bool(torch.isfinite(a).all()) and close(a, b[:B], 2 ** -9)
 
 
-@pytest.mark.parametrize('L', [97, 130, 160, 201, 333])
-@pytest.mark.parametrize('causal', [False, True])
-def test_attention_by_halves_at_any_length(L, causal):
-    """4, 5, 7 and 11 tiles with an end inside, 0 to 4 of them in the list of a mask: a layer's two samples alone (few blocks) and in
-    front of 68 others, without dropout.  The outputs pass through the same operators and sums in another order: a fraction of the
+@pytest.mark.parametrize('L,few,causal', [(L, 2, c) for L in (97, 130, 160, 201, 333) for c in (False, True)] +
+                         [(400, 20, True), (1001, 12, True)])      # (more blocks, behind a mask that leaves long ones)
+def test_attention_by_halves_at_any_length(L, few, causal):
+    """4 to 32 tiles with an end inside, 0 to 32 of them in the list of a mask: a layer's few samples alone (few blocks) and in
+    front of the others of 70, without dropout.  The outputs pass through the same operators and sums in another order: a fraction of the
     1e-2 that parity allows."""
     from substation_amd import Encoder, causal_mask, mi355x_layouts
-    many, few, H, E = 70, 2, 2, 128
+    many, H, E = 70, 2, 128
     g = torch.Generator(device='cuda').manual_seed(L)
     x = torch.randn(many, L, E, generator=g, device='cuda').half()
     dy = torch.randn(many, L, E, generator=g, device='cuda').half()
