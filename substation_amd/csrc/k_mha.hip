@@ -95,7 +95,7 @@ template <int P, bool WALK, bool RAGGED, int PARTS>
 struct Tiles {
     const half_t* p;
     __device__ __forceinline__ Tiles(const AttnSide& t, unsigned h, unsigned b, unsigned first, int tid)
-        : p(t.p + (long)h * t.sh + (long)b * t.sb + (long)(first * 32 + tid / (P / 8)) * t.sr + tid % (P / 8) * 8) {}
+        : p(WALK ? t.p + (long)h * t.sh + (long)b * t.sb + (long)(first * 32 + tid / (P / 8)) * t.sr + tid % (P / 8) * 8 : nullptr) {}
     __device__ __forceinline__ void fetch(const AttnSide& t, unsigned h, unsigned b, unsigned tile, unsigned limit, int tid,
                                           h8 (&r)[Geo<P>::VL * PARTS]) {
         if (!WALK) { tile_fetch<P, RAGGED, PARTS>(t, h, b, tile * 32, limit, tid, r); return; }
@@ -203,6 +203,14 @@ __device__ __forceinline__ float column_sum(const float* sums, int feature) {
 // x where bit `pos` of `bits` is set, else +0.0
 __device__ __forceinline__ float keep_if(float x, uint32_t bits, int pos) {
     return __int_as_float(__float_as_int(x) & __builtin_amdgcn_sbfe((int)bits, pos, 1));
+}
+// The same of what a vector instruction has made (not of a product: nothing waits for one here).  Spelled out: as a choice it is
+// three instructions, and that is what the compiler makes of a mask in the forward kernel (4 x 1024: 47.8 us, as a choice 50.5).
+template <int pos>
+__device__ __forceinline__ float keep_probability(float x, uint32_t bits) {
+    float r;
+    asm("v_bfe_i32 %0, %1, %2, 1\n\tv_and_b32 %0, %0, %3" : "=&v"(r) : "v"(bits), "n"(pos), "v"(x));
+    return r;
 }
 
 // Scores of positions from `limit` on (the tile starts at tile0, register v of a lane holds position reg_pos(v, hi) of
@@ -571,8 +579,7 @@ __device__ __forceinline__ void mha_fwd(const AttnArgs& a, const PhiloxKey& key_
             for (int v = 0; v < 16; ++v) l4[v & 3] += s[v];
             l_run += (l4[0] + l4[1]) + (l4[2] + l4[3]);
         }
-#pragma unroll
-        for (int v = 0; v < 16; ++v) s[v] = keep_if(s[v], nib, reg_pos(v, 0));
+        each<16>([&](auto V) __attribute__((always_inline)) { constexpr int v = V; s[v] = keep_probability<reg_pos(v, 0)>(s[v], nib); });
 #pragma unroll
         for (int v = 0; v < 16; ++v) pb[v >> 3][v & 7] = (half_t)s[v];
 #pragma unroll
@@ -589,12 +596,11 @@ __device__ __forceinline__ void mha_fwd(const AttnArgs& a, const PhiloxKey& key_
         const int x = cur; cur = nxt; nxt = nn; nn = x;
         e0 = e1; e1 = e2; e2 = e3;
     }
-    const int w = __builtin_amdgcn_readfirstlane(wave);
-    half_t* out = w < 2 ? kt[w] : vt[w - 2];
+    [[maybe_unused]] float* left = nullptr;
     if constexpr (PARTS > 1) {
         // (the tiles' places are free)
         static_assert(Place<PARTS>::WAVES * G::NPT * 16 * 64 * sizeof(float) <= sizeof(kt_), "two waves' accumulators");
-        float* const left = reinterpret_cast<float*>(kt_) + wave * (G::NPT * 16 * 64);
+        left = reinterpret_cast<float*>(kt_) + wave * (G::NPT * 16 * 64);
         float* const stats = reinterpret_cast<float*>(vt_) + wave * 128;
         if (at.half) {
             leave(left, lane, o);
@@ -610,9 +616,10 @@ __device__ __forceinline__ void mha_fwd(const AttnArgs& a, const PhiloxKey& key_
         l_run = l_run * mine + stats[64 + lane] * theirs;
         collect(left, lane, o, mine, theirs);
         m_ref = m_new;
-        out = reinterpret_cast<half_t*>(left);
     }
     const float l_tot = l_run + __shfl_xor(l_run, 32);
+    const int w = __builtin_amdgcn_readfirstlane(wave);
+    half_t* const out = PARTS > 1 ? reinterpret_cast<half_t*>(left) : w < 2 ? kt[w] : vt[w - 2];
     store_rows<P, RAGGED>(a.o, h, b, qb * QB + (piece + w) * 32, a.J, lane, o, 1.0f / l_tot, out, nullptr);
     if (mine_ && hi == 0) a.lse[row] = m_ref * c + __builtin_amdgcn_logf(l_tot);
 }
