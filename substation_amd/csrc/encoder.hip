@@ -759,7 +759,7 @@ const BackwardPlan& backward_plan(Handle& h, const GemmJob (&jobs)[7], bool late
 // The launches of a group of contractions: the longest first, in one launch or, from some place of that order on, in another.  Kept for the
 // last groups asked for (a decoder layer's backward pass has two): shapes, strides, alignments, the option and the scratch are all that
 // they depend on.  Ten products of 8 x 256 on 512, E 1024: a call that makes its plan takes the host 31 us with every choice of tiles
-// at hand and 130 without, one that finds it 14, and a decoder layer of that size waits for its host (724 -> 700 us a pass).
+// at hand and 130 without, one that finds it 14 (a decoder layer of that size, when it waited for its host: 724 -> 700 us a pass).
 const GroupPlan& group_plan(Handle& h, const std::vector<GemmJob>& jobs) {
     const int n = (int)jobs.size();
     GroupPlan q;

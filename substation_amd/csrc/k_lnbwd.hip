@@ -376,8 +376,8 @@ inline int lnbwd_blocks(long nrows) {
 }
 
 // Waves of a workgroup of k_lnbwd_flat for rows of up to 1024 features, a row each: as few as leave no more than 256 partial rows, one
-// workgroup per CU.  A CU draws 33 KB a us of what is not in its L2, however few of them do: with sixteen, 1024 rows were
-// read by 64 CUs.  us of the two launches of a layer, E 768, with sixteen waves and now: 256 rows 7.9 and 7.4, 5.7 and 5.1; 1024 rows 9.2 and
+// workgroup per CU.  With sixteen, 1024 rows lay on 64 CUs, each with sixteen rows to read, to write and to add up through LDS.
+// us of the two launches of a layer, E 768, with sixteen waves and now: 256 rows 7.9 and 7.4, 5.7 and 5.1; 1024 rows 9.2 and
 // 7.7, 6.8 and 5.6.  2048 rows of 1024, mask as a tensor, 12.3 and (four sums, in the kernel above) 14.9, 10.0 and 10.4.  Beyond that
 // two workgroups of eight waves to a CU take what one of sixteen does (2613 and 4096 rows: 0.7 us either way), and the launch that adds
 // up 512 partial rows 1.5 us more.

@@ -777,8 +777,8 @@ void launch_bdrln(const RowSpace& rs, View in, View resid, View lin_bias, View s
         sums.p = nullptr;
     }
     if (flat) {
-        // Few rows: each in a workgroup of its own, since a CU draws 33 KB a us of what is not in its L2, however few CUs do (64 rows of 768,
-        // us with four rows to a workgroup and now: 3.9 and 3.7, with the parts of a split sum 5.3 and 4.5; 256 rows: no difference).
+        // Few rows: each in a workgroup of its own, on a CU of its own (64 rows of 768, us with four rows to a workgroup and now: 3.9 and 3.7,
+        // with the parts of a split sum 5.3 and 4.5; 256 rows: no difference).
         const unsigned waves = extra_blocks || nrows >= 256 ? WPB : 1;
         const dim3 grid(waves == WPB ? row_grid(nrows, 1) + extra_blocks : nrows), block(waves * WAVE);
 #define SUB_BDRLN_FLAT(V, S) hipLaunchKernelGGL((k_bdrln_flat<V, S>), grid, block, 0, st, rs.R, nrows, in, resid, lin_bias, \

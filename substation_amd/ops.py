@@ -14,8 +14,8 @@ from . import _lib
 from . import layouts as _lay
 
 
-# What a call costs the host beside its launch is what bounds the layers that are made of these calls: a decoder layer's 40
-# calls with their 330 tensors took 790 us to issue where its kernels take 650.  Hence addresses as plain integers (the
+# What a call costs the host beside its launch is what bounds a layer that is made of these calls (a decoder layer's 40
+# with their 330 tensors took 790 us to issue where its kernels take 650; it makes them from C++ now).  Hence addresses as plain integers (the
 # entry points' argument types say what they are), the stream asked for without an object around it, shapes looked up.
 def _p(t):
     if t is None:
