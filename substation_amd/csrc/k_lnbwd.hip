@@ -386,6 +386,14 @@ inline int lnbwd_flat_blocks(long nrows) {
     const int waves = lnbwd_waves(nrows);
     return waves == 16 ? lnbwd_blocks(nrows) : (int)((nrows + waves - 1) / waves);
 }
+// Longer rows, which two or four of sixteen waves share: a workgroup for each eight or four of them, as long as that is no more than one
+// per CU, then for as many times that as it takes.  us of the two launches with a workgroup for sixteen rows and now: 100 rows of 4096 22.3
+// and 23.2, 8.9 and 9.2; 512 of 4096 23.7 and 26.0, 11.8 and 12.3; 2048 of 4096 28.7 and 30.9, 22.0 and 22.5; 600 of 2048 13.6 and 15.0, 10.5 and
+// 10.2; 2048 of 2048 16.6 and 17.5, 13.5 and 14.2 (3000 of 2048 on all CUs, some with a row more: 18.2 and 19.1, 20.4 and 20.1).
+inline int lnbwd_wide_blocks(long nrows, int R) {
+    const long rows = R <= 2048 ? 8 : 4, groups = (nrows + rows - 1) / rows, passes = (groups + 255) / 256;
+    return (int)((groups + passes - 1) / passes);
+}
 // (the extended form with its four sums does not fit the 128 registers of sixteen waves)
 inline bool lnbwd_flat(const RowSpace& rs, const LnBwdArgs& a, bool ext) {
     return rs.flat && !(ext && !a.move_sum && lnbwd_waves(rs.rows()) == 16);
@@ -405,7 +413,7 @@ bool lnbwd_supported(const RowSpace& rs, const LnBwdArgs& a, bool ext) {
 }
 
 size_t lnbwd_ws_floats(const RowSpace& rs, bool ext) {
-    const int blocks = rs.R <= 1024 ? std::max(lnbwd_blocks(rs.rows()), lnbwd_flat_blocks(rs.rows())) : lnbwd_blocks(rs.rows());
+    const int blocks = rs.R <= 1024 ? std::max(lnbwd_blocks(rs.rows()), lnbwd_flat_blocks(rs.rows())) : lnbwd_wide_blocks(rs.rows(), rs.R);
     return (size_t)(ext ? 4 : 3) * blocks * rs.R;      // (3: the plain form with move_sum)
 }
 
@@ -415,7 +423,7 @@ void launch_lnbwd(const RowSpace& rs, const LnBwdArgs& a, bool ext, half_t* cons
     if (!ws) fail("fused LayerNorm backward: no reduction workspace");
     const unsigned nrows = (unsigned)rs.rows();
     const bool flat = rs.R <= 1024 && lnbwd_flat(rs, a, ext);
-    const int blocks = flat ? lnbwd_flat_blocks(nrows) : lnbwd_blocks(nrows);
+    const int blocks = rs.R > 1024 ? lnbwd_wide_blocks(nrows, rs.R) : flat ? lnbwd_flat_blocks(nrows) : lnbwd_blocks(nrows);
     const int vpl = rs.R <= 512 ? 1 : 2;
     if (rs.R > 1024) {
         // (lnbwd_supported has ruled out the extended form without move_sum: MOVE_ is EXT_ || move_sum)
