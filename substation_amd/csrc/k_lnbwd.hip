@@ -381,10 +381,13 @@ inline int lnbwd_blocks(long nrows) {
 // 7.7, 6.8 and 5.6.  2048 rows of 1024, mask as a tensor, 12.3 and (four sums, in the kernel above) 14.9, 10.0 and 10.4.  Beyond that
 // two workgroups of eight waves to a CU take what one of sixteen does (2613 and 4096 rows: 0.7 us either way), and the launch that adds
 // up 512 partial rows 1.5 us more.
-inline int lnbwd_waves(long nrows) { return nrows <= 1024 ? 4 : nrows <= 2048 ? 8 : 16; }
-inline int lnbwd_flat_blocks(long nrows) {
-    const int waves = lnbwd_waves(nrows);
-    return waves == 16 ? lnbwd_blocks(nrows) : (int)((nrows + waves - 1) / waves);
+// Four sums (the extended form without move_sum) do not fit the 128 registers of sixteen waves; with eight, two rows each and more, they
+// take less than in the kernel above, which row spaces that are not flat are left to: 4096 rows of 1024 18.9 -> 16.7 us, 8192 30.4 -> 28.7, 3072 of
+// 768 14.5 -> 12.7.
+inline int lnbwd_waves(long nrows, bool four) { return nrows <= 1024 ? 4 : nrows <= 2048 || four ? 8 : 16; }
+inline int lnbwd_flat_blocks(long nrows, bool four) {
+    const int waves = lnbwd_waves(nrows, four);
+    return waves == 16 ? lnbwd_blocks(nrows) : (int)std::min((nrows + waves - 1) / waves, 256L);
 }
 // Longer rows, which two or four of sixteen waves share: a workgroup for each eight or four of them, as long as that is no more than one
 // per CU, then for as many times that as it takes.  us of the two launches with a workgroup for sixteen rows and now: 100 rows of 4096 22.3
@@ -394,11 +397,6 @@ inline int lnbwd_wide_blocks(long nrows, int R) {
     const long rows = R <= 2048 ? 8 : 4, groups = (nrows + rows - 1) / rows, passes = (groups + 255) / 256;
     return (int)((groups + passes - 1) / passes);
 }
-// (the extended form with its four sums does not fit the 128 registers of sixteen waves)
-inline bool lnbwd_flat(const RowSpace& rs, const LnBwdArgs& a, bool ext) {
-    return rs.flat && !(ext && !a.move_sum && lnbwd_waves(rs.rows()) == 16);
-}
-
 }  // namespace
 
 bool lnbwd_supported(const RowSpace& rs, const LnBwdArgs& a, bool ext) {
@@ -413,7 +411,7 @@ bool lnbwd_supported(const RowSpace& rs, const LnBwdArgs& a, bool ext) {
 }
 
 size_t lnbwd_ws_floats(const RowSpace& rs, bool ext) {
-    const int blocks = rs.R <= 1024 ? std::max(lnbwd_blocks(rs.rows()), lnbwd_flat_blocks(rs.rows())) : lnbwd_wide_blocks(rs.rows(), rs.R);
+    const int blocks = rs.R <= 1024 ? std::max(lnbwd_blocks(rs.rows()), lnbwd_flat_blocks(rs.rows(), ext)) : lnbwd_wide_blocks(rs.rows(), rs.R);
     return (size_t)(ext ? 4 : 3) * blocks * rs.R;      // (3: the plain form with move_sum)
 }
 
@@ -422,8 +420,8 @@ void launch_lnbwd(const RowSpace& rs, const LnBwdArgs& a, bool ext, half_t* cons
     if (!lnbwd_supported(rs, a, ext)) fail("fused LayerNorm backward: unsupported shape or layout");
     if (!ws) fail("fused LayerNorm backward: no reduction workspace");
     const unsigned nrows = (unsigned)rs.rows();
-    const bool flat = rs.R <= 1024 && lnbwd_flat(rs, a, ext);
-    const int blocks = rs.R > 1024 ? lnbwd_wide_blocks(nrows, rs.R) : flat ? lnbwd_flat_blocks(nrows) : lnbwd_blocks(nrows);
+    const bool four = ext && !a.move_sum, flat = rs.R <= 1024 && rs.flat;
+    const int blocks = rs.R > 1024 ? lnbwd_wide_blocks(nrows, rs.R) : flat ? lnbwd_flat_blocks(nrows, four) : lnbwd_blocks(nrows);
     const int vpl = rs.R <= 512 ? 1 : 2;
     if (rs.R > 1024) {
         // (lnbwd_supported has ruled out the extended form without move_sum: MOVE_ is EXT_ || move_sum)
@@ -449,7 +447,7 @@ void launch_lnbwd(const RowSpace& rs, const LnBwdArgs& a, bool ext, half_t* cons
     do {                                                                                                          \
         const dim3 grid(blocks);                                                                                  \
         if (!flat) hipLaunchKernelGGL((k_lnbwd<VPL_, EXT_, BITS_, MOVE_>), grid, dim3(LN_BLOCK), 0, st, rs, a, ws, nrows);       \
-        else switch (lnbwd_waves(nrows)) {                                                                        \
+        else switch (lnbwd_waves(nrows, four)) {                                                                        \
             case 4: hipLaunchKernelGGL((k_lnbwd_flat<VPL_, EXT_, BITS_, MOVE_, 1, 4>), grid, dim3(4 * WAVE), 0, st, rs.R, a, ws, nrows); break; \
             case 8: hipLaunchKernelGGL((k_lnbwd_flat<VPL_, EXT_, BITS_, MOVE_, 1, 8>), grid, dim3(8 * WAVE), 0, st, rs.R, a, ws, nrows); break; \
             default:                                                                                              \
