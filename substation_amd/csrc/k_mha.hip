@@ -1172,7 +1172,7 @@ __global__ __launch_bounds__(256, (P == 64 && MASKED) ? 2 : 1) void k_mha_bwd_dk
     mha_bwd_dkv<P, MASKED, RAGGED, 1>(a);
 }
 template <int P, bool MASKED, bool RAGGED>
-__global__ __launch_bounds__(256) void k_mha_bwd_dkv_halves(AttnArgs a) {
+__global__ __launch_bounds__(256, MASKED ? 2 : 1) void k_mha_bwd_dkv_halves(AttnArgs a) {
     mha_bwd_dkv<P, MASKED, RAGGED, 2>(a);
 }
 
@@ -1255,14 +1255,16 @@ void for_variant(int P, const AttnArgs& a, Fn&& fn) {
 // blocks and with halves, H 12, P 64: 1 x 1024 (96 blocks) 30.9, 24.0, 31.2 and 21.2, 17.4, 21.6, causal 36.6, 30.6, 41.0 and 24.7, 19.8,
 // 25.1; 4 x 256 causal (96) 13.3, 12.4, 15.1 and 10.3, 9.7, 11.7; 3 x 300 (108) 13.6, 11.8, 15.9 and 10.3, 9.7, 11.8; 8 x 128 (96) 7.0, 7.4,
 // 8.2 and 6.5, 7.1, 7.4.  Beyond: 8 x 256 on 512, H 16 (256) no difference, 13 x 201 (312) 15.0, 14.4, 16.4 and 17.4, 15.5, 20.2.
-// (One workgroup on a CU then: the kernels of halves may take the registers of a whole SIMD.)
-// With a mask the block with the most to do is what a launch waits for (causal, 32 tiles: 36 us alone, as much as without a mask, where
-// the average has half of it), and a half of that is won wherever there are tiles enough.  us as above, causal: 4 x 512 (192
-// blocks, 16 tiles) 22.7, 19.1, 24.6 and 16.9, 14.7, 21.4; 2 x 1024, H 16 (256, 32) 38.8, 32.4, 43.0 and 27.3, 23.3, 36.1; 3 x 1024 (288, 32)
-// 50.7, 41.6, 52.5 and 34.5, 29.7, 48.0; 2 x 2048 (384, 64) 71.3, 65.6, 85.8 and 54.8, 49.9, 90.4.  But 8 x 384 (288, 12) 22.6, 20.2, 25.0 and
-// 22.1, 20.0, 27.7, 8 x 512 (384, 16) 21.1, 23.0, 29.8 and 22.2, 24.6, 36.4; 8 x 256, H 16 (256, 8) 13.9, 13.6, 16.6 and 15.1, 13.8, 21.5.
+// With a mask a tile has more to wait for (its mask values, a list's next entry), and the second wave that the halves put on a SIMD fills that,
+// whatever the mask leaves to do, as long as whole blocks are no more than one to a CU and there are tiles enough: then every kernel gains
+// under every mask that was timed, with lists of tiles (a layer's) and without (an operator's).  us of whole blocks and of halves, 256 blocks of
+// 32 tiles, H 4: causal 37.9, 31.8, 42.0 and 24.6, 22.1, 29.9; all zeros 39.7, 33.4, 42.6 and 33.5, 28.7, 36.2; a quarter of the keys gone 31.2,
+// 26.6, 41.2 and 27.2, 24.0, 34.7; a window of a quarter 19.8, 18.0, 22.5 and 17.7, 16.9, 21.0; a slope 43.8, 42.4, 59.9 and 36.6, 33.2, 46.3; causal without
+// lists 37.1, 38.0, 56.8 and 31.4, 31.8, 44.4.  192 blocks of 12 tiles: causal 17.8, 16.2, 20.1 and 14.9, 14.6, 17.7, a quarter gone 15.2, 13.2, 24.4 and
+// 14.5, 14.2, 19.9.  Beyond, some lose: 320 blocks of 32 tiles causal 39.5, 34.5, 45.2 and 28.4, 28.6, 35.5, but zeros 51.9, 42.3, 52.1 and 46.5, 40.1, 53.9,
+// a window 23.4, 21.1, 26.7 and 24.2, 23.2, 31.0; so they do with fewer tiles: 256 blocks of 8, a window 12.8, 12.8, 13.9 and 13.2, 13.5, 14.8.
 int parts(const AttnArgs& a, int P, long rows, long others) {
-    const long few = !a.amask || tiles(others) < 12 ? kFewBlocks : tiles(others) < 32 ? 2 * kFewBlocks : 3 * kFewBlocks;
+    const long few = a.amask && tiles(others) >= 12 ? 2 * kFewBlocks : kFewBlocks;
     return P == 64 && a.H * (long)a.B * blocks(rows) <= few && tiles(others) >= 4 ? 2 : 1;
 }
 }  // namespace
@@ -1307,7 +1309,10 @@ void launch_mha_backward_dkv(const AttnArgs& a, int P, hipStream_t st) {
     dim3 grid((unsigned)(a.H * a.B * blocks(a.K) * n));
     for_variant(P, a, [&](auto p, auto masked, auto rag) {
         if constexpr (p() == 64) {
-            if (n == 2) { hipLaunchKernelGGL((k_mha_bwd_dkv_halves<p(), masked(), rag()>), grid, dim3(256), 0, st, a); return; }
+            // (behind a mask the kernel for any length at every length: without the end checks it takes 284 registers, one wave per SIMD,
+            // where this one takes 249; held to 256 it spills around the mask values.  us at 256 blocks of 32 tiles, all zeros, H 16:
+            // whole blocks 40.8, halves 49.1 with 284 registers, 36.2 now)
+            if (n == 2) { hipLaunchKernelGGL((k_mha_bwd_dkv_halves<p(), masked(), masked() || rag()>), grid, dim3(256), 0, st, a); return; }
         }
         hipLaunchKernelGGL((k_mha_bwd_dkv<p(), masked(), rag()>), grid, dim3(256), 0, st, a);
     });

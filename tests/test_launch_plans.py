@@ -227,3 +227,67 @@ def test_order_of_the_sums_in_front_of_a_relu(tmp_path):
     """It is a fixed function of the shape: another one moves gates, and with them whole rows of gradients."""
     lines = launches.run(_orders_in_front_of_a_relu, tmp_path)
     assert dict(zip(ORDERS, lines)) == ORDERS
+
+
+# (samples, heads, queries, keys, head size, mask, activation): blocks of 128 queries and of keys; whether forward, dQ, and dK and dV take the
+# kernels in which two waves share a block's other side (h) or those of whole blocks (w)
+ATTENTION = {
+    (2, 16, 512, 512, 64, False, 'gelu'): 'hhh',      # 128 blocks
+    (3, 12, 512, 512, 64, False, 'gelu'): 'www',      # 144
+    (8, 16, 128, 512, 64, False, 'gelu'): 'hhw',      # 128 of queries, 512 of keys
+    (2, 16, 512, 512, 64, False, 'relu'): 'whh',
+    (2, 16, 512, 512, 64, True, 'relu'): 'whh',
+    (2, 16, 512, 512, 128, False, 'gelu'): 'www',
+    (4, 12, 384, 384, 64, True, 'gelu'): 'hhh',       # 144 blocks of 12 tiles
+    (4, 16, 512, 512, 64, True, 'gelu'): 'hhh',       # 256 of 16
+    (2, 16, 1024, 1024, 64, True, 'gelu'): 'hhh',     # 256 of 32
+    (8, 16, 256, 256, 64, True, 'gelu'): 'www',       # 256 of 8
+    (3, 12, 1024, 1024, 64, True, 'gelu'): 'www',     # 288 of 32
+    (2, 12, 2048, 2048, 64, True, 'gelu'): 'www',     # 384 of 64
+    (2, 24, 128, 384, 64, True, 'gelu'): 'hhw',       # 48 of queries; 144 of keys, of 4 tiles
+    (2, 16, 1000, 1000, 64, True, 'gelu'): 'hhh',     # (a layer's: lengths with an end inside a tile)
+    (5, 10, 201, 201, 64, False, 'gelu'): 'hhh',      # 100
+    (13, 12, 201, 201, 64, False, 'gelu'): 'www',     # 312
+}
+
+
+def _attention_launches():
+    from substation_amd import _lib, layouts as L
+    lib = _lib.load()
+    for (B, H, J, K, P, mask, act) in ATTENTION:
+        h = _lib.Handle(_lib.make_config(B, J, H, H * P, L.mi355x_layouts(), 0.1, 0.1, 0.1, 0.1, activation=act))
+        q, k, v, out, dout, dq, dk, dv, m, bq, bk, bv, stats, keep = launches.tensors(14)
+        m = m if mask else None
+        calls = []
+        if J % 128 == 0 and K % 128 == 0:
+            calls.append(lambda: (
+                _lib.check(lib.sub_op_attention_forward(h.ptr, J, K, q, b'BJHP', k, v, b'BKHP', out, b'BJHP', stats, keep, m, b'JK', 0.125, 0.1, 0)),
+                _lib.check(lib.sub_op_attention_backward_biases(h.ptr, J, K, q, b'BJHP', k, v, b'BKHP', out, b'BJHP', dout, b'BJHP', stats, keep, dq,
+                                                                b'BJHP', dk, dv, b'BKHP', m, b'JK', 0.125, bq, bk, bv))))
+        if J == K:
+            if mask:
+                h.set_attention_mask(m, 'JK')
+            calls.append(lambda: (_lib.check(lib.sub_encoder_forward(h.ptr, *_pointers(launches.tensors(37)))),
+                                  _lib.check(lib.sub_encoder_backward(h.ptr, *_pointers(launches.tensors(64, first=64))))))
+        blocks = lambda n: B * H * -(-n // 128)
+        seen = set()
+        for call in calls:
+            row = ''
+            for name, (grid, *_) in launches.launched(call):
+                kernel = re.search(r'k_mha_(fwd|bwd_dq|bwd_dkv)(_halves)?ILi(\d+)ELb(\d)ELb(\d)E', name)
+                if not kernel:
+                    continue
+                which, halves, p, masked, any_length = kernel.groups()
+                whole = blocks(K if which == 'bwd_dkv' else J)
+                assert (int(p), int(masked)) == (P, mask) and grid == whole * (2 if halves else 1)
+                # (the one that spills or has a SIMD to itself is not built; see tests/test_kernel_registers.py)
+                assert not (halves and which == 'bwd_dkv' and mask) or any_length == '1'
+                row += 'h' if halves else 'w'
+            seen.add(row)
+        print(' '.join(sorted(seen)))
+
+
+def test_which_attention_launches_share_a_block_between_two_waves(tmp_path):
+    """Operators and layers alike: up to 128 blocks, behind a mask up to one for each of 256 CUs where a block has 12 tiles to walk."""
+    lines = launches.run(_attention_launches, tmp_path)
+    assert dict(zip(ATTENTION, lines)) == ATTENTION
