@@ -439,6 +439,37 @@ struct DecoderPasses {
         return t.data_ptr();
     }
     static void* at_(const Maybe& t) { return t ? at_(*t) : nullptr; }
+    // The kernels are handed bare pointers: what a caller brings, or hooks on saved tensors restore, has as many elements as the layer's
+    // sizes say, or the pass is refused before its first launch.
+    static void holds(const at::Tensor& t, int64_t numel, const char* what) {
+        if (t.numel() == numel) return;
+        raise("DecoderLayer: " + std::string(what) + " has " + std::to_string(t.numel()) + " elements, the sizes of the layer need " +
+              std::to_string(numel), PyExc_ValueError);
+    }
+    void check_sizes(const at::Tensor& x, const at::Tensor& enc, const std::vector<at::Tensor>& w, const Maybe& mask) const {
+        const int64_t EE = E * H * P, in_b = 3 * H * P;
+        const struct { const char* name; int64_t numel; } parameters[PARAMETERS] = {
+            {"sattn_wkqv", 3 * EE}, {"sattn_in_b", in_b}, {"sattn_wo", EE}, {"sattn_out_b", E}, {"edattn_wq", EE}, {"edattn_wk", EE},
+            {"edattn_wv", EE}, {"edattn_in_b", in_b}, {"edattn_wo", EE}, {"edattn_out_b", E}, {"norm1_scale", E}, {"norm1_bias", E},
+            {"norm2_scale", E}, {"norm2_bias", E}, {"norm3_scale", E}, {"norm3_bias", E}, {"linear1_w", U * E}, {"linear1_b", U},
+            {"linear2_w", E * U}, {"linear2_b", E}};
+        if (w.size() != PARAMETERS) raise("DecoderLayer: 20 parameters", PyExc_ValueError);
+        for (int i = 0; i < PARAMETERS; ++i) holds(w[i], parameters[i].numel, parameters[i].name);
+        holds(x, B * Lt * E, "x");
+        holds(enc, B * Ls * E, "the encoder's output");
+        if (mask) holds(*mask, Lt * Lt, "the mask of the self-attention");
+    }
+    void check_kept(const std::vector<Maybe>& k, const at::Tensor& dy) const {
+        const int64_t bji = B * Lt * E, bki = B * Ls * E, bj = B * Lt, bju = B * Lt * U, rows = H * B * Lt;
+        const int64_t numels[KEPT] = {3 * bji, 2 * rows, rows * (Lt / 32), bji, bji, bji, bji, bji, bj, bji, bki, bki, 2 * rows, rows * (Ls / 32), bji,
+                                      bji, bji, bji, bji, bj, bju, bju, bju, bju / 8, bji, bji, bji, bj};
+        if (k.size() < KEPT) raise("DecoderLayer: not what a forward pass has saved", PyExc_ValueError);
+        for (int i = 0; i < KEPT; ++i) {
+            if (k[i]) holds(*k[i], numels[i], "what a forward pass has saved");
+            else if (i != LIN1 && i != MASK3 && i != BITS) raise("DecoderLayer: not what a forward pass has saved", PyExc_ValueError);
+        }
+        holds(dy, bji, "the gradient of the output");
+    }
     static char* part(const at::Tensor& t, int64_t i, int64_t of) { return static_cast<char*>(at_(t)) + 2 * (t.numel() / of) * i; }
 
     // A pass: the current device's stream, tensors on that device.
@@ -458,13 +489,13 @@ struct DecoderPasses {
                                uint32_t step, bool epilogues) {
         py::gil_scoped_release nogil;
         const std::lock_guard<std::mutex> one(busy);
+        check_sizes(x, enc, w, mask);
         const Place e(*this);
         check(lib.set_rng(target, seed, step), "sub_set_rng");
         check(lib.set_rng(source, seed, step), "sub_set_rng");
         std::vector<Maybe> k(KEPT + 1);                      // and the output
         std::vector<void*> wp;
         wp.reserve(PARAMETERS);
-        if (w.size() != PARAMETERS) raise("DecoderLayer: 20 parameters", PyExc_ValueError);
         for (const auto& t : w) wp.push_back(at_(t));
         const auto make = [&](Kept i, at::IntArrayRef shape) { k[i] = e(shape); return k[i]->data_ptr(); };
         const std::initializer_list<int64_t> bji = {B, Lt, E}, bj = {B, Lt}, bjhp = {B, Lt, H, P}, bkhp = {B, Ls, H, P}, bju = {B, Lt, U};
@@ -564,7 +595,8 @@ struct DecoderPasses {
                                      const at::Tensor& dy, const Maybe& mask) {
         py::gil_scoped_release nogil;
         const std::lock_guard<std::mutex> one(busy);
-        if (w.size() != PARAMETERS || k.size() < KEPT) raise("DecoderLayer: not what a forward pass has saved", PyExc_ValueError);
+        check_sizes(x, enc, w, mask);
+        check_kept(k, dy);
         // (the products with an epilogue need whole 16-byte words, wherever a parameter lies or was restored to)
         for (const Parameter i : {LINEAR2_W, EDATTN_WV, SATTN_WKQV})
             if (misaligned(w[i])) w[i] = w[i].clone();

@@ -189,3 +189,48 @@ def test_decoder_layer_refuses_a_tensor_of_another_type_and_goes_on(lengths):
         y.backward(dy)
     for a, b in zip(run(2 ** 64 - 3), want):
         assert torch.equal(a, b)
+
+
+def test_decoder_layer_refuses_tensors_of_other_sizes_before_it_launches():
+    """Of a call, of the module, or restored by hooks: a ValueError, and the layer goes on as before."""
+    from substation_amd import DecoderLayer
+    B, Lt, Ls, H, E = 2, 256, 128, 2, 128
+    torch.manual_seed(3)
+    layer = DecoderLayer(B, Lt, Ls, H, E, activation='gelu').cuda()
+    half = lambda *shape: torch.randn(shape).half().cuda()
+    x, enc, dy = half(B, Lt, E), half(B, Ls, E), half(B, Lt, E)
+
+    def run():
+        layer.set_rng(5, 7)
+        layer.zero_grad(set_to_none=True)
+        y = layer(x, enc)
+        y.backward(dy)
+        return [y.detach()] + [p.grad for p in layer.parameters()]
+
+    want = run()
+    for a, b in ((x, half(B, Ls + 128, E)), (x, half(B, Ls // 2, E)), (x, half(B - 1, Ls, E)), (half(B, Lt - 128, E), enc), (half(B, Lt, 2 * E), enc)):
+        with pytest.raises(ValueError, match='the sizes of the layer need'):
+            layer(a, b)
+    mask = layer.sattn_mask
+    for n in (128, 512):
+        layer.sattn_mask = torch.zeros(n, n, dtype=torch.float16, device='cuda')
+        with pytest.raises(ValueError, match='mask of the self-attention'):
+            layer(x, enc)
+    layer.sattn_mask = mask
+    for name in layer.param_names:
+        p = getattr(layer, name)
+        setattr(layer, name, torch.nn.Parameter(p.detach()[..., :p.shape[-1] // 2].contiguous()))
+        with pytest.raises(ValueError, match=name):
+            layer(x, enc)
+        setattr(layer, name, p)
+    for shape in ((B, Ls, E), (E, 4 * E), (E,)):              # the encoder's output, linear2_w, the biases
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t[..., :t.shape[-1] // 2].contiguous() if tuple(t.shape) == shape else t):
+            y = layer(x, enc)
+        with pytest.raises(ValueError, match='the sizes of the layer need'):
+            y.backward(dy)
+    # (as many elements in another shape are what they were)
+    with torch.no_grad():
+        layer.set_rng(5, 7)
+        assert torch.equal(layer(x.view(B * Lt, E), enc.view(-1)), want[0])
+    for a, b in zip(run(), want):
+        assert torch.equal(a, b)
