@@ -601,7 +601,6 @@ struct DecoderPasses {
         for (const Parameter i : {LINEAR2_W, EDATTN_WV, SATTN_WKQV})
             if (misaligned(w[i])) w[i] = w[i].clone();
         const Place e(*this);
-        Deferred deferred(*this);
         std::vector<at::Tensor> out(2);                      // dx and d(encoder output), then the parameters'
         std::vector<void*> wp, g;
         wp.reserve(PARAMETERS); g.reserve(PARAMETERS);
@@ -610,6 +609,10 @@ struct DecoderPasses {
             out.push_back(at::empty_like(t));
             g.push_back(at_(out.back()));
         }
+        const at::Tensor unused = at::empty_like(out[2 + SATTN_OUT_B]);      // norm1's column sums of the third input are not needed
+        // (behind all that receives such a sum: what a refusal further down leaves on the list is launched on the way out, into memory
+        // that must still be this pass's)
+        Deferred deferred(*this);
         const std::initializer_list<int64_t> bji = {B, Lt, E}, bjhp = {B, Lt, H, P}, bkhp = {B, Ls, H, P}, bju = {B, Lt, U};
         // a LayerNorm's backward pass, its dropout's and (second: with a second gradient) the sums next to it
         struct Norm { at::Tensor dln, dres, ddrop; };
@@ -660,7 +663,6 @@ struct DecoderPasses {
         group({{nullptr, at_(dq2), "BJHP", wp[EDATTN_WQ], "HPI", nullptr, nullptr, at_(dnormed1), "BJI", 1.f},
                {source, at_(dk2), "BKHP", wp[EDATTN_WK], "HPI", nullptr, nullptr, denc, "BKI", 1.f}});
         // norm1, residual, self-attention
-        const at::Tensor unused = at::empty_like(out[2 + SATTN_OUT_B]);      // the column sums of the third input are not needed here
         const Norm n1 = norm(LN1, NORM1_SCALE, n2.dres, ISTD1, DIFF1, MASK1, &dnormed1, &datt2, at_(unused), g[SATTN_OUT_B]);
         const at::Tensor& datt1 = n1.ddrop;
         const at::Tensor dgamma1 = e(bjhp);

@@ -234,3 +234,33 @@ def test_decoder_layer_refuses_tensors_of_other_sizes_before_it_launches():
         assert torch.equal(layer(x.view(B * Lt, E), enc.view(-1)), want[0])
     for a, b in zip(run(), want):
         assert torch.equal(a, b)
+
+
+def test_decoder_layer_goes_on_behind_a_refusal_in_the_middle_of_a_backward_pass():
+    """x restored with another type is found at the last products, with column sums of the pass still to be added up: they end
+    in the pass's own memory, and the handle no longer puts any off."""
+    from substation_amd import DecoderLayer
+    B, Lt, Ls, H, E = 2, 128, 256, 2, 128
+    torch.manual_seed(3)
+    layer = DecoderLayer(B, Lt, Ls, H, E, activation='gelu').cuda()
+    half = lambda *shape: torch.randn(shape).half().cuda()
+    x, enc, dy = half(B, Lt, E), half(B, Ls, E), half(B, Lt, E)
+
+    def run():
+        layer.set_rng(5, 7)
+        layer.zero_grad(set_to_none=True)
+        y = layer(x, enc)
+        y.backward(dy)
+        return [y.detach()] + [p.grad for p in layer.parameters()]
+
+    want = run()
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t.float() if tuple(t.shape) == (B, Lt, E) else t):
+        y = layer(x, enc)
+    with pytest.raises(ValueError, match='contiguous fp16'):
+        y.backward(dy)
+    taken = [torch.full_like(p, 3.0) for p in layer.parameters()]
+    sums = torch.full((E,), -1.0, dtype=torch.float16, device='cuda')
+    layer.ops_t.baob(torch.ones_like(dy), 'BJI', sums)
+    assert all(bool((t == 3.0).all()) for t in taken) and bool((sums == B * Lt).all())
+    for a, b in zip(run(), want):
+        assert torch.equal(a, b)
