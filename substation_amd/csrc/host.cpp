@@ -571,11 +571,13 @@ struct DecoderPasses {
     // The second stage of every column sum of a pass in one launch at its end (whatever becomes of the pass).
     struct Deferred {
         std::vector<void*> handles;
-        explicit Deferred(const DecoderPasses& d) {
+        Deferred() = default;
+        // (by way of the constructor above: from there on a refusal of the second handle runs the destructor for the first)
+        explicit Deferred(const DecoderPasses& d) : Deferred() {
             for (void* h : {d.target, d.source}) {
                 if (std::find(handles.begin(), handles.end(), h) != handles.end()) continue;
-                check(lib.ops_defer(h, 1), "sub_ops_defer");
                 handles.push_back(h);
+                check(lib.ops_defer(h, 1), "sub_ops_defer");
             }
         }
         void finish() {

@@ -264,3 +264,21 @@ def test_decoder_layer_goes_on_behind_a_refusal_in_the_middle_of_a_backward_pass
     assert all(bool((t == 3.0).all()) for t in taken) and bool((sums == B * Lt).all())
     for a, b in zip(run(), want):
         assert torch.equal(a, b)
+
+
+def test_decoder_layer_puts_no_sums_off_where_one_of_its_handles_cannot():
+    """A backward pass that the source's handle refuses (its configuration was replaced by one that is none) leaves the target's as it was."""
+    import ctypes
+    from substation_amd import DecoderLayer, _lib
+    layer = DecoderLayer(1, 128, 128, 2, 128, activation='gelu').cuda()
+    x, enc, dy = (torch.randn(1, 128, 128).half().cuda() for _ in range(3))
+    y = layer(x, enc)
+    source = layer.ops_s.handle
+    source._config.output_layout = b'BJP'
+    with pytest.raises(_lib.SubstationError):
+        _lib.check(source.lib.sub_configure(source.ptr, ctypes.byref(source._config)))
+    with pytest.raises(_lib.SubstationError):
+        y.backward(dy)
+    sums = torch.full((128,), -1.0, dtype=torch.float16, device='cuda')
+    layer.ops_t.baob(torch.ones_like(dy), 'BJI', sums)
+    assert bool((sums == 128).all())
