@@ -709,9 +709,17 @@ PYBIND11_MODULE(_host, m) {
         .def_property("mask", [](const EncoderLayer& l) { return l.mask; }, &EncoderLayer::use_mask)
         .def("set_step_counter", &EncoderLayer::set_step_counter)
         .def("forward", &EncoderLayer::forward);
-    py::class_<DecoderPasses>(m, "DecoderPasses")
+    py::class_<DecoderPasses> decoder(m, "DecoderPasses");
+    decoder
         .def(py::init<uintptr_t, uintptr_t, py::object, const std::vector<int64_t>&, const std::vector<double>&, const std::vector<uint32_t>&, bool,
                       double>())
         .def("forward", &DecoderPasses::forward)
         .def("backward", &DecoderPasses::backward);
+    // places in what a forward pass returns
+    decoder.attr("MASK1") = (int)DecoderPasses::MASK1;
+    decoder.attr("MASK2") = (int)DecoderPasses::MASK2;
+    decoder.attr("MASK3") = (int)DecoderPasses::MASK3;
+    decoder.attr("BITS") = (int)DecoderPasses::BITS;
+    decoder.attr("MASK4") = (int)DecoderPasses::MASK4;
+    decoder.attr("OUTPUT") = (int)DecoderPasses::KEPT;
 }

@@ -100,11 +100,11 @@ def _make_function(m):
     o, os_ = m.ops_t, m.ops_s
     scale = 1.0 / math.sqrt(m.proj_size)
     # the operators of both passes (host.cpp, DecoderPasses): parameters in the order in which they are registered above
-    passes = _lib.host().DecoderPasses(
+    Passes = _lib.host().DecoderPasses            # (and its places in what a forward pass returns)
+    passes = Passes(
         o.handle.ptr, os_.handle.ptr, (o, os_),
         [m.batch_size, m.target_len, m.source_len, m.num_heads, m.proj_size, m.embedding_size, m.intermediate_size],
         [float(p) for p in m.probs], [SITE_SATTN, SITE_EDATTN, SITE_LINEAR1, SITE_FF], m.activation == 'relu', scale)
-    mask1, mask2, mask3, bits, mask4, output = 4, 15, 21, 23, 24, 28        # (of what a forward pass returns)
 
     class DecoderFunction(torch.autograd.Function):
         @staticmethod
@@ -115,11 +115,11 @@ def _make_function(m):
             step, m.step = m.step, m.step + 1
             ctx.mask = m.sattn_mask
             kept = passes.forward(x, enc, params, ctx.mask, m.seed & (2**64 - 1), step & (2**32 - 1), bool(m.activation_epilogues))
-            y = kept.pop(output)
-            m.ffn_in_epilogues = kept[bits] is not None
+            y = kept.pop(Passes.OUTPUT)
+            m.ffn_in_epilogues = kept[Passes.BITS] is not None
             ctx.save_for_backward(x, enc, *params)
             ctx.kept = kept
-            m.last_masks = dict(sattn=kept[mask1], edattn=kept[mask2], linear1=kept[mask3], ff=kept[mask4])
+            m.last_masks = dict(sattn=kept[Passes.MASK1], edattn=kept[Passes.MASK2], linear1=kept[Passes.MASK3], ff=kept[Passes.MASK4])
             return y
 
         @staticmethod
