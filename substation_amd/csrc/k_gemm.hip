@@ -34,17 +34,22 @@ namespace {
 // 41 and 52, 24 and 30; 24 x 77 21 and 23, 14 and 15; 3 x 300 22 and 67, 15 and 30; 2 x 1500, H 16: 215 and 321, 109 and 172 (a third
 // of that instruction's rate: the single elements of a row that starts anywhere).
 // ---------------------------------------------------------------------------
-constexpr int FM = 128, FN = 64, FK = 32, FPITCH = FK + 8;
+// A product of up to 64 rows has tiles of 64 x 64, 32 x 32 per wave, where half of the waves would have none; one of up to 24 k goes by steps of
+// 8, read one by one: with 32 a thread brings 24 elements, most of them zeros.  us with v_fma_f32, with 128 x 64 and 32 k alone, and now: product with
+// V, H 12, P 64, 24 x 33 9.9, 11.1, 7.2; 1 x 1 4.4, 5.9, 3.7; 24 x 7 6.1, 6.7, 4.1; weight gradient of 4 rows, 2000 x 500, 5.9, 7.2, 5.4.  (17 to 24 k:
+// 1024 x 5 of 20 7.6, 8.2, 6.9, the product with V of 1 x 17 6.6, 4.6 with 32, 5.0.)
+constexpr int FN = 64;
 typedef float f16v __attribute__((ext_vector_type(16)));
 enum : int { FMA_SINGLE = 0, FMA_ALONG_K = 1, FMA_ALONG_ROWS = 2 };       // how an operand is read: whole 16-byte words or not
 
-// What a thread brings of an operand's ROWS x 32 elements: words, or elements that lie side by side over the threads along k or
+// What a thread brings of an operand's ROWS x FK elements: words, or elements that lie side by side over the threads along k or
 // along the rows.  What lies outside is read from a place that there is, and put down as zero where it is a k: no branch around a
 // load, where the wait for it would go.  Single elements are kept apart: of two in a register, the second's load waits for the first's.
 // In LDS [row][k], as half values: 16 bytes are four steps of a matrix instruction.
-template <int ROWS, int HOW>
+template <int ROWS, int HOW, int FK>
 struct FmaPart {
-    static constexpr int N = ROWS * FK / 256, WORDS = N / 8, L = HOW == FMA_SINGLE ? N : WORDS;
+    static constexpr int N = ROWS * FK / 256, WORDS = HOW == FMA_SINGLE ? 1 : N / 8, L = HOW == FMA_SINGLE ? N : WORDS, FPITCH = FK + 8;
+    static_assert(HOW == FMA_SINGLE || FK == 32, "words of 8 k");
     int row, k, drow, dk;                    // of the first, and on to the next
     h8 word[WORDS];
     uint16_t one[N];
@@ -82,11 +87,12 @@ struct FmaPart {
     }
 };
 
-template <int HOW_A, int HOW_B>
+template <int HOW_A, int HOW_B, int FM, int FK>
 __global__ __launch_bounds__(256, 4) void k_gemm_fma(GemmArgs g) {
+    constexpr int FPITCH = FK + 8, NACC = FM / 64;
     __shared__ __attribute__((aligned(16))) half_t ta[2][FM][FPITCH], tb[2][FN][FPITCH];
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hi = lane >> 5;
-    const int wm = __builtin_amdgcn_readfirstlane(tid >> 6) * 32;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave % (FM / 32) * 32, wn = wave / (FM / 32) * 32;
     const unsigned tiles_m = (g.M + FM - 1) / FM, tiles_n = (g.N + FN - 1) / FN;
     unsigned id = blockIdx.x;
     const unsigned n0 = id % tiles_n * FN; id /= tiles_n;
@@ -96,12 +102,12 @@ __global__ __launch_bounds__(256, 4) void k_gemm_fma(GemmArgs g) {
     const half_t* const a = g.A + b0 * g.sAb[0] + b1 * g.sAb[1] + b2 * g.sAb[2] + (long)m0 * g.sAM;
     const half_t* const b = g.B + b0 * g.sBb[0] + b1 * g.sBb[1] + b2 * g.sBb[2] + (long)n0 * g.sBN;
     const int rows = min(g.M - (int)m0, FM), cols = min(g.N - (int)n0, FN);
-    FmaPart<FM, HOW_A> pa(g.sAK1 == 1, tid);
-    FmaPart<FN, HOW_B> pb(g.sBK1 == 1, tid);
-    const bool working = wm < rows;                          // (a wave whose outputs all lie outside only helps with the operands)
-    f16v acc[2];
+    FmaPart<FM, HOW_A, FK> pa(g.sAK1 == 1, tid);
+    FmaPart<FN, HOW_B, FK> pb(g.sBK1 == 1, tid);
+    const bool working = wm < rows && wn < cols;             // (a wave whose outputs all lie outside only helps with the operands)
+    f16v acc[NACC];
 #pragma unroll
-    for (int v = 0; v < 16; ++v) acc[0][v] = acc[1][v] = 0.f;
+    for (int v = 0; v < 16 * NACC; ++v) acc[v / 16][v % 16] = 0.f;
     auto fetch = [&](int k0, int k) __attribute__((always_inline)) {
         pa.fetch(a + (long)k0 * g.sAK0 + (long)k * g.sAK1, g.sAM, g.sAK1, rows, g.K1 - k);
         pb.fetch(b + (long)k0 * g.sBK0 + (long)k * g.sBK1, g.sBN, g.sBK1, cols, g.K1 - k);
@@ -123,36 +129,47 @@ __global__ __launch_bounds__(256, 4) void k_gemm_fma(GemmArgs g) {
                 };
                 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
                 auto read = [&](const half_t* p) __attribute__((always_inline)) { return *reinterpret_cast<const u4*>(p); };
-                const half_t *const x = ta[buf][wm + l32], *const y0 = tb[buf][l32], *const y1 = tb[buf][32 + l32];
-                for (int i = 0; i < ks; i += 16) {
-                    const u4 fx[2] = {read(x + i), read(x + i + 8)}, f0[2] = {read(y0 + i), read(y0 + i + 8)}, f1[2] = {read(y1 + i), read(y1 + i + 8)};
+                constexpr int R = FK < 16 ? 1 : 2;           // reads of 8 k
+                const half_t *const x = ta[buf][wm + l32], *const y = tb[buf][wn + l32];
+                for (int i = 0; i < ks; i += 8 * R) {
+                    u4 fx[R], fy[NACC][R];
 #pragma unroll
-                    for (int p = 0; p < 8; ++p) {
+                    for (int r = 0; r < R; ++r) fx[r] = read(x + i + 8 * r);
+#pragma unroll
+                    for (int r = 0; r < NACC * R; ++r) fy[r / R][r % R] = read(y + r / R * 32 * FPITCH + i + 8 * (r % R));
+#pragma unroll
+                    for (int p = 0; p < 4 * R; ++p) {
                         const float xv = value(fx[p >> 2][p & 3]);
-                        acc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(xv, value(f0[p >> 2][p & 3]), acc[0], 0, 0, 0);
-                        acc[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(xv, value(f1[p >> 2][p & 3]), acc[1], 0, 0, 0);
+#pragma unroll
+                        for (int t = 0; t < NACC; ++t)
+                            acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(xv, value(fy[t][p >> 2][p & 3]), acc[t], 0, 0, 0);
                     }
                 }
             }
             buf ^= 1;
         }
     if (!working) return;
-    // register v of a lane: row 8 (v / 4) + 4 hi + v % 4 of the wave's, column l32 of 32.  The halves of the wave trade, so that a lane has
-    // column `lane` of rows 8 (v / 4) + v % 4 and of those 4 further: rows of 128 bytes for an instruction.
-    const int n = (int)n0 + lane;
+    // register v of a lane: row 8 (v / 4) + 4 hi + v % 4 of the wave's, column l32 of 32.  Of 64 columns the halves of the wave trade, so that
+    // a lane has column `lane` of rows 8 (v / 4) + v % 4 and of those 4 further: rows of 128 bytes for an instruction.
+    const int n = (int)n0 + (NACC == 2 ? lane : wn + l32);
     half_t* const c = g.C + b0 * g.sCb[0] + b1 * g.sCb[1] + b2 * g.sCb[2] + (long)n * g.sCN;
+    auto store = [&](int m, float sum) __attribute__((always_inline)) {
+        if (m >= g.M || n >= g.N) return;
+        half_t out = (half_t)(sum * g.alpha);
+        if (g.bias)     // same two roundings as the product followed by a separate add
+            out = (half_t)((float)out + (float)g.bias[b0 * g.sbb[0] + b1 * g.sbb[1] + b2 * g.sbb[2] +
+                                                      (long)m * g.sbM + (long)n * g.sbN]);
+        c[(long)m * g.sCM] = out;
+    };
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
-        const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[0][v]), __float_as_uint(acc[1][v]), false, false);
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const int m = (int)m0 + wm + (v >> 2) * 8 + q * 4 + (v & 3);
-            if (m >= g.M || n >= g.N) continue;
-            half_t out = (half_t)(__uint_as_float(both[q]) * g.alpha);
-            if (g.bias)     // same two roundings as the product followed by a separate add
-                out = (half_t)((float)out + (float)g.bias[b0 * g.sbb[0] + b1 * g.sbb[1] + b2 * g.sbb[2] +
-                                                          (long)m * g.sbM + (long)n * g.sbN]);
-            c[(long)m * g.sCM] = out;
+        const int m = (int)m0 + wm + (v >> 2) * 8 + (v & 3);
+        if constexpr (NACC == 2) {
+            const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[0][v]), __float_as_uint(acc[1][v]), false, false);
+            store(m, __uint_as_float(both[0]));
+            store(m + 4, __uint_as_float(both[1]));
+        } else {
+            store(m + 4 * hi, acc[0][v]);
         }
     }
 }
@@ -541,8 +558,10 @@ void launch_gemm(const GemmShape& s, const half_t* A, const half_t* B, half_t* C
         }
     } else {
         if (ep.relu_dropout || ep.gate) fail("gemm: the ReLU-dropout epilogue needs the MFMA kernel");
-        const long blocks = batch * ((c.a.M + FM - 1) / FM) * ((c.a.N + FN - 1) / FN);
+        const bool low = c.a.M <= 64;
+        const long blocks = batch * (low ? 1 : (c.a.M + 127) / 128) * ((c.a.N + FN - 1) / FN);
         if (blocks > 0x7fffffffL) fail("gemm: problem too large for the scalar kernel");
+        const bool few_k = c.a.K1 <= 24;
         // whole 16-byte words along k, or else along the operand's rows (of the output: m resp. n)
         auto how = [&](const half_t* p, long rows, long s_row, long s_k, long s_k0, const long (&sb)[3]) {
             const bool apart = al16(p) && mult8(s_k0) && mult8(sb[0]) && mult8(sb[1]) && mult8(sb[2]);
@@ -550,13 +569,19 @@ void launch_gemm(const GemmShape& s, const half_t* A, const half_t* B, half_t* C
             return apart && s_row == 1 && mult8(s_k) && mult8(rows) ? FMA_ALONG_ROWS : FMA_SINGLE;
         };
         const int how_a = how(c.a.A, c.a.M, c.a.sAM, c.a.sAK1, c.a.sAK0, c.a.sAb), how_b = how(c.a.B, c.a.N, c.a.sBN, c.a.sBK1, c.a.sBK0, c.a.sBb);
+        auto launch = [&](auto ha, auto hb, auto fk) {
+            const dim3 grid((unsigned)blocks);
+            if (low) hipLaunchKernelGGL((k_gemm_fma<ha(), hb(), 64, fk()>), grid, dim3(256), 0, st, c.a);
+            else hipLaunchKernelGGL((k_gemm_fma<ha(), hb(), 128, fk()>), grid, dim3(256), 0, st, c.a);
+        };
         auto run = [&](auto ha) {
-            auto with = [&](auto hb) { hipLaunchKernelGGL((k_gemm_fma<ha(), hb()>), dim3((unsigned)blocks), dim3(256), 0, st, c.a); };
+            auto with = [&](auto hb) { launch(ha, hb, std::integral_constant<int, 32>{}); };
             if (how_b == FMA_ALONG_K) with(std::integral_constant<int, FMA_ALONG_K>{});
             else if (how_b == FMA_ALONG_ROWS) with(std::integral_constant<int, FMA_ALONG_ROWS>{});
             else with(std::integral_constant<int, FMA_SINGLE>{});
         };
-        if (how_a == FMA_ALONG_K) run(std::integral_constant<int, FMA_ALONG_K>{});
+        if (few_k) launch(std::integral_constant<int, FMA_SINGLE>{}, std::integral_constant<int, FMA_SINGLE>{}, std::integral_constant<int, 8>{});
+        else if (how_a == FMA_ALONG_K) run(std::integral_constant<int, FMA_ALONG_K>{});
         else if (how_a == FMA_ALONG_ROWS) run(std::integral_constant<int, FMA_ALONG_ROWS>{});
         else run(std::integral_constant<int, FMA_SINGLE>{});
     }

@@ -318,7 +318,9 @@ def test_nothing_behind_what_an_activation_epilogue_leaves_is_written(L, E, U, a
 # k left over, tiles of 128 x 64 with 1, 32, 33 and 64 columns in the last one)
 @pytest.mark.parametrize('la,lb,lc', [('BJHP', 'BKHP', 'HBJK'), ('HBJK', 'BKHP', 'BJHP'), ('HBKJ', 'KBHP', 'BJHP'), ('HPBJ', 'BKHP', 'BHKJ'),
                                       ('BHJP', 'HBPK', 'JBHK'), ('BHJK', 'BJHP', 'HBPK')])
-@pytest.mark.parametrize('dims', [(2, 33, 2, 24), (1, 97, 1, 64), (1, 129, 3, 192), (3, 65, 1, 31), (1, 255, 1, 8)])
+# (up to 24 k in steps of 8: 1 to 24 positions; products of up to 64 rows in tiles of 64: 1, 32, 33, 64)
+@pytest.mark.parametrize('dims', [(2, 33, 2, 24), (1, 97, 1, 64), (1, 129, 3, 192), (3, 65, 1, 31), (1, 255, 1, 8), (2, 1, 2, 10), (1, 8, 2, 66),
+                                  (2, 9, 1, 64), (3, 24, 2, 50), (1, 25, 2, 48), (2, 32, 1, 17), (1, 64, 2, 130), (2, 63, 3, 3)])
 def test_sums_without_whole_words_are_one_chain_of_fused_multiply_adds(la, lb, lc, dims):
     """Bit for bit, in the order of k: products of halves are exact in float64, and so are their sums with an fp32 value (here: 11 + 11
     bits at exponents within 2 ** +-24), so that rounding each sum to float32 is what fmaf does."""
