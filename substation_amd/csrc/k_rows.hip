@@ -778,8 +778,11 @@ void launch_bdrln(const RowSpace& rs, View in, View resid, View lin_bias, View s
     }
     if (flat) {
         // Few rows: each in a workgroup of its own, on a CU of its own (64 rows of 768, us with four rows to a workgroup and now: 3.9 and 3.7,
-        // with the parts of a split sum 5.3 and 4.5; 256 rows: no difference).
-        const unsigned waves = extra_blocks || nrows >= 256 ? WPB : 1;
+        // with the parts of a split sum 5.3 and 4.5; 256 rows: no difference).  Not the fewest, which share what they read of the three
+        // vectors, unless they have parts to add up or are long: 4, 8 and 16 rows of 768 3.4, 3.7 and 3.8, each alone 3.6, 4.1 and 4.0; the two
+        // launches of a layer, 8 rows of 2048 8.0 and 9.2, with parts of 1024 9.5 and 8.9, 16 rows of 4096 15.0 and 12.5.
+        const bool apart = nrows > 16 || sums.p || rs.R > 2048;
+        const unsigned waves = extra_blocks || nrows >= 256 || !apart ? WPB : 1;
         const dim3 grid(waves == WPB ? row_grid(nrows, 1) + extra_blocks : nrows), block(waves * WAVE);
 #define SUB_BDRLN_FLAT(V, S) hipLaunchKernelGGL((k_bdrln_flat<V, S>), grid, block, 0, st, rs.R, nrows, in, resid, lin_bias, \
                                              scale, bias, lin, mask, diff, normed, out, istd, key, eps, mask_bits, write_lin, job, sums, saves, waves)
