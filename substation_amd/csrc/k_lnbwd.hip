@@ -384,9 +384,13 @@ inline int lnbwd_blocks(long nrows) {
 // Four sums (the extended form without move_sum) do not fit the 128 registers of sixteen waves; with eight, two rows each and more, they
 // take less than in the kernel above, which row spaces that are not flat are left to: 4096 rows of 1024 18.9 -> 16.7 us, 8192 30.4 -> 28.7, 3072 of
 // 768 14.5 -> 12.7.
-inline int lnbwd_waves(long nrows, bool four) { return nrows <= 1024 ? 4 : nrows <= 2048 || four ? 8 : 16; }
-inline int lnbwd_flat_blocks(long nrows, bool four) {
-    const int waves = lnbwd_waves(nrows, four);
+// Rows of up to 512 features: four up to 512 rows, eight up to 1536, since what more partial rows cost the launch that adds them up outweighs the
+// rest (with that launch, us with sixteen, four and eight: 900 rows of 384 8.4, 9.0 and 7.9, 1024 of 512 8.8, 9.4 and 8.6; 2048 of 256 9.1 and, eight, 9.5).
+inline int lnbwd_waves(long nrows, int R, bool four) {
+    return nrows <= (R <= 512 ? 512 : 1024) ? 4 : nrows <= (R <= 512 ? 1536 : 2048) || four ? 8 : 16;
+}
+inline int lnbwd_flat_blocks(long nrows, int R, bool four) {
+    const int waves = lnbwd_waves(nrows, R, four);
     return waves == 16 ? lnbwd_blocks(nrows) : (int)std::min((nrows + waves - 1) / waves, 256L);
 }
 // Longer rows, which two or four of sixteen waves share: a workgroup for each eight or four of them, as long as that is no more than one
@@ -411,7 +415,7 @@ bool lnbwd_supported(const RowSpace& rs, const LnBwdArgs& a, bool ext) {
 }
 
 size_t lnbwd_ws_floats(const RowSpace& rs, bool ext) {
-    const int blocks = rs.R <= 1024 ? std::max(lnbwd_blocks(rs.rows()), lnbwd_flat_blocks(rs.rows(), ext)) : lnbwd_wide_blocks(rs.rows(), rs.R);
+    const int blocks = rs.R <= 1024 ? std::max(lnbwd_blocks(rs.rows()), lnbwd_flat_blocks(rs.rows(), rs.R, ext)) : lnbwd_wide_blocks(rs.rows(), rs.R);
     return (size_t)(ext ? 4 : 3) * blocks * rs.R;      // (3: the plain form with move_sum)
 }
 
@@ -421,7 +425,7 @@ void launch_lnbwd(const RowSpace& rs, const LnBwdArgs& a, bool ext, half_t* cons
     if (!ws) fail("fused LayerNorm backward: no reduction workspace");
     const unsigned nrows = (unsigned)rs.rows();
     const bool four = ext && !a.move_sum, flat = rs.R <= 1024 && rs.flat;
-    const int blocks = rs.R > 1024 ? lnbwd_wide_blocks(nrows, rs.R) : flat ? lnbwd_flat_blocks(nrows, four) : lnbwd_blocks(nrows);
+    const int blocks = rs.R > 1024 ? lnbwd_wide_blocks(nrows, rs.R) : flat ? lnbwd_flat_blocks(nrows, rs.R, four) : lnbwd_blocks(nrows);
     const int vpl = rs.R <= 512 ? 1 : 2;
     if (rs.R > 1024) {
         // (lnbwd_supported has ruled out the extended form without move_sum: MOVE_ is EXT_ || move_sum)
@@ -447,7 +451,7 @@ void launch_lnbwd(const RowSpace& rs, const LnBwdArgs& a, bool ext, half_t* cons
     do {                                                                                                          \
         const dim3 grid(blocks);                                                                                  \
         if (!flat) hipLaunchKernelGGL((k_lnbwd<VPL_, EXT_, BITS_, MOVE_>), grid, dim3(LN_BLOCK), 0, st, rs, a, ws, nrows);       \
-        else switch (lnbwd_waves(nrows, four)) {                                                                        \
+        else switch (lnbwd_waves(nrows, rs.R, four)) {                                                            \
             case 4: hipLaunchKernelGGL((k_lnbwd_flat<VPL_, EXT_, BITS_, MOVE_, 1, 4>), grid, dim3(4 * WAVE), 0, st, rs.R, a, ws, nrows); break; \
             case 8: hipLaunchKernelGGL((k_lnbwd_flat<VPL_, EXT_, BITS_, MOVE_, 1, 8>), grid, dim3(8 * WAVE), 0, st, rs.R, a, ws, nrows); break; \
             default:                                                                                              \

@@ -516,7 +516,7 @@ def test_ln_backward_one_launch_or_separate(B, L, H, E, extended):
 # (where the number of waves of a workgroup changes: 1024 and 2048 rows, a last workgroup of one row; one, two packs a lane)
 # (rows of more than 1024 features: a workgroup for each of the last ones, two passes of which the last leaves waves without a row)
 @pytest.mark.parametrize('B,L,E', [(1, 1, 1024), (1, 5, 520), (1, 1024, 512), (5, 205, 776), (2, 1024, 1024), (3, 683, 512),
-                                   (1, 3, 4096), (1, 1030, 4096), (3, 687, 2048), (1, 2049, 512), (5, 821, 776)])
+                                   (1, 3, 4096), (1, 1030, 4096), (3, 687, 2048), (1, 2049, 512), (5, 821, 776), (1, 513, 512), (1, 1537, 512)])
 @pytest.mark.parametrize('extended', [False, True])
 def test_ln_backward_in_workgroups_of_every_size(B, L, E, extended):
     test_ln_backward_one_launch_or_separate(B, L, 1, E, extended)
