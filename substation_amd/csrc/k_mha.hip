@@ -1261,21 +1261,25 @@ void for_variant(int P, const AttnArgs& a, Fn&& fn) {
 // 32 tiles, H 4: causal 37.9, 31.8, 42.0 and 24.6, 22.1, 29.9; all zeros 39.7, 33.4, 42.6 and 33.5, 28.7, 36.2; a quarter of the keys gone 31.2,
 // 26.6, 41.2 and 27.2, 24.0, 34.7; a window of a quarter 19.8, 18.0, 22.5 and 17.7, 16.9, 21.0; a slope 43.8, 42.4, 59.9 and 36.6, 33.2, 46.3; causal without
 // lists 37.1, 38.0, 56.8 and 31.4, 31.8, 44.4.  192 blocks of 12 tiles: causal 17.8, 16.2, 20.1 and 14.9, 14.6, 17.7, a quarter gone 15.2, 13.2, 24.4 and
-// 14.5, 14.2, 19.9.  Beyond, some lose: 320 blocks of 32 tiles causal 39.5, 34.5, 45.2 and 28.4, 28.6, 35.5, but zeros 51.9, 42.3, 52.1 and 46.5, 40.1, 53.9,
-// a window 23.4, 21.1, 26.7 and 24.2, 23.2, 31.0; so they do with fewer tiles: 256 blocks of 8, a window 12.8, 12.8, 13.9 and 13.2, 13.5, 14.8.
-int parts(const AttnArgs& a, int P, long rows, long others) {
-    const long few = a.amask && tiles(others) >= 12 ? 2 * kFewBlocks : kFewBlocks;
+// 14.5, 14.2, 19.9.  With fewer tiles some lose: 256 blocks of 8, a window 12.8, 12.8, 13.9 and 13.2, 13.5, 14.8.
+// Up to one and a half to a CU dK and dV lose too (320 blocks of 32 tiles, zeros 52.1 and 53.9, a window 26.7 and 31.0), forward and dQ of 32 tiles
+// and more do not, but for masks that leave a block a few tiles.  us of forward and dQ in ten layers of 288 to 384 blocks, each timed alone by
+// events: 3 x 1024, H 12, causal 60.1, 46.4 and 42.7, 33.2; zeros 60.7, 47.6 and 56.4, 43.7; a quarter gone 48.3, 37.8 and 46.2, 35.8; windows of a
+// half, a quarter and an eighth 43.9, 33.9 and 36.9, 28.6; 33.1, 25.6 and 30.0, 23.4; 27.8, 21.9 and 26.4, 20.8; documents of 256 25.9, 19.9 and 26.5,
+// 20.5; all of them between 0.65 and 1.07 (3 x 1000, H 12, documents, dQ 19.8 and 21.0), in the middle 0.93 and 0.92.
+int parts(const AttnArgs& a, int P, long rows, long others, bool kv) {
+    const long few = !a.amask || tiles(others) < 12 ? kFewBlocks : kv || tiles(others) < 32 ? 2 * kFewBlocks : 3 * kFewBlocks;
     return P == 64 && a.H * (long)a.B * blocks(rows) <= few && tiles(others) >= 4 ? 2 : 1;
 }
 }  // namespace
 
-long mha_bias_rows_q(const AttnArgs& a, int P) { return a.B * blocks(a.J) * parts(a, P, a.J, a.K); }
-long mha_bias_rows_kv(const AttnArgs& a, int P) { return a.B * blocks(a.K) * parts(a, P, a.K, a.J); }
+long mha_bias_rows_q(const AttnArgs& a, int P) { return a.B * blocks(a.J) * parts(a, P, a.J, a.K, false); }
+long mha_bias_rows_kv(const AttnArgs& a, int P) { return a.B * blocks(a.K) * parts(a, P, a.K, a.J, true); }
 size_t mha_bias_floats(long H, long B, long J, long K, long P) { return (size_t)(2 * H * P * B * (blocks(J) + 2 * blocks(K))); }
 
 void launch_mha_forward(const AttnArgs& a, int P, PhiloxKey key, bool same_order, hipStream_t st) {
     if (!mha_forward_ok(a, P)) fail("attention forward: shape, strides or alignment not supported");
-    const int n = same_order ? 1 : parts(a, P, a.J, a.K);
+    const int n = same_order ? 1 : parts(a, P, a.J, a.K, false);
     dim3 grid((unsigned)(a.H * a.B * blocks(a.J) * n));
     for_variant(P, a, [&](auto p, auto masked, auto rag) {
         if constexpr (p() == 64) {
@@ -1292,7 +1296,7 @@ bool mha_backward_ok(const AttnArgs& a, int P) {
 
 void launch_mha_backward_dq(const AttnArgs& a, int P, hipStream_t st) {
     if (!mha_backward_ok(a, P)) fail("attention backward: shape, strides or alignment not supported");
-    const int n = parts(a, P, a.J, a.K);
+    const int n = parts(a, P, a.J, a.K, false);
     dim3 grid((unsigned)(a.H * a.B * blocks(a.J) * n));
     for_variant(P, a, [&](auto p, auto masked, auto rag) {
         if constexpr (p() == 64) {
@@ -1305,7 +1309,7 @@ void launch_mha_backward_dq(const AttnArgs& a, int P, hipStream_t st) {
 
 void launch_mha_backward_dkv(const AttnArgs& a, int P, hipStream_t st) {
     if (!mha_backward_ok(a, P)) fail("attention backward: shape, strides or alignment not supported");
-    const int n = parts(a, P, a.K, a.J);
+    const int n = parts(a, P, a.K, a.J, true);
     dim3 grid((unsigned)(a.H * a.B * blocks(a.K) * n));
     for_variant(P, a, [&](auto p, auto masked, auto rag) {
         if constexpr (p() == 64) {

@@ -242,8 +242,10 @@ ATTENTION = {
     (4, 16, 512, 512, 64, True, 'gelu'): 'hhh',       # 256 of 16
     (2, 16, 1024, 1024, 64, True, 'gelu'): 'hhh',     # 256 of 32
     (8, 16, 256, 256, 64, True, 'gelu'): 'www',       # 256 of 8
-    (3, 12, 1024, 1024, 64, True, 'gelu'): 'www',     # 288 of 32
-    (2, 12, 2048, 2048, 64, True, 'gelu'): 'www',     # 384 of 64
+    (9, 8, 512, 512, 64, True, 'gelu'): 'www',        # 288 of 16
+    (3, 12, 1024, 1024, 64, True, 'gelu'): 'hhw',     # 288 of 32
+    (2, 12, 2048, 2048, 64, True, 'gelu'): 'hhw',     # 384 of 64
+    (25, 16, 128, 1024, 64, True, 'gelu'): 'www',     # 400 of queries, 3200 of keys
     (2, 24, 128, 384, 64, True, 'gelu'): 'hhw',       # 48 of queries; 144 of keys, of 4 tiles
     (2, 16, 1000, 1000, 64, True, 'gelu'): 'hhh',     # (a layer's: lengths with an end inside a tile)
     (5, 10, 201, 201, 64, False, 'gelu'): 'hhh',      # 100
@@ -288,6 +290,7 @@ def _attention_launches():
 
 
 def test_which_attention_launches_share_a_block_between_two_waves(tmp_path):
-    """Operators and layers alike: up to 128 blocks, behind a mask up to one for each of 256 CUs where a block has 12 tiles to walk."""
+    """Operators and layers alike: up to 128 blocks, behind a mask up to one for each of 256 CUs where a block has 12 tiles to walk, but
+    for dK and dV up to one and a half where it has 32."""
     lines = launches.run(_attention_launches, tmp_path)
     assert dict(zip(ATTENTION, lines)) == ATTENTION
