@@ -229,6 +229,8 @@ def test_order_of_the_sums_in_front_of_a_relu(tmp_path):
     assert dict(zip(ORDERS, lines)) == ORDERS
 
 
+HALVES_TESTED = [(128, 128), (256, 128), (128, 384), (512, 512), (384, 1024)]
+
 # (samples, heads, queries, keys, head size, mask, activation): blocks of 128 queries and of keys; whether forward, dQ, and dK and dV take the
 # kernels in which two waves share a block's other side (h) or those of whole blocks (w)
 ATTENTION = {
@@ -250,6 +252,10 @@ ATTENTION = {
     (2, 16, 1000, 1000, 64, True, 'gelu'): 'hhh',     # (a layer's: lengths with an end inside a tile)
     (5, 10, 201, 201, 64, False, 'gelu'): 'hhh',      # 100
     (13, 12, 201, 201, 64, False, 'gelu'): 'www',     # 312
+    # what tests/test_ops_gpu.py takes for halves and for whole blocks
+    **{(2, 2, J, K, 64, mask, 'gelu'): 'hhh' for J, K in HALVES_TESTED for mask in (False, True)},
+    **{(130, 2, J, K, 64, mask, 'gelu'): 'www' for J, K in HALVES_TESTED for mask in (False, True)},
+    **{(n, 2, L, L, 64, True, 'gelu'): row for L, few in ((97, 2), (400, 20), (1001, 12)) for n, row in ((few, 'hhh'), (70, 'www'))},
 }
 
 

@@ -405,7 +405,7 @@ def test_attention_by_halves_of_the_other_side_equals_the_whole(J, K, p, mask):
     from substation_amd.ops import Ops
     B, H, P = 2, 2, 64
     g = torch.Generator(device='cuda').manual_seed(J + K)
-    many = 40                                                # samples: more than 128 blocks
+    many = 130                                               # samples: more than 256 blocks (tests/test_launch_plans.py has both)
     full = lambda n: torch.randn((many, n, H, P), generator=g, device='cuda').half()
     q, k, v, d_out = full(J), full(K), full(K), full(J)
     am = None
