@@ -1172,7 +1172,7 @@ __global__ __launch_bounds__(256, (P == 64 && MASKED) ? 2 : 1) void k_mha_bwd_dk
     mha_bwd_dkv<P, MASKED, RAGGED, 1>(a);
 }
 template <int P, bool MASKED, bool RAGGED>
-__global__ __launch_bounds__(256, MASKED ? 2 : 1) void k_mha_bwd_dkv_halves(AttnArgs a) {
+__global__ __launch_bounds__(256, MASKED && RAGGED ? 2 : 1) void k_mha_bwd_dkv_halves(AttnArgs a) {
     mha_bwd_dkv<P, MASKED, RAGGED, 2>(a);
 }
 
@@ -1313,10 +1313,17 @@ void launch_mha_backward_dkv(const AttnArgs& a, int P, hipStream_t st) {
     dim3 grid((unsigned)(a.H * a.B * blocks(a.K) * n));
     for_variant(P, a, [&](auto p, auto masked, auto rag) {
         if constexpr (p() == 64) {
-            // (behind a mask the kernel for any length at every length: without the end checks it takes 284 registers, one wave per SIMD,
-            // where this one takes 249; held to 256 it spills around the mask values.  us at 256 blocks of 32 tiles, all zeros, H 16:
-            // whole blocks 40.8, halves 49.1 with 284 registers, 36.2 now)
-            if (n == 2) { hipLaunchKernelGGL((k_mha_bwd_dkv_halves<p(), masked(), masked() || rag()>), grid, dim3(256), 0, st, a); return; }
+            // (behind a mask and with two workgroups on a CU the kernel for any length at every length: without the end checks it takes 284
+            // registers, one wave per SIMD, where this one takes 249; held to 256 it spills around the mask values.  us at 256 blocks of 32
+            // tiles, all zeros, H 16: whole blocks 40.8, halves 49.1 with 284 registers, 36.2 now.  Alone on a CU the one without is the faster:
+            // dQ, dK and dV of 1 x 2048 on 128, H 16, 60.6 and 67.1; 1 x 2048, H 8, 101 and 108; 2 x 512, H 16, 33.4 and 35.4)
+            if constexpr (masked()) {
+                if (n == 2 && a.H * (long)a.B * blocks(a.K) > kFewBlocks) {
+                    hipLaunchKernelGGL((k_mha_bwd_dkv_halves<p(), true, true>), grid, dim3(256), 0, st, a);
+                    return;
+                }
+            }
+            if (n == 2) { hipLaunchKernelGGL((k_mha_bwd_dkv_halves<p(), masked(), rag()>), grid, dim3(256), 0, st, a); return; }
         }
         hipLaunchKernelGGL((k_mha_bwd_dkv<p(), masked(), rag()>), grid, dim3(256), 0, st, a);
     });
