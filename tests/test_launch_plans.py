@@ -301,3 +301,51 @@ def test_which_attention_launches_share_a_block_between_two_waves(tmp_path):
     for dK and dV up to one and a half where it has 32."""
     lines = launches.run(_attention_launches, tmp_path)
     assert dict(zip(ATTENTION, lines)) == ATTENTION
+
+
+# rows, features: rows to a workgroup of k_bdrln_flat (one row: either)
+BDRLN = {(4, 768): 4, (16, 768): 4, (17, 768): 1, (255, 768): 1, (256, 768): 4, (16, 2048): 4, (16, 2056): 1, (8, 4096): 1}
+# rows, features: waves and workgroups of k_lnbwd_flat, for two sums and for four
+LNBWD = {(1, 512): '4:1 4:1', (512, 512): '4:128 4:128', (513, 512): '8:65 8:65', (1536, 512): '8:192 8:192', (1537, 512): '16:97 8:193',
+         (1024, 520): '4:256 4:256', (1025, 520): '8:129 8:129', (2048, 1024): '8:256 8:256', (2049, 1024): '16:129 8:256', (8192, 1024): '16:256 8:256'}
+# positions, head size: rows and k of the tiles of the scores' product, workgroups of four products
+ANY_STRIDES = {(1, 10): '64 8 4', (63, 24): '64 8 4', (64, 25): '64 32 4', (65, 24): '128 8 8', (65, 25): '128 32 8', (201, 64): '128 32 32'}
+
+
+def _few_rows_and_odd_products():
+    from substation_amd import _lib, layouts as L
+    lib = _lib.load()
+    t = launches.tensors(16)
+
+    def handle(*dims):
+        return _lib.Handle(_lib.make_config(*dims, L.mi355x_layouts(), 0.1, 0.1, 0.1, 0.1))
+
+    def only(kernel, call):
+        (found, grid), = [(re.search(kernel, name), grid[0]) for name, grid in launches.launched(lambda: _lib.check(call())) if re.search(kernel, name)]
+        return [int(n) for n in found.groups()] + [grid]
+
+    for rows, features in BDRLN:
+        h = handle(rows, 1, 1, features)
+        grid, = only('k_bdrln_flat', lambda: lib.sub_op_bdrln(
+            h.ptr, t[0], b'BJI', t[1], b'BJI', t[2], t[3], t[4], t[5], b'BJI', t[6], b'BJI', t[7], b'BJI', t[8], b'BJI', t[9], b'BJI', t[10], b'BJ', 0.1, 1))
+        print({rows: 1, -(-rows // 4): 4}.get(grid))
+    for rows, features in LNBWD:
+        h, row = handle(rows, 1, 1, features), []
+        for four in (False, True):
+            second = [x if four else None for x in t[11:15]]
+            waves, grid = only(r'k_lnbwd_flatILi\dELb\dELb\dELb\dELi1ELi(\d+)E', lambda: lib.sub_op_ln_backward(
+                h.ptr, int(four), t[0], b'BJI', t[1], t[2], b'BJI', second[0], b'BJI', second[1], b'BJI', t[3], b'BJ', t[4], b'BJI', t[5], b'BJI', t[6],
+                b'BJI', t[7], b'BJI', t[8], b'BJI', t[9], t[10], second[2], second[3]))
+            row.append(f'{waves}:{grid}')
+        print(*row)
+    for n, size in ANY_STRIDES:
+        h = handle(2, n, 2, 2 * size)
+        print(*only(r'k_gemm_fmaILi\dELi\dELi(\d+)ELi(\d+)E',
+                    lambda: lib.sub_op_einsum(h.ptr, t[0], b'BJHP', t[1], b'BKHP', t[2], b'HBJK', 1.0)))
+
+
+def test_launches_of_few_rows_and_of_products_without_whole_words(tmp_path):
+    """Where a rule changes its answer: nothing that a result shows (each was timed on both sides)."""
+    lines = launches.run(_few_rows_and_odd_products, tmp_path)
+    want = [str(v) for v in [*BDRLN.values(), *LNBWD.values(), *ANY_STRIDES.values()]]
+    assert lines == want
