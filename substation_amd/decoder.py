@@ -18,6 +18,7 @@ without rescaling; as in the reference there is none on the attention
 probabilities of this layer.
 """
 import math
+from operator import index
 
 import torch
 
@@ -114,7 +115,7 @@ def _make_function(m):
             x, enc = x.contiguous(), enc.contiguous()
             step, m.step = m.step, m.step + 1
             ctx.mask = m.sattn_mask
-            kept = passes.forward(x, enc, params, ctx.mask, m.seed & (2**64 - 1), step & (2**32 - 1), bool(m.activation_epilogues))
+            kept = passes.forward(x, enc, params, ctx.mask, index(m.seed) & (2**64 - 1), index(step) & (2**32 - 1), bool(m.activation_epilogues))
             y = kept.pop(Passes.OUTPUT)
             m.ffn_in_epilogues = kept[Passes.BITS] is not None
             ctx.save_for_backward(x, enc, *params)

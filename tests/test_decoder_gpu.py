@@ -282,3 +282,18 @@ def test_decoder_layer_puts_no_sums_off_where_one_of_its_handles_cannot():
     sums = torch.full((128,), -1.0, dtype=torch.float16, device='cuda')
     layer.ops_t.baob(torch.ones_like(dy), 'BJI', sums)
     assert bool((sums == 128).all())
+
+
+def test_decoder_layer_takes_any_integer_type_as_seed_and_step():
+    from substation_amd import DecoderLayer
+    layer = DecoderLayer(1, 128, 128, 2, 128, activation='gelu').cuda()
+    x, enc = (torch.randn(1, 128, 128).half().cuda() for _ in range(2))
+
+    def run(seed, step):
+        layer.set_rng(seed, step)
+        with torch.no_grad():
+            return layer(x, enc)
+
+    want = run(5, 7)
+    for seed, step in ((np.int64(5), np.int32(7)), (np.uint64(5), np.uint8(7)), (torch.tensor(5), torch.tensor(7))):
+        assert torch.equal(run(seed, step), want)
