@@ -228,6 +228,7 @@ struct Handle {
     bool ops_deferring = false;   // the same across operator calls, between sub_ops_defer(h, 1) and sub_ops_defer(h, 0)
     size_t ws_cursor = 0;
     FinishJobs deferred;
+    bool deferred_elsewhere = false;  // the stream has changed since a sum on the list was put off
     float* gws = nullptr;         // split-k partials of the small-output contractions
     size_t gws_floats = 0, gws_need = 0;
     bool profiling = false;
@@ -389,6 +390,7 @@ float* take_ws(Handle& h, size_t floats) {
         if (!h.ops_deferring) fail("column-reduction workspace exhausted");
         if (h.deferred.n > 0) launch_colfinish(h.deferred, h.stream);
         h.deferred.n = 0;
+        h.deferred_elsewhere = false;
         h.ws_cursor = 0;
         // twice the size as well, and no less than two backward passes of the layer take: a new handle's first block of calls
         // asks the device for memory once, where it went on doubling (each time a wait for all that runs)
@@ -1694,7 +1696,11 @@ void* init_cfg(const sub_config* cfg) {
 }
 
 int sub_set_stream(void* handle, void* hip_stream) {
-    return guarded([&] { as_handle(handle).stream = (hipStream_t)hip_stream; });
+    return guarded([&] {
+        Handle& h = as_handle(handle);
+        if ((hipStream_t)hip_stream != h.stream && h.deferred.n > 0) h.deferred_elsewhere = true;
+        h.stream = (hipStream_t)hip_stream;
+    });
 }
 
 int sub_set_rng(void* handle, uint64_t seed, uint32_t step) {
@@ -2191,6 +2197,7 @@ int sub_ops_defer(void* handle, int on) {
             h.ops_deferring = h.deferring = true;
             h.ws_cursor = 0;
             h.deferred.n = 0;
+            h.deferred_elsewhere = false;
         } else if (h.ops_deferring) {
             h.ops_deferring = h.deferring = false;
             FinishJobs jobs = h.deferred;
@@ -2383,12 +2390,12 @@ int sub_op_einsum_group(void* handle, const SubEinsum* p, int n) {
         // (entries of the per-launch timing are a layer call's: nothing would take an operator call's away again)
         // What column sums wait (sub_ops_defer) are finished in places that the tiles of the group's last launch leave free, as in
         // encoder_backward.  (The backward pass of a decoder layer, 8 x 256 on 512, E 1024: 5.2 and 4.0 us
-        // of launches of their own, and nothing more here.)
+        // of launches of their own, and nothing more here.)  Not sums of another stream than this group's, which does not wait for it.
         const GroupPlan& plan = group_plan(h, jobs);
         const GemmLaunch* last = nullptr;
         for (const GemmStage& stage : plan.stage)
             for (int i = 0; i < stage.n; ++i) last = &stage.launch[i];
-        FinishJobs* const waiting = h.ops_deferring && h.finish_in_pair && h.deferred.n > 0 ? &h.deferred : nullptr;
+        FinishJobs* const waiting = h.ops_deferring && h.finish_in_pair && h.deferred.n > 0 && !h.deferred_elsewhere ? &h.deferred : nullptr;
         for (const GemmStage& stage : plan.stage)
             for (int i = 0; i < stage.n; ++i) run_launch(h, jobs.data(), stage.launch[i], &stage.launch[i] == last ? waiting : nullptr);
     });

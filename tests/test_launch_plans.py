@@ -152,6 +152,31 @@ def test_groups_that_a_handle_has_seen_before(tmp_path):
     assert len(lines) == 60 and set(lines) == {'same'}, [l for l in lines if l != 'same'][:2]
 
 
+def _groups_in_a_block_of_sums():
+    for streams in ((1, 1, 1), (1, 2, 1), (1, 2, 2), (1, 1, 2), (2, 2, 1)):        # of a sum, of the group, where the block ends
+        g = Group()
+        h = g.handles[0]
+        a, b = launches.tensors(2, first=64)
+        for turn in range(2):                # (the first one makes the buffer)
+            h.set_stream(streams[0])
+            h.defer_column_sums(True)
+            g.l.check(g.lib.sub_op_baob(h.ptr, a, b'BJI', b))
+            h.set_stream(streams[1])
+            g.launched()
+
+            def end():
+                h.set_stream(streams[2])
+                h.defer_column_sums(False)
+            last = [name for name, _ in launches.launched(end)]
+        print(streams, len(last))
+
+
+def test_a_group_finishes_no_column_sums_of_another_stream(tmp_path):
+    """It would not wait for them; they end with the block, on the stream that is current there."""
+    lines = launches.run(_groups_in_a_block_of_sums, tmp_path)
+    assert lines == ['(1, 1, 1) 0', '(1, 2, 1) 1', '(1, 2, 2) 1', '(1, 1, 2) 0', '(2, 2, 1) 0']
+
+
 def _two_threads():
     import threading
     from substation_amd import _lib, layouts as L
