@@ -220,7 +220,9 @@ def test_default_path_matches_the_oracle(dims, p, masked, compact):
 @pytest.mark.parametrize('dims,masked,compact', [
     ((3, 8, 2, 128), False, False), ((2, 33, 2, 128), True, False), ((5, 77, 3, 192), False, True),
     ((2, 127, 1, 128), False, False), ((3, 129, 2, 128), True, True), ((2, 201, 2, 256), False, True),
-    ((1, 200, 2, 256), True, False), ((1, 285, 3, 192), True, True)])
+    ((1, 200, 2, 256), True, False), ((1, 285, 3, 192), True, True),
+    # five and six tiles to two waves, of which the second begins at the fourth
+    ((3, 130, 2, 128), False, False), ((2, 161, 2, 128), False, True), ((2, 333, 2, 128), True, False)])
 def test_attention_in_registers_at_any_sequence_length(dims, masked, compact):
     """Sequence lengths that are not multiples of 128, head sizes 64 and 128: the layer as shipped against the oracle."""
     L, launches = dims[1], []
