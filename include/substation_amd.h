@@ -429,8 +429,8 @@ int sub_op_baob(void* handle, const void* datt, const char* l_datt, void* dbo);
  * reduction; no counterpart there).  The gradient vectors are complete only after
  * that call; same bits as without.  When the list (6 entries) or the scratch buffer
  * is full, what is on the list is finished early, and so it is by a group of contractions
- * (sub_op_einsum_group), whose last launch has room for it.  encoder_backward refuses to run
- * in between. */
+ * (sub_op_einsum_group) on the stream of the sums, whose last launch has room for it.  encoder_backward
+ * refuses to run in between. */
 int sub_ops_defer(void* handle, int on);
 /* block_aib.cuh:64-155, on the Q-stacked tensors */
 int sub_op_aib(void* handle, const void* in, const char* l_in, const void* bias, const char* l_bias,
